@@ -272,6 +272,81 @@ def test_moe_sort_and_grouped_gemm(dt, granule, P, E, top):
     assert rel(o.numpy(np.float32, (P, W)), want) < 1e-5
 
 
+# the row-major prompt GEMM (csrc/gemm_rows.cuh): edges of its 64 / 128 / 256-wide tiles, remainders in M and N, the shortest and longer K rings,
+# every epilogue; bf16 only.  f32 outputs: sums of K products of bf16 values in f32, K ascending — relative error of a chain of K
+# roundings, far below 2e-6 of the result's norm; bf16 outputs: one rounding more (2^-9 of the value)
+@pytest.mark.parametrize("M,N,K", [(33, 16, 64), (64, 128, 128), (65, 130, 192), (127, 256, 64), (129, 264, 320), (257, 72, 256), (300, 1000, 64)])
+@pytest.mark.parametrize("form", ["f32", "bf16", "bias", "unaligned", "scatter", "gelu", "batch"])
+def test_gemm_rows_edges(M, N, K, form):
+    L = _lib.load()
+    r = np.random.default_rng(M + N + K)
+    nb = 3 if form == "batch" else 1
+    a = so.bf16_round(r.standard_normal((M, nb * K)).astype(np.float32))
+    w = so.bf16_round((r.standard_normal((nb, N, K)) / np.sqrt(K)).astype(np.float32))
+    ref = np.stack([a[:, z * K:(z + 1) * K].astype(np.float64) @ w[z].astype(np.float64).T for z in range(nb)], 1)  # [M, nb, N]
+    ad, wd = to_dev(a, BF16), to_dev(w, BF16)
+    ldo = nb * N + (3 if form == "unaligned" else 0)
+    rows = M + 5
+    out = empty(rows * ldo * 4).fill_bytes(0)
+    if form == "scatter":  # every third row is not written, the others land in reverse order
+        dst = np.arange(M - 1, -1, -1, dtype=np.int32)
+        dst[::3] = -1
+        L.vra_stack_op_gemm(ad.ptr, K, wd.ptr, 0, out.ptr, ldo, 1, M, N, K, 1.0, None, 0, None, None, raw(dst, np.int32).ptr, 0, 0.0, BF16, 0)
+        check()
+        got = out.numpy(np.float32, (rows, ldo))
+        keep_rows = dst >= 0
+        assert rel(got[dst[keep_rows]], ref[keep_rows, 0]) < 2e-6
+        assert (np.delete(got, dst[keep_rows], axis=0) == 0).all()
+        return
+    bias = r.standard_normal(N).astype(np.float32)
+    f32_out = form not in ("bf16", "gelu", "unaligned")
+    if form in ("bias", "gelu", "batch"):
+        L.vra_stack_op_gemm_ex(ad.ptr, nb * K, wd.ptr, out.ptr, ldo, int(f32_out), M, N, K, 0.5, raw(bias, np.float32).ptr if form != "batch" else None,
+                               2 if form == "gelu" else 0, 3 if form == "gelu" else 0, nb, K, N * K, N, BF16, 0)
+        ref = 0.5 * ref + (bias if form != "batch" else 0.0)
+        if form == "gelu":
+            ref = 0.5 * ref * (1.0 + np.vectorize(math.erf)(ref / math.sqrt(2.0)))
+    else:
+        L.vra_stack_op_gemm(ad.ptr, K, wd.ptr, 0, out.ptr, ldo, int(f32_out), M, N, K, 1.0, None, 0, None, None, None, 0, 0.0, BF16, 0)
+    check()
+    got = (out.numpy(np.float32, (rows, ldo)) if f32_out else from_dev(out, (rows, ldo), BF16))
+    assert (got[M:] == 0).all() and (got[:, nb * N:] == 0).all()  # nothing beyond the matrix
+    got = got[:M, :nb * N].astype(np.float64).reshape(M, nb, N)
+    if f32_out:
+        assert rel(got, ref) < 2e-6
+    else:
+        assert (np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 1e-5).all()
+
+
+@pytest.mark.parametrize("design", ["ditilix", "pesivik"])
+def test_experts_on_128_row_tiles(design):
+    """prompts with 96 and more rows an expert: granules of 128 rows (an expert with few rows, tiles that end inside), weights ahead of the first
+    product (Ditilix) and rows gathered inside it (Pesivik); against the oracle, and against the same tokens in short portions"""
+    if design == "ditilix":
+        cfg = dict(architecture="Ditilix", width=128, vocab=90, residual_mult=0.5, logit_scale=1.0, norm=dict(eps=1e-5, groups=2), layers=[
+            dict(type="attention", mixer=mixer(heads=4, kv_heads=2, dim=24, vdim=16), mlp=moe(experts=3, top=2, ff=64, shared=(64, 1.0)))])
+        tensors = so.random_tensors(cfg, 3)
+        forward = so.forward
+    else:
+        from tests import pesivik_oracle as po
+        from vllm_rs_amd.stack_bench import pesivik_config
+        cfg = pesivik_config(128, 4, 32, 1, 90, 64, 64, 16, 300, 4, 2, 64, 64, 2, 2)
+        tensors = po.random_tensors(cfg, 3)
+        forward = po.forward
+    T = 260
+    toks = tokens_of(cfg, T, 8)
+    eng = build(cfg, tensors, BF16)
+    got = eng.replay_step([(1, toks, list(range(T)))], [1])
+    agree(got, forward(cfg, tensors, toks), BF16)
+    at, parts = 0, []
+    while at < T:
+        n = min(20, T - at)
+        parts.append(eng.replay_step([(2, toks[at:at + n], list(range(n)))], [2] if at + n == T else []))
+        at += n
+    agree(got, np.concatenate(parts), BF16)
+    eng.close()
+
+
 @pytest.mark.parametrize("dt", [F32, BF16])
 @pytest.mark.parametrize("F", [72, 11, 1000])
 def test_polynorm(dt, F):

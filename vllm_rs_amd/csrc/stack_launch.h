@@ -29,6 +29,7 @@ struct StkGemmArgs {
   const int* tile_group = nullptr;
   int granule = 0;
   const int* a_row = nullptr;
+  int a_rows = 0;  // rows of A behind a_row (0: unknown)
   const float* a_scale = nullptr;
   const int* out_row = nullptr;
   int epi = 0;
@@ -43,8 +44,11 @@ struct StkGemmArgs {
   int64_t bias_batch_stride = 0;  // elements between the bias rows of two products of a batch
 };
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream);
-// rows per granule the grouped launches of an M-row problem over `groups` groups want (16 or 64)
-int vra_stack_gemm_granule(int rows, int groups);
+// rows per granule the grouped launches of an M-row problem over `groups` groups want (16, 64, or 128 where `tiles128`: both products of the
+// expert are bf16 with K a multiple of 64)
+int vra_stack_gemm_granule(int rows, int groups, bool tiles128);
+// out[r] = round_bf16(a[row_token[r]] * row_scale[r]) for the rows that hold a pair (row_token >= 0); the others are left alone
+void vra_stack_scale_rows(const void* a, int W, const int* row_token, const float* row_scale, void* out, int rows, int64_t stream);
 
 // x[t, c] = embed[ids[t], c] + pe(positions[t], c),  pe(p, 2i) = sin(p * inv_freq[i]),  pe(p, 2i+1) = cos(p * inv_freq[i])  (f32);
 // inv_freq null: no position vector

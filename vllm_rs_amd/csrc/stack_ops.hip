@@ -8,7 +8,9 @@
 #include <math.h>
 
 #include <algorithm>
+#include <type_traits>
 
+#include "gemm_rows.cuh"
 #include "stack_common.cuh"
 #include "stack_launch.h"
 
@@ -155,6 +157,21 @@ __global__ __launch_bounds__(1024) void stk_moe_sort_kernel(const int* pair_expe
     row_token[r] = p / top;
     row_scale[r] = pair_weight[p];
     row_pair[r] = p;
+  }
+}
+
+// the rows of a mixture's first product, times their weights (bound: HBM, one read and one write of the pairs' rows): 1500 tokens, two experts
+// each, width 2048: 6 us; scaled inside the product, that took 192 us where an unscaled one of its size took 111
+__global__ __launch_bounds__(256) void stk_scale_rows_kernel(const uint16_t* a, int W, const int* row_token, const float* row_scale, uint16_t* out) {
+  const int r = blockIdx.x, t = row_token[r];
+  if (t < 0) return;
+  const float s = row_scale[r];
+  for (int c = threadIdx.x * 8; c < W; c += 256 * 8) {
+    float f[8];
+    unpack8<BF16>(*(const u32x4*)(a + (size_t)t * W + c), f);
+#pragma unroll
+    for (int e = 0; e < 8; e++) f[e] *= s;
+    *(u32x4*)(out + (size_t)r * W + c) = pack8<BF16>(f);
   }
 }
 
@@ -423,6 +440,88 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g)
     else ((uint16_t*)g.out)[ob + (int64_t)orow * g.ldo + n] = BF16::from_f32(v);
   }
 }
+
+// Epilogue of gemm_rows_kernel for these products: alpha, bias, FN, row scatter.  FN as a template parameter: with all functions in one epilogue
+// the kernel is 28 000 instructions long and a launch pays ~12 us for fetching what it jumps over (2048 x 2048 x 2048: 37 us, 24 so).
+// vec: rows of the output start on 16 bytes, a lane stores whole 16-byte pieces (bf16: after trading columns with its row's other
+// three lanes).
+enum StkFn { FN_NONE, FN_PAIR_CLAMPED, FN_PAIR_GELU, FN_PAIR_SILU, FN_GELU, FN_RELU2, FN_TANH, FN_EXPEXP, FN_SOFTCAP };
+template <int FN>
+struct StkRowsEpi {
+  void* out;
+  const int* out_row;
+  const float* bias;
+  int64_t out_batch_stride, bias_batch_stride;
+  float alpha, limit, act_alpha, softcap;
+  int ldo, out_f32, vec;
+  static constexpr bool pair = FN == FN_PAIR_CLAMPED || FN == FN_PAIR_GELU || FN == FN_PAIR_SILU;
+  __device__ __forceinline__ float fn(float v) const {
+    if (FN == FN_GELU) return gelu_erf_(v);
+    if (FN == FN_RELU2) return v > 0.f ? v * v : 0.f;
+    if (FN == FN_TANH) return tanhf(v);
+    if (FN == FN_EXPEXP) return expf(-expf(v));
+    if (FN == FN_SOFTCAP) return softcap * tanhf(v / softcap);
+    return v;
+  }
+  __device__ __forceinline__ void store(int m, int, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
+    constexpr int NJ = pair ? 2 : 4;  // blocks of 16 output columns
+    const int orow = m < 0 ? -1 : (out_row ? out_row[m] : m);
+    const int64_t ob = (int64_t)blockIdx.y * out_batch_stride + (int64_t)max(orow, 0) * ldo;
+    float* const of = (float*)out + ob;
+    uint16_t* const oh = (uint16_t*)out + ob;
+    const int no = pair ? n0 / 2 : n0, lim = pair ? N / 2 : N;
+    float y[NJ][4];
+    if constexpr (pair) {
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[j][e] = gated_pair(acc[2 * j][e], acc[2 * j + 1][e], limit, act_alpha, FN == FN_PAIR_GELU ? 1 : (FN == FN_PAIR_SILU ? 2 : 0));
+    } else {
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[j][e] = acc[j][e] * alpha + 0.f;  // (the sum of the form with a bias: -0 becomes 0)
+      if (bias) {
+        const float* const b = bias + (int64_t)blockIdx.y * bias_batch_stride;
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) y[j][e] = acc[j][e] * alpha + b[min(no + j * 16 + q4 * 4 + e, lim - 1)];
+      }
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[j][e] = fn(y[j][e]);
+    }
+    if (vec && !out_f32) {
+      u32x2 v[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; j++) v[j] = u32x2{BF16::pack2(y[j][0], y[j][1]), BF16::pack2(y[j][2], y[j][3])};
+      gr_gather_columns(v);
+#pragma unroll
+      for (int h = 0; h < NJ / 2; h++) {
+        const int n = no + q4 * (NJ * 4) + h * 8;
+        if (orow >= 0 && n < lim) *(u32x4*)(oh + n) = u32x4{v[2 * h][0], v[2 * h][1], v[2 * h + 1][0], v[2 * h + 1][1]};
+      }
+      return;
+    }
+    if (orow < 0) return;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+      const int n = no + j * 16 + q4 * 4;
+      if (vec && n + 4 <= lim) {
+        *(f32x4*)(of + n) = f32x4{y[j][0], y[j][1], y[j][2], y[j][3]};
+        continue;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (n + e < lim) {
+          if (out_f32) of[n + e] = y[j][e];
+          else oh[n + e] = BF16::from_f32(y[j][e]);
+        }
+    }
+  }
+};
 
 // ------------------------------------------------------------------------------------------------ activations
 template <typename T>
@@ -1150,18 +1249,39 @@ size_t vra_stack_diff_scratch(int max_len, int max_seqs, int heads, int vdim) { 
   return vra_stack_diff_splits(max_len, 1, heads) > 1 ? (size_t)STK_DIFF_PARTS * 2 * (vdim + 2) * sizeof(float) : 0;
 }
 
-int vra_stack_gemm_granule(int rows, int groups) { return groups > 0 && rows / groups >= 128 ? 64 : 16; }
+// (128-row tiles: a tile row costs the same however few of its rows hold pairs — from 96 rows an expert on they are full enough)
+int vra_stack_gemm_granule(int rows, int groups, bool tiles128) {
+  if (groups > 0 && tiles128 && rows / groups >= 96) return 128;
+  return groups > 0 && rows / groups >= 128 ? 64 : 16;
+}
+void vra_stack_scale_rows(const void* a, int W, const int* row_token, const float* row_scale, void* out, int rows, int64_t stream) {
+  VRA_CHECK_ARG(a && row_token && row_scale && out && rows > 0 && W > 0 && W % 8 == 0, "stack scale rows: null pointer or bad shape");
+  launch_checked("stack scale rows", [&] { stk_scale_rows_kernel<<<rows, 256, 0, as_stream(stream)>>>((const uint16_t*)a, W, row_token, row_scale, (uint16_t*)out); });
+}
+
+// Steps of more than 32 rows on gemm_rows_kernel: whole 64-steps of K, and operands whose byte offsets stay within 31 bits (a gathered
+// operand must say how many rows it has)
+static int rows_fn(const StkGemmArgs& g) {
+  if (g.epi == 1) return g.act == 1 ? FN_PAIR_GELU : (g.act == 2 ? FN_PAIR_SILU : FN_PAIR_CLAMPED);
+  if (g.epi == 2) return g.act == 3 ? FN_GELU : (g.act == 4 ? FN_RELU2 : (g.act == 5 ? FN_TANH : FN_EXPEXP));
+  return g.softcap > 0.f ? FN_SOFTCAP : FN_NONE;
+}
+static bool rows_kernel_takes(const StkGemmArgs& g) {
+  if (g.epi == 2 && g.softcap > 0.f) return false;  // (both at once: nobody asks for it)
+  const int64_t rows = g.a_row ? g.a_rows : g.M;
+  return g.K % 64 == 0 && rows > 0 && rows * g.lda * 2 < 0x7FFF0000ll && (int64_t)g.N * g.K * 2 < 0x7FFF0000ll && g.batch <= 65535;
+}
 
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
   VRA_CHECK_ARG(g.a && g.w && g.out && g.M > 0 && g.N > 0 && g.K > 0, "stack gemm: null pointer or empty shape");
   VRA_CHECK_ARG(dtype == VRA_BF16 || dtype == VRA_F32, "stack gemm: dtype must be bf16 or f32");
-  VRA_CHECK_ARG(!g.tile_group || g.granule == 16 || g.granule == 64, "stack gemm: granule must be 16 or 64");
+  VRA_CHECK_ARG(!g.tile_group || g.granule == 16 || g.granule == 64 || g.granule == 128, "stack gemm: granule must be 16, 64 or 128");
   VRA_CHECK_ARG(g.batch >= 1 && (g.batch == 1 || !g.tile_group), "stack gemm: a batched product has no row groups");
   hipStream_t st = as_stream(stream);
   const int nb = g.batch;
   // (few columns over a long K, the first stage of a low-rank projection: the 64-row tiles would leave most of the chip idle)
   const bool narrow = dtype == VRA_BF16 && !g.tile_group && !g.a_scale && nb == 1 && g.N <= 128 && g.K >= 1024 && g.M <= 8192;
-  const bool big = g.tile_group ? g.granule == 64 : g.M > 32 && !narrow;
+  const bool big = g.tile_group ? g.granule >= 64 : g.M > 32 && !narrow;
   const bool mfma = dtype == VRA_BF16 && g.K % 8 == 0 && g.lda % 8 == 0 && ((uintptr_t)g.a % 16 == 0) && ((uintptr_t)g.w % 16 == 0) &&
                     (g.w_group_stride % 8 == 0) && (g.a_batch_stride % 8 == 0) && (g.w_batch_stride % 8 == 0);
   VRA_CHECK_ARG(g.epi >= 0 && g.epi <= 2 && (g.epi != 2 || (g.act >= 3 && g.act <= 6)) && (g.softcap <= 0.f || g.epi != 1), "stack gemm: unknown epilogue");
@@ -1169,13 +1289,32 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
   VRA_CHECK_ARG(!post || !g.a_scale, "stack gemm: scaled rows and an element-wise epilogue do not come together");
   VRA_CHECK_ARG(g.epi != 1 || (mfma && g.N % 32 == 0), "stack gemm: the gated epilogue needs the bf16 MFMA path and whole gate / up blocks");
   if (mfma) {
-    if (big && !g.tile_group && !g.a_scale && g.M >= 256 && (int64_t)((g.M + 127) / 128) * ((g.N + 127) / 128) * nb >= 256) {
-      // enough 128 x 128 tiles to fill the chip: a wave owns 64 x 64 (16 MFMAs per 8 fragment requests instead of 8 per 6)
-      dim3 grid((g.M + 127) / 128, (g.N + 127) / 128, nb);
-      if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<4, 4, 2, 2, false, true><<<grid, 256, 0, st>>>(g); });
-      else launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<4, 4, 2, 2, false><<<grid, 256, 0, st>>>(g); });
+    if (big && !g.a_scale && rows_kernel_takes(g)) {
+      GemmRowsArgs r;
+      r.x = g.a, r.x_ld = g.lda, r.x_row = g.a_row, r.w[0] = g.w, r.n[0] = g.N, r.M = g.M, r.K = g.K;
+      r.tile_group = g.tile_group, r.w_group_stride = g.w_group_stride, r.x_batch_stride = g.a_batch_stride, r.w_batch_stride = g.w_batch_stride;
+      int tile = gemm_rows_tile(g.M, r.n, 1, nb);
+      if (g.tile_group) tile = g.granule == 64 ? 16 + 2 : (tile == 16 + 2 ? 32 + 2 : tile);  // (a tile row is one granule)
+      auto go = [&](auto fn) {
+        const int per = g.out_f32 ? 4 : 8;  // elements of 16 bytes
+        const bool vec = (uintptr_t)g.out % 16 == 0 && g.ldo % per == 0 && g.out_batch_stride % per == 0 && (g.out_f32 || (g.epi == 1 ? g.N % 32 : g.N % 8) == 0);
+        StkRowsEpi<decltype(fn)::value> e{g.out, g.out_row, g.bias, g.out_batch_stride, g.bias_batch_stride, g.alpha, g.limit, g.act_alpha, g.softcap, g.ldo, g.out_f32, vec ? 1 : 0};
+        launch_checked("stack gemm", [&] { gemm_rows_launch<BF16, false>(r, e, tile, nb, st); });
+      };
+      switch (rows_fn(g)) {
+        case FN_PAIR_CLAMPED: go(std::integral_constant<int, FN_PAIR_CLAMPED>{}); break;
+        case FN_PAIR_GELU: go(std::integral_constant<int, FN_PAIR_GELU>{}); break;
+        case FN_PAIR_SILU: go(std::integral_constant<int, FN_PAIR_SILU>{}); break;
+        case FN_GELU: go(std::integral_constant<int, FN_GELU>{}); break;
+        case FN_RELU2: go(std::integral_constant<int, FN_RELU2>{}); break;
+        case FN_TANH: go(std::integral_constant<int, FN_TANH>{}); break;
+        case FN_EXPEXP: go(std::integral_constant<int, FN_EXPEXP>{}); break;
+        case FN_SOFTCAP: go(std::integral_constant<int, FN_SOFTCAP>{}); break;
+        default: go(std::integral_constant<int, FN_NONE>{}); break;
+      }
     } else if (big) {
       dim3 grid((g.M + 63) / 64, (g.N + 127) / 128, nb);
+      VRA_CHECK_ARG(!g.tile_group || g.granule == 64, "stack gemm: granules of 128 rows need an unscaled product with K a multiple of 64 and a known row count");
       if (g.a_scale) launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<2, 4, 2, 2, true><<<grid, 256, 0, st>>>(g); });
       else if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<2, 4, 2, 2, false, true><<<grid, 256, 0, st>>>(g); });
       else launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<2, 4, 2, 2, false><<<grid, 256, 0, st>>>(g); });
@@ -1187,6 +1326,7 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
     }
     return;
   }
+  VRA_CHECK_ARG(!g.tile_group || g.granule != 128, "stack gemm: granules of 128 rows are for bf16 products on the matrix cores");
   if (big) {
     dim3 grid((g.M + 63) / 64, (g.N + 63) / 64, nb);
     if (dtype == VRA_F32) launch_checked("stack gemm", [&] { stk_gemm_simple_kernel<float, 4><<<grid, 256, 0, st>>>(g); });
@@ -1220,7 +1360,7 @@ void vra_stack_group_norm(const StkNormArgs& a, int dtype, int64_t stream) {
 void vra_stack_moe_sort(const int* pair_expert, const float* pair_weight, int P, int top, int n_groups, int granule, int max_rows, int* row_token,
                         float* row_scale, int* row_pair, int* tile_group, int64_t stream) {
   VRA_CHECK_ARG(pair_expert && pair_weight && row_token && row_scale && row_pair && tile_group && P > 0 && top > 0, "stack moe sort: null pointer");
-  VRA_CHECK_ARG((granule == 16 || granule == 64) && max_rows % granule == 0 && max_rows >= P + n_groups * (granule - 1), "stack moe sort: row space too small");
+  VRA_CHECK_ARG((granule == 16 || granule == 64 || granule == 128) && max_rows % granule == 0 && max_rows >= P + n_groups * (granule - 1), "stack moe sort: row space too small");
   const size_t lds = (size_t)n_groups * 3 * sizeof(int);
   VRA_CHECK_ARG(lds <= 48 * 1024, "stack moe sort: too many experts");
   launch_checked("stack moe sort", [&] {
@@ -1371,6 +1511,7 @@ extern "C" void vra_stack_op_group_norm(const float* x, const float* w, void* h,
 extern "C" void vra_stack_op_gemm(const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32, int32_t M,
                                   int32_t N, int32_t K, float alpha, const int32_t* tile_group, int32_t granule, const int32_t* a_row,
                                   const float* a_scale, const int32_t* out_row, int32_t epi, float limit, int32_t dtype, int64_t stream) {
+  VRA_CHECK_ARG(!tile_group || granule == 16 || granule == 64, "stack gemm: granule must be 16 or 64");
   StkGemmArgs g;
   g.a = a, g.lda = lda, g.w = w, g.w_group_stride = w_group_stride, g.out = out, g.ldo = ldo, g.out_f32 = out_f32, g.M = M, g.N = N, g.K = K;
   g.alpha = alpha, g.tile_group = tile_group, g.granule = granule, g.a_row = a_row, g.a_scale = a_scale, g.out_row = out_row, g.epi = epi, g.limit = limit;
@@ -1378,6 +1519,7 @@ extern "C" void vra_stack_op_gemm(const void* a, int32_t lda, const void* w, int
 }
 extern "C" void vra_stack_op_moe_sort(const int32_t* pair_expert, const float* pair_weight, int32_t P, int32_t top, int32_t n_groups, int32_t granule,
                                       int32_t max_rows, int32_t* row_token, float* row_scale, int32_t* row_pair, int32_t* tile_group, int64_t stream) {
+  VRA_CHECK_ARG(granule == 16 || granule == 64, "stack moe sort: granule must be 16 or 64");
   vra_stack_moe_sort(pair_expert, pair_weight, P, top, n_groups, granule, max_rows, row_token, row_scale, row_pair, tile_group, stream);
 }
 extern "C" void vra_stack_op_gated_act(const float* gu, void* out, int32_t M, int32_t F, float limit, float act_alpha, int32_t dtype, int64_t stream) {
@@ -1408,6 +1550,7 @@ extern "C" void vra_stack_op_attention(const void* q, int32_t ldq, void* out, co
 extern "C" void vra_stack_op_gemm_post(const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32, int32_t M,
                                        int32_t N, int32_t K, float alpha, const float* bias, const int32_t* tile_group, int32_t granule, const int32_t* a_row,
                                        const int32_t* out_row, int32_t epi, int32_t act, float softcap, int32_t dtype, int64_t stream) {
+  VRA_CHECK_ARG(!tile_group || granule == 16 || granule == 64, "stack gemm: granule must be 16 or 64");
   StkGemmArgs g;
   g.a = a, g.lda = lda, g.w = w, g.w_group_stride = w_group_stride, g.out = out, g.ldo = ldo, g.out_f32 = out_f32, g.M = M, g.N = N, g.K = K;
   g.alpha = alpha, g.bias = bias, g.tile_group = tile_group, g.granule = granule, g.a_row = a_row, g.out_row = out_row, g.epi = epi, g.act = act;

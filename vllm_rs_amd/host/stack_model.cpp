@@ -1011,12 +1011,13 @@ bool StackModel::init_buffers(int max_tokens, int max_seqs) {
       roc = std::max(roc, sh * sv);
     }
   }
-  max_rows_ = (int)round_up((int)(T * std::max<size_t>(top, 1) + experts * 63), 64);
+  max_rows_ = (int)round_up((int)(T * std::max<size_t>(top, 1) + experts * 127), 128);
   for (const StackLayer& L : layers_) {
     if (L.mlp == 1) zc = std::max(zc, T * L.ff), actc = std::max(actc, T * L.ff);
     if (L.mlp == 2 && L.n_identity > 0) experts = std::max(experts, (size_t)L.experts);
     if (L.mlp == 2) {
       zc = std::max(zc, std::max((size_t)max_rows_ * 2 * L.ffp, T * 2 * L.sffp));
+      if (L.router_kind == 0) zc = std::max(zc, (size_t)max_rows_ * W * es_ / 4);  // (expert_pair's scaled rows)
       actc = std::max(actc, std::max((size_t)max_rows_ * L.ffp, T * L.sffp));
     }
   }
@@ -1070,6 +1071,12 @@ static bool take_stack_err(std::string& error, const char* where) {
   return false;
 }
 
+// both products of an expert run on the 128-row tiles of the row-major prompt GEMM
+bool StackModel::tiles128(const StackLayer& L) const {
+  const int64_t most = 0x7FFF0000ll;
+  return dt_ == VRA_BF16 && width_ % 64 == 0 && L.ffp % 64 == 0 && (int64_t)max_rows_ * std::max(width_, L.ffp) * 2 < most &&
+         (int64_t)2 * L.ffp * width_ * 2 < most;
+}
 // gate / up -> clamped gated activation -> down for `rows` logical rows (one expert per granule, or one weight set for all):
 // bf16: the activation is the epilogue of the gate / up launch; f32: product, activation and product as three launches
 bool StackModel::expert_pair(const void* a, int lda, const void* w_gu, int64_t gu_stride, const void* w_down, int64_t down_stride, int rows, int fp,
@@ -1077,6 +1084,11 @@ bool StackModel::expert_pair(const void* a, int lda, const void* w_gu, int64_t g
                              float* out, int64_t stream, int act) {
   const int W = width_;
   StkGemmArgs g;
+  if (granule == 128 && a_scale) {  // (the 128-row tiles take their rows as they are)
+    vra_stack_scale_rows(a, W, a_row, a_scale, z_, rows, stream);  // (z_: the f32 products of the unfused form, unused here)
+    a = z_, lda = W, a_row = nullptr, a_scale = nullptr;
+  }
+  g.a_rows = max_tokens_;
   g.a = a, g.lda = lda, g.w = w_gu, g.w_group_stride = gu_stride, g.M = rows, g.N = (act >= 3 ? 1 : 2) * fp, g.K = W;
   g.tile_group = tile_group, g.granule = granule, g.a_row = a_row, g.a_scale = a_scale;
   g.limit = limit, g.act = act;
@@ -1116,7 +1128,7 @@ bool StackModel::feed_forward(const StackLayer& L, int T, int64_t stream) {
   }
   if (L.mlp == 2) {
     const int P = T * L.top;
-    const int granule = vra_stack_gemm_granule(P, L.experts);
+    const int granule = vra_stack_gemm_granule(P, L.experts, tiles128(L));
     const int rows = round_up(P + L.experts * (granule - 1), granule);
     if (rows > max_rows_) return error = "feed-forward: more expert rows than the buffers hold", false;
     vra_stack_moe_sort(pair_expert_, pair_weight_, P, L.top, L.experts, granule, rows, row_token_, row_scale_, row_pair_, tile_group_, stream);
@@ -1505,7 +1517,7 @@ bool StackModel::forward_sandwich(const InputMetadata& md, int64_t stream) {
     if (L.mlp == 2) {
       if (!seam(L.norm2_w, L.norm2_b, L.norm2_alpha, &L, true)) return false;
       const int P = T * L.top;
-      const int granule = vra_stack_gemm_granule(P, L.experts);
+      const int granule = vra_stack_gemm_granule(P, L.experts, tiles128(L));
       const int rows = round_up(P + L.experts * (granule - 1), granule);
       if (rows > max_rows_) return error = "feed-forward: more expert rows than the buffers hold", false;
       vra_stack_moe_sort(pair_expert_, pair_weight_, P, L.top, L.experts, granule, rows, row_token_, row_scale_, row_pair_, tile_group_, stream);
