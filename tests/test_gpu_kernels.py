@@ -262,6 +262,27 @@ def test_dense_gemm(M, out_f32):
         assert_close_dt(out.numpy(np.uint16, (M, N)), ref, BF16, name="dense", abs_floor=2e-3)
 
 
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("M,K,N", [(33, 128, 16), (64, 256, 272), (129, 128, 1040), (200, 384, 128), (257, 128, 4112)])
+@pytest.mark.parametrize("with_bias,out_f32", [(False, False), (True, False), (True, True)])
+def test_dense_gemm_prompt_rows(M, K, N, dt, with_bias, out_f32):
+    """unquantised products of prompt steps (gemm_rows.cuh): tile edges in M and N, 16-byte pieces at the last columns"""
+    r = rng(M + N)
+    x, w = rand_dt(r, (M, K), dt), rand_dt(r, (N, K), dt, 0.05)
+    bias = rand_dt(r, (N,), dt, 0.2) if with_bias else None
+    od = F32 if out_f32 else dt
+    out = ops.dense_gemm(ops.dev(x), ops.dev(w), ops.dev(bias) if with_bias else None, M, K, N, dt, od)
+    ref = orc.dense_gemm(x, w, bias, dt, od)
+    g0 = np.abs(orc.dense_gemm(x, w, None, dt, F32)) if with_bias else None  # (the sum is rounded before the bias is added)
+    if out_f32:
+        got = out.numpy(np.float32, (M, N))
+        assert np.abs(got - ref).max() <= (2.0 ** -7 if dt == BF16 else 2.0 ** -10) * max(1.0, float(np.abs(ref).max()))
+    else:
+        # near zero an ulp is finer than f32 sums of different order agree: K roundings of partial sums (|.| < 4) at 2^-24 each
+        # (with a bias two roundings, of the product and of the sum, may each fall the other way: 2 ulp)
+        assert_close_dt(out.numpy(np.uint16, (M, N)), ref, dt, max_ulp=2.0 if with_bias else 1.0, name="dense prompt gemm", mag=g0, abs_floor=K * 4 * 2.0 ** -24)
+
+
 @pytest.mark.parametrize("M", [8, 9, 16, 17, 32])
 @pytest.mark.parametrize("K,N,dt,with_bias", [(4096, 4112, BF16, False), (2048, 8192, BF16, True), (3584, 4096, F16, False), (1024, 2064, F16, True)])
 def test_dense_gemm_decode_batches(M, K, N, dt, with_bias):

@@ -61,9 +61,9 @@ static inline size_t gemm_rows_lds_bytes(int wm, int wn, int s) { return (size_t
 
 // EPI::store(m, seg, n0, q4, acc): the wave's 64 columns n0 .. n0 + 63 (of segment seg) of output row m; the lane holds columns n0 + 16 j + 4 q4 ..
 // + 3 in acc[j].  Called by all lanes (lanes beyond the matrix with m = -1), so that a lane may trade columns with its row's other three.
-// PAIR: w[0] and w[1] (gate, up) interleaved in blocks of 16 virtual columns, n[0] = virtual columns.
+// PAIR: w[0] and w[1] (gate, up; neither grouped nor batched) interleaved in blocks of 16 virtual columns, n[0] = virtual columns.
 template <class DT, int WM, int WN, int S, bool SPREAD, bool PAIR, class EPI>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const GemmRowsArgs a, const EPI epi) {
+__global__ __launch_bounds__(64 * WM * WN + (SPREAD ? 0 : 64)) void gemm_rows_kernel(const GemmRowsArgs a, const EPI epi) {
 #ifdef __HIP_DEVICE_COMPILE__
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int NW = WM * WN, XB = 4 * WM, NB = 4 * (WM + WN), PER = NB / NW, D = 2 * PER, STG = NB * 2048, PEND = (S - 3) * D;
@@ -125,6 +125,47 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const GemmRowsA
         }
         vo[i][h] = ((uint32_t)row * ld + (uint32_t)sc * 8u) * 2u;
       }
+  }
+  if constexpr (!SPREAD) {
+    // One wave more, which computes nothing: it touches a line of K step ks + 8 for its share of the panels that the workgroups of an XCD
+    // have in common (8 tile rows x 4 tile columns at a time: a quarter of this tile's rows of x, an eighth of its columns of w), so that
+    // the ring's requests find them in L2.  With two stages in flight the ring alone does not cover the way to memory (2048 x 8192, K =
+    // 2048, weights not in any cache: 94 -> 82 us); the 128 x 128 tile's three stages do, and gain nothing.
+    if (wave == NW) {
+      constexpr int XL = 16 * WM, WL = 8 * WN;
+      static_assert(XL + WL <= 64, "a lane a line");
+      const bool isx = lane < XL;
+      const int xr = min(m0 + (nt & 3) * XL + lane, a.M - 1), wrow = (mt & 7) * WL + (lane - XL);
+      int nr = min(n0 + wrow, N - 1);
+      const uint16_t* wp = w;
+      if (PAIR) {  // (this wave's w is the gate tensor's)
+        const uint16_t* const up = static_cast<const uint16_t*>(a.w[1]);
+        nr = min((n0 >> 1) + (wrow >> 1), (N >> 1) - 1);
+        if (wrow & 1) wp = up;
+      }
+      const int xi = isx && a.x_row ? max(a.x_row[xr], 0) : xr;
+      const uint16_t* const p = isx ? x + (int64_t)xi * a.x_ld : wp + (int64_t)nr * K;
+      const bool live = lane < XL + WL;
+      uint32_t v[8] = {}, seen = 0;
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (live) v[u] = *reinterpret_cast<const uint32_t*>(p + min(u, KT - 1) * 64);
+      __builtin_amdgcn_s_barrier();
+      for (int ks = 0; ks < KT; ks += 8) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          if (ks + u >= KT) break;  // (one barrier a step, as the other waves)
+          seen ^= v[u];
+          if (live) v[u] = *reinterpret_cast<const uint32_t*>(p + min(ks + u + 8, KT - 1) * 64);
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_barrier();
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++) seen ^= v[u];
+      asm volatile("" ::"v"(seen));
+      return;
+    }
   }
   typedef __attribute__((address_space(3))) void* lds_ptr;
   auto request = [&](int ks, int e) {  // the e-th of the wave's D instructions for stage ks (beyond K: the last step again, never read)
@@ -199,9 +240,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_rows_kernel(const GemmRowsA
 }
 
 // Tile for a product of M rows x ncols[0..nseg) columns x `batch`: workgroups run in rounds of one per CU, a round of a tile takes (us per 64
-// of K, measured with all CUs at work) 0.50 at 64 x 128, 0.58 at 128 x 128, 1.10 at 128 x 256.  -> WM * 16 + WN
-static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch) {
-  const struct { int wm, wn; double us; } t[3] = {{2, 4, 1.10}, {2, 2, 0.58}, {1, 2, 0.50}};
+// of K, measured with all CUs at work) 0.55 at 64 x 128, 0.62 at 128 x 128, 1.10 at 128 x 256.  -> WM * 16 + WN; *us: the time per 64 of K
+static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch, double* us = nullptr) {
+  const struct { int wm, wn; double us; } t[3] = {{2, 4, 1.10}, {2, 2, 0.62}, {1, 2, 0.55}};
   int best = 0;
   double cost = 0.0;
   for (const auto& c : t) {
@@ -211,6 +252,7 @@ static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch)
     const double v = (double)((tiles + 255) / 256) * c.us;
     if (!best || v < cost) best = c.wm * 16 + c.wn, cost = v;
   }
+  if (us) *us = cost;
   return best;
 }
 // fills the tile counts and launches
@@ -228,7 +270,7 @@ static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStr
     attr_devs |= (uint64_t)1 << (dev & 63);
   }
   gemm_rows_kernel<DT, WM, WN, S, SPREAD, PAIR, EPI>
-      <<<dim3((unsigned)(a.MT * a.NT), (unsigned)batch), dim3(64 * WM * WN), gemm_rows_lds_bytes(WM, WN, S), st>>>(a, epi);
+      <<<dim3((unsigned)(a.MT * a.NT), (unsigned)batch), dim3(64 * WM * WN + (SPREAD ? 0 : 64)), gemm_rows_lds_bytes(WM, WN, S), st>>>(a, epi);
 }
 template <class DT, bool PAIR, class EPI>
 static void gemm_rows_launch(const GemmRowsArgs& a, const EPI& epi, int tile, int batch, hipStream_t st) {

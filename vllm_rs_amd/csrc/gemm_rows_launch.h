@@ -1,0 +1,30 @@
+// gemm_rows_launch.h — the row-major prompt GEMM (gemm_rows.cuh) as the C entry points and the native runtime call it.
+#pragma once
+#include <type_traits>
+
+#include "gemm_rows.cuh"
+
+struct GemmRowsOut {
+  void* out;
+  const void* bias;
+  int ld;
+};
+struct GemmRowsCall {
+  const void* x = nullptr;
+  int x_ld = 0, M = 0, K = 0;
+  int nseg = 1;
+  const void* w[GR_MAX_SEG] = {};  // dual: gate, up
+  int n[GR_MAX_SEG] = {};
+  const void* bias[GR_MAX_SEG] = {};
+  void* out[GR_MAX_SEG] = {};  // dual: out[0] = silu(gate) * up
+  int out_ld[GR_MAX_SEG] = {};
+  const void* residual = nullptr;  // added to segment 0
+  int res_ld = 0;
+  int out_f32 = 0;
+  bool dual = false;
+};
+// whether the product can run here and is expected to be faster than on kernel B (and behind it the element-wise launches the fused form
+// saves).  Measured, bf16, cold weights, us (here / kernel B): 64 rows, 2048 x 5632: 50 / 22; 128 rows, 5632 x 2048: 24 / 34; 256 rows, 4096 x 4096:
+// 40 / 39; 400 rows, 14336 x 4096: 80 / 234; 2120 rows, 2048 x 5632: 95 / 219
+bool vra_gemm_rows_fits(const GemmRowsCall& c);
+void vra_launch_gemm_rows(const GemmRowsCall& c, int dtype, int64_t stream);

@@ -120,6 +120,7 @@ extern "C" void vra_wna16_dequant(const void* qweight_tiled, const void* scales,
 // launch helpers (shared with the native runtime through gemm_launch.h)
 // ------------------------------------------------------------------------------------------------
 #include "gemm_launch.h"
+#include "gemm_rows_launch.h"
 #include "gemm_dense_launch.h"
 
 static const int kMaxDynLds = 160 * 1024;
@@ -1288,6 +1289,12 @@ extern "C" void vra_dense_gemm(const void* x, const void* w, const void* bias, v
     a.M = m, a.K = k, a.n_units = n / 16;
     vra_launch_gemv_dw(a, dtype, stream);
   } else {
+    GemmRowsCall r;
+    r.x = x, r.x_ld = k, r.M = m, r.K = k, r.w[0] = w, r.n[0] = n, r.bias[0] = bias, r.out[0] = out, r.out_ld[0] = n, r.out_f32 = out_dtype == VRA_F32;
+    if (vra_gemm_rows_fits(r)) {
+      vra_launch_gemm_rows(r, dtype, stream);
+      return;
+    }
     GemmBArgs b = {};
     b.w0 = w;
     b.bias0 = bias;

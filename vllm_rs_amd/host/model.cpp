@@ -10,6 +10,7 @@
 #include "../csrc/attn_launch.h"
 #include "../csrc/gemm_dense_launch.h"
 #include "../csrc/gemm_launch.h"
+#include "../csrc/gemm_rows_launch.h"
 #include "../csrc/scratch.h"
 #include "host_utils.h"
 
@@ -634,8 +635,15 @@ bool Model::linear(const QLinear& l0, const void* x, void* out, int M, const voi
       a.group_size = -1;
       vra_launch_gemv(a, false, dt_, stream);
     } else {
-      vra_dense_gemm(x, l.w, l.bias, tmp_, M, l.K, l.N, dt_, dt_, stream);
-      vra_add(tmp_, residual, out, (int64_t)M * l.N, dt_, stream);
+      GemmRowsCall r;  // prompts: the residual in the product's epilogue
+      r.x = x, r.x_ld = l.K, r.M = M, r.K = l.K, r.w[0] = l.w, r.n[0] = l.N, r.bias[0] = l.bias, r.out[0] = out, r.out_ld[0] = l.N;
+      r.residual = residual, r.res_ld = l.N;
+      if (vra_gemm_rows_fits(r)) {
+        vra_launch_gemm_rows(r, dt_, stream);
+      } else {
+        vra_dense_gemm(x, l.w, l.bias, tmp_, M, l.K, l.N, dt_, dt_, stream);
+        vra_add(tmp_, residual, out, (int64_t)M * l.N, dt_, stream);
+      }
     }
   }
   return !take_err(error, "linear");
@@ -666,6 +674,19 @@ bool Model::linear_fused_norm(const QLinear* ls, int nl, void* const* outs, cons
     a.scales_layout = VRA_SCALES_ROWMAJOR;
     vra_launch_gemv(a, ls[0].quant, dt_, stream);
     return !take_err(error, "fused norm gemv");
+  }
+  // unquantised prompts: all projections in one launch behind the norm
+  bool dense = !ls[0].quant && nl <= GR_MAX_SEG;
+  for (int i = 1; i < nl; i++) dense = dense && !ls[i].quant && ls[i].K == K;
+  if (dense) {
+    GemmRowsCall r;
+    r.x = xn_, r.x_ld = K, r.M = M, r.K = K, r.nseg = nl;
+    for (int i = 0; i < nl; i++) r.w[i] = ls[i].w, r.n[i] = ls[i].N, r.bias[i] = ls[i].bias, r.out[i] = outs[i], r.out_ld[i] = ls[i].N;
+    if (vra_gemm_rows_fits(r)) {
+      vra_rms_norm(x, norm_w, xn_, M, K, mc_.rms_norm_eps, dt_, stream);
+      vra_launch_gemm_rows(r, dt_, stream);
+      return !take_err(error, "norm + gemm_rows (segments)");
+    }
   }
   bool same = ls[0].quant && nl <= GEMV_MAX_SEG;
   for (int i = 1; i < nl; i++) same = same && ls[i].quant && ls[i].K == K && ls[i].awq == ls[0].awq;
@@ -831,6 +852,16 @@ bool Model::gate_up(const LayerWeights& L, const void* x, const void* norm_w, vo
     a.M = M, a.K = K, a.group_size = -1;
     vra_launch_gemv(a, false, dt_, stream);
     return !take_err(error, "gate_up dense pair");
+  }
+  if (!L.up.quant && L.gate.K == L.up.K && L.gate.N == L.up.N) {  // prompts: both projections and SiLU * mul in one launch
+    GemmRowsCall r;
+    r.x = xn_, r.x_ld = K, r.M = M, r.K = K, r.nseg = 2, r.dual = true;
+    r.w[0] = L.gate.w, r.w[1] = L.up.w, r.n[0] = r.n[1] = N, r.bias[0] = L.gate.bias, r.bias[1] = L.up.bias, r.out[0] = act, r.out_ld[0] = N;
+    if (vra_gemm_rows_fits(r)) {
+      vra_rms_norm(x, norm_w, xn_, M, K, mc_.rms_norm_eps, dt_, stream);
+      vra_launch_gemm_rows(r, dt_, stream);
+      return !take_err(error, "gate_up (gemm_rows)");
+    }
   }
   const QLinear ls[2] = {L.gate, L.up};
   void* outs[2] = {gate_, up_};
