@@ -432,6 +432,63 @@ def test_attention_random(dt, decode, H, G, dim, vdim):
     assert rel(got, ref) < (2e-6 if dt == F32 else 4e-3)
 
 
+# the tile kernel of prompt steps (csrc/stack_prompt_attn.hip: pages of whole 64-key tiles, heads of 64 / 128 channels) against float64 and against the
+# general kernel, which the same call with 32-token pages takes.  bf16: the output's rounding, 2^-9 of a value, and a weight's tail at 2^-17
+@pytest.mark.parametrize("H,G,dim,vdim", [(2, 2, 64, 64), (6, 2, 64, 128), (16, 4, 128, 128), (3, 1, 128, 64)])
+@pytest.mark.parametrize("form", ["causal", "cap", "temperature", "window", "chunk", "sink-scale-gate"])
+@pytest.mark.parametrize("first,Tq,BS", [(0, 1, 64), (0, 64, 64), (63, 66, 64), (130, 61, 128), (0, 333, 64)])
+def test_prompt_attention_tiles(H, G, dim, vdim, form, first, Tq, BS):
+    L = _lib.load()
+    r = np.random.default_rng(H + dim + vdim + first + Tq)
+    Tk = first + Tq
+    k = so.bf16_round(r.standard_normal((Tk, G, dim)).astype(np.float32))
+    v = so.bf16_round(r.standard_normal((Tk, G, vdim)).astype(np.float32))
+    q = so.bf16_round((2.0 * r.standard_normal((Tq, H, dim))).astype(np.float32))
+    p = np.arange(first, Tk)
+    scale, cap = dim ** -0.5, 5.0 if form == "cap" else 0.0
+    sink, hs = r.standard_normal(H).astype(np.float32), r.uniform(0.5, 1.5, H).astype(np.float32)
+    gate = r.standard_normal((Tq, H)).astype(np.float32)
+    every = 7 if form == "temperature" else 0
+    window, chunk = (40 if form == "window" else 0), (48 if form == "chunk" else 0)
+    lo = np.maximum(p - window + 1, 0) if window else (p // chunk * chunk if chunk else np.zeros_like(p))
+    sx = form == "sink-scale-gate"
+    ref = np.zeros((Tq, H, vdim))
+    for h in range(H):
+        g = h // (H // G)
+        s = (q[:, h].astype(np.float64) @ k[:, g].astype(np.float64).T) * scale
+        if every:
+            s *= so.query_temperature(p.astype(np.float64), 0.3, every)[:, None]
+        if sx:
+            s *= hs[h]
+        if cap:
+            s = cap * np.tanh(s / cap)
+        j = np.arange(Tk)
+        s = np.where((j[None] <= p[:, None]) & (j[None] >= lo[:, None]), s, -np.inf)
+        top = np.maximum(s.max(-1, keepdims=True), sink[h] if sx else -np.inf)
+        e = np.exp(s - top)
+        ref[:, h] = (e / (e.sum(-1, keepdims=True) + (np.exp(sink[h] - top) if sx else 0.0))) @ v[:, g].astype(np.float64)
+        if sx:
+            ref[:, h] *= so.sigmoid(gate[:, h].astype(np.float64))[:, None]
+
+    def run(page):
+        kc, vc, table = paged(k, v, page, r, BF16)
+        out = empty(Tq * H * vdim * 2)
+        args = (to_dev(q.reshape(Tq, -1), BF16).ptr, H * dim, out.ptr, kc.ptr, vc.ptr, raw(p, np.int64).ptr, raw(table, np.uint32).ptr, raw([Tk], np.uint32).ptr,
+                raw([0, Tq], np.uint32).ptr, 1, Tq, Tq, H, G, dim, vdim, page, len(table), scale)
+        if sx or window:
+            f = lambda a: raw(a, np.float32).ptr if sx else None
+            L.vra_stack_op_attention_window(*args, window, f(sink), f(hs), f(gate), H, BF16, 0)
+        elif chunk:
+            L.vra_stack_op_attention_chunk(*args, chunk, BF16, 0)
+        else:
+            L.vra_stack_op_attention(*args, cap, 0.3 if every else 0.0, every, BF16, 0)
+        check()
+        return from_dev(out, (Tq, H, vdim), BF16)
+    got, general = run(BS), run(32)
+    assert rel(got, ref) < 3e-3 and rel(general, ref) < 3e-3
+    assert np.abs(got - general).max() <= 2.0 ** -7 * np.abs(ref).max()  # (one rounding apart where their f32 sums fall on either side)
+
+
 @pytest.mark.parametrize("dt", [F32, BF16])
 @pytest.mark.parametrize("decode", [False, True])
 @pytest.mark.parametrize("softcap,temp", [(0.0, None), (20.0, dict(coef=0.3, every=64))])

@@ -141,6 +141,8 @@ size_t vra_stack_diff_scratch(int max_len, int max_seqs, int heads, int vdim);
 int vra_stack_latent_splits(int window, int max_len, int max_seqs, int heads, int vdim);
 bool vra_stack_latent_decode(const StkAttnArgs& a, int dtype, int64_t stream);
 bool vra_stack_latent_prefill(const StkAttnArgs& a, int dtype, int64_t stream);
+// prompt steps with 64- or 128-channel heads (stack_prompt_attn.hip); false: not a shape of that kernel, nothing was launched
+bool vra_stack_prompt_attention(const StkAttnArgs& a, int dtype, int64_t stream);
 
 // rows of a [*, W] f32 matrix picked by index -> dst (f32)
 void vra_stack_gather_rows_f32(const float* src, const uint32_t* rows, float* dst, int n, int W, int64_t stream);
