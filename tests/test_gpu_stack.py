@@ -361,6 +361,33 @@ def test_polynorm(dt, F):
     assert rel(from_dev(out, (M, F), dt), so.polynorm(z.astype(np.float64), coef, 1e-5)) < (2e-6 if dt == F32 else 4e-3)
 
 
+# rows whose sizes end at, just before and beyond what a thread keeps in registers, by fours and one by one; as test_group_norm / test_polynorm
+@pytest.mark.parametrize("dt", [F32, BF16])
+@pytest.mark.parametrize("W,groups", [(2048, 4), (2052, 1), (2051, 1), (4100, 5), (8192, 8), (6, 3)])
+def test_group_norm_row_sizes(dt, W, groups):
+    test_group_norm(dt, W, groups)
+
+
+@pytest.mark.parametrize("dt", [F32, BF16])
+@pytest.mark.parametrize("F", [4, 8192, 8196, 8195, 12300])
+def test_polynorm_row_sizes(dt, F):
+    test_polynorm(dt, F)
+
+
+# few rows: 16 columns a workgroup below 256 workgroups, 32 from there on; both sides of the line, and K that gives some waves nothing
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (5, 40, 72), (16, 8160, 64), (16, 8192, 64), (17, 4064, 328), (32, 4096, 256), (3, 2000, 2048)])
+def test_gemm_few_rows(M, N, K):
+    L = _lib.load()
+    r = np.random.default_rng(M + N + K)
+    a = so.bf16_round(r.standard_normal((M, K)).astype(np.float32))
+    w = so.bf16_round((r.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32))
+    out = empty((M + 1) * N * 4).fill_bytes(0)
+    L.vra_stack_op_gemm(to_dev(a, BF16).ptr, K, to_dev(w, BF16).ptr, 0, out.ptr, N, 1, M, N, K, 1.0, None, 0, None, None, None, 0, 0.0, BF16, 0)
+    check()
+    got = out.numpy(np.float32, (M + 1, N))
+    assert rel(got[:M], a.astype(np.float64) @ w.astype(np.float64).T) < 2e-6 and (got[M] == 0).all()
+
+
 def test_residual_combine():
     L = _lib.load()
     r = np.random.default_rng(5)

@@ -59,8 +59,17 @@ void vra_stack_embed_sinpos(const uint32_t* ids, const int64_t* positions, const
 // Router (router_w != null, [n_router (+1 when gate_row), W] in dtype): z = router_w . h in f32 on the unrounded h; the `top` largest of the
 // first n_router give pair_expert / pair_weight [T, top] (weight = sigmoid(z), not renormalised; ties: the lower index); with
 // gate_row the last row gives gate_out[t] = sigmoid(z_last).
+// With `o`: the row first becomes x + mult * (o + sum_{j < n1} p1[t * n1 + j] + gate_in[t] * p2[t]) and is written back (vra_stack_residual_combine
+// of the layer before, in the launch that reads its result).
 struct StkNormArgs {
   const float* x = nullptr;
+  float* x_out = nullptr;  // (with `o`: x itself)
+  const float* o = nullptr;
+  const float* p1 = nullptr;
+  int n1 = 0;
+  const float* p2 = nullptr;
+  const float* gate_in = nullptr;
+  float mult = 1.f;
   const float* w = nullptr;
   void* h = nullptr;
   int T = 0, W = 0, groups = 1;

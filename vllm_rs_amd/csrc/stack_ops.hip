@@ -16,6 +16,9 @@
 
 namespace {
 
+// a wave's sum by DPP and permlane swaps: a VALU operation per step where a shuffle is an LDS round trip
+__device__ __forceinline__ float wave_total(float v) { return vra_xor32_sum(vra_xor16_sum(row16_sum(v))); }
+
 __device__ __forceinline__ float gelu_tanh_(float z) { return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))); }
 __device__ __forceinline__ float gelu_erf_(float z) { return 0.5f * z * (1.f + erff(z * 0.7071067811865476f)); }
 // the finished value of a plain product: element-wise activation (epi 2), soft cap
@@ -48,13 +51,12 @@ __global__ __launch_bounds__(256) void stk_embed_sinpos_kernel(const uint32_t* i
   uint32_t id = ids[t];
   if (id >= (uint32_t)V) id = 0;
   const float p = (float)pos[t];
-  for (int c = threadIdx.x; c < W; c += 256) {
-    float pe = 0.f;
-    if (inv_freq) {
-      const float ang = p * inv_freq[c >> 1];
-      pe = (c & 1) ? cosf(ang) : sinf(ang);
-    }
-    x[(size_t)t * W + c] = El<T>::ld(embed + (size_t)id * W + c) + pe;
+  // (a thread takes both entries of an angle: lanes that alternate between sine and cosine would each wait for the other's)
+  for (int i = threadIdx.x; i < (W + 1) / 2; i += 256) {
+    float sn = 0.f, cs = 0.f;
+    if (inv_freq) sincosf(p * inv_freq[i], &sn, &cs);
+    x[(size_t)t * W + 2 * i] = El<T>::ld(embed + (size_t)id * W + 2 * i) + sn;
+    if (2 * i + 1 < W) x[(size_t)t * W + 2 * i + 1] = El<T>::ld(embed + (size_t)id * W + 2 * i + 1) + cs;
   }
 }
 
@@ -68,54 +70,115 @@ __global__ __launch_bounds__(256) void stk_group_norm_kernel(StkNormArgs a) {
   const int t = blockIdx.x, W = a.W, gs = W / a.groups;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const float* x = a.x + (size_t)t * W;
-  for (int c = threadIdx.x; c < W; c += 256) xs[c] = x[c];
-  __syncthreads();
-  for (int g = wave; g < a.groups; g += 4) {
-    float s = 0.f;
-    for (int c = lane; c < gs; c += 64) {
-      const float v = xs[g * gs + c];
-      s = fmaf(v, v, s);
-    }
-    s = wave_sum(s);
-    if (lane == 0) rs[g] = 1.f / sqrtf(s / (float)gs + a.eps);
-  }
-  __syncthreads();
   T* h = (T*)a.h + (size_t)t * W;
-  for (int c = threadIdx.x; c < W; c += 256) {
-    const float v = xs[c] * rs[c / gs] * a.w[c];
-    xs[c] = v;
-    El<T>::st(h + c, v);
-  }
+  auto sums = [&] {
+    __syncthreads();
+    for (int g = wave; g < a.groups; g += 4) {
+      float s = 0.f;
+      for (int c = lane; c < gs; c += 64) {
+        const float v = xs[g * gs + c];
+        s = fmaf(v, v, s);
+      }
+      s = wave_total(s);
+      if (lane == 0) rs[g] = 1.f / sqrtf(s / (float)gs + a.eps);
+    }
+    __syncthreads();
+  };
+  // (four values a load where rows and groups allow it, the weights with them: a row's parts arrive in one round trip instead of W / 256, and the
+  // row stays in registers: 8 rows of 2048: 6.6 us, now 4.0)
+  auto row = [&](auto width, auto rounds) {
+    constexpr int N = decltype(width)::value, R = decltype(rounds)::value;
+    typedef float vec __attribute__((ext_vector_type(N)));
+    vec keep[R], wt[R];
+    const float gt = a.gate_in ? a.gate_in[t] : 1.f;
+    auto load = [&](int c) {
+      vec v = *(const vec*)(x + c);
+      if (a.o) {
+        vec s = *(const vec*)(a.o + (size_t)t * W + c);
+        for (int j = 0; j < a.n1; j++) s += *(const vec*)(a.p1 + ((size_t)t * a.n1 + j) * W + c);
+        if (a.p2) s += gt * *(const vec*)(a.p2 + (size_t)t * W + c);
+        v += a.mult * s;
+        *(vec*)(a.x_out + (size_t)t * W + c) = v;
+      }
+      *(vec*)(xs + c) = v;
+      return v;
+    };
+    auto put = [&](int c, vec v, vec w) {
+      const vec y = v * rs[c / gs] * w;
+      if (a.router_w) *(vec*)(xs + c) = y;
+#pragma unroll
+      for (int e = 0; e < N; e++) El<T>::st(h + c + e, y[e]);
+    };
+#pragma unroll
+    for (int n = 0; n < R; n++) {
+      const int c = threadIdx.x * N + n * 256 * N;
+      if (c < W) wt[n] = *(const vec*)(a.w + c), keep[n] = load(c);
+    }
+    for (int c = threadIdx.x * N + R * 256 * N; c < W; c += 256 * N) load(c);
+    sums();
+#pragma unroll
+    for (int n = 0; n < R; n++) {
+      const int c = threadIdx.x * N + n * 256 * N;
+      if (c < W) put(c, keep[n], wt[n]);
+    }
+    for (int c = threadIdx.x * N + R * 256 * N; c < W; c += 256 * N) put(c, *(const vec*)(xs + c), *(const vec*)(a.w + c));
+  };
+  const bool quads = W % 4 == 0 && gs % 4 == 0 && (((uintptr_t)a.x | (uintptr_t)a.x_out | (uintptr_t)a.o | (uintptr_t)a.p1 | (uintptr_t)a.p2 | (uintptr_t)a.w) % 16) == 0;
+  if (quads) row(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
+  else row(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
   if (!a.router_w) return;
   __syncthreads();
   const int nz = a.n_router + (a.gate_row ? 1 : 0);
   const T* rw = (const T*)a.router_w;
-  for (int e = wave; e < nz; e += 4) {
-    float s = 0.f;
-    if (sizeof(T) == 2 && W % 8 == 0 && ((uintptr_t)rw % 16) == 0) {  // 8 weights a load; the lane's partial sums keep one order for a given W
+  if (sizeof(T) == 2 && W % 8 == 0 && ((uintptr_t)rw % 16) == 0) {  // 8 weights a load; the lane's partial sums keep one order for a given W
+    for (int e0 = wave; e0 < nz; e0 += 16) {  // four outputs of a wave side by side: their weights are under way together, the row is read once
+      float s[4] = {0.f, 0.f, 0.f, 0.f};
       for (int c = lane * 8; c < W; c += 64 * 8) {
-        const u32x4 v = *(const u32x4*)((const uint16_t*)rw + (size_t)e * W + c);
-        for (int i = 0; i < 4; i++) {
-          s = fmaf(xs[c + 2 * i], __uint_as_float(v[i] << 16), s);
-          s = fmaf(xs[c + 2 * i + 1], __uint_as_float(v[i] & 0xffff0000u), s);
-        }
+        u32x4 v[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = *(const u32x4*)((const uint16_t*)rw + (size_t)min(e0 + q * 4, nz - 1) * W + c);
+        float f[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) f[i] = xs[c + i];
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            s[q] = fmaf(f[2 * i], __uint_as_float(v[q][i] << 16), s[q]);
+            s[q] = fmaf(f[2 * i + 1], __uint_as_float(v[q][i] & 0xffff0000u), s[q]);
+          }
       }
-    } else {
-      for (int c = lane; c < W; c += 64) s = fmaf(xs[c], El<T>::ld(rw + (size_t)e * W + c), s);
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        s[q] = wave_sum(s[q]);
+        if (lane == 0 && e0 + q * 4 < nz) zs[e0 + q * 4] = s[q];
+      }
     }
-    s = wave_sum(s);
-    if (lane == 0) zs[e] = s;
+  } else {
+    for (int e = wave; e < nz; e += 4) {
+      float s = 0.f;
+      for (int c = lane; c < W; c += 64) s = fmaf(xs[c], El<T>::ld(rw + (size_t)e * W + c), s);
+      s = wave_sum(s);
+      if (lane == 0) zs[e] = s;
+    }
   }
   __syncthreads();
+  // the picks, by one thread from LDS (the row is not needed any more: its place holds the marks)
   if (threadIdx.x == 0) {
+    int* taken = (int*)xs;
+    const bool marks = a.n_router <= W;  // (more outputs than channels: look the earlier picks up)
+    if (marks)
+      for (int e = 0; e < a.n_router; e++) taken[e] = 0;
     for (int j = 0; j < a.top; j++) {
       int best = -1;
       float bz = -INFINITY;
       for (int e = 0; e < a.n_router; e++) {
-        bool taken = false;
-        for (int q = 0; q < j; q++) taken = taken || a.pair_expert[(size_t)t * a.top + q] == e;
-        if (!taken && (best < 0 || zs[e] > bz)) best = e, bz = zs[e];
+        bool skip = marks && taken[e];
+        if (!marks)
+          for (int q = 0; q < j; q++) skip = skip || a.pair_expert[(size_t)t * a.top + q] == e;
+        if (!skip && (best < 0 || zs[e] > bz)) best = e, bz = zs[e];
       }
+      if (marks) taken[best] = 1;
       a.pair_expert[(size_t)t * a.top + j] = best;
       a.pair_weight[(size_t)t * a.top + j] = sigmoidf_(bz);
     }
@@ -356,12 +419,14 @@ __global__ __launch_bounds__(64 * WM * WN) void stk_gemm_mfma_kernel(StkGemmArgs
   }
 }
 
-// Steps of up to 32 rows (decoding): the weights are the whole traffic, so a workgroup takes only 32 output columns and its 8 waves
-// take an eighth of K each (whole K-steps of 32, ascending inside a wave); the 8 partial tiles meet in LDS and are summed in wave order.
-// One fixed order for a given K — another one than the large-M kernel's single chain, so the two agree to rounding, not to the bit.
-template <bool SCALED, bool POST = false>
+// Steps of up to 32 rows (decoding): the weights are the whole traffic, and what bounds it is the CUs that pull at them.  A
+// workgroup takes 16 * NT output columns and its 8 waves take an eighth of K each (whole K-steps of 32, ascending inside a wave); the partial
+// tiles meet in LDS and are summed in wave order.  One fixed order for a given K — another one than the large-M kernel's single chain, so the
+// two agree to rounding, not to the bit.
+template <bool SCALED, bool POST, int NT>
 __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g) {
-  __shared__ float part[8][16 * 32];
+  constexpr int BN = 16 * NT, NW = 8;
+  __shared__ float part[NW][16 * BN];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, rq = lane & 15, oct = lane >> 4;
   int group = 0;
   if (g.tile_group) {
@@ -371,26 +436,31 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g)
   const uint16_t* A = (const uint16_t*)g.a + (int64_t)blockIdx.z * g.a_batch_stride;
   const uint16_t* Wt = (const uint16_t*)g.w + (int64_t)group * g.w_group_stride + (int64_t)blockIdx.z * g.w_batch_stride;
   const int64_t ob = (int64_t)blockIdx.z * g.out_batch_stride;
-  const int m_base = blockIdx.x * 16, n_base = blockIdx.y * 32;
+  const int m_base = blockIdx.x * 16, n_base = blockIdx.y * BN;
   const int r = m_base + rq;
   const int idx = r < g.M ? (g.a_row ? g.a_row[r] : r) : -1;
   const uint16_t* ap = A + (int64_t)(idx >= 0 ? idx : 0) * g.lda;
   const float asc = SCALED && idx >= 0 ? g.a_scale[r] : 1.f;
-  const uint16_t* wp[2];
-  bool wv[2];
-  for (int nt = 0; nt < 2; nt++) {
+  const uint16_t* wp[NT];
+  bool wv[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; nt++) {
     const int n = n_base + nt * 16 + rq;
     wv[nt] = n < g.N;
     wp[nt] = Wt + (int64_t)(n < g.N ? n : 0) * g.K;
   }
-  const int ksteps = (g.K + 31) / 32, per = (ksteps + 7) / 8;
+  const int ksteps = (g.K + 31) / 32, per = (ksteps + NW - 1) / NW;
   const int k_lo = wave * per * 32, k_hi = min(g.K, (wave + 1) * per * 32);
-  f32x4 acc[2] = {vra_zero_acc(), vra_zero_acc()};
+  f32x4 acc[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; nt++) acc[nt] = vra_zero_acc();
   const u32x4 zero4 = {0u, 0u, 0u, 0u};
-  // four K-steps per round: their twelve 16-byte requests are in flight together, then the eight MFMAs (steps beyond the wave's range
-  // load from offset 0 and count as zeros: same order of the sum, no branch between the MFMAs)
+  // four K-steps per round: their 16-byte requests are in flight together, then the MFMAs (steps beyond the wave's range load from offset 0 and
+  // count as zeros: same order of the sum, no branch between the MFMAs).  Eight at a time, the next round ahead of the MFMAs, or 16 waves
+  // are slower at every size (2048 columns, K = 8192: 15.0 us; 16.5, 15.8 and 15.3).
   for (int k0 = k_lo; k0 < k_hi; k0 += 4 * 32) {
-    u32x4 af[4], wf[4][2];
+    u32x4 af[4], wf[4][NT];
+#pragma unroll
     for (int u = 0; u < 4; u++) {
       const int k = k0 + u * 32 + oct * 8;
       const bool kin = k < k_hi;
@@ -400,19 +470,25 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g)
         for (int i = 0; i < 4; i++) a4[i] = BF16::pack2(__uint_as_float(a4[i] << 16) * asc, __uint_as_float(a4[i] & 0xffff0000u) * asc);
       }
       af[u] = (idx >= 0 && kin) ? a4 : zero4;
-      for (int nt = 0; nt < 2; nt++) {
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++) {
         const u32x4 v = *(const u32x4*)(wp[nt] + kc);
         wf[u][nt] = (wv[nt] && kin) ? v : zero4;
       }
     }
+#pragma unroll
     for (int u = 0; u < 4; u++)
-      for (int nt = 0; nt < 2; nt++) BF16::mfma(acc[nt], __builtin_bit_cast(s16x8, wf[u][nt]), __builtin_bit_cast(s16x8, af[u]));
+#pragma unroll
+      for (int nt = 0; nt < NT; nt++) BF16::mfma(acc[nt], __builtin_bit_cast(s16x8, wf[u][nt]), __builtin_bit_cast(s16x8, af[u]));
   }
   VRA_MFMA_DRAIN();
-  for (int nt = 0; nt < 2; nt++)
-    for (int j = 0; j < 4; j++) part[wave][rq * 32 + nt * 16 + oct * 4 + j] = acc[nt][j];
+#pragma unroll
+  for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) part[wave][rq * BN + nt * 16 + oct * 4 + j] = acc[nt][j];
   __syncthreads();
-  const int e = threadIdx.x, m = e >> 5, c = e & 31;  // one output element per thread
+  const int e = threadIdx.x, m = e / BN, c = e % BN;  // one output element per thread
+  if (e >= 16 * BN) return;
   const int row = m_base + m;
   if (row >= g.M) return;
   const int ridx = g.a_row ? g.a_row[row] : row;
@@ -420,11 +496,12 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g)
   const int orow = g.out_row ? g.out_row[row] : row;
   if (orow < 0) return;
   auto total = [&](int col) {
-    float s = part[0][m * 32 + col];
-    for (int w = 1; w < 8; w++) s += part[w][m * 32 + col];
+    float s = part[0][m * BN + col];
+#pragma unroll
+    for (int w = 1; w < NW; w++) s += part[w][m * BN + col];
     return s;
   };
-  if (g.epi == 1) {
+  if (NT == 2 && g.epi == 1) {
     if (c >= 16) return;
     const int n = n_base / 2 + c;
     if (n >= g.N / 2) return;
@@ -537,61 +614,81 @@ __global__ __launch_bounds__(256) void stk_gated_act_kernel(const float* gu, T* 
 }
 
 #define STK_PN_THREADS 1024
-__device__ __forceinline__ float block_sum_pn(float v, float* red) {
-  v = wave_sum(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  float s = 0.f;
-  for (int w = 0; w < STK_PN_THREADS / 64; w++) s += red[w];
-  return s;
-}
-// one workgroup of 1024 threads per token: up to 8 values per thread stay in registers between the sums and the output
-template <typename T>
+// one workgroup of 1024 threads per token (bound: HBM, z read and the activation written once): 8 values a thread stay in registers between the
+// sums and the output — two loads of four where rows start on 16 bytes — and the three sums meet behind one barrier.  2048 tokens x 8192: 35 us
+// with single values and a pair of barriers per sum, now 21
+template <typename T, int N>
 __global__ __launch_bounds__(STK_PN_THREADS) void stk_polynorm_kernel(const float* z, T* out, const float* coef, int F, float eps) {
-  __shared__ float red[STK_PN_THREADS / 64];
+  typedef float vec __attribute__((ext_vector_type(N)));
+  constexpr int R = 8 / N, STEP = STK_PN_THREADS * N;
+  __shared__ float red[3][STK_PN_THREADS / 64];
   const int m = blockIdx.x;
   const float* zr = z + (size_t)m * F;
-  float keep[8];
-  float s1 = 0.f, s2 = 0.f, s3 = 0.f;
-#pragma unroll
-  for (int n = 0; n < 8; n++) {  // the first 8192 values: one per thread and round, kept in registers
-    const int f = threadIdx.x + n * STK_PN_THREADS;
-    const float v = f < F ? zr[f] : 0.f, v2 = v * v, v3 = v2 * v;
-    keep[n] = v;
-    s1 = fmaf(v, v, s1), s2 = fmaf(v2, v2, s2), s3 = fmaf(v3, v3, s3);
-  }
-  for (int f = threadIdx.x + 8 * STK_PN_THREADS; f < F; f += STK_PN_THREADS) {
-    const float v = zr[f], v2 = v * v, v3 = v2 * v;
-    s1 = fmaf(v, v, s1), s2 = fmaf(v2, v2, s2), s3 = fmaf(v3, v3, s3);
-  }
-  s1 = block_sum_pn(s1, red);
-  s2 = block_sum_pn(s2, red);
-  s3 = block_sum_pn(s3, red);
-  const float r1 = 1.f / sqrtf(s1 / (float)F + eps), r2 = 1.f / sqrtf(s2 / (float)F + eps), r3 = 1.f / sqrtf(s3 / (float)F + eps);
   const float ca = coef[0], cb = coef[1], cc = coef[2], ce = coef[3];
+  vec keep[R];
+  float s1 = 0.f, s2 = 0.f, s3 = 0.f;
+  auto add = [&](vec x) {
 #pragma unroll
-  for (int n = 0; n < 8; n++) {
-    const int f = threadIdx.x + n * STK_PN_THREADS;
-    const float v = keep[n], v2 = v * v, v3 = v2 * v;
-    if (f < F) El<T>::st(out + (size_t)m * F + f, ca * (v * r1) + cb * (v2 * r2) + cc * (v3 * r3) + ce);
+    for (int e = 0; e < N; e++) {
+      const float v = x[e], v2 = v * v, v3 = v2 * v;
+      s1 = fmaf(v, v, s1), s2 = fmaf(v2, v2, s2), s3 = fmaf(v3, v3, s3);
+    }
+  };
+#pragma unroll
+  for (int n = 0; n < R; n++) {
+    const int f = threadIdx.x * N + n * STEP;
+    keep[n] = f < F ? *(const vec*)(zr + f) : (vec)(0.f);
   }
-  for (int f = threadIdx.x + 8 * STK_PN_THREADS; f < F; f += STK_PN_THREADS) {
-    const float v = zr[f], v2 = v * v, v3 = v2 * v;
-    El<T>::st(out + (size_t)m * F + f, ca * (v * r1) + cb * (v2 * r2) + cc * (v3 * r3) + ce);
+#pragma unroll
+  for (int n = 0; n < R; n++) add(keep[n]);
+  for (int f = threadIdx.x * N + R * STEP; f < F; f += STEP) add(*(const vec*)(zr + f));
+  s1 = wave_total(s1), s2 = wave_total(s2), s3 = wave_total(s3);
+  if ((threadIdx.x & 63) == 0) red[0][threadIdx.x >> 6] = s1, red[1][threadIdx.x >> 6] = s2, red[2][threadIdx.x >> 6] = s3;
+  __syncthreads();
+  s1 = s2 = s3 = 0.f;
+  for (int w = 0; w < STK_PN_THREADS / 64; w++) s1 += red[0][w], s2 += red[1][w], s3 += red[2][w];
+  const float r1 = 1.f / sqrtf(s1 / (float)F + eps), r2 = 1.f / sqrtf(s2 / (float)F + eps), r3 = 1.f / sqrtf(s3 / (float)F + eps);
+  auto put = [&](int f, vec x) {
+    float y[N];
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+      const float v = x[e], v2 = v * v, v3 = v2 * v;
+      y[e] = ca * (v * r1) + cb * (v2 * r2) + cc * (v3 * r3) + ce;
+    }
+    T* const o = out + (size_t)m * F + f;
+    if constexpr (N == 4 && sizeof(T) == 2) {
+      *(u32x2*)o = u32x2{BF16::pack2(y[0], y[1]), BF16::pack2(y[2], y[3])};
+    } else if constexpr (N == 4) {
+      *(f32x4*)o = f32x4{y[0], y[1], y[2], y[3]};
+    } else {
+      El<T>::st(o, y[0]);
+    }
+  };
+#pragma unroll
+  for (int n = 0; n < R; n++) {
+    const int f = threadIdx.x * N + n * STEP;
+    if (f < F) put(f, keep[n]);
   }
+  for (int f = threadIdx.x * N + R * STEP; f < F; f += STEP) put(f, *(const vec*)(zr + f));
 }
 
 __global__ __launch_bounds__(256) void stk_residual_combine_kernel(float* x, const float* o, const float* p1, int n1, const float* p2, const float* gate,
-                                                                   float mult, int W) {
+                                                                   float mult, int W, int quads) {
   const int t = blockIdx.x;
   const float gt = gate ? gate[t] : 1.f;
-  for (int c = threadIdx.x; c < W; c += 256) {
-    float s = o ? o[(size_t)t * W + c] : 0.f;
-    for (int j = 0; j < n1; j++) s += p1[((size_t)t * n1 + j) * W + c];
-    if (p2) s += gt * p2[(size_t)t * W + c];
-    x[(size_t)t * W + c] += mult * s;
-  }
+  auto row = [&](auto width) {
+    constexpr int N = decltype(width)::value;
+    typedef float vec __attribute__((ext_vector_type(N)));
+    for (int c = threadIdx.x * N; c < W; c += 256 * N) {
+      vec s = 0.f;
+      if (o) s = *(const vec*)(o + (size_t)t * W + c);
+      for (int j = 0; j < n1; j++) s += *(const vec*)(p1 + ((size_t)t * n1 + j) * W + c);
+      if (p2) s += gt * *(const vec*)(p2 + (size_t)t * W + c);
+      *(vec*)(x + (size_t)t * W + c) += mult * s;
+    }
+  };
+  if (quads) row(std::integral_constant<int, 4>{});
+  else row(std::integral_constant<int, 1>{});
 }
 
 __global__ __launch_bounds__(256) void stk_gather_rows_kernel(const float* src, const uint32_t* rows, float* dst, int W) {
@@ -1319,10 +1416,19 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
       else if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<2, 4, 2, 2, false, true><<<grid, 256, 0, st>>>(g); });
       else launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<2, 4, 2, 2, false><<<grid, 256, 0, st>>>(g); });
     } else {
-      dim3 grid((g.M + 15) / 16, (g.N + 31) / 32, nb);
-      if (g.a_scale) launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<true><<<grid, 512, 0, st>>>(g); });
-      else if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false, true><<<grid, 512, 0, st>>>(g); });
-      else launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false><<<grid, 512, 0, st>>>(g); });
+      // 32 columns a workgroup read x half as often, but below 256 workgroups they leave CUs idle (8 rows: 2048 columns, K = 2048 / 8192: 7.3 / 22.8 us,
+      // with 16 columns 5.6 / 15.0; 8192 columns, K = 2048: 10.6 against 10.8; 32 000: 29.8 against 32.5).  A gated pair needs both its blocks.
+      const bool wide = g.epi == 1 || (int64_t)((g.M + 15) / 16) * ((g.N + 31) / 32) * nb >= 256;
+#define STK_SMALL(NTV)                                                                                                                 \
+  do {                                                                                                                               \
+    dim3 grid((g.M + 15) / 16, (g.N + 16 * NTV - 1) / (16 * NTV), nb);                                                               \
+    if (g.a_scale) launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<true, false, NTV><<<grid, 512, 0, st>>>(g); });     \
+    else if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false, true, NTV><<<grid, 512, 0, st>>>(g); });     \
+    else launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false, false, NTV><<<grid, 512, 0, st>>>(g); });              \
+  } while (0)
+      if (wide) STK_SMALL(2);
+      else STK_SMALL(1);
+#undef STK_SMALL
     }
     return;
   }
@@ -1350,6 +1456,7 @@ void vra_stack_embed_sinpos(const uint32_t* ids, const int64_t* positions, const
 void vra_stack_group_norm(const StkNormArgs& a, int dtype, int64_t stream) {
   VRA_CHECK_ARG(a.x && a.w && a.h && a.T > 0 && a.W > 0, "stack norm: null pointer or empty shape");
   VRA_CHECK_ARG(a.groups >= 1 && a.W % a.groups == 0, "stack norm: the width must split into equal groups");
+  VRA_CHECK_ARG(!a.o || (a.x_out == a.x && (a.n1 == 0 || a.p1)), "stack norm: parts of the row without a place for the sum");
   VRA_CHECK_ARG(!a.router_w || (a.pair_expert && a.pair_weight && a.top >= 1 && a.top <= a.n_router && (!a.gate_row || a.gate_out)), "stack norm: router outputs");
   const size_t lds = ((size_t)a.W + a.groups + a.n_router + 2) * sizeof(float);
   VRA_CHECK_ARG(lds <= 64 * 1024, "stack norm: row does not fit LDS");
@@ -1376,14 +1483,23 @@ void vra_stack_gated_act(const float* gu, void* out, int M, int F, float limit, 
 
 void vra_stack_polynorm(const float* z, void* out, const float* coef, int M, int F, float eps, int dtype, int64_t stream) {
   VRA_CHECK_ARG(z && out && coef && M > 0 && F > 0, "stack polynorm: null pointer or empty shape");
-  if (dtype == VRA_F32) launch_checked("stack polynorm", [&] { stk_polynorm_kernel<float><<<M, STK_PN_THREADS, 0, as_stream(stream)>>>(z, (float*)out, coef, F, eps); });
-  else launch_checked("stack polynorm", [&] { stk_polynorm_kernel<uint16_t><<<M, STK_PN_THREADS, 0, as_stream(stream)>>>(z, (uint16_t*)out, coef, F, eps); });
+  const bool quads = F % 4 == 0 && (((uintptr_t)z | (uintptr_t)out) % 16) == 0;
+  launch_checked("stack polynorm", [&] {
+    if (dtype == VRA_F32) {
+      if (quads) stk_polynorm_kernel<float, 4><<<M, STK_PN_THREADS, 0, as_stream(stream)>>>(z, (float*)out, coef, F, eps);
+      else stk_polynorm_kernel<float, 1><<<M, STK_PN_THREADS, 0, as_stream(stream)>>>(z, (float*)out, coef, F, eps);
+    } else {
+      if (quads) stk_polynorm_kernel<uint16_t, 4><<<M, STK_PN_THREADS, 0, as_stream(stream)>>>(z, (uint16_t*)out, coef, F, eps);
+      else stk_polynorm_kernel<uint16_t, 1><<<M, STK_PN_THREADS, 0, as_stream(stream)>>>(z, (uint16_t*)out, coef, F, eps);
+    }
+  });
 }
 
 void vra_stack_residual_combine(float* x, const float* o, const float* p1, int n1, const float* p2, const float* gate, float mult, int T, int W,
                                 int64_t stream) {
   VRA_CHECK_ARG(x && T > 0 && W > 0 && (n1 == 0 || p1), "stack combine: null pointer or empty shape");
-  launch_checked("stack combine", [&] { stk_residual_combine_kernel<<<T, 256, 0, as_stream(stream)>>>(x, o, p1, n1, p2, gate, mult, W); });
+  const int quads = W % 4 == 0 && (((uintptr_t)x | (uintptr_t)o | (uintptr_t)p1 | (uintptr_t)p2) % 16) == 0;
+  launch_checked("stack combine", [&] { stk_residual_combine_kernel<<<T, 256, 0, as_stream(stream)>>>(x, o, p1, n1, p2, gate, mult, W, quads); });
 }
 
 void vra_stack_gather_rows_f32(const float* src, const uint32_t* rows, float* dst, int n, int W, int64_t stream) {

@@ -1113,6 +1113,7 @@ bool StackModel::expert_pair(const void* a, int lda, const void* w_gu, int64_t g
   return !take_stack_err(error, "expert feed-forward");
 }
 
+// the layer's sum into the residual is left due: the next layer's norm adds it on its way in, the last layer's (or a traced one's) gets a launch
 bool StackModel::feed_forward(const StackLayer& L, int T, int64_t stream) {
   const int W = width_;
   if (L.mlp == 1) {
@@ -1123,7 +1124,7 @@ bool StackModel::feed_forward(const StackLayer& L, int T, int64_t stream) {
     StkGemmArgs d;
     d.a = act_, d.lda = L.ff, d.w = L.down, d.M = T, d.N = W, d.K = L.ff, d.out = pair_out_, d.ldo = W, d.out_f32 = 1;
     vra_stack_gemm(d, dt_, stream);
-    vra_stack_residual_combine(x_, o_, pair_out_, 1, nullptr, nullptr, residual_mult_, T, W, stream);
+    due_ = {o_, pair_out_, 1, nullptr, nullptr};
     return !take_stack_err(error, "dense feed-forward");
   }
   if (L.mlp == 2) {
@@ -1139,11 +1140,11 @@ bool StackModel::feed_forward(const StackLayer& L, int T, int64_t stream) {
     if (L.shared_ff > 0 &&
         !expert_pair(h_, W, L.s_gu, 0, L.s_down, 0, T, L.sffp, L.shared_ff, L.shared_limit, nullptr, 0, nullptr, nullptr, nullptr, sh_, stream))
       return false;
-    vra_stack_residual_combine(x_, o_, pair_out_, L.top, L.shared_ff > 0 ? sh_ : nullptr, L.shared_ff > 0 ? gate_ : nullptr, residual_mult_, T, W, stream);
+    due_ = {o_, pair_out_, L.top, L.shared_ff > 0 ? sh_ : nullptr, L.shared_ff > 0 ? gate_ : nullptr};
     return !take_stack_err(error, "mixture of experts");
   }
-  vra_stack_residual_combine(x_, o_, nullptr, 0, nullptr, nullptr, residual_mult_, T, W, stream);
-  return !take_stack_err(error, "residual");
+  due_ = {o_, nullptr, 0, nullptr, nullptr};
+  return true;
 }
 
 // h = norm(x + add) with x updated in place (add null: x as it is); sequential blocks norm every sub-block's input
@@ -1268,6 +1269,7 @@ bool StackModel::forward(const InputMetadata& md, int64_t stream, uint32_t* toke
     vra_stack_embed_sinpos(md.input_ids, md.positions, embed_, pos_kind_ == 0 ? inv_freq_ : nullptr, x_, T, W, vocab_, dt_, stream);
     if (take_stack_err(error, "embedding")) return false;
   }
+  due_ = {};  // (a step that failed may have left one)
   // sequential blocks: the output of a sub-block is added to the residual inside the launch of the next norm (`pending`)
   const float* pending = nullptr;
   for (size_t li = 0; li < layers_.size() && block_ < 2; li++) {
@@ -1276,6 +1278,8 @@ bool StackModel::forward(const InputMetadata& md, int64_t stream, uint32_t* toke
       // h = norm(x); a mixture-of-experts layer's router (and its shared expert's gate) reads h inside the same launch
       StkNormArgs n;
       n.x = x_, n.w = L.norm_w, n.h = h_, n.T = T, n.W = W, n.groups = groups_, n.eps = eps_;
+      if (due_.o) n.x_out = x_, n.o = due_.o, n.p1 = due_.p1, n.n1 = due_.n1, n.p2 = due_.p2, n.gate_in = due_.gate, n.mult = residual_mult_;
+      due_ = {};
       if (L.mlp == 2) {
         n.router_w = L.router, n.n_router = L.experts, n.top = L.top, n.gate_row = L.shared_ff > 0;
         n.pair_expert = pair_expert_, n.pair_weight = pair_weight_, n.gate_out = gate_;
@@ -1283,6 +1287,11 @@ bool StackModel::forward(const InputMetadata& md, int64_t stream, uint32_t* toke
       vra_stack_group_norm(n, dt_, stream);
       if (!mixer_softmax(L, md, stream)) return false;
       if (!feed_forward(L, T, stream)) return false;
+      if (trace_on_ || li + 1 == layers_.size()) {
+        vra_stack_residual_combine(x_, due_.o, due_.p1, due_.n1, due_.p2, due_.gate, residual_mult_, T, W, stream);
+        due_ = {};
+        if (take_stack_err(error, "residual")) return false;
+      }
     } else {
       if (!norm_into_h(L.norm_w, L.norm_b, L.norm_alpha, pending, x_, h_, T, stream)) return false;
       if (!(L.mixer == 1 ? mixer_latent(L, md, stream) : (L.mixer == 2 ? mixer_sigmoid(L, md, stream) : mixer_softmax(L, md, stream)))) return false;

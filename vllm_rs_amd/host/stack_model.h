@@ -242,6 +242,11 @@ class StackModel : public ModelBase {
   void rotary_table(StackLayer& L);
   float* upload_floats(const std::vector<float>& v);
   bool norm_into_h(const float* w, const float* b, float alpha, const float* add, float* x, void* h, int T, int64_t stream);
+  struct Due {  // parts of a parallel block's sum that x_ does not hold yet
+    const float *o = nullptr, *p1 = nullptr;
+    int n1 = 0;
+    const float *p2 = nullptr, *gate = nullptr;
+  } due_;
   bool tiles128(const StackLayer& L) const;
   bool expert_pair(const void* a, int lda, const void* w_gu, int64_t gu_stride, const void* w_down, int64_t down_stride, int rows, int fp, int f,
                    float limit, const int* tile_group, int granule, const int* a_row, const float* a_scale, const int* out_row, float* out,
