@@ -576,6 +576,36 @@ def test_linear_recurrence_alone(form, H, rep, D, V):
     assert rel(again, ref) < 1e-5
 
 
+@pytest.mark.parametrize("T", [1, 15, 17, 31, 32, 33, 64, 97])
+@pytest.mark.parametrize("D,V,pad", [(4, 5, 0), (32, 64, 0), (32, 33, 1), (36, 20, 4), (132, 12, 0), (256, 8, 0)])
+def test_linear_recurrence_tiles(D, V, pad, T):
+    """the recurrence kernel at the edges of its tiles of tokens (32, or 16 for keys beyond 128): whole tiles of whole 16-byte rows, which are
+    fetched without bounds, beside ragged ones, rows off 16 bytes (pad 1) and rows of part of the lanes (36, 132); a key size of one lane.
+    float32 sums of D terms along chains that contract (decays below 1, unit keys): 1e-5 of the largest output, as for the forms above"""
+    L = _lib.load()
+    r = np.random.default_rng(D * 131 + T)
+    H = 2
+    q = r.standard_normal((T, H, D)).astype(np.float32)
+    k = r.standard_normal((T, H, D)).astype(np.float32)
+    k /= np.sqrt((k * k).sum(-1, keepdims=True))
+    v = r.standard_normal((T, H, V)).astype(np.float32)
+    decay = (0.7 + 0.3 * r.random((T, H, D))).astype(np.float32)
+    beta = r.random((T, H)).astype(np.float32)
+    state, out = raw(np.full(2 * H * V * D, 50.0, np.float32), np.float32), empty(T * H * V * 4)
+
+    def rows(x):  # the rows of x, `pad` floats apart
+        y = np.full((T, H * x.shape[2] + pad), 9.0, np.float32)
+        y[:, :H * x.shape[2]] = x.reshape(T, -1)
+        return raw(y, np.float32).ptr
+
+    L.vra_stack_op_linear_scan(rows(q), H * D + pad, rows(k), H * D + pad, rows(v), H * V + pad, rows(decay), H * D + pad, None, raw(beta, np.float32).ptr, H, 0.5,
+                               state.ptr, raw([1], np.int32).ptr, raw(np.arange(T), np.int64).ptr, raw([0, T], np.uint32).ptr, out.ptr, H * V, 1, H, 1, D, V, 0)
+    check()
+    ref = zo.linear_recurrence(q.astype(np.float64) * 0.5, k.astype(np.float64), v.astype(np.float64), decay.astype(np.float64), beta.astype(np.float64))
+    assert rel(out.numpy(np.float32, (T, H, V)), ref) < 1e-5
+    assert (state.numpy(np.float32, (2, H * V * D))[0] == 50.0).all()
+
+
 
 @pytest.mark.parametrize("dt", [F32, BF16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("W,E,top", [(96, 5, 2), (51, 3, 3), (256, 40, 1), (64, 8, 4)])

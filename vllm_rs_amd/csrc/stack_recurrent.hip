@@ -715,31 +715,40 @@ __global__ __launch_bounds__(256) void stk_sigmoid_pow_kernel(const float* z, in
 
 // ------------------------------------------------------------------------------------------------ the linear recurrence
 // A workgroup owns 256 / P columns of one head's state (a column = one value channel); a column's `dim` rows are spread over P
-// neighbouring lanes, R rows each, in registers for the whole step.  Sums over the rows (S^T k, S^T q) add a lane's R products in order,
-// then the P lanes by xor shuffles: an order fixed by `dim` alone.  q, k and the decays of TT tokens are staged in LDS once for all
-// columns.
+// neighbouring lanes, R = 4 rows each, in registers for the whole step.  What bounds it is the serial chain over the tokens: a token's S^T k
+// has to be summed over the lanes before its row enters S, about 50 instructions a wave, and the grid seldom has more than one wave a SIMD to fill
+// the waits.  So: 4 rows a lane, which gives 16 heads of 128 x 128 a wave on every SIMD (8 rows leave half of the CUs idle) and 16-byte
+// LDS reads beside the neighbours' (32 bytes apart they meet in the same banks); S^T q taken of the state before the token's row
+// enters, (S + k u^T)^T q = S^T q + (k . q) u, so that both sums run side by side; q, k, decays of TT tokens staged in LDS for all columns, the
+// next tile's requested ahead of a tile's tokens; the outputs stored a tile at a time.  2048 tokens, 16 heads, delta rule (us): 470 with 8 rows a
+// lane and tiles of 16 tokens; 425 with 4 rows, 392 with stores a tile, 371 with the two sums side by side, 319 with tiles of 32 tokens, 306
+// with whole tiles requested without bounds; operands fetched further ahead than two tokens: no change.  Sums over the rows add a lane's R
+// products in order, then the P lanes: an order fixed by `dim` alone.
 // sum over the P neighbouring lanes that share a column (P a power of two, lanes aligned to P), left in all of them.  Inside a row of 16
 // lanes the partner comes by DPP (quad permutes, then mirrors of half a row and of a row: after each step the lanes of a group hold one
-// value, so a mirror is as good as an xor); beyond 16 lanes by a cross-lane read.  One fixed order for a given P.
+// value, so a mirror is as good as an xor); beyond 16 lanes by permlane swaps.  One fixed order for a given P.
 template <int P>
 __device__ __forceinline__ float group_sum(float v) {
   if (P >= 2) v += dpp_f32<0xB1>(v);    // quad_perm [1, 0, 3, 2]
   if (P >= 4) v += dpp_f32<0x4E>(v);    // quad_perm [2, 3, 0, 1]
   if (P >= 8) v += dpp_f32<0x141>(v);   // row_half_mirror
   if (P >= 16) v += dpp_f32<0x140>(v);  // row_mirror
-  if (P >= 32) v += __shfl_xor(v, 16, 64);
+  if (P >= 32) v = vra_xor16_sum(v);    // permlane swaps: the other row of 16, the other half of the wave
+  if (P >= 64) v = vra_xor32_sum(v);
   return v;
 }
 
-// P, the presence of per-row decays and of the delta rule are template parameters: the 16 tokens of a tile are one straight line of code, so
+// P, the presence of per-row decays and of the delta rule are template parameters: the tokens of a whole tile are one straight line of code, so
 // the LDS reads of the tokens ahead are in flight while a token's sums run.
 // DECAY 0: one constant per head; 1: one per row and key channel; 2: one per row and head.  ACT: q, k, v pass silu on their way into LDS.
 // BONUS (per-channel decays, no delta rule): the output is read before the decay, this token enters it through bonus (bs: sum_d q_d bonus_d k_d).
+// tokens staged at a time: the next tile's operands are requested ahead of a tile's tokens, whose time has to cover their way from memory
+constexpr int scan_tile(int dimP) { return dimP > 128 ? 16 : 32; }
 template <int R, int P, int DECAY, bool BETA, bool ACT, bool BONUS = false>
 __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
-  constexpr int TT = 16, NL = 4;     // tokens a tile; 16-byte loads a thread and array for one tile (TT * dimP / 4 / 256, dimP <= 256)
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  constexpr int dimP = P * R, CPB = 256 / P, d4n = dimP / 4;
+  constexpr int dimP = P * R, CPB = 256 / P, d4n = dimP / 4, TT = scan_tile(dimP), NL = (TT * d4n + 255) / 256;  // tokens a tile; 16-byte loads a thread and array for one
+  static_assert(d4n == P, "the lanes that stage a token's row are as many as those that hold a column");
   const int dim = a.dim, vdim = a.vdim;
   float* ks = lds;                   // [TT][dimP]
   float* qs = ks + TT * dimP;        // [TT][dimP]
@@ -747,6 +756,8 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
   float* vs = ds + TT * dimP;        // [TT][CPB]
   float* bs = vs + TT * CPB;         // [TT]
   float* gs = bs + TT;               // [TT] one decay per token (DECAY 2)
+  float* cs = gs + TT;               // [TT] k . (q_scale q)
+  float* os = cs + TT;               // [TT][CPB] the tile's outputs
   const int b = blockIdx.z, h = blockIdx.y, hq = h / a.qk_rep, tid = threadIdx.x;
   const int slot = a.state_slots[b];
   if (slot < 0) return;
@@ -771,8 +782,8 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
   // A tile's q, k, decays, values and write strengths travel global memory -> registers -> LDS; the registers of the NEXT tile are requested
   // before the current tile's tokens run, so their way from memory lies beside the arithmetic.
   float4 kn[NL], qn[NL], dn[NL];
-  float vbuf[16], bn = 0.f, gn = 1.f;
-  constexpr int vcount = TT * CPB;     // values of a tile: a thread takes elements tid, tid + 256, ... (at most 16)
+  constexpr int vcount = TT * CPB, NV = (vcount + 255) / 256;  // values of a tile: a thread takes elements tid, tid + 256, ...
+  float vbuf[NV], bn = 0.f, gn = 1.f;
   auto row4 = [&](const float* base, int ld, int hh, size_t t, int d, float fill) {
     const float* p = base + t * ld + hh * dim + d;
     if (vec && d + 3 < dim) return *(const float4*)p;
@@ -780,8 +791,22 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
     o.x = d < dim ? p[0] : fill, o.y = d + 1 < dim ? p[1] : fill, o.z = d + 2 < dim ? p[2] : fill, o.w = d + 3 < dim ? p[3] : fill;
     return o;
   };
+  // A whole tile of whole 16-byte rows, the common case, is requested without a bound a load: a thread's row of the u-th load is u * RS rows on.
+  const bool plain = vec && dim == dimP && TT * P >= 256;
+  constexpr int RS = 256 / P;
+  const float* kp = a.k + (size_t)(t0 + tid / P) * a.ldk + hq * dim + tid % P * 4;
+  const float* qp = a.q + (size_t)(t0 + tid / P) * a.ldq + hq * dim + tid % P * 4;
+  const float* dp = DECAY == 1 ? a.decay + (size_t)(t0 + tid / P) * a.ldd + h * dim + tid % P * 4 : nullptr;
   auto request = [&](int i0) {
     const int nt = min(TT, n - i0);
+    if (plain && nt == TT) {
+#pragma unroll
+      for (int u = 0; u < NL; u++) {
+        kn[u] = *(const float4*)(kp + (size_t)(i0 + u * RS) * a.ldk);
+        qn[u] = *(const float4*)(qp + (size_t)(i0 + u * RS) * a.ldq);
+        if (DECAY == 1) dn[u] = *(const float4*)(dp + (size_t)(i0 + u * RS) * a.ldd);
+      }
+    } else
 #pragma unroll
     for (int u = 0; u < NL; u++) {
       const int e = tid + u * 256, i = e / d4n, d = (e % d4n) * 4;
@@ -794,7 +819,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
       }
     }
 #pragma unroll
-    for (int u = 0; u < 16; u++) {
+    for (int u = 0; u < NV; u++) {
       const int e = tid + u * 256;
       if (e < vcount) {
         const int i = e / CPB, cc = blockIdx.x * CPB + e % CPB;
@@ -818,6 +843,10 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
         qv.x *= a.q_scale, qv.y *= a.q_scale, qv.z *= a.q_scale, qv.w *= a.q_scale;
         *(float4*)(qs + e * 4) = qv;
         if (DECAY == 1) *(float4*)(ds + e * 4) = dn[u];
+        if (!BONUS) {  // (the d4n = P neighbouring lanes that hold a token's row; zeros beyond its size)
+          const float c = group_sum<P>(fmaf(kk.x, qv.x, fmaf(kk.y, qv.y, fmaf(kk.z, qv.z, kk.w * qv.w))));
+          if (e % d4n == 0) cs[e / d4n] = c;
+        }
       }
       if (BONUS) {  // the d4n neighbouring lanes that hold a token's q and k (zeros beyond its size) sum q . (bonus k)
         const float4 kk = kn[u], qv = qn[u];
@@ -828,22 +857,32 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
       }
     }
 #pragma unroll
-    for (int u = 0; u < 16; u++) {
+    for (int u = 0; u < NV; u++) {
       const int e = tid + u * 256;
       if (e < vcount) vs[e] = ACT ? siluf_(vbuf[u]) : vbuf[u];
     }
     if (BETA && tid < TT) bs[tid] = bn;
     if (DECAY == 2 && tid < TT) gs[tid] = gn;
   };
+  // A tile's outputs leave together, behind the next tile's deposit: a store a token, under a branch, would make the wait for the next tile's
+  // operands (loads and stores are counted together) a wait for every store's way to memory.
+  auto leave = [&](int i0, int nt) {
+#pragma unroll
+    for (int u = 0; u < NV; u++) {
+      const int e = tid + u * 256, i = e / CPB, cc = blockIdx.x * CPB + e % CPB;
+      if (e < vcount && i < nt && cc < vdim) a.out[(size_t)(t0 + i0 + i) * a.ldo + h * vdim + cc] = os[e];
+    }
+  };
   request(0);
   for (int i0 = 0; i0 < n; i0 += TT) {
     const int nt = min(TT, n - i0);
     __syncthreads();
     deposit();
+    if (i0 > 0) leave(i0 - TT, TT);
     __syncthreads();
     if (i0 + TT < n) request(i0 + TT);
-    // a token's operands come from LDS one token ahead of its arithmetic (two register sets, 16-byte reads)
-    float kv[2][R], qv[2][R], dv[2][R], uv[2], bv[2], gv[2];
+    // a token's operands come from LDS two tokens ahead of its arithmetic (16-byte reads): one token's work is shorter than their way
+    float kv[4][R], qv[4][R], dv[4][R], uv[4], bv[4], gv[4], cv[4];
     auto fetch = [&](int i, int w) {
 #pragma unroll
       for (int j = 0; j < R; j += 4) {
@@ -857,6 +896,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
       }
       uv[w] = vs[i * CPB + cl];
       if (BETA || BONUS) bv[w] = bs[i];
+      if (!BONUS) cv[w] = cs[i];
       if (DECAY == 2) gv[w] = gs[i];
     };
     auto token = [&](int i, int w) {
@@ -869,33 +909,32 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
           S[j] = fmaf(kv[w][j], u, S[j] * dv[w][j]), S[j + 1] = fmaf(kv[w][j + 1], u, S[j + 1] * dv[w][j + 1]);
         }
         const float o_ = fmaf(bv[w], u, group_sum<P>(o0 + o1));
-        if (r == 0 && col) a.out[(size_t)(t0 + i0 + i) * a.ldo + h * vdim + c] = o_;
+        if (r == 0) os[i * CPB + cl] = o_;
         return;
       }
 #pragma unroll
       for (int j = 0; j < R; j++) S[j] *= DECAY == 1 ? dv[w][j] : (DECAY == 2 ? gv[w] : hd);
-      float u = uv[w];
-      if (BETA) {
-        float d0 = 0.f, d1 = 0.f;  // (two chains; their sum order is fixed)
-#pragma unroll
-        for (int j = 0; j < R; j += 2) d0 = fmaf(S[j], kv[w][j], d0), d1 = fmaf(S[j + 1], kv[w][j + 1], d1);
-        u = bv[w] * (u - group_sum<P>(d0 + d1));
-      }
-      float o0 = 0.f, o1 = 0.f;
+      // S^T k and S^T q of the decayed state side by side (two chains each; their sum order is fixed): the output of the new state is
+      // (S + k u^T)^T q = S^T q + (k . q) u, so it does not wait for u, and one chain's steps fill the other's wait states
+      float u = uv[w], d0 = 0.f, d1 = 0.f, o0 = 0.f, o1 = 0.f;
 #pragma unroll
       for (int j = 0; j < R; j += 2) {
-        S[j] = fmaf(kv[w][j], u, S[j]), S[j + 1] = fmaf(kv[w][j + 1], u, S[j + 1]);
+        if (BETA) d0 = fmaf(S[j], kv[w][j], d0), d1 = fmaf(S[j + 1], kv[w][j + 1], d1);
         o0 = fmaf(S[j], qv[w][j], o0), o1 = fmaf(S[j + 1], qv[w][j + 1], o1);
       }
-      const float o_ = group_sum<P>(o0 + o1);
-      if (r == 0 && col) a.out[(size_t)(t0 + i0 + i) * a.ldo + h * vdim + c] = o_;
+      if (BETA) u = bv[w] * (u - group_sum<P>(d0 + d1));
+#pragma unroll
+      for (int j = 0; j < R; j++) S[j] = fmaf(kv[w][j], u, S[j]);
+      const float o_ = fmaf(cv[w], u, group_sum<P>(o0 + o1));
+      if (r == 0) os[i * CPB + cl] = o_;
     };
-    fetch(0, 0);
     if (nt == TT) {
+      fetch(0, 0);
+      fetch(1, 1);
 #pragma unroll
       for (int i = 0; i < TT; i++) {
-        if (i + 1 < TT) fetch(i + 1, (i + 1) & 1);
-        token(i, i & 1);
+        if (i + 2 < TT) fetch(i + 2, (i + 2) & 3);
+        token(i, i & 3);
       }
     } else {
       for (int i = 0; i < nt; i++) {
@@ -904,6 +943,8 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
       }
     }
   }
+  __syncthreads();
+  if (n > 0) leave((n - 1) / TT * TT, (n - 1) % TT + 1);
   if (col)
 #pragma unroll
     for (int j = 0; j < R; j++)
@@ -1207,11 +1248,12 @@ void vra_stack_sigmoid_pow(const float* z, int ldz, float* out, int ldo, int T, 
 void vra_stack_linear_scan(const StkScanArgs& a, int64_t stream) {
   VRA_CHECK_ARG(a.q && a.k && a.v && a.state && a.state_slots && a.positions && a.out && (a.decay || a.head_decay), "stack linear scan: null pointer");
   VRA_CHECK_ARG(a.B > 0 && a.H > 0 && a.qk_rep >= 1 && a.H % a.qk_rep == 0 && a.dim > 0 && a.dim <= 256 && a.vdim > 0, "stack linear scan: key size at most 256");
-  constexpr int R = 8;
+  constexpr int R = 4;
   int P = 1;
   while (P * R < a.dim) P <<= 1;
   const int CPB = 256 / P, dimP = P * R;
-  const size_t lds = ((size_t)16 * dimP * 3 + (size_t)16 * CPB + 32) * sizeof(float);
+  const int TT = scan_tile(dimP);
+  const size_t lds = ((size_t)TT * dimP * 3 + (size_t)2 * TT * CPB + 3 * TT) * sizeof(float);
   dim3 grid((a.vdim + CPB - 1) / CPB, a.H, a.B);
   hipStream_t st = as_stream(stream);
   const bool decay = a.decay != nullptr, beta = a.beta != nullptr, per_head = decay && a.decay_per_head;
@@ -1234,7 +1276,8 @@ void vra_stack_linear_scan(const StkScanArgs& a, int64_t stream) {
     case 4: STK_SCAN(4); break;
     case 8: STK_SCAN(8); break;
     case 16: STK_SCAN(16); break;
-    default: STK_SCAN(32); break;
+    case 32: STK_SCAN(32); break;
+    default: STK_SCAN(64); break;
   }
 #undef STK_SCAN
 }
