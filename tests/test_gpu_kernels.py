@@ -185,6 +185,58 @@ def test_gate_up_silu_143_to_221_rows_at_the_llama3_8b_widths(M):
     assert float((got != ref).mean()) <= 0.04
 
 
+# ---------------------------------------------------------------- kernel M (33 rows up: short and middle prompts)
+# Few columns, where kernel W does not take the launch: blocks of 64 / 96 / 128 / 160 rows and two row blocks, whole and ragged; a column tile with
+# missing n-blocks (272 = 17 blocks); K in one piece and in slices, 37 k-tiles in uneven ones whose row sums are read one by one.  The kernel sums
+# (C + q) x in float32 (C 128 or 64, q < 16) and takes (C + z) sum x off at the end: a few float32 roundings of the largest partial sum are the floor.
+@pytest.mark.parametrize("M", [64, 65, 97, 150, 161, 200])
+@pytest.mark.parametrize("K,N", [(512, 272), (4608, 512), (4736, 64)])
+@pytest.mark.parametrize("dt,awq,gs", [(BF16, False, 128), (F16, False, 128), (BF16, True, 128), (F16, True, -1), (BF16, False, 256)])
+def test_wna16_gemm_middle_rows(dt, awq, gs, K, N, M):
+    if gs > 0 and K % gs:
+        pytest.skip("K is not a multiple of the group")
+    r = rng(M * 3 + K + N + dt + awq + gs)
+    q = make_quant(r, K, N, gs, dt, awq)
+    x, bias, res = rand_dt(r, (M, K), dt), rand_dt(r, (N,), dt), rand_dt(r, (M, N), dt)
+    tiled = ops.marlin_weight_repack(ops.dev(q["qweight"]), q["qweight"].shape, 4, awq)
+    qz = ops.dev(q["qzeros"]) if awq else None
+    sums = np.abs(orc.from_dt(x, dt)).sum(1).max() * np.abs(orc.from_dt(q["scales"], dt)).max()
+    floor = float(4 * 2.0 ** -24 * (144 if dt == BF16 else 80) * sums)
+    out = ops.wna16_gemm(ops.dev(x), tiled, ops.dev(q["scales"]), qz, M, K, N, gs, awq, 0, None, None, dt)
+    ref = orc.wna16_gemm(x, q["idx"], q["zeros"] if awq else None, q["scales"], gs, dt)
+    assert_close_dt(out.numpy(np.uint16, (M, N)), ref, dt, name="kernel M", abs_floor=floor)
+    out = ops.wna16_gemm(ops.dev(x), tiled, ops.dev(q["scales"]), qz, M, K, N, gs, awq, 0, ops.dev(bias), ops.dev(res), dt)
+    ref2 = orc.wna16_gemm(x, q["idx"], q["zeros"] if awq else None, q["scales"], gs, dt, bias, res)
+    g0 = orc.from_dt(ref, dt)
+    mag = np.maximum(np.abs(g0), np.abs(g0 + orc.from_dt(bias, dt)[None, :]))
+    # (three roundings, each of which may land on the neighbouring value)
+    assert_close_dt(out.numpy(np.uint16, (M, N)), ref2, dt, max_ulp=3.0, name="kernel M bias + residual", mag=mag, abs_floor=floor)
+    assert ops.lib().vra_take_device_error() == 0
+
+
+@pytest.mark.parametrize("dt,awq", [(BF16, False), (F16, False), (BF16, True)])
+@pytest.mark.parametrize("M,K,N", [(70, 512, 272), (128, 4608, 64), (150, 4736, 208), (200, 640, 272)])
+def test_gate_up_silu_middle_rows(dt, awq, M, K, N):
+    r = rng(M * 5 + K + N + dt + awq)
+    qg, qu = make_quant(r, K, N, 128, dt, awq), make_quant(r, K, N, 128, dt, awq)
+    x = rand_dt(r, (M, K), dt)
+    tg = ops.marlin_weight_repack(ops.dev(qg["qweight"]), qg["qweight"].shape, 4, awq)
+    tu = ops.marlin_weight_repack(ops.dev(qu["qweight"]), qu["qweight"].shape, 4, awq)
+    zg, zu = (ops.dev(qg["qzeros"]), ops.dev(qu["qzeros"])) if awq else (None, None)
+    out = ops.wna16_gate_up_silu(ops.dev(x), tg, ops.dev(qg["scales"]), zg, tu, ops.dev(qu["scales"]), zu, M, K, N, 128, awq, dtype=dt)
+    g = orc.wna16_gemm(x, qg["idx"], qg["zeros"] if awq else None, qg["scales"], 128, dt)
+    u = orc.wna16_gemm(x, qu["idx"], qu["zeros"] if awq else None, qu["scales"], 128, dt)
+    ref = orc.silu_mul(g, u, dt)
+    # one ulp of gate through silu' (and half an ulp of the re-rounded silu), one ulp of up, 1.5 ulp of the product; the floor as above, through up
+    gf, uf = orc.from_dt(g, dt).astype(np.float64), orc.from_dt(u, dt).astype(np.float64)
+    sg = 1.0 / (1.0 + np.exp(-gf))
+    tol = (ulp_of(gf, dt) * np.abs(sg * (1.0 + gf * (1.0 - sg))) + 0.5 * ulp_of(gf * sg, dt)) * np.abs(uf) + ulp_of(uf, dt) * np.abs(gf * sg) + 1.5 * ulp_of(orc.from_dt(ref, dt), dt)
+    sums = np.abs(orc.from_dt(x, dt)).sum(1).max() * max(np.abs(orc.from_dt(z["scales"], dt)).max() for z in (qg, qu))
+    floor = 4 * 2.0 ** -24 * (144 if dt == BF16 else 80) * sums * (1.1 * np.abs(uf) + np.abs(gf * sg))
+    diff = np.abs(orc.from_dt(out.numpy(np.uint16, (M, N)), dt).astype(np.float64) - orc.from_dt(ref, dt))
+    assert (diff <= 1.0001 * tol + floor).all(), float((diff / (tol + floor)).max())
+
+
 @pytest.mark.parametrize("gs,with_g_idx", [(128, True), (64, True), (64, False), (32, False), (128, False)])
 def test_gemm_half_q_half_alt(gs, with_g_idx):
     """the non-Marlin GPTQ path (gptq.rs:181-198): asymmetric zeros (stored z-1), groups from g_idx — or, without it, from the

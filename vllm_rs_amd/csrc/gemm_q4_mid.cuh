@@ -1,0 +1,368 @@
+// gemm_q4_mid.cuh — "kernel M": int4 GEMM for 33 rows up (short and middle prompts), every row of a block of up to 160 in one workgroup.
+//
+// What bounds a short prompt's int4 product is not memory (the codes of a gate/up pair of 4096 x 14336 take 13 us) but converting the codes: a
+// matrix instruction and a conversion take their SUM on a SIMD, also from different waves (tools/mfma_valu_probe.hip), and the kernels of 32- or
+// 64-row tiles convert every code once per row block.  Here a workgroup owns 128 virtual columns (64 gate + 64 up of a pair) and ALL rows of
+// the block, 32 MB of them (MB 2..5): 8 waves as 4 (columns, two n-blocks each) x 2 (rows, MB m-tiles each), so a code is converted twice for up to
+// 160 rows, and a k-tile's 8 MB MFMAs of a wave are 2 MB independent chains.  x, codes and scales of a k-tile of 128 travel by LDS-DMA through a
+// ring of three stages (one barrier a k-tile); the 16-byte chunks of an x row lie at slot chunk ^ (row mod 16), so the fragment reads meet no bank
+// twice.  Two n-blocks a wave read each x fragment from LDS four times a workgroup: 160 KB a k-tile at MB = 5, 1280 cycles beside 1380 of MFMAs
+// and 500 of conversions on each SIMD; four n-blocks a wave would halve that and double the conversions.
+//
+// The zero points stay out of the k loop for every type and format: acc += s_g acc_g inside, and behind it
+//     acc -= sum_g (C + z_g) s_g[n] . Sx_g[m],
+// a small product over the k-tiles on the matrix cores.  w = (C + z) s is exact in float32 (11 + 8 bits) and goes in as three bf16 pieces (24
+// bits), the float32 row sums Sx (xsum_rows_kernel, or the norm's launch) as three as well; the six products of pieces down to 2^-16 of the
+// largest are kept (the three left out are below 2^-24 of it).
+//
+// Few columns leave the chip idle: K is then split over gridDim.z, with the exchange of kernel D (slabs written through, a flag line a slice;
+// only the last slice, whose workgroups start last, waits, and adds the slabs in slice order).
+#pragma once
+#include "gemm_q4_big.cuh"  // GemmDArgs
+
+#define GM_THREADS 512
+static inline size_t gemm_q4_mid_lds_bytes(int mb) { return (size_t)3 * (32 * mb * 256 + 8 * 1024 + 8 * 256); }
+
+template <class DT, bool DUAL, int MB>
+__global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs a, int awq) {
+#ifdef __HIP_DEVICE_COMPILE__
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr int NB = 2, ROWS = 32 * MB, XB = ROWS * 256, WB = 8 * 1024, SB = 8 * 256, STG = XB + WB + SB, PER = MB + 2;
+  constexpr uint32_t RSRC3 = 0x00020000u;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nn = lane & 15, oct = lane >> 4, wn = wave & 3, wm = wave >> 2;
+  const int K = a.K, M = a.M, KT = K >> 7;
+  const bool grouped = a.group_size > 0 && a.group_size < K;
+  const int gsh = grouped ? 31 - __builtin_clz(a.group_size) : 31;
+  const int m0 = (int)blockIdx.y * ROWS;
+
+  // ---- the wave's two n-blocks: DUAL, block nb0 of gate and of up; else blocks nb0, nb0 + 1 of one tensor (segments are whole 64 columns)
+  const void* wt[2] = {a.w0, DUAL ? a.w1 : a.w0};
+  const void* sct[2] = {a.sc0, DUAL ? a.sc1 : a.sc0};
+  const uint32_t* qzt[2] = {a.qz0, DUAL ? a.qz1 : a.qz0};
+  const void* biast[2] = {a.bias0, a.bias1};
+  void* outp = a.out;
+  int N = a.N, out_ld = a.out_ld, nb0;
+  if (DUAL) {
+    nb0 = (int)blockIdx.x * 4 + wn;
+  } else {
+    nb0 = (int)blockIdx.x * 8 + wn * 2;
+    if (a.nseg > 1) {
+      const int s = (a.nseg > 2 && nb0 >= a.xseg[1].blk_start) ? 1 : (nb0 >= a.xseg[0].blk_start ? 0 : -1);
+      if (s >= 0) {
+        const GemvSeg& sg = a.xseg[s];
+        wt[0] = wt[1] = sg.w, sct[0] = sct[1] = sg.scales, qzt[0] = qzt[1] = sg.qzeros, biast[0] = sg.bias, outp = sg.out, N = sg.n, out_ld = sg.out_ld;
+        nb0 -= sg.blk_start;
+      }
+    }
+  }
+  bool ok[NB];
+  int nbc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    const int nb = nb0 + (DUAL ? 0 : b);
+    ok[b] = nb * 16 < N;
+    nbc[b] = ok[b] ? nb : 0;  // (a missing block streams block 0; its results are never stored)
+  }
+  // this workgroup's k-tiles: all of them, or slice blockIdx.z of a.splitk
+  const int SK = a.splitk > 1 ? a.splitk : 1, zi = (int)blockIdx.z;
+  const int kt0 = (int)((long)KT * zi / SK), kt1 = (int)((long)KT * (zi + 1) / SK);
+
+  // ---- DMA sources.  A wave fetches MB KiB of x (4 rows each), the codes of its block wm (the other wave of the column pair the other's),
+  // and its own copy of its two blocks' scales (lanes 0..15; the rest fetch the same again)
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, 0x7FFFFFF0, RSRC3);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(wm ? wt[1] : wt[0]), 0, 0x7FFFFFF0, RSRC3);
+  uint32_t vo_x[MB];
+#pragma unroll
+  for (int i = 0; i < MB; i++) {
+    const int row = (wave * MB + i) * 4 + oct;
+    vo_x[i] = ((uint32_t)min(m0 + row, M - 1) * (uint32_t)a.x_ld + (uint32_t)(nn ^ (row & 15)) * 8u) * 2u;  // rows >= M alias row M - 1 (never stored)
+  }
+  const uint32_t vo_w = (uint32_t)lane * 16u, so_w = (uint32_t)(wm ? nbc[1] : nbc[0]) * (uint32_t)KT;
+  typedef const __attribute__((address_space(1))) void* glb_ptr;
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  const unsigned char* sc_src = static_cast<const unsigned char*>((lane & 8) ? sct[1] : sct[0]) + (((lane & 8) ? nbc[1] : nbc[0]) * 32 + (lane & 7) * 4);
+  auto request = [&](int kt) {
+    unsigned char* const d = smem + ((kt - kt0) % 3) * STG;
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(d + (wave * MB + i) * 1024), 16, vo_x[i], (uint32_t)kt * 256u, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(d + XB + (2 * wn + wm) * 1024), 16, vo_w, (so_w + (uint32_t)kt) * 1024u, 0, 2);  // nt
+    const int grp = grouped ? (kt * 128) >> gsh : 0;
+    __builtin_amdgcn_global_load_lds((glb_ptr)(sc_src + (size_t)grp * N * 2), (lds_ptr)(d + XB + WB + wave * 256), 4, 0, 0);
+  };
+
+  f32x4 acc[NB][MB];
+#pragma unroll
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int t = 0; t < MB; t++) acc[b][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int xrow = (wm * MB * 16 + nn) * 256;
+  u32x4 wq[NB], xf[2][MB];
+  u32x2 scw[NB];
+  auto read_w = [&](int kt) {
+    const unsigned char* const st = smem + ((kt - kt0) % 3) * STG + XB;
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      wq[b] = *reinterpret_cast<const u32x4*>(st + (2 * wn + b) * 1024 + lane * 16);
+      scw[b] = *reinterpret_cast<const u32x2*>(st + WB + wave * 256 + b * 32 + oct * 8);
+    }
+  };
+  auto read_x = [&](int kt, int j) {
+    const unsigned char* const st = smem + ((kt - kt0) % 3) * STG + xrow + (((j * 4 + oct) ^ nn) * 16);
+#pragma unroll
+    for (int t = 0; t < MB; t++) xf[j & 1][t] = *reinterpret_cast<const u32x4*>(st + t * 4096);
+  };
+  // Three stages in flight; stage kt + 1 is waited for before the LAST fragments' MFMAs of tile kt, so its first reads, the barrier's skew and the
+  // next requests (into the buffer of tile kt, whose last fragments are in registers by then) lie beside them.
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+    if (kt0 + i < kt1) request(kt0 + i);
+  auto arrive = [&](int kt) {  // stage kt is here: this wave's own requests are, and the barrier says the same of the other waves'
+    if (kt + 1 < kt1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER) : "memory");  // (at most stage kt + 1 is still on its way)
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (kt0 + 2 < kt1) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER) : "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  } else {
+    arrive(kt0);
+  }
+  read_w(kt0);
+  read_x(kt0, 0);
+  for (int kt = kt0; kt < kt1; kt++) {
+    f32x4 ag[NB][MB];
+    s16x8 af[2][NB];
+    u32x2 scc[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) af[0][b] = magic_word<DT>(wq[b][0]), scc[b] = scw[b];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if (j == 3 && kt + 1 < kt1) {
+        arrive(kt + 1);
+        if (kt + 3 < kt1) request(kt + 3);
+      }
+#pragma unroll
+      for (int t = 0; t < MB; t++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+          if (j == 0) DT::mfma0(ag[b][t], af[0][b], __builtin_bit_cast(s16x8, xf[0][t]));
+          else DT::mfma(ag[b][t], af[j & 1][b], __builtin_bit_cast(s16x8, xf[j & 1][t]));
+          if (t == 0 && b == 0) {  // (behind the wait for fragment j: fragment j + 1 is not part of it)
+            __builtin_amdgcn_sched_barrier(0);
+            if (j < 3) read_x(kt, j + 1);
+            else if (kt + 1 < kt1) read_w(kt + 1), read_x(kt + 1, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (j < 3 && t == 1) af[(j + 1) & 1][b] = magic_word<DT>(wq[b][j + 1]);
+        }
+    }
+    VRA_MFMA_DRAIN();
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      const float s0 = DT::to_f32((uint16_t)(scc[b][0] & 0xffffu)), s1 = DT::to_f32((uint16_t)(scc[b][0] >> 16));
+      const float s2 = DT::to_f32((uint16_t)(scc[b][1] & 0xffffu)), s3 = DT::to_f32((uint16_t)(scc[b][1] >> 16));
+#pragma unroll
+      for (int t = 0; t < MB; t++) {
+        acc[b][t][0] = fmaf(s0, ag[b][t][0], acc[b][t][0]), acc[b][t][1] = fmaf(s1, ag[b][t][1], acc[b][t][1]);
+        acc[b][t][2] = fmaf(s2, ag[b][t][2], acc[b][t][2]), acc[b][t][3] = fmaf(s3, ag[b][t][3], acc[b][t][3]);
+      }
+    }
+  }
+
+  // ---- the zero points of this workgroup's k-tiles, 32 tiles a step: A, lane (column nn, octet oct) holds (C + z) s of tiles t0 + 8 oct .. + 7 (zero
+  // outside [kt0, kt1)); B, lane (row nn of the m-tile, oct) the row sums of those tiles.  Each block's and m-tile's pieces are made by one wave and
+  // meet the others in the ring's memory (made by every wave that needs them: 11 us a launch at 150 rows).
+  auto split3 = [&](const float (&v)[8], unsigned char* to) {  // hi + mid + lo bf16 pieces, a KiB each
+    u32x4 q[3];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      uint32_t h[2], m[2], l[2];
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        const float x = v[2 * i + c];
+        const uint32_t hb = __float_as_uint(x) & 0xffff0000u;  // (truncated: the rest is exact)
+        const float r1 = x - __uint_as_float(hb);
+        const uint32_t mb = __float_as_uint(r1) & 0xffff0000u;
+        h[c] = hb >> 16, m[c] = mb >> 16, l[c] = (uint32_t)BF16::from_f32(r1 - __uint_as_float(mb));
+      }
+      q[0][i] = h[0] | (h[1] << 16), q[1][i] = m[0] | (m[1] << 16), q[2][i] = l[0] | (l[1] << 16);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4*>(to + i * 1024 + lane * 16) = q[i];
+  };
+  constexpr int MT = 2 * MB, XI = (MT + 7) / 8;  // m-tiles of the workgroup; of a wave
+  static_assert((8 + MT) * 3072 <= 3 * STG, "the pieces fit the ring");
+  for (int t0 = kt0 & ~3; t0 < kt1; t0 += 32) {
+    const int tb = t0 + oct * 8;
+    uint16_t sr[8];
+    uint32_t zr[8];
+    f32x4 sv[XI][2];
+    const int col = (wm ? nbc[1] : nbc[0]) * 16 + nn;
+    const uint16_t* const sp = static_cast<const uint16_t*>(wm ? sct[1] : sct[0]) + col;
+#pragma unroll
+    for (int e = 0; e < 8; e++) sr[e] = sp[(size_t)(grouped ? (min(tb + e, KT - 1) * 128) >> gsh : 0) * N];
+    if (awq) {
+      const uint32_t* const zp = (wm ? qzt[1] : qzt[0]) + (col >> 3);
+#pragma unroll
+      for (int e = 0; e < 8; e++) zr[e] = zp[(size_t)(grouped ? (min(tb + e, KT - 1) * 128) >> gsh : 0) * (N >> 3)] >> (4 * awq_rev(nn & 7));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; e++) zr[e] = 8u;
+    }
+#pragma unroll
+    for (int u = 0; u < XI; u++) {
+      const float* const xr = a.xsum + (size_t)min(m0 + min(wave + 8 * u, MT - 1) * 16 + nn, M - 1) * KT;
+      if (KT % 4 == 0) {
+        sv[u][0] = *reinterpret_cast<const f32x4*>(xr + min(tb, KT - 4)), sv[u][1] = *reinterpret_cast<const f32x4*>(xr + min(tb + 4, KT - 4));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) sv[u][e >> 2][e & 3] = xr[min(tb + e, KT - 1)];
+      }
+    }
+    __syncthreads();  // (nobody reads the ring, or the step before, any more)
+    float w[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) w[e] = tb + e >= kt0 && tb + e < kt1 ? (Magic<DT>::bias + (float)(zr[e] & 0xFu)) * DT::to_f32(sr[e]) : 0.f;
+    split3(w, smem + (2 * wn + wm) * 3072);
+#pragma unroll
+    for (int u = 0; u < XI; u++)
+      if (wave + 8 * u < MT) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) w[e] = sv[u][e >> 2][e & 3];
+        split3(w, smem + (8 + wave + 8 * u) * 3072);
+      }
+    __syncthreads();
+    s16x8 wp[NB][3];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int i = 0; i < 3; i++) wp[b][i] = *reinterpret_cast<const s16x8*>(smem + (2 * wn + b) * 3072 + i * 1024 + lane * 16);
+#pragma unroll
+    for (int mt = 0; mt < MB; mt++) {
+      s16x8 xp[3];
+#pragma unroll
+      for (int i = 0; i < 3; i++) xp[i] = *reinterpret_cast<const s16x8*>(smem + (8 + wm * MB + mt) * 3072 + i * 1024 + lane * 16);
+      f32x4 zt[NB];
+#pragma unroll
+      for (int b = 0; b < NB; b++) BF16::mfma0(zt[b], wp[b][2], xp[0]);  // smallest pieces first
+#pragma unroll
+      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][1], xp[1]);
+#pragma unroll
+      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][0], xp[2]);
+#pragma unroll
+      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][1], xp[0]);
+#pragma unroll
+      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][0], xp[1]);
+#pragma unroll
+      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][0], xp[0]);
+      VRA_MFMA_DRAIN();
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[b][mt][r] -= zt[b][r];
+    }
+  }
+
+  // ---- split K: kernel D's exchange
+  if (SK > 1) {
+    const int tile = (int)(blockIdx.y * gridDim.x + blockIdx.x), ntiles = (int)(gridDim.x * gridDim.y);
+    const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(a.slabs, 0, 0x7FFFFFF0, RSRC3);
+    auto slab_off = [&](int z, int b, int mt) { return (uint32_t)((((z * ntiles + tile) * NB + b) * MB + mt) * GM_THREADS + tid) * 16u; };
+    uint32_t* fl = a.counters + (size_t)tile * SK * 16;
+    if (zi != SK - 1) {
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int mt = 0; mt < MB; mt++) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[b][mt]), srs, slab_off(zi, b, mt), 0, 16);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // write-through stores: acknowledged by memory
+      __syncthreads();
+      if (tid == 0) __hip_atomic_store(fl + zi * 16, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+    if (tid < SK - 1) {
+      const uint64_t c0 = __builtin_readcyclecounter();
+      while (__hip_atomic_load(fl + tid * 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
+        __builtin_amdgcn_s_sleep(1);
+        if (__builtin_readcyclecounter() - c0 > (1ull << 31)) {  // never hang the device on a lost slice
+          __hip_atomic_store(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          break;
+        }
+      }
+      __hip_atomic_store(fl + tid * 16, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    // a slab's 2 MB loads a lane are requested one slab ahead of their sum; slice order
+    u32x4 p[2][NB][MB];
+    auto fetch = [&](int z, u32x4 (&d)[NB][MB]) {
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int mt = 0; mt < MB; mt++) d[b][mt] = __builtin_amdgcn_raw_buffer_load_b128(srs, slab_off(z, b, mt), 0, 16);
+    };
+    auto add = [&](const u32x4 (&d)[NB][MB]) {
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int mt = 0; mt < MB; mt++) acc[b][mt] += __builtin_bit_cast(f32x4, d[b][mt]);
+    };
+    fetch(0, p[0]);
+    for (int z = 0; z < SK - 1; z += 2) {
+      fetch(min(z + 1, SK - 2), p[1]);
+      __builtin_amdgcn_sched_barrier(0);
+      add(p[0]);
+      fetch(min(z + 2, SK - 2), p[0]);
+      __builtin_amdgcn_sched_barrier(0);
+      if (z + 1 < SK - 1) add(p[1]);
+    }
+  }
+
+  // ---- epilogue: column oct * 4 + r of the block, row nn of the m-tile
+#pragma unroll
+  for (int b = 0; b < (DUAL ? 1 : NB); b++) {
+    if (!ok[b]) continue;
+    const int n = nbc[b] * 16 + oct * 4;
+    auto four = [&](const void* p, size_t at, float (&f)[4]) {
+      const u32x2 v = *reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(p) + at);
+      f[0] = DT::to_f32((uint16_t)(v[0] & 0xffffu)), f[1] = DT::to_f32((uint16_t)(v[0] >> 16));
+      f[2] = DT::to_f32((uint16_t)(v[1] & 0xffffu)), f[3] = DT::to_f32((uint16_t)(v[1] >> 16));
+    };
+    float bs[4] = {0.f, 0.f, 0.f, 0.f}, bs2[4] = {0.f, 0.f, 0.f, 0.f};
+    if (biast[0]) four(biast[0], n, bs);
+    if (DUAL && biast[1]) four(biast[1], n, bs2);
+#pragma unroll
+    for (int mt = 0; mt < MB; mt++) {
+      const int m = m0 + wm * (MB * 16) + mt * 16 + nn;
+      if (m >= M) continue;
+      float v[4], rs[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        float t = rnd_dt<DT>(acc[b][mt][r]);
+        if (biast[0]) t = rnd_dt<DT>(t + bs[r]);
+        if (DUAL) {
+          float u = rnd_dt<DT>(acc[1][mt][r]);
+          if (biast[1]) u = rnd_dt<DT>(u + bs2[r]);
+          t = rnd_dt<DT>(t / (1.0f + expf(-t))) * u;
+        }
+        v[r] = t;
+      }
+      if (a.residual) {
+        four(a.residual, (size_t)m * a.res_ld + n, rs);
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = rnd_dt<DT>(v[r]) + rs[r];
+      }
+      if (a.out_f32) {
+        const f32x4 o = {rnd_dt<DT>(v[0]), rnd_dt<DT>(v[1]), rnd_dt<DT>(v[2]), rnd_dt<DT>(v[3])};
+        *reinterpret_cast<f32x4*>(static_cast<float*>(outp) + (size_t)m * out_ld + n) = o;
+      } else {
+        const u32x2 o = {DT::pack2(v[0], v[1]), DT::pack2(v[2], v[3])};
+        *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(outp) + (size_t)m * out_ld + n) = o;
+      }
+    }
+  }
+#endif
+}

@@ -463,7 +463,7 @@ static void gemv_w_plan(int ns, int M, int n_units, bool plain, int* grid, int* 
 }
 // K > 4096 (down_proj, 5..32 rows): kz K slices of at most 32 k-tiles (what 8 waves hold as x fragments), kz_groups = CUs / kz
 // unit groups; workgroup (z, g) = blockIdx.x z * groups + g — the owners (z = kz - 1) carry the highest ids and start last
-// Round 4 (last part): 33..128 rows (down_proj of short prefills) as `rb` row blocks of 32 rows in blockIdx.y, each with its own slabs
+// 33..96 and 129..160 rows (down_proj of short prefills) as `rb` row blocks of 32 rows in blockIdx.y, each with its own slabs
 // and flags; groups = CUs / (kz * rb), so the whole launch is still one round of workgroups
 static int gemv_w_kz_max_rows() {
   static int v = -1;
@@ -494,9 +494,8 @@ bool vra_gemv_w_fits(int ns, int M, int K, int group_size, int n_units, bool has
     if (g < K && (g < 128 || (g & (g - 1)))) return false;
     int kz, ktz, groups;
     const int rb = (M + 31) / 32;
-    // which row counts: measured against kernel D (+ its row-sum pass) on the Llama-3-8B down projection, us per launch
-    // (profiles/r04_ab_kernel_w_k_slices_row_blocks.txt): 64 rows 38.6 -> 25.5, 96 rows 49.3 -> 36.4, 160 rows 77.7 -> 50.9 — but
-    // 128 rows 36.4 -> 39.6 and 200 rows 57.0 -> 65.6 (two / four full 64-row tiles per column block are kernel D's good cases)
+    // which row counts: a row of such a launch is the same row of a 32-row launch, bit for bit, so where the launch is near the others it stays
+    // (Llama-3-8B down projection, us, here / kernel M: 64 rows 25.5 / 25.6, 96 rows 35 / 31, 150 rows 50 / 42; 128 rows 40 / 36, 200 rows 66 / 48)
     static const char* any_rb = getenv("VRA_GEMV_W_KZ_ANY_RB");  // tuning aid: 1 = every row-block count up to the row limit
     if (rb > 3 && rb != 5 && !(any_rb && any_rb[0] == '1')) return false;
     if (!gemv_w_kz_plan(K, n_units, rb, &kz, &ktz, &groups)) return false;
@@ -506,7 +505,8 @@ bool vra_gemv_w_fits(int ns, int M, int K, int group_size, int n_units, bool has
     return gemv_q4w_lds_bytes(1, mt, mu, has_res, true) <= (size_t)kMaxDynLds;
   }
   static const char* pair_env = getenv("VRA_GEMV_W_PAIR_MAX_ROWS");  // tuning aid: 16 puts 17+-row gate/up launches back on kernels C / D
-  const int pair_max = pair_env ? atoi(pair_env) : gemv_w_max_rows();
+  // (pairs: 64 rows 37.1 us / kernel M 36.9, 96 rows 50 / 42, 128 rows 59 / 48, Llama-3-8B with the norm's launch)
+  const int pair_max = pair_env ? atoi(pair_env) : 64;
   if (M < 5 || M > (ns == 1 ? gemv_w_max_rows() : (pair_max > 16 ? pair_max : 16)) || K % 128 || K > 4096) return false;
   const int g = group_size > 0 && group_size < K ? group_size : K;
   if (g < K && (g < 128 || (g & (g - 1)))) return false;
@@ -743,7 +743,8 @@ void vra_launch_skinny(GemmBArgs a, bool int4, bool dual, int dtype, int64_t str
 }
 
 // ---- kernel D launcher
-int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs) {
+static const int kMidPlan = 1 << 24;  // vra_gemm_q4_big_fits: the rest is kernel M's plan
+int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, int dtype) {
   static const char* off = getenv("VRA_NO_KERNEL_D");  // tuning aid
   if (off && atoi(off)) return 0;
   if (M < 64 || K % 128 || cols % 16) return 0;
@@ -764,12 +765,18 @@ int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, cons
   // e.g. M = 512: o 50.9 (B) / 39.8 (D, mb 2) / 58.3 (mb 4); down 143 / 117 / 180; gate/up 169 (mb 4) / 189 (mb 2).
   const int gx = dual ? (cols + 127) / 128 : (cols + 255) / 256;
   const int cus = num_cus();
+  static const char* mid_env = getenv("VRA_NO_KERNEL_M");  // tuning aid
+  const bool mid_off = mid_env && mid_env[0] == '1';
   if (mb_env && (atoi(mb_env) == 2 || atoi(mb_env) == 4) && !getenv("VRA_GD_SPLITK")) return atoi(mb_env);
   const double kf = (double)K / 4096.0;
+  // (those are the times without the zero points' hoisting; gate/up of Llama-3-8B in bf16 with symmetric codes at 200..760 rows, us: 76 / 134 / 150 / 219
+  // for 2 / 3 / 4 / 6 workgroups of 64 rows a CU; with zero points, Qwen2-7B: 95 / 125 + 15 / 272 for 2 / 3 / 5, and 88 for 3 of 32 rows)
+  const bool hoisted = !awq && dtype == VRA_BF16;
+  const double pair4 = hoisted ? 68.0 : 97.0, lone4 = hoisted ? 47.0 : 55.0, pair2 = hoisted ? 46.0 : 52.0, lone2 = hoisted ? 28.0 : 31.0;
   auto est_d = [&](int mb) {
     const long w = (long)gx * ((M + 16 * mb - 1) / (16 * mb));
     const long q = (w + cus - 1) / cus;
-    const double pair = mb == 4 ? 82.0 : 46.0, lone = mb == 4 ? 47.0 : 28.0;
+    const double pair = mb == 4 ? pair4 : pair2, lone = mb == 4 ? lone4 : lone2;
     // (round 6: the gate/up pair on 32-row tiles runs ~15 % behind this model above 256 rows — 320 rows: 152 us against the 64-row tiles' 142,
     // profiles/r06_llama_midm_gemm_shapes.txt)
     const double pen = dual && mb == 2 && M > 256 ? 1.15 : 1.0;
@@ -805,12 +812,15 @@ int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, cons
           continue;
         }
         const long q = (tiles * S + cus - 1) / cus;
-        const double pair = mb == 4 ? 82.0 : 46.0, lone = mb == 4 ? 47.0 : 28.0;
+        const double pair = mb == 4 ? pair4 : pair2, lone = mb == 4 ? lone4 : lone2;
         const double body = ((double)(q / 2) * pair + (double)(q % 2) * lone) * kf / S;
         const double est = 15.0 + 3.0 + body + 6.0 + (mb == 4 ? 0.5 : 0.25) * (S - 1);
         if (est < best) best = est, pick = mb | (S << 8);
       }
   }
+  double mid_us = 0.0;
+  if (const int plan = vra_gemm_q4_mid_plan(dual, M, cols, K, group_size, segs, &mid_us))  // kernel M, by its own estimate
+    if (mid_us < best && !mid_off) return plan | kMidPlan;
   return pick;
 }
 template <class DT, bool DUAL, int MB>
@@ -833,7 +843,7 @@ float* vra_gemm_q4_big_xsum_table(int M, int K) {
 }
 void vra_launch_gemm_q4_big(const GemmDArgs& a0, bool dual, bool awq, int mb_sk, int dtype, int64_t stream) {
   GemmDArgs a = a0;
-  const int mb = mb_sk & 0xff, sk = mb_sk >> 8 > 1 ? mb_sk >> 8 : 1;  // vra_gemm_q4_big_fits: m-tiles | split-K << 8
+  const int mb = mb_sk & 0xff, sk = mb_sk >> 8 > 1 ? (mb_sk >> 8) & 0xffff : 1;  // vra_gemm_q4_big_fits: m-tiles | split-K << 8
   if (!a.xsum) {  // row sums of x per k-tile, once per GEMM (scratch: the tail of the split-K slab region) — unless the caller's
                   // norm launch already left them there (vra_gemm_q4_big_xsum_table + vra_rms_norm_xsum)
     float* tbl = vra_gemm_q4_big_xsum_table(a.M, a.K);
@@ -847,6 +857,7 @@ void vra_launch_gemm_q4_big(const GemmDArgs& a0, bool dual, bool awq, int mb_sk,
     else xsum_rows_kernel<F16><<<(unsigned)((total + 255) / 256), 256, 0, as_stream(stream)>>>(a.x, a.x_ld, a.M, KT, tbl);
     a.xsum = tbl;
   }
+  if (mb_sk & kMidPlan) return vra_launch_gemm_q4_mid(a, dual, awq, mb_sk & (kMidPlan - 1), dtype, stream);
 #ifdef VRA_GEMV_TS
   a.ts = vra_gemv_ts_buf();
 #endif
@@ -1104,7 +1115,7 @@ extern "C" void vra_wna16_gemm(const void* in, const void* qweight_tiled, const 
     c.group_size = group_size;
     c.n_blocks = n / 16;
     vra_launch_gemm_q4(c, is_awq != 0 && qzeros != nullptr, dtype, stream);
-  } else if (int mb = vra_gemm_q4_big_fits(false, m, n, k, group_size, nullptr)) {
+  } else if (int mb = vra_gemm_q4_big_fits(false, m, n, k, group_size, nullptr, is_awq != 0 && qzeros != nullptr, dtype)) {
     GemmDArgs d = {};
     d.w0 = qweight_tiled, d.sc0 = scales, d.qz0 = (const uint32_t*)qzeros, d.bias0 = bias;
     d.x = in, d.x_ld = k, d.residual = residual, d.res_ld = n, d.out = out, d.out_ld = n;
@@ -1195,7 +1206,7 @@ extern "C" void vra_wna16_gate_up_silu(const void* in, const void* qw_gate, cons
     c.group_size = group_size;
     c.n_blocks = n / 16;
     vra_launch_gemm_q4(c, is_awq != 0 && qz_gate != nullptr, dtype, stream);
-  } else if (int mb = vra_gemm_q4_big_fits(true, m, n, k, group_size, nullptr)) {
+  } else if (int mb = vra_gemm_q4_big_fits(true, m, n, k, group_size, nullptr, is_awq != 0 && qz_gate != nullptr, dtype)) {
     GemmDArgs d = {};
     d.w0 = qw_gate, d.w1 = qw_up, d.sc0 = sc_gate, d.sc1 = sc_up, d.qz0 = (const uint32_t*)qz_gate, d.qz1 = (const uint32_t*)qz_up;
     d.x = in, d.x_ld = k, d.out = out, d.out_ld = n;
