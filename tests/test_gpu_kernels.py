@@ -214,6 +214,19 @@ def test_wna16_gemm_middle_rows(dt, awq, gs, K, N, M):
     assert ops.lib().vra_take_device_error() == 0
 
 
+@pytest.mark.parametrize("off", [0, 4, 8])
+def test_wna16_gemm_middle_rows_off_16_bytes(off):
+    """x that does not start on 16 bytes, which the DMA of kernel M does not take: the launch goes to kernel D, with the same product"""
+    M, K, N = 97, 512, 272
+    r = rng(77)
+    q = make_quant(r, K, N, 128, BF16, False)
+    x = rand_dt(r, (M, K), BF16)
+    tiled = ops.marlin_weight_repack(ops.dev(q["qweight"]), q["qweight"].shape)
+    buf = ops.dev(np.concatenate([np.zeros(off // 2, np.uint16), x.reshape(-1)]))
+    out = ops.wna16_gemm(buf.ptr + off, tiled, ops.dev(q["scales"]), None, M, K, N, 128)
+    assert_close_dt(out.numpy(np.uint16, (M, N)), orc.wna16_gemm(x, q["idx"], None, q["scales"], 128, BF16), BF16, name="kernel M / D", abs_floor=2e-3)
+
+
 @pytest.mark.parametrize("dt,awq", [(BF16, False), (F16, False), (BF16, True)])
 @pytest.mark.parametrize("M,K,N", [(70, 512, 272), (128, 4608, 64), (150, 4736, 208), (200, 640, 272)])
 def test_gate_up_silu_middle_rows(dt, awq, M, K, N):

@@ -843,6 +843,13 @@ float* vra_gemm_q4_big_xsum_table(int M, int K) {
 }
 void vra_launch_gemm_q4_big(const GemmDArgs& a0, bool dual, bool awq, int mb_sk, int dtype, int64_t stream) {
   GemmDArgs a = a0;
+  // kernel M's LDS-DMA takes 16-byte pieces of x and the codes and 4-byte pieces of the scales: operands off those go to kernel D's 64-row tiles
+  const void* const own[] = {a.x, a.w0, dual ? a.w1 : a.w0, a.nseg > 1 ? a.xseg[0].w : a.w0, a.nseg > 2 ? a.xseg[1].w : a.w0};
+  const void* const scs[] = {a.sc0, dual ? a.sc1 : a.sc0, a.nseg > 1 ? a.xseg[0].scales : a.sc0, a.nseg > 2 ? a.xseg[1].scales : a.sc0};
+  bool dma = a.x_ld % 8 == 0;
+  for (const void* p : own) dma = dma && (uintptr_t)p % 16 == 0;
+  for (const void* p : scs) dma = dma && (uintptr_t)p % 4 == 0;
+  if ((mb_sk & kMidPlan) && !dma) mb_sk = 4;
   const int mb = mb_sk & 0xff, sk = mb_sk >> 8 > 1 ? (mb_sk >> 8) & 0xffff : 1;  // vra_gemm_q4_big_fits: m-tiles | split-K << 8
   if (!a.xsum) {  // row sums of x per k-tile, once per GEMM (scratch: the tail of the split-K slab region) — unless the caller's
                   // norm launch already left them there (vra_gemm_q4_big_xsum_table + vra_rms_norm_xsum)
