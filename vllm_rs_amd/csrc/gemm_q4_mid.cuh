@@ -6,8 +6,9 @@
 // the block, 32 MB of them (MB 2..5): 8 waves as 4 (columns, two n-blocks each) x 2 (rows, MB m-tiles each), so a code is converted twice for up to
 // 160 rows, and a k-tile's 8 MB MFMAs of a wave are 2 MB independent chains.  x, codes and scales of a k-tile of 128 travel by LDS-DMA through a
 // ring of three stages (one barrier a k-tile); the 16-byte chunks of an x row lie at slot chunk ^ (row mod 16), so the fragment reads meet no bank
-// twice.  Two n-blocks a wave read each x fragment from LDS four times a workgroup: 160 KB a k-tile at MB = 5, 1280 cycles beside 1380 of MFMAs
-// and 500 of conversions on each SIMD; four n-blocks a wave would halve that and double the conversions.
+// twice.  Two n-blocks a wave read each x fragment from LDS four times a workgroup: 160 KB a k-tile at MB = 5, 1280 cycles (and 880 for the DMA's
+// writes) beside 1380 of MFMAs and 500 of conversions on each SIMD; four n-blocks a wave would halve the reads and double the conversions.  Gate/up of 4096 x 14336 with 150 rows: 87 -> 50 us a launch; 96 rows
+// 45 -> 37 (kernel W); down with 200 rows 53 -> 44; below 65 rows, and at K <= 4096 where kernel W takes the launch, it gains nothing.
 //
 // The zero points stay out of the k loop for every type and format: acc += s_g acc_g inside, and behind it
 //     acc -= sum_g (C + z_g) s_g[n] . Sx_g[m],
