@@ -214,6 +214,34 @@ def test_wna16_gemm_middle_rows(dt, awq, gs, K, N, M):
     assert ops.lib().vra_take_device_error() == 0
 
 
+# The codes enter as C + q (C = 128, f16: 64) and the zero points' part, (C + z) times the sum of x, comes off per k-tile of 128: x of mean 0.5
+# or with large channels must not push it into the sum over the whole K.  Error of the float32 sums: a k-tile's partial sums of up to
+# (C + 16) sqrt(128) rms(x) round at 2^-24, four times over, K / 128 tiles add at random; the result is 4.6 sqrt(K) rms(x), all times the scale:
+# E = 4 (C + 16) / 4.6 x 2^-24 of it.  An output is not the 64-bit result's rounding where it lies within E of a boundary: a share 2 E / ulp, the
+# ulp at least 2^-8 (f16: 2^-11) of the value: 0.4 % and 1.7 %; seen 0.01..0.1 % and 0.1..0.7 %.  (Taken off behind the whole K: 0.2..0.6 % and 0.9..2.1 %.)
+@pytest.mark.parametrize("dt,awq", [(BF16, False), (BF16, True), (F16, False), (F16, True)])
+@pytest.mark.parametrize("x_kind", ["mean", "channels"])
+def test_wna16_gemm_middle_rows_precision(dt, awq, x_kind):
+    M, K, N = 200, 14336, 4096  # (kernel M, four slices of K)
+    r = rng(5 + dt + awq)
+    q = make_quant(r, K, N, 128, dt, awq)
+    if awq:  # (as checkpoints have them: near the middle, so that the result does not grow with the mean of x)
+        q["zeros"] = r.integers(7, 10, q["zeros"].shape, dtype=np.uint8)
+        q["qzeros"] = orc.awq_pack(q["zeros"])
+    x = r.standard_normal((M, K)).astype(np.float32) + (0.5 if x_kind == "mean" else 0.0)
+    if x_kind == "channels":
+        x[:, r.choice(K, 64, replace=False)] += 12.0
+    x = orc.to_dt(x, dt)
+    tiled = ops.marlin_weight_repack(ops.dev(q["qweight"]), q["qweight"].shape, 4, awq)
+    out = ops.wna16_gemm(ops.dev(x), tiled, ops.dev(q["scales"]), ops.dev(q["qzeros"]) if awq else None, M, K, N, 128, awq, 0, None, None, dt)
+    got = out.numpy(np.uint16, (M, N))[:, ::64]
+    z = q["zeros"][:, ::64].astype(np.float64) if awq else 8.0
+    w = ((q["idx"][:, ::64].reshape(K // 128, 128, -1) - (z[:, None] if awq else z)) * orc.from_dt(q["scales"], dt)[:, None, ::64].astype(np.float64)).reshape(K, -1)
+    ref = orc.to_dt((orc.from_dt(x, dt).astype(np.float64) @ w).astype(np.float32), dt)
+    share = float((got != ref).mean())
+    assert share <= (0.004 if dt == BF16 else 0.017), share
+
+
 @pytest.mark.parametrize("off", [0, 4, 8])
 def test_wna16_gemm_middle_rows_off_16_bytes(off):
     """x that does not start on 16 bytes, which the DMA of kernel M does not take: the launch goes to kernel D, with the same product"""

@@ -7,14 +7,15 @@
 // 160 rows, and a k-tile's 8 MB MFMAs of a wave are 2 MB independent chains.  x, codes and scales of a k-tile of 128 travel by LDS-DMA through a
 // ring of three stages (one barrier a k-tile); the 16-byte chunks of an x row lie at slot chunk ^ (row mod 16), so the fragment reads meet no bank
 // twice.  Two n-blocks a wave read each x fragment from LDS four times a workgroup: 160 KB a k-tile at MB = 5, 1280 cycles (and 880 for the DMA's
-// writes) beside 1380 of MFMAs and 500 of conversions on each SIMD; four n-blocks a wave would halve the reads and double the conversions.  Gate/up of 4096 x 14336 with 150 rows: 87 -> 50 us a launch; 96 rows
-// 45 -> 37 (kernel W); down with 200 rows 53 -> 44; below 65 rows, and at K <= 4096 where kernel W takes the launch, it gains nothing.
+// writes) beside 1380 of MFMAs and 500 of conversions on each SIMD; four n-blocks a wave would halve the reads and double the conversions.
+// us a launch, kernel D or W / here: gate/up of 4096 x 14336 behind its norm, 150 rows 91 / 56, 96 rows 50 / 42; down of 14336 x 4096 with its row sums, 200
+// rows 56 / 49.  AWQ: gate/up of 3584 x 18944, 320 rows 190 / 156.
 //
-// The zero points stay out of the k loop for every type and format: acc += s_g acc_g inside, and behind it
-//     acc -= sum_g (C + z_g) s_g[n] . Sx_g[m],
-// a small product over the k-tiles on the matrix cores.  w = (C + z) s is exact in float32 (11 + 8 bits) and goes in as three bf16 pieces (24
-// bits), the float32 row sums Sx (xsum_rows_kernel, or the norm's launch) as three as well; the six products of pieces down to 2^-16 of the
-// largest are kept (the three left out are below 2^-24 of it).
+// The zero points come off per k-tile, acc += s (acc_g - (C + z) Sx): acc never holds more than the result's own size.  (Taken off once behind the
+// k loop, x of mean 0.5 left the float32 sums of K = 14336 ten times as far from the 64-bit result.)  Symmetric codes have one z: a row's group sums
+// start from -(C + 8) Sx as the C operand of the first MFMAs, four products for all columns; AWQ, and only it, takes (C + z) Sx off
+// a column at a time.  The row sums Sx (xsum_rows_kernel, or the norm's launch) and the zero points travel with the ring.  That costs 3..5 % of a
+// launch with symmetric codes and 10 % with AWQ against one product behind the loop.
 //
 // Few columns leave the chip idle: K is then split over gridDim.z, with the exchange of kernel D (slabs written through, a flag line a slice;
 // only the last slice, whose workgroups start last, waits, and adds the slabs in slice order).
@@ -22,13 +23,13 @@
 #include "gemm_q4_big.cuh"  // GemmDArgs
 
 #define GM_THREADS 512
-static inline size_t gemm_q4_mid_lds_bytes(int mb) { return (size_t)3 * (32 * mb * 256 + 8 * 1024 + 8 * 256); }
+static inline size_t gemm_q4_mid_lds_bytes(int mb) { return (size_t)3 * (32 * mb * 256 + 8 * 1024 + 8 * 256 + 32 * mb * 4); }
 
-template <class DT, bool DUAL, int MB>
-__global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs a, int awq) {
+template <class DT, bool DUAL, bool AWQ, int MB>
+__global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  constexpr int NB = 2, ROWS = 32 * MB, XB = ROWS * 256, WB = 8 * 1024, SB = 8 * 256, STG = XB + WB + SB, PER = MB + 2;
+  constexpr int NB = 2, ROWS = 32 * MB, XB = ROWS * 256, WB = 8 * 1024, SB = 8 * 256, STG = XB + WB + SB + ROWS * 4, PER = MB + 3;
   constexpr uint32_t RSRC3 = 0x00020000u;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -71,7 +72,7 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
   const int kt0 = (int)((long)KT * zi / SK), kt1 = (int)((long)KT * (zi + 1) / SK);
 
   // ---- DMA sources.  A wave fetches MB KiB of x (4 rows each), the codes of its block wm (the other wave of the column pair the other's),
-  // and its own copy of its two blocks' scales (lanes 0..15; the rest fetch the same again)
+  // its own copy of its two blocks' scales (lanes 0..15) and zero points (lanes 16..19; the rest fetch the same again), and 4 MB row sums
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, 0x7FFFFFF0, RSRC3);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(wm ? wt[1] : wt[0]), 0, 0x7FFFFFF0, RSRC3);
   uint32_t vo_x[MB];
@@ -83,7 +84,16 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
   const uint32_t vo_w = (uint32_t)lane * 16u, so_w = (uint32_t)(wm ? nbc[1] : nbc[0]) * (uint32_t)KT;
   typedef const __attribute__((address_space(1))) void* glb_ptr;
   typedef __attribute__((address_space(3))) void* lds_ptr;
-  const unsigned char* sc_src = static_cast<const unsigned char*>((lane & 8) ? sct[1] : sct[0]) + (((lane & 8) ? nbc[1] : nbc[0]) * 32 + (lane & 7) * 4);
+  const int second = (lane & 16) ? (lane >> 1) & 1 : (lane >> 3) & 1;  // (the lane's block of the two)
+  const bool zero_lane = AWQ && (lane & 16);
+  const unsigned char *z0 = reinterpret_cast<const unsigned char*>(qzt[0]), *z1 = reinterpret_cast<const unsigned char*>(qzt[1]);
+  const unsigned char *s0 = static_cast<const unsigned char*>(sct[0]), *s1 = static_cast<const unsigned char*>(sct[1]);
+  asm("" : "+s"(z0), "+s"(z1), "+s"(s0), "+s"(s1));  // (in scalar registers: selected under a lane's index, they would be fetched by vector loads)
+  const unsigned char* const sc_src = zero_lane ? (second ? z1 : z0) + ((second ? nbc[1] : nbc[0]) * 2 + (lane & 1)) * 4
+                                                : (second ? s1 : s0) + ((second ? nbc[1] : nbc[0]) * 32 + (lane & 7) * 4);
+  const uint32_t sc_ld = zero_lane ? (uint32_t)N / 2 : (uint32_t)N * 2;  // bytes between two groups
+  const int srow = wave * 4 * MB;  // row sums of the rows srow + lane, lane < 4 MB
+  const float* const sum_src = a.xsum + (size_t)min(m0 + srow + lane, M - 1) * KT;
   auto request = [&](int kt) {
     unsigned char* const d = smem + ((kt - kt0) % 3) * STG;
 #pragma unroll
@@ -91,7 +101,8 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(d + (wave * MB + i) * 1024), 16, vo_x[i], (uint32_t)kt * 256u, 0, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(d + XB + (2 * wn + wm) * 1024), 16, vo_w, (so_w + (uint32_t)kt) * 1024u, 0, 2);  // nt
     const int grp = grouped ? (kt * 128) >> gsh : 0;
-    __builtin_amdgcn_global_load_lds((glb_ptr)(sc_src + (size_t)grp * N * 2), (lds_ptr)(d + XB + WB + wave * 256), 4, 0, 0);
+    __builtin_amdgcn_global_load_lds((glb_ptr)(sc_src + (size_t)grp * sc_ld), (lds_ptr)(d + XB + WB + wave * 256), 4, 0, 0);
+    if (lane < 4 * MB) __builtin_amdgcn_global_load_lds((glb_ptr)(sum_src + kt), (lds_ptr)(d + XB + WB + SB + srow * 4), 4, 0, 0);
   };
 
   f32x4 acc[NB][MB];
@@ -102,13 +113,18 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
   const int xrow = (wm * MB * 16 + nn) * 256;
   u32x4 wq[NB], xf[2][MB];
   u32x2 scw[NB];
+  uint32_t zw[NB];
+  float sx[MB];
   auto read_w = [&](int kt) {
     const unsigned char* const st = smem + ((kt - kt0) % 3) * STG + XB;
 #pragma unroll
     for (int b = 0; b < NB; b++) {
       wq[b] = *reinterpret_cast<const u32x4*>(st + (2 * wn + b) * 1024 + lane * 16);
       scw[b] = *reinterpret_cast<const u32x2*>(st + WB + wave * 256 + b * 32 + oct * 8);
+      if (AWQ) zw[b] = *reinterpret_cast<const uint32_t*>(st + WB + wave * 256 + 64 + b * 8 + (oct >> 1) * 4);
     }
+#pragma unroll
+    for (int t = 0; t < MB; t++) sx[t] = *reinterpret_cast<const float*>(st + WB + SB + ((wm * MB + t) * 16 + nn) * 4);
   };
   auto read_x = [&](int kt, int j) {
     const unsigned char* const st = smem + ((kt - kt0) % 3) * STG + xrow + (((j * 4 + oct) ^ nn) * 16);
@@ -139,8 +155,17 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
     f32x4 ag[NB][MB];
     s16x8 af[2][NB];
     u32x2 scc[NB];
+    uint32_t zc[NB];
+    float sxc[MB];
+    f32x4 zx[MB];  // symmetric codes: the zero points' part of a row's group sums, the same for every column
 #pragma unroll
-    for (int b = 0; b < NB; b++) af[0][b] = magic_word<DT>(wq[b][0]), scc[b] = scw[b];
+    for (int b = 0; b < NB; b++) af[0][b] = magic_word<DT>(wq[b][0]), scc[b] = scw[b], zc[b] = zw[b];
+#pragma unroll
+    for (int t = 0; t < MB; t++) {
+      sxc[t] = sx[t];
+      const float z = -(Magic<DT>::bias + 8.f) * sx[t];
+      zx[t] = f32x4{z, z, z, z};
+    }
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       if (j == 3 && kt + 1 < kt1) {
@@ -151,7 +176,8 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
       for (int t = 0; t < MB; t++)
 #pragma unroll
         for (int b = 0; b < NB; b++) {
-          if (j == 0) DT::mfma0(ag[b][t], af[0][b], __builtin_bit_cast(s16x8, xf[0][t]));
+          if (j == 0 && AWQ) DT::mfma0(ag[b][t], af[0][b], __builtin_bit_cast(s16x8, xf[0][t]));
+          else if (j == 0) DT::mfma_from(ag[b][t], af[0][b], __builtin_bit_cast(s16x8, xf[0][t]), zx[t]);
           else DT::mfma(ag[b][t], af[j & 1][b], __builtin_bit_cast(s16x8, xf[j & 1][t]));
           if (t == 0 && b == 0) {  // (behind the wait for fragment j: fragment j + 1 is not part of it)
             __builtin_amdgcn_sched_barrier(0);
@@ -165,107 +191,12 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
     VRA_MFMA_DRAIN();
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-      const float s0 = DT::to_f32((uint16_t)(scc[b][0] & 0xffffu)), s1 = DT::to_f32((uint16_t)(scc[b][0] >> 16));
-      const float s2 = DT::to_f32((uint16_t)(scc[b][1] & 0xffffu)), s3 = DT::to_f32((uint16_t)(scc[b][1] >> 16));
+      float s4[4], z4[4];
+      unpack_scale4<DT>(scc[b], zc[b], oct * 4, s4, z4);
 #pragma unroll
-      for (int t = 0; t < MB; t++) {
-        acc[b][t][0] = fmaf(s0, ag[b][t][0], acc[b][t][0]), acc[b][t][1] = fmaf(s1, ag[b][t][1], acc[b][t][1]);
-        acc[b][t][2] = fmaf(s2, ag[b][t][2], acc[b][t][2]), acc[b][t][3] = fmaf(s3, ag[b][t][3], acc[b][t][3]);
-      }
-    }
-  }
-
-  // ---- the zero points of this workgroup's k-tiles, 32 tiles a step: A, lane (column nn, octet oct) holds (C + z) s of tiles t0 + 8 oct .. + 7 (zero
-  // outside [kt0, kt1)); B, lane (row nn of the m-tile, oct) the row sums of those tiles.  Each block's and m-tile's pieces are made by one wave and
-  // meet the others in the ring's memory (made by every wave that needs them: 11 us a launch at 150 rows).
-  auto split3 = [&](const float (&v)[8], unsigned char* to) {  // hi + mid + lo bf16 pieces, a KiB each
-    u32x4 q[3];
+      for (int t = 0; t < MB; t++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      uint32_t h[2], m[2], l[2];
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const float x = v[2 * i + c];
-        const uint32_t hb = __float_as_uint(x) & 0xffff0000u;  // (truncated: the rest is exact)
-        const float r1 = x - __uint_as_float(hb);
-        const uint32_t mb = __float_as_uint(r1) & 0xffff0000u;
-        h[c] = hb >> 16, m[c] = mb >> 16, l[c] = (uint32_t)BF16::from_f32(r1 - __uint_as_float(mb));
-      }
-      q[0][i] = h[0] | (h[1] << 16), q[1][i] = m[0] | (m[1] << 16), q[2][i] = l[0] | (l[1] << 16);
-    }
-#pragma unroll
-    for (int i = 0; i < 3; i++) *reinterpret_cast<u32x4*>(to + i * 1024 + lane * 16) = q[i];
-  };
-  constexpr int MT = 2 * MB, XI = (MT + 7) / 8;  // m-tiles of the workgroup; of a wave
-  static_assert((8 + MT) * 3072 <= 3 * STG, "the pieces fit the ring");
-  for (int t0 = kt0 & ~3; t0 < kt1; t0 += 32) {
-    const int tb = t0 + oct * 8;
-    uint16_t sr[8];
-    uint32_t zr[8];
-    f32x4 sv[XI][2];
-    const int col = (wm ? nbc[1] : nbc[0]) * 16 + nn;
-    const uint16_t* const sp = static_cast<const uint16_t*>(wm ? sct[1] : sct[0]) + col;
-#pragma unroll
-    for (int e = 0; e < 8; e++) sr[e] = sp[(size_t)(grouped ? (min(tb + e, KT - 1) * 128) >> gsh : 0) * N];
-    if (awq) {
-      const uint32_t* const zp = (wm ? qzt[1] : qzt[0]) + (col >> 3);
-#pragma unroll
-      for (int e = 0; e < 8; e++) zr[e] = zp[(size_t)(grouped ? (min(tb + e, KT - 1) * 128) >> gsh : 0) * (N >> 3)] >> (4 * awq_rev(nn & 7));
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; e++) zr[e] = 8u;
-    }
-#pragma unroll
-    for (int u = 0; u < XI; u++) {
-      const float* const xr = a.xsum + (size_t)min(m0 + min(wave + 8 * u, MT - 1) * 16 + nn, M - 1) * KT;
-      if (KT % 4 == 0) {
-        sv[u][0] = *reinterpret_cast<const f32x4*>(xr + min(tb, KT - 4)), sv[u][1] = *reinterpret_cast<const f32x4*>(xr + min(tb + 4, KT - 4));
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++) sv[u][e >> 2][e & 3] = xr[min(tb + e, KT - 1)];
-      }
-    }
-    __syncthreads();  // (nobody reads the ring, or the step before, any more)
-    float w[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) w[e] = tb + e >= kt0 && tb + e < kt1 ? (Magic<DT>::bias + (float)(zr[e] & 0xFu)) * DT::to_f32(sr[e]) : 0.f;
-    split3(w, smem + (2 * wn + wm) * 3072);
-#pragma unroll
-    for (int u = 0; u < XI; u++)
-      if (wave + 8 * u < MT) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) w[e] = sv[u][e >> 2][e & 3];
-        split3(w, smem + (8 + wave + 8 * u) * 3072);
-      }
-    __syncthreads();
-    s16x8 wp[NB][3];
-#pragma unroll
-    for (int b = 0; b < NB; b++)
-#pragma unroll
-      for (int i = 0; i < 3; i++) wp[b][i] = *reinterpret_cast<const s16x8*>(smem + (2 * wn + b) * 3072 + i * 1024 + lane * 16);
-#pragma unroll
-    for (int mt = 0; mt < MB; mt++) {
-      s16x8 xp[3];
-#pragma unroll
-      for (int i = 0; i < 3; i++) xp[i] = *reinterpret_cast<const s16x8*>(smem + (8 + wm * MB + mt) * 3072 + i * 1024 + lane * 16);
-      f32x4 zt[NB];
-#pragma unroll
-      for (int b = 0; b < NB; b++) BF16::mfma0(zt[b], wp[b][2], xp[0]);  // smallest pieces first
-#pragma unroll
-      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][1], xp[1]);
-#pragma unroll
-      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][0], xp[2]);
-#pragma unroll
-      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][1], xp[0]);
-#pragma unroll
-      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][0], xp[1]);
-#pragma unroll
-      for (int b = 0; b < NB; b++) BF16::mfma(zt[b], wp[b][0], xp[0]);
-      VRA_MFMA_DRAIN();
-#pragma unroll
-      for (int b = 0; b < NB; b++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[b][mt][r] -= zt[b][r];
+        for (int r = 0; r < 4; r++) acc[b][t][r] = fmaf(s4[r], AWQ ? fmaf(-z4[r], sxc[t], ag[b][t][r]) : ag[b][t][r], acc[b][t][r]);
     }
   }
 

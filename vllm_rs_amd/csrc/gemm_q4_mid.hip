@@ -1,6 +1,7 @@
 // gemm_q4_mid.hip — kernel M (gemm_q4_mid.cuh): which launches take it, and the launch (the reference's int4 linear layers,
 // src/models/layers/linear.rs; its prompts go through the Marlin kernel, src/models/layers/others.rs).
 #include <algorithm>
+#include <type_traits>
 
 #include "gemm_launch.h"
 #include "gemm_q4_mid.cuh"
@@ -19,7 +20,7 @@ static int mid_cus() {
   return n;
 }
 
-int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, double* us) {
+int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, double* us) {
   if (M < 33 || K % 128 || cols % 16) return 0;
   if (group_size > 0 && group_size < K && (group_size < 128 || (group_size & (group_size - 1)))) return 0;
   if (segs && segs->nseg > 1) {  // a wave's columns must not straddle tensors
@@ -36,35 +37,39 @@ int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, cons
   for (int S = 1; S <= 16; S *= 2) {
     if (S > 1 && (!split || KT < 2 * S || tiles * S > cus)) break;  // the whole grid is resident: the owners find their slices running
     if (S > 1 && ((size_t)S * tiles * 2 * mb * GM_THREADS * 16 > vra_scratch_slab_bytes() - kXsum || (size_t)tiles * S * 16 > vra_scratch_counter_count())) break;
-    // Fitted to the Llama-3-8B and Qwen2-7B shapes at 64..760 rows (us): a launch 3 and 5.5 a round of workgroups; a k-tile as in `tile` (gate/up of
-    // 4096 x 14336, one round of 224 workgroups: 32 / 37 / 43 / 50 at MB 2..5); a slab of the exchange 0.43 per 32 rows beyond the first (down of
-    // Llama, 8 slices: 22 / 27 / 33 / 39); two workgroups of MB 2 share a CU, 13 % faster than one after the other; 4 for the row sums where no
-    // norm's launch leaves them
-    static const double tile[6] = {0, 0, 0.73, 0.90, 1.09, 1.38};
+    // Fitted to the Llama-3-8B and Qwen2-7B shapes at 64..760 rows (us): a launch 3 and 5.5 a round of workgroups; a k-tile as in `tile`, symmetric
+    // codes and AWQ (which unpacks its zero points and takes them off a column at a time): gate/up of 4096 x 14336, one round of 224 workgroups: 33 / 39 /
+    // 46 / 53 at MB 2..5; down of 18944 x 3584, 256 rows in 4 slices: 65; a slab of the exchange 0.43 per 32 rows beyond the first; two
+    // workgroups of MB 2 share a CU, 13 % faster than one after the other; 4 for the row sums where no norm's launch leaves them
+    static const double tile[2][6] = {{0, 0, 0.76, 0.93, 1.17, 1.44}, {0, 0, 0.82, 1.00, 1.28, 1.57}};
     const double rounds = (double)((tiles * S + cus - 1) / cus), q = rounds * (mb == 2 && rounds > 1 ? 0.87 : 1.0);
-    const double t = 3.0 + 5.5 * rounds + q * ((KT + S - 1) / S) * tile[mb] + (S > 1 ? 0.43 * (mb - 1) * (S - 1) : 0.0) + (dual || (segs && segs->nseg > 1) ? 0.0 : 4.0);
+    const double t = 3.0 + 5.5 * rounds + q * ((KT + S - 1) / S) * tile[awq][mb] + (S > 1 ? 0.43 * (mb - 1) * (S - 1) : 0.0) + (dual || (segs && segs->nseg > 1) ? 0.0 : 4.0);
     if (!best || t < *us) best = mb | (S << 8), *us = t;
   }
   return best;
 }
 
-template <class DT, bool DUAL, int MB>
-static void launch_t(const GemmDArgs& a, bool awq, dim3 grid, hipStream_t st) {
+template <class DT, bool DUAL, bool AWQ, int MB>
+static void launch_t(const GemmDArgs& a, dim3 grid, hipStream_t st) {
   static uint64_t seen = 0;  // per device: function attributes belong to the device current at the call
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (!((__atomic_load_n(&seen, __ATOMIC_RELAXED) >> (dev & 63)) & 1)) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_q4_mid_kernel<DT, DUAL, MB>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_q4_mid_kernel<DT, DUAL, AWQ, MB>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     __atomic_fetch_or(&seen, 1ull << (dev & 63), __ATOMIC_RELAXED);
   }
-  gemm_q4_mid_kernel<DT, DUAL, MB><<<grid, GM_THREADS, gemm_q4_mid_lds_bytes(MB), st>>>(a, awq ? 1 : 0);
+  gemm_q4_mid_kernel<DT, DUAL, AWQ, MB><<<grid, GM_THREADS, gemm_q4_mid_lds_bytes(MB), st>>>(a);
 }
 template <class DT, bool DUAL>
 static void launch_mb(const GemmDArgs& a, bool awq, int mb, dim3 grid, hipStream_t st) {
-  if (mb == 2) launch_t<DT, DUAL, 2>(a, awq, grid, st);
-  else if (mb == 3) launch_t<DT, DUAL, 3>(a, awq, grid, st);
-  else if (mb == 4) launch_t<DT, DUAL, 4>(a, awq, grid, st);
-  else launch_t<DT, DUAL, 5>(a, awq, grid, st);
+  auto go = [&](auto m) {
+    constexpr int MB = decltype(m)::value;
+    awq ? launch_t<DT, DUAL, true, MB>(a, grid, st) : launch_t<DT, DUAL, false, MB>(a, grid, st);
+  };
+  if (mb == 2) go(std::integral_constant<int, 2>{});
+  else if (mb == 3) go(std::integral_constant<int, 3>{});
+  else if (mb == 4) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, 5>{});
 }
 
 void vra_launch_gemm_q4_mid(GemmDArgs a, bool dual, bool awq, int plan, int dtype, int64_t stream) {

@@ -819,7 +819,7 @@ int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, cons
       }
   }
   double mid_us = 0.0;
-  if (const int plan = vra_gemm_q4_mid_plan(dual, M, cols, K, group_size, segs, &mid_us))  // kernel M, by its own estimate
+  if (const int plan = vra_gemm_q4_mid_plan(dual, M, cols, K, group_size, segs, awq, &mid_us))  // kernel M, by its own estimate
     if (mid_us < best && !mid_off) return plan | kMidPlan;
   return pick;
 }
