@@ -112,6 +112,11 @@ void vra_wna16_gate_up_silu(const void* in, const void* qw_gate, const void* sc_
                             const void* qz_up, void* out, int32_t m, int32_t k, int32_t n,
                             int32_t group_size, int32_t is_awq, int32_t scales_layout,
                             int32_t dtype, int64_t stream);
+/* The kernel that the two calls above (pair != 0: the second; has_norm != 0: the two below) run for a shape with row-major scales, as its letter:
+ * 'E', 'W' (decode and short prompts), 'X' (long prompts on dequantised weights), 'A', 'C', 'B' (general), 'D', 'M' (prompts; x, codes or scales off 16 / 16 / 4 bytes: 'D' for
+ * 'M').  0: a shape they refuse. */
+int32_t vra_wna16_kernel(int32_t pair, int32_t m, int32_t k, int32_t n, int32_t group_size, int32_t is_awq, int32_t has_norm,
+                         int32_t has_bias, int32_t has_residual);
 /* NormX::forward + QLinear::forward in one call (others.rs:11-29 in front of wna16.rs:263-306):
  * out = rmsnorm(in, norm_weight, eps)·W (+ bias).  Decode batches of 1..4 rows run fused (the
  * normalised activations never reach HBM); other shapes write rmsnorm(in) to `xn_workspace`

@@ -242,6 +242,25 @@ def test_wna16_gemm_middle_rows_precision(dt, awq, x_kind):
     assert share <= (0.004 if dt == BF16 else 0.017), share
 
 
+# us of a launch on the kernels in question (MI355X, cold weights): small products, where the launch is all, on kernel B; large ones on the faster of D and M
+@pytest.mark.parametrize("pair,M,K,N,awq,want", [
+    (0, 150, 512, 272, False, "B"),  # 9.5 / M 15
+    (0, 700, 512, 272, True, "B"),  # 10 / M 16
+    (0, 500, 1024, 1024, False, "B"),  # 10.6 / M 16
+    (0, 500, 2048, 512, False, "B"),  # 12 / M 18
+    (1, 300, 1024, 1024, False, "BD"),  # 16 / M 19
+    (0, 352, 14336, 4096, False, "D"),  # 77 / M 80
+    (0, 704, 18944, 3584, True, "D"),  # 220 / M 239
+    (1, 704, 4096, 14336, False, "D"),  # 202 / M 246
+    (0, 200, 14336, 4096, False, "M"),  # 49 / D 56
+    (0, 576, 14336, 4096, False, "M"),  # 96 / D 129
+    (1, 150, 4096, 14336, False, "M"),  # 56 / D 91
+    (1, 512, 3584, 18944, True, "M"),  # 216 / D 280
+])
+def test_wna16_kernel_is_the_faster_one(pair, M, K, N, awq, want):
+    assert ops.wna16_kernel(pair, M, K, N, 128, awq) in want
+
+
 @pytest.mark.parametrize("off", [0, 4, 8])
 def test_wna16_gemm_middle_rows_off_16_bytes(off):
     """x that does not start on 16 bytes, which the DMA of kernel M does not take: the launch goes to kernel D, with the same product"""

@@ -20,7 +20,7 @@ static int mid_cus() {
   return n;
 }
 
-int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, double* us) {
+int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, bool summed, double* us) {
   if (M < 33 || K % 128 || cols % 16) return 0;
   if (group_size > 0 && group_size < K && (group_size < 128 || (group_size & (group_size - 1)))) return 0;
   if (segs && segs->nseg > 1) {  // a wave's columns must not straddle tensors
@@ -43,7 +43,7 @@ int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, cons
     // workgroups of MB 2 share a CU, 13 % faster than one after the other; 4 for the row sums where no norm's launch leaves them
     static const double tile[2][6] = {{0, 0, 0.76, 0.93, 1.17, 1.44}, {0, 0, 0.82, 1.00, 1.28, 1.57}};
     const double rounds = (double)((tiles * S + cus - 1) / cus), q = rounds * (mb == 2 && rounds > 1 ? 0.87 : 1.0);
-    const double t = 3.0 + 5.5 * rounds + q * ((KT + S - 1) / S) * tile[awq][mb] + (S > 1 ? 0.43 * (mb - 1) * (S - 1) : 0.0) + (dual || (segs && segs->nseg > 1) ? 0.0 : 4.0);
+    const double t = 3.0 + 5.5 * rounds + q * ((KT + S - 1) / S) * tile[awq][mb] + (S > 1 ? 0.43 * (mb - 1) * (S - 1) : 0.0) + (summed ? 0.0 : 4.0);
     if (!best || t < *us) best = mb | (S << 8), *us = t;
   }
   return best;

@@ -744,7 +744,7 @@ void vra_launch_skinny(GemmBArgs a, bool int4, bool dual, int dtype, int64_t str
 
 // ---- kernel D launcher
 static const int kMidPlan = 1 << 24;  // vra_gemm_q4_big_fits: the rest is kernel M's plan
-int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, int dtype) {
+int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, bool summed) {
   static const char* off = getenv("VRA_NO_KERNEL_D");  // tuning aid
   if (off && atoi(off)) return 0;
   if (M < 64 || K % 128 || cols % 16) return 0;
@@ -755,32 +755,31 @@ int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, cons
     for (int i = 0; i + 1 < segs->nseg; i++)
       if (segs->xseg[i].n % 64) return 0;
   }
-  // Which of kernel B (slices K, every CU busy on narrow / short problems), kernel D with 64-row tiles (mb 4) or with 32-row
-  // tiles (mb 2)?  A small cost model fitted to the Llama-3-8B shapes at M = 128..4096 (tools/gemv_s_microbench.py, us):
-  //   kernel D: workgroups are co-resident in pairs (2 per CU, 4 waves each); per K = 4096 a pair of 64-row workgroups takes
-  //             82 us and a lone one 47; 32-row workgroups 46 and 28; + 15 us of launch, row-sum pass and epilogue;
-  //   kernel B: 17 us + FLOPs at 490 TFLOP/s; the gate/up pair form at 420 (round 5: it was priced at 650 and therefore picked for
-  //             ~143..221 rows, where it really takes 110-129 us against kernel D's 85-92: a 200-token prompt was slower than a
-  //             256-token one, profiles/r04_probe_kernel_d_tile_choice_160_256_rows.txt).
-  // e.g. M = 512: o 50.9 (B) / 39.8 (D, mb 2) / 58.3 (mb 4); down 143 / 117 / 180; gate/up 169 (mb 4) / 189 (mb 2).
+  // Which of kernel B (slices K, every CU busy on narrow / short problems), kernel D with 64-row tiles (mb 4) or with 32-row tiles (mb 2), or
+  // kernel M?  A cost model in us, fitted to the Llama-3-8B, Qwen2-7B, Llama-70B rank, TinyLlama and 3072-wide shapes at 64..760 rows, bf16 and
+  // f16, and to products from 512 x 272 up:
+  //   kernel D: workgroups are co-resident in pairs (2 per CU, 4 waves each); per K = 4096 a pair of 64-row workgroups takes 68 and a lone one 47,
+  //             of 32-row ones 46 and 28 (AWQ, which unpacks zero points in the loop, 97 / 57 and 52 / 31); 15 of launch, row sums and epilogue (13 at
+  //             K = 1024); in K slices a pair is quicker, 58 (AWQ 84), behind 24 (32-row tiles 15) and 1 (0.5) a slice of the exchange;
+  //   kernel B: 17 and FLOPs at 400 TFLOP/s, pairs at 345 (K off 1024: 250 and 215), less at a short K (below);
+  //   kernel M: vra_gemm_q4_mid_plan.
+  // e.g. down of Llama at 352 rows: 77 (D, 4 slices) / 80 (M); at 576 rows 129 / 96; 1024 x 1024 at 500 rows 10.6 (B) / 16 (M); down of
+  // Qwen2-7B at 704 rows 220 (D) / 239 (M).
   const int gx = dual ? (cols + 127) / 128 : (cols + 255) / 256;
   const int cus = num_cus();
   static const char* mid_env = getenv("VRA_NO_KERNEL_M");  // tuning aid
   const bool mid_off = mid_env && mid_env[0] == '1';
   if (mb_env && (atoi(mb_env) == 2 || atoi(mb_env) == 4) && !getenv("VRA_GD_SPLITK")) return atoi(mb_env);
   const double kf = (double)K / 4096.0;
-  // (those are the times without the zero points' hoisting; gate/up of Llama-3-8B in bf16 with symmetric codes at 200..760 rows, us: 76 / 134 / 150 / 219
-  // for 2 / 3 / 4 / 6 workgroups of 64 rows a CU; with zero points, Qwen2-7B: 95 / 125 + 15 / 272 for 2 / 3 / 5, and 88 for 3 of 32 rows)
-  const bool hoisted = !awq && dtype == VRA_BF16;
-  const double pair4 = hoisted ? 68.0 : 97.0, lone4 = hoisted ? 47.0 : 55.0, pair2 = hoisted ? 46.0 : 52.0, lone2 = hoisted ? 28.0 : 31.0;
+  const double pair4 = awq ? 97.0 : 68.0, lone4 = awq ? 57.0 : 47.0, pair2 = awq ? 52.0 : 46.0, lone2 = awq ? 31.0 : 28.0;
   auto est_d = [&](int mb) {
     const long w = (long)gx * ((M + 16 * mb - 1) / (16 * mb));
     const long q = (w + cus - 1) / cus;
     const double pair = mb == 4 ? pair4 : pair2, lone = mb == 4 ? lone4 : lone2;
     // (round 6: the gate/up pair on 32-row tiles runs ~15 % behind this model above 256 rows — 320 rows: 152 us against the 64-row tiles' 142,
     // profiles/r06_llama_midm_gemm_shapes.txt)
-    const double pen = dual && mb == 2 && M > 256 ? 1.15 : 1.0;
-    return 15.0 + ((double)(q / 2) * pair + (double)(q % 2) * lone) * kf * pen;
+    const double pen = dual && mb == 2 && M > 256 && K >= 2048 ? 1.15 : 1.0;
+    return 12.0 + 3.0 * std::min(1.0, kf) + ((double)(q / 2) * pair + (double)(q % 2) * lone) * kf * pen;
   };
   const double flops = 2.0 * (double)M * (double)cols * (dual ? 2.0 : 1.0) * (double)K;
   // (round 6: the rates above were fitted at K = 4096 / 14336.  Where K is not a multiple of 1024 — Qwen2-7B: 3584, 18944 — kernel B measures
@@ -790,7 +789,10 @@ int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, cons
   // it took q/k/v at 384 rows (81 us against kernel D's 60), o_proj at 576 / 640 rows (79 against 58) and down_proj at 576 (218 against ~145);
   // at 400 those go to kernel D and the launches where B does win (down_proj at 288 / 320 rows: 120 against 140) stay
   const bool k_odd = (K % 1024) != 0;
-  const double est_b = 17.0 + flops / ((dual ? (k_odd ? 215.0 : 345.0) : (k_odd ? 250.0 : 400.0)) * 1e6);
+  // (below K = 5440, pairs 2560, kernel B's launch is shorter: 9.5 us at K = 512, 12 at 2048; pairs 14.2, 18; it grows with its tiles: K = 1024,
+  // 64 tiles 10.6, 192 tiles 21)
+  const double kb = 0.2 * (K >> 7) + 0.05 * std::max(0, (M + 63) / 64 * ((cols + 127) / 128) - 32);
+  const double est_b = (dual ? 13.0 + std::min(4.0, kb) : 8.5 + std::min(8.5, kb)) + flops / ((dual ? (k_odd ? 215.0 : 345.0) : (k_odd ? 250.0 : 400.0)) * 1e6);
   double best = est_b;
   int pick = 0;
   const double d4 = est_d(4), d2 = est_d(2);
@@ -812,14 +814,14 @@ int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, cons
           continue;
         }
         const long q = (tiles * S + cus - 1) / cus;
-        const double pair = mb == 4 ? pair4 : pair2, lone = mb == 4 ? lone4 : lone2;
+        const double pair = mb == 4 ? (awq ? 84.0 : 58.0) : pair2, lone = mb == 4 ? lone4 : lone2;
         const double body = ((double)(q / 2) * pair + (double)(q % 2) * lone) * kf / S;
-        const double est = 15.0 + 3.0 + body + 6.0 + (mb == 4 ? 0.5 : 0.25) * (S - 1);
+        const double est = (mb == 4 ? (summed ? 20.0 : 24.0) : (summed ? 20.0 : 15.0)) + body + (mb == 4 ? 1.0 : 0.5) * (S - 1);
         if (est < best) best = est, pick = mb | (S << 8);
       }
   }
   double mid_us = 0.0;
-  if (const int plan = vra_gemm_q4_mid_plan(dual, M, cols, K, group_size, segs, awq, &mid_us))  // kernel M, by its own estimate
+  if (const int plan = vra_gemm_q4_mid_plan(dual, M, cols, K, group_size, segs, awq, summed, &mid_us))  // kernel M, by its own estimate
     if (mid_us < best && !mid_off) return plan | kMidPlan;
   return pick;
 }
@@ -1035,19 +1037,40 @@ static bool check_gemm_shape(const char* who, int m, int k, int n, int group_siz
   return true;
 }
 
+// kernel W or E where the product can run straight from the caller's tensors, or 0
+static int direct_kernel(int ns, int m, int k, int n, int group_size, bool has_res, bool has_bias, int scales_layout, bool norm) {
+  if (n % 16) return 0;
+  const bool grouped = group_size > 0 && group_size < k;
+  if (scales_layout == VRA_SCALES_MARLIN && (!grouped || n % 64)) return 0;  // channel-wise permutation: converted copy (rowmajor_scales)
+  // (this entry point: one output segment; the 17+-row pair form of kernel W exists with the fused norm only; K slices do not see whole rows: no
+  // fused norm)
+  if (vra_gemv_w_fits(ns, m, k, group_size, n / 16, has_res, has_bias) && !(ns == 2 && m > 16 && !norm) && !(k > 4096 && norm)) return 'W';
+  return vra_gemv_s_fits(ns, m, k, group_size, n / 16, norm) ? 'E' : 0;
+}
+// the kernel of a product (ns = 2: of a gate / up pair) that neither they nor the dense path take: A, C, D or M (with its plan), B
+static int general_kernel(int ns, int m, int k, int n, int group_size, bool awq, int* plan) {
+  if (vra_gemv_fits(true, ns, m, k, group_size)) return 'A';
+  if (vra_gemm_q4_fits(ns, m, k, group_size)) return 'C';
+  *plan = vra_gemm_q4_big_fits(ns == 2, m, n, k, group_size, nullptr, awq, false);
+  return *plan ? (*plan & kMidPlan ? 'M' : 'D') : 'B';
+}
+extern "C" int32_t vra_wna16_kernel(int32_t pair, int32_t m, int32_t k, int32_t n, int32_t group_size, int32_t is_awq, int32_t has_norm, int32_t has_bias, int32_t has_residual) {
+  if (!check_gemm_shape("vra_wna16_kernel", m, k, n, group_size)) return 0;
+  const int ns = pair ? 2 : 1;
+  if (const int c = direct_kernel(ns, m, k, n, group_size, has_residual != 0, has_bias != 0, VRA_SCALES_ROWMAJOR, has_norm != 0)) return c;
+  if (vra_dense_prefill_fits(m, k, ns * n, group_size)) return 'X';
+  int plan = 0;
+  return general_kernel(ns, m, k, n, group_size, is_awq != 0, &plan);
+}
+
 // decode batches of 1..4 rows on kernel E straight from the caller's tensors: row-major scales / zeros as in the
 // checkpoint, or the Marlin-permuted scales the reference passes (grouped form: a per-lane index inside 64 columns, no copy)
 static bool gemv_s_direct(int ns, const void* in, const void* w0, const void* sc0, const void* qz0, const void* w1, const void* sc1, const void* qz1,
                           const void* bias, const void* residual, void* out, int m, int k, int n, int group_size, int is_awq, int scales_layout,
                           int dtype, int64_t stream, const void* norm_w = nullptr, float eps = 0.f) {
-  const bool use_w = n % 16 == 0 && vra_gemv_w_fits(ns, m, k, group_size, n / 16, residual != nullptr, bias != nullptr) &&
-                     !(ns == 2 && m > 16 && !norm_w) &&  // (the 17+-row pair form of kernel W exists with the fused norm only)
-                     !(k > 4096 && norm_w);              // (K slices do not see whole rows: no fused norm)
-  // (this entry point: one output segment)
-  if (n % 16 || !(use_w || vra_gemv_s_fits(ns, m, k, group_size, n / 16, norm_w != nullptr))) return false;
-  const bool grouped = group_size > 0 && group_size < k;
-  if (scales_layout == VRA_SCALES_MARLIN && (!grouped || n % 64)) return false;  // channel-wise permutation: converted copy (rowmajor_scales)
-  const bool awq = is_awq != 0 && qz0 != nullptr;
+  const int kernel = direct_kernel(ns, m, k, n, group_size, residual != nullptr, bias != nullptr, scales_layout, norm_w != nullptr);
+  if (!kernel) return false;
+  const bool use_w = kernel == 'W', awq = is_awq != 0 && qz0 != nullptr;
   GemvSArgs a = {};
   a.w[0] = w0, a.scales[0] = sc0, a.zeros[0] = awq ? (const uint32_t*)qz0 : nullptr;
   a.w[1] = w1, a.scales[1] = sc1, a.zeros[1] = awq ? (const uint32_t*)qz1 : nullptr;
@@ -1095,7 +1118,9 @@ extern "C" void vra_wna16_gemm(const void* in, const void* qweight_tiled, const 
     scales = rs;
     scales_layout = VRA_SCALES_ROWMAJOR;
   }
-  if (vra_gemv_fits(true, 1, m, k, group_size)) {
+  int plan = 0;
+  const int kernel = general_kernel(1, m, k, n, group_size, is_awq != 0 && qzeros != nullptr, &plan);
+  if (kernel == 'A') {
     GemvArgs a = {};
     a.nseg = 1;
     a.seg[0] = GemvSeg{qweight_tiled, scales, (const uint32_t*)qzeros, bias, out, n, n, 0};
@@ -1109,7 +1134,7 @@ extern "C" void vra_wna16_gemm(const void* in, const void* qweight_tiled, const 
     a.is_awq = is_awq;
     a.scales_layout = scales_layout;
     vra_launch_gemv(a, true, dtype, stream);
-  } else if (vra_gemm_q4_fits(1, m, k, group_size)) {
+  } else if (kernel == 'C') {
     GemmCArgs c = {};
     c.nseg = 1;
     c.seg[0] = GemvSeg{qweight_tiled, scales, (const uint32_t*)qzeros, bias, out, n, n, 0};
@@ -1122,12 +1147,12 @@ extern "C" void vra_wna16_gemm(const void* in, const void* qweight_tiled, const 
     c.group_size = group_size;
     c.n_blocks = n / 16;
     vra_launch_gemm_q4(c, is_awq != 0 && qzeros != nullptr, dtype, stream);
-  } else if (int mb = vra_gemm_q4_big_fits(false, m, n, k, group_size, nullptr, is_awq != 0 && qzeros != nullptr, dtype)) {
+  } else if (plan) {
     GemmDArgs d = {};
     d.w0 = qweight_tiled, d.sc0 = scales, d.qz0 = (const uint32_t*)qzeros, d.bias0 = bias;
     d.x = in, d.x_ld = k, d.residual = residual, d.res_ld = n, d.out = out, d.out_ld = n;
     d.M = m, d.N = n, d.K = k, d.group_size = group_size;
-    vra_launch_gemm_q4_big(d, false, is_awq != 0 && qzeros != nullptr, mb, dtype, stream);
+    vra_launch_gemm_q4_big(d, false, is_awq != 0 && qzeros != nullptr, plan, dtype, stream);
   } else {
     GemmBArgs b = {};
     b.w0 = qweight_tiled;
@@ -1186,7 +1211,9 @@ extern "C" void vra_wna16_gate_up_silu(const void* in, const void* qw_gate, cons
     sc_up = u0;
     scales_layout = VRA_SCALES_ROWMAJOR;
   }
-  if (vra_gemv_fits(true, 2, m, k, group_size)) {
+  int plan = 0;
+  const int kernel = general_kernel(2, m, k, n, group_size, is_awq != 0 && qz_gate != nullptr, &plan);
+  if (kernel == 'A') {
     GemvArgs a = {};
     a.nseg = 2;
     a.seg[0] = GemvSeg{qw_gate, sc_gate, (const uint32_t*)qz_gate, nullptr, out, n, n, 0};
@@ -1200,7 +1227,7 @@ extern "C" void vra_wna16_gate_up_silu(const void* in, const void* qw_gate, cons
     a.is_awq = is_awq;
     a.scales_layout = scales_layout;
     vra_launch_gemv(a, true, dtype, stream);
-  } else if (vra_gemm_q4_fits(2, m, k, group_size)) {
+  } else if (kernel == 'C') {
     GemmCArgs c = {};
     c.nseg = 2;
     c.seg[0] = GemvSeg{qw_gate, sc_gate, (const uint32_t*)qz_gate, nullptr, out, n, n, 0};
@@ -1213,12 +1240,12 @@ extern "C" void vra_wna16_gate_up_silu(const void* in, const void* qw_gate, cons
     c.group_size = group_size;
     c.n_blocks = n / 16;
     vra_launch_gemm_q4(c, is_awq != 0 && qz_gate != nullptr, dtype, stream);
-  } else if (int mb = vra_gemm_q4_big_fits(true, m, n, k, group_size, nullptr, is_awq != 0 && qz_gate != nullptr, dtype)) {
+  } else if (plan) {
     GemmDArgs d = {};
     d.w0 = qw_gate, d.w1 = qw_up, d.sc0 = sc_gate, d.sc1 = sc_up, d.qz0 = (const uint32_t*)qz_gate, d.qz1 = (const uint32_t*)qz_up;
     d.x = in, d.x_ld = k, d.out = out, d.out_ld = n;
     d.M = m, d.N = n, d.K = k, d.group_size = group_size;
-    vra_launch_gemm_q4_big(d, true, is_awq != 0 && qz_gate != nullptr, mb, dtype, stream);
+    vra_launch_gemm_q4_big(d, true, is_awq != 0 && qz_gate != nullptr, plan, dtype, stream);
   } else {
     GemmBArgs b = {};
     b.w0 = qw_gate;

@@ -735,7 +735,7 @@ bool Model::linear_fused_norm(const QLinear* ls, int nl, void* const* outs, cons
       cols += ls[i].N;
     }
     d.x = xn_, d.x_ld = K, d.M = M, d.K = K, d.group_size = mc_.group_size;
-    mb_d = vra_gemm_q4_big_fits(false, M, cols, K, mc_.group_size, &d, ls[0].awq, dt_);
+    mb_d = vra_gemm_q4_big_fits(false, M, cols, K, mc_.group_size, &d, ls[0].awq, true);
   }
   float* xsum_tbl = mb_d && K % 128 == 0 ? vra_gemm_q4_big_xsum_table(M, K) : nullptr;
   if (xsum_tbl) {
@@ -823,7 +823,7 @@ bool Model::gate_up(const LayerWeights& L, const void* x, const void* norm_w, vo
         vra_launch_gemm_dense(a, true, dt_, vra_gemm_dense_tile(M, 2 * N, K), stream);
         return !take_err(error, "gate_up (gemm_dense, resident weights)");
       }
-      const int mb = !dense && M >= 64 && K % 128 == 0 ? vra_gemm_q4_big_fits(true, M, N, K, mc_.group_size, nullptr, L.gate.awq && L.gate.qzeros != nullptr, dt_) : 0;
+      const int mb = !dense && M >= 64 && K % 128 == 0 ? vra_gemm_q4_big_fits(true, M, N, K, mc_.group_size, nullptr, L.gate.awq && L.gate.qzeros != nullptr, true) : 0;
       float* tbl = mb ? vra_gemm_q4_big_xsum_table(M, K) : nullptr;
       if (tbl) {
         vra_rms_norm_xsum(x, norm_w, xn_, tbl, M, K, mc_.rms_norm_eps, dt_, stream);

@@ -117,6 +117,13 @@ def wna16_gemm(x, qweight_tiled, scales, qzeros, m, k, n, group_size, is_awq=Fal
     return out
 
 
+def wna16_kernel(pair, m, k, n, group_size, is_awq=False, has_norm=False, has_bias=False, has_residual=False):
+    """letter of the kernel that wna16_gemm (pair: wna16_gate_up_silu; has_norm: their rms_norm forms) runs for a shape (include/vllm_rs_amd.h)"""
+    c = lib().vra_wna16_kernel(int(pair), m, k, n, group_size, int(is_awq), int(has_norm), int(has_bias), int(has_residual))
+    check_error()
+    return chr(c)
+
+
 def wna16_gate_up_silu(x, qw_g, sc_g, qz_g, qw_u, sc_u, qz_u, m, k, n, group_size, is_awq=False,
                        scales_layout=SCALES_ROWMAJOR, dtype=BF16):
     out = DevBuf(m * n * 2)
