@@ -1,0 +1,22 @@
+"""Which kernel a shape runs on, where that is decided without a GPU (vra_wna16_kernel)."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+QUERY = "from vllm_rs_amd import ops; print(''.join(ops.wna16_kernel(%d, m, 4096, 14336, 128, has_norm=True) for m in (16, 32, 33, 64)))"
+
+
+def kernels(pair, **env):
+    """the letters for 16, 32, 33 and 64 rows in a process of its own: the tuning aids are read once"""
+    out = subprocess.run([sys.executable, "-c", QUERY % pair], cwd=ROOT, env=dict(os.environ, **env), capture_output=True, text=True, check=True)
+    return out.stdout.strip()
+
+
+@pytest.mark.parametrize("pair", [0, 1])
+def test_rows_limit_of_kernel_w_holds_for_single_products_and_pairs(pair):
+    assert kernels(pair) == "WWWW"
+    short = kernels(pair, VRA_GEMV_W_MAX_ROWS="32")
+    assert short[:2] == "WW" and "W" not in short[2:], short

@@ -343,6 +343,24 @@ def test_gemv_w_row_blocks_gate_up_pair(M, awq):
     assert_close_dt(out.numpy(np.uint16, (M, N)), orc.silu_mul(g, u, BF16), BF16, max_ulp=6.0, max_mismatch_frac=0.05, name="gemv_w row blocks gate/up", abs_floor=8e-3)
 
 
+@pytest.mark.parametrize("M", [4, 32, 65, 100, 128])
+def test_gate_up_pair_without_a_workspace(M):
+    """a caller that passes no place for the normalised rows: every row count that the fused form can run is taken"""
+    K, N = 512, 2048
+    r = rng(M * 3 + K)
+    qg, qu = make_quant(r, K, N, 128, BF16), make_quant(r, K, N, 128, BF16)
+    x, nw = rand_dt(r, (M, K), BF16, 2.0), orc.to_dt((1.0 + 0.1 * r.standard_normal(K)).astype(np.float32), BF16)
+    out = ops.DevBuf(M * N * 2)
+    xd, nd, tg, tu, sg, su = ops.dev(x), ops.dev(nw), _tiled(qg), _tiled(qu), ops.dev(qg["scales"]), ops.dev(qu["scales"])
+    ops.lib().vra_rms_norm_wna16_gate_up_silu(xd.ptr, nd.ptr, 1e-5, tg.ptr, sg.ptr, None, tu.ptr, su.ptr, None, out.ptr, None, M, K, N, 128, 0, 0, BF16, 0)
+    ops.check_error()
+    xn = orc.rms_norm(x, nw, 1e-5, BF16)
+    g, u = (orc.wna16_gemm(xn, q["idx"], q["zeros"], q["scales"], 128, BF16) for q in (qg, qu))
+    # (the fused form rounds x * weight and applies the row's factor behind the sum: about one bf16 rounding of every operand, 2^-9, apart)
+    got, ref = orc.from_dt(out.numpy(np.uint16, (M, N)), BF16).astype(np.float64), orc.from_dt(orc.silu_mul(g, u, BF16), BF16).astype(np.float64)
+    assert np.linalg.norm(got - ref) <= 2.0 ** -7 * np.linalg.norm(ref)
+
+
 # ---------------------------------------------------------------------------------------------
 # kernel W, K > 4096 (down_proj): K slices across workgroups — the slices' f32 partial tiles meet through memory and the last slice
 # of a unit group sums them in slice order.  Slice shapes: 14336 = 4 x 28 tiles (waves 4..7 hold three), 18944 = 4 x 30 + 28

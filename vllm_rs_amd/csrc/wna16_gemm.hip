@@ -438,7 +438,7 @@ void vra_launch_gemv_s(GemvSArgs a, int ns, int group_size, bool awq, int dtype,
 static int gemv_w_max_rows() {
   static int v = -1;
   if (v < 0) {
-    const char* e = getenv("VRA_GEMV_W_MAX_ROWS");  // tuning aid: 32 puts the short prefills back on kernels B / D
+    const char* e = getenv("VRA_GEMV_W_MAX_ROWS");  // tuning aid: 32 puts the short prefills back on kernels B / D / M
     v = e ? atoi(e) : 256;
   }
   return v;
@@ -484,7 +484,7 @@ static bool gemv_w_kz_plan(int K, int n_units, int rb, int* kz, int* ktz, int* g
   *kz = z, *ktz = t, *groups = g;
   return true;
 }
-bool vra_gemv_w_fits(int ns, int M, int K, int group_size, int n_units, bool has_res, bool has_bias, bool norm_or_segments) {
+bool vra_gemv_w_fits(int ns, int M, int K, int group_size, int n_units, bool has_res, bool has_bias, bool norm_or_segments, bool no_other) {
   static const char* off = getenv("VRA_NO_GEMV_W");
   if (off && off[0] == '1') return false;
   if (K > 4096) {
@@ -505,8 +505,9 @@ bool vra_gemv_w_fits(int ns, int M, int K, int group_size, int n_units, bool has
     return gemv_q4w_lds_bytes(1, mt, mu, has_res, true) <= (size_t)kMaxDynLds;
   }
   static const char* pair_env = getenv("VRA_GEMV_W_PAIR_MAX_ROWS");  // tuning aid: 16 puts 17+-row gate/up launches back on kernels C / D
-  // (pairs: 64 rows 37.1 us / kernel M 36.9, 96 rows 50 / 42, 128 rows 59 / 48, Llama-3-8B with the norm's launch)
-  const int pair_max = pair_env ? atoi(pair_env) : 64;
+  // (pairs: 64 rows 37.1 us / kernel M 36.9, 96 rows 50 / 42, 128 rows 59 / 49, Llama-3-8B with the norm's launch; beyond 64 rows only where no
+  // other kernel can take the launch, `no_other`: a caller without a place for the normalised rows)
+  const int pair_max = pair_env ? atoi(pair_env) : (no_other ? gemv_w_max_rows() : std::min(64, gemv_w_max_rows()));
   if (M < 5 || M > (ns == 1 ? gemv_w_max_rows() : (pair_max > 16 ? pair_max : 16)) || K % 128 || K > 4096) return false;
   const int g = group_size > 0 && group_size < K ? group_size : K;
   if (g < K && (g < 128 || (g & (g - 1)))) return false;
@@ -1038,13 +1039,13 @@ static bool check_gemm_shape(const char* who, int m, int k, int n, int group_siz
 }
 
 // kernel W or E where the product can run straight from the caller's tensors, or 0
-static int direct_kernel(int ns, int m, int k, int n, int group_size, bool has_res, bool has_bias, int scales_layout, bool norm) {
+static int direct_kernel(int ns, int m, int k, int n, int group_size, bool has_res, bool has_bias, int scales_layout, bool norm, bool no_other = false) {
   if (n % 16) return 0;
   const bool grouped = group_size > 0 && group_size < k;
   if (scales_layout == VRA_SCALES_MARLIN && (!grouped || n % 64)) return 0;  // channel-wise permutation: converted copy (rowmajor_scales)
   // (this entry point: one output segment; the 17+-row pair form of kernel W exists with the fused norm only; K slices do not see whole rows: no
   // fused norm)
-  if (vra_gemv_w_fits(ns, m, k, group_size, n / 16, has_res, has_bias) && !(ns == 2 && m > 16 && !norm) && !(k > 4096 && norm)) return 'W';
+  if (vra_gemv_w_fits(ns, m, k, group_size, n / 16, has_res, has_bias, false, no_other) && !(ns == 2 && m > 16 && !norm) && !(k > 4096 && norm)) return 'W';
   return vra_gemv_s_fits(ns, m, k, group_size, n / 16, norm) ? 'E' : 0;
 }
 // the kernel of a product (ns = 2: of a gate / up pair) that neither they nor the dense path take: A, C, D or M (with its plan), B
@@ -1067,8 +1068,8 @@ extern "C" int32_t vra_wna16_kernel(int32_t pair, int32_t m, int32_t k, int32_t 
 // checkpoint, or the Marlin-permuted scales the reference passes (grouped form: a per-lane index inside 64 columns, no copy)
 static bool gemv_s_direct(int ns, const void* in, const void* w0, const void* sc0, const void* qz0, const void* w1, const void* sc1, const void* qz1,
                           const void* bias, const void* residual, void* out, int m, int k, int n, int group_size, int is_awq, int scales_layout,
-                          int dtype, int64_t stream, const void* norm_w = nullptr, float eps = 0.f) {
-  const int kernel = direct_kernel(ns, m, k, n, group_size, residual != nullptr, bias != nullptr, scales_layout, norm_w != nullptr);
+                          int dtype, int64_t stream, const void* norm_w = nullptr, float eps = 0.f, bool no_other = false) {
+  const int kernel = direct_kernel(ns, m, k, n, group_size, residual != nullptr, bias != nullptr, scales_layout, norm_w != nullptr, no_other);
   if (!kernel) return false;
   const bool use_w = kernel == 'W', awq = is_awq != 0 && qz0 != nullptr;
   GemvSArgs a = {};
@@ -1519,7 +1520,7 @@ extern "C" void vra_rms_norm_wna16_gate_up_silu(const void* in, const void* norm
   VRA_CHECK_ARG(dtype == VRA_BF16 || dtype == VRA_F16, "vra_rms_norm_wna16_gate_up_silu: dtype must be bf16/f16");
   if (!check_gemm_shape("vra_rms_norm_wna16_gate_up_silu", m, k, n, group_size)) return;
   if (gemv_s_direct(2, in, qw_gate, sc_gate, qz_gate, qw_up, sc_up, qz_up, nullptr, nullptr, out, m, k, n, group_size, is_awq, scales_layout, dtype,
-                    stream, norm_weight, eps))
+                    stream, norm_weight, eps, xn_workspace == nullptr))
     return;
   VRA_CHECK_ARG(xn_workspace != nullptr, "vra_rms_norm_wna16_gate_up_silu: this shape needs xn_workspace [m, k]");
   vra_rms_norm(in, norm_weight, xn_workspace, m, k, eps, dtype, stream);
