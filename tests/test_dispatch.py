@@ -5,6 +5,8 @@ import sys
 
 import pytest
 
+from vllm_rs_amd import _lib
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 QUERY = "from vllm_rs_amd import ops; print(''.join(ops.wna16_kernel(%d, m, 4096, 14336, 128, has_norm=True) for m in (16, 32, 33, 64)))"
 
@@ -20,3 +22,10 @@ def test_rows_limit_of_kernel_w_holds_for_single_products_and_pairs(pair):
     assert kernels(pair) == "WWWW"
     short = kernels(pair, VRA_GEMV_W_MAX_ROWS="32")
     assert short[:2] == "WW" and "W" not in short[2:], short
+
+
+def test_linear_recurrence_stays_within_the_default_lds():
+    """its launch raises no limit, so 64 KB is all it may ask for, at every key size"""
+    L = _lib.load()
+    assert max(L.vra_stack_op_linear_scan_lds(dim) for dim in range(1, 257)) <= 64 * 1024
+    assert L.vra_stack_op_linear_scan_lds(0) < 0 and L.vra_stack_op_linear_scan_lds(257) < 0

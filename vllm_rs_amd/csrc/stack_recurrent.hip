@@ -743,7 +743,8 @@ __device__ __forceinline__ float group_sum(float v) {
 // DECAY 0: one constant per head; 1: one per row and key channel; 2: one per row and head.  ACT: q, k, v pass silu on their way into LDS.
 // BONUS (per-channel decays, no delta rule): the output is read before the decay, this token enters it through bonus (bs: sum_d q_d bonus_d k_d).
 // tokens staged at a time: the next tile's operands are requested ahead of a tile's tokens, whose time has to cover their way from memory
-constexpr int scan_tile(int dimP) { return dimP > 128 ? 16 : 32; }
+// (one lane a column, keys of up to 4: the values and outputs of 32 tokens would take 64 KB)
+constexpr int scan_tile(int dimP) { return dimP > 128 || dimP <= 4 ? 16 : 32; }
 template <int R, int P, int DECAY, bool BETA, bool ACT, bool BONUS = false>
 __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -1245,15 +1246,22 @@ void vra_stack_sigmoid_pow(const float* z, int ldz, float* out, int ldo, int T, 
   launch_checked("stack decay", [&] { stk_sigmoid_pow_kernel<<<grid, 256, 0, as_stream(stream)>>>(z, ldz, out, ldo, n, total, inv_tau); });
 }
 
+extern "C" int32_t vra_stack_op_linear_scan_lds(int32_t dim) {
+  if (dim < 1 || dim > 256) return -1;
+  int P = 1;
+  while (P * 4 < dim) P <<= 1;
+  const int TT = scan_tile(P * 4);
+  return (int32_t)((TT * P * 4 * 3 + 2 * TT * (256 / P) + 3 * TT) * sizeof(float));
+}
 void vra_stack_linear_scan(const StkScanArgs& a, int64_t stream) {
   VRA_CHECK_ARG(a.q && a.k && a.v && a.state && a.state_slots && a.positions && a.out && (a.decay || a.head_decay), "stack linear scan: null pointer");
   VRA_CHECK_ARG(a.B > 0 && a.H > 0 && a.qk_rep >= 1 && a.H % a.qk_rep == 0 && a.dim > 0 && a.dim <= 256 && a.vdim > 0, "stack linear scan: key size at most 256");
   constexpr int R = 4;
   int P = 1;
   while (P * R < a.dim) P <<= 1;
-  const int CPB = 256 / P, dimP = P * R;
-  const int TT = scan_tile(dimP);
-  const size_t lds = ((size_t)TT * dimP * 3 + (size_t)2 * TT * CPB + 3 * TT) * sizeof(float);
+  const int CPB = 256 / P;
+  const size_t lds = (size_t)vra_stack_op_linear_scan_lds(a.dim);
+  VRA_CHECK_ARG(lds <= 64 * 1024, "stack linear scan: staging does not fit LDS");
   dim3 grid((a.vdim + CPB - 1) / CPB, a.H, a.B);
   hipStream_t st = as_stream(stream);
   const bool decay = a.decay != nullptr, beta = a.beta != nullptr, per_head = decay && a.decay_per_head;
