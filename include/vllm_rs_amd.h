@@ -701,8 +701,9 @@ void vra_stack_op_linear_scan(const float* q, int32_t ldq, const float* k, int32
                               int32_t ldd, const float* head_decay, const float* beta, int32_t ldb, float q_scale, float* state,
                               const int32_t* state_slots, const int64_t* positions, const uint32_t* cu_q, float* out, int32_t ldo,
                               int32_t B, int32_t H, int32_t qk_rep, int32_t dim, int32_t vdim, int64_t stream);
-/* bytes of LDS a workgroup of that launch asks for at a key size (at most 64 KB: it raises no limit) */
-int32_t vra_stack_op_linear_scan_lds(int32_t dim);
+/* bytes of LDS a workgroup of that launch asks for (at most 64 KB: it raises no limit); max_q: most tokens of a sequence, 0 unknown (as in
+ * that call with cu_q), 1: cu_q null */
+int32_t vra_stack_op_linear_scan_lds(int32_t dim, int32_t vdim, int32_t H, int32_t B, int32_t max_q);
 void vra_stack_op_sandwich_norm(float* x, const float* p1, int32_t n1, const float* pw, float c1, const float* p2, float c2,
                                 const float* post_w, const float* pre_w, void* h, float eps, int32_t T, int32_t W, const void* router_w,
                                 const float* router_bias, int32_t n_router, int32_t top, int32_t* pair_expert, float* pair_weight,

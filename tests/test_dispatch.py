@@ -25,7 +25,14 @@ def test_rows_limit_of_kernel_w_holds_for_single_products_and_pairs(pair):
 
 
 def test_linear_recurrence_stays_within_the_default_lds():
-    """its launch raises no limit, so 64 KB is all it may ask for, at every key size"""
-    L = _lib.load()
-    assert max(L.vra_stack_op_linear_scan_lds(dim) for dim in range(1, 257)) <= 64 * 1024
-    assert L.vra_stack_op_linear_scan_lds(0) < 0 and L.vra_stack_op_linear_scan_lds(257) < 0
+    """its launch raises no limit, so 64 KB is all it may ask for, at every key size and form"""
+    lds = _lib.load().vra_stack_op_linear_scan_lds
+    assert max(lds(dim, dim, 16, B, n) for dim in range(1, 257) for B in (1, 64) for n in (0, 1, 5, 100)) <= 64 * 1024
+    assert lds(0, 1, 1, 1, 0) < 0 and lds(257, 1, 1, 1, 0) < 0
+
+
+@pytest.mark.parametrize("dim", [4, 32, 64, 128, 256])
+def test_linear_recurrence_stages_one_token_for_one(dim):
+    """a decode step's workgroups stage one token: q, k, decays, value and output of it and three numbers"""
+    P = max(1, dim // 4)
+    assert _lib.load().vra_stack_op_linear_scan_lds(dim, dim, 16, 8, 1) == 4 * (3 * dim + 2 * (256 // P) + 3)

@@ -606,6 +606,48 @@ def test_linear_recurrence_tiles(D, V, pad, T):
     assert (state.numpy(np.float32, (2, H * V * D))[0] == 50.0).all()
 
 
+@pytest.mark.parametrize("T", [1, 7, 16, 33, 64])
+@pytest.mark.parametrize("form", ["delta", "decays", "per head", "bonus"])
+@pytest.mark.parametrize("D,V", [(64, 64), (128, 128), (128, 72), (256, 256)])
+def test_linear_recurrence_does_not_depend_on_the_other_sequences(D, V, form, T):
+    """one sequence alone (4 rows of the state a lane), 33 copies of it at once (8 rows a lane) and its first token as a decode step (one token
+    staged): the same bits, and the float64 recurrence to 1e-5 (float32 sums of D terms along chains that contract)"""
+    L = _lib.load()
+    r = np.random.default_rng(D + V + T)
+    H, B = 512 // D, 33
+    x = {n: r.standard_normal((T, H, d)).astype(np.float32) for n, d in (("q", D), ("k", D), ("v", V))}
+    x["k"] /= np.sqrt((x["k"] * x["k"]).sum(-1, keepdims=True))
+    per_head = form == "per head"
+    x["decay"] = (0.7 + 0.3 * r.random((T, H) if per_head else (T, H, D))).astype(np.float32)
+    x["beta"] = r.random((T, H)).astype(np.float32)
+    bonus = (r.standard_normal((H, D)) / D).astype(np.float32)
+
+    def run(copies, cu):
+        rows = {n: raw(np.concatenate([a[:T if cu else 1].reshape(T if cu else 1, -1)] * copies), np.float32) for n, a in x.items()}
+        n = T if cu else 1
+        state, out = empty(copies * H * V * D * 4).fill_bytes(0), empty(copies * n * H * V * 4)
+        args = (rows["q"].ptr, H * D, rows["k"].ptr, H * D, rows["v"].ptr, H * V, rows["decay"].ptr, H if per_head else H * D)
+        slots, pos = raw(np.arange(copies), np.int32), raw(np.tile(np.arange(n), copies), np.int64)
+        cud = raw(np.arange(copies + 1) * n, np.uint32)
+        tail = (0.5, state.ptr, slots.ptr, pos.ptr, cud.ptr if cu else None, out.ptr, H * V, copies, H, 1, D, V)
+        beta = rows["beta"].ptr if form in ("delta", "per head") else None
+        if form == "bonus":
+            bd = raw(bonus, np.float32)
+            L.vra_stack_op_bonus_scan(*args, bd.ptr, *tail, 0)
+        elif per_head:
+            L.vra_stack_op_linear_scan_ex(*args, 1, 0, None, beta, H, *tail, 0)
+        else:
+            L.vra_stack_op_linear_scan(*args, None, beta, H if beta else 0, *tail, 0)
+        check()
+        return out.numpy(np.float32, (copies, n, H, V)), state.numpy(np.float32, (copies, H, V, D))
+
+    (one, s1), (many, s33), (first, _) = run(1, True), run(B, True), run(B, False)
+    assert (many == one).all() and (s33 == s1).all() and (first[:, 0] == one[:, 0]).all()
+    if form == "delta":
+        ref = zo.linear_recurrence(x["q"].astype(np.float64) * 0.5, *(x[n].astype(np.float64) for n in ("k", "v", "decay", "beta")))
+        assert rel(one[0], ref) < 1e-5
+
+
 
 @pytest.mark.parametrize("dt", [F32, BF16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("W,E,top", [(96, 5, 2), (51, 3, 3), (256, 40, 1), (64, 8, 4)])

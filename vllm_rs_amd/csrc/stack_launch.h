@@ -400,6 +400,7 @@ struct StkScanArgs {
   float* out = nullptr;
   int ldo = 0;
   int B = 0, H = 0, qk_rep = 1, dim = 0, vdim = 0;
+  int max_q = 0;  // most tokens of a sequence (0: unknown)
 };
 void vra_stack_linear_scan(const StkScanArgs& a, int64_t stream);
 

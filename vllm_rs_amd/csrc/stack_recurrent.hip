@@ -715,15 +715,18 @@ __global__ __launch_bounds__(256) void stk_sigmoid_pow_kernel(const float* z, in
 
 // ------------------------------------------------------------------------------------------------ the linear recurrence
 // A workgroup owns 256 / P columns of one head's state (a column = one value channel); a column's `dim` rows are spread over P
-// neighbouring lanes, R = 4 rows each, in registers for the whole step.  What bounds it is the serial chain over the tokens: a token's S^T k
-// has to be summed over the lanes before its row enters S, about 50 instructions a wave, and the grid seldom has more than one wave a SIMD to fill
-// the waits.  So: 4 rows a lane, which gives 16 heads of 128 x 128 a wave on every SIMD (8 rows leave half of the CUs idle) and 16-byte
-// LDS reads beside the neighbours' (32 bytes apart they meet in the same banks); S^T q taken of the state before the token's row
-// enters, (S + k u^T)^T q = S^T q + (k . q) u, so that both sums run side by side; q, k, decays of TT tokens staged in LDS for all columns, the
-// next tile's requested ahead of a tile's tokens; the outputs stored a tile at a time.  2048 tokens, 16 heads, delta rule (us): 470 with 8 rows a
-// lane and tiles of 16 tokens; 425 with 4 rows, 392 with stores a tile, 371 with the two sums side by side, 319 with tiles of 32 tokens, 306
-// with whole tiles requested without bounds; operands fetched further ahead than two tokens: no change.  Sums over the rows add a lane's R
-// products in order, then the P lanes: an order fixed by `dim` alone.
+// neighbouring lanes, R rows each, in registers for the whole step.  q, k, decays of TT tokens are staged in LDS for all columns, the next tile's
+// requested ahead of a tile's tokens; a whole tile's outputs are stored together.
+// What bounds it is the serial chain over the tokens: a token's S^T k has to be summed over the lanes before its row enters S.  S^T q is taken of the
+// state before the token's row enters, (S + k u^T)^T q = S^T q + (k . q) u, so that both sums run side by side.
+//  - Few columns (less than two workgroups a CU at R = 8): R = 4 gives twice the workgroups, and tiles of 32 tokens cover the way to memory.  2048
+//    tokens, 16 heads of 128 x 128, delta rule: 306 us (470 with R = 8 and tiles of 16 tokens, the sums one after the other).
+//  - More: the SIMDs are full, and R = 8 takes half the instructions for the sums of an element; tiles of 16 tokens leave room for four workgroups
+//    a CU.  8 sequences of 256 tokens: 132 us (R = 4: 158).
+//  - Steps of at most 16 tokens a sequence, where the host knows it: R = 4, tiles of 16 (8 sequences of 4 tokens: 9.8 us; R = 8 12.9).
+//  - One token a sequence: nothing to stage ahead (TT = 1: a fraction of the LDS and registers, 8 sequences 7.3 us, 32 21; with tiles 11, 37).
+// Sums over the rows add four rows' products in order, then pairs of neighbours, pairs of pairs and so on up to `dim`, in a lane or across lanes: one
+// order, fixed by `dim` alone, whatever the form.
 // sum over the P neighbouring lanes that share a column (P a power of two, lanes aligned to P), left in all of them.  Inside a row of 16
 // lanes the partner comes by DPP (quad permutes, then mirrors of half a row and of a row: after each step the lanes of a group hold one
 // value, so a mirror is as good as an xor); beyond 16 lanes by permlane swaps.  One fixed order for a given P.
@@ -738,18 +741,16 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
-// P, the presence of per-row decays and of the delta rule are template parameters: the tokens of a whole tile are one straight line of code, so
+// R, P, TT, the presence of per-row decays and of the delta rule are template parameters: the tokens of a whole tile are one straight line of code, so
 // the LDS reads of the tokens ahead are in flight while a token's sums run.
 // DECAY 0: one constant per head; 1: one per row and key channel; 2: one per row and head.  ACT: q, k, v pass silu on their way into LDS.
 // BONUS (per-channel decays, no delta rule): the output is read before the decay, this token enters it through bonus (bs: sum_d q_d bonus_d k_d).
-// tokens staged at a time: the next tile's operands are requested ahead of a tile's tokens, whose time has to cover their way from memory
-// (one lane a column, keys of up to 4: the values and outputs of 32 tokens would take 64 KB)
-constexpr int scan_tile(int dimP) { return dimP > 128 || dimP <= 4 ? 16 : 32; }
-template <int R, int P, int DECAY, bool BETA, bool ACT, bool BONUS = false>
+template <int R, int P, int TT, int DECAY, bool BETA, bool ACT, bool BONUS = false>
 __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  constexpr int dimP = P * R, CPB = 256 / P, d4n = dimP / 4, TT = scan_tile(dimP), NL = (TT * d4n + 255) / 256;  // tokens a tile; 16-byte loads a thread and array for one
-  static_assert(d4n == P, "the lanes that stage a token's row are as many as those that hold a column");
+  constexpr int dimP = P * R, CPB = 256 / P, d4n = dimP / 4, NL = (TT * d4n + 255) / 256;  // 16-byte loads a thread and array for a tile
+  constexpr int AHEAD = R == 4 ? 2 : 1, SETS = 2 * AHEAD, NH = R / 4;  // tokens whose operands are fetched ahead; parts of a lane's sums
+  static_assert(d4n <= 64 && R % 4 == 0, "a token's row is staged by lanes of one wave");
   const int dim = a.dim, vdim = a.vdim;
   float* ks = lds;                   // [TT][dimP]
   float* qs = ks + TT * dimP;        // [TT][dimP]
@@ -793,11 +794,11 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
     return o;
   };
   // A whole tile of whole 16-byte rows, the common case, is requested without a bound a load: a thread's row of the u-th load is u * RS rows on.
-  const bool plain = vec && dim == dimP && TT * P >= 256;
-  constexpr int RS = 256 / P;
-  const float* kp = a.k + (size_t)(t0 + tid / P) * a.ldk + hq * dim + tid % P * 4;
-  const float* qp = a.q + (size_t)(t0 + tid / P) * a.ldq + hq * dim + tid % P * 4;
-  const float* dp = DECAY == 1 ? a.decay + (size_t)(t0 + tid / P) * a.ldd + h * dim + tid % P * 4 : nullptr;
+  const bool plain = vec && dim == dimP && TT * d4n >= 256;
+  constexpr int RS = 256 / d4n;
+  const float* kp = a.k + (size_t)(t0 + tid / d4n) * a.ldk + hq * dim + tid % d4n * 4;
+  const float* qp = a.q + (size_t)(t0 + tid / d4n) * a.ldq + hq * dim + tid % d4n * 4;
+  const float* dp = DECAY == 1 ? a.decay + (size_t)(t0 + tid / d4n) * a.ldd + h * dim + tid % d4n * 4 : nullptr;
   auto request = [&](int i0) {
     const int nt = min(TT, n - i0);
     if (plain && nt == TT) {
@@ -830,11 +831,11 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
     if (BETA && tid < nt) bn = a.beta[(size_t)(t0 + i0 + tid) * a.ldb + h];
     if (DECAY == 2 && tid < nt) gn = a.decay[(size_t)(t0 + i0 + tid) * a.ldd + h];
   };
-  auto deposit = [&]() {
+  auto deposit = [&](int nt) {
 #pragma unroll
     for (int u = 0; u < NL; u++) {
       const int e = tid + u * 256;
-      if (e < TT * d4n) {
+      if (e < nt * d4n) {
         float4 kk = kn[u], qv = qn[u];
         if (ACT) {
           kk.x = siluf_(kk.x), kk.y = siluf_(kk.y), kk.z = siluf_(kk.z), kk.w = siluf_(kk.w);
@@ -844,8 +845,8 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
         qv.x *= a.q_scale, qv.y *= a.q_scale, qv.z *= a.q_scale, qv.w *= a.q_scale;
         *(float4*)(qs + e * 4) = qv;
         if (DECAY == 1) *(float4*)(ds + e * 4) = dn[u];
-        if (!BONUS) {  // (the d4n = P neighbouring lanes that hold a token's row; zeros beyond its size)
-          const float c = group_sum<P>(fmaf(kk.x, qv.x, fmaf(kk.y, qv.y, fmaf(kk.z, qv.z, kk.w * qv.w))));
+        if (!BONUS) {  // (the d4n neighbouring lanes that hold a token's row; zeros beyond its size)
+          const float c = group_sum<d4n>(fmaf(kk.x, qv.x, fmaf(kk.y, qv.y, fmaf(kk.z, qv.z, kk.w * qv.w))));
           if (e % d4n == 0) cs[e / d4n] = c;
         }
       }
@@ -860,7 +861,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
 #pragma unroll
     for (int u = 0; u < NV; u++) {
       const int e = tid + u * 256;
-      if (e < vcount) vs[e] = ACT ? siluf_(vbuf[u]) : vbuf[u];
+      if (e < nt * CPB) vs[e] = ACT ? siluf_(vbuf[u]) : vbuf[u];
     }
     if (BETA && tid < TT) bs[tid] = bn;
     if (DECAY == 2 && tid < TT) gs[tid] = gn;
@@ -878,12 +879,12 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
   for (int i0 = 0; i0 < n; i0 += TT) {
     const int nt = min(TT, n - i0);
     __syncthreads();
-    deposit();
+    deposit(nt);
     if (i0 > 0) leave(i0 - TT, TT);
     __syncthreads();
     if (i0 + TT < n) request(i0 + TT);
-    // a token's operands come from LDS two tokens ahead of its arithmetic (16-byte reads): one token's work is shorter than their way
-    float kv[4][R], qv[4][R], dv[4][R], uv[4], bv[4], gv[4], cv[4];
+    // a token's operands come from LDS ahead of its arithmetic (16-byte reads), two tokens with 4 rows a lane: one token's work is shorter than their way
+    float kv[SETS][R], qv[SETS][R], dv[SETS][R], uv[SETS], bv[SETS], gv[SETS], cv[SETS];
     auto fetch = [&](int i, int w) {
 #pragma unroll
       for (int j = 0; j < R; j += 4) {
@@ -900,52 +901,61 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
       if (!BONUS) cv[w] = cs[i];
       if (DECAY == 2) gv[w] = gs[i];
     };
-    auto token = [&](int i, int w) {
+    auto lane_sum = [](const float (&v)[NH][2]) {  // (8 rows as two lanes of 4 would add theirs)
+      float t = v[0][0] + v[0][1];
+      if constexpr (NH == 2) t += v[1][0] + v[1][1];
+      return t;
+    };
+    auto token = [&](int i, int w, auto whole) {  // outputs of a whole tile leave together, those of a part of one at once
+      auto put = [&](float o) {
+        if (r == 0 && whole) os[i * CPB + cl] = o;
+        if (r == 0 && !whole && col) a.out[(size_t)(t0 + i0 + i) * a.ldo + h * vdim + c] = o;
+      };
       if (BONUS) {
         const float u = uv[w];
-        float o0 = 0.f, o1 = 0.f;
+        float o[NH][2] = {};
 #pragma unroll
-        for (int j = 0; j < R; j += 2) {
-          o0 = fmaf(S[j], qv[w][j], o0), o1 = fmaf(S[j + 1], qv[w][j + 1], o1);
-          S[j] = fmaf(kv[w][j], u, S[j] * dv[w][j]), S[j + 1] = fmaf(kv[w][j + 1], u, S[j + 1] * dv[w][j + 1]);
+        for (int j = 0; j < R; j++) {
+          o[j / 4][j & 1] = fmaf(S[j], qv[w][j], o[j / 4][j & 1]);
+          S[j] = fmaf(kv[w][j], u, S[j] * dv[w][j]);
         }
-        const float o_ = fmaf(bv[w], u, group_sum<P>(o0 + o1));
-        if (r == 0) os[i * CPB + cl] = o_;
+        put(fmaf(bv[w], u, group_sum<P>(lane_sum(o))));
         return;
       }
 #pragma unroll
       for (int j = 0; j < R; j++) S[j] *= DECAY == 1 ? dv[w][j] : (DECAY == 2 ? gv[w] : hd);
       // S^T k and S^T q of the decayed state side by side (two chains each; their sum order is fixed): the output of the new state is
       // (S + k u^T)^T q = S^T q + (k . q) u, so it does not wait for u, and one chain's steps fill the other's wait states
-      float u = uv[w], d0 = 0.f, d1 = 0.f, o0 = 0.f, o1 = 0.f;
+      float u = uv[w], d[NH][2] = {}, o[NH][2] = {};
 #pragma unroll
-      for (int j = 0; j < R; j += 2) {
-        if (BETA) d0 = fmaf(S[j], kv[w][j], d0), d1 = fmaf(S[j + 1], kv[w][j + 1], d1);
-        o0 = fmaf(S[j], qv[w][j], o0), o1 = fmaf(S[j + 1], qv[w][j + 1], o1);
+      for (int j = 0; j < R; j++) {
+        if (BETA) d[j / 4][j & 1] = fmaf(S[j], kv[w][j], d[j / 4][j & 1]);
+        o[j / 4][j & 1] = fmaf(S[j], qv[w][j], o[j / 4][j & 1]);
       }
-      if (BETA) u = bv[w] * (u - group_sum<P>(d0 + d1));
+      if (BETA) u = bv[w] * (u - group_sum<P>(lane_sum(d)));
 #pragma unroll
       for (int j = 0; j < R; j++) S[j] = fmaf(kv[w][j], u, S[j]);
-      const float o_ = fmaf(cv[w], u, group_sum<P>(o0 + o1));
-      if (r == 0) os[i * CPB + cl] = o_;
+      put(fmaf(cv[w], u, group_sum<P>(lane_sum(o))));
     };
     if (nt == TT) {
-      fetch(0, 0);
-      fetch(1, 1);
+#pragma unroll
+      for (int i = 0; i < AHEAD && i < TT; i++) fetch(i, i);
 #pragma unroll
       for (int i = 0; i < TT; i++) {
-        if (i + 2 < TT) fetch(i + 2, (i + 2) & 3);
-        token(i, i & 3);
+        if (i + AHEAD < TT) fetch(i + AHEAD, (i + AHEAD) % SETS);
+        token(i, i % SETS, std::true_type{});
       }
     } else {
       for (int i = 0; i < nt; i++) {
         fetch(i, 0);
-        token(i, 0);
+        token(i, 0, std::false_type{});
       }
     }
   }
-  __syncthreads();
-  if (n > 0) leave((n - 1) / TT * TT, (n - 1) % TT + 1);
+  if (n > 0 && n % TT == 0) {
+    __syncthreads();
+    leave(n - TT, TT);
+  }
   if (col)
 #pragma unroll
     for (int j = 0; j < R; j++)
@@ -1246,47 +1256,78 @@ void vra_stack_sigmoid_pow(const float* z, int ldz, float* out, int ldo, int T, 
   launch_checked("stack decay", [&] { stk_sigmoid_pow_kernel<<<grid, 256, 0, as_stream(stream)>>>(z, ldz, out, ldo, n, total, inv_tau); });
 }
 
-extern "C" int32_t vra_stack_op_linear_scan_lds(int32_t dim) {
-  if (dim < 1 || dim > 256) return -1;
-  int P = 1;
-  while (P * 4 < dim) P <<= 1;
-  const int TT = scan_tile(P * 4);
-  return (int32_t)((TT * P * 4 * 3 + 2 * TT * (256 / P) + 3 * TT) * sizeof(float));
+namespace {
+struct ScanForm {
+  int R, P, TT;  // rows of the state a lane, lanes a column, tokens staged at a time
+};
+// (the lines: measured at 1..32 sequences, 8..32 heads of 32..256 channels, 1..1000 tokens)
+ScanForm scan_form(const StkScanArgs& a) {
+  ScanForm f = {4, 1, 32};
+  while (f.P * 4 < a.dim) f.P <<= 1;
+  if (!a.cu_q) return {4, f.P, 1};
+  const bool few = a.max_q > 0 && a.max_q <= 16;
+  const int cols8 = 512 / f.P;  // columns of a workgroup at 8 rows a lane
+  if (a.dim > 32 && !few && (int64_t)((a.vdim + cols8 - 1) / cols8) * a.H * a.B >= 2 * 256) return {8, f.P / 2, 16};
+  f.TT = few || f.P == 1 || f.P == 64 ? 16 : 32;  // (one lane a column: the values and outputs of 32 tokens would take 64 KB of LDS)
+  return f;
+}
+size_t scan_lds_bytes(const ScanForm& f) {
+  return ((size_t)f.TT * f.P * f.R * 3 + (size_t)2 * f.TT * (256 / f.P) + 3 * f.TT) * sizeof(float);
+}
+}  // namespace
+extern "C" int32_t vra_stack_op_linear_scan_lds(int32_t dim, int32_t vdim, int32_t H, int32_t B, int32_t max_q) {
+  if (dim < 1 || dim > 256 || vdim < 1 || H < 1 || B < 1 || max_q < 0) return -1;
+  static const uint32_t ragged[2] = {};
+  StkScanArgs a;
+  a.dim = dim, a.vdim = vdim, a.H = H, a.B = B, a.max_q = max_q, a.cu_q = max_q == 1 ? nullptr : ragged;
+  return (int32_t)scan_lds_bytes(scan_form(a));
 }
 void vra_stack_linear_scan(const StkScanArgs& a, int64_t stream) {
   VRA_CHECK_ARG(a.q && a.k && a.v && a.state && a.state_slots && a.positions && a.out && (a.decay || a.head_decay), "stack linear scan: null pointer");
   VRA_CHECK_ARG(a.B > 0 && a.H > 0 && a.qk_rep >= 1 && a.H % a.qk_rep == 0 && a.dim > 0 && a.dim <= 256 && a.vdim > 0, "stack linear scan: key size at most 256");
-  constexpr int R = 4;
-  int P = 1;
-  while (P * R < a.dim) P <<= 1;
-  const int CPB = 256 / P;
-  const size_t lds = (size_t)vra_stack_op_linear_scan_lds(a.dim);
+  const ScanForm f = scan_form(a);
+  dim3 grid((a.vdim + 256 / f.P - 1) / (256 / f.P), a.H, a.B);
+  const size_t lds = scan_lds_bytes(f);
   VRA_CHECK_ARG(lds <= 64 * 1024, "stack linear scan: staging does not fit LDS");
-  dim3 grid((a.vdim + CPB - 1) / CPB, a.H, a.B);
   hipStream_t st = as_stream(stream);
   const bool decay = a.decay != nullptr, beta = a.beta != nullptr, per_head = decay && a.decay_per_head;
   VRA_CHECK_ARG(decay || !beta, "stack linear scan: the delta rule comes with per-row decays");
   VRA_CHECK_ARG(!a.act_silu || (!decay && !beta), "stack linear scan: the activation on the way in goes with constant decays");
   VRA_CHECK_ARG(!a.bonus || (decay && !per_head && !beta), "stack linear scan: the bonus goes with per-row decays per channel, without the delta rule");
   VRA_CHECK_ARG(!per_head || beta, "stack linear scan: one decay per head and token goes with the delta rule");
-#define STK_SCAN(PV)                                                                                                            \
-  launch_checked("stack linear scan", [&] {                                                                                     \
-    if (a.bonus) stk_linear_scan_kernel<R, PV, 1, false, false, true><<<grid, 256, lds, st>>>(a);                               \
-    else if (per_head) stk_linear_scan_kernel<R, PV, 2, true, false><<<grid, 256, lds, st>>>(a);                                \
-    else if (beta) stk_linear_scan_kernel<R, PV, 1, true, false><<<grid, 256, lds, st>>>(a);                                    \
-    else if (decay) stk_linear_scan_kernel<R, PV, 1, false, false><<<grid, 256, lds, st>>>(a);                                  \
-    else if (a.act_silu) stk_linear_scan_kernel<R, PV, 0, false, true><<<grid, 256, lds, st>>>(a);                              \
-    else stk_linear_scan_kernel<R, PV, 0, false, false><<<grid, 256, lds, st>>>(a);                                             \
+#define STK_SCAN(RV, PV, TV)                                                                                                       \
+  launch_checked("stack linear scan", [&] {                                                                                        \
+    if (a.bonus) stk_linear_scan_kernel<RV, PV, TV, 1, false, false, true><<<grid, 256, lds, st>>>(a);                             \
+    else if (per_head) stk_linear_scan_kernel<RV, PV, TV, 2, true, false><<<grid, 256, lds, st>>>(a);                              \
+    else if (beta) stk_linear_scan_kernel<RV, PV, TV, 1, true, false><<<grid, 256, lds, st>>>(a);                                  \
+    else if (decay) stk_linear_scan_kernel<RV, PV, TV, 1, false, false><<<grid, 256, lds, st>>>(a);                                \
+    else if (a.act_silu) stk_linear_scan_kernel<RV, PV, TV, 0, false, true><<<grid, 256, lds, st>>>(a);                            \
+    else stk_linear_scan_kernel<RV, PV, TV, 0, false, false><<<grid, 256, lds, st>>>(a);                                           \
   })
-  switch (P) {
-    case 1: STK_SCAN(1); break;
-    case 2: STK_SCAN(2); break;
-    case 4: STK_SCAN(4); break;
-    case 8: STK_SCAN(8); break;
-    case 16: STK_SCAN(16); break;
-    case 32: STK_SCAN(32); break;
-    default: STK_SCAN(64); break;
+#define STK_SCAN_P(PV, TV)                   \
+  case PV:                                   \
+    if (f.TT == 1) STK_SCAN(4, PV, 1);       \
+    else if (f.TT == 16) STK_SCAN(4, PV, 16); \
+    else STK_SCAN(4, PV, TV);                \
+    break
+  if (f.R == 8) {
+    switch (f.P) {
+      case 8: STK_SCAN(8, 8, 16); break;
+      case 16: STK_SCAN(8, 16, 16); break;
+      default: STK_SCAN(8, 32, 16); break;
+    }
+    return;
   }
+  switch (f.P) {
+    STK_SCAN_P(1, 16);
+    STK_SCAN_P(2, 32);
+    STK_SCAN_P(4, 32);
+    STK_SCAN_P(8, 32);
+    STK_SCAN_P(16, 32);
+    STK_SCAN_P(32, 32);
+    STK_SCAN_P(64, 16);
+  }
+#undef STK_SCAN_P
 #undef STK_SCAN
 }
 

@@ -1356,7 +1356,7 @@ bool StackModel::recurrent_tail(const StackLayer& L, const InputMetadata& md, co
 }
 
 static void scan_common(StkScanArgs& sc, const StackLayer& L, const InputMetadata& md, float* out) {
-  sc.state = L.state, sc.state_slots = md.state_slots, sc.positions = md.positions, sc.cu_q = md.is_prefill ? md.cu_seqlens_q : nullptr;
+  sc.state = L.state, sc.state_slots = md.state_slots, sc.positions = md.positions, sc.cu_q = md.is_prefill ? md.cu_seqlens_q : nullptr, sc.max_q = md.is_prefill ? md.max_seqlen_q : 1;
   sc.out = out, sc.ldo = L.s_heads() * L.s_vdim(), sc.B = md.n_seqs, sc.H = L.s_heads(), sc.dim = L.s_dim(), sc.vdim = L.s_vdim();
 }
 
