@@ -36,3 +36,14 @@ def test_linear_recurrence_stages_one_token_for_one(dim):
     """a decode step's workgroups stage one token: q, k, decays, value and output of it and three numbers"""
     P = max(1, dim // 4)
     assert _lib.load().vra_stack_op_linear_scan_lds(dim, dim, 16, 8, 1) == 4 * (3 * dim + 2 * (256 // P) + 3)
+
+
+@pytest.mark.parametrize("experts", [4, 16, 64])
+@pytest.mark.parametrize("pairs", [1, 40, 1000, 16384])
+def test_expert_rows(pairs, experts):
+    """the row space a mixture sizes its buffers by: what its granule can need and no more, and enough for every shorter step"""
+    rows = _lib.load().vra_stack_op_expert_rows
+    for tiles in (0, 1):
+        pad = 16 if pairs // experts < (96 if tiles else 128) else (128 if tiles else 64)
+        assert pairs + experts * (pad - 1) <= rows(pairs, experts, tiles) < pairs + experts * (pad - 1) + pad
+        assert rows(pairs, experts, tiles) >= max(rows(n, experts, tiles) for n in range(1, pairs + 1, max(1, pairs // 97)))

@@ -47,6 +47,8 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream);
 // rows per granule the grouped launches of an M-row problem over `groups` groups want (16, 64, or 128 where `tiles128`: both products of the
 // expert are bf16 with K a multiple of 64)
 int vra_stack_gemm_granule(int rows, int groups, bool tiles128);
+// rows of the row space that `pairs` token-expert pairs over `experts` experts take with that granule; the most of any smaller number of pairs, too
+extern "C" int32_t vra_stack_op_expert_rows(int32_t pairs, int32_t experts, int32_t tiles128);
 // out[r] = round_bf16(a[row_token[r]] * row_scale[r]) for the rows that hold a pair (row_token >= 0); the others are left alone
 void vra_stack_scale_rows(const void* a, int W, const int* row_token, const float* row_scale, void* out, int rows, int64_t stream);
 

@@ -1351,6 +1351,10 @@ int vra_stack_gemm_granule(int rows, int groups, bool tiles128) {
   if (groups > 0 && tiles128 && rows / groups >= 96) return 128;
   return groups > 0 && rows / groups >= 128 ? 64 : 16;
 }
+int32_t vra_stack_op_expert_rows(int32_t pairs, int32_t experts, int32_t tiles128) {
+  const int g = vra_stack_gemm_granule(pairs, experts, tiles128 != 0);
+  return (pairs + experts * (g - 1) + g - 1) / g * g;
+}
 void vra_stack_scale_rows(const void* a, int W, const int* row_token, const float* row_scale, void* out, int rows, int64_t stream) {
   VRA_CHECK_ARG(a && row_token && row_scale && out && rows > 0 && W > 0 && W % 8 == 0, "stack scale rows: null pointer or bad shape");
   launch_checked("stack scale rows", [&] { stk_scale_rows_kernel<<<rows, 256, 0, as_stream(stream)>>>((const uint16_t*)a, W, row_token, row_scale, (uint16_t*)out); });

@@ -1011,7 +1011,9 @@ bool StackModel::init_buffers(int max_tokens, int max_seqs) {
       roc = std::max(roc, sh * sv);
     }
   }
-  max_rows_ = (int)round_up((int)(T * std::max<size_t>(top, 1) + experts * 127), 128);
+  max_rows_ = round_up((int)(T * std::max<size_t>(top, 1)), 16);
+  for (const StackLayer& L : layers_)
+    if (L.mlp == 2) max_rows_ = std::max(max_rows_, vra_stack_op_expert_rows((int)T * L.top, L.experts, tiles128(L)));
   for (const StackLayer& L : layers_) {
     if (L.mlp == 1) zc = std::max(zc, T * L.ff), actc = std::max(actc, T * L.ff);
     if (L.mlp == 2 && L.n_identity > 0) experts = std::max(experts, (size_t)L.experts);
@@ -1073,9 +1075,8 @@ static bool take_stack_err(std::string& error, const char* where) {
 
 // both products of an expert run on the 128-row tiles of the row-major prompt GEMM
 bool StackModel::tiles128(const StackLayer& L) const {
-  const int64_t most = 0x7FFF0000ll;
-  return dt_ == VRA_BF16 && width_ % 64 == 0 && L.ffp % 64 == 0 && (int64_t)max_rows_ * std::max(width_, L.ffp) * 2 < most &&
-         (int64_t)2 * L.ffp * width_ * 2 < most;
+  const int64_t most = 0x7FFF0000ll, rows = vra_stack_op_expert_rows(max_tokens_ * L.top, L.experts, 1);
+  return dt_ == VRA_BF16 && width_ % 64 == 0 && L.ffp % 64 == 0 && rows * std::max(width_, L.ffp) * 2 < most && (int64_t)2 * L.ffp * width_ * 2 < most;
 }
 // gate / up -> clamped gated activation -> down for `rows` logical rows (one expert per granule, or one weight set for all):
 // bf16: the activation is the epilogue of the gate / up launch; f32: product, activation and product as three launches
@@ -1130,7 +1131,7 @@ bool StackModel::feed_forward(const StackLayer& L, int T, int64_t stream) {
   if (L.mlp == 2) {
     const int P = T * L.top;
     const int granule = vra_stack_gemm_granule(P, L.experts, tiles128(L));
-    const int rows = round_up(P + L.experts * (granule - 1), granule);
+    const int rows = vra_stack_op_expert_rows(P, L.experts, tiles128(L));
     if (rows > max_rows_) return error = "feed-forward: more expert rows than the buffers hold", false;
     vra_stack_moe_sort(pair_expert_, pair_weight_, P, L.top, L.experts, granule, rows, row_token_, row_scale_, row_pair_, tile_group_, stream);
     if (take_stack_err(error, "expert rows")) return false;
@@ -1527,7 +1528,7 @@ bool StackModel::forward_sandwich(const InputMetadata& md, int64_t stream) {
       if (!seam(L.norm2_w, L.norm2_b, L.norm2_alpha, &L, true)) return false;
       const int P = T * L.top;
       const int granule = vra_stack_gemm_granule(P, L.experts, tiles128(L));
-      const int rows = round_up(P + L.experts * (granule - 1), granule);
+      const int rows = vra_stack_op_expert_rows(P, L.experts, tiles128(L));
       if (rows > max_rows_) return error = "feed-forward: more expert rows than the buffers hold", false;
       vra_stack_moe_sort(pair_expert_, pair_weight_, P, L.top, L.experts, granule, rows, row_token_, row_scale_, row_pair_, tile_group_, stream);
       if (take_stack_err(error, "expert rows")) return false;
