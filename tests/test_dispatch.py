@@ -47,3 +47,18 @@ def test_expert_rows(pairs, experts):
         pad = 16 if pairs // experts < (96 if tiles else 128) else (128 if tiles else 64)
         assert pairs + experts * (pad - 1) <= rows(pairs, experts, tiles) < pairs + experts * (pad - 1) + pad
         assert rows(pairs, experts, tiles) >= max(rows(n, experts, tiles) for n in range(1, pairs + 1, max(1, pairs // 97)))
+
+
+# us, 32 columns a workgroup / 16 (MI355X, weights not in any cache)
+@pytest.mark.parametrize("M,N,K,want", [
+    (8, 2048, 8192, 16),  # 22.9 / 14.6
+    (32, 2048, 256, 16),  # 5.3 / 4.4
+    (17, 3072, 8192, 32),  # 25.4 / 31.1
+    (32, 4000, 4096, 32),  # 15.9 / 18.1
+    (32, 3072, 512, 32),  # 5.6 / 6.2
+    (8, 8000, 4096, 16),  # 17.9 / 16.2
+    (8, 6144, 512, 32),  # 5.1 / 5.6
+])
+def test_columns_of_few_row_products(M, N, K, want):
+    L = _lib.load()
+    assert L.vra_stack_op_gemm_few_columns(M, N, K, 1, 0) == want and L.vra_stack_op_gemm_few_columns(M, N, K, 1, 1) == 32

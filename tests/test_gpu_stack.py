@@ -374,8 +374,9 @@ def test_polynorm_row_sizes(dt, F):
     test_polynorm(dt, F)
 
 
-# few rows: 16 columns a workgroup below 256 workgroups, 32 from there on; both sides of the line, and K that gives some waves nothing
-@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (5, 40, 72), (16, 8160, 64), (16, 8192, 64), (17, 4064, 328), (32, 4096, 256), (3, 2000, 2048)])
+# few rows: 16 or 32 columns a workgroup; both sides of the lines (vra_stack_op_gemm_few_columns), and K that gives some waves nothing
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (5, 40, 72), (16, 8160, 64), (16, 8192, 64), (17, 4064, 328), (32, 4096, 256), (3, 2000, 2048), (16, 4096, 72),
+                                   (16, 4128, 72), (17, 2048, 64), (17, 2080, 64), (16, 4128, 2048), (16, 4128, 4104)])
 def test_gemm_few_rows(M, N, K):
     L = _lib.load()
     r = np.random.default_rng(M + N + K)
