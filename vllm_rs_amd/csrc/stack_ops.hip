@@ -61,8 +61,11 @@ __global__ __launch_bounds__(256) void stk_embed_sinpos_kernel(const uint32_t* i
 }
 
 // ------------------------------------------------------------------------------------------------ grouped RMS norm (+ router)
-template <typename T>
-__global__ __launch_bounds__(256) void stk_group_norm_kernel(StkNormArgs a) {
+// (ROUTER a template parameter and 8 waves a SIMD: a norm that carries the router's registers, or a router with the 74 it would take, leaves room for 6
+// waves, and 2048 rows are two rounds of workgroups.  2048 rows, us: norm of 2048 7.6 -> 6.8, of 2051 12.4 -> 9.5; with eight router
+// outputs 21.1 -> 19.1, of 1001 17.6 -> 13.3)
+template <typename T, bool ROUTER>
+__global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
   extern __shared__ float lds[];
   float* xs = lds;                      // [W] the row, then the normalised row
   float* rs = lds + a.W;                // [groups] 1 / rms
@@ -84,49 +87,65 @@ __global__ __launch_bounds__(256) void stk_group_norm_kernel(StkNormArgs a) {
     }
     __syncthreads();
   };
-  // (four values a load where rows and groups allow it, the weights with them: a row's parts arrive in one round trip instead of W / 256, and the
-  // row stays in registers: 8 rows of 2048: 6.6 us, now 4.0)
-  auto row = [&](auto width, auto rounds) {
-    constexpr int N = decltype(width)::value, R = decltype(rounds)::value;
-    typedef float vec __attribute__((ext_vector_type(N)));
-    vec keep[R], wt[R];
-    const float gt = a.gate_in ? a.gate_in[t] : 1.f;
+  const float gt = a.gate_in ? a.gate_in[t] : 1.f;
+  const bool quads = W % 4 == 0 && gs % 4 == 0 && (((uintptr_t)a.x | (uintptr_t)a.x_out | (uintptr_t)a.o | (uintptr_t)a.p1 | (uintptr_t)a.p2 | (uintptr_t)a.w) % 16) == 0;
+  if (quads) {
+    // (four values a load where rows and groups allow it, the weights with them: a row's parts arrive in one round trip instead of W / 256, and the
+    // row stays in registers: 8 rows of 2048: 6.6 us, now 4.0)
+    constexpr int R = 2;
+    f32x4 keep[R], wt[R];
     auto load = [&](int c) {
-      vec v = *(const vec*)(x + c);
+      f32x4 v = *(const f32x4*)(x + c);
       if (a.o) {
-        vec s = *(const vec*)(a.o + (size_t)t * W + c);
-        for (int j = 0; j < a.n1; j++) s += *(const vec*)(a.p1 + ((size_t)t * a.n1 + j) * W + c);
-        if (a.p2) s += gt * *(const vec*)(a.p2 + (size_t)t * W + c);
+        f32x4 s = *(const f32x4*)(a.o + (size_t)t * W + c);
+        for (int j = 0; j < a.n1; j++) s += *(const f32x4*)(a.p1 + ((size_t)t * a.n1 + j) * W + c);
+        if (a.p2) s += gt * *(const f32x4*)(a.p2 + (size_t)t * W + c);
         v += a.mult * s;
-        *(vec*)(a.x_out + (size_t)t * W + c) = v;
+        *(f32x4*)(a.x_out + (size_t)t * W + c) = v;
       }
-      *(vec*)(xs + c) = v;
+      *(f32x4*)(xs + c) = v;
       return v;
     };
-    auto put = [&](int c, vec v, vec w) {
-      const vec y = v * rs[c / gs] * w;
-      if (a.router_w) *(vec*)(xs + c) = y;
+    auto put = [&](int c, f32x4 v, f32x4 w) {
+      const f32x4 y = v * rs[c / gs] * w;
+      if (ROUTER) *(f32x4*)(xs + c) = y;
 #pragma unroll
-      for (int e = 0; e < N; e++) El<T>::st(h + c + e, y[e]);
+      for (int e = 0; e < 4; e++) El<T>::st(h + c + e, y[e]);
     };
 #pragma unroll
     for (int n = 0; n < R; n++) {
-      const int c = threadIdx.x * N + n * 256 * N;
-      if (c < W) wt[n] = *(const vec*)(a.w + c), keep[n] = load(c);
+      const int c = threadIdx.x * 4 + n * 1024;
+      if (c < W) wt[n] = *(const f32x4*)(a.w + c), keep[n] = load(c);
     }
-    for (int c = threadIdx.x * N + R * 256 * N; c < W; c += 256 * N) load(c);
+    for (int c = threadIdx.x * 4 + R * 1024; c < W; c += 1024) load(c);
     sums();
 #pragma unroll
     for (int n = 0; n < R; n++) {
-      const int c = threadIdx.x * N + n * 256 * N;
+      const int c = threadIdx.x * 4 + n * 1024;
       if (c < W) put(c, keep[n], wt[n]);
     }
-    for (int c = threadIdx.x * N + R * 256 * N; c < W; c += 256 * N) put(c, *(const vec*)(xs + c), *(const vec*)(a.w + c));
-  };
-  const bool quads = W % 4 == 0 && gs % 4 == 0 && (((uintptr_t)a.x | (uintptr_t)a.x_out | (uintptr_t)a.o | (uintptr_t)a.p1 | (uintptr_t)a.p2 | (uintptr_t)a.w) % 16) == 0;
-  if (quads) row(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{});
-  else row(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
-  if (!a.router_w) return;
+    for (int c = threadIdx.x * 4 + R * 1024; c < W; c += 1024) put(c, *(const f32x4*)(xs + c), *(const f32x4*)(a.w + c));
+  } else {
+    if (a.o) {
+      for (int c = threadIdx.x; c < W; c += 256) {
+        float s = a.o[(size_t)t * W + c];
+        for (int j = 0; j < a.n1; j++) s += a.p1[((size_t)t * a.n1 + j) * W + c];
+        if (a.p2) s += gt * a.p2[(size_t)t * W + c];
+        const float v = x[c] + a.mult * s;
+        a.x_out[(size_t)t * W + c] = v;
+        xs[c] = v;
+      }
+    } else {
+      for (int c = threadIdx.x; c < W; c += 256) xs[c] = x[c];
+    }
+    sums();
+    for (int c = threadIdx.x; c < W; c += 256) {
+      const float v = xs[c] * rs[c / gs] * a.w[c];
+      if (ROUTER) xs[c] = v;
+      El<T>::st(h + c, v);
+    }
+  }
+  if constexpr (!ROUTER) return;
   __syncthreads();
   const int nz = a.n_router + (a.gate_row ? 1 : 0);
   const T* rw = (const T*)a.router_w;
@@ -1471,8 +1490,10 @@ void vra_stack_group_norm(const StkNormArgs& a, int dtype, int64_t stream) {
   VRA_CHECK_ARG(!a.router_w || (a.pair_expert && a.pair_weight && a.top >= 1 && a.top <= a.n_router && (!a.gate_row || a.gate_out)), "stack norm: router outputs");
   const size_t lds = ((size_t)a.W + a.groups + a.n_router + 2) * sizeof(float);
   VRA_CHECK_ARG(lds <= 64 * 1024, "stack norm: row does not fit LDS");
-  if (dtype == VRA_F32) launch_checked("stack norm", [&] { stk_group_norm_kernel<float><<<a.T, 256, lds, as_stream(stream)>>>(a); });
-  else launch_checked("stack norm", [&] { stk_group_norm_kernel<uint16_t><<<a.T, 256, lds, as_stream(stream)>>>(a); });
+  launch_checked("stack norm", [&] {
+    if (dtype == VRA_F32) a.router_w ? stk_group_norm_kernel<float, true><<<a.T, 256, lds, as_stream(stream)>>>(a) : stk_group_norm_kernel<float, false><<<a.T, 256, lds, as_stream(stream)>>>(a);
+    else a.router_w ? stk_group_norm_kernel<uint16_t, true><<<a.T, 256, lds, as_stream(stream)>>>(a) : stk_group_norm_kernel<uint16_t, false><<<a.T, 256, lds, as_stream(stream)>>>(a);
+  });
 }
 
 void vra_stack_moe_sort(const int* pair_expert, const float* pair_weight, int P, int top, int n_groups, int granule, int max_rows, int* row_token,
