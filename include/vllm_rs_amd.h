@@ -117,6 +117,10 @@ void vra_wna16_gate_up_silu(const void* in, const void* qw_gate, const void* sc_
  * 'M').  0: a shape they refuse. */
 int32_t vra_wna16_kernel(int32_t pair, int32_t m, int32_t k, int32_t n, int32_t group_size, int32_t is_awq, int32_t has_norm,
                          int32_t has_bias, int32_t has_residual);
+/* the same products (qw_up null: a single one) on a named kernel, 64 rows up and row-major scales: 'D' (64-row tiles), 'd' (32-row tiles) or 'M' */
+void vra_wna16_gemm_on(int32_t kernel, const void* in, const void* qweight_tiled, const void* scales, const void* qzeros, const void* qw_up,
+                       const void* sc_up, const void* qz_up, const void* bias, const void* residual, void* out, int32_t m, int32_t k,
+                       int32_t n, int32_t group_size, int32_t is_awq, int32_t dtype, int64_t stream);
 /* NormX::forward + QLinear::forward in one call (others.rs:11-29 in front of wna16.rs:263-306):
  * out = rmsnorm(in, norm_weight, eps)·W (+ bias).  Decode batches of 1..4 rows run fused (the
  * normalised activations never reach HBM); other shapes write rmsnorm(in) to `xn_workspace`
@@ -282,6 +286,12 @@ void vra_swap_blocks(const void* src, void* dst, const int64_t* h_pairs, int32_t
  * (llama.rs:317-319): values are rounded to `dtype` first, then widened. */
 void vra_dense_gemm(const void* x, const void* w, const void* bias, void* out, int32_t m, int32_t k,
                     int32_t n, int32_t dtype, int32_t out_dtype, int64_t stream);
+/* the same product of 33 rows up on a named tile of the row-major prompt GEMM (rows / 64 * 16 + columns / 64: 0x12, 0x22 or 0x24): `nseg` (1..3) tensors of
+ * n[s] columns side by side, each with its own bias (or null) and output [m, n[s]], or (pair, nseg 2) silu(x . w[0]) * (x . w[1]) into
+ * out[0].  The tile changes no bit of the result. */
+void vra_dense_gemm_tile(int32_t tile, const void* x, const void* const* w, const void* const* bias, const int32_t* n, int32_t nseg,
+                         int32_t pair, const void* residual, void* const* out, int32_t out_f32, int32_t m, int32_t k, int32_t dtype,
+                         int64_t stream);
 /* logits.argmax(-1) (logits_processor.rs:67-70): first maximal index per row. */
 void vra_argmax_f32(const float* logits, uint32_t* out, int32_t rows, int32_t cols, int64_t stream);
 /* lm_head + greedy sampling as one launch (llama.rs:311-320 followed by logits_processor.rs:67-70): f32 logits as
@@ -645,6 +655,10 @@ void vra_stack_op_group_norm(const float* x, const float* w, void* h, int32_t T,
 void vra_stack_op_gemm(const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32,
                        int32_t M, int32_t N, int32_t K, float alpha, const int32_t* tile_group, int32_t granule, const int32_t* a_row,
                        const float* a_scale, const int32_t* out_row, int32_t epi, float limit, int32_t dtype, int64_t stream);
+/* the bf16 product of more than 32 rows on a named tile (0x12, 0x22, 0x24: rows / 64 * 16 + columns / 64), granules of a tile's rows */
+void vra_stack_op_gemm_tile(int32_t tile, const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32,
+                            int32_t M, int32_t N, int32_t K, const int32_t* tile_group, const int32_t* a_row, int32_t a_rows,
+                            const int32_t* out_row, int32_t epi, float limit, int64_t stream);
 /* columns a workgroup of vra_stack_op_gemm takes at up to 32 rows in bf16 (pair: with the gated epilogue): 16 or 32, with the same sums */
 int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t pair);
 /* rows of the row space that a model gives `pairs` token-expert pairs over `experts` experts (tiles128: its products run on 128-row tiles) */

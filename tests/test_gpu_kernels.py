@@ -116,51 +116,75 @@ def test_gate_up_silu(M):
     assert_close_dt(got, ref, BF16, max_ulp=3.0, max_mismatch_frac=0.04, name="gate_up_silu", abs_floor=4e-3)
 
 
-# ---------------------------------------------------------------- kernel D (many rows: prefill)
-# shapes that the default dispatch routes to gemm_q4_big_kernel: M >= 256 and >= 192 workgroup tiles (256 columns x 128 rows)
-@pytest.mark.parametrize("N", [16384, 12288])   # 64 column tiles x 3 row tiles of 128 (4 m-tiles per wave) / 48 x 5 row tiles of 64 (2)
+# ---------------------------------------------------------------- kernels D and M (64 rows up: prefill)
+def wna16_on(kernel, x, q, M, K, N, gs, dt, awq=False, bias=None, residual=None, up=None, off=(0, 0)):
+    """the product (up: the gate / up pair) on the kernel that the shape is dispatched to (None) or on a named one: 'D' 64-row tiles, 'd' 32-row tiles, 'M';
+    x and the scales `off` 16-bit elements behind a 16-byte boundary"""
+    keep = []
+
+    def put(a, n=0):
+        keep.append(ops.dev(np.concatenate([np.zeros(n, a.dtype), a.reshape(-1)]) if n else a))
+        return keep[-1].ptr + n * a.itemsize
+
+    def tensor(t):
+        keep.append(ops.marlin_weight_repack(ops.dev(t["qweight"]), t["qweight"].shape, 4, awq))
+        return keep[-1].ptr, put(t["scales"], off[1]), put(t["qzeros"]) if awq else None
+    w = tensor(q)
+    wu = tensor(up) if up is not None else (None, None, None)
+    b, r = (put(a) if a is not None else None for a in (bias, residual))
+    xp, out = put(x, off[0]), ops.DevBuf(M * N * 2)
+    if kernel:
+        ops.lib().vra_wna16_gemm_on(ord(kernel), xp, *w, *wu, b, r, out.ptr, M, K, N, gs, int(awq), dt, 0)
+    elif up is not None:
+        ops.lib().vra_wna16_gate_up_silu(xp, *w, *wu, out.ptr, M, K, N, gs, int(awq), 0, dt, 0)
+    else:
+        ops.lib().vra_wna16_gemm(xp, *w, b, r, out.ptr, M, K, N, gs, int(awq), 0, dt, 0)
+    ops.check_error()
+    return out.numpy(np.uint16, (M, N))
+
+
+KERNELS = [None, "D", "d", "M"]
+
+
+@pytest.mark.parametrize("N", [16384, 12288])
 @pytest.mark.parametrize("dt,awq,gs", [(BF16, False, 128), (F16, False, 128), (BF16, True, 128), (BF16, False, -1), (F16, True, 256)])
 def test_wna16_gemm_many_rows(dt, awq, gs, N):
-    M, K = 300, 512                      # the last row tile is ragged (44 rows)
+    M, K = 300, 512                      # the last row tile is ragged on every kernel
     r = rng(11 + dt + awq + gs)
     q = make_quant(r, K, N, gs, dt, awq)
     x, bias, res = rand_dt(r, (M, K), dt), rand_dt(r, (N,), dt), rand_dt(r, (M, N), dt)
-    tiled = ops.marlin_weight_repack(ops.dev(q["qweight"]), q["qweight"].shape, 4, awq)
-    qz = ops.dev(q["qzeros"]) if awq else None
-    out = ops.wna16_gemm(ops.dev(x), tiled, ops.dev(q["scales"]), qz, M, K, N, gs, awq, 0, None, None, dt)
     ref = orc.wna16_gemm(x, q["idx"], q["zeros"] if awq else None, q["scales"], gs, dt)
-    assert_close_dt(out.numpy(np.uint16, (M, N)), ref, dt, name="kernel D", abs_floor=2e-3)
-    out = ops.wna16_gemm(ops.dev(x), tiled, ops.dev(q["scales"]), qz, M, K, N, gs, awq, 0, ops.dev(bias), ops.dev(res), dt)
     ref2 = orc.wna16_gemm(x, q["idx"], q["zeros"] if awq else None, q["scales"], gs, dt, bias, res)
     g0 = orc.from_dt(ref, dt)
     mag = np.maximum(np.abs(g0), np.abs(g0 + orc.from_dt(bias, dt)[None, :]))
-    # 4.9 M outputs and three roundings (GEMM, +bias, +residual), each of which may land on the neighbouring value:
-    # ~5e-5 of the outputs see two flips, ~2e-7 all three (measured: 263 and 1 elements) => bound 3 ulp of the
-    # intermediate magnitude (the 10 k-element test above never sees a double flip)
-    assert_close_dt(out.numpy(np.uint16, (M, N)), ref2, dt, max_ulp=3.0, name="kernel D bias+residual", mag=mag)
+    for kernel in KERNELS:
+        got = wna16_on(kernel, x, q, M, K, N, gs, dt, awq)
+        assert_close_dt(got, ref, dt, name=f"kernel {kernel}", abs_floor=2e-3)
+        got = wna16_on(kernel, x, q, M, K, N, gs, dt, awq, bias, res)
+        # 4.9 M outputs and three roundings (GEMM, +bias, +residual), each of which may land on the neighbouring value:
+        # ~5e-5 of the outputs see two flips, ~2e-7 all three (measured: 263 and 1 elements) => bound 3 ulp of the
+        # intermediate magnitude (the 10 k-element test above never sees a double flip)
+        assert_close_dt(got, ref2, dt, max_ulp=3.0, name=f"kernel {kernel} bias+residual", mag=mag)
 
 
 @pytest.mark.parametrize("awq", [False, True])
 def test_gate_up_silu_many_rows(awq):
-    M, K, N = 260, 512, 8192             # dual: 64 column tiles of 128 x 3 row tiles
+    M, K, N = 260, 512, 8192
     r = rng(23 + awq)
     qg, qu = make_quant(r, K, N, 128, BF16, awq), make_quant(r, K, N, 128, BF16, awq)
     x = rand_dt(r, (M, K), BF16)
-    tg = ops.marlin_weight_repack(ops.dev(qg["qweight"]), qg["qweight"].shape, 4, awq)
-    tu = ops.marlin_weight_repack(ops.dev(qu["qweight"]), qu["qweight"].shape, 4, awq)
-    zg, zu = (ops.dev(qg["qzeros"]), ops.dev(qu["qzeros"])) if awq else (None, None)
-    out = ops.wna16_gate_up_silu(ops.dev(x), tg, ops.dev(qg["scales"]), zg, tu, ops.dev(qu["scales"]), zu, M, K, N, 128, awq)
     g = orc.wna16_gemm(x, qg["idx"], qg["zeros"] if awq else None, qg["scales"], 128, BF16)
     u = orc.wna16_gemm(x, qu["idx"], qu["zeros"] if awq else None, qu["scales"], 128, BF16)
     ref = orc.silu_mul(g, u, BF16)
-    assert_close_dt(out.numpy(np.uint16, (M, N)), ref, BF16, max_ulp=3.0, max_mismatch_frac=0.04, name="kernel D gate_up_silu", abs_floor=4e-3)
+    for kernel in KERNELS:
+        got = wna16_on(kernel, x, qg, M, K, N, 128, BF16, awq, up=qu)
+        assert_close_dt(got, ref, BF16, max_ulp=3.0, max_mismatch_frac=0.04, name=f"kernel {kernel} gate_up_silu", abs_floor=4e-3)
 
 
 @pytest.mark.parametrize("M", [143, 160, 200, 221])
 def test_gate_up_silu_143_to_221_rows_at_the_llama3_8b_widths(M):
-    """the row range where the launcher's cost model changed its choice in round 5 (kernel B's pair form priced at its measured
-    420 TFLOP/s: kernel D with four m-tiles per wave takes these launches now, wna16_gemm.hip `vra_gemm_q4_big_fits`), at the
-    real gate/up shape of BASELINE config 2: K = 4096, N = 14336, ragged last row tile at every M"""
+    """the row range where kernels B, D and M have each been the launcher's choice (wna16_gemm.hip `vra_gemm_q4_big_fits`; kernel M now), at the
+    gate/up shape of Llama-3-8B: K = 4096, N = 14336, ragged last row tile at every M"""
     K, N = 4096, 14336
     r = rng(1000 + M)
     qg, qu = make_quant(r, K, N, 128, BF16), make_quant(r, K, N, 128, BF16)
@@ -185,10 +209,10 @@ def test_gate_up_silu_143_to_221_rows_at_the_llama3_8b_widths(M):
     assert float((got != ref).mean()) <= 0.04
 
 
-# ---------------------------------------------------------------- kernel M (33 rows up: short and middle prompts)
-# Few columns, where kernel W does not take the launch: blocks of 64 / 96 / 128 / 160 rows and two row blocks, whole and ragged; a column tile with
-# missing n-blocks (272 = 17 blocks); K in one piece and in slices, 37 k-tiles in uneven ones whose row sums are read one by one.  The kernel sums
-# (C + q) x in float32 (C 128 or 64, q < 16) and takes (C + z) sum x off at the end: a few float32 roundings of the largest partial sum are the floor.
+# ---------------------------------------------------------------- kernel M (64 rows up: short and middle prompts)
+# Few columns, on kernel M and on the kernel that the shape is dispatched to: blocks of 64 / 96 / 128 / 160 rows and two row blocks, whole and ragged; a column tile with
+# missing n-blocks (272 = 17 blocks); K in one piece and in slices, 37 k-tiles in uneven ones.  The kernel sums (C + q) x in float32 (C 128 or 64,
+# q < 16) and takes (C + z) sum x off per k-tile: a few float32 roundings of the largest partial sum are the floor.
 @pytest.mark.parametrize("M", [64, 65, 97, 150, 161, 200])
 @pytest.mark.parametrize("K,N", [(512, 272), (4608, 512), (4736, 64)])
 @pytest.mark.parametrize("dt,awq,gs", [(BF16, False, 128), (F16, False, 128), (BF16, True, 128), (F16, True, -1), (BF16, False, 256)])
@@ -198,19 +222,18 @@ def test_wna16_gemm_middle_rows(dt, awq, gs, K, N, M):
     r = rng(M * 3 + K + N + dt + awq + gs)
     q = make_quant(r, K, N, gs, dt, awq)
     x, bias, res = rand_dt(r, (M, K), dt), rand_dt(r, (N,), dt), rand_dt(r, (M, N), dt)
-    tiled = ops.marlin_weight_repack(ops.dev(q["qweight"]), q["qweight"].shape, 4, awq)
-    qz = ops.dev(q["qzeros"]) if awq else None
     sums = np.abs(orc.from_dt(x, dt)).sum(1).max() * np.abs(orc.from_dt(q["scales"], dt)).max()
     floor = float(4 * 2.0 ** -24 * (144 if dt == BF16 else 80) * sums)
-    out = ops.wna16_gemm(ops.dev(x), tiled, ops.dev(q["scales"]), qz, M, K, N, gs, awq, 0, None, None, dt)
     ref = orc.wna16_gemm(x, q["idx"], q["zeros"] if awq else None, q["scales"], gs, dt)
-    assert_close_dt(out.numpy(np.uint16, (M, N)), ref, dt, name="kernel M", abs_floor=floor)
-    out = ops.wna16_gemm(ops.dev(x), tiled, ops.dev(q["scales"]), qz, M, K, N, gs, awq, 0, ops.dev(bias), ops.dev(res), dt)
     ref2 = orc.wna16_gemm(x, q["idx"], q["zeros"] if awq else None, q["scales"], gs, dt, bias, res)
     g0 = orc.from_dt(ref, dt)
     mag = np.maximum(np.abs(g0), np.abs(g0 + orc.from_dt(bias, dt)[None, :]))
-    # (three roundings, each of which may land on the neighbouring value)
-    assert_close_dt(out.numpy(np.uint16, (M, N)), ref2, dt, max_ulp=3.0, name="kernel M bias + residual", mag=mag, abs_floor=floor)
+    for kernel in (None, "M"):
+        got = wna16_on(kernel, x, q, M, K, N, gs, dt, awq)
+        assert_close_dt(got, ref, dt, name=f"kernel {kernel}", abs_floor=floor)
+        # (three roundings, each of which may land on the neighbouring value)
+        got = wna16_on(kernel, x, q, M, K, N, gs, dt, awq, bias, res)
+        assert_close_dt(got, ref2, dt, max_ulp=3.0, name=f"kernel {kernel} bias + residual", mag=mag, abs_floor=floor)
     assert ops.lib().vra_take_device_error() == 0
 
 
@@ -261,17 +284,21 @@ def test_wna16_kernel_is_the_faster_one(pair, M, K, N, awq, want):
     assert ops.wna16_kernel(pair, M, K, N, 128, awq) in want
 
 
-@pytest.mark.parametrize("off", [0, 4, 8])
-def test_wna16_gemm_middle_rows_off_16_bytes(off):
-    """x that does not start on 16 bytes, which the DMA of kernel M does not take: the launch goes to kernel D, with the same product"""
+@pytest.mark.parametrize("dt,awq,pair", [(BF16, False, False), (F16, False, True), (BF16, True, False), (F16, True, False), (BF16, True, True)])
+@pytest.mark.parametrize("off", [(2, 0), (4, 0), (0, 1), (0, 2), (1, 1)])
+def test_wna16_gemm_middle_rows_off_16_bytes(dt, awq, pair, off):
+    """x that does not start on 16 bytes or scales off 4, which the DMA of kernel M does not take: the launch goes to kernel D's 64-row tiles,
+    bit for bit, with the product of the same operands on whole boundaries"""
     M, K, N = 97, 512, 272
     r = rng(77)
-    q = make_quant(r, K, N, 128, BF16, False)
-    x = rand_dt(r, (M, K), BF16)
-    tiled = ops.marlin_weight_repack(ops.dev(q["qweight"]), q["qweight"].shape)
-    buf = ops.dev(np.concatenate([np.zeros(off // 2, np.uint16), x.reshape(-1)]))
-    out = ops.wna16_gemm(buf.ptr + off, tiled, ops.dev(q["scales"]), None, M, K, N, 128)
-    assert_close_dt(out.numpy(np.uint16, (M, N)), orc.wna16_gemm(x, q["idx"], None, q["scales"], 128, BF16), BF16, name="kernel M / D", abs_floor=2e-3)
+    q, up = make_quant(r, K, N, 128, dt, awq), make_quant(r, K, N, 128, dt, awq) if pair else None
+    x = rand_dt(r, (M, K), dt)
+    got = wna16_on("M", x, q, M, K, N, 128, dt, awq, up=up, off=off)
+    want = "M" if off == (0, 2) else "D"  # (scales on 4 bytes)
+    assert np.array_equal(got, wna16_on(want, x, q, M, K, N, 128, dt, awq, up=up))
+    if not pair:
+        ref = orc.wna16_gemm(x, q["idx"], q["zeros"] if awq else None, q["scales"], 128, dt)
+        assert_close_dt(got, ref, dt, name="kernel M / D", abs_floor=2e-3)
 
 
 @pytest.mark.parametrize("dt,awq", [(BF16, False), (F16, False), (BF16, True)])
@@ -280,10 +307,6 @@ def test_gate_up_silu_middle_rows(dt, awq, M, K, N):
     r = rng(M * 5 + K + N + dt + awq)
     qg, qu = make_quant(r, K, N, 128, dt, awq), make_quant(r, K, N, 128, dt, awq)
     x = rand_dt(r, (M, K), dt)
-    tg = ops.marlin_weight_repack(ops.dev(qg["qweight"]), qg["qweight"].shape, 4, awq)
-    tu = ops.marlin_weight_repack(ops.dev(qu["qweight"]), qu["qweight"].shape, 4, awq)
-    zg, zu = (ops.dev(qg["qzeros"]), ops.dev(qu["qzeros"])) if awq else (None, None)
-    out = ops.wna16_gate_up_silu(ops.dev(x), tg, ops.dev(qg["scales"]), zg, tu, ops.dev(qu["scales"]), zu, M, K, N, 128, awq, dtype=dt)
     g = orc.wna16_gemm(x, qg["idx"], qg["zeros"] if awq else None, qg["scales"], 128, dt)
     u = orc.wna16_gemm(x, qu["idx"], qu["zeros"] if awq else None, qu["scales"], 128, dt)
     ref = orc.silu_mul(g, u, dt)
@@ -293,8 +316,10 @@ def test_gate_up_silu_middle_rows(dt, awq, M, K, N):
     tol = (ulp_of(gf, dt) * np.abs(sg * (1.0 + gf * (1.0 - sg))) + 0.5 * ulp_of(gf * sg, dt)) * np.abs(uf) + ulp_of(uf, dt) * np.abs(gf * sg) + 1.5 * ulp_of(orc.from_dt(ref, dt), dt)
     sums = np.abs(orc.from_dt(x, dt)).sum(1).max() * max(np.abs(orc.from_dt(z["scales"], dt)).max() for z in (qg, qu))
     floor = 4 * 2.0 ** -24 * (144 if dt == BF16 else 80) * sums * (1.1 * np.abs(uf) + np.abs(gf * sg))
-    diff = np.abs(orc.from_dt(out.numpy(np.uint16, (M, N)), dt).astype(np.float64) - orc.from_dt(ref, dt))
-    assert (diff <= 1.0001 * tol + floor).all(), float((diff / (tol + floor)).max())
+    for kernel in (None, "M"):
+        got = wna16_on(kernel, x, qg, M, K, N, 128, dt, awq, up=qu)
+        diff = np.abs(orc.from_dt(got, dt).astype(np.float64) - orc.from_dt(ref, dt))
+        assert (diff <= 1.0001 * tol + floor).all(), (kernel, float((diff / (tol + floor)).max()))
 
 
 @pytest.mark.parametrize("gs,with_g_idx", [(128, True), (64, True), (64, False), (32, False), (128, False)])
@@ -393,6 +418,52 @@ def test_dense_gemm_prompt_rows(M, K, N, dt, with_bias, out_f32):
         # near zero an ulp is finer than f32 sums of different order agree: K roundings of partial sums (|.| < 4) at 2^-24 each
         # (with a bias two roundings, of the product and of the sum, may each fall the other way: 2 ulp)
         assert_close_dt(out.numpy(np.uint16, (M, N)), ref, dt, max_ulp=2.0 if with_bias else 1.0, name="dense prompt gemm", mag=g0, abs_floor=K * 4 * 2.0 ** -24)
+
+
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("M,K", [(33, 64), (64, 128), (129, 192), (150, 576), (257, 1024)])
+@pytest.mark.parametrize("form", ["plain", "bias f32", "residual", "segments", "pair", "pair bias"])
+def test_dense_gemm_on_every_tile(form, M, K, dt):
+    """gemm_rows.cuh at 64 x 128, 128 x 128 and 128 x 256: ragged last tiles in M and N, K from one step to more than the ring and the touching
+    wave's eight lines, segments that end inside a tile, the gate / up pair: the same bits from every tile, and the reference's product"""
+    r = rng(M + K + dt)
+    pair, ns = form.startswith("pair"), {"segments": [272, 16, 400], "pair": [144] * 2, "pair bias": [144] * 2}.get(form, [528])
+    x, ws = rand_dt(r, (M, K), dt), [rand_dt(r, (n, K), dt, 0.05) for n in ns]
+    bias = [rand_dt(r, (n,), dt, 0.2) if "bias" in form or form == "segments" else None for n in ns]
+    res = rand_dt(r, (M, ns[0]), dt) if form == "residual" else None
+    f32 = form == "bias f32"
+    xd, wd, bd = ops.dev(x), [ops.dev(w) for w in ws], [ops.dev(b) if b is not None else None for b in bias]
+    rd = ops.dev(res) if res is not None else None
+
+    def run(tile):
+        outs = [ops.DevBuf((M + 1) * n * 4).fill_bytes(0) for n in ns]
+        ptrs = [(C.c_void_p * len(ns))(*[b.ptr if b else None for b in bufs]) for bufs in (wd, bd, outs)]
+        ops.lib().vra_dense_gemm_tile(tile, xd.ptr, ptrs[0], ptrs[1], (C.c_int32 * len(ns))(*ns), len(ns), int(pair), rd.ptr if rd else None, ptrs[2],
+                                      int(f32), M, K, dt, 0)
+        ops.check_error()
+        got = [o.numpy(np.float32 if f32 else np.uint16, (M + 1, n)) for o, n in zip(outs, ns)][:1 if pair else None]
+        assert all((g[M] == 0).all() for g in got)
+        return [g[:M] for g in got]
+    one = run(0x12)
+    for tile in (0x22, 0x24):
+        assert all(np.array_equal(a, b) for a, b in zip(run(tile), one)), hex(tile)
+    sums = [orc.dense_gemm(x, w, None, dt, dt) for w in ws]
+    if pair:
+        g, u = (orc.dense_gemm(x, w, b, dt, dt) for w, b in zip(ws, bias))
+        gf, uf, ref = (orc.from_dt(t, dt).astype(np.float64) for t in (g, u, orc.silu_mul(g, u, dt)))
+        # one ulp of gate (two with a bias: sum and bias each rounded) through silu' and half an ulp of the re-rounded silu, the same of up, 1.5 ulp of the product
+        n = 2.0 if bias[0] is not None else 1.0
+        gm, um = (np.maximum(np.abs(orc.from_dt(t, dt).astype(np.float64)), np.abs(f)) for t, f in zip(sums, (gf, uf)))
+        sg = 1.0 / (1.0 + np.exp(-gf))
+        tol = (n * ulp_of(gm, dt) * np.abs(sg * (1.0 + gf * (1.0 - sg))) + 0.5 * ulp_of(gf * sg, dt)) * np.abs(uf) + n * ulp_of(um, dt) * np.abs(gf * sg) + 1.5 * ulp_of(ref, dt)
+        floor = K * 4 * 2.0 ** -24 * (1.1 * np.abs(uf) + np.abs(gf * sg))
+        assert (np.abs(orc.from_dt(one[0], dt) - ref) <= 1.0001 * tol + floor).all()
+        return
+    for got, w, b, s in zip(one, ws, bias, sums):
+        ref = orc.from_dt(orc.dense_gemm(x, w, b, dt, dt), dt).astype(np.float64) + (orc.from_dt(res, dt) if res is not None else 0.0)
+        # each of the roundings (sum, bias or residual added) may fall on the neighbouring value of its own size; K roundings of partial sums (|.| < 4)
+        mag = np.maximum(np.abs(orc.from_dt(s, dt).astype(np.float64)), np.abs(ref))
+        assert (np.abs((got if f32 else orc.from_dt(got, dt)) - ref) <= 2.0 * ulp_of(mag, dt) + K * 4 * 2.0 ** -24).all()
 
 
 @pytest.mark.parametrize("M", [8, 9, 16, 17, 32])

@@ -272,7 +272,7 @@ def test_moe_sort_and_grouped_gemm(dt, granule, P, E, top):
     assert rel(o.numpy(np.float32, (P, W)), want) < 1e-5
 
 
-# the row-major prompt GEMM (csrc/gemm_rows.cuh): edges of its 64 / 128 / 256-wide tiles, remainders in M and N, the shortest and longer K rings,
+# the row-major prompt GEMM (csrc/gemm_rows.cuh) on the tile that these shapes are dispatched to, 64 x 128: remainders in M and N, the shortest and longer K rings,
 # every epilogue; bf16 only.  f32 outputs: sums of K products of bf16 values in f32, K ascending — relative error of a chain of K
 # roundings, far below 2e-6 of the result's norm; bf16 outputs: one rounding more (2^-9 of the value)
 @pytest.mark.parametrize("M,N,K", [(33, 16, 64), (64, 128, 128), (65, 130, 192), (127, 256, 64), (129, 264, 320), (257, 72, 256), (300, 1000, 64)])
@@ -316,6 +316,89 @@ def test_gemm_rows_edges(M, N, K, form):
         assert rel(got, ref) < 2e-6
     else:
         assert (np.abs(got - ref) <= 2.0 ** -8 * np.abs(ref) + 1e-5).all()
+
+
+# (the tile that a shape is dispatched to is the cheapest: at these sizes always 64 x 128)
+@pytest.mark.parametrize("M,N,K", [(33, 16, 64), (65, 130, 128), (127, 256, 192), (129, 264, 576), (257, 520, 1024)])
+@pytest.mark.parametrize("form", ["f32", "bf16", "gated", "scatter"])
+def test_gemm_rows_on_every_tile(M, N, K, form):
+    """64 x 128, 128 x 128 and 128 x 256 outputs a workgroup, ragged in M and N, K from one step to more than the ring and the touching wave's
+    eight lines: the same bits from every tile, the dispatched product among them, and the float64 product"""
+    L = _lib.load()
+    r = np.random.default_rng(M + N + K)
+    N = (N + 31) // 32 * 32 if form == "gated" else N
+    a = so.bf16_round(r.standard_normal((M, K)).astype(np.float32))
+    w = so.bf16_round((r.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32))
+    f32 = form in ("f32", "scatter")
+    ldo = N // 2 if form == "gated" else N
+    dst = np.arange(M - 1, -1, -1, dtype=np.int32)
+    dst[::3] = -1
+    ad, wd, dd = to_dev(a, BF16), to_dev(w, BF16), raw(dst, np.int32) if form == "scatter" else None
+
+    def run(tile):
+        out = empty((M + 1) * ldo * 4).fill_bytes(0)
+        tail = (dd.ptr if dd else None, int(form == "gated"), 1.5)
+        if tile:
+            L.vra_stack_op_gemm_tile(tile, ad.ptr, K, wd.ptr, 0, out.ptr, ldo, int(f32), M, N, K, None, None, 0, *tail, 0)
+        else:
+            L.vra_stack_op_gemm(ad.ptr, K, wd.ptr, 0, out.ptr, ldo, int(f32), M, N, K, 1.0, None, 0, None, None, *tail, BF16, 0)
+        check()
+        return out.numpy(np.float32, (M + 1, ldo)) if f32 else from_dev(out, (M + 1, ldo), BF16)
+    one = run(0)
+    for tile in (0x12, 0x22, 0x24):
+        assert (run(tile) == one).all(), hex(tile)
+    assert (one[M] == 0).all()
+    ref = a.astype(np.float64) @ w.astype(np.float64).T
+    if form == "gated":
+        z = ref.reshape(M, N // 32, 2, 16)
+        g, u = np.minimum(z[:, :, 0], 1.5), np.clip(z[:, :, 1], -1.5, 1.5)
+        ref = (g * so.sigmoid(1.702 * g) * (u + 1)).reshape(M, N // 2)
+    if form == "scatter":
+        assert (one[:M][np.setdiff1d(np.arange(M), dst)] == 0).all()
+        one, ref = one[dst[dst >= 0]], ref[dst >= 0]
+    assert rel(one[:M], ref) < (2e-6 if f32 else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("N,K,out", [(130, 64, "f32"), (264, 576, "f32"), (288, 192, "gated")])
+def test_gemm_rows_grouped_on_every_tile(N, K, out):
+    """rows of x gathered by a row list with holes, a group a tile row and an empty tile row: the same bits from every tile, and the float64 product"""
+    L = _lib.load()
+    r = np.random.default_rng(N + K)
+    T, E, rows = 70, 3, 4 * 128
+    a = so.bf16_round(r.standard_normal((T, K)).astype(np.float32))
+    w = so.bf16_round((r.standard_normal((E, N, K)) / np.sqrt(K)).astype(np.float32))
+    idx = r.integers(0, T, rows).astype(np.int32)
+    idx[r.random(rows) < 0.3] = -1
+    group = np.array([2, -1, 0, 1], np.int32)
+    gated = out == "gated"
+    ldo = N // 2 if gated else N
+    ad, wd, xd = to_dev(a, BF16), to_dev(w, BF16), raw(idx, np.int32)
+
+    def run(tile):
+        g = raw(np.repeat(group, 128 // ((tile >> 4) * 64)), np.int32)
+        o = empty(rows * ldo * 4).fill_bytes(0)
+        L.vra_stack_op_gemm_tile(tile, ad.ptr, K, wd.ptr, N * K, o.ptr, ldo, int(not gated), rows, N, K, g.ptr, xd.ptr, T, None, int(gated), 1.5, 0)
+        check()
+        return from_dev(o, (rows, ldo), BF16) if gated else o.numpy(np.float32, (rows, ldo))
+    one = run(0x12)
+    assert (run(0x22) == one).all() and (run(0x24) == one).all()
+    live = (idx >= 0) & (np.repeat(group, 128) >= 0)
+    assert (one[~live] == 0).all()
+    ref = np.stack([w[g].astype(np.float64) @ a[i].astype(np.float64) for g, i in zip(np.repeat(group, 128)[live], idx[live])])
+    if gated:
+        z = ref.reshape(len(ref), N // 32, 2, 16)
+        g, u = np.minimum(z[:, :, 0], 1.5), np.clip(z[:, :, 1], -1.5, 1.5)
+        ref = (g * so.sigmoid(1.702 * g) * (u + 1)).reshape(len(ref), N // 2)
+    assert rel(one[live], ref) < (2.0 ** -8 if gated else 2e-6)
+
+
+def test_gemm_rows_named_tile_is_refused_where_it_does_not_fit():
+    L = _lib.load()
+    a, w, out = (to_dev(np.zeros((64, 64), np.float32), BF16) for _ in range(3))
+    for tile, M, K in ((0, 64, 64), (0x11, 64, 64), (0x44, 64, 64), (0x22, 32, 64), (0x22, 64, 40)):
+        L.vra_stack_op_gemm_tile(tile, a.ptr, K, w.ptr, 0, out.ptr, 16, 0, M, 16, K, None, None, 0, None, 0, 0.0, 0)
+        with pytest.raises(RuntimeError):
+            check()
 
 
 @pytest.mark.parametrize("design", ["ditilix", "pesivik"])
@@ -515,6 +598,48 @@ def test_prompt_attention_tiles(H, G, dim, vdim, form, first, Tq, BS):
     got, general = run(BS), run(32)
     assert rel(got, ref) < 3e-3 and rel(general, ref) < 3e-3
     assert np.abs(got - general).max() <= 2.0 ** -7 * np.abs(ref).max()  # (one rounding apart where their f32 sums fall on either side)
+
+
+@pytest.mark.parametrize("copies", [1, 12])
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (64, 64)])
+def test_prompt_attention_of_several_sequences(dim, vdim, copies):
+    """sequences of unequal length behind unequal prefixes in one launch, below and beyond 512 workgroups (the two orders of the row blocks): the same bits
+    as each alone, and float64"""
+    L = _lib.load()
+    r = np.random.default_rng(dim + copies)
+    H, G, BS, shapes = 16, 4, 64, [(0, 70), (130, 1), (63, 200)] * copies  # (tokens in the cache, tokens of the step)
+    mx = dict(scale=dim ** -0.5, softcap=5.0)
+    ks, vs, qs = [], [], []
+    blocks = [(p + n + BS - 1) // BS for p, n in shapes]
+    assert (4 * H * len(shapes) > 512) == (copies > 1)  # (four blocks of 64 rows, the longest's, a sequence)
+    order, at = r.permutation(sum(blocks)).astype(np.uint32), 0
+    kc, vc = np.full((sum(blocks) * BS, G * dim), 1e4, np.float32), np.full((sum(blocks) * BS, G * vdim), -1e4, np.float32)
+    tables = np.zeros((len(shapes), max(blocks)), np.uint32)
+    for i, (p, n) in enumerate(shapes):
+        tables[i, :blocks[i]] = order[at:at + blocks[i]]
+        at += blocks[i]
+        ks.append(so.bf16_round(r.standard_normal((p + n, G, dim)).astype(np.float32)))
+        vs.append(so.bf16_round(r.standard_normal((p + n, G, vdim)).astype(np.float32)))
+        qs.append(so.bf16_round((2.0 * r.standard_normal((n, H, dim))).astype(np.float32)))
+        slots = tables[i, np.arange(p + n) // BS].astype(np.int64) * BS + np.arange(p + n) % BS
+        kc[slots], vc[slots] = ks[i].reshape(p + n, -1), vs[i].reshape(p + n, -1)
+    kd, vd = to_dev(kc, BF16), to_dev(vc, BF16)
+
+    def run(which):
+        q = np.concatenate([qs[i].reshape(-1, H * dim) for i in which])
+        pos = np.concatenate([np.arange(shapes[i][0], sum(shapes[i])) for i in which])
+        lens, n = [sum(shapes[i]) for i in which], [shapes[i][1] for i in which]
+        out = empty(len(q) * H * vdim * 2)
+        L.vra_stack_op_attention(to_dev(q, BF16).ptr, H * dim, out.ptr, kd.ptr, vd.ptr, raw(pos, np.int64).ptr, raw(tables[which], np.uint32).ptr, raw(lens, np.uint32).ptr,
+                                 raw(np.concatenate([[0], np.cumsum(n)]), np.uint32).ptr, len(which), len(q), max(n), H, G, dim, vdim, BS, tables.shape[1],
+                                 mx["scale"], mx["softcap"], 0.0, 0, BF16, 0)
+        check()
+        return np.split(from_dev(out, (len(q), H, vdim), BF16), np.cumsum(n)[:-1])
+    for i, got in enumerate(run(list(range(len(shapes))))):
+        assert (got == run([i])[0]).all()
+        if i < 3:
+            ref = so.attention_core(*(t[i].astype(np.float64) for t in (qs, ks, vs)), mx, np.arange(shapes[i][0], sum(shapes[i])))
+            assert rel(got, ref) < 4e-3
 
 
 @pytest.mark.parametrize("dt", [F32, BF16])

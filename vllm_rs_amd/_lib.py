@@ -94,6 +94,7 @@ def load():
     _sig(lib, "vra_version", C.c_char_p)
     _sig(lib, "vra_wna16_gemm", None, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_wna16_gate_up_silu", None, P, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
+    _sig(lib, "vra_wna16_gemm_on", None, c_i32, P, P, P, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_wna16_kernel", c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32)
     _sig(lib, "vra_rms_norm_wna16_gemm", None, P, P, c_f32, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_rms_norm_wna16_gate_up_silu", None, P, P, c_f32, P, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
@@ -124,6 +125,7 @@ def load():
          c_i32, c_i32, c_i32, c_f32, P, c_i32, c_i32, c_i64)
     _sig(lib, "vra_causal_mask", None, P, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_swap_blocks", None, P, P, P, c_i32, c_i64, c_i32, c_i64)
+    _sig(lib, "vra_dense_gemm_tile", None, c_i32, P, P, P, P, c_i32, c_i32, P, P, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_dense_gemm", None, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_argmax_f32", None, P, P, c_i32, c_i32, c_i64)
     _sig(lib, "vra_dense_gemm_argmax_workspace_bytes", c_i64)
@@ -221,6 +223,7 @@ def load():
          c_f32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_linear_scan", None, P, c_i32, P, c_i32, P, c_i32, P, c_i32, P, P, c_i32, c_f32, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32,
          c_i32, c_i32, c_i64)
+    _sig(lib, "vra_stack_op_gemm_tile", None, c_i32, P, c_i32, P, c_i64, P, c_i32, c_i32, c_i32, c_i32, c_i32, P, P, c_i32, P, c_i32, c_f32, c_i64)
     _sig(lib, "vra_stack_op_gemm_few_columns", c_i32, c_i32, c_i32, c_i32, c_i32, c_i32)
     _sig(lib, "vra_stack_op_expert_rows", c_i32, c_i32, c_i32, c_i32)
     _sig(lib, "vra_stack_op_linear_scan_lds", c_i32, c_i32, c_i32, c_i32, c_i32, c_i32)

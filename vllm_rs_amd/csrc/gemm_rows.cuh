@@ -255,6 +255,7 @@ static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch,
   if (us) *us = cost;
   return best;
 }
+static inline bool gemm_rows_has_tile(int tile) { return tile == 2 * 16 + 4 || tile == 2 * 16 + 2 || tile == 16 + 2; }
 // fills the tile counts and launches
 template <class DT, int WM, int WN, int S, bool SPREAD, bool PAIR, class EPI>
 static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStream_t st) {

@@ -81,15 +81,20 @@ struct DenseRowsEpi {
 
 }  // namespace
 
-// x rows and every tensor within 31-bit byte offsets, whole 64-steps of K, 16-byte pieces in all rows; then time against time: a round of
-// workgroups here (gemm_rows_tile), kernel B at 250 TFLOP/s on whole 64-row blocks behind ~10 us of exchange between its K slices
-bool vra_gemm_rows_fits(const GemmRowsCall& c) {
+// x rows and every tensor within 31-bit byte offsets, whole 64-steps of K, 16-byte pieces in all rows
+bool vra_gemm_rows_takes(const GemmRowsCall& c) {
   if (c.M <= 32 || c.K % 64 || (int64_t)c.M * c.x_ld * 2 >= 0x7FFF0000ll || c.x_ld % 8 || (uintptr_t)c.x % 16) return false;
   for (int s = 0; s < c.nseg; s++)
     if ((int64_t)c.n[s] * c.K * 2 >= 0x7FFF0000ll || c.n[s] % 16 || (uintptr_t)c.w[s] % 16 || (uintptr_t)c.bias[s] % 8) return false;
   for (int s = 0; s < (c.dual ? 1 : c.nseg); s++)
     if ((uintptr_t)c.out[s] % 16 || c.out_ld[s] % 8) return false;
   if (c.residual && ((uintptr_t)c.residual % 16 || c.res_ld % 8 || c.out_f32)) return false;
+  return true;
+}
+// then time against time: a round of workgroups here (gemm_rows_tile), kernel B at 250 TFLOP/s on whole 64-row blocks behind ~10 us of exchange
+// between its K slices
+bool vra_gemm_rows_fits(const GemmRowsCall& c) {
+  if (!vra_gemm_rows_takes(c)) return false;
   int n[GR_MAX_SEG] = {};
   double b_us = 0.0;
   for (int s = 0; s < c.nseg; s++) n[s] = c.n[s], b_us += 10.0 + 2.0 * ((c.M + 63) / 64 * 64) * (double)c.n[s] * c.K / 250e6;
@@ -105,7 +110,7 @@ void vra_launch_gemm_rows(const GemmRowsCall& c, int dtype, int64_t stream) {
   a.nseg = c.dual ? 1 : c.nseg;
   for (int s = 0; s < c.nseg; s++) a.w[s] = c.w[s], a.n[s] = c.n[s];
   if (c.dual) a.n[0] = 2 * c.n[0];
-  const int tile = gemm_rows_tile(c.M, a.n, a.nseg, 1);
+  const int tile = c.tile ? c.tile : gemm_rows_tile(c.M, a.n, a.nseg, 1);
   auto go = [&](auto dt, auto dual) {
     DenseRowsEpi<decltype(dt), decltype(dual)::value> e = {};
     for (int s = 0; s < a.nseg; s++) e.o[s] = GemmRowsOut{c.out[s], c.bias[s], c.out_ld[s]};
@@ -115,4 +120,19 @@ void vra_launch_gemm_rows(const GemmRowsCall& c, int dtype, int64_t stream) {
   };
   if (dtype == VRA_BF16) c.dual ? go(BF16{}, std::true_type{}) : go(BF16{}, std::false_type{});
   else c.dual ? go(F16{}, std::true_type{}) : go(F16{}, std::false_type{});
+}
+
+extern "C" void vra_dense_gemm_tile(int32_t tile, const void* x, const void* const* w, const void* const* bias, const int32_t* n, int32_t nseg,
+                                    int32_t pair, const void* residual, void* const* out, int32_t out_f32, int32_t m, int32_t k, int32_t dtype,
+                                    int64_t stream) {
+  VRA_CHECK_ARG(x && w && bias && n && out && m > 0 && k > 0 && (pair ? nseg == 2 && n[0] == n[1] : nseg >= 1 && nseg <= GR_MAX_SEG), "dense gemm tile: null pointer or bad segments");
+  VRA_CHECK_ARG((dtype == VRA_BF16 || dtype == VRA_F16) && gemm_rows_has_tile(tile) && !(pair && residual), "dense gemm tile: no such form");
+  GemmRowsCall r;
+  r.x = x, r.x_ld = k, r.M = m, r.K = k, r.nseg = nseg, r.dual = pair != 0, r.tile = tile, r.out_f32 = out_f32, r.residual = residual, r.res_ld = n[0];
+  for (int s = 0; s < nseg; s++) {
+    VRA_CHECK_ARG(w[s] && n[s] > 0 && (out[s] || (pair && s)), "dense gemm tile: null pointer or bad segments");
+    r.w[s] = w[s], r.n[s] = n[s], r.bias[s] = bias[s], r.out[s] = out[s], r.out_ld[s] = n[s];
+  }
+  VRA_CHECK_ARG(vra_gemm_rows_takes(r), "dense gemm tile: a shape or an alignment that these tiles do not take");
+  vra_launch_gemm_rows(r, dtype, stream);
 }

@@ -22,9 +22,11 @@ struct GemmRowsCall {
   int res_ld = 0;
   int out_f32 = 0;
   bool dual = false;
+  int tile = 0;  // WM * 16 + WN instead of gemm_rows_tile's choice
 };
 // whether the product can run here and is expected to be faster than on kernel B (and behind it the element-wise launches the fused form
 // saves).  Measured, bf16, cold weights, us (here / kernel B): 64 rows, 2048 x 5632: 50 / 22; 128 rows, 5632 x 2048: 24 / 34; 256 rows, 4096 x 4096:
 // 40 / 39; 400 rows, 14336 x 4096: 80 / 234; 2120 rows, 2048 x 5632: 95 / 219
 bool vra_gemm_rows_fits(const GemmRowsCall& c);
+bool vra_gemm_rows_takes(const GemmRowsCall& c);  // whether it can
 void vra_launch_gemm_rows(const GemmRowsCall& c, int dtype, int64_t stream);

@@ -1418,12 +1418,14 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
   VRA_CHECK_ARG(!post || !g.a_scale, "stack gemm: scaled rows and an element-wise epilogue do not come together");
   VRA_CHECK_ARG(g.epi != 1 || (mfma && g.N % 32 == 0), "stack gemm: the gated epilogue needs the bf16 MFMA path and whole gate / up blocks");
   if (mfma) {
-    if (big && !g.a_scale && rows_kernel_takes(g)) {
+    const bool rows = big && !g.a_scale && rows_kernel_takes(g);
+    VRA_CHECK_ARG(!g.tile || (rows && gemm_rows_has_tile(g.tile) && (!g.tile_group || g.granule == (g.tile >> 4) * 64)), "stack gemm: no such tile for this product");
+    if (rows) {
       GemmRowsArgs r;
       r.x = g.a, r.x_ld = g.lda, r.x_row = g.a_row, r.w[0] = g.w, r.n[0] = g.N, r.M = g.M, r.K = g.K;
       r.tile_group = g.tile_group, r.w_group_stride = g.w_group_stride, r.x_batch_stride = g.a_batch_stride, r.w_batch_stride = g.w_batch_stride;
-      int tile = gemm_rows_tile(g.M, r.n, 1, nb);
-      if (g.tile_group) tile = g.granule == 64 ? 16 + 2 : (tile == 16 + 2 ? 32 + 2 : tile);  // (a tile row is one granule)
+      int tile = g.tile ? g.tile : gemm_rows_tile(g.M, r.n, 1, nb);
+      if (g.tile_group && !g.tile) tile = g.granule == 64 ? 16 + 2 : (tile == 16 + 2 ? 32 + 2 : tile);  // (a tile row is one granule)
       auto go = [&](auto fn) {
         const int per = g.out_f32 ? 4 : 8;  // elements of 16 bytes
         const bool vec = (uintptr_t)g.out % 16 == 0 && g.ldo % per == 0 && g.out_batch_stride % per == 0 && (g.out_f32 || (g.epi == 1 ? g.N % 32 : g.N % 8) == 0);
@@ -1462,6 +1464,7 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
     }
     return;
   }
+  VRA_CHECK_ARG(!g.tile, "stack gemm: no such tile for this product");
   VRA_CHECK_ARG(!g.tile_group || g.granule != 128, "stack gemm: granules of 128 rows are for bf16 products on the matrix cores");
   if (big) {
     dim3 grid((g.M + 63) / 64, (g.N + 63) / 64, nb);
@@ -1665,6 +1668,15 @@ extern "C" void vra_stack_op_gemm(const void* a, int32_t lda, const void* w, int
   g.a = a, g.lda = lda, g.w = w, g.w_group_stride = w_group_stride, g.out = out, g.ldo = ldo, g.out_f32 = out_f32, g.M = M, g.N = N, g.K = K;
   g.alpha = alpha, g.tile_group = tile_group, g.granule = granule, g.a_row = a_row, g.a_scale = a_scale, g.out_row = out_row, g.epi = epi, g.limit = limit;
   vra_stack_gemm(g, dtype, stream);
+}
+extern "C" void vra_stack_op_gemm_tile(int32_t tile, const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32,
+                                       int32_t M, int32_t N, int32_t K, const int32_t* tile_group, const int32_t* a_row, int32_t a_rows,
+                                       const int32_t* out_row, int32_t epi, float limit, int64_t stream) {
+  VRA_CHECK_ARG(tile != 0, "stack gemm: no such tile for this product");
+  StkGemmArgs g;
+  g.a = a, g.lda = lda, g.w = w, g.w_group_stride = w_group_stride, g.out = out, g.ldo = ldo, g.out_f32 = out_f32, g.M = M, g.N = N, g.K = K;
+  g.tile_group = tile_group, g.granule = (tile >> 4) * 64, g.a_row = a_row, g.a_rows = a_rows, g.out_row = out_row, g.epi = epi, g.limit = limit, g.tile = tile;
+  vra_stack_gemm(g, VRA_BF16, stream);
 }
 extern "C" void vra_stack_op_moe_sort(const int32_t* pair_expert, const float* pair_weight, int32_t P, int32_t top, int32_t n_groups, int32_t granule,
                                       int32_t max_rows, int32_t* row_token, float* row_scale, int32_t* row_pair, int32_t* tile_group, int64_t stream) {

@@ -1064,6 +1064,22 @@ extern "C" int32_t vra_wna16_kernel(int32_t pair, int32_t m, int32_t k, int32_t 
   return general_kernel(ns, m, k, n, group_size, is_awq != 0, &plan);
 }
 
+extern "C" void vra_wna16_gemm_on(int32_t kernel, const void* in, const void* w0, const void* sc0, const void* qz0, const void* w1, const void* sc1,
+                                  const void* qz1, const void* bias, const void* residual, void* out, int32_t m, int32_t k, int32_t n, int32_t group_size,
+                                  int32_t is_awq, int32_t dtype, int64_t stream) {
+  const bool dual = w1 != nullptr, awq = is_awq != 0 && qz0 != nullptr;
+  VRA_CHECK_ARG(in && w0 && sc0 && out && (!dual || (sc1 && (!awq || qz1) && !bias && !residual)), "vra_wna16_gemm_on: null pointer, or a pair with bias or residual");
+  VRA_CHECK_ARG((dtype == VRA_BF16 || dtype == VRA_F16) && (kernel == 'D' || kernel == 'd' || kernel == 'M'), "vra_wna16_gemm_on: dtype or kernel");
+  if (!check_gemm_shape("vra_wna16_gemm_on", m, k, n, group_size)) return;
+  double us = 0.0;
+  const int plan = m >= 64 ? vra_gemm_q4_mid_plan(dual, m, n, k, group_size, nullptr, awq, false, &us) : 0;  // (kernel D takes the same shapes)
+  VRA_CHECK_ARG(plan != 0, "vra_wna16_gemm_on: a shape that these kernels do not take");
+  GemmDArgs d = {};
+  d.w0 = w0, d.w1 = w1, d.sc0 = sc0, d.sc1 = sc1, d.qz0 = (const uint32_t*)qz0, d.qz1 = (const uint32_t*)qz1, d.bias0 = bias;
+  d.x = in, d.x_ld = k, d.residual = residual, d.res_ld = n, d.out = out, d.out_ld = n, d.M = m, d.N = n, d.K = k, d.group_size = group_size;
+  vra_launch_gemm_q4_big(d, dual, awq, kernel == 'M' ? plan | kMidPlan : (kernel == 'D' ? 4 : 2), dtype, stream);
+}
+
 // decode batches of 1..4 rows on kernel E straight from the caller's tensors: row-major scales / zeros as in the
 // checkpoint, or the Marlin-permuted scales the reference passes (grouped form: a per-lane index inside 64 columns, no copy)
 static bool gemv_s_direct(int ns, const void* in, const void* w0, const void* sc0, const void* qz0, const void* w1, const void* sc1, const void* qz1,
