@@ -14,11 +14,11 @@ void vra_launch_skinny(GemmBArgs a, bool int4, bool dual, int dtype, int64_t str
 bool vra_gemm_q4_fits(int nbw, int M, int K, int group_size);
 void vra_launch_gemm_q4(GemmCArgs a, bool awq, int dtype, int64_t stream);
 // kernel D (gemm_q4_big.cuh): int4, many rows (prefill), scale groups >= 128.  `cols` = output columns over all segments
-// (DUAL: of one tensor); summed: a norm's launch leaves the row sums in vra_gemm_q4_big_xsum_table.  Returns the plan to launch with (m-tiles per wave | K slices << 8 of kernel D, or kernel M's), or 0 when the shape
-// belongs to kernel B.
+// (DUAL: of one tensor); summed: a norm's launch leaves the row sums in vra_gemm_q4_big_xsum_table.  Returns the plan to launch with (m-tiles per
+// wave | K slices << 8 of kernel D, or kernel M's), or 0 when the shape belongs to kernel B.
 int vra_gemm_q4_big_fits(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, bool summed);
 void vra_launch_gemm_q4_big(const GemmDArgs& a, bool dual, bool awq, int mb, int dtype, int64_t stream);
-// kernel M (gemm_q4_mid.cuh): int4, 33 rows up, scale groups >= 128: the launch's plan (m-tiles a wave | K slices << 8) and its estimated time,
+// kernel M (gemm_q4_mid.cuh): int4, 64 rows up, scale groups >= 128: the launch's plan (m-tiles a wave | K slices << 8) and its estimated time,
 // or 0 where the shape is not its own.  GemmDArgs::xsum has to be set.
 int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, bool summed, double* us);
 void vra_launch_gemm_q4_mid(GemmDArgs a, bool dual, bool awq, int plan, int dtype, int64_t stream);

@@ -1,4 +1,4 @@
-// gemm_q4_mid.cuh — "kernel M": int4 GEMM for 33 rows up (short and middle prompts), every row of a block of up to 160 in one workgroup.
+// gemm_q4_mid.cuh — "kernel M": int4 GEMM for 64 rows up (short and middle prompts), every row of a block of up to 160 in one workgroup.
 //
 // What bounds a short prompt's int4 product is not memory (the codes of a gate/up pair of 4096 x 14336 take 13 us) but converting the codes: a
 // matrix instruction and a conversion take their SUM on a SIMD, also from different waves (tools/mfma_valu_probe.hip), and the kernels of 32- or
@@ -8,8 +8,8 @@
 // ring of three stages (one barrier a k-tile); the 16-byte chunks of an x row lie at slot chunk ^ (row mod 16), so the fragment reads meet no bank
 // twice.  Two n-blocks a wave read each x fragment from LDS four times a workgroup: 160 KB a k-tile at MB = 5, 1280 cycles (and 880 for the DMA's
 // writes) beside 1380 of MFMAs and 500 of conversions on each SIMD; four n-blocks a wave would halve the reads and double the conversions.
-// us a launch, kernel D or W / here: gate/up of 4096 x 14336 behind its norm, 150 rows 91 / 56, 96 rows 50 / 42; down of 14336 x 4096 with its row sums, 200
-// rows 56 / 49.  AWQ: gate/up of 3584 x 18944, 320 rows 190 / 156.
+// us a launch, kernel D or W / here: gate/up of 4096 x 14336 behind its norm, 150 rows 91 / 56 (f16 in a model's step 55), 96 rows 50 / 42; down of
+// 14336 x 4096 with its row sums, 200 rows 56 / 49.  AWQ: gate/up of 3584 x 18944, 320 rows 190 / 156.
 //
 // The zero points come off per k-tile, acc += s (acc_g - (C + z) Sx): acc never holds more than the result's own size.  (Taken off once behind the
 // k loop, x of mean 0.5 left the float32 sums of K = 14336 ten times as far from the 64-bit result.)  Symmetric codes have one z: a row's group sums

@@ -21,7 +21,7 @@ static int mid_cus() {
 }
 
 int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, bool summed, double* us) {
-  if (M < 33 || K % 128 || cols % 16) return 0;
+  if (M < 64 || K % 128 || cols % 16) return 0;
   if (group_size > 0 && group_size < K && (group_size < 128 || (group_size & (group_size - 1)))) return 0;
   if (segs && segs->nseg > 1) {  // a wave's columns must not straddle tensors
     if (dual || segs->residual || segs->N % 64) return 0;

@@ -1,10 +1,11 @@
 // gemm_rows.cuh — 16-bit GEMM of prompt steps on ROW-MAJOR weights: out[m, n] = epilogue( sum_k x[row(m), k] * w[n, k] ), f32 accumulation.
 //
-// Bound: what a CU can pull out of L2.  LDS-DMA alone (no LDS reads, no MFMAs) delivers ~28 B per clock and CU on full 128-byte lines and
-// ~21 on half lines, whatever the depth of the ring, the row stride or the number of CUs at work; a 128 x 128 tile needs 32 KiB per
-// 512 clocks of MFMAs.  So: whole lines per request (a DMA instruction fetches 8 rows x 128 bytes), the largest tiles the problem has
-// enough of, and the DMA instructions spread between the MFMAs — issued in one run they stall the wave in front of its LDS reads.
-// Measured (2048 x 2048 outputs, K = 8192, 256 tiles of 128 x 128): 87 us with the requests in one run, 74 spread, 62 for the DMA alone.
+// Bound: what a CU can pull past L2, and how well that overlaps with the matrix work.  LDS-DMA alone (no LDS reads, no MFMAs) delivers ~28 B
+// per clock and CU on full 128-byte lines and ~21 on half lines where the panels come from past L2, whatever the depth of the ring or the row
+// stride (panels that stay in L2: 58..60, on either); a 128 x 128 tile needs 32 KiB per 512 clocks of MFMAs.  So: whole lines per request
+// (a DMA instruction fetches 8 rows x 128 bytes), the largest tiles the problem has enough of, and the DMA instructions spread between the MFMAs —
+// issued in one run they stall the wave in front of its LDS reads.  Measured (2048 x 2048 outputs, K = 8192, 256 tiles of 128 x 128): 87 us
+// with the requests in one run, 74 spread; without the MFMAs 67, and 47 with the weights in L2: requests and MFMAs do not overlap as well as they could.
 //
 // Tile: WM x WN waves, 64 x 64 outputs each (16 accumulator tiles of v_mfma_f32_16x16x32: weights = A, rows of x = B, so a lane holds 4
 // consecutive columns of one row).  K in steps of 64, ascending, one accumulation chain per output: the result of a row does not depend

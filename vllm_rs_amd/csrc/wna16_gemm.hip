@@ -494,8 +494,9 @@ bool vra_gemv_w_fits(int ns, int M, int K, int group_size, int n_units, bool has
     if (g < K && (g < 128 || (g & (g - 1)))) return false;
     int kz, ktz, groups;
     const int rb = (M + 31) / 32;
-    // which row counts: a row of such a launch is the same row of a 32-row launch, bit for bit, so where the launch is near the others it stays
-    // (Llama-3-8B down projection, us, here / kernel M: 64 rows 25.5 / 25.6, 96 rows 35 / 31, 150 rows 50 / 42; 128 rows 40 / 36, 200 rows 66 / 48)
+    // which row counts: up to 63 rows no other kernel but B takes the launch; 64..96 and 129..160 rows stayed here when kernel M came, with the bits of a
+    // 32-row launch, though kernel M is quicker at most of them (down of Llama-3-8B with its residual, us, here / kernel M: 64 rows 27.9 /
+    // 25.6, 96 rows 38.4 / 32.0, 150 rows 55.0 / 45.1); at 97..128 rows and beyond 160 this form was the slower one before, too
     static const char* any_rb = getenv("VRA_GEMV_W_KZ_ANY_RB");  // tuning aid: 1 = every row-block count up to the row limit
     if (rb > 3 && rb != 5 && !(any_rb && any_rb[0] == '1')) return false;
     if (!gemv_w_kz_plan(K, n_units, rb, &kz, &ktz, &groups)) return false;
@@ -1072,7 +1073,7 @@ extern "C" void vra_wna16_gemm_on(int32_t kernel, const void* in, const void* w0
   VRA_CHECK_ARG((dtype == VRA_BF16 || dtype == VRA_F16) && (kernel == 'D' || kernel == 'd' || kernel == 'M'), "vra_wna16_gemm_on: dtype or kernel");
   if (!check_gemm_shape("vra_wna16_gemm_on", m, k, n, group_size)) return;
   double us = 0.0;
-  const int plan = m >= 64 ? vra_gemm_q4_mid_plan(dual, m, n, k, group_size, nullptr, awq, false, &us) : 0;  // (kernel D takes the same shapes)
+  const int plan = vra_gemm_q4_mid_plan(dual, m, n, k, group_size, nullptr, awq, false, &us);  // (kernel D takes the same shapes)
   VRA_CHECK_ARG(plan != 0, "vra_wna16_gemm_on: a shape that these kernels do not take");
   GemmDArgs d = {};
   d.w0 = w0, d.w1 = w1, d.sc0 = sc0, d.sc1 = sc1, d.qz0 = (const uint32_t*)qz0, d.qz1 = (const uint32_t*)qz1, d.bias0 = bias;
