@@ -608,7 +608,7 @@ def test_linear_recurrence_tiles(D, V, pad, T):
 
 @pytest.mark.parametrize("T", [1, 7, 16, 33, 64])
 @pytest.mark.parametrize("form", ["delta", "decays", "per head", "bonus"])
-@pytest.mark.parametrize("D,V", [(64, 64), (128, 128), (128, 72), (256, 256)])
+@pytest.mark.parametrize("D,V", [(64, 64), (128, 128), (128, 72), (256, 256), (24, 64), (32, 130)])
 def test_linear_recurrence_does_not_depend_on_the_other_sequences(D, V, form, T):
     """one sequence alone (4 rows of the state a lane), 33 copies of it at once (8 rows a lane) and its first token as a decode step (one token
     staged): the same bits, and the float64 recurrence to 1e-5 (float32 sums of D terms along chains that contract)"""

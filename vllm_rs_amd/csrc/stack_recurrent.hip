@@ -716,13 +716,17 @@ __global__ __launch_bounds__(256) void stk_sigmoid_pow_kernel(const float* z, in
 // ------------------------------------------------------------------------------------------------ the linear recurrence
 // A workgroup owns 256 / P columns of one head's state (a column = one value channel); a column's `dim` rows are spread over P
 // neighbouring lanes, R rows each, in registers for the whole step.  q, k, decays of TT tokens are staged in LDS for all columns, the next tile's
-// requested ahead of a tile's tokens; a whole tile's outputs are stored together.
-// What bounds it is the serial chain over the tokens: a token's S^T k has to be summed over the lanes before its row enters S.  S^T q is taken of the
-// state before the token's row enters, (S + k u^T)^T q = S^T q + (k . q) u, so that both sums run side by side.
+// requested ahead of a tile's tokens.
+// What bounds the delta rule is the serial chain over the tokens: a token's S^T k has to be summed over the lanes before its row enters S.  S^T q is
+// taken of the state before the token's row enters, (S + k u^T)^T q = S^T q + (k . q) u, so that both sums run side by side.  Without the delta rule
+// a row enters at once and the output is summed of the new state, off the chain.
 //  - Few columns (less than two workgroups a CU at R = 8): R = 4 gives twice the workgroups, and tiles of 32 tokens cover the way to memory.  2048
 //    tokens, 16 heads of 128 x 128, delta rule: 306 us (470 with R = 8 and tiles of 16 tokens, the sums one after the other).
 //  - More: the SIMDs are full, and R = 8 takes half the instructions for the sums of an element; tiles of 16 tokens leave room for four workgroups
-//    a CU.  8 sequences of 256 tokens: 132 us (R = 4: 158).
+//    a CU (five with constant decays).  8 sequences of 256 tokens: 139 us (R = 4: 158).  Here registers and code count: outputs are stored at
+//    once and every request is bounded, which the R = 4 form trades for a whole tile's outputs together and a tile's requests without bounds (64
+//    sequences, us, so / as at R = 4: constant decays, 16 tokens 80 / 102; delta rule, 5 tokens 72 / 78; 100 tokens 402 / 394).  Keys of up to 32
+//    channels: where the values fill a workgroup's columns (64 sequences of 100 tokens, 16 heads of 24 x 64: 45 us, R = 4 60).
 //  - Steps of at most 16 tokens a sequence, where the host knows it: R = 4, tiles of 16 (8 sequences of 4 tokens: 9.8 us; R = 8 12.9).
 //  - One token a sequence: nothing to stage ahead (TT = 1: a fraction of the LDS and registers, 8 sequences 7.3 us, 32 21; with tiles 11, 37).
 // Sums over the rows add four rows' products in order, then pairs of neighbours, pairs of pairs and so on up to `dim`, in a lane or across lanes: one
@@ -749,6 +753,7 @@ template <int R, int P, int TT, int DECAY, bool BETA, bool ACT, bool BONUS = fal
 __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   constexpr int dimP = P * R, CPB = 256 / P, d4n = dimP / 4, NL = (TT * d4n + 255) / 256;  // 16-byte loads a thread and array for a tile
+  constexpr bool TILED = R == 4;
   constexpr int AHEAD = R == 4 ? 2 : 1, SETS = 2 * AHEAD, NH = R / 4;  // tokens whose operands are fetched ahead; parts of a lane's sums
   static_assert(d4n <= 64 && R % 4 == 0, "a token's row is staged by lanes of one wave");
   const int dim = a.dim, vdim = a.vdim;
@@ -794,7 +799,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
     return o;
   };
   // A whole tile of whole 16-byte rows, the common case, is requested without a bound a load: a thread's row of the u-th load is u * RS rows on.
-  const bool plain = vec && dim == dimP && TT * d4n >= 256;
+  const bool plain = R == 4 && vec && dim == dimP && TT * d4n >= 256;
   constexpr int RS = 256 / d4n;
   const float* kp = a.k + (size_t)(t0 + tid / d4n) * a.ldk + hq * dim + tid % d4n * 4;
   const float* qp = a.q + (size_t)(t0 + tid / d4n) * a.ldq + hq * dim + tid % d4n * 4;
@@ -835,7 +840,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
 #pragma unroll
     for (int u = 0; u < NL; u++) {
       const int e = tid + u * 256;
-      if (e < nt * d4n) {
+      if (e < (TILED ? nt : TT) * d4n) {
         float4 kk = kn[u], qv = qn[u];
         if (ACT) {
           kk.x = siluf_(kk.x), kk.y = siluf_(kk.y), kk.z = siluf_(kk.z), kk.w = siluf_(kk.w);
@@ -845,7 +850,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
         qv.x *= a.q_scale, qv.y *= a.q_scale, qv.z *= a.q_scale, qv.w *= a.q_scale;
         *(float4*)(qs + e * 4) = qv;
         if (DECAY == 1) *(float4*)(ds + e * 4) = dn[u];
-        if (!BONUS) {  // (the d4n neighbouring lanes that hold a token's row; zeros beyond its size)
+        if (BETA) {  // (the d4n neighbouring lanes that hold a token's row; zeros beyond its size)
           const float c = group_sum<d4n>(fmaf(kk.x, qv.x, fmaf(kk.y, qv.y, fmaf(kk.z, qv.z, kk.w * qv.w))));
           if (e % d4n == 0) cs[e / d4n] = c;
         }
@@ -861,12 +866,12 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
 #pragma unroll
     for (int u = 0; u < NV; u++) {
       const int e = tid + u * 256;
-      if (e < nt * CPB) vs[e] = ACT ? siluf_(vbuf[u]) : vbuf[u];
+      if (e < (TILED ? nt : TT) * CPB) vs[e] = ACT ? siluf_(vbuf[u]) : vbuf[u];
     }
     if (BETA && tid < TT) bs[tid] = bn;
     if (DECAY == 2 && tid < TT) gs[tid] = gn;
   };
-  // A tile's outputs leave together, behind the next tile's deposit: a store a token, under a branch, would make the wait for the next tile's
+  // R = 4: a tile's outputs leave together, behind the next tile's deposit: a store a token, under a branch, would make the wait for the next tile's
   // operands (loads and stores are counted together) a wait for every store's way to memory.
   auto leave = [&](int i0, int nt) {
 #pragma unroll
@@ -880,7 +885,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
     const int nt = min(TT, n - i0);
     __syncthreads();
     deposit(nt);
-    if (i0 > 0) leave(i0 - TT, TT);
+    if (TILED && i0 > 0) leave(i0 - TT, TT);
     __syncthreads();
     if (i0 + TT < n) request(i0 + TT);
     // a token's operands come from LDS ahead of its arithmetic (16-byte reads), two tokens with 4 rows a lane: one token's work is shorter than their way
@@ -898,7 +903,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
       }
       uv[w] = vs[i * CPB + cl];
       if (BETA || BONUS) bv[w] = bs[i];
-      if (!BONUS) cv[w] = cs[i];
+      if (BETA) cv[w] = cs[i];
       if (DECAY == 2) gv[w] = gs[i];
     };
     auto lane_sum = [](const float (&v)[NH][2]) {  // (8 rows as two lanes of 4 would add theirs)
@@ -908,8 +913,8 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
     };
     auto token = [&](int i, int w, auto whole) {  // outputs of a whole tile leave together, those of a part of one at once
       auto put = [&](float o) {
-        if (r == 0 && whole) os[i * CPB + cl] = o;
-        if (r == 0 && !whole && col) a.out[(size_t)(t0 + i0 + i) * a.ldo + h * vdim + c] = o;
+        if (r == 0 && TILED && whole) os[i * CPB + cl] = o;
+        if (r == 0 && !(TILED && whole) && col) a.out[(size_t)(t0 + i0 + i) * a.ldo + h * vdim + c] = o;
       };
       if (BONUS) {
         const float u = uv[w];
@@ -924,15 +929,24 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
       }
 #pragma unroll
       for (int j = 0; j < R; j++) S[j] *= DECAY == 1 ? dv[w][j] : (DECAY == 2 ? gv[w] : hd);
+      float u = uv[w], d[NH][2] = {}, o[NH][2] = {};
+      if (!BETA) {  // (u is known: no token waits for another's sum)
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+          S[j] = fmaf(kv[w][j], u, S[j]);
+          o[j / 4][j & 1] = fmaf(S[j], qv[w][j], o[j / 4][j & 1]);
+        }
+        put(group_sum<P>(lane_sum(o)));
+        return;
+      }
       // S^T k and S^T q of the decayed state side by side (two chains each; their sum order is fixed): the output of the new state is
       // (S + k u^T)^T q = S^T q + (k . q) u, so it does not wait for u, and one chain's steps fill the other's wait states
-      float u = uv[w], d[NH][2] = {}, o[NH][2] = {};
 #pragma unroll
       for (int j = 0; j < R; j++) {
-        if (BETA) d[j / 4][j & 1] = fmaf(S[j], kv[w][j], d[j / 4][j & 1]);
+        d[j / 4][j & 1] = fmaf(S[j], kv[w][j], d[j / 4][j & 1]);
         o[j / 4][j & 1] = fmaf(S[j], qv[w][j], o[j / 4][j & 1]);
       }
-      if (BETA) u = bv[w] * (u - group_sum<P>(lane_sum(d)));
+      u = bv[w] * (u - group_sum<P>(lane_sum(d)));
 #pragma unroll
       for (int j = 0; j < R; j++) S[j] = fmaf(kv[w][j], u, S[j]);
       put(fmaf(cv[w], u, group_sum<P>(lane_sum(o))));
@@ -952,7 +966,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
       }
     }
   }
-  if (n > 0 && n % TT == 0) {
+  if (TILED && n > 0 && n % TT == 0) {
     __syncthreads();
     leave(n - TT, TT);
   }
@@ -1267,7 +1281,7 @@ ScanForm scan_form(const StkScanArgs& a) {
   if (!a.cu_q) return {4, f.P, 1};
   const bool few = a.max_q > 0 && a.max_q <= 16;
   const int cols8 = 512 / f.P;  // columns of a workgroup at 8 rows a lane
-  if (a.dim > 32 && !few && (int64_t)((a.vdim + cols8 - 1) / cols8) * a.H * a.B >= 2 * 256) return {8, f.P / 2, 16};
+  if (a.dim > 16 && (a.dim > 32 || a.vdim >= cols8) && !few && (int64_t)((a.vdim + cols8 - 1) / cols8) * a.H * a.B >= 2 * 256) return {8, f.P / 2, 16};
   f.TT = few || f.P == 1 || f.P == 64 ? 16 : 32;  // (one lane a column: the values and outputs of 32 tokens would take 64 KB of LDS)
   return f;
 }
@@ -1312,6 +1326,7 @@ void vra_stack_linear_scan(const StkScanArgs& a, int64_t stream) {
     break
   if (f.R == 8) {
     switch (f.P) {
+      case 4: STK_SCAN(8, 4, 16); break;
       case 8: STK_SCAN(8, 8, 16); break;
       case 16: STK_SCAN(8, 16, 16); break;
       default: STK_SCAN(8, 32, 16); break;
