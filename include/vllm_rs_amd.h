@@ -660,7 +660,7 @@ void vra_stack_op_gemm_tile(int32_t tile, const void* a, int32_t lda, const void
                             int32_t M, int32_t N, int32_t K, const int32_t* tile_group, const int32_t* a_row, int32_t a_rows,
                             const int32_t* out_row, int32_t epi, float limit, int64_t stream);
 /* columns a workgroup of vra_stack_op_gemm takes at up to 32 rows in bf16 (pair: with the gated epilogue): 16 or 32, with the same sums */
-int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t pair);
+int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t batch, int32_t pair);
 /* rows of the row space that a model gives `pairs` token-expert pairs over `experts` experts (tiles128: its products run on 128-row tiles) */
 int32_t vra_stack_op_expert_rows(int32_t pairs, int32_t experts, int32_t tiles128);
 void vra_stack_op_moe_sort(const int32_t* pair_expert, const float* pair_weight, int32_t P, int32_t top, int32_t n_groups,

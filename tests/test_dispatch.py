@@ -56,9 +56,10 @@ def test_expert_rows(pairs, experts):
     (17, 3072, 8192, 32),  # 25.4 / 31.1
     (32, 4000, 4096, 32),  # 15.9 / 18.1
     (32, 3072, 512, 32),  # 5.6 / 6.2
-    (8, 8000, 4096, 16),  # 17.9 / 16.2
+    (16, 6144, 4096, 32),  # 16.7 / 19.2
+    (16, 4096, 4096, 16),  # 16.1 / 11.9
     (8, 6144, 512, 32),  # 5.1 / 5.6
 ])
 def test_columns_of_few_row_products(M, N, K, want):
     L = _lib.load()
-    assert L.vra_stack_op_gemm_few_columns(M, N, K, 1, 0) == want and L.vra_stack_op_gemm_few_columns(M, N, K, 1, 1) == 32
+    assert L.vra_stack_op_gemm_few_columns(M, N, 1, 0) == want and L.vra_stack_op_gemm_few_columns(M, N, 1, 1) == 32

@@ -224,7 +224,7 @@ def load():
     _sig(lib, "vra_stack_op_linear_scan", None, P, c_i32, P, c_i32, P, c_i32, P, c_i32, P, P, c_i32, c_f32, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32,
          c_i32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_gemm_tile", None, c_i32, P, c_i32, P, c_i64, P, c_i32, c_i32, c_i32, c_i32, c_i32, P, P, c_i32, P, c_i32, c_f32, c_i64)
-    _sig(lib, "vra_stack_op_gemm_few_columns", c_i32, c_i32, c_i32, c_i32, c_i32, c_i32)
+    _sig(lib, "vra_stack_op_gemm_few_columns", c_i32, c_i32, c_i32, c_i32, c_i32)
     _sig(lib, "vra_stack_op_expert_rows", c_i32, c_i32, c_i32, c_i32)
     _sig(lib, "vra_stack_op_linear_scan_lds", c_i32, c_i32, c_i32, c_i32, c_i32, c_i32)
     _sig(lib, "vra_stack_op_sandwich_norm", None, P, P, c_i32, P, c_f32, P, c_f32, P, P, P, c_f32, c_i32, c_i32, P, P, c_i32, c_i32, P, P, c_i32, c_i64)

@@ -46,7 +46,7 @@ struct StkGemmArgs {
 };
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream);
 // columns a workgroup takes of a bf16 product of up to 32 rows (pair: with the gated epilogue): 16 or 32, the sums are the same
-extern "C" int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t pair);
+extern "C" int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t batch, int32_t pair);
 // rows per granule the grouped launches of an M-row problem over `groups` groups want (16, 64, or 128 where `tiles128`: both products of the
 // expert are bf16 with K a multiple of 64)
 int vra_stack_gemm_granule(int rows, int groups, bool tiles128);

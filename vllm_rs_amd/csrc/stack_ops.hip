@@ -1393,12 +1393,12 @@ static bool rows_kernel_takes(const StkGemmArgs& g) {
 }
 
 // Columns a workgroup takes of a product of up to 32 rows.  32 read x half as often, but while 16 fit one round of the CUs they leave CUs idle (8 rows:
-// 2048 columns, K = 2048 / 8192: 7.3 / 22.9 us, with 16 columns 5.5 / 14.6; 17 rows, 2048 columns: 8.3 / 24.9, 6.2 / 17.3).  Beyond that round 16 lose where
-// x is read by two row blocks (17 rows, 3072 columns, K = 8192: 25.4, with 16 columns 31.1); with one they still gain at K = 2048..4096
-// (8 rows, 8000 columns: 10.4 / 17.9, 9.9 / 16.2) and not beside (K = 512: 5.3, 5.6; K = 8192 29.3, 29.0).  A gated pair needs both its blocks.
-int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t K, int32_t batch, int32_t pair) {
+// 2048 columns, K = 2048 / 8192: 7.3 / 22.9 us, with 16 columns 5.5 / 14.6; 17 rows, 2048 columns: 8.3 / 24.9, 6.2 / 17.3).  Beyond that round 16
+// lose (17 rows, 3072 columns, K = 8192: 25.4, with 16 columns 31.1; 16 rows, 6144 columns, K = 4096: 16.7, 19.2) or change little (8 rows, 8000
+// columns, K = 512 / 4096: 5.3 / 17.9, 5.6 / 16.2).  A gated pair needs both its blocks.
+int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t batch, int32_t pair) {
   const int64_t wide = (int64_t)((M + 15) / 16) * ((N + 31) / 32) * batch;
-  return pair || (wide > 128 && !(M <= 16 && K >= 2048 && K <= 4096 && wide < 256)) ? 32 : 16;
+  return pair || wide > 128 ? 32 : 16;
 }
 
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
@@ -1450,7 +1450,7 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
       else if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<2, 4, 2, 2, false, true><<<grid, 256, 0, st>>>(g); });
       else launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<2, 4, 2, 2, false><<<grid, 256, 0, st>>>(g); });
     } else {
-      const bool wide = vra_stack_op_gemm_few_columns(g.M, g.N, g.K, nb, g.epi == 1) == 32;
+      const bool wide = vra_stack_op_gemm_few_columns(g.M, g.N, nb, g.epi == 1) == 32;
 #define STK_SMALL(NTV)                                                                                                                 \
   do {                                                                                                                               \
     dim3 grid((g.M + 15) / 16, (g.N + 16 * NTV - 1) / (16 * NTV), nb);                                                               \
