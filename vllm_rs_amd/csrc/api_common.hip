@@ -103,6 +103,7 @@ struct ScratchSet {
   float* slabs = nullptr;
   unsigned char* scales = nullptr;
   uint32_t* counters = nullptr;
+  uint32_t* error = nullptr;  // pinned host memory: kernels write it (a wait that gave up), the host reads it behind a step's synchronisation without a copy
 };
 static ScratchSet g_scratch[kMaxDevices];
 static std::mutex g_scratch_mu;
@@ -110,10 +111,10 @@ static ScratchSet* scratch_for_current_device(bool create) {
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
   ScratchSet& s = g_scratch[dev];
-  if (s.slabs && s.counters && s.scales) return &s;
+  if (s.slabs && s.counters && s.error && s.scales) return &s;
   if (!create) return nullptr;
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  if (s.slabs && s.counters && s.scales) return &s;
+  if (s.slabs && s.counters && s.error && s.scales) return &s;
   void* p = nullptr;
   if (!s.slabs) {
     if (hipMalloc(&p, kSlabBytes) != hipSuccess) return nullptr;
@@ -124,9 +125,14 @@ static ScratchSet* scratch_for_current_device(bool create) {
     s.slabs = (float*)p;
   }
   if (!s.counters) {
-    if (hipMalloc(&p, (kCounters + 16) * sizeof(uint32_t)) != hipSuccess) return nullptr;
-    if (hipMemset(p, 0, (kCounters + 16) * sizeof(uint32_t)) != hipSuccess) return nullptr;
+    if (hipMalloc(&p, kCounters * sizeof(uint32_t)) != hipSuccess) return nullptr;
+    if (hipMemset(p, 0, kCounters * sizeof(uint32_t)) != hipSuccess) return nullptr;
     s.counters = (uint32_t*)p;
+  }
+  if (!s.error) {
+    if (hipHostMalloc(&p, 64, hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) return nullptr;
+    memset(p, 0, 64);
+    s.error = (uint32_t*)p;
   }
   if (!s.scales) {
     if (hipMalloc(&p, 2 * kScaleBytes) != hipSuccess) return nullptr;
@@ -152,21 +158,29 @@ size_t vra_scratch_slab_bytes() { return kSlabBytes; }
 size_t vra_scratch_counter_count() { return kCounters; }
 uint32_t* vra_scratch_error_word() {
   ScratchSet* s = scratch_for_current_device(true);
-  return s ? s->counters + kCounters : nullptr;
+  return s ? s->error : nullptr;
+}
+uint32_t vra_scratch_error_seen() {
+  ScratchSet* s = scratch_for_current_device(false);
+  return s ? *(volatile uint32_t*)s->error : 0;
 }
 int vra_scratch_take_error() {
   ScratchSet* s = scratch_for_current_device(false);
-  if (!s) return 0;
-  uint32_t v = 0;
-  if (hipMemcpy(&v, s->counters + kCounters, sizeof(v), hipMemcpyDeviceToHost) != hipSuccess) return 0;
+  if (!s || hipDeviceSynchronize() != hipSuccess) return 0;
+  const uint32_t v = *(volatile uint32_t*)s->error;
   // a wait that gave up leaves the exchange state of that launch undefined: the owner cleared a flag it never saw raised and the
-  // late slice may still raise it afterwards — the next launch would then consume stale slabs without waiting (ADVICE r4).  The
-  // device is idle here (the copy above synchronised): every flag goes back to zero together with the error word.
-  if (v) (void)hipMemset(s->counters, 0, (kCounters + 1) * sizeof(uint32_t));
+  // late slice may still raise it afterwards — the next launch would then consume stale slabs without waiting.  The
+  // device is idle here: every flag goes back to zero together with the error word.
+  if (v) {
+    (void)hipMemset(s->counters, 0, kCounters * sizeof(uint32_t));
+    *(volatile uint32_t*)s->error = 0;
+  }
   return v != 0;
 }
-// the same for callers that read the error word with their own copy (host/engine.cpp): queue the reset of flags + error word
+// the same for callers that read the error word themselves behind a synchronisation (host/engine.cpp): queue the reset of the flags
 void vra_scratch_reset_after_error(hipStream_t st) {
   ScratchSet* s = scratch_for_current_device(false);
-  if (s) (void)hipMemsetAsync(s->counters, 0, (kCounters + 1) * sizeof(uint32_t), st);
+  if (!s) return;
+  *(volatile uint32_t*)s->error = 0;
+  (void)hipMemsetAsync(s->counters, 0, kCounters * sizeof(uint32_t), st);
 }

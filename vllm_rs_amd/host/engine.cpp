@@ -127,7 +127,7 @@ class Engine {
   size_t off_ids_, off_pos_, off_slots_, off_bt_, off_ctx_, off_cuq_, off_last_, off_dids_, off_dpos_, off_dslots_, off_rows_, off_state_, off_prev_;
   uint32_t* d_tokens_ = nullptr;
   uint32_t* h_tokens_ = nullptr;
-  uint32_t* h_err_ = nullptr;  // pinned copy of the device error words (split-K exchange, one-shot all-reduce), read every step
+  uint32_t* h_err_ = nullptr;  // pinned copy of the one-shot all-reduce's error word ([1]), read every step
   std::map<int64_t, hipGraphExec_t> graphs_;
   hipGraphExec_t last_graph_ = nullptr;  // the decode graph of the most recent step (vra_engine_bench_replay)
   bool prepared_ = false;
@@ -533,9 +533,7 @@ class Engine {
     }
     if (!sample_stochastic(ids, is_prefill)) return false;
     if (hipMemcpyAsync(h_tokens_, d_tokens_, (size_t)B * 4, hipMemcpyDeviceToHost, stream_) != hipSuccess) return fail("token download failed");
-    // the split-K exchange's error word rides along with the tokens: EVERY step is checked before its tokens are committed
-    uint32_t* dev_err = vra_scratch_error_word();
-    if (dev_err && hipMemcpyAsync(h_err_, dev_err, 4, hipMemcpyDeviceToHost, stream_) != hipSuccess) return fail("error-word download failed");
+    // the split-K exchange's error word is host memory that the kernels write: EVERY step is checked before its tokens are committed
     uint32_t* comm_err = comm_ ? vra_comm_error_word(comm_) : nullptr;
     if (comm_err && hipMemcpyAsync(h_err_ + 1, comm_err, 4, hipMemcpyDeviceToHost, stream_) != hipSuccess) return fail("error-word download failed");
     if (hipStreamSynchronize(stream_) != hipSuccess) return fail(std::string("stream error: ") + hipGetErrorString(hipGetLastError()));
@@ -544,8 +542,7 @@ class Engine {
       (void)hipMemsetAsync(comm_err, 0, 4, stream_);
       return fail("one-shot all-reduce timed out waiting for a peer (results of this step are invalid)" + comm_timeout_detail(comm_));
     }
-    if (h_err_[0]) {
-      h_err_[0] = 0;
+    if (vra_scratch_error_seen()) {
       vra_scratch_reset_after_error(stream_);  // flags too: a timed-out exchange leaves them undefined
       return fail("split-K exchange timed out on the device (results of this step are invalid)");
     }
@@ -1221,10 +1218,8 @@ static int32_t forward_raw_impl(Engine* en, const uint32_t* h_ids, const int64_t
     }
     if (hipMemcpyAsync(en->h_tokens_, en->d_tokens_, (size_t)n_seqs * 4, hipMemcpyDeviceToHost, en->stream_) != hipSuccess) return en->error = "token download failed", -1;
   }
-  // the device error words (a split-K slice or a tensor-parallel peer that never arrived) ride along, as in step()
-  uint32_t* dev_err = vra_scratch_error_word();
+  // the error words (a split-K slice or a tensor-parallel peer that never arrived) are checked as in step()
   uint32_t* comm_err = en->comm_ ? vra_comm_error_word(en->comm_) : nullptr;
-  if (dev_err) (void)hipMemcpyAsync(en->h_err_, dev_err, 4, hipMemcpyDeviceToHost, en->stream_);
   if (comm_err) (void)hipMemcpyAsync(en->h_err_ + 1, comm_err, 4, hipMemcpyDeviceToHost, en->stream_);
   if (hipStreamSynchronize(en->stream_) != hipSuccess) {
     en->error = "stream error in forward_raw";
@@ -1236,8 +1231,7 @@ static int32_t forward_raw_impl(Engine* en, const uint32_t* h_ids, const int64_t
     en->error = "one-shot all-reduce timed out waiting for a peer (results of this forward are invalid)" + comm_timeout_detail(en->comm_);
     return -1;
   }
-  if (dev_err && en->h_err_[0]) {
-    en->h_err_[0] = 0;
+  if (vra_scratch_error_seen()) {
     vra_scratch_reset_after_error(en->stream_);  // flags too: a timed-out exchange leaves them undefined
     en->error = "split-K exchange timed out on the device (results of this forward are invalid)";
     return -1;
