@@ -742,6 +742,13 @@ void vra_stack_op_attention_window(const void* q, int32_t ldq, void* out, const 
                                    int32_t max_q, int32_t H, int32_t G, int32_t dim, int32_t vdim, int32_t BS, int32_t max_blocks,
                                    float scale, int32_t window, const float* sink, const float* head_scale, const float* gate,
                                    int32_t gate_ld, int32_t dtype, int64_t stream);
+/* attention_decode: the decode form (one token a sequence) as a model's step calls it: scratch for `splits` parts of a context and `arrived`, B * G
+ * counters that are zero before the call and after it (null: the form without parts). */
+void vra_stack_op_attention_decode(const void* q, int32_t ldq, void* out, const void* kc, const void* vc, const int64_t* positions,
+                                   const uint32_t* block_tables, const uint32_t* context_lens, int32_t B, int32_t H, int32_t G, int32_t dim,
+                                   int32_t vdim, int32_t BS, int32_t max_blocks, float scale, float softcap, float temp_coef, int32_t temp_every,
+                                   int32_t chunk, int32_t window, const float* sink, const float* head_scale, const float* gate, int32_t gate_ld,
+                                   float* scratch, int64_t scratch_bytes, int32_t splits, uint32_t* arrived, int32_t dtype, int64_t stream);
 void vra_stack_op_seam(float* x, const float* p1, int32_t n1, const float* pw, const int32_t* pe, float c1, const float* p2, const float* p2w,
                        float c2, const float* p1_norm_w, const float* p2_norm_w, int32_t norm_kind, const float* post_w, const float* post_b,
                        float post_alpha, const float* pre_w, const float* pre_b, float pre_alpha, void* h, float* h32, float eps, int32_t T,

@@ -230,6 +230,8 @@ def load():
     _sig(lib, "vra_stack_op_sandwich_norm", None, P, P, c_i32, P, c_f32, P, c_f32, P, P, P, c_f32, c_i32, c_i32, P, P, c_i32, c_i32, P, P, c_i32, c_i64)
     _sig(lib, "vra_stack_op_attention_window", None, P, c_i32, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
          c_f32, c_i32, P, P, P, c_i32, c_i32, c_i64)
+    _sig(lib, "vra_stack_op_attention_decode", None, P, c_i32, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_f32, c_f32, c_f32, c_i32,
+         c_i32, c_i32, P, P, P, c_i32, P, c_i64, c_i32, P, c_i32, c_i64)
     _sig(lib, "vra_stack_op_seam", None, P, P, c_i32, P, P, c_f32, P, P, c_f32, P, P, c_i32, P, P, c_f32, P, P, c_f32, P, P, c_f32, c_i32, c_i32, P, P,
          c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, P, P, P, c_i32, c_i64)
     _sig(lib, "vra_stack_op_conv_rows", None, P, c_i32, c_i32, c_i32, P, P, P, c_i32, P, c_i32, P, P, P, c_i32, c_i32, c_i64)

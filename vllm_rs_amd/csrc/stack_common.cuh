@@ -5,6 +5,12 @@
 #include "common.cuh"
 #include "stack_launch.h"
 
+// v of the lane that the DPP control names (rows of 16 lanes)
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+
 namespace {
 
 template <typename T>

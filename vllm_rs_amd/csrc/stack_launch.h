@@ -142,7 +142,15 @@ struct StkAttnArgs {
   float* scratch = nullptr;
   size_t scratch_bytes = 0;
   int splits = 0;
+  uint32_t* arrived = nullptr;  // plain decode form in parts (vra_stack_decode_group): B * G counters, zero before and after a launch
 };
+// most parts a decoded token's context is cut into
+#define STK_DEC_PARTS 32
+// the plain decode form with a key/value head's query heads together, in parts (stack_decode_attn.hip): its parts for a model (0: not its shapes), the
+// scratch they take, and the launch (false: not a shape of that kernel, or no scratch; nothing was launched)
+int vra_stack_decode_parts(int max_len, int max_seqs, int heads, int kv_heads, int dim, int vdim, int dtype);
+size_t vra_stack_decode_scratch(int parts, int max_seqs, int heads, int kv_heads, int dim, int vdim);
+bool vra_stack_decode_group(const StkAttnArgs& a, int dtype, int64_t stream);
 void vra_stack_attention(const StkAttnArgs& a, int dtype, int64_t stream);
 // parts of the key range the differential decode form takes for a batch of B sequences (few heads a step: more parts, so that a long context spreads
 // over the chip), and the scratch that holds them for any batch up to max_seqs

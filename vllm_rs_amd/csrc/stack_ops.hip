@@ -1114,7 +1114,7 @@ __global__ __launch_bounds__(256 * MAPS, MAPS == 2 && DC <= 2 ? 4 : 1) void stk_
     }
 }
 
-// One decoded token per sequence: a workgroup per (sequence, query head); its 8 waves take the 64-key tiles of the context in turn,
+// One decoded token per sequence, for what stack_decode_attn.hip does not take: a workgroup per (sequence, query head); its 8 waves take the 64-key tiles of the context in turn,
 // read K rows straight from the cache (lane = key, 16 bytes a load where the row allows) and V rows channel-wise (lane = channel), and
 // meet once in LDS.  The order of the sums depends on the context length alone.
 // MAPS 2: the differential form of StkAttnArgs (both maps' scores of a key, then one pass over the values for both);
@@ -1563,7 +1563,7 @@ void vra_stack_attention(const StkAttnArgs& a, int dtype, int64_t stream) {
   const size_t dm = (size_t)a.maps * a.dim;
   hipStream_t st = as_stream(stream);
   if (!a.cu_q) {
-    if (!two && vra_stack_latent_decode(a, dtype, stream)) return;
+    if (!two && a.arrived ? vra_stack_decode_group(a, dtype, stream) : !two && vra_stack_latent_decode(a, dtype, stream)) return;
     const size_t lds = (std::max<size_t>(dm, STK_DW) + (a.maps + 1) * STK_DW * 64 + a.maps * (2 * STK_DW + STK_DW * (size_t)a.vdim)) * sizeof(float);
     VRA_CHECK_ARG(lds <= 64 * 1024, "stack attention: head does not fit LDS");
     StkAttnArgs k = a;

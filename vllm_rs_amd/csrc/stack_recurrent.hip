@@ -83,10 +83,6 @@ __device__ __forceinline__ float center_rows(float* xs, int W, int tid, float ep
 }
 
 // a lane's partner by DPP (row-local controls only)
-template <int CTRL>
-__device__ __forceinline__ float dpp_f32(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
 __device__ __forceinline__ float wave_sum_dpp(float v) {
   v += dpp_f32<0xB1>(v);
   v += dpp_f32<0x4E>(v);

@@ -1050,6 +1050,17 @@ bool StackModel::init_buffers(int max_tokens, int max_seqs) {
     if (L.mixer == 7) lat_scratch_bytes_ = std::max(lat_scratch_bytes_, vra_stack_diff_scratch(mc_.max_position_embeddings, max_seqs, L.heads, L.vdim));
   }
   if (lat_scratch_bytes_ && !(lat_scratch_ = (float*)dalloc(lat_scratch_bytes_))) return false;
+  size_t arrivals = 0;
+  for (const StackLayer& L : layers_) {
+    if (L.mixer != 0 && L.mixer != 5) continue;
+    const int s = vra_stack_decode_parts(mc_.max_position_embeddings, max_seqs, L.heads, L.kv_heads, L.dim, L.vdim, dt_);
+    if (s < 1) continue;
+    dec_scratch_bytes_ = std::max(dec_scratch_bytes_, vra_stack_decode_scratch(s, max_seqs, L.heads, L.kv_heads, L.dim, L.vdim));
+    arrivals = std::max(arrivals, (size_t)max_seqs * L.kv_heads);
+  }
+  if (arrivals && (!(dec_scratch_ = (float*)dalloc(dec_scratch_bytes_)) || !(dec_arrived_ = (uint32_t*)dalloc(arrivals * 4)) ||
+                   hipMemset(dec_arrived_, 0, arrivals * 4) != hipSuccess))
+    return false;
   if (nmix && !(mix_ = dalloc(nmix * T * W * es_))) return false;
   if (want_h32 && ((block_ != 3 && !(h32_ = (float*)dalloc(T * W * 4))) || !(id_weight_ = (float*)dalloc(T * 4)))) return false;
   const size_t P = T * std::max<size_t>(top, 1);
@@ -1179,11 +1190,19 @@ bool StackModel::mixer_softmax(const StackLayer& L, const InputMetadata& md, int
   a.B = B, a.T = T, a.max_q = md.is_prefill ? md.max_seqlen_q : 1, a.H = L.heads, a.G = L.kv_heads, a.dim = L.dim, a.vdim = L.vdim;
   a.BS = ec_.block_size, a.max_blocks = md.max_blocks;
   a.scale = L.scale, a.softcap = L.softcap, a.temp_coef = L.temp_coef, a.temp_every = L.temp_every;
+  in_parts(L, a);
   vra_stack_attention(a, dt_, stream);
   StkGemmArgs o;
   o.a = attn_, o.lda = L.heads * L.vdim, o.w = L.o, o.M = T, o.N = W, o.K = L.heads * L.vdim, o.out = o_, o.ldo = W, o.out_f32 = 1;
   vra_stack_gemm(o, dt_, stream);
   return !take_stack_err(error, "mixer");
+}
+
+// decode steps of bf16 models: a key/value head's query heads together, the context in parts
+void StackModel::in_parts(const StackLayer& L, StkAttnArgs& a) const {
+  if (a.cu_q || !dec_scratch_) return;
+  a.splits = vra_stack_decode_parts(mc_.max_position_embeddings, max_seqs_, L.heads, L.kv_heads, L.dim, L.vdim, dt_);
+  if (a.splits > 0) a.scratch = dec_scratch_, a.scratch_bytes = dec_scratch_bytes_, a.arrived = dec_arrived_;
 }
 
 // Latent attention in its absorbed form: the cache row of a token is [normed kv latent | rotated key part]; a head's query becomes
@@ -1458,6 +1477,7 @@ bool StackModel::mixer_parallel(const StackLayer& L, const InputMetadata& md, in
   a.cu_q = md.is_prefill ? md.cu_seqlens_q : nullptr;
   a.B = B, a.T = T, a.max_q = md.is_prefill ? md.max_seqlen_q : 1, a.H = H, a.G = L.kv_heads, a.dim = L.dim, a.vdim = L.vdim;
   a.BS = ec_.block_size, a.max_blocks = md.max_blocks, a.scale = L.scale, a.chunk = L.chunk;
+  in_parts(L, a);
   vra_stack_attention(a, dt_, stream);
   StkGemmArgs o;
   o.a = attn_, o.lda = H * L.vdim, o.w = L.o, o.M = T, o.N = W, o.K = H * L.vdim, o.out = o_, o.ldo = W, o.out_f32 = 1;
@@ -1668,6 +1688,7 @@ bool StackModel::mixer_hybrid(const StackLayer& L, const InputMetadata& md, int6
   a.BS = ec_.block_size, a.max_blocks = md.max_blocks, a.scale = L.scale, a.chunk = L.chunk, a.window = L.window;
   a.sink = L.sink ? L.sink_w : nullptr, a.head_scale = L.head_temp ? L.temp_w : nullptr;
   if (L.head_gate) a.gate = z_ + g0, a.gate_ld = n1;
+  in_parts(L, a);
   vra_stack_attention(a, dt_, stream);
   StkGemmArgs o;
   o.a = attn_, o.lda = H * L.vdim, o.w = L.o, o.M = T, o.N = W, o.K = H * L.vdim, o.out = o_, o.ldo = W, o.out_f32 = 1;

@@ -77,6 +77,7 @@
 
 #include "model_base.h"
 
+struct StkAttnArgs;
 namespace vra {
 
 struct StackLayer {
@@ -227,6 +228,7 @@ class StackModel : public ModelBase {
   bool parse_spec(const char* spec);
   bool feed_forward(const StackLayer& L, int T, int64_t stream);
   bool mixer_softmax(const StackLayer& L, const InputMetadata& md, int64_t stream);
+  void in_parts(const StackLayer& L, StkAttnArgs& a) const;
   bool mixer_latent(const StackLayer& L, const InputMetadata& md, int64_t stream);
   bool mixer_sigmoid(const StackLayer& L, const InputMetadata& md, int64_t stream);
   bool mixer_delta(const StackLayer& L, const InputMetadata& md, int64_t stream);
@@ -295,6 +297,9 @@ class StackModel : public ModelBase {
   size_t sig_scratch_bytes_ = 0;
   float* lat_scratch_ = nullptr;  // decoded tokens of latent and differential layers: partial sums over parts of the key range
   size_t lat_scratch_bytes_ = 0;
+  float* dec_scratch_ = nullptr;  // decoded tokens of softmax layers: the same, and the counters of parts that are done (zero between launches)
+  size_t dec_scratch_bytes_ = 0;
+  uint32_t* dec_arrived_ = nullptr;
   bool trace_on_ = false;
   float* trace_ = nullptr;
   size_t trace_cap_ = 0, trace_bytes_ = 0;
