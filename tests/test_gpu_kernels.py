@@ -675,6 +675,14 @@ def test_rope_cache_prefill_equals_the_two_launches(dt, fp8, Hq, Hkv, D, T):
     assert np.array_equal(k2.numpy(np.uint16, k.shape), k), "k itself is left un-rotated"
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,D,T", [(28, 4, 128, 800), (9, 3, 64, 1100), (8, 1, 128, 1030), (32, 8, 128, 391), (24, 24, 64, 1024)])
+def test_rope_cache_prefill_slices_of_heads(fp8, Hq, Hkv, D, T):
+    """heads divided over the grid's second dimension: slices of unequal size (3 heads over 8 workgroups' worth, one head), short steps of wide
+    models in groups of 8 tokens, a last group of 7 tokens"""
+    test_rope_cache_prefill_equals_the_two_launches(BF16, fp8, Hq, Hkv, D, T)
+
+
 # ---------------------------------------------------------------- paged KV + attention
 def _paged_setup(r, ctxs, Hkv, D, BS, dt, NB=64):
     """random K/V history scattered into a shuffled block pool through reshape_and_cache."""

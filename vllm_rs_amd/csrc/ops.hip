@@ -463,16 +463,24 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(uint16_t* __restrict__ 
                                                          int Hkv, int D, int BS) {
   typedef typename KVT<KV8>::elem kv_t;
   extern __shared__ __attribute__((aligned(16))) unsigned char rc_smem[];  // TG == 8: the group's V rows [8][Hkv*D] in cache format
+  __shared__ int64_t ps[TG], ss[TG];
   const int tid = threadIdx.x;
   const int t0 = blockIdx.x * TG, nt = min(TG, T - t0);
   const int half = D >> 1, per_head = half >> 3;  // 16-byte pair groups per head
-  const int n = Hkv * D;
-  auto rotate = [&](const uint16_t* base, int c, const uint16_t* cs_row, const uint16_t* sn_row, u32x4& r1, u32x4& r2) {
+  const int q0 = Hq * blockIdx.y / gridDim.y, nq = Hq * (blockIdx.y + 1) / gridDim.y - q0;    // this slice's query heads
+  const int h0 = Hkv * blockIdx.y / gridDim.y, nh = Hkv * (blockIdx.y + 1) / gridDim.y - h0;  // and key/value heads
+  const int n = nh * D;
+  const int64_t pos0 = positions[t0], slot0 = slots[t0];
+  if (TG > 1) {
+    if (tid < nt) ps[tid] = positions[t0 + tid], ss[tid] = slots[t0 + tid];
+    __syncthreads();
+  }
+  auto rotate = [&](const uint16_t* base, int c, int64_t pos, u32x4& r1, u32x4& r2) {
     float x1[8], x2[8], cs[8], sn[8], y1[8], y2[8];
     unpack8<DT>(*reinterpret_cast<const u32x4*>(base + c * 8), x1);
     unpack8<DT>(*reinterpret_cast<const u32x4*>(base + half + c * 8), x2);
-    unpack8<DT>(*reinterpret_cast<const u32x4*>(cs_row + c * 8), cs);
-    unpack8<DT>(*reinterpret_cast<const u32x4*>(sn_row + c * 8), sn);
+    unpack8<DT>(*reinterpret_cast<const u32x4*>(cosv + pos * half + c * 8), cs);
+    unpack8<DT>(*reinterpret_cast<const u32x4*>(sinv + pos * half + c * 8), sn);
 #pragma unroll
     for (int e = 0; e < 8; e++) {
       y1[e] = x1[e] * cs[e] - x2[e] * sn[e];
@@ -482,44 +490,22 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(uint16_t* __restrict__ 
   };
   // the group's slots: vector V stores need slot0 % 8 == 0 inside one block and slots slot0 .. slot0 + 7
   bool vec = TG == 8 && nt == 8;
-  const int64_t slot0 = slots[t0];
   if (TG == 8) {
 #pragma unroll
-    for (int i = 0; i < 8; i++) vec = vec && i < nt && slots[t0 + min(i, nt - 1)] == slot0 + i;
+    for (int i = 0; i < TG; i++) vec = vec && ss[min(i, nt - 1)] == slot0 + i;
     vec = vec && slot0 >= 0 && (slot0 % BS) % 8 == 0 && (slot0 % BS) + 8 <= BS;
   }
-  for (int ti = 0; ti < nt; ti++) {
-    const int t = t0 + ti;
-    const int64_t pos = positions[t], slot = slots[t];
-    const uint16_t* cs_row = cosv + pos * half;
-    const uint16_t* sn_row = sinv + pos * half;
-    for (int w = tid; w < Hq * per_head; w += blockDim.x) {  // q: in place
-      const int h = w / per_head, c = w - h * per_head;
-      uint16_t* base = q + ((size_t)t * Hq + h) * D;
-      u32x4 r1, r2;
-      rotate(base, c, cs_row, sn_row, r1, r2);
-      *reinterpret_cast<u32x4*>(base + c * 8) = r1;
-      *reinterpret_cast<u32x4*>(base + half + c * 8) = r2;
-    }
-    if (slot < 0) continue;  // padded lane: nothing is cached
-    const int64_t blk = slot / BS;
-    const int off = (int)(slot % BS);
-    for (int w = tid; w < Hkv * per_head; w += blockDim.x) {  // k: rotated into the cache row
-      const int h = w / per_head, c = w - h * per_head;
-      u32x4 r1, r2;
-      rotate(k + ((size_t)t * Hkv + h) * D, c, cs_row, sn_row, r1, r2);
-      kv_t* row = kc + ((blk * Hkv + h) * BS + off) * D;
-      kv_store8<DT, KV8>(row + c * 8, r1);
-      kv_store8<DT, KV8>(row + half + c * 8, r2);
-    }
-    for (int w = tid; w < Hkv * (D >> 3); w += blockDim.x) {  // v: 8 channels per thread
-      const int h = w / (D >> 3), c = w - h * (D >> 3);
-      const u32x4 vv = *reinterpret_cast<const u32x4*>(v + ((size_t)t * Hkv + h) * D + c * 8);
+  auto values = [&]() {  // 8 channels per thread
+    for (int w = tid; w < nt * nh * (D >> 3); w += 256) {
+      const int ti = TG > 1 ? w / (nh * (D >> 3)) : 0, wt = w - ti * nh * (D >> 3), h = wt / (D >> 3), c = wt - h * (D >> 3);
+      const int64_t slot = TG > 1 ? ss[ti] : slot0;
+      if (slot < 0) continue;  // padded lane: nothing is cached
+      const u32x4 vv = *reinterpret_cast<const u32x4*>(v + ((size_t)(t0 + ti) * Hkv + h0 + h) * D + c * 8);
       if (TG == 8 && vec) {  // staged in cache format; stored token-minor below
         kv_store8<DT, KV8>(reinterpret_cast<kv_t*>(rc_smem) + (size_t)ti * n + h * D + c * 8, vv);
         continue;
       }
-      kv_t* col = vc + ((blk * Hkv + h) * D + c * 8) * BS + off;
+      kv_t* col = vc + ((slot / BS * Hkv + h0 + h) * D + c * 8) * BS + (int)(slot % BS);
       if constexpr (KV8) {
         const u32x2 q8 = vra_pack_e4m3x8<DT>(vv);
 #pragma unroll
@@ -532,18 +518,38 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(uint16_t* __restrict__ 
         }
       }
     }
+  };
+  if (TG == 8) values();  // (staged while q and k are rotated)
+  for (int w = tid; w < nt * nq * per_head; w += 256) {  // q: in place
+    const int ti = TG > 1 ? w / (nq * per_head) : 0, wt = w - ti * nq * per_head, h = wt / per_head, c = wt - h * per_head;
+    uint16_t* base = q + ((size_t)(t0 + ti) * Hq + q0 + h) * D;
+    u32x4 r1, r2;
+    rotate(base, c, TG > 1 ? ps[ti] : pos0, r1, r2);
+    *reinterpret_cast<u32x4*>(base + c * 8) = r1;
+    *reinterpret_cast<u32x4*>(base + half + c * 8) = r2;
   }
+  for (int w = tid; w < nt * nh * per_head; w += 256) {  // k: rotated into the cache row
+    const int ti = TG > 1 ? w / (nh * per_head) : 0, wt = w - ti * nh * per_head, h = wt / per_head, c = wt - h * per_head;
+    const int64_t slot = TG > 1 ? ss[ti] : slot0;
+    if (slot < 0) continue;
+    u32x4 r1, r2;
+    rotate(k + ((size_t)(t0 + ti) * Hkv + h0 + h) * D, c, TG > 1 ? ps[ti] : pos0, r1, r2);
+    kv_t* row = kc + ((slot / BS * Hkv + h0 + h) * BS + (int)(slot % BS)) * D;
+    kv_store8<DT, KV8>(row + c * 8, r1);
+    kv_store8<DT, KV8>(row + half + c * 8, r2);
+  }
+  if (TG != 8) values();
   if (TG == 8 && vec) {
     __syncthreads();
     const int64_t blk = slot0 / BS;
     const int off = (int)(slot0 % BS);
     const kv_t* sv = reinterpret_cast<const kv_t*>(rc_smem);
-    for (int i = tid; i < n; i += blockDim.x) {  // channel i = (h, d): its 8 tokens are 8 consecutive cache elements
+    for (int i = tid; i < n; i += 256) {  // channel i = (h, d): its 8 tokens are 8 consecutive cache elements
       const int h = i / D, d = i - h * D;
       kv_t tok[8];
 #pragma unroll
       for (int e = 0; e < 8; e++) tok[e] = sv[(size_t)e * n + i];
-      kv_t* dst = vc + ((blk * Hkv + h) * D + d) * BS + off;
+      kv_t* dst = vc + ((blk * Hkv + h0 + h) * D + d) * BS + off;
       if constexpr (KV8) {
         u32x2 o;
         o[0] = (uint32_t)tok[0] | ((uint32_t)tok[1] << 8) | ((uint32_t)tok[2] << 16) | ((uint32_t)tok[3] << 24);
@@ -568,13 +574,17 @@ extern "C" void vra_rope_cache_prefill(void* q, const void* k, const void* v, vo
   if (tokens <= 0) return;
   hipStream_t st = as_stream(stream);
   const bool kv8 = kv_dtype == VRA_FP8_E4M3;
-  // groups of 8 tokens (vector V stores) when there are enough tokens to fill the chip that way and the staging fits in LDS
-  const size_t lds8 = (size_t)8 * kv_heads * head_dim * (kv8 ? 1 : 2);
-  const bool g8 = tokens >= 1024 && lds8 <= 64 * 1024 && block_size % 8 == 0;
+  // Groups of 8 tokens (vector V stores) when there are enough values to fill the chip that way and the staging fits in LDS; the heads are divided
+  // over grid.y until there are four workgroups a CU.  us, groups of 8 / single tokens: 32 + 8 heads of 128, 512 tokens 5.8 / 7.1, 256 5.0 / 5.0;
+  // 28 + 4 heads of 128, 768 tokens 6.6 / 6.7, 512 5.6 / 5.5; 32 + 4 heads of 64, 768 tokens 5.3 / 4.9, 1024 5.5 / 6.  With all heads and the tokens of a
+  // group one after the other in one workgroup: 1024 tokens 13..16, 2120 tokens of 28 + 4 heads of 128 17.6 (now 9.7), 8192 of 32 + 8 40.6 (39.7).
+  const int groups = (tokens + 7) / 8, ny = std::max(1, std::min(kv_heads, (1024 + groups - 1) / groups));
+  const size_t lds8 = (size_t)8 * ((kv_heads + ny - 1) / ny) * head_dim * (kv8 ? 1 : 2);
+  const bool g8 = (tokens >= 1024 || (tokens >= 256 && (int64_t)tokens * kv_heads * head_dim >= 384 << 10)) && lds8 <= 64 * 1024 && block_size % 8 == 0;
 #define VRA_RC(DT, K8)                                                                                                                    \
   do {                                                                                                                                    \
     if (g8)                                                                                                                               \
-      rope_cache_kernel<DT, K8, 8><<<(tokens + 7) / 8, 256, lds8, st>>>((uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,             \
+      rope_cache_kernel<DT, K8, 8><<<dim3(groups, ny), 256, lds8, st>>>((uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,             \
                                                                         (typename KVT<K8>::elem*)k_cache, (typename KVT<K8>::elem*)v_cache, \
                                                                         (const uint16_t*)cos, (const uint16_t*)sin, positions, slot_mapping, \
                                                                         tokens, q_heads, kv_heads, head_dim, block_size);                  \
