@@ -717,7 +717,8 @@ __global__ __launch_bounds__(256) void stk_sigmoid_pow_kernel(const float* z, in
 // taken of the state before the token's row enters, (S + k u^T)^T q = S^T q + (k . q) u, so that both sums run side by side.  Without the delta rule
 // a row enters at once and the output is summed of the new state, off the chain.
 //  - Few columns (less than two workgroups a CU at R = 8): R = 4 gives twice the workgroups, and tiles of 32 tokens cover the way to memory.  2048
-//    tokens, 16 heads of 128 x 128, delta rule: 306 us (470 with R = 8 and tiles of 16 tokens, the sums one after the other).
+//    tokens, 16 heads of 128 x 128, delta rule: 306 us (470 with R = 8 and tiles of 16 tokens, the sums one after the other); the delta rule with whole
+//    rows of 64 or 128 channels goes to stk_delta_pair_kernel below.
 //  - More: the SIMDs are full, and R = 8 takes half the instructions for the sums of an element; tiles of 16 tokens leave room for four workgroups
 //    a CU (five with constant decays).  8 sequences of 256 tokens: 139 us (R = 4: 158).  Here registers and code count: outputs are stored at
 //    once and every request is bounded, which the R = 4 form trades for a whole tile's outputs together and a tile's requests without bounds (64
@@ -970,6 +971,222 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
 #pragma unroll
     for (int j = 0; j < R; j++)
       if (r * R + j < dim) sp[j] = S[j];
+}
+
+// The delta rule of few columns, three groups of waves a workgroup.  A wave alone on its SIMD issues an instruction every sixth cycle, whatever
+// depends on what, and the SIMD takes one every second cycle from several waves.  So four waves run nothing but the chain (S^T k, u, the state, and a lane's own
+// part of S^T q), two, a tile behind, add the parts of S^T q and store the outputs, and two fetch the tiles to come.  Sums and bits are those of
+// stk_linear_scan_kernel.  What bounds it: the chain's 33 instructions a token (LDS, at 128 bytes a cycle, is half as long).  2048 tokens, 16 heads of
+// 128 x 128: 307 us with one group, 193 now (64 channels, 1000 tokens: 132, 88); with a second copy of the state for the outputs (LDS reads bound it) 219.
+template <int P>
+struct PairForm {
+  static constexpr int TT = 8, CPB = 256 / P, DIMP = 4 * P;        // tokens a tile, columns a workgroup
+  static constexpr int TILE = 3 * TT * DIMP + CPB * TT + 2 * TT;   // k, q, decays, values, write strengths, decays of a head
+  static constexpr int PARTS = TT * CPB * P;                       // the lanes' parts of a tile's S^T q
+  static constexpr int FLOATS = 3 * TILE + 2 * PARTS + 2 * CPB * TT + 4 * TT;  // three tiles, two tiles' parts and u, four tiles' k . q
+};
+template <int P, int DECAY>
+__global__ __launch_bounds__(512) void stk_delta_pair_kernel(StkScanArgs a) {
+  typedef PairForm<P> F;
+  constexpr int TT = F::TT, CPB = F::CPB, dimP = F::DIMP, Q4 = TT / 4;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int vdim = a.vdim;
+  const int b = blockIdx.z, h = blockIdx.y, hq = h / a.qk_rep, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int slot = a.state_slots[b];
+  if (slot < 0) return;
+  const int t0 = __builtin_amdgcn_readfirstlane((int)a.cu_q[b]), n = __builtin_amdgcn_readfirstlane((int)a.cu_q[b + 1]) - t0;
+  const int tiles = (n + TT - 1) / TT, steps = (tiles + 1) & ~1;  // (an even number: two sets of registers in turn)
+  float* parts = lds + 3 * F::TILE;         // [2][TT][CPB][P]
+  float* us = parts + 2 * F::PARTS;         // [2][CPB][TT]
+  float* kqs = us + 2 * CPB * TT;           // [4][TT]
+  struct Tile {
+    float *k, *q, *d, *v, *b, *g;
+  };
+  auto tile = [&](int i) {
+    float* p = lds + i % 3 * F::TILE;
+    return Tile{p, p + TT * dimP, p + 2 * TT * dimP, p + 3 * TT * dimP, p + 3 * TT * dimP + CPB * TT, p + 3 * TT * dimP + CPB * TT + TT};
+  };
+  auto quad = [](const float* p, float (&o)[4]) {
+    const float4 x = *(const float4*)p;
+    o[0] = x.x, o[1] = x.y, o[2] = x.z, o[3] = x.w;
+  };
+
+  if (wave < 4) {
+    const int tid = threadIdx.x, r = tid % P, cl = tid / P, c = blockIdx.x * CPB + cl;
+    const bool col = c < vdim, fresh = a.positions[t0] == 0;
+    float* sp = a.state + (((size_t)slot * a.H + h) * vdim + (col ? c : 0)) * dimP + r * 4;
+    float S[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) S[j] = !fresh && col ? sp[j] : 0.f;
+    float kv[4][4], qv[4][4], dv[4][4];
+    auto fetch = [&](const Tile& t, int e, int w) {
+      quad(t.k + e * dimP + r * 4, kv[w]);
+      quad(t.q + e * dimP + r * 4, qv[w]);
+      if (DECAY == 1) quad(t.d + e * dimP + r * 4, dv[w]);
+    };
+    __syncthreads();
+    fetch(tile(0), 0, 0);
+    fetch(tile(0), 1, 1);
+    for (int i = 0; i < tiles; i++) {
+      const Tile t = tile(i), next = tile(i + 1);  // (the tile after the last: whatever is there, not used)
+      const int nt = min(TT, n - i * TT);
+      float* pp = parts + (i & 1) * F::PARTS + tid;
+      float vb[Q4][4], bb[Q4][4], gb[Q4][4], mine = 0.f;
+#pragma unroll
+      for (int e = 0; e < Q4; e++) {
+        quad(t.v + cl * TT + e * 4, vb[e]);
+        quad(t.b + e * 4, bb[e]);
+        if (DECAY == 2) quad(t.g + e * 4, gb[e]);
+      }
+      auto token = [&](int e, int w, float v, float be, float g) {
+        float d[2] = {0.f, 0.f}, o[2] = {0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; j++) S[j] *= DECAY == 1 ? dv[w][j] : g;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          d[j & 1] = fmaf(S[j], kv[w][j], d[j & 1]);
+          o[j & 1] = fmaf(S[j], qv[w][j], o[j & 1]);
+        }
+        const float u = be * (v - group_sum<P>(d[0] + d[1]));
+        pp[e * 256] = o[0] + o[1];
+#pragma unroll
+        for (int j = 0; j < 4; j++) S[j] = fmaf(kv[w][j], u, S[j]);
+        mine = r == e ? u : mine;
+      };
+      if (nt == TT) {
+#pragma unroll
+        for (int e = 0; e < TT; e++) {
+          fetch(e + 2 < TT ? t : next, (e + 2) % TT, (e + 2) & 3);
+          token(e, e & 3, vb[e / 4][e & 3], bb[e / 4][e & 3], DECAY == 2 ? gb[e / 4][e & 3] : 0.f);
+        }
+      } else {
+        for (int e = 0; e < nt; e++) {
+          fetch(t, e, 0);
+          token(e, 0, t.v[cl * TT + e], t.b[e], DECAY == 2 ? t.g[e] : 0.f);
+        }
+      }
+      if (r < TT) us[(i & 1) * CPB * TT + cl * TT + r] = mine;
+      __syncthreads();
+    }
+    if (steps > tiles) __syncthreads();
+    if (col)
+#pragma unroll
+      for (int j = 0; j < 4; j++) sp[j] = S[j];
+    return;
+  }
+
+  if (wave < 6) {
+    // a lane adds four lanes' parts, P / 4 lanes an output: the tree of group_sum, its first two steps inside the lane
+    constexpr int LO = P / 4, NP = TT * CPB * LO / 128;  // lanes an output; passes of two waves over a tile
+    const int lane = threadIdx.x & 63, sub = lane % LO;
+    auto outputs = [&](int i) {
+      const float* pp = parts + (i & 1) * F::PARTS;
+      const float* uc = us + (i & 1) * CPB * TT;
+      const float* kq = kqs + (i & 3) * TT;
+      float* op = a.out + (size_t)(t0 + i * TT) * a.ldo + h * vdim + blockIdx.x * CPB;
+      float o[NP], x[NP][4];
+#pragma unroll
+      for (int p = 0; p < NP; p++) quad(pp + ((p * 2 + wave - 4) * (64 / LO) + lane / LO) * P + sub * 4, x[p]);
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        float y = (x[p][0] + x[p][1]) + (x[p][2] + x[p][3]);
+        y += dpp_f32<0xB1>(y);
+        y += dpp_f32<0x4E>(y);
+        if (LO == 8) y += dpp_f32<0x141>(y);
+        o[p] = y;
+      }
+#pragma unroll
+      for (int p = 0; p < NP; p++) {
+        const int pair = (p * 2 + wave - 4) * (64 / LO) + lane / LO, e = pair / CPB, cl = pair % CPB;
+        if (sub == 0 && i * TT + e < n && blockIdx.x * CPB + cl < vdim) op[(size_t)e * a.ldo + cl] = fmaf(kq[e], uc[cl * TT + e], o[p]);
+      }
+    };
+    __syncthreads();
+    for (int i = 0; i < tiles; i++) {
+      if (i > 0) outputs(i - 1);
+      __syncthreads();
+    }
+    if (tiles > 0) outputs(tiles - 1);
+    if (steps > tiles) __syncthreads();
+    return;
+  }
+
+  // whole rows of 16-byte pieces (the launcher's condition) through buffer descriptors: what lies beyond the sequence's last row, or is no value of this
+  // thread, reads as 0 without a branch, so that the waits for a tile's rows count what was asked for after them
+  const int tid = threadIdx.x - 384, r = tid % P;
+  constexpr int NL = TT * P / 128, NV = (CPB * TT + 127) / 128;
+  typedef __amdgpu_buffer_rsrc_t rsrc;
+  auto rows_of = [&](const float* p, int ld, int cols, int i) {  // (no row left: a size of 0, as cols <= ld)
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p + ((size_t)t0 + (size_t)i * TT) * ld), 0, max(((min(n - i * TT, TT) - 1) * ld + cols) * 4, 0), 0x00020000u);
+  };
+  auto four = [](rsrc rs, int byte) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, byte, 0, 0)); };
+  auto one = [](rsrc rs, int byte) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, byte, 0, 0)); };
+  f32x4 kn[2][NL], qn[2][NL], dn[2][NL];
+  float vn[2][NV], bn[2], gn[2];
+  int ko[NL], qo[NL], dof[NL], vo[NV];
+#pragma unroll
+  for (int u = 0; u < NL; u++) {
+    const int row = (tid + u * 128) / P;
+    ko[u] = (row * a.ldk + r * 4) * 4, qo[u] = (row * a.ldq + r * 4) * 4, dof[u] = (row * a.ldd + r * 4) * 4;
+  }
+#pragma unroll
+  for (int u = 0; u < NV; u++) {
+    const int e = tid + u * 128, cc = blockIdx.x * CPB + e % CPB;
+    vo[u] = e < CPB * TT && cc < vdim ? (e / CPB * a.ldv + cc) * 4 : 0x7ffffff0;
+  }
+  const int bo = tid < TT ? tid * a.ldb * 4 : 0x7ffffff0, go = tid < TT ? tid * a.ldd * 4 : 0x7ffffff0;
+  auto request = [&](int i, int w) {
+    const rsrc kb = rows_of(a.k + hq * dimP, a.ldk, dimP, i), qb = rows_of(a.q + hq * dimP, a.ldq, dimP, i);
+    const rsrc vb = rows_of(a.v + h * vdim, a.ldv, vdim, i), bb = rows_of(a.beta + h, a.ldb, 1, i);
+    const rsrc db = rows_of(a.decay + (DECAY == 1 ? h * dimP : h), a.ldd, DECAY == 1 ? dimP : 1, i);
+#pragma unroll
+    for (int u = 0; u < NL; u++) {
+      kn[w][u] = four(kb, ko[u]), qn[w][u] = four(qb, qo[u]);
+      if (DECAY == 1) dn[w][u] = four(db, dof[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < NV; u++) vn[w][u] = one(vb, vo[u]);
+    bn[w] = one(bb, bo);
+    if (DECAY == 2) gn[w] = one(db, go);
+  };
+  auto deposit = [&](int i, int w) {
+    const Tile t = tile(i);
+#pragma unroll
+    for (int u = 0; u < NL; u++) {
+      const int e = tid + u * 128;
+      const f32x4 q = qn[w][u] * a.q_scale, k = kn[w][u];
+      *(f32x4*)(t.k + e * 4) = k;
+      *(f32x4*)(t.q + e * 4) = q;
+      if (DECAY == 1) *(f32x4*)(t.d + e * 4) = dn[w][u];
+      const float kq = group_sum<P>(fmaf(k.x, q.x, fmaf(k.y, q.y, fmaf(k.z, q.z, k.w * q.w))));
+      if (r == 0) kqs[(i & 3) * TT + e / P] = kq;
+    }
+#pragma unroll
+    for (int u = 0; u < NV; u++) {
+      const int e = tid + u * 128;
+      if (e < CPB * TT) t.v[e % CPB * TT + e / CPB] = vn[w][u];
+    }
+    if (tid < TT) {
+      t.b[tid] = bn[w];
+      if (DECAY == 2) t.g[tid] = gn[w];
+    }
+  };
+  request(0, 0);
+  request(1, 1);
+  deposit(0, 0);
+  request(2, 0);
+  deposit(1, 1);
+  request(3, 1);
+  __syncthreads();
+  auto step = [&](int i, int w) {  // beside the chain's tile i: tile i + 2 goes to LDS, tile i + 4 is asked for
+    deposit(i + 2, w);
+    request(i + 4, w);
+    __syncthreads();
+  };
+  for (int i = 0; i < steps; i += 2) {
+    step(i, 0);
+    step(i + 1, 1);
+  }
 }
 
 // ------------------------------------------------------------------------------------------------ per-head output norm and gate
@@ -1281,6 +1498,13 @@ ScanForm scan_form(const StkScanArgs& a) {
   f.TT = few || f.P == 1 || f.P == 64 ? 16 : 32;  // (one lane a column: the values and outputs of 32 tokens would take 64 KB of LDS)
   return f;
 }
+// floats of LDS of the form in three groups (0: not that form): prompts of the delta rule with 64 or 128 key channels, whole 16-byte rows and few columns
+size_t pair_floats(const StkScanArgs& a, const ScanForm& f) {
+  auto al16 = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+  if (!a.cu_q || (a.max_q > 0 && a.max_q <= 16) || !a.beta || !a.decay || f.R != 4 || (f.P != 16 && f.P != 32) || a.dim != 4 * f.P) return 0;
+  if (a.ldk % 4 || a.ldq % 4 || !al16(a.k) || !al16(a.q) || (!a.decay_per_head && (a.ldd % 4 || !al16(a.decay)))) return 0;
+  return f.P == 16 ? PairForm<16>::FLOATS : PairForm<32>::FLOATS;
+}
 size_t scan_lds_bytes(const ScanForm& f) {
   return ((size_t)f.TT * f.P * f.R * 3 + (size_t)2 * f.TT * (256 / f.P) + 3 * f.TT) * sizeof(float);
 }
@@ -1290,7 +1514,10 @@ extern "C" int32_t vra_stack_op_linear_scan_lds(int32_t dim, int32_t vdim, int32
   static const uint32_t ragged[2] = {};
   StkScanArgs a;
   a.dim = dim, a.vdim = vdim, a.H = H, a.B = B, a.max_q = max_q, a.cu_q = max_q == 1 ? nullptr : ragged;
-  return (int32_t)scan_lds_bytes(scan_form(a));
+  const ScanForm f = scan_form(a);
+  float decay, beta;  // (the delta rule where its form in groups asks for more)
+  a.decay = &decay, a.beta = &beta, a.decay_per_head = 1;
+  return (int32_t)std::max(scan_lds_bytes(f), pair_floats(a, f) * sizeof(float));
 }
 void vra_stack_linear_scan(const StkScanArgs& a, int64_t stream) {
   VRA_CHECK_ARG(a.q && a.k && a.v && a.state && a.state_slots && a.positions && a.out && (a.decay || a.head_decay), "stack linear scan: null pointer");
@@ -1305,6 +1532,18 @@ void vra_stack_linear_scan(const StkScanArgs& a, int64_t stream) {
   VRA_CHECK_ARG(!a.act_silu || (!decay && !beta), "stack linear scan: the activation on the way in goes with constant decays");
   VRA_CHECK_ARG(!a.bonus || (decay && !per_head && !beta), "stack linear scan: the bonus goes with per-row decays per channel, without the delta rule");
   VRA_CHECK_ARG(!per_head || beta, "stack linear scan: one decay per head and token goes with the delta rule");
+  if (const size_t floats = pair_floats(a, f)) {
+    grid.x = (a.vdim + 256 / f.P - 1) / (256 / f.P);
+#define STK_PAIR(PV)                                                                                                                          \
+  launch_checked("stack linear scan (three groups)", [&] {                                                                                      \
+    if (per_head) stk_delta_pair_kernel<PV, 2><<<grid, 512, floats * sizeof(float), st>>>(a);                                                 \
+    else stk_delta_pair_kernel<PV, 1><<<grid, 512, floats * sizeof(float), st>>>(a);                                                          \
+  })
+    if (f.P == 16) STK_PAIR(16);
+    else STK_PAIR(32);
+#undef STK_PAIR
+    return;
+  }
 #define STK_SCAN(RV, PV, TV)                                                                                                       \
   launch_checked("stack linear scan", [&] {                                                                                        \
     if (a.bonus) stk_linear_scan_kernel<RV, PV, TV, 1, false, false, true><<<grid, 256, lds, st>>>(a);                             \
