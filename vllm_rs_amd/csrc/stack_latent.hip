@@ -201,6 +201,13 @@ __global__ __launch_bounds__(64 * NW) void stk_latent_prefill_kernel(StkAttnArgs
   }
 }
 
+// a barrier for what went through LDS by its own instructions: rows on their way from memory to LDS stay on their way (__syncthreads waits for them)
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // part: f32 [B][S][H][vdim] sums weighted by e^(score - m), then f32 [B][S][H][2] (m, sum of the weights)
 template <int DC, int VT>
 __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, float* part, int S, int nbuf) {
@@ -213,6 +220,9 @@ __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, f
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), rq = lane & 15, oct = lane >> 4;
   const int head = blockIdx.z * 16 + rq;
   const bool hv = head < H;
+  const uint32_t* bt = a.block_tables + (size_t)b * a.max_blocks;
+  // the first two tiles' pages where no window moves them, asked for beside the position
+  uint32_t page0 = bt[min(s * KT / a.BS, a.max_blocks - 1)], page1 = bt[min((s + S) * KT / a.BS, a.max_blocks - 1)];
   const int64_t p = a.positions[b];
   const int n_keys = __builtin_amdgcn_readfirstlane((int)min((int64_t)a.context_lens[b], p + 1));
   const int key_lo = __builtin_amdgcn_readfirstlane(a.window > 0 ? (int)max((int64_t)0, p - a.window + 1) : 0);
@@ -225,10 +235,9 @@ __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, f
     return;
   }
   const uint16_t* kc = (const uint16_t*)a.kc;
-  const uint32_t* bt = a.block_tables + (size_t)b * a.max_blocks;
   const int k_ld = a.k_ld;
-  auto request_tile = [&](int buf, int k0) {  // (the page size is a multiple of 64: a tile lies in one page)
-    const int64_t slot0 = (int64_t)bt[k0 / a.BS] * a.BS + k0 % a.BS;
+  auto request_tile = [&](int buf, int k0, uint32_t page) {  // (the page size is a multiple of 64: a tile lies in one page)
+    const int64_t slot0 = (int64_t)page * a.BS + k0 % a.BS;
     const uint16_t* base = kc + slot0 * k_ld;
     const int last = n_keys - 1 - k0;
 #pragma unroll
@@ -239,7 +248,6 @@ __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, f
       __builtin_amdgcn_global_load_lds((glb_void_ptr)(base + off), (lds_void_ptr)(smem + buf * TILEB + idx * 1024), 16, 0, 0);
     }
   };
-  request_tile(0, kt0);
   s16x8 qf[DC];
   {
     const uint16_t* q = (const uint16_t*)a.q + (size_t)b * a.ldq + (size_t)(hv ? head : 0) * dim;
@@ -253,6 +261,13 @@ __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, f
     }
   }
   const float sc = a.scale * (a.head_scale && hv ? a.head_scale[head] : 1.f);
+  // both buffers' tiles are under way from the start (what they depend on has arrived: no wait between them)
+  bool ahead = nbuf == 2 && kt0 + S * KT < n_keys;
+  if (kt0 != s * KT) page0 = bt[kt0 / a.BS], page1 = bt[min((kt0 + S * KT) / a.BS, a.max_blocks - 1)];
+  page0 = __builtin_amdgcn_readfirstlane(page0), page1 = __builtin_amdgcn_readfirstlane(page1);
+  asm volatile("" ::"v"(sc));
+  request_tile(0, kt0, page0);
+  if (ahead) request_tile(1, kt0 + S * KT, page1);
   const int ka = (wave * 16 + rq) * ROWB + (oct ^ lat_swz(rq)) * 16;
   const int vrow = oct * 4 + (rq >> 2);
   const int va = vrow * ROWB + (((rq & 3) >> 1) ^ lat_swz(vrow)) * 16 + (rq & 1) * 8;
@@ -262,9 +277,11 @@ __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, f
   float m = -INFINITY, l = 0.f;
   int buf = 0;
   for (; kt0 < n_keys; kt0 += S * KT) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (nbuf == 2 && kt0 + S * KT < n_keys) request_tile(buf ^ 1, kt0 + S * KT);
+    if (ahead) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL / 4) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (nbuf == 2 && !ahead && kt0 + S * KT < n_keys) request_tile(buf ^ 1, kt0 + S * KT, bt[(kt0 + S * KT) / a.BS]);
+    ahead = false;
     const unsigned char* tile = smem + buf * TILEB;
     f32x4 s0 = vra_zero_acc(), s1 = vra_zero_acc();
     s16x8 kf[2][2];
@@ -292,7 +309,7 @@ __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, f
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
     if (oct == 0) wm[wave][rq] = tmax;
-    __syncthreads();
+    lds_barrier();
     // (the tile holds at least one visible key: the maximum is finite)
     const float mn = fmaxf(m, fmaxf(fmaxf(wm[0][rq], wm[1][rq]), fmaxf(wm[2][rq], wm[3][rq])));
     const float corr = m > -INFINITY ? __expf(m - mn) : 0.f;
@@ -313,7 +330,7 @@ __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, f
       *(uint2*)(p_hi + at) = hi;
       *(uint2*)(p_lo + at) = lo;
     }
-    __syncthreads();
+    lds_barrier();
 #pragma unroll
     for (int t = 0; t < TW; t++) acc[t][0] *= corr, acc[t][1] *= corr, acc[t][2] *= corr, acc[t][3] *= corr;
     s16x8 pf[2][2];
@@ -343,7 +360,7 @@ __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, f
     VRA_MFMA_DRAIN();
     if (nbuf == 1 && kt0 + S * KT < n_keys) {
       __syncthreads();  // (everyone has read the tile)
-      request_tile(0, kt0 + S * KT);
+      request_tile(0, kt0 + S * KT, bt[(kt0 + S * KT) / a.BS]);
     }
     if (nbuf == 2) buf ^= 1;
   }
@@ -361,46 +378,40 @@ __global__ __launch_bounds__(256) void stk_latent_decode_kernel(StkAttnArgs a, f
   }
 }
 
-// joins the S parts of a (sequence, head): out = sum_s e^(m_s - M) o_s / (sum_s e^(m_s - M) l_s + e^(sink - M)) * sigmoid(gate); S <= 64
-__global__ __launch_bounds__(128) void stk_latent_decode_join_kernel(StkAttnArgs a, const float* part, int S) {
-  __shared__ float ws[64];
-  __shared__ float total;
-  const int b = blockIdx.x, h = blockIdx.y, H = a.H, vdim = a.vdim, tid = threadIdx.x;
+// joins the S parts of a (sequence, head): out = sum_s e^(m_s - M) o_s / (sum_s e^(m_s - M) l_s + e^(sink - M)) * sigmoid(gate); S <= 64.  A wave a
+// workgroup, 256 channels; the rows of 32 parts are asked for beside the maxima and sums that decide their weights (8 sequences of up to 3900 tokens, 16
+// heads of 512: 6.8 us with the rows behind the weights, eight at a time, 128 workgroups; 4.8 so)
+__global__ __launch_bounds__(64) void stk_latent_decode_join_kernel(StkAttnArgs a, const float* part, int S) {
+  const int b = blockIdx.x, h = blockIdx.y, H = a.H, vdim = a.vdim, lane = threadIdx.x, c = blockIdx.z * 256 + lane * 4;
   const float* ml = part + (size_t)gridDim.x * S * H * vdim;
-  if (tid < 64) {
-    const size_t at = (((size_t)b * S + (tid < S ? tid : 0)) * H + h) * 2;
-    const float ms = tid < S ? ml[at] : -INFINITY, ls = tid < S ? ml[at + 1] : 0.f;
-    const float sink = a.sink ? a.sink[h] : -INFINITY;
-    const float M = fmaxf(wave_max(ms), sink);
-    const float w = ms > -INFINITY ? __expf(ms - M) : 0.f;
-    ws[tid] = w;
-    const float L = wave_sum(w * ls) + (a.sink ? __expf(sink - M) : 0.f);
-    if (tid == 0) total = L > 0.f ? (a.gate ? sigmoidf_(a.gate[(size_t)b * a.gate_ld + h]) : 1.f) / L : 0.f;
-  }
-  __syncthreads();
-  const float inv = total;
-  uint16_t* out = (uint16_t*)a.out + ((size_t)b * H + h) * vdim;
-  for (int c = tid * 4; c < vdim; c += 512) {
-    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-    // eight parts' rows are requested together; a part without a key has weight 0 and an unwritten row: not read
-    for (int s0 = 0; s0 < S; s0 += 8) {
-      float4 v[8];
+  const size_t at = (((size_t)b * S + min(lane, S - 1)) * H + h) * 2;
+  const float ms = lane < S ? ml[at] : -INFINITY, ls = lane < S ? ml[at + 1] : 0.f;
+  const float sink = a.sink ? a.sink[h] : -INFINITY, gate = a.gate ? a.gate[(size_t)b * a.gate_ld + h] : 0.f;
+  const float* rows = part + ((size_t)b * S * H + h) * vdim + min(c, vdim - 4);
+  f32x4 v[32];
+  auto fetch = [&](int s0) {
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int s = s0 + u;
-        const bool in = s < S && ws[s < S ? s : 0] > 0.f;
-        v[u] = in ? *(const float4*)(part + (((size_t)b * S + s) * H + h) * vdim + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
+    for (int u = 0; u < 32; u++) v[u] = *(const f32x4*)(rows + (size_t)min(s0 + u, S - 1) * H * vdim);
+  };
+  fetch(0);
+  const float M = fmaxf(wave_max(ms), sink), w = ms > -INFINITY ? __expf(ms - M) : 0.f;
+  const float L = wave_sum(w * ls) + (a.sink ? __expf(sink - M) : 0.f);
+  const float inv = L > 0.f ? (a.gate ? sigmoidf_(gate) : 1.f) / L : 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < S; s0 += 32) {
+    if (s0 > 0) fetch(s0);
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const float w = s0 + u < S ? ws[s0 + u] : 0.f;
-        o.x = fmaf(w, v[u].x, o.x), o.y = fmaf(w, v[u].y, o.y), o.z = fmaf(w, v[u].z, o.z), o.w = fmaf(w, v[u].w, o.w);
-      }
+    for (int u = 0; u < 32; u++) {
+      // (a part without a key has weight 0 and an unwritten row: whatever it holds is not felt)
+      const float ws = s0 + u < S ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), (s0 + u) & 63)) : 0.f;
+      if (ws > 0.f)
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = fmaf(ws, v[u][e], o[e]);
     }
-    uint2 r;
-    r.x = BF16::pack2(o.x * inv, o.y * inv), r.y = BF16::pack2(o.z * inv, o.w * inv);
-    *(uint2*)(out + c) = r;
   }
+  uint2 r;
+  r.x = BF16::pack2(o[0] * inv, o[1] * inv), r.y = BF16::pack2(o[2] * inv, o[3] * inv);
+  if (c < vdim) *(uint2*)((uint16_t*)a.out + ((size_t)b * H + h) * vdim + c) = r;
 }
 
 // the shapes both forms take
@@ -443,7 +454,7 @@ bool vra_stack_latent_decode(const StkAttnArgs& a, int dtype, int64_t stream) {
   else if (a.dim <= 384) STK_LATD(12, 24);
   else STK_LATD(18, 32);
 #undef STK_LATD
-  launch_checked("stack latent attention (join)", [&] { stk_latent_decode_join_kernel<<<dim3(a.B, a.H), 128, 0, st>>>(a, a.scratch, a.splits); });
+  launch_checked("stack latent attention (join)", [&] { stk_latent_decode_join_kernel<<<dim3(a.B, a.H, (a.vdim + 255) / 256), 64, 0, st>>>(a, a.scratch, a.splits); });
   return true;
 }
 
