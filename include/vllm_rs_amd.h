@@ -659,7 +659,8 @@ void vra_stack_op_gemm(const void* a, int32_t lda, const void* w, int64_t w_grou
 void vra_stack_op_gemm_tile(int32_t tile, const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32,
                             int32_t M, int32_t N, int32_t K, const int32_t* tile_group, const int32_t* a_row, int32_t a_rows,
                             const int32_t* out_row, int32_t epi, float limit, int64_t stream);
-/* columns a workgroup of vra_stack_op_gemm takes at up to 32 rows in bf16 (pair: with the gated epilogue): 16 or 32, with the same sums */
+/* columns of vra_stack_op_gemm's tiles at up to 32 rows in bf16 (pair: with the gated epilogue): 16 or 32, with the same sums (up to 8 rows and 2048
+ * columns a tile of 16 is two workgroups) */
 int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t batch, int32_t pair);
 /* rows of the row space that a model gives `pairs` token-expert pairs over `experts` experts (tiles128: its products run on 128-row tiles) */
 int32_t vra_stack_op_expert_rows(int32_t pairs, int32_t experts, int32_t tiles128);

@@ -537,6 +537,80 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g)
   }
 }
 
+// Products of up to 8 rows over columns that sixteen a workgroup would leave on half of the chip or less: eight a workgroup, with the sums of the kernel
+// above to the bit.  A load's sixteen weight rows are the eight columns at an even K-step and at the odd one behind it, its sixteen activation rows the same
+// two steps of the eight rows: every lane loads, whole 128-byte lines, and half as many of either.  The first eight rows and columns of a tile
+// count: the even step as loaded, the odd one with the halves of the lanes' rows of sixteen traded.  What bounds it is what a CU pulls past L2 and the latency
+// of its rounds.  8 rows, us, sixteen columns / eight: 2048 columns, K = 2048 6.7 / 5.6, 5632 11.8 / 8.6, 8192 14.8 / 10.4 (one row 11.8 / 8.4); 1024
+// columns, K = 8192 14.4 / 9.9.  Beyond one workgroup a CU it gives nothing: 3072 columns, K = 2048 6.9 / 6.9; 4096, K = 4096 9.5 / 10.0, 14336 25.4 / 29.4.
+template <bool POST>
+__global__ __launch_bounds__(512) void stk_gemm_mfma_eight_kernel(StkGemmArgs g) {
+  constexpr int NW = 8, U = 2;  // steps of 64 a round, the next round's loads ahead of this one's MFMAs (without: 12.8 us at 2048 x 8192)
+  __shared__ float part[NW][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c8 = lane & 7, odd = (lane >> 3) & 1, oct = lane >> 4;
+  const uint16_t* A = (const uint16_t*)g.a + (int64_t)blockIdx.z * g.a_batch_stride;
+  const uint16_t* Wt = (const uint16_t*)g.w + (int64_t)blockIdx.z * g.w_batch_stride;
+  const int n_base = blockIdx.y * 8;
+  const int idx = c8 < g.M ? (g.a_row ? g.a_row[c8] : c8) : -1;
+  const bool wv = n_base + c8 < g.N;
+  const uint16_t* ap = A + (int64_t)(idx >= 0 ? idx : 0) * g.lda;
+  const uint16_t* wp = Wt + (int64_t)(wv ? n_base + c8 : 0) * g.K;
+  const int ksteps = (g.K + 31) / 32, per = (ksteps + NW - 1) / NW;
+  const int k_lo = wave * per * 32, k_hi = min(g.K, (wave + 1) * per * 32);
+  f32x4 acc = vra_zero_acc();
+  auto traded = [](u32x4 v) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = __builtin_amdgcn_mov_dpp((int)v[i], 0x128, 0xf, 0xf, true);  // row_ror:8
+    return __builtin_bit_cast(s16x8, v);
+  };
+  const u32x4 zero4 = {0u, 0u, 0u, 0u};
+  u32x4 af[2][U], wf[2][U];
+  auto ask = [&](int b, int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = k0 + u * 64 + odd * 32 + oct * 8, kc = k < k_hi ? k : 0;
+      wf[b][u] = *(const u32x4*)(wp + kc);
+      af[b][u] = *(const u32x4*)(ap + kc);
+    }
+  };
+  auto use = [&](int b, int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const bool kin = k0 + u * 64 + odd * 32 + oct * 8 < k_hi;
+      const u32x4 w4 = wv && kin ? wf[b][u] : zero4, a4 = idx >= 0 && kin ? af[b][u] : zero4;
+      BF16::mfma(acc, __builtin_bit_cast(s16x8, w4), __builtin_bit_cast(s16x8, a4));
+      BF16::mfma(acc, traded(w4), traded(a4));
+    }
+  };
+  if (k_lo < k_hi) ask(0, k_lo);
+  for (int k0 = k_lo; k0 < k_hi; k0 += U * 128) {
+    if (k0 + U * 64 < k_hi) ask(1, k0 + U * 64);
+    use(0, k0);
+    if (k0 + U * 64 >= k_hi) break;
+    if (k0 + U * 128 < k_hi) ask(0, k0 + U * 128);
+    use(1, k0 + U * 64);
+  }
+  VRA_MFMA_DRAIN();
+  // lane: activation row lane % 16, columns oct * 4 + j
+  if (oct < 2 && !odd)
+#pragma unroll
+    for (int j = 0; j < 4; j++) part[wave][c8 * 8 + oct * 4 + j] = acc[j];
+  __syncthreads();
+  const int e = threadIdx.x, row = e >> 3, n = n_base + (e & 7);  // one output element per thread
+  if (e >= 64 || row >= g.M || n >= g.N) return;
+  if (g.a_row && g.a_row[row] < 0) return;
+  const int orow = g.out_row ? g.out_row[row] : row;
+  if (orow < 0) return;
+  float v = part[0][e];
+#pragma unroll
+  for (int w = 1; w < NW; w++) v += part[w][e];
+  v = v * g.alpha + (g.bias ? g.bias[(int64_t)blockIdx.z * g.bias_batch_stride + n] : 0.f);
+  if (POST) v = plain_value(g, v);
+  const int64_t at = (int64_t)blockIdx.z * g.out_batch_stride + (int64_t)orow * g.ldo + n;
+  if (g.out_f32) ((float*)g.out)[at] = v;
+  else ((uint16_t*)g.out)[at] = BF16::from_f32(v);
+}
+
 // Epilogue of gemm_rows_kernel for these products: alpha, bias, FN, row scatter.  FN as a template parameter: with all functions in one epilogue
 // the kernel is 28 000 instructions long and a launch pays ~12 us for fetching what it jumps over (2048 x 2048 x 2048: 37 us, 24 so).
 // vec: rows of the output start on 16 bytes, a lane stores whole 16-byte pieces (bf16: after trading columns with its row's other
@@ -1458,7 +1532,11 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
     else if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false, true, NTV><<<grid, 512, 0, st>>>(g); });     \
     else launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false, false, NTV><<<grid, 512, 0, st>>>(g); });              \
   } while (0)
-      if (wide) STK_SMALL(2);
+      if (!wide && g.M <= 8 && (int64_t)((g.N + 7) / 8) * nb <= 256 && !g.a_scale && !g.tile_group) {
+        dim3 grid(1, (g.N + 7) / 8, nb);
+        if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_eight_kernel<true><<<grid, 512, 0, st>>>(g); });
+        else launch_checked("stack gemm", [&] { stk_gemm_mfma_eight_kernel<false><<<grid, 512, 0, st>>>(g); });
+      } else if (wide) STK_SMALL(2);
       else STK_SMALL(1);
 #undef STK_SMALL
     }
