@@ -325,6 +325,30 @@ def test_scores_that_rise_by_little_and_by_much(form):
         assert np.abs(high).max() < 1e-20
 
 
+@pytest.mark.parametrize("kr,rd,H", [(64, 16, 2), (192, 64, 5), (512, 64, 16)])
+@pytest.mark.parametrize("splits", [1, 3, 7, 40])
+def test_a_score_beyond_float32_is_not_hidden_by_the_join(kr, rd, H, splits):
+    """one key's score is larger than float32 holds: the part that holds it has no finite sum, and the row that is joined from the parts says so; rows that
+    do not see the key are as ever (parts without a key, more than 32 parts among them)"""
+    L = _lib.load()
+    r = np.random.default_rng(kr + splits)
+    Tk, j = 700, 333
+    rows = po.bf16_round((0.1 * r.standard_normal((Tk, kr + rd))).astype(np.float32))
+    positions = np.array([0, 64, j - 1, j, j + 1, j + 99, j + 100, 699], np.int64)
+    q = po.bf16_round(r.standard_normal((len(positions), H, kr + rd)).astype(np.float32))
+    q[:, :, kr + 3] = 4.0
+    rows[:, kr + 3] = 0.0
+    gate = r.standard_normal((len(positions), H)).astype(np.float32)
+    for window in (0, 100):
+        ref = latent_reference(q, positions, rows, kr, 1.0, window, gate)
+        over = rows.copy()
+        over[j, kr + 3] = 3e38
+        sees = (positions >= j) & ((positions < j + window) if window else True)
+        got = run_latent(L, q, positions, over, kr, 1.0, window, gate, BF16, "parts", r, splits=splits)
+        assert np.isnan(got[sees]).all(), window
+        assert rel(got[~sees], ref[~sees]) < 4e-3, window
+
+
 def test_prompt_rows_do_not_depend_on_their_neighbours():
     """one query row alone, in a short portion and in a step that fills the chip (another workgroup size): the same bits"""
     L = _lib.load()

@@ -402,9 +402,10 @@ __global__ __launch_bounds__(64) void stk_latent_decode_join_kernel(StkAttnArgs 
     if (s0 > 0) fetch(s0);
 #pragma unroll
     for (int u = 0; u < 32; u++) {
-      // (a part without a key has weight 0 and an unwritten row: whatever it holds is not felt)
+      // (a part without a key has weight 0 and an unwritten row: whatever it holds is not felt.  A score beyond float32 leaves its part a weight that
+      // is no number, which passes on to the row)
       const float ws = s0 + u < S ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), (s0 + u) & 63)) : 0.f;
-      if (ws > 0.f)
+      if (ws != 0.f)
 #pragma unroll
         for (int e = 0; e < 4; e++) o[e] = fmaf(ws, v[u][e], o[e]);
     }
