@@ -922,6 +922,18 @@ def test_argument_errors_are_reported():
     L.vra_clear_error()
 
 
+def test_a_refused_host_allocation_leaves_no_error_for_the_next_launch():
+    """results fall back to ordinary arrays where no pinned memory is to be had: the step that follows, whose launches are checked, runs as ever"""
+    L = ops.lib()
+    L.vra_clear_error()
+    assert not L.vra_malloc_host(1 << 60) and b"hipHostMalloc" in L.vra_last_error()
+    L.vra_clear_error()
+    a, w, out = ops.dev(np.full((1, 32), 0x3F80, np.uint16)), ops.dev(np.full((16, 32), 0x3F80, np.uint16)), ops.DevBuf(16 * 4)  # (ones in bf16)
+    L.vra_stack_op_gemm(a.ptr, 32, w.ptr, 0, out.ptr, 16, 1, 1, 16, 32, 1.0, None, 0, None, None, None, 0, 0.0, BF16, 0)
+    ops.check_error()
+    assert (out.numpy(np.float32, (16,)) == 32.0).all()
+
+
 def test_rccl_all_reduce_single_rank():
     """ncclGetUniqueId -> ncclCommInitRank -> ncclAllReduce at world size 1: a REAL one-rank RCCL communicator (no dummy
     object), all-reduce(sum) in the storage dtype, in place and out of place (identity at one rank).  The two-rank product

@@ -21,8 +21,10 @@ extern "C" void vra_clear_error(void) { g_err[0] = 0; }
 extern "C" int32_t vra_take_device_error(void) { return vra_scratch_take_error(); }
 extern "C" const char* vra_version(void) { return "vllm_rs_amd 0.1.0 (gfx950, hip)"; }
 
+// (the runtime's own last error goes with the report: a caller may do without the call, and the next checked launch must not find it)
 static int hip_ok(hipError_t e, const char* what) {
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     vra_set_error("%s: %s", what, hipGetErrorString(e));
     return -1;
   }
