@@ -216,6 +216,9 @@ void vra_rope_cache_prefill(void* q, const void* k, const void* v, void* k_cache
                             const int64_t* slot_mapping, int32_t tokens, int32_t q_heads, int32_t kv_heads,
                             int32_t head_dim, int32_t block_size, int32_t dtype, int32_t kv_dtype,
                             int64_t stream);
+/* workgroups that launch divides a group of 8 tokens' heads over (0: a workgroup takes one token), and the bytes of LDS of one (may be null; at most 64 KB:
+ * the launch raises no limit) */
+int32_t vra_rope_cache_prefill_slices(int32_t tokens, int32_t kv_heads, int32_t head_dim, int32_t block_size, int32_t kv_dtype, int32_t* lds_bytes);
 /* decode half of PagedAttention::forward: one query token per sequence.
  * q/out [B,Hq,D]; block_tables [B,max_blocks] u32 (right-padded with 0, Appendix A5);
  * context_lens [B] u32 (includes the token just written). `workspace` must hold

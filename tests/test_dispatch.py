@@ -1,4 +1,5 @@
 """Which kernel a shape runs on, where that is decided without a GPU (vra_wna16_kernel)."""
+import ctypes
 import os
 import subprocess
 import sys
@@ -29,6 +30,20 @@ def test_linear_recurrence_stays_within_the_default_lds():
     lds = _lib.load().vra_stack_op_linear_scan_lds
     assert max(lds(dim, dim, 16, B, n) for dim in range(1, 257) for B in (1, 64) for n in (0, 1, 5, 100)) <= 64 * 1024
     assert lds(0, 1, 1, 1, 0) < 0 and lds(257, 1, 1, 1, 0) < 0
+
+
+def test_rotary_and_cache_store_stay_within_the_default_lds():
+    """as above: what is staged for a group of 8 tokens and what the kernel keeps beside it; prompts of many tokens and heads are still taken in groups"""
+    plan, lds = _lib.load().vra_rope_cache_prefill_slices, ctypes.c_int32()
+    for kv_heads in (1, 3, 8, 12, 16, 24, 31, 32, 33, 40, 64, 128):
+        for dim in (64, 80, 128, 256):
+            for tokens in (100, 256, 700, 1024, 2100, 4096, 8184, 8185, 8192, 30000):
+                for kv_dtype in (0, 3):
+                    slices = plan(tokens, kv_heads, dim, 64, kv_dtype, ctypes.addressof(lds))
+                    assert 0 <= slices <= kv_heads and lds.value <= 64 * 1024, (kv_heads, dim, tokens, kv_dtype, slices, lds.value)
+                    assert (slices > 0) == (tokens >= 1024 or tokens >= 256 and tokens * kv_heads * dim >= 384 << 10)
+                    assert plan(tokens, kv_heads, dim, 20, kv_dtype, None) == 0  # (pages off 8 tokens)
+    assert [plan(n, 8, 128, 64, 0, None) for n in (1200, 1500, 3000, 8192)] == [7, 6, 3, 1]
 
 
 @pytest.mark.parametrize("dim", [4, 32, 64, 128, 256])

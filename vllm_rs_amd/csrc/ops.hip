@@ -455,6 +455,7 @@ extern "C" void vra_reshape_and_cache(const void* k, const void* v, void* k_cach
 // positions and slots run together) write the token-minor V cache with ONE 16-byte (FP8: 8-byte) store per channel instead of
 // 8 two-byte stores 128 bytes apart — the scattered stores were 3/4 of this kernel's time at 4096 tokens.  Groups that are not
 // (chunk edges, block edges that are not multiples of 8, padded lanes) take the per-token stores.  Same bytes either way.
+constexpr size_t kRopeSlotBytes = 2 * 8 * sizeof(int64_t);  // a group's positions and slots in LDS, beside what is staged
 template <class DT, bool KV8, int TG>
 __global__ __launch_bounds__(256) void rope_cache_kernel(uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                                          typename KVT<KV8>::elem* __restrict__ kc, typename KVT<KV8>::elem* __restrict__ vc,
@@ -464,6 +465,7 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(uint16_t* __restrict__ 
   typedef typename KVT<KV8>::elem kv_t;
   extern __shared__ __attribute__((aligned(16))) unsigned char rc_smem[];  // TG == 8: the group's V rows [8][Hkv*D] in cache format
   __shared__ int64_t ps[TG], ss[TG];
+  static_assert(TG != 8 || sizeof(ps) + sizeof(ss) == kRopeSlotBytes, "what the launcher counts beside the staging");
   const int tid = threadIdx.x;
   const int t0 = blockIdx.x * TG, nt = min(TG, T - t0);
   const int half = D >> 1, per_head = half >> 3;  // 16-byte pair groups per head
@@ -564,6 +566,27 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(uint16_t* __restrict__ 
     }
   }
 }
+// Groups of 8 tokens (vector V stores) when there are enough values to fill the chip that way; the heads are divided over grid.y until there are four
+// workgroups a CU and a workgroup's share fits in 64 KB of LDS (the launch raises no limit).  us, groups of 8 / single tokens: 32 + 8 heads of 128, 512 tokens 5.8 / 7.1, 256 5.0 / 5.0;
+// 28 + 4 heads of 128, 768 tokens 6.6 / 6.7, 512 5.6 / 5.5; 32 + 4 heads of 64, 768 tokens 5.3 / 4.9, 1024 5.5 / 6.  With all heads and the tokens of a
+// group one after the other in one workgroup: 1024 tokens 13..16, 2120 tokens of 28 + 4 heads of 128 17.6 (now 9.7), 8192 of 32 + 8 40.6 (39.7).
+struct RopeGroups {
+  int slices;     // of the heads, over grid.y; 0: single tokens
+  size_t staged;  // bytes of dynamic LDS
+};
+static RopeGroups rope_groups(int tokens, int kv_heads, int head_dim, int block_size, bool kv8) {
+  if (block_size % 8 != 0 || !(tokens >= 1024 || (tokens >= 256 && (int64_t)tokens * kv_heads * head_dim >= 384 << 10))) return {0, 0};
+  const int groups = (tokens + 7) / 8;
+  int ny = std::max(1, std::min(kv_heads, (1024 + groups - 1) / groups));
+  auto staged = [&] { return (size_t)8 * ((kv_heads + ny - 1) / ny) * head_dim * (kv8 ? 1 : 2); };
+  while (ny < kv_heads && staged() + kRopeSlotBytes > 64 * 1024) ny++;  // (one head of 256 channels is 4 KB)
+  return {ny, staged()};
+}
+extern "C" int32_t vra_rope_cache_prefill_slices(int32_t tokens, int32_t kv_heads, int32_t head_dim, int32_t block_size, int32_t kv_dtype, int32_t* lds_bytes) {
+  const RopeGroups g = rope_groups(tokens, kv_heads, head_dim, block_size, kv_dtype == VRA_FP8_E4M3);
+  if (lds_bytes) *lds_bytes = (int32_t)(g.staged + (g.slices ? kRopeSlotBytes : 0));
+  return g.slices;
+}
 extern "C" void vra_rope_cache_prefill(void* q, const void* k, const void* v, void* k_cache, void* v_cache, const void* cos, const void* sin,
                                        const int64_t* positions, const int64_t* slot_mapping, int32_t tokens, int32_t q_heads, int32_t kv_heads,
                                        int32_t head_dim, int32_t block_size, int32_t dtype, int32_t kv_dtype, int64_t stream) {
@@ -574,20 +597,13 @@ extern "C" void vra_rope_cache_prefill(void* q, const void* k, const void* v, vo
   if (tokens <= 0) return;
   hipStream_t st = as_stream(stream);
   const bool kv8 = kv_dtype == VRA_FP8_E4M3;
-  // Groups of 8 tokens (vector V stores) when there are enough values to fill the chip that way and the staging fits in LDS; the heads are divided
-  // over grid.y until there are four workgroups a CU.  us, groups of 8 / single tokens: 32 + 8 heads of 128, 512 tokens 5.8 / 7.1, 256 5.0 / 5.0;
-  // 28 + 4 heads of 128, 768 tokens 6.6 / 6.7, 512 5.6 / 5.5; 32 + 4 heads of 64, 768 tokens 5.3 / 4.9, 1024 5.5 / 6.  With all heads and the tokens of a
-  // group one after the other in one workgroup: 1024 tokens 13..16, 2120 tokens of 28 + 4 heads of 128 17.6 (now 9.7), 8192 of 32 + 8 40.6 (39.7).
-  const int groups = (tokens + 7) / 8, ny = std::max(1, std::min(kv_heads, (1024 + groups - 1) / groups));
-  const size_t lds8 = (size_t)8 * ((kv_heads + ny - 1) / ny) * head_dim * (kv8 ? 1 : 2);
-  const bool g8 = (tokens >= 1024 || (tokens >= 256 && (int64_t)tokens * kv_heads * head_dim >= 384 << 10)) && lds8 <= 64 * 1024 && block_size % 8 == 0;
+  const RopeGroups g = rope_groups(tokens, kv_heads, head_dim, block_size, kv8);
 #define VRA_RC(DT, K8)                                                                                                                    \
   do {                                                                                                                                    \
-    if (g8)                                                                                                                               \
-      rope_cache_kernel<DT, K8, 8><<<dim3(groups, ny), 256, lds8, st>>>((uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,             \
-                                                                        (typename KVT<K8>::elem*)k_cache, (typename KVT<K8>::elem*)v_cache, \
-                                                                        (const uint16_t*)cos, (const uint16_t*)sin, positions, slot_mapping, \
-                                                                        tokens, q_heads, kv_heads, head_dim, block_size);                  \
+    if (g.slices)                                                                                                                         \
+      rope_cache_kernel<DT, K8, 8><<<dim3((tokens + 7) / 8, g.slices), 256, g.staged, st>>>(                                               \
+          (uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (typename KVT<K8>::elem*)k_cache, (typename KVT<K8>::elem*)v_cache,         \
+          (const uint16_t*)cos, (const uint16_t*)sin, positions, slot_mapping, tokens, q_heads, kv_heads, head_dim, block_size);            \
     else                                                                                                                                  \
       rope_cache_kernel<DT, K8, 1><<<tokens, 256, 0, st>>>((uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v,                           \
                                                            (typename KVT<K8>::elem*)k_cache, (typename KVT<K8>::elem*)v_cache,              \
