@@ -629,14 +629,8 @@ def test_fused_rope(interleaved, table_f32, D, rot):
     assert np.array_equal(kd.numpy(np.uint16, k.shape), kr)
 
 
-@pytest.mark.parametrize("dt", [BF16, F16])
-@pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("Hq,Hkv,D,T", [(32, 8, 128, 37), (14, 2, 64, 37), (32, 8, 128, 1100), (8, 2, 64, 1029)])
-def test_rope_cache_prefill_equals_the_two_launches(dt, fp8, Hq, Hkv, D, T):
-    """vra_rope_cache_prefill == vra_fused_rope + vra_reshape_and_cache bit for bit: rotated q, K-cache rows, V-cache columns
-    (16-bit and FP8 caches), a padded token (slot -1) writes nothing.  T >= 1024: workgroups take 8 tokens and write V with one
-    vector store per channel where the 8 slots are consecutive and aligned inside a block — runs of consecutive slots through
-    shuffled blocks, a run that starts mid-block at an odd offset, a hole, and a ragged last group"""
+def rope_cache_against_two_launches(dt, fp8, Hq, Hkv, D, T, runs):
+    """runs: slots in runs through shuffled blocks, else shuffled one by one"""
     L = ops.lib()
     BS = 64
     NB = max(8, (T + BS - 1) // BS + 3)
@@ -645,7 +639,7 @@ def test_rope_cache_prefill_equals_the_two_launches(dt, fp8, Hq, Hkv, D, T):
     cos_t, sin_t = orc.to_dt(cos, dt), orc.to_dt(sin, dt)
     q, k, v = rand_dt(r, (T, Hq, D), dt), rand_dt(r, (T, Hkv, D), dt), rand_dt(r, (T, Hkv, D), dt)
     pos = r.integers(0, 512, size=T).astype(np.int64)
-    if T < 1024:
+    if not runs:
         slots = r.permutation(NB * BS)[:T].astype(np.int64)
     else:  # two "sequences": one from the start of its blocks, one that continues 13 tokens into a block
         blocks = r.permutation(NB)
@@ -675,12 +669,28 @@ def test_rope_cache_prefill_equals_the_two_launches(dt, fp8, Hq, Hkv, D, T):
     assert np.array_equal(k2.numpy(np.uint16, k.shape), k), "k itself is left un-rotated"
 
 
+@pytest.mark.parametrize("dt", [BF16, F16])
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("Hq,Hkv,D,T", [(28, 4, 128, 800), (9, 3, 64, 1100), (8, 1, 128, 1030), (32, 8, 128, 391), (24, 24, 64, 1024)])
+@pytest.mark.parametrize("Hq,Hkv,D,T", [(32, 8, 128, 37), (14, 2, 64, 37), (32, 8, 128, 1100), (8, 2, 64, 1029)])
+def test_rope_cache_prefill_equals_the_two_launches(dt, fp8, Hq, Hkv, D, T):
+    """vra_rope_cache_prefill == vra_fused_rope + vra_reshape_and_cache bit for bit: rotated q, K-cache rows, V-cache columns
+    (16-bit and FP8 caches), a padded token (slot -1) writes nothing.  T >= 1024: workgroups take 8 tokens and write V with one
+    vector store per channel where the 8 slots are consecutive and aligned inside a block — runs of consecutive slots through
+    shuffled blocks, a run that starts mid-block at an odd offset, a hole, and a ragged last group"""
+    rope_cache_against_two_launches(dt, fp8, Hq, Hkv, D, T, T >= 1024)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,D,T", [(28, 4, 128, 800), (9, 3, 64, 1100), (8, 1, 128, 1030), (32, 8, 128, 391), (24, 24, 64, 1024), (32, 8, 128, 1200),
+                                        (32, 8, 128, 1500), (32, 8, 128, 3000), (28, 4, 128, 2900), (33, 11, 64, 2051), (32, 32, 128, 8192)])
 def test_rope_cache_prefill_slices_of_heads(fp8, Hq, Hkv, D, T):
-    """heads divided over the grid's second dimension: slices of unequal size (3 heads over 8 workgroups' worth, one head), short steps of wide
-    models in groups of 8 tokens, a last group of 7 tokens"""
-    test_rope_cache_prefill_equals_the_two_launches(BF16, fp8, Hq, Hkv, D, T)
+    """heads divided over the grid's second dimension: a key/value head a slice, slices of equal and of unequal size (8 key/value heads over 7, 6 and 3
+    workgroups, 4 over 3, 11 over 4), short steps of wide models in groups of 8 tokens, more staging than one workgroup's LDS, last groups of 3 to 8
+    tokens"""
+    slices = ops.lib().vra_rope_cache_prefill_slices(T, Hkv, D, 64, 3 if fp8 else BF16, None)
+    assert slices == {(4, 800): 4, (3, 1100): 3, (1, 1030): 1, (8, 391): 8, (24, 1024): 8, (8, 1200): 7, (8, 1500): 6, (8, 3000): 3, (4, 2900): 3, (11, 2051): 4,
+                      (32, 8192): 1 if fp8 else 2}[Hkv, T]
+    rope_cache_against_two_launches(BF16, fp8, Hq, Hkv, D, T, True)
 
 
 # ---------------------------------------------------------------- paged KV + attention
