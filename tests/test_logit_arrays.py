@@ -80,3 +80,49 @@ def test_threads():
     [t.join() for t in threads]
     gc.collect()
     assert not bad and len(heap.blocks) <= 12 and pool.live == sum(len(b) for b in heap.blocks.values())
+
+
+def counted(pool):
+    pool.L.taken = 0
+    real = pool.L.vra_malloc_host
+
+    def take(n):
+        pool.L.taken += 1
+        return real(n)
+
+    pool.L.vra_malloc_host = take
+    return pool
+
+
+def test_repeated_large_results_are_pinned_once():
+    """a loop that holds the last result while the next one is made (two alive), and one that releases it first: results of more than KEEP are no more
+    pinned anew at every call than small ones, and no more than an eighth beyond their size is pinned for them"""
+    for rows in (3, 80, 262):
+        pool = counted(_PinnedPool(Heap()))
+        pool.LIVE, pool.KEEP = 1 << 25, 1 << 20
+        nbytes = rows * 8016 * 4
+        for _ in range(6):
+            pool.take((rows, 8016))
+        assert pool.L.taken == 1, rows
+        out = None
+        for _ in range(6):
+            out = pool.take((rows, 8016))
+        assert pool.L.taken <= 2 and all(len(b) <= max(nbytes * 9 // 8, 2 * nbytes if nbytes < 1 << 20 else 0, 1 << 17) for b in pool.L.blocks.values())
+        del out
+        assert pool.idle <= max(pool.KEEP, nbytes * 9 // 8) and len(pool.L.blocks) in (1, 2)
+
+
+def test_idle_memory_makes_room():
+    """memory that is idle does not stand in the way of a result that needs other memory, and a buffer that was given back is the last to go"""
+    pool = counted(_PinnedPool(Heap()))
+    pool.LIVE, pool.KEEP = 1 << 23, 1 << 22
+    small = [pool.take((1 << 18,)) for _ in range(6)]  # 1 MiB each
+    del small
+    gc.collect()
+    assert pool.idle == 1 << 22 and pool.live == 1 << 22
+    big = pool.take((7 << 18,))  # 7 MiB: three of the four idle ones go
+    assert pool.live == 1 << 23 and pool.idle == 1 << 20 and len(pool.L.blocks) == 2
+    del big
+    assert pool.idle == 7 << 20 and len(pool.L.blocks) == 1
+    pool.close()
+    assert not pool.L.blocks and pool.live == 0
