@@ -1,6 +1,6 @@
 """The decode attention of layer stacks with a key/value head's query heads together and the context in parts, against softmax attention in
-float64: part and tile edges (128 and 32 keys), one key, more keys than `splits` parts of 128, no key at all; 1..8 query heads a key/value head;
-head sizes of every template and between them; cap, temperature, block mask, window, sink, scale and gate per head; three launches on one scratch.
+float64: part and tile edges (128 and 16 keys), one key, more keys than `splits` parts of 128, no key at all, 32 parts; 1..8 query heads a key/value head;
+pages of 8 to 128 keys; head sizes of every template and between them; cap, temperature, block mask, window, sink, scale and gate per head; three launches on one scratch.
 
 The weights and sums are float32 and the stored row is bf16: 2^-9 of a value, 4e-3 of the rows' norm."""
 import math
@@ -13,7 +13,6 @@ from vllm_rs_amd import _lib, checkpoint
 
 pytestmark = pytest.mark.gpu
 
-BS = 64
 b16 = lambda x: (checkpoint.f32_to_bf16_bits(np.ascontiguousarray(x, np.float32)).astype(np.uint32) << 16).view(np.float32)
 
 
@@ -41,12 +40,9 @@ def reference(q, k, v, p, scale, softcap, coef, every, chunk, window, sink, hs, 
     return out
 
 
-@pytest.mark.parametrize("form", ["plain", "capped", "block", "window", "dressed"])
-@pytest.mark.parametrize("H,G,dim,vdim,splits", [(16, 4, 128, 128, 8), (8, 8, 64, 64, 8), (16, 2, 72, 40, 3), (4, 2, 256, 200, 2), (6, 2, 24, 136, 32), (8, 1, 128, 128, 1)])
-def test_decode_attention_in_parts(H, G, dim, vdim, splits, form):
+def decode_in_parts(H, G, dim, vdim, splits, form, lens, BS):
     L = _lib.load()
     r = np.random.default_rng(dim + vdim + splits)
-    lens = [1, 31, 32, 33, 127, 128, 129, 300, 1100, 0]
     B = len(lens)
     per = [max(1, (n + BS - 1) // BS) for n in lens]
     order = r.permutation(sum(per) + 2).astype(np.uint32)
@@ -92,3 +88,23 @@ def test_decode_attention_in_parts(H, G, dim, vdim, splits, form):
         ref = reference(q[i], ks[i], vs[i], int(pos[i]), scale, softcap, coef, every, chunk, window, sink, hs, gate[i] if gate is not None else None)
         for a in (got[0], got[3]):
             assert rel(a[i], ref) < 4e-3 if ref.any() else not a[i].any(), (lens[i], rel(a[i], ref))
+
+
+@pytest.mark.parametrize("form", ["plain", "capped", "block", "window", "dressed"])
+@pytest.mark.parametrize("H,G,dim,vdim,splits", [(16, 4, 128, 128, 8), (8, 8, 64, 64, 8), (16, 2, 72, 40, 3), (4, 2, 256, 200, 2), (6, 2, 24, 136, 32), (8, 1, 128, 128, 1)])
+def test_decode_attention_in_parts(H, G, dim, vdim, splits, form):
+    decode_in_parts(H, G, dim, vdim, splits, form, [1, 31, 32, 33, 127, 128, 129, 300, 1100, 0], 64)
+
+
+@pytest.mark.parametrize("form", ["plain", "capped", "dressed"])
+@pytest.mark.parametrize("H,G,dim,vdim", [(8, 4, 64, 64), (16, 4, 128, 128), (8, 2, 256, 256), (8, 1, 256, 200)])
+def test_long_contexts_fill_the_parts(H, G, dim, vdim, form):
+    """17 and 32 parts of 128 keys, 18 of 256: the upper half of the lanes that weigh the parts, all four rounds of their rows"""
+    decode_in_parts(H, G, dim, vdim, 32, form, [2049, 4096, 4500, 130], 64)
+
+
+@pytest.mark.parametrize("BS", [8, 24, 100, 128])
+@pytest.mark.parametrize("H,G,dim,vdim,splits,form", [(16, 4, 128, 128, 8, "plain"), (8, 8, 64, 64, 2, "block"), (16, 2, 72, 40, 3, "dressed"), (4, 2, 256, 200, 4, "window")])
+def test_pages_that_a_wave_crosses(H, G, dim, vdim, splits, form, BS):
+    """pages smaller than a wave's 16 keys or off them: lanes of one load lie in several pages, and the page asked for ahead is some lanes' only"""
+    decode_in_parts(H, G, dim, vdim, splits, form, [1, BS - 1, BS, BS + 1, 127, 129, 333, 1100, 0], BS)

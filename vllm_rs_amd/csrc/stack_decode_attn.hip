@@ -43,7 +43,7 @@ __global__ __launch_bounds__(64 * group_waves(R, OC)) void stk_attn_decode_group
   const int len = max(1, (span + 128 * a.splits - 1) / (128 * a.splits)) * 128, parts = max(1, (span + len - 1) / len);
   if (part >= parts) return;
   const int k0 = lo + part * len, k1 = min(n_keys, k0 + len);
-  const int dim = a.dim, vdim = a.vdim, kld = a.k_ld ? a.k_ld : a.G * dim, vld = a.v_ld ? a.v_ld : a.G * vdim;
+  const int dim = a.dim, vdim = a.vdim, kld = a.G * dim, vld = a.G * vdim;
   const u32x4 zero4 = {0u, 0u, 0u, 0u};
   const bool hv = rq < HR;
   s16x8 qf[DC];
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(64 * group_waves(R, OC)) void stk_attn_decode_group
       for (int u = 0; u < 8; u++) v[e][u] = o[e];
   }
   __syncthreads();
-  // a head's weights of its parts: wave w takes heads w, w + 8, ..; a lane a part (at most 32: both halves of the wave hold the same)
+  // a head's weights of its parts: wave w takes heads w, w + NW, ..; a lane a part (at most 32: both halves of the wave hold the same)
   for (int r = wave; r < HR; r += NW) {
     const int i = lane & 31;
     const float mi = i < parts ? pm[r][i] : -INFINITY, li = i < parts ? pl[r][i] : 0.f;
@@ -272,7 +272,8 @@ size_t vra_stack_decode_scratch(int parts, int max_seqs, int heads, int kv_heads
 bool vra_stack_decode_group(const StkAttnArgs& a, int dtype, int64_t stream) {
   auto al16 = [](const void* p) { return (uintptr_t)p % 16 == 0; };
   if (dtype != VRA_BF16 || a.maps != 1 || a.cu_q || !a.arrived || !a.scratch || a.splits < 1 || a.splits > STK_DEC_PARTS || a.B > 65535 || a.G > 65535) return false;
-  if (!group_shape(a.H, a.G, a.dim, a.vdim) || a.ldq % 8 || a.k_ld % 8 || a.v_ld % 8 || !al16(a.q) || !al16(a.kc) || !al16(a.vc)) return false;
+  if (a.k_ld || a.v_ld) return false;  // (cache rows apart: no model's heads have them)
+  if (!group_shape(a.H, a.G, a.dim, a.vdim) || a.ldq % 8 || !al16(a.q) || !al16(a.kc) || !al16(a.vc)) return false;
   if (vra_stack_decode_scratch(a.splits, a.B, a.H, a.G, a.dim, a.vdim) > a.scratch_bytes) return false;
   const dim3 grid(std::min<int64_t>(a.splits, ((int64_t)a.max_blocks * a.BS + 127) / 128), a.G, a.B);
   const int R = group_width(a.H / a.G), w = value_width(a.dim, a.vdim);
