@@ -569,7 +569,8 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(uint16_t* __restrict__ 
 // Groups of 8 tokens (vector V stores) when there are enough values to fill the chip that way; the heads are divided over grid.y until there are four
 // workgroups a CU and a workgroup's share fits in 64 KB of LDS (the launch raises no limit).  us, groups of 8 / single tokens: 32 + 8 heads of 128, 512 tokens 5.8 / 7.1, 256 5.0 / 5.0;
 // 28 + 4 heads of 128, 768 tokens 6.6 / 6.7, 512 5.6 / 5.5; 32 + 4 heads of 64, 768 tokens 5.3 / 4.9, 1024 5.5 / 6.  With all heads and the tokens of a
-// group one after the other in one workgroup: 1024 tokens 13..16, 2120 tokens of 28 + 4 heads of 128 17.6 (now 9.7), 8192 of 32 + 8 40.6 (39.7).
+// group one after the other in one workgroup: 1024 tokens 13..16, 2120 tokens of 28 + 4 heads of 128 17.6 (now 9.7), 8192 of 32 + 8 40.6 (39.7).  8192
+// tokens of 32 + 32 heads of 128: 108 in two slices, 121 with 65 KB in one; of 40 + 40: 158, single tokens 524.
 struct RopeGroups {
   int slices;     // of the heads, over grid.y; 0: single tokens
   size_t staged;  // bytes of dynamic LDS

@@ -978,6 +978,7 @@ __global__ __launch_bounds__(256) void stk_linear_scan_kernel(StkScanArgs a) {
 // part of S^T q), two, a tile behind, add the parts of S^T q and store the outputs, and two fetch the tiles to come.  Sums and bits are those of
 // stk_linear_scan_kernel.  What bounds it: the chain's 33 instructions a token (LDS, at 128 bytes a cycle, is half as long).  2048 tokens, 16 heads of
 // 128 x 128: 307 us with one group, 193 now (64 channels, 1000 tokens: 132, 88); with a second copy of the state for the outputs (LDS reads bound it) 219.
+// All in long runs: a process's first dozen launches, before the clock has risen, take 215..227.
 template <int P>
 struct PairForm {
   static constexpr int TT = 8, CPB = 256 / P, DIMP = 4 * P;        // tokens a tile, columns a workgroup
