@@ -1,0 +1,57 @@
+"""The 256 x 256 tile of the row-major prompt GEMM (csrc/gemm_rows.cuh): the bits of the 64 x 128 tile, which the other tests compare with the oracle."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tests.util import BF16, F16, rand_dt, rng
+from vllm_rs_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+# rows that end in the first or second 64 of either half of a tile and just behind it, columns that leave waves without any, K of one pair of steps and more
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("M", [33, 65, 129, 200, 256, 257, 530])
+@pytest.mark.parametrize("K", [128, 384, 1024])
+@pytest.mark.parametrize("form", ["plain", "bias f32", "residual", "segments", "pair"])
+def test_wide_tile(form, M, K, dt):
+    r = rng(M + K + dt)
+    pair, ns = form == "pair", {"segments": [272, 16, 528], "pair": [144] * 2}.get(form, [560])
+    x, ws = rand_dt(r, (M, K), dt), [rand_dt(r, (n, K), dt, 0.05) for n in ns]
+    bias = [rand_dt(r, (n,), dt, 0.2) if form in ("bias f32", "segments") else None for n in ns]
+    res, f32 = rand_dt(r, (M, ns[0]), dt) if form == "residual" else None, form == "bias f32"
+    xd, wd, bd = ops.dev(x), [ops.dev(w) for w in ws], [ops.dev(b) if b is not None else None for b in bias]
+    rd = ops.dev(res) if res is not None else None
+
+    def run(tile):
+        outs = [ops.DevBuf((M + 1) * n * 4).fill_bytes(0) for n in ns]
+        ptrs = [(C.c_void_p * len(ns))(*[b.ptr if b else None for b in bufs]) for bufs in (wd, bd, outs)]
+        ops.lib().vra_dense_gemm_tile(tile, xd.ptr, ptrs[0], ptrs[1], (C.c_int32 * len(ns))(*ns), len(ns), int(pair), rd.ptr if rd else None, ptrs[2],
+                                      int(f32), M, K, dt, 0)
+        ops.check_error()
+        return [o.numpy(np.float32 if f32 else np.uint16, (M + 1, n)) for o, n in zip(outs, ns)][:1 if pair else None]
+    one, wide = run(0x12), run(0x44)
+    assert all(g[:M].any() and not g[M].any() for g in wide)  # something in every tensor, nothing beyond the rows
+    assert all(np.array_equal(a, b) for a, b in zip(wide, one))
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 40, 128), (257, 300, 256), (400, 513, 384)])
+@pytest.mark.parametrize("scatter", [False, True])
+def test_wide_tile_of_a_layer_stack(M, N, K, scatter):
+    """f32 outputs off 16 bytes, rows scattered with holes"""
+    L = _lib.load()
+    r = rng(M + N)
+    xd, wd = ops.dev(rand_dt(r, (M, K), BF16)), ops.dev(rand_dt(r, (N, K), BF16, 0.05))
+    dst = np.arange(M - 1, -1, -1, dtype=np.int32)
+    dst[::3] = -1
+    dd = ops.dev(dst.view(np.uint32)) if scatter else None
+
+    def run(tile):
+        out = ops.DevBuf((M + 1) * N * 4).fill_bytes(0)
+        L.vra_stack_op_gemm_tile(tile, xd.ptr, K, wd.ptr, 0, out.ptr, N, 1, M, N, K, None, None, 0, dd.ptr if dd else None, 0, 0.0, 0)
+        ops.check_error()
+        return out.numpy(np.float32, (M + 1, N))
+    one, wide = run(0x12), run(0x44)
+    assert np.array_equal(wide, one) and wide[:M].any() and not wide[M].any()
+    assert not scatter or not wide[np.setdiff1d(np.arange(M), dst)].any()

@@ -6,6 +6,8 @@ For every v_mfma in the given .s files:
   (2) within the next 12 wait states nothing but an MFMA accumulating into the SAME destination may
       read or write the destination registers (the inline-asm form is invisible to hipcc's hazard
       recogniser, so the code places VRA_MFMA_DRAIN() = `s_nop 7; s_nop 4` itself).
+  (2b) its operands must not be written by a vector instruction within the two wait states before it (most of the
+      inline-asm forms carry an `s_nop 1`; DT::mfma_ready does not and is for operands that come from LDS).
 Exit status 1 if any violation is found (the Makefile fails the build).
 
 Also a performance lint (round 4): (3) no kernel may fetch KERNEL ARGUMENTS with vector loads.  A struct field selected under a
@@ -67,6 +69,18 @@ def check(path):
                 bad += 1
                 print(f"[overlap] {fn}: {t}", file=sys.stderr)
                 continue
+            back, ops = 0, A | B | regset(c)
+            for u in reversed(body[max(0, i - 3):i]):
+                mn = re.match(r"s_nop\s+(\d+)", u)
+                if back >= 2 or u.startswith(("s_cbranch", "s_branch", "s_barrier")):
+                    break
+                if u.startswith("v_") and not u.startswith(("v_mfma", "v_cmp", "v_readfirstlane", "v_readlane")):
+                    dst = [regset(x) for x in u.split(None, 1)[1].split(",")[:2 if "swap" in u else 1]]
+                    if set().union(*dst) & ops:
+                        bad += 1
+                        print(f"[operand written {back} states ahead] {fn}: {u}  ->  {t}", file=sys.stderr)
+                        break
+                back += int(mn.group(1)) + 1 if mn else 1
             waited = 0
             for u in body[i + 1:]:
                 if waited >= WAIT:

@@ -109,6 +109,9 @@ struct BF16 {
   static __device__ __forceinline__ void mfma(f32x4& acc, s16x8 a, s16x8 b) {  // acc += A·B
     asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
   }
+  static __device__ __forceinline__ void mfma_ready(f32x4& acc, s16x8 a, s16x8 b) {  // (A, B not written by VALU within two wait states)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+  }
   static __device__ __forceinline__ void mfma0(f32x4& acc, s16x8 a, s16x8 b) {  // acc = A·B (early clobber: D never on A/B)
     asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
   }
@@ -127,6 +130,9 @@ struct F16 {
   }
   static __device__ __forceinline__ void mfma(f32x4& acc, s16x8 a, s16x8 b) {  // acc += A·B
     asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+  }
+  static __device__ __forceinline__ void mfma_ready(f32x4& acc, s16x8 a, s16x8 b) {  // (A, B not written by VALU within two wait states)
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
   }
   static __device__ __forceinline__ void mfma0(f32x4& acc, s16x8 a, s16x8 b) {  // acc = A·B (early clobber: D never on A/B)
     asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));

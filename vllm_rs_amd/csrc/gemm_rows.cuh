@@ -1,22 +1,26 @@
 // gemm_rows.cuh — 16-bit GEMM of prompt steps on ROW-MAJOR weights: out[m, n] = epilogue( sum_k x[row(m), k] * w[n, k] ), f32 accumulation.
 //
-// Bound: what a CU can pull past L2, and how well that overlaps with the matrix work.  LDS-DMA alone (no LDS reads, no MFMAs) delivers ~28 B
-// per clock and CU on full 128-byte lines and ~21 on half lines where the panels come from past L2, whatever the depth of the ring or the row
-// stride (panels that stay in L2: 58..60, on either); a 128 x 128 tile needs 32 KiB per 512 clocks of MFMAs.  So: whole lines per request
-// (a DMA instruction fetches 8 rows x 128 bytes), the largest tiles the problem has enough of, and the DMA instructions spread between the MFMAs —
-// issued in one run they stall the wave in front of its LDS reads.  Measured (2048 x 2048 outputs, K = 8192, 256 tiles of 128 x 128): 87 us
-// with the requests in one run, 74 spread; without the MFMAs 67, and 47 with the weights in L2: requests and MFMAs do not overlap as well as they could.
+// Bound: 256 x 256 outputs a workgroup, the chip's power — the loop runs 2240 clocks a K step of 64 (its MFMAs are 2048), at a clock that
+// settles at 1.3..1.5 GHz (matrix instructions alone: 1.9); smaller tiles, what a CU gets past L2: 28..35 B per clock where lines come from
+// memory, whatever the number of buffers, the cache policy or a wave that touches lines ahead (requests in flight a CU are limited, and
+// a line that another CU has asked for costs as long).  A 128 x 128 tile needs 32 KiB per 512 clocks of MFMAs, 256 x 256 64 KiB per 2048.
 //
-// Tile: WM x WN waves, 64 x 64 outputs each (16 accumulator tiles of v_mfma_f32_16x16x32: weights = A, rows of x = B, so a lane holds 4
-// consecutive columns of one row).  K in steps of 64, ascending, one accumulation chain per output: the result of a row does not depend
-// on the tile, the row's place in it or the rows beside it, and is bit-equal to any other kernel that walks K in steps of 32 on this
-// instruction.
-// LDS ring of S stages; a stage holds 4 (WM + WN) blocks of 16 rows x 64 k (2 KiB): row r of a block at r * 128 bytes, its 16-byte chunk c in
-// slot c ^ (r & 7), which spreads a fragment read's lanes over all banks.  At the top of step ks the stages ks and ks + 1 have landed
-// and the first half of ks is in registers; the step reads its second half, runs the first half's MFMAs, reads the first half of ks + 1,
-// runs the second half's, requests stage ks + S - 1 into the buffer of ks - 1 (every wave is past its reads: the barrier at the end of
-// ks - 1) and waits until stage ks + 2 is complete before the barrier.
+// Two groups of four waves (a wave of each on every SIMD) run one barrier apart: while one group's MFMAs run, the other reads its operands of the
+// next phase from LDS and requests tiles.  A phase is a K step of 64 — with 256 rows two of them a step, the upper and the lower 64 rows of every wave —
+//   { LDS reads | requests | vmcnt: the next phase's tiles have landed, lgkmcnt: this phase's reads are done | barrier | MFMAs | barrier }
+// and requests go to the buffer that the phase before read: both groups' reads ended ahead of a barrier that the requesting wave has passed.
+// Fragments come from LDS only, so the MFMAs need no wait states between them (10 % of a group's phase).  Against one group in step with itself
+// (128 x 256: 8 waves and one touching lines; 128 x 128: 4 waves), us: 2048 x 8192, K = 2048: 84 -> 63 (256 x 256; 128 x 256 78); 2048 x 2048 x 2048
+// 25.5 -> 23.5 (128 x 128); 2048 x 2048, K = 8192: 82 -> 76; 2120 rows x 2048, K = 2048 / 5632: 35.9 -> 30.7 / 84.5 -> 78.6 (128 x 256).
+//
+// Weights = A, rows of x = B of v_mfma_f32_16x16x32, so a lane holds 4 consecutive columns of one row.  K ascending, one accumulation chain per
+// output: the result of a row does not depend on the tile, the row's place in it or the rows beside it, and is bit-equal to any other kernel
+// that walks K in steps of 32 on this instruction.
+// LDS: blocks of 16 rows x 64 k (2 KiB): row r of a block at r * 128 bytes, its 16-byte chunk c in slot c ^ (r & 7), which spreads a fragment
+// read's lanes over all banks; a request (LDS-DMA) fetches 8 rows x 128 bytes, whole lines.
 #pragma once
+#include <type_traits>
+
 #include "common.cuh"
 
 #define GR_MAX_SEG 3
@@ -30,7 +34,7 @@ struct GemmRowsArgs {
   int nseg = 1;
   int M = 0, K = 0;  // K % 64 == 0
   int MT = 0, NT = 0;  // tiles along m, and along n over all segments
-  // grouped rows: tile row t (BM rows) multiplies with w[0] + tile_group[t] * w_group_stride (elements); -1: an empty tile row
+  // grouped rows (not on 256-row tiles): tile row t (BM rows) multiplies with w[0] + tile_group[t] * w_group_stride (elements); -1: an empty tile row
   const int* tile_group = nullptr;
   int64_t w_group_stride = 0;
   int64_t x_batch_stride = 0, w_batch_stride = 0;  // elements between the operands of two products of a batch (grid y)
@@ -58,20 +62,41 @@ __device__ __forceinline__ void gr_gather_columns(u32x2 (&v)[2]) {
   }
 }
 
-static inline size_t gemm_rows_lds_bytes(int wm, int wn, int s) { return (size_t)s * 4 * (wm + wn) * 2048; }
+// tile of a workgroup: the ids of one XCD (id mod 8) take a contiguous run of an order that walks 8 tile rows before the next tile column, so the
+// workgroups of an XCD share their operands' panels in its L2
+__device__ __forceinline__ void gr_tile(const GemmRowsArgs& a, int& mt, int& nt) {
+  const int nwg = (int)gridDim.x, bid = (int)blockIdx.x, q = nwg >> 3, r = nwg & 7, xcd = bid & 7;
+  const int lin = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
+  constexpr int GM = 8;
+  const int per = GM * a.NT, grp = lin / per, rem = lin - grp * per, first = grp * GM, gsz = min(a.MT - first, GM);
+  mt = first + rem % gsz;
+  nt = rem / gsz;
+}
 
-// EPI::store(m, seg, n0, q4, acc): the wave's 64 columns n0 .. n0 + 63 (of segment seg) of output row m; the lane holds columns n0 + 16 j + 4 q4 ..
+// waves of a tile: two groups of four (rows 0 .. BM/2 - 1 and the others), CW of them side by side with 64 columns each
+template <int BM, int BN>
+struct GrTile {
+  static constexpr int H = BM == 256 ? 2 : 1;                           // phases of a K step (the upper, the lower rows of a wave)
+  static constexpr int S = BM == 256 ? 2 : (BM == 128 && BN == 128 ? 4 : 3);  // LDS buffers
+  static constexpr int CW = BN / 64, RW = 4 / CW;
+  static constexpr int NX = BM / 32 / RW / H;  // 16-row blocks of a wave in a phase
+  static constexpr int XB = BM / 16, WB = BN / 16, STG = (XB + WB) * 2048;
+  static constexpr int EX = BM / 64, EW = BN / 64;  // a wave's DMA instructions (8 rows of 128 bytes) a K step
+};
+
+// EPI::store(m, seg, n0, N, q4, acc): the wave's 64 columns n0 .. n0 + 63 (of segment seg) of output row m; the lane holds columns n0 + 16 j + 4 q4 ..
 // + 3 in acc[j].  Called by all lanes (lanes beyond the matrix with m = -1), so that a lane may trade columns with its row's other three.
 // PAIR: w[0] and w[1] (gate, up; neither grouped nor batched) interleaved in blocks of 16 virtual columns, n[0] = virtual columns.
-template <class DT, int WM, int WN, int S, bool SPREAD, bool PAIR, class EPI>
-__global__ __launch_bounds__(64 * WM * WN + (SPREAD ? 0 : 64)) void gemm_rows_kernel(const GemmRowsArgs a, const EPI epi) {
+template <class DT, int BM, int BN, bool PAIR, class EPI>
+__global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a, const EPI epi) {
 #ifdef __HIP_DEVICE_COMPILE__
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  constexpr int NW = WM * WN, XB = 4 * WM, NB = 4 * (WM + WN), PER = NB / NW, D = 2 * PER, STG = NB * 2048, PEND = (S - 3) * D;
-  static_assert(NB % NW == 0 && XB % NW == 0 && S >= 3 && (!PAIR || NW % 2 == 0), "block split");
+  using T = GrTile<BM, BN>;
+  constexpr int H = T::H, S = T::S, NX = T::NX, STG = T::STG, EX = T::EX, EW = T::EW, D = EX + EW;
+  static_assert(EW == 4 || EW == 2, "a wave has 64 columns");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave % WM, wn = wave / WM, r16 = lane & 15, q4 = lane >> 4;
+  const int wg = wave >> 2, cw = (wave & 3) % T::CW, rw = (wave & 3) / T::CW, r16 = lane & 15, q4 = lane >> 4;
   // tile: the ids of one XCD (id mod 8) take a contiguous run of an order that walks 8 tile rows before the next tile column, so the
   // workgroups of an XCD share their operands' panels in its L2
   int mt, nt;
@@ -84,7 +109,7 @@ __global__ __launch_bounds__(64 * WM * WN + (SPREAD ? 0 : 64)) void gemm_rows_ke
     nt = rem / gsz;
   }
   int group = 0;
-  if (a.tile_group) {
+  if (H == 1 && a.tile_group) {
     group = __builtin_amdgcn_readfirstlane(a.tile_group[mt]);
     if (group < 0) return;
   }
@@ -92,191 +117,197 @@ __global__ __launch_bounds__(64 * WM * WN + (SPREAD ? 0 : 64)) void gemm_rows_ke
   int seg = 0, N = a.n[0];
   const uint16_t* w = static_cast<const uint16_t*>(a.w[0]);
   if (!PAIR) {
-    if (a.nseg > 1 && nt >= (N + 64 * WN - 1) / (64 * WN)) nt -= (N + 64 * WN - 1) / (64 * WN), seg = 1, N = a.n[1], w = static_cast<const uint16_t*>(a.w[1]);
-    if (seg == 1 && a.nseg > 2 && nt >= (N + 64 * WN - 1) / (64 * WN)) nt -= (N + 64 * WN - 1) / (64 * WN), seg = 2, N = a.n[2], w = static_cast<const uint16_t*>(a.w[2]);
-  } else if (wave & 1) {
-    w = static_cast<const uint16_t*>(a.w[1]);  // (virtual block f: tensor f & 1; a wave requests the blocks wave + i * NW, all of one parity)
+    if (a.nseg > 1 && nt >= (N + BN - 1) / BN) nt -= (N + BN - 1) / BN, seg = 1, N = a.n[1], w = static_cast<const uint16_t*>(a.w[1]);
+    if (seg == 1 && a.nseg > 2 && nt >= (N + BN - 1) / BN) nt -= (N + BN - 1) / BN, seg = 2, N = a.n[2], w = static_cast<const uint16_t*>(a.w[2]);
   }
-  const int m0 = mt * 64 * WM, n0 = nt * 64 * WN, K = a.K, KT = K >> 6;
+  const int m0 = mt * BM, n0 = nt * BN, K = a.K, KT = K >> 6;
   const uint16_t* const x = static_cast<const uint16_t*>(a.x) + (int64_t)blockIdx.y * a.x_batch_stride;
   w += (int64_t)group * a.w_group_stride + (int64_t)blockIdx.y * a.w_batch_stride;
+  // (PAIR: virtual block f is of tensor f & 1.  A wave requests the blocks 2 wave and 2 wave + 1 of a 256-column tile, block wave of a 128-column one)
+  const uint16_t* const wlo = PAIR && EW == 2 && (wave & 1) ? static_cast<const uint16_t*>(a.w[1]) : w;
+  const uint16_t* const whi = PAIR && EW == 4 ? static_cast<const uint16_t*>(a.w[1]) : wlo;
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, 0x7FFFFFF0, 0x00020000u);
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(w), 0, 0x7FFFFFF0, 0x00020000u);
-  // DMA sources: lane p fetches row p >> 3 (and 8 + (p >> 3) with the second instruction of a block), the chunk that slot p & 7 holds
-  uint32_t vo[PER][2];
-  {
-    const int sr = lane >> 3, sc = (lane & 7) ^ (lane >> 3);
+  const __amdgpu_buffer_rsrc_t rlo = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wlo), 0, 0x7FFFFFF0, 0x00020000u);
+  const __amdgpu_buffer_rsrc_t rhi = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(whi), 0, 0x7FFFFFF0, 0x00020000u);
+  // DMA sources: lane p fetches row p >> 3 of an instruction's eight, the chunk that slot p & 7 holds
+  const int sr = lane >> 3, sc = (lane & 7) ^ sr;
+  auto xrow8 = [&](int e) {  // instruction e of this wave: eight rows from this one on (two phases: e = 0, 1 upper rows, 2, 3 lower rows)
+    return H == 2 ? (wave < 4 ? wave : wave + 4) * 16 + (e >> 1) * 64 + (e & 1) * 8 : (wave * EX + e) * 8;
+  };
+  uint32_t vx[EX], vw[EW];
 #pragma unroll
-    for (int i = 0; i < PER; i++)
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const int b = wave + i * NW;
-        int row;
-        uint32_t ld;
-        if (i * NW < XB) {
-          row = min(m0 + b * 16 + h * 8 + sr, a.M - 1);
-          if (a.x_row) row = max(a.x_row[row], 0);
-          ld = (uint32_t)a.x_ld;
-        } else if (PAIR) {
-          row = min(((n0 >> 4) + b - XB) / 2 * 16 + h * 8 + sr, (N >> 1) - 1);
-          ld = (uint32_t)K;
-        } else {
-          row = min(n0 + (b - XB) * 16 + h * 8 + sr, N - 1);
-          ld = (uint32_t)K;
-        }
-        vo[i][h] = ((uint32_t)row * ld + (uint32_t)sc * 8u) * 2u;
-      }
+  for (int e = 0; e < EX; e++) {
+    int row = min(m0 + xrow8(e) + sr, a.M - 1);
+    if (a.x_row) row = max(a.x_row[row], 0);
+    vx[e] = ((uint32_t)row * (uint32_t)a.x_ld + (uint32_t)sc * 8u) * 2u;
   }
-  if constexpr (!SPREAD) {
-    // One wave more, which computes nothing: it touches a line of K step ks + 8 for its share of the panels that the workgroups of an XCD
-    // have in common (8 tile rows x 4 tile columns at a time: a quarter of this tile's rows of x, an eighth of its columns of w), so that
-    // the ring's requests find them in L2.  With two stages in flight the ring alone does not cover the way to memory (2048 x 8192, K =
-    // 2048, weights not in any cache: 94 -> 82 us); the 128 x 128 tile's three stages do, and gain nothing.
-    if (wave == NW) {
-      constexpr int XL = 16 * WM, WL = 8 * WN;
-      static_assert(XL + WL <= 64, "a lane a line");
-      const bool isx = lane < XL;
-      const int xr = min(m0 + (nt & 3) * XL + lane, a.M - 1), wrow = (mt & 7) * WL + (lane - XL);
-      int nr = min(n0 + wrow, N - 1);
-      const uint16_t* wp = w;
-      if (PAIR) {  // (this wave's w is the gate tensor's)
-        const uint16_t* const up = static_cast<const uint16_t*>(a.w[1]);
-        nr = min((n0 >> 1) + (wrow >> 1), (N >> 1) - 1);
-        if (wrow & 1) wp = up;
-      }
-      const int xi = isx && a.x_row ? max(a.x_row[xr], 0) : xr;
-      const uint16_t* const p = isx ? x + (int64_t)xi * a.x_ld : wp + (int64_t)nr * K;
-      const bool live = lane < XL + WL;
-      uint32_t v[8] = {}, seen = 0;
 #pragma unroll
-      for (int u = 0; u < 8; u++)
-        if (live) v[u] = *reinterpret_cast<const uint32_t*>(p + min(u, KT - 1) * 64);
-      __builtin_amdgcn_s_barrier();
-      for (int ks = 0; ks < KT; ks += 8) {
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-          if (ks + u >= KT) break;  // (one barrier a step, as the other waves)
-          seen ^= v[u];
-          if (live) v[u] = *reinterpret_cast<const uint32_t*>(p + min(ks + u + 8, KT - 1) * 64);
-          __builtin_amdgcn_sched_barrier(0);
-          __builtin_amdgcn_s_barrier();
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) seen ^= v[u];
-      asm volatile("" ::"v"(seen));
-      return;
-    }
+  for (int e = 0; e < EW; e++) {
+    const int r8 = (wave * EW + e) * 8;  // (of a pair: block r8 / 16, half of the virtual columns' row in its tensor)
+    const int row = PAIR ? min((((n0 + r8) >> 4) >> 1) * 16 + (r8 & 15) + sr, (N >> 1) - 1) : min(n0 + r8 + sr, N - 1);
+    vw[e] = ((uint32_t)row * (uint32_t)K + (uint32_t)sc * 8u) * 2u;
   }
   typedef __attribute__((address_space(3))) void* lds_ptr;
-  auto request = [&](int ks, int e) {  // the e-th of the wave's D instructions for stage ks (beyond K: the last step again, never read)
+  // requests of K step ks (beyond K: the last step again, never read) into the buffer at byte `o`
+  auto stage_x = [&](int o, int ks, int e0, int e1) {
     const uint32_t so = (uint32_t)min(ks, KT - 1) * 128u;
-    const int i = e >> 1, h = e & 1;
-    unsigned char* const d = smem + (ks % S) * STG + (wave + i * NW) * 2048 + h * 1024;
-    if (i * NW < XB) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)d, 16, vo[i][h], so, 0, 0);
-    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)d, 16, vo[i][h], so, 0, 0);
+#pragma unroll
+    for (int e = e0; e < e1; e++) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(smem + o + xrow8(e) * 128), 16, vx[e], so, 0, 0);
   };
-  const int c0 = r16 * 128 + (q4 ^ (r16 & 7)) * 16, c1 = r16 * 128 + ((4 + q4) ^ (r16 & 7)) * 16;
-  const unsigned char* const xb = smem + wm * 4 * 2048;
-  const unsigned char* const wb = smem + (XB + wn * 4) * 2048;
-  s16x8 xa[2][4], wa[2][4];
-  auto read = [&](int half, int ks) {  // k half `half` of step ks
-    const int o = (ks % S) * STG + (half ? c1 : c0);
+  auto stage_w = [&](int o, int ks) {
+    const uint32_t so = (uint32_t)min(ks, KT - 1) * 128u;
 #pragma unroll
-    for (int j = 0; j < 4; j++) wa[half][j] = *reinterpret_cast<const s16x8*>(wb + o + j * 2048);
-#pragma unroll
-    for (int i = 0; i < 4; i++) xa[half][i] = *reinterpret_cast<const s16x8*>(xb + o + i * 2048);
+    for (int e = 0; e < EW; e++) {
+      unsigned char* const d = smem + o + T::XB * 2048 + (wave * EW + e) * 1024;
+      if (e < EW / 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rlo, (lds_ptr)d, 16, vw[e], so, 0, 0);
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(rhi, (lds_ptr)d, 16, vw[e], so, 0, 0);
+    }
   };
-  f32x4 acc[4][4];
+  const int row0 = wg * (BM / 2) + rw * (BM / 2 / T::RW);  // the wave's first row in the tile
+  const int c0 = r16 * 128 + (q4 ^ (r16 & 7)) * 16, c1 = c0 ^ 64;
+  const unsigned char* const xb = smem + row0 * 128;
+  const unsigned char* const wb = smem + T::XB * 2048 + cw * 4 * 2048;
+  s16x8 xa[NX][2], wa[4][2];
+  auto read_x = [&](int o, int h) {
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+    for (int i = 0; i < NX; i++) {
+      xa[i][0] = *reinterpret_cast<const s16x8*>(xb + o + c0 + (h * NX + i) * 2048);
+      xa[i][1] = *reinterpret_cast<const s16x8*>(xb + o + c1 + (h * NX + i) * 2048);
+    }
+  };
+  auto read_w = [&](int o) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      wa[j][0] = *reinterpret_cast<const s16x8*>(wb + o + c0 + j * 2048);
+      wa[j][1] = *reinterpret_cast<const s16x8*>(wb + o + c1 + j * 2048);
+    }
+  };
+  f32x4 acc[H * NX][4];
+#pragma unroll
+  for (int i = 0; i < H * NX; i++)
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[i][j] = vra_zero_acc();
-  auto mma = [&](int half, int ks) {  // 16 MFMAs, with the instructions of that half of stage ks + S - 1 between them
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      if constexpr (SPREAD) {
-#pragma unroll
-        for (int e = half * PER + PER * i / 4; e < half * PER + PER * (i + 1) / 4; e++) request(ks + S - 1, e);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < 4; j++) DT::mfma(acc[i][j], wa[half][j], xa[half][i]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-#pragma unroll
-  for (int s = 0; s < S - 1; s++)
-#pragma unroll
-    for (int e = 0; e < D; e++) request(s, e);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PEND) : "memory");
-  __builtin_amdgcn_s_barrier();
-  read(0, 0);
-  for (int ks = 0; ks < KT; ks++) {
-    if constexpr (!SPREAD) {
-#pragma unroll
-      for (int e = 0; e < D; e++) request(ks + S - 1, e);
-    }
-    read(1, ks);
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(1);
-    mma(0, ks);
-    read(0, ks + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(1, ks);
-    __builtin_amdgcn_s_setprio(0);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PEND) : "memory");
+  // (a wave's 64 columns, a phase's rows: nothing of them in the matrix, no MFMAs)
+  const bool in = n0 + cw * 64 < N && m0 + row0 < a.M, in1 = H == 2 && n0 + cw * 64 < N && m0 + row0 + NX * 16 < a.M;
+  auto compute = [&](auto HH) {
+    constexpr int h = decltype(HH)::value;
+    // the next phase's requests have landed (those of the last S - 2 steps, with two phases of the last step, may be on their way), this phase's reads are done
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(H == 2 ? D : (S - 2) * D) : "memory");
     __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if (h ? in1 : in) {
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int kc = 0; kc < 2; kc++)
+#pragma unroll
+        for (int i = 0; i < NX; i++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) DT::mfma_ready(acc[h * NX + i][j], wa[j][kc], xa[i][kc]);
+      __builtin_amdgcn_s_setprio(0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+  if constexpr (H == 2) {
+    stage_x(0, 0, 0, 2);
+    stage_w(0, 0);
+    stage_x(0, 0, 2, 4);
+    stage_x(STG, 1, 0, 2);
+    stage_w(STG, 1);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(D) : "memory");
+    __builtin_amdgcn_s_barrier();
+    if (wg == 1) __builtin_amdgcn_s_barrier();  // the second group runs one barrier behind the first
+    auto step = [&](auto B, int ks) {
+      constexpr int o = decltype(B)::value * STG;
+      read_w(o);
+      __builtin_amdgcn_sched_barrier(0);
+      read_x(o, 0);
+      stage_x(STG - o, ks + 1, 2, 4);
+      compute(C0{});
+      read_x(o, 1);
+      stage_x(o, ks + 2, 0, 2);
+      stage_w(o, ks + 2);
+      compute(C1{});
+    };
+    for (int ks = 0; ks < KT; ks += 2) {
+      step(C0{}, ks);
+      step(C1{}, ks + 1);
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < S - 1; s++) stage_x(s * STG, s, 0, EX), stage_w(s * STG, s);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * D) : "memory");
+    __builtin_amdgcn_s_barrier();
+    if (wg == 1) __builtin_amdgcn_s_barrier();
+    int o = 0, p = (S - 1) * STG;  // buffers of this step and of the one before it
+    for (int ks = 0; ks < KT; ks++) {
+      read_w(o);
+      read_x(o, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      stage_x(p, ks + S - 1, 0, EX);
+      stage_w(p, ks + S - 1);
+      compute(C0{});
+      p = o;
+      o = o == (S - 1) * STG ? 0 : o + STG;
+    }
   }
+  if (wg == 0) __builtin_amdgcn_s_barrier();
   // (the requests beyond K still write LDS: they end before the workgroup does)
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   VRA_MFMA_DRAIN();
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    int m = m0 + wm * 64 + i * 16 + r16;
+  for (int i = 0; i < H * NX; i++) {
+    int m = m0 + row0 + i * 16 + r16;
     if (m >= a.M || (a.x_row && a.x_row[m] < 0)) m = -1;
-    epi.store(m, seg, n0 + wn * 64, N, q4, acc[i]);
+    epi.store(m, seg, n0 + cw * 64, N, q4, acc[i]);
   }
 #endif
 }
 
-// Tile for a product of M rows x ncols[0..nseg) columns x `batch`: workgroups run in rounds of one per CU, a round of a tile takes (us per 64
-// of K, measured with all CUs at work) 0.55 at 64 x 128, 0.62 at 128 x 128, 1.10 at 128 x 256.  -> WM * 16 + WN; *us: the time per 64 of K
-static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch, double* us = nullptr) {
-  const struct { int wm, wn; double us; } t[3] = {{2, 4, 1.10}, {2, 2, 0.62}, {1, 2, 0.55}};
+// Tile for a product of M rows x ncols[0..nseg) columns x `batch`: the least time by this model (us; 198 shapes of 64..8192 rows, 2048..14336 columns,
+// K = 1024..14336, weights from memory: within 4..7 % rms): workgroups run in rounds of `slots`; a launch costs t0, a round `round` (first
+// requests, outputs) and `full` for 64 of K, the last round between `one` (a few workgroups) and `full`.  rows: only tiles of that many (0: any).
+// -> rows / 64 * 16 + columns / 64; *us: the time
+static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch, int K, int rows = 0, double* us = nullptr) {
+  const struct { int bm, bn, slots; double t0, round, one, full; } t[4] = {
+      {256, 256, 256, 3.1, 13.7, 0.80, 1.41}, {128, 256, 256, 1.6, 8.7, 0.54, 0.82}, {128, 128, 256, 1.4, 5.3, 0.33, 0.50}, {64, 128, 512, 2.0, 2.7, 0.28, 0.58}};
   int best = 0;
   double cost = 0.0;
   for (const auto& c : t) {
+    if ((rows && c.bm != rows) || (c.bm == 256 && K % 128)) continue;
     long cols = 0;
-    for (int s = 0; s < nseg; s++) cols += (ncols[s] + 64 * c.wn - 1) / (64 * c.wn);
-    const long tiles = (M + 64 * c.wm - 1) / (64 * c.wm) * cols * batch;
-    const double v = (double)((tiles + 255) / 256) * c.us;
-    if (!best || v < cost) best = c.wm * 16 + c.wn, cost = v;
+    for (int s = 0; s < nseg; s++) cols += (ncols[s] + c.bn - 1) / c.bn;
+    const long tiles = (M + c.bm - 1) / c.bm * cols * batch, full = tiles / c.slots, rem = tiles % c.slots;
+    const double v = c.t0 + (full + (rem ? 1 : 0)) * c.round + K / 64 * (full * c.full + (rem ? c.one + (c.full - c.one) * rem / c.slots : 0.0));
+    if (!best || v < cost) best = c.bm / 64 * 16 + c.bn / 64, cost = v;
   }
   if (us) *us = cost;
   return best;
 }
-static inline bool gemm_rows_has_tile(int tile) { return tile == 2 * 16 + 4 || tile == 2 * 16 + 2 || tile == 16 + 2; }
+static inline bool gemm_rows_has_tile(int tile, int K) { return (tile == 4 * 16 + 4 && K % 128 == 0) || tile == 2 * 16 + 4 || tile == 2 * 16 + 2 || tile == 16 + 2; }
 // fills the tile counts and launches
-template <class DT, int WM, int WN, int S, bool SPREAD, bool PAIR, class EPI>
+template <class DT, int BM, int BN, bool PAIR, class EPI>
 static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStream_t st) {
-  a.MT = (a.M + 64 * WM - 1) / (64 * WM);
+  a.MT = (a.M + BM - 1) / BM;
   a.NT = 0;
-  for (int s = 0; s < a.nseg; s++) a.NT += (a.n[s] + 64 * WN - 1) / (64 * WN);
+  for (int s = 0; s < a.nseg; s++) a.NT += (a.n[s] + BN - 1) / BN;
   static uint64_t attr_devs = 0;  // function attributes belong to the device current at the call
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (!((attr_devs >> (dev & 63)) & 1)) {
-    void (*const k)(GemmRowsArgs, EPI) = gemm_rows_kernel<DT, WM, WN, S, SPREAD, PAIR, EPI>;
+    void (*const k)(GemmRowsArgs, EPI) = gemm_rows_kernel<DT, BM, BN, PAIR, EPI>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr_devs |= (uint64_t)1 << (dev & 63);
   }
-  gemm_rows_kernel<DT, WM, WN, S, SPREAD, PAIR, EPI>
-      <<<dim3((unsigned)(a.MT * a.NT), (unsigned)batch), dim3(64 * WM * WN + (SPREAD ? 0 : 64)), gemm_rows_lds_bytes(WM, WN, S), st>>>(a, epi);
+  using T = GrTile<BM, BN>;
+  gemm_rows_kernel<DT, BM, BN, PAIR, EPI><<<dim3((unsigned)(a.MT * a.NT), (unsigned)batch), dim3(512), (size_t)T::S * T::STG, st>>>(a, epi);
 }
 template <class DT, bool PAIR, class EPI>
 static void gemm_rows_launch(const GemmRowsArgs& a, const EPI& epi, int tile, int batch, hipStream_t st) {
-  if (tile == 2 * 16 + 4) gemm_rows_launch_t<DT, 2, 4, 3, false, PAIR>(a, epi, batch, st);
-  else if (tile == 2 * 16 + 2) gemm_rows_launch_t<DT, 2, 2, 4, true, PAIR>(a, epi, batch, st);
-  else gemm_rows_launch_t<DT, 1, 2, 4, true, PAIR>(a, epi, batch, st);
+  if (tile == 4 * 16 + 4) gemm_rows_launch_t<DT, 256, 256, PAIR>(a, epi, batch, st);
+  else if (tile == 2 * 16 + 4) gemm_rows_launch_t<DT, 128, 256, PAIR>(a, epi, batch, st);
+  else if (tile == 2 * 16 + 2) gemm_rows_launch_t<DT, 128, 128, PAIR>(a, epi, batch, st);
+  else gemm_rows_launch_t<DT, 64, 128, PAIR>(a, epi, batch, st);
 }

@@ -91,7 +91,7 @@ bool vra_gemm_rows_takes(const GemmRowsCall& c) {
   if (c.residual && ((uintptr_t)c.residual % 16 || c.res_ld % 8 || c.out_f32)) return false;
   return true;
 }
-// then time against time: a round of workgroups here (gemm_rows_tile), kernel B at 250 TFLOP/s on whole 64-row blocks behind ~10 us of exchange
+// then time against time: gemm_rows_tile's here, kernel B at 250 TFLOP/s on whole 64-row blocks behind ~10 us of exchange
 // between its K slices
 bool vra_gemm_rows_fits(const GemmRowsCall& c) {
   if (!vra_gemm_rows_takes(c)) return false;
@@ -100,8 +100,8 @@ bool vra_gemm_rows_fits(const GemmRowsCall& c) {
   for (int s = 0; s < c.nseg; s++) n[s] = c.n[s], b_us += 10.0 + 2.0 * ((c.M + 63) / 64 * 64) * (double)c.n[s] * c.K / 250e6;
   if (c.dual) n[0] = 2 * c.n[0];
   double us = 0.0;
-  (void)gemm_rows_tile(c.M, n, c.dual ? 1 : c.nseg, 1, &us);
-  return us * (c.K / 64) < b_us;
+  (void)gemm_rows_tile(c.M, n, c.dual ? 1 : c.nseg, 1, c.K, 0, &us);
+  return us < b_us;
 }
 
 void vra_launch_gemm_rows(const GemmRowsCall& c, int dtype, int64_t stream) {
@@ -110,7 +110,7 @@ void vra_launch_gemm_rows(const GemmRowsCall& c, int dtype, int64_t stream) {
   a.nseg = c.dual ? 1 : c.nseg;
   for (int s = 0; s < c.nseg; s++) a.w[s] = c.w[s], a.n[s] = c.n[s];
   if (c.dual) a.n[0] = 2 * c.n[0];
-  const int tile = c.tile ? c.tile : gemm_rows_tile(c.M, a.n, a.nseg, 1);
+  const int tile = c.tile ? c.tile : gemm_rows_tile(c.M, a.n, a.nseg, 1, c.K);
   auto go = [&](auto dt, auto dual) {
     DenseRowsEpi<decltype(dt), decltype(dual)::value> e = {};
     for (int s = 0; s < a.nseg; s++) e.o[s] = GemmRowsOut{c.out[s], c.bias[s], c.out_ld[s]};
@@ -126,7 +126,7 @@ extern "C" void vra_dense_gemm_tile(int32_t tile, const void* x, const void* con
                                     int32_t pair, const void* residual, void* const* out, int32_t out_f32, int32_t m, int32_t k, int32_t dtype,
                                     int64_t stream) {
   VRA_CHECK_ARG(x && w && bias && n && out && m > 0 && k > 0 && (pair ? nseg == 2 && n[0] == n[1] : nseg >= 1 && nseg <= GR_MAX_SEG), "dense gemm tile: null pointer or bad segments");
-  VRA_CHECK_ARG((dtype == VRA_BF16 || dtype == VRA_F16) && gemm_rows_has_tile(tile) && !(pair && residual), "dense gemm tile: no such form");
+  VRA_CHECK_ARG((dtype == VRA_BF16 || dtype == VRA_F16) && gemm_rows_has_tile(tile, k) && !(pair && residual), "dense gemm tile: no such form");
   GemmRowsCall r;
   r.x = x, r.x_ld = k, r.M = m, r.K = k, r.nseg = nseg, r.dual = pair != 0, r.tile = tile, r.out_f32 = out_f32, r.residual = residual, r.res_ld = n[0];
   for (int s = 0; s < nseg; s++) {

@@ -22,7 +22,7 @@ struct GemmRowsCall {
   int res_ld = 0;
   int out_f32 = 0;
   bool dual = false;
-  int tile = 0;  // WM * 16 + WN instead of gemm_rows_tile's choice
+  int tile = 0;  // rows / 64 * 16 + columns / 64 instead of gemm_rows_tile's choice
 };
 // whether the product can run here and is expected to be faster than on kernel B (and behind it the element-wise launches the fused form
 // saves).  Measured, bf16, cold weights, us (here / kernel B): 64 rows, 2048 x 5632: 50 / 22; 128 rows, 5632 x 2048: 24 / 34; 256 rows, 4096 x 4096:

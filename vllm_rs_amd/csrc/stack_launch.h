@@ -42,7 +42,7 @@ struct StkGemmArgs {
   int batch = 1;
   int64_t a_batch_stride = 0, w_batch_stride = 0, out_batch_stride = 0;
   int64_t bias_batch_stride = 0;  // elements between the bias rows of two products of a batch
-  int tile = 0;  // the tile of gemm_rows_kernel (WM * 16 + WN) instead of the one of gemm_rows_tile; refused where that kernel does not take the product
+  int tile = 0;  // the tile of gemm_rows_kernel (rows / 64 * 16 + columns / 64) instead of the one of gemm_rows_tile; refused where that kernel does not take the product
 };
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream);
 // columns a workgroup takes of a bf16 product of up to 32 rows (pair: with the gated epilogue): 16 or 32, the sums are the same
