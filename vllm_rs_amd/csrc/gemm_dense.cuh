@@ -16,19 +16,21 @@
 //     MFMA FRAGMENTS: a 16-row x 32-k block of x, or 16 columns x 32 k of w.  The dequantised weights are WRITTEN in fragment order
 //     by the dequant pass (one wave load = one contiguous KiB in lane order: the LDS image is lane-linear and `ds_read_b128` at
 //     lane*16 is conflict-free); x is row-major in memory, so a fragment's 64 chunks of 16 B are fetched row by row (4 lanes = 64
-//     contiguous bytes of a row) with the chunk slot XOR-ed by (row >> 2) & 3 — the 16 lanes of a `ds_read_b128` group then cover
-//     all 64 banks (rows r: slot (r & 3) * 64 + (q ^ (r >> 2)) * 16 bytes);
-//   * a wave owns 128 rows x BN/4 columns = 8 x (BN/64) accumulator tiles; a K-step is FOUR phases (quadrants of the wave's tile:
-//     4 m-frags x BN/128 n-frags x 2 k-halves = 16 MFMAs at BN = 256), each  { LDS reads of the quadrant's operands | one staging
-//     unit of LDS-DMA issued | counted vmcnt | barrier | MFMAs | barrier }.  The two wave groups (m halves; one wave of each per
-//     SIMD) run ONE barrier apart, so one group's MFMAs cover the other's LDS reads and DMA issue;
+//     contiguous bytes of a row) with the chunk slot XOR-ed by gx_slot_xor(row): a ds_read_b128 serves lanes 0-3, 12-15 and 20-27 together (then 4-11,
+//     16-19 and 28-31, the upper lanes likewise), and with these slots each such set covers all 64 banks (with (row >> 2) & 3 counted: two
+//     thirds more LDS cycles; 8192 x 8192 x 8192 805 -> 769 us);
+//   * a wave owns 128 rows x BN/4 columns = 8 x (BN/64) accumulator tiles; a K-step is TWO phases (the upper and the lower 64 of its rows:
+//     4 m-frags x BN/64 n-frags x 2 k-halves = 32 MFMAs at BN = 256), each  { LDS reads of the phase's operands | staging units of LDS-DMA
+//     issued | counted vmcnt, lgkmcnt(0) | barrier | MFMAs | barrier }.  The two wave groups (m halves; one wave of each per
+//     SIMD) run ONE barrier apart, so one group's MFMAs cover the other's LDS reads and DMA issue.  The operands come from LDS only: no wait
+//     states between the MFMAs (with them a group's 16 take 296 clocks instead of 256).  Against phases of 16 MFMAs, 8192 x 8192 x 8192:
+//     769 -> 750 us, 2048 clocks of MFMAs in 2240; what is left is the clock, 1.3..1.5 GHz at this power;
 //   * two 64 KiB LDS buffers (even / odd K-step), recycled per STAGING UNIT (16 KiB at BN = 256): U0 = the first 64 rows of both
-//     groups' x, U2 = the other 64, U3 = the first half of every wave's columns, U1 = the other half.  Phase 0 reads U0 + U3
-//     (the U3 fragments stay in registers for phase 3), phase 1 reads U1, phase 2 U2, phase 3 nothing.  A unit is re-staged two
-//     phases after its last read (so both wave groups have retired their reads behind a barrier): phase 0 stages U1(t+1), phase 1
-//     U2(t+1), phase 2 U0(t+2), phase 3 U3(t+2) — every unit has 5-6 phases (1.25 K-steps of MFMAs) to land, with two buffers.
-//     After issuing a phase's unit a wave waits `vmcnt` down to the four newest units; the unit that leaves the count was issued
-//     four phases earlier and is read in the NEXT phase (one barrier later: LDS-DMA data is ordered for a reader only by the
+//     groups' x, U2 = the other 64, U3 = the first half of every wave's columns, U1 = the other half.  Phase 0 reads U0, U3 and U1
+//     (the columns' fragments stay in registers for phase 1), phase 1 reads U2.  A unit is re-staged one phase after its last read (both wave
+//     groups' reads ended before a barrier that the staging wave has passed): phase 0 stages U2(t+1), phase 1 U0, U3 and U1 (t+2) — every
+//     unit has a K-step to land, with two buffers.  After issuing a phase's units a wave waits `vmcnt` down to the newest K-step's
+//     worth of them; what leaves the count is read in the NEXT phase (one barrier later: LDS-DMA data is ordered for a reader only by the
 //     issuing wave's count plus a barrier the reader has passed).  vmcnt never reaches 0 inside the loop;
 //   * workgroup ids are remapped so that the workgroups of one XCD (ids = xcd mod 8) work on neighbouring tiles: 8 m-tiles x 4
 //     n-tiles in flight per XCD share their x and w panels in that XCD's L2;
@@ -122,17 +124,23 @@ __global__ __launch_bounds__(256) void dequant_frag_kernel(const DequantFragBatc
   }
 }
 
+// slot of a row's chunk q in a fragment of x: q ^ this (rows 0-3: 0, 4-7: 2, 8-11: 3, 12-15: 1)
+__device__ __forceinline__ int gx_slot_xor(int row) {
+  const int a = (row >> 2) & 3;
+  return (a >> 1) | (((a ^ (a >> 1)) & 1) << 1);
+}
+
 template <class DT, int BN, bool DUAL>
 __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int NF = BN / 16;    // n-frags of the tile
   constexpr int WNF = NF / 4;    // n-frags of a wave (4 | 2)
-  constexpr int HNF = WNF / 2;   // ... of one phase
+  constexpr int HNF = WNF / 2;   // ... of one unit
   constexpr int XB = 32 * 1024;  // bytes of x per buffer: 16 m-frags x 2 k-chunks
   constexpr int WB = NF * 2 * 1024;
   constexpr int BUF = XB + WB;
   constexpr int WPU = HNF * 8 / 8;  // LDS-DMA instructions per wave for a unit of w: 4 waves' worth of HNF n-frags x 2 k-chunks over 8 waves
-  constexpr int VMW = 2 * 2 + 2 * (HNF == 2 ? 2 : 1);  // DMA instructions of the four newest units (one of each kind)
+  constexpr int VMW = 2 * 2 + 2 * (HNF == 2 ? 2 : 1);  // DMA instructions of a K-step (the newest unit of each kind)
   constexpr uint32_t RSRC3 = 0x00020000u;
   static_assert(BN == 256 || BN == 128, "tile width");
 
@@ -176,10 +184,10 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
   }
   const int m0 = mt * GX_BM;
 
-  // ---- LDS-DMA sources.  x: lane p of a fragment fetch = row p >> 2, chunk slot p & 3 holding chunk (p & 3) ^ ((row >> 2) & 3)
+  // ---- LDS-DMA sources.  x: lane p of a fragment fetch = row p >> 2, chunk slot p & 3 holding chunk (p & 3) ^ gx_slot_xor(row)
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, 0x7FFFFFF0, RSRC3);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.wd), 0, 0x7FFFFFF0, RSRC3);
-  const int srow = lane >> 2, schunk = (lane & 3) ^ ((srow >> 2) & 3);
+  const int srow = lane >> 2, schunk = (lane & 3) ^ gx_slot_xor(srow);
   //   this wave stages m-frag mfs (+4 for U2) of the tile: {0,1,2,3,8,9,10,11}[wave]
   const int mfs = wave < 4 ? wave : wave + 4;
   uint32_t vo_x[2];
@@ -213,20 +221,20 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
   };
 
   // ---- LDS reads: x fragment (m-frag, kc) of this wave's rows, w fragment (n-frag, kc) of its columns
-  const unsigned char* xrd = smem + (wr * 8) * 2048 + (r16 * 4 + (q4 ^ ((r16 >> 2) & 3))) * 16;
+  const unsigned char* xrd = smem + (wr * 8) * 2048 + (r16 * 4 + (q4 ^ gx_slot_xor(r16))) * 16;
   const unsigned char* wrd = smem + XB + (wc * WNF) * 2048 + lane * 16;
-  s16x8 xa[4][2], w0[HNF][2], w1[HNF][2];
+  s16x8 xa[4][2], wa[WNF][2];
   auto read_x = [&](int buf, int mh) {
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
       for (int kc = 0; kc < 2; kc++) xa[i][kc] = *reinterpret_cast<const s16x8*>(xrd + buf * BUF + ((mh * 4 + i) * 2 + kc) * 1024);
   };
-  auto read_w = [&](int buf, int nh, s16x8 (&w)[HNF][2]) {
+  auto read_w = [&](int buf) {
 #pragma unroll
-    for (int j = 0; j < HNF; j++)
+    for (int j = 0; j < WNF; j++)
 #pragma unroll
-      for (int kc = 0; kc < 2; kc++) w[j][kc] = *reinterpret_cast<const s16x8*>(wrd + buf * BUF + ((nh * HNF + j) * 2 + kc) * 1024);
+      for (int kc = 0; kc < 2; kc++) wa[j][kc] = *reinterpret_cast<const s16x8*>(wrd + buf * BUF + (j * 2 + kc) * 1024);
   };
 
   f32x4 acc[8][WNF];
@@ -234,77 +242,63 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
   for (int i = 0; i < 8; i++)
 #pragma unroll
     for (int j = 0; j < WNF; j++) acc[i][j] = vra_zero_acc();
-  auto mma = [&](int mh, int nh, const s16x8 (&w)[HNF][2]) {  // A = weights (16 columns x 32 k), B = x (16 rows x 32 k): D[column][row]
+  // waits for the phase's own LDS reads and the next phase's units, then the matrix work between two barriers.  A = weights (16 columns x
+  // 32 k), B = x (16 rows x 32 k): D[column][row]
+  auto compute = [&](auto MH) {
+    constexpr int mh = decltype(MH)::value;
+    if constexpr (VMW == 8) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int kc = 0; kc < 2; kc++)
 #pragma unroll
       for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int j = 0; j < HNF; j++) DT::mfma(acc[mh * 4 + i][nh * HNF + j], w[j][kc], xa[i][kc]);
+        for (int j = 0; j < WNF; j++) DT::mfma_ready(acc[mh * 4 + i][j], wa[j][kc], xa[i][kc]);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
   };
-#define GX_WAIT_VM()                                                   \
-  do {                                                                 \
-    if constexpr (VMW == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); \
-    else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");              \
-  } while (0)
-#define GX_COMPUTE(MH, NH, W)                        \
-  do {                                               \
-    __builtin_amdgcn_s_barrier();                    \
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); \
-    __builtin_amdgcn_sched_barrier(0);               \
-    __builtin_amdgcn_s_setprio(1);                   \
-    mma(MH, NH, W);                                  \
-    __builtin_amdgcn_s_setprio(0);                   \
-    __builtin_amdgcn_sched_barrier(0);               \
-    __builtin_amdgcn_s_barrier();                    \
-  } while (0)
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
 
   // this workgroup's K-steps (an even count: launcher) — all of them, or slice zi of SK
   const int ks0 = KS / SK * zi, ks1 = ks0 + KS / SK;
-  // ---- prologue: the first K-step entirely, U0 / U3 of the second (the order the counted waits assume: oldest first)
+  // ---- prologue: the first K-step entirely, U0 / U3 / U1 of the second (the order the counted waits assume: oldest first)
   stage_x(0, 0, ks0);
   stage_w(0, 0, ks0);
   stage_w(0, 1, ks0);
   stage_x(0, 1, ks0);
   stage_x(1, 0, ks0 + 1);
   stage_w(1, 0, ks0 + 1);
-  GX_WAIT_VM();
+  stage_w(1, 1, ks0 + 1);
+  if constexpr (VMW == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   if (wr == 1) __builtin_amdgcn_s_barrier();  // the second wave group runs one barrier behind the first
 
   auto kstep = [&](auto BUFC, int ks) {
     constexpr int b = decltype(BUFC)::value;
-    // phase 0: quadrant (rows 0..63, first column half)
-    read_w(b, 0, w0);
+    read_w(b);
     __builtin_amdgcn_sched_barrier(0);
     read_x(b, 0);
-    stage_w(b ^ 1, 1, ks + 1);
-    GX_WAIT_VM();
-    GX_COMPUTE(0, 0, w0);
-    // phase 1: (rows 0..63, second column half)
-    read_w(b, 1, w1);
     stage_x(b ^ 1, 1, ks + 1);
-    GX_WAIT_VM();
-    GX_COMPUTE(0, 1, w1);
-    // phase 2: (rows 64..127, second column half)
+    compute(C0{});
     read_x(b, 1);
     stage_x(b, 0, ks + 2);
-    GX_WAIT_VM();
-    GX_COMPUTE(1, 1, w1);
-    // phase 3: (rows 64..127, first column half) — operands already in registers
     stage_w(b, 0, ks + 2);
-    GX_WAIT_VM();
-    GX_COMPUTE(1, 0, w0);
+    stage_w(b, 1, ks + 2);
+    compute(C1{});
   };
   for (int ks = ks0; ks < ks1; ks += 2) {
-    kstep(std::integral_constant<int, 0>{}, ks);
-    kstep(std::integral_constant<int, 1>{}, ks + 1);
+    kstep(C0{}, ks);
+    kstep(C1{}, ks + 1);
   }
   if (wr == 0) __builtin_amdgcn_s_barrier();
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped stagings of the last K-steps
   VRA_MFMA_DRAIN();
-#undef GX_WAIT_VM
-#undef GX_COMPUTE
 
   // ---- split-K: the slices of a tile meet through memory (gemm_q4_big.cuh): write-through 16-byte stores, one flag line per slice,
   // the last slice ("owner") polls, adds the slabs to its own partial in slice order and resets the flags
