@@ -1,15 +1,18 @@
 // gemm_q4_mid.cuh — "kernel M": int4 GEMM for 64 rows up (short and middle prompts), every row of a block of up to 160 in one workgroup.
 //
-// What bounds a short prompt's int4 product is not memory (the codes of a gate/up pair of 4096 x 14336 take 13 us) but converting the codes: a
-// matrix instruction and a conversion take their SUM on a SIMD, also from different waves (tools/mfma_valu_probe.hip), and the kernels of 32- or
-// 64-row tiles convert every code once per row block.  Here a workgroup owns 128 virtual columns (64 gate + 64 up of a pair) and ALL rows of
-// the block, 32 MB of them (MB 2..5): 8 waves as 4 (columns, two n-blocks each) x 2 (rows, MB m-tiles each), so a code is converted twice for up to
-// 160 rows, and a k-tile's 8 MB MFMAs of a wave are 2 MB independent chains.  x, codes and scales of a k-tile of 128 travel by LDS-DMA through a
-// ring of three stages (one barrier a k-tile); the 16-byte chunks of an x row lie at slot chunk ^ (row mod 16), so the fragment reads meet no bank
-// twice.  Two n-blocks a wave read each x fragment from LDS four times a workgroup: 160 KB a k-tile at MB = 5, 1280 cycles (and 880 for the DMA's
-// writes) beside 1380 of MFMAs and 500 of conversions on each SIMD; four n-blocks a wave would halve the reads and double the conversions.
-// us a launch, kernel D or W / here: gate/up of 4096 x 14336 behind its norm, 150 rows 91 / 56 (f16 in a model's step 55), 96 rows 50 / 42; down of
-// 14336 x 4096 with its row sums, 200 rows 56 / 49.  AWQ: gate/up of 3584 x 18944, 320 rows 190 / 156.
+// What bounds a short prompt's int4 product is not memory (the codes of a gate/up pair of 4096 x 14336 take 13 us) but the instructions beside the
+// MFMAs: converting the codes, scaling the group sums, LDS reads, requests; and the kernels of 32- or 64-row tiles convert every code once per row
+// block.  Here a workgroup owns 128 virtual columns (64 gate + 64 up of a pair) and ALL rows of the block, 32 MB of them (MB 2..5): 8 waves as 4
+// (columns, two n-blocks each) x 2 (rows, MB m-tiles each), so a code is converted twice for up to 160 rows, and a k-tile's 8 MB MFMAs of a wave are
+// 2 MB independent chains.  x, codes and scales of a k-tile of 128 travel by LDS-DMA through a ring of three stages; the 16-byte chunks of an x row
+// lie at slot chunk ^ (row mod 16), so the fragment reads meet no bank twice.
+// The two row halves (a wave of each on every SIMD) run one barrier apart: while one multiplies, the other scales its last group sums into acc and
+// prepares its next tile.  A lone wave issues an instruction every five cycles or so, so the two phases are of about 130 instructions each; the
+// conversions of a tile's later fragments lie between the MFMAs of its earlier ones.  Codes, scales and row sums are fetched by the first half
+// alone: it asks for them a phase earlier and so two and a half phases ahead.
+// us a launch with its row sums, both halves in step / so: gate/up of 4096 x 14336, 64 rows 37.6 / 34.6, 150 rows 57.7 / 54.8, 320 rows 104 / 97; down
+// of 18944 x 3584, 150 rows 46.7 / 43.7, 700 rows 218 / 186; AWQ 62.3 / 61.5, 113 / 112, 49.3 / 47.9, 237 / 219 (no shape more than 1.5 % slower).
+// Against kernel D or W: gate/up of 4096 x 14336 behind its norm, 150 rows 91 / 53; AWQ, 3584 x 18944, 320 rows 190 / 147.
 //
 // The zero points come off per k-tile, acc += s (acc_g - (C + z) Sx): acc never holds more than the result's own size.  (Taken off once behind the
 // k loop, x of mean 0.5 left the float32 sums of K = 14336 ten times as far from the 64-bit result.)  Symmetric codes have one z: a row's group sums
@@ -23,13 +26,13 @@
 #include "gemm_q4_big.cuh"  // GemmDArgs
 
 #define GM_THREADS 512
-static inline size_t gemm_q4_mid_lds_bytes(int mb) { return (size_t)3 * (32 * mb * 256 + 8 * 1024 + 8 * 256 + 32 * mb * 4); }
+static inline size_t gemm_q4_mid_lds_bytes(int mb) { return (size_t)3 * (32 * mb * 256 + 8 * 1024 + 4 * 256 + 32 * mb * 4); }
 
 template <class DT, bool DUAL, bool AWQ, int MB>
 __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  constexpr int NB = 2, ROWS = 32 * MB, XB = ROWS * 256, WB = 8 * 1024, SB = 8 * 256, STG = XB + WB + SB + ROWS * 4, PER = MB + 3;
+  constexpr int NB = 2, ROWS = 32 * MB, XB = ROWS * 256, WB = 8 * 1024, SB = 4 * 256, STG = XB + WB + SB + ROWS * 4, PER = MB + 4;
   constexpr uint32_t RSRC3 = 0x00020000u;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -74,14 +77,15 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
   // ---- DMA sources.  A wave fetches MB KiB of x (4 rows each), the codes of its block wm (the other wave of the column pair the other's),
   // its own copy of its two blocks' scales (lanes 0..15) and zero points (lanes 16..19; the rest fetch the same again), and 4 MB row sums
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, 0x7FFFFFF0, RSRC3);
-  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(wm ? wt[1] : wt[0]), 0, 0x7FFFFFF0, RSRC3);
+  const __amdgpu_buffer_rsrc_t rw0 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(wt[0]), 0, 0x7FFFFFF0, RSRC3);
+  const __amdgpu_buffer_rsrc_t rw1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(wt[1]), 0, 0x7FFFFFF0, RSRC3);
   uint32_t vo_x[MB];
 #pragma unroll
   for (int i = 0; i < MB; i++) {
     const int row = (wave * MB + i) * 4 + oct;
     vo_x[i] = ((uint32_t)min(m0 + row, M - 1) * (uint32_t)a.x_ld + (uint32_t)(nn ^ (row & 15)) * 8u) * 2u;  // rows >= M alias row M - 1 (never stored)
   }
-  const uint32_t vo_w = (uint32_t)lane * 16u, so_w = (uint32_t)(wm ? nbc[1] : nbc[0]) * (uint32_t)KT;
+  const uint32_t vo_w = (uint32_t)lane * 16u, so_w0 = (uint32_t)nbc[0] * (uint32_t)KT, so_w1 = (uint32_t)nbc[1] * (uint32_t)KT;
   typedef const __attribute__((address_space(1))) void* glb_ptr;
   typedef __attribute__((address_space(3))) void* lds_ptr;
   const int second = (lane & 16) ? (lane >> 1) & 1 : (lane >> 3) & 1;  // (the lane's block of the two)
@@ -92,102 +96,45 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
   const unsigned char* const sc_src = zero_lane ? (second ? z1 : z0) + ((second ? nbc[1] : nbc[0]) * 2 + (lane & 1)) * 4
                                                 : (second ? s1 : s0) + ((second ? nbc[1] : nbc[0]) * 32 + (lane & 7) * 4);
   const uint32_t sc_ld = zero_lane ? (uint32_t)N / 2 : (uint32_t)N * 2;  // bytes between two groups
-  const int srow = wave * 4 * MB;  // row sums of the rows srow + lane, lane < 4 MB
+  const int srow = wn * 8 * MB;  // row sums of the rows srow + lane, lane < 8 MB
   const float* const sum_src = a.xsum + (size_t)min(m0 + srow + lane, M - 1) * KT;
-  auto request = [&](int kt) {
-    unsigned char* const d = smem + ((kt - kt0) % 3) * STG;
+  // requests of k-tile kt (beyond the last: the last again, never read) into the stage at byte `o`
+  auto request = [&](int o, int kt) {
+    unsigned char* const d = smem + o;
+    kt = min(kt, kt1 - 1);
 #pragma unroll
     for (int i = 0; i < MB; i++)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(d + (wave * MB + i) * 1024), 16, vo_x[i], (uint32_t)kt * 256u, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(d + XB + (2 * wn + wm) * 1024), 16, vo_w, (so_w + (uint32_t)kt) * 1024u, 0, 2);  // nt
+    if (wm) return;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw0, (lds_ptr)(d + XB + 2 * wn * 1024), 16, vo_w, (so_w0 + (uint32_t)kt) * 1024u, 0, 2);  // nt
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rw1, (lds_ptr)(d + XB + (2 * wn + 1) * 1024), 16, vo_w, (so_w1 + (uint32_t)kt) * 1024u, 0, 2);
     const int grp = grouped ? (kt * 128) >> gsh : 0;
-    __builtin_amdgcn_global_load_lds((glb_ptr)(sc_src + (size_t)grp * sc_ld), (lds_ptr)(d + XB + WB + wave * 256), 4, 0, 0);
-    if (lane < 4 * MB) __builtin_amdgcn_global_load_lds((glb_ptr)(sum_src + kt), (lds_ptr)(d + XB + WB + SB + srow * 4), 4, 0, 0);
+    __builtin_amdgcn_global_load_lds((glb_ptr)(sc_src + (size_t)grp * sc_ld), (lds_ptr)(d + XB + WB + wn * 256), 4, 0, 0);
+    if (lane < 8 * MB) __builtin_amdgcn_global_load_lds((glb_ptr)(sum_src + kt), (lds_ptr)(d + XB + WB + SB + srow * 4), 4, 0, 0);
   };
 
-  f32x4 acc[NB][MB];
+  f32x4 acc[NB][MB], ag[NB][MB];
 #pragma unroll
   for (int b = 0; b < NB; b++)
 #pragma unroll
     for (int t = 0; t < MB; t++) acc[b][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int xrow = (wm * MB * 16 + nn) * 256;
-  u32x4 wq[NB], xf[2][MB];
-  u32x2 scw[NB];
-  uint32_t zw[NB];
-  float sx[MB];
-  auto read_w = [&](int kt) {
-    const unsigned char* const st = smem + ((kt - kt0) % 3) * STG + XB;
+  const unsigned char* const xl = smem + (wm * MB * 16 + nn) * 256;
+  const unsigned char* const wl = smem + XB + 2 * wn * 1024 + lane * 16;
+  const unsigned char* const scl = smem + XB + WB + wn * 256;
+  const unsigned char* const sml = smem + XB + WB + SB + (wm * MB * 16 + nn) * 4;
+  u32x4 xf[4][MB];
+  u32x4 wq[NB];
+  s16x8 af[2][NB];
+  u32x2 scc[NB];
+  uint32_t zc[NB];
+  float sxc[MB];
+  f32x4 zx[MB];  // symmetric codes: the zero points' part of a row's group sums, the same for every column
+  auto read_x = [&](int o, int j) {
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-      wq[b] = *reinterpret_cast<const u32x4*>(st + (2 * wn + b) * 1024 + lane * 16);
-      scw[b] = *reinterpret_cast<const u32x2*>(st + WB + wave * 256 + b * 32 + oct * 8);
-      if (AWQ) zw[b] = *reinterpret_cast<const uint32_t*>(st + WB + wave * 256 + 64 + b * 8 + (oct >> 1) * 4);
-    }
-#pragma unroll
-    for (int t = 0; t < MB; t++) sx[t] = *reinterpret_cast<const float*>(st + WB + SB + ((wm * MB + t) * 16 + nn) * 4);
+    for (int t = 0; t < MB; t++) xf[j][t] = *reinterpret_cast<const u32x4*>(xl + o + (((j * 4 + oct) ^ nn) * 16) + t * 4096);
   };
-  auto read_x = [&](int kt, int j) {
-    const unsigned char* const st = smem + ((kt - kt0) % 3) * STG + xrow + (((j * 4 + oct) ^ nn) * 16);
-#pragma unroll
-    for (int t = 0; t < MB; t++) xf[j & 1][t] = *reinterpret_cast<const u32x4*>(st + t * 4096);
-  };
-  // Three stages in flight; stage kt + 1 is waited for before the LAST fragments' MFMAs of tile kt, so its first reads, the barrier's skew and the
-  // next requests (into the buffer of tile kt, whose last fragments are in registers by then) lie beside them.
-#pragma unroll
-  for (int i = 0; i < 3; i++)
-    if (kt0 + i < kt1) request(kt0 + i);
-  auto arrive = [&](int kt) {  // stage kt is here: this wave's own requests are, and the barrier says the same of the other waves'
-    if (kt + 1 < kt1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(PER) : "memory");  // (at most stage kt + 1 is still on its way)
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  if (kt0 + 2 < kt1) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER) : "memory");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-  } else {
-    arrive(kt0);
-  }
-  read_w(kt0);
-  read_x(kt0, 0);
-  for (int kt = kt0; kt < kt1; kt++) {
-    f32x4 ag[NB][MB];
-    s16x8 af[2][NB];
-    u32x2 scc[NB];
-    uint32_t zc[NB];
-    float sxc[MB];
-    f32x4 zx[MB];  // symmetric codes: the zero points' part of a row's group sums, the same for every column
-#pragma unroll
-    for (int b = 0; b < NB; b++) af[0][b] = magic_word<DT>(wq[b][0]), scc[b] = scw[b], zc[b] = zw[b];
-#pragma unroll
-    for (int t = 0; t < MB; t++) {
-      sxc[t] = sx[t];
-      const float z = -(Magic<DT>::bias + 8.f) * sx[t];
-      zx[t] = f32x4{z, z, z, z};
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      if (j == 3 && kt + 1 < kt1) {
-        arrive(kt + 1);
-        if (kt + 3 < kt1) request(kt + 3);
-      }
-#pragma unroll
-      for (int t = 0; t < MB; t++)
-#pragma unroll
-        for (int b = 0; b < NB; b++) {
-          if (j == 0 && AWQ) DT::mfma0(ag[b][t], af[0][b], __builtin_bit_cast(s16x8, xf[0][t]));
-          else if (j == 0) DT::mfma_from(ag[b][t], af[0][b], __builtin_bit_cast(s16x8, xf[0][t]), zx[t]);
-          else DT::mfma(ag[b][t], af[j & 1][b], __builtin_bit_cast(s16x8, xf[j & 1][t]));
-          if (t == 0 && b == 0) {  // (behind the wait for fragment j: fragment j + 1 is not part of it)
-            __builtin_amdgcn_sched_barrier(0);
-            if (j < 3) read_x(kt, j + 1);
-            else if (kt + 1 < kt1) read_w(kt + 1), read_x(kt + 1, 0);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          if (j < 3 && t == 1) af[(j + 1) & 1][b] = magic_word<DT>(wq[b][j + 1]);
-        }
-    }
+  // a k-tile's group sums, scaled, into acc
+  auto fix = [&]() {
     VRA_MFMA_DRAIN();
 #pragma unroll
     for (int b = 0; b < NB; b++) {
@@ -198,7 +145,86 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
 #pragma unroll
         for (int r = 0; r < 4; r++) acc[b][t][r] = fmaf(s4[r], AWQ ? fmaf(-z4[r], sxc[t], ag[b][t][r]) : ag[b][t][r], acc[b][t][r]);
     }
+  };
+  // the vector half of k-tile kt: codes, scales, zero points and row sums from LDS; the sums of tile kt - 1 into acc meanwhile; conversions
+  auto prepare = [&](int o, bool first) {
+    u32x2 scw[NB];
+    uint32_t zw[NB];
+    float sx[MB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      wq[b] = *reinterpret_cast<const u32x4*>(wl + o + b * 1024);
+      scw[b] = *reinterpret_cast<const u32x2*>(scl + o + b * 32 + oct * 8);
+      if (AWQ) zw[b] = *reinterpret_cast<const uint32_t*>(scl + o + 64 + b * 8 + (oct >> 1) * 4);
+    }
+#pragma unroll
+    for (int t = 0; t < MB; t++) sx[t] = *reinterpret_cast<const float*>(sml + o + t * 64);
+    read_x(o, 0);
+    read_x(o, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (!first) fix();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      scc[b] = scw[b], zc[b] = AWQ ? zw[b] : 0;
+      af[0][b] = magic_word<DT>(wq[b][0]);
+    }
+#pragma unroll
+    for (int t = 0; t < MB; t++) {
+      sxc[t] = sx[t];
+      const float z = AWQ ? 0.f : -(Magic<DT>::bias + 8.f) * sx[t];
+      zx[t] = f32x4{z, z, z, z};
+      asm volatile("" : "+v"(zx[t]));
+    }
+#pragma unroll
+    for (int b = 0; b < NB; b++) asm volatile("" : "+v"(af[0][b]));
+  };
+  auto multiply = [&](int o) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if (j < 2) read_x(o, j + 2);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < MB; t++)
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+          const s16x8 xv = __builtin_bit_cast(s16x8, xf[j][t]);
+          if (j == 0 && AWQ) DT::mfma0(ag[b][t], af[0][b], xv);
+          else if (j == 0) DT::mfma_from(ag[b][t], af[0][b], xv, zx[t]);
+          else if (t == 0) DT::mfma(ag[b][t], af[j & 1][b], xv);
+          else DT::mfma_ready(ag[b][t], af[j & 1][b], xv);
+          if (j < 3 && t == 1) af[(j + 1) & 1][b] = magic_word<DT>(wq[b][j + 1]);
+        }
+    }
+    __builtin_amdgcn_s_setprio(0);
+  };
+  auto barrier = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  request(0, kt0);
+  request(STG, kt0 + 1);
+  if (wm == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
+  else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(MB) : "memory");
+  barrier();
+  if (wm == 1) barrier();  // the second group runs one barrier behind the first
+  int o = 0, q = 2 * STG;  // stages of this k-tile and of the one after the next
+  for (int kt = kt0; kt < kt1; kt++) {
+    prepare(o, kt == kt0);
+    if (wm == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    barrier();
+    request(q, kt + 2);
+    multiply(o);
+    if (wm == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
+    barrier();
+    o = o == 2 * STG ? 0 : o + STG;
+    q = q == 2 * STG ? 0 : q + STG;
   }
+  if (wm == 0) barrier();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the requests beyond the last tile still write LDS)
+  fix();
 
   // ---- split K: kernel D's exchange
   if (SK > 1) {

@@ -39,7 +39,8 @@ int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, cons
     if (S > 1 && ((size_t)S * tiles * 2 * mb * GM_THREADS * 16 > vra_scratch_slab_bytes() - kXsum || (size_t)tiles * S * 16 > vra_scratch_counter_count())) break;
     // Fitted to the Llama-3-8B and Qwen2-7B shapes at 64..760 rows (us): a launch 3 and 5.5 a round of workgroups; a k-tile as in `tile`, symmetric
     // codes and AWQ (which unpacks its zero points and takes them off a column at a time): gate/up of 4096 x 14336, one round of 224 workgroups: 33 / 39 /
-    // 46 / 53 at MB 2..5; down of 18944 x 3584, 256 rows in 4 slices: 65; a slab of the exchange 0.43 per 32 rows beyond the first; two
+    // 46 / 53 at MB 2..5; down of 18944 x 3584, 256 rows in 4 slices: 65 (with the row halves a barrier apart symmetric codes take 5 % less: the
+    // lines to the other kernels stayed where they were); a slab of the exchange 0.43 per 32 rows beyond the first; two
     // workgroups of MB 2 share a CU, 13 % faster than one after the other; 4 for the row sums where no norm's launch leaves them
     static const double tile[2][6] = {{0, 0, 0.76, 0.93, 1.17, 1.44}, {0, 0, 0.82, 1.00, 1.28, 1.57}};
     const double rounds = (double)((tiles * S + cus - 1) / cus), q = rounds * (mb == 2 && rounds > 1 ? 0.87 : 1.0);
