@@ -55,3 +55,31 @@ def test_wide_tile_of_a_layer_stack(M, N, K, scatter):
     one, wide = run(0x12), run(0x44)
     assert np.array_equal(wide, one) and wide[:M].any() and not wide[M].any()
     assert not scatter or not wide[np.setdiff1d(np.arange(M), dst)].any()
+
+
+@pytest.mark.parametrize("tile", [0x12, 0x22, 0x24])
+@pytest.mark.parametrize("rows128", [1, 17, 33])
+@pytest.mark.parametrize("N", [40, 300])
+def test_grouped_rows_reach_every_tile(N, rows128, tile):
+    """tile rows around whole rounds of pairs by eight XCDs, empty ones at the end and between, one and several tile columns; every product of a row is
+    a sum of 64 bf16 products in f32: 2e-6 of the result's norm (a chain of 64 roundings), rows of empty tiles are left alone"""
+    L = _lib.load()
+    r = rng(N + rows128 + tile)
+    K, E, rows = 64, 5, rows128 * 128
+    x = (r.standard_normal((rows, K)).astype(np.float32).view(np.uint32) & 0xFFFF0000).view(np.float32)  # bf16 values
+    w = (r.standard_normal((E, N, K)).astype(np.float32).view(np.uint32) & 0xFFFF0000).view(np.float32)
+    group = r.integers(0, E, rows128).astype(np.int32)
+    group[r.random(rows128) < 0.2] = -1
+    group[rows128 - rows128 // 4:] = -1
+    bits = lambda a: ops.dev((a.view(np.uint32) >> 16).astype(np.uint16))
+    gd = ops.dev(np.repeat(group, 128 // ((tile >> 4) * 64)).view(np.uint32))
+    xd, wd, out = bits(x), bits(w), ops.DevBuf(rows * N * 4).fill_bytes(0)
+    L.vra_stack_op_gemm_tile(tile, xd.ptr, K, wd.ptr, N * K, out.ptr, N, 1, rows, N, K, gd.ptr, None, 0, None, 0, 0.0, 0)
+    ops.check_error()
+    got = out.numpy(np.float32, (rows, N)).astype(np.float64)
+    of_row = np.repeat(group, 128)
+    ref = np.zeros((rows, N))
+    for e in range(E):
+        ref[of_row == e] = x[of_row == e].astype(np.float64) @ w[e].astype(np.float64).T
+    assert (got[of_row < 0] == 0).all()
+    assert np.linalg.norm(got - ref) <= 2e-6 * max(np.linalg.norm(ref), 1e-30)

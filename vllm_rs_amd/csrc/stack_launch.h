@@ -28,6 +28,7 @@ struct StkGemmArgs {
   float alpha = 1.f;
   const int* tile_group = nullptr;
   int granule = 0;
+  int likely_rows = 0;  // grouped: rows that granules with a group are likely to take, of the M there is room for (0: unknown); for the choice of a tile
   const int* a_row = nullptr;
   int a_rows = 0;  // rows of A behind a_row (0: unknown)
   const float* a_scale = nullptr;

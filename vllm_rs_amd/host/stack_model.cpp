@@ -1093,7 +1093,7 @@ bool StackModel::tiles128(const StackLayer& L) const {
 // bf16: the activation is the epilogue of the gate / up launch; f32: product, activation and product as three launches
 bool StackModel::expert_pair(const void* a, int lda, const void* w_gu, int64_t gu_stride, const void* w_down, int64_t down_stride, int rows, int fp,
                              int f, float limit, const int* tile_group, int granule, const int* a_row, const float* a_scale, const int* out_row,
-                             float* out, int64_t stream, int act) {
+                             float* out, int64_t stream, int act, int likely_rows) {
   const int W = width_;
   StkGemmArgs g;
   if (granule == 128 && a_scale) {  // (the 128-row tiles take their rows as they are)
@@ -1102,7 +1102,7 @@ bool StackModel::expert_pair(const void* a, int lda, const void* w_gu, int64_t g
   }
   g.a_rows = max_tokens_;
   g.a = a, g.lda = lda, g.w = w_gu, g.w_group_stride = gu_stride, g.M = rows, g.N = (act >= 3 ? 1 : 2) * fp, g.K = W;
-  g.tile_group = tile_group, g.granule = granule, g.a_row = a_row, g.a_scale = a_scale;
+  g.tile_group = tile_group, g.granule = granule, g.likely_rows = likely_rows, g.a_row = a_row, g.a_scale = a_scale;
   g.limit = limit, g.act = act;
   const bool fused = dt_ == VRA_BF16 && W % 8 == 0 && lda % 8 == 0;
   if (act >= 3) {  // no gate: an element-wise activation, in the epilogue whatever the type
@@ -1119,7 +1119,7 @@ bool StackModel::expert_pair(const void* a, int lda, const void* w_gu, int64_t g
   StkGemmArgs d;
   d.a = act_, d.lda = fp, d.w = w_down, d.w_group_stride = down_stride, d.M = rows, d.N = W, d.K = fp;
   d.out = out, d.ldo = W, d.out_f32 = 1;
-  d.tile_group = tile_group, d.granule = granule, d.out_row = out_row;
+  d.tile_group = tile_group, d.granule = granule, d.likely_rows = likely_rows, d.out_row = out_row;
   // rows of a granule that hold no pair are neither read nor written: a_row of the first launch marks them, the second sees them through out_row
   vra_stack_gemm(d, dt_, stream);
   return !take_stack_err(error, "expert feed-forward");
@@ -1147,7 +1147,7 @@ bool StackModel::feed_forward(const StackLayer& L, int T, int64_t stream) {
     vra_stack_moe_sort(pair_expert_, pair_weight_, P, L.top, L.experts, granule, rows, row_token_, row_scale_, row_pair_, tile_group_, stream);
     if (take_stack_err(error, "expert rows")) return false;
     if (!expert_pair(h_, W, L.e_gu, (int64_t)2 * L.ffp * W, L.e_down, (int64_t)W * L.ffp, rows, L.ffp, L.ff, L.limit, tile_group_, granule, row_token_,
-                     row_scale_, row_pair_, pair_out_, stream))
+                     row_scale_, row_pair_, pair_out_, stream, 0, std::min(rows, P + L.experts * granule / 2)))
       return false;
     if (L.shared_ff > 0 &&
         !expert_pair(h_, W, L.s_gu, 0, L.s_down, 0, T, L.sffp, L.shared_ff, L.shared_limit, nullptr, 0, nullptr, nullptr, nullptr, sh_, stream))
@@ -1554,7 +1554,7 @@ bool StackModel::forward_sandwich(const InputMetadata& md, int64_t stream) {
       if (take_stack_err(error, "expert rows")) return false;
       // (the weights of a softmax router multiply the experts' OUTPUTS: the rows go in unscaled, the sum over a token's pairs carries them)
       if (!expert_pair(h_, W, L.e_gu, (int64_t)(L.gated() ? 2 : 1) * L.ffp * W, L.e_down, (int64_t)W * L.ffp, rows, L.ffp, L.ff, L.limit, tile_group_, granule, row_token_,
-                       L.router_kind >= 1 ? nullptr : row_scale_, row_pair_, pair_out_, stream, L.act_kind))
+                       L.router_kind >= 1 ? nullptr : row_scale_, row_pair_, pair_out_, stream, L.act_kind, std::min(rows, P + L.experts * granule / 2)))
         return false;
       pend.p1 = pair_out_, pend.n1 = L.top, pend.pw = L.router_kind >= 1 ? pair_weight_ : nullptr;
       pend.post_w = L.post2_w, pend.post_b = L.post2_b, pend.post_alpha = L.post2_alpha;

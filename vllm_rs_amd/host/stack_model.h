@@ -252,7 +252,7 @@ class StackModel : public ModelBase {
   bool tiles128(const StackLayer& L) const;
   bool expert_pair(const void* a, int lda, const void* w_gu, int64_t gu_stride, const void* w_down, int64_t down_stride, int rows, int fp, int f,
                    float limit, const int* tile_group, int granule, const int* a_row, const float* a_scale, const int* out_row, float* out,
-                   int64_t stream, int act = 0);
+                   int64_t stream, int act = 0, int likely_rows = 0);
   vra_model_config mc_;
   vra_engine_config ec_;
   std::string spec_error_;
