@@ -23,7 +23,11 @@
 // staging instructions per wave, parity-green, and slower: 618 against 738 TFLOP/s at 16 384 tokens, 448 against 486 at 8192
 // (profiles/r06_ab_attn_prefill_8_waves.txt).  Two independent 4-wave workgroups per CU drift apart and cover each other's
 // softmax; eight waves behind one barrier do not.)
-// Roofline: MFMA.  FLOPs = 4 * D * (causal query-key pairs) per head.
+// What bounds it: vector instructions beside the MFMAs and, in long prompts, the chip's power (2.0 GHz).  Of 260 a wave and tile 50 went: no zeroed score
+// tiles, maxima without quieting, loads on scalar bases, rescaling by row tiles; and MFMAs whose operands come from LDS carry no wait states.  8192 tokens, 32 / 8
+// heads of 128: 700 -> 666 us a layer; four prompts of up to 700 tokens, 32 / 4 heads of 64: 24.0 -> 22.3.  (Two LDS buffers, one barrier a tile and all
+// loads in the score phase: the same times.  Row references that stay until a score passes them by 8, so that O is hardly ever rescaled: 2..3 % more, other
+// roundings.)
 #pragma once
 #include "common.cuh"
 #include "kvcache.cuh"
@@ -66,6 +70,28 @@ __device__ __forceinline__ int pf_kswz(int key, int c) {  // K tile: chunk c of 
   return c ^ (f >> 1);  // D = 64: 8 chunks per row, two rows per 256-byte bank row
 }
 __device__ __forceinline__ int pf_vswz(int ch, int c) { return c ^ ((ch >> 1) & 7); }  // V tile rows are 128 B (8 chunks)
+
+// maxima as the instructions are (a number wins over a NaN): fmaxf first quiets operands that come out of inline asm or lane swaps
+__device__ __forceinline__ float vra_max(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ float vra_max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+__device__ __forceinline__ float pf_xor16_max(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  return vra_max(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float pf_xor32_max(float x) {
+  const unsigned u = __float_as_uint(x);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return vra_max(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
 
 template <class DT, int D, bool KV8, int MT>
 __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const PrefillAttnArgs a) {
@@ -160,7 +186,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
       blk[h] = tok < ctx ? table_entry(block_of(tok)) : 0u;
     }
   };
-  // thread -> chunks of the tile.  K: chunk i = n*256 + tid of [64 keys][KCH chunks]; V: chunk i of [D channels][8 chunks].
+  // thread -> chunks of the tile.  K: chunk i = n*256 + tid of [64 keys][KCH chunks]; V: four chunks of a 32-token half of 64 channels.
   // The 2*KLD loads of the next tile are NOT issued as one burst behind the barrier: all waves of the workgroup would
   // queue 32 KB at the CU's texture-address unit at the same moment and sit in the issue stall (1600 of 5500 cycles per
   // tile in the phase timers).  next_bases() computes the wave-uniform bases, the loads go out one by one between the MFMA
@@ -178,16 +204,19 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
     vb0 = c0 + off0;
     vb1 = c1 + off1;
   };
+  // (bases in scalar registers, one 32-bit offset a lane for K and one for V: K load n fetches 256 / KCH keys, V load n the half n & 1 of 64 channels — four
+  // lanes a channel, channels 0, 8, 1, 9, .. of a group of 16 in turn, so that the writes of a tile meet no LDS bank twice)
+  constexpr int KPL = PF_THREADS / KCH;
+  const int vch = ((tid >> 2) & 48) | (((tid >> 2) & 1) << 3) | ((tid >> 3) & 7);
+  const uint32_t klo = (uint32_t)((tid / KCH) * D + (tid % KCH) * 8) * (uint32_t)sizeof(kv_t);
+  const uint32_t vlo = (uint32_t)(vch * a.BS + (tid & 3) * 8) * (uint32_t)sizeof(kv_t);
   auto issue_k = [&](int n) {
-    const int i = n * PF_THREADS + tid;
-    const int key = i / KCH, c = i % KCH;
-    const bool h = ((n * PF_THREADS / KCH) >> 5) != 0;  // compile-time: 256 chunks never span two halves
-    kst[n] = *reinterpret_cast<const raw_t*>(kcache + (h ? kb1 : kb0) + (size_t)(key & 31) * D + c * 8);
+    const kv_t* const base = kcache + (((n * KPL) >> 5) ? kb1 : kb0) + ((n * KPL) & 31) * D;
+    kst[n] = *reinterpret_cast<const raw_t*>(reinterpret_cast<const unsigned char*>(base) + klo);
   };
   auto issue_v = [&](int n) {
-    const int i = n * PF_THREADS + tid;
-    const int ch = i >> 3, c = i & 7, h = c >> 2;
-    vst[n] = *reinterpret_cast<const raw_t*>(vcache + (h ? vb1 : vb0) + (size_t)ch * a.BS + (c & 3) * 8);
+    const kv_t* const base = vcache + ((n & 1) ? vb1 : vb0) + (size_t)((n >> 1) * 64) * (uint32_t)a.BS;
+    vst[n] = *reinterpret_cast<const raw_t*>(reinterpret_cast<const unsigned char*>(base) + vlo);
   };
   auto issue_loads = [&](int tile, const uint32_t (&blk)[2]) {
     next_bases(tile, blk);
@@ -209,7 +238,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
         *reinterpret_cast<u32x4*>(Ks + key * D + pf_kswz<D>(key, c) * 8) = widen(kst[n]);
       }
       {
-        const int ch = i >> 3, c = i & 7;
+        const int ch = (n >> 1) * 64 + vch, c = (n & 1) * 4 + (tid & 3);
         u32x4 v = widen(vst[n]);
         if (tail) {  // slots past the context hold arbitrary bits (0 * NaN = NaN): zero them
 #pragma unroll
@@ -252,10 +281,6 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
     // sub-tile u are issued (the MFMAs are volatile asm in program order: hipcc does not hoist the reads by itself, and
     // read -> wait -> 2 MFMAs left the matrix pipe idle for the LDS latency: 1577 cycles for 32 MFMAs)
     f32x4 s[MT][4];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-      for (int u = 0; u < 4; u++) s[mt][u] = vra_zero_acc();
     auto k_frags = [&](int u, u32x4 (&kf)[DJ]) {
       const int key = 32 * (u >> 1) + (rq >> 2) * 8 + (u & 1) * 4 + (rq & 3);
 #pragma unroll
@@ -272,7 +297,11 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
 #pragma unroll
         for (int j = 0; j < DJ; j++)
 #pragma unroll
-          for (int mt = 0; mt < MT; mt++) DT::mfma(s[mt][u], __builtin_bit_cast(s16x8, kfr[u & 1][j]), qf[mt][j]);
+          for (int mt = 0; mt < MT; mt++) {
+            const s16x8 kf = __builtin_bit_cast(s16x8, kfr[u & 1][j]);
+            if (j == 0) DT::mfma0(s[mt][u], kf, qf[mt][j]);
+            else DT::mfma_ready(s[mt][u], kf, qf[mt][j]);
+          }
       }
     }
     // the first V fragments are requested now: they land while the softmax runs
@@ -287,7 +316,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
     VRA_MFMA_DRAIN();  // s (and the previous tile's O updates) are complete past this point
     PF_STAMP(t5);
     // ---- softmax update, row tile by row tile; scores in the log2 domain.  The maximum is taken over the raw scores
-    // (scale > 0) and the scale rides in the FMA in front of the exp: exp2(s*c - m*c).
+    // (scale > 0) and the scale rides in the FMA in front of the exp: exp2(s*c - m).
     const bool need_mask = T0 + PF_KEYS - 1 > w_first_pos || T0 + PF_KEYS > ctx;  // wave-uniform
     s16x8 pf[MT][2];
     float x[MT][16], tmax[MT];
@@ -321,23 +350,23 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
     // row maxima of all row tiles together: in-lane, then the two cross-lane steps as VALU lane swaps (no LDS round trip)
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-      float m = x[mt][0];
+      float m = vra_max(x[mt][0], x[mt][1]);
 #pragma unroll
-      for (int e = 1; e < 16; e++) m = fmaxf(m, x[mt][e]);
+      for (int e = 2; e < 16; e += 2) m = vra_max3(m, x[mt][e], x[mt][e + 1]);
       tmax[mt] = m;
     }
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) tmax[mt] = vra_xor16_max(tmax[mt]);
+    for (int mt = 0; mt < MT; mt++) tmax[mt] = pf_xor16_max(tmax[mt]);
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) tmax[mt] = vra_xor32_max(tmax[mt]);
+    for (int mt = 0; mt < MT; mt++) tmax[mt] = pf_xor32_max(tmax[mt]);
     float alpha[MT];
-    bool moved = false;
+    bool moved[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-      const float m_new = fmaxf(m_run[mt], tmax[mt] * cs);
+      const float m_new = vra_max(m_run[mt], tmax[mt] * cs);
       const float m_safe = m_new == -INFINITY ? 0.f : m_new;
       alpha[mt] = __builtin_amdgcn_exp2f(m_run[mt] - m_safe);
-      moved = moved || alpha[mt] != 1.0f;
+      moved[mt] = alpha[mt] != 1.0f;
       float psum = 0.f;
 #pragma unroll
       for (int e = 0; e < 16; e++) {
@@ -356,15 +385,15 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
         pf[mt][h] = __builtin_bit_cast(s16x8, pa);
       }
     }
-    // rescale O (row rq is this lane's own row): skipped when no row of the wave moved its maximum
-    if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+    // rescale O (row rq is this lane's own row): a row tile is skipped when no row of it moved its maximum
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++)
+    for (int mt = 0; mt < MT; mt++)
+      if (__builtin_amdgcn_ballot_w64(moved[mt]) != 0) {
 #pragma unroll
         for (int t = 0; t < DT16; t++)
 #pragma unroll
           for (int r = 0; r < 4; r++) o[mt][t][r] *= alpha[mt];
-    }
+      }
     PF_STAMP(t6);
     // ---- O^T += V^T.P^T, the V fragments two channel tiles ahead of their MFMAs
 #pragma unroll
@@ -375,7 +404,10 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
 #pragma unroll
       for (int h = 0; h < 2; h++)
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) DT::mfma(o[mt][t], __builtin_bit_cast(s16x8, vfr[t % 3][h]), pf[mt][h]);
+        for (int mt = 0; mt < MT; mt++) {
+          if (t == 0) DT::mfma(o[mt][t], __builtin_bit_cast(s16x8, vfr[t % 3][h]), pf[mt][h]);
+          else DT::mfma_ready(o[mt][t], __builtin_bit_cast(s16x8, vfr[t % 3][h]), pf[mt][h]);
+        }
     }
     PF_STAMP(t7);
     sE += t5 - t4, sF += t6 - t5, sG += t7 - t6;
