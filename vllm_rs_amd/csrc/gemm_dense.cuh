@@ -175,7 +175,7 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
       zi = lin_sk - lin * SK;
       xtile = lin, xtiles = a.MT * a.NT;
     }
-    constexpr int GM = 8;
+    const int groups = max((a.MT + 4) >> 3, 1), GM = (a.MT + groups - 1) / groups;  // (equal groups: the weights come by once a group)
     const int per = GM * a.NT;
     const int grp = lin / per, rem = lin - grp * per;
     const int first = grp * GM, gsz = min(a.MT - first, GM);

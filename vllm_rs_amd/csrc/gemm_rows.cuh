@@ -62,22 +62,12 @@ __device__ __forceinline__ void gr_gather_columns(u32x2 (&v)[2]) {
   }
 }
 
-// tile of a workgroup: the ids of one XCD (id mod 8) take a contiguous run of an order that walks 8 tile rows before the next tile column, so the
-// workgroups of an XCD share their operands' panels in its L2
-__device__ __forceinline__ void gr_tile(const GemmRowsArgs& a, int& mt, int& nt) {
-  const int nwg = (int)gridDim.x, bid = (int)blockIdx.x, q = nwg >> 3, r = nwg & 7, xcd = bid & 7;
-  const int lin = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
-  constexpr int GM = 8;
-  const int per = GM * a.NT, grp = lin / per, rem = lin - grp * per, first = grp * GM, gsz = min(a.MT - first, GM);
-  mt = first + rem % gsz;
-  nt = rem / gsz;
-}
-
 // waves of a tile: two groups of four (rows 0 .. BM/2 - 1 and the others), CW of them side by side with 64 columns each
-template <int BM, int BN>
+template <int BM, int BN, bool DEEP>
 struct GrTile {
   static constexpr int H = BM == 256 ? 2 : 1;                           // phases of a K step (the upper, the lower rows of a wave)
-  static constexpr int S = BM == 256 ? 2 : (BM == 128 && BN == 128 ? 4 : 3);  // LDS buffers
+  static constexpr int KP = DEEP ? 2 : 1;                                     // K steps of a phase
+  static constexpr int S = BM == 256 ? 2 : (BM == 128 && BN == 128 ? 4 : 3);  // LDS buffers (of a phase's K steps)
   static constexpr int CW = BN / 64, RW = 4 / CW;
   static constexpr int NX = BM / 32 / RW / H;  // 16-row blocks of a wave in a phase
   static constexpr int XB = BM / 16, WB = BN / 16, STG = (XB + WB) * 2048;
@@ -87,18 +77,19 @@ struct GrTile {
 // EPI::store(m, seg, n0, N, q4, acc): the wave's 64 columns n0 .. n0 + 63 (of segment seg) of output row m; the lane holds columns n0 + 16 j + 4 q4 ..
 // + 3 in acc[j].  Called by all lanes (lanes beyond the matrix with m = -1), so that a lane may trade columns with its row's other three.
 // PAIR: w[0] and w[1] (gate, up; neither grouped nor batched) interleaved in blocks of 16 virtual columns, n[0] = virtual columns.
-template <class DT, int BM, int BN, bool PAIR, class EPI>
+template <class DT, int BM, int BN, bool DEEP, bool PAIR, class EPI>
 __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a, const EPI epi) {
 #ifdef __HIP_DEVICE_COMPILE__
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  using T = GrTile<BM, BN>;
-  constexpr int H = T::H, S = T::S, NX = T::NX, STG = T::STG, EX = T::EX, EW = T::EW, D = EX + EW;
+  using T = GrTile<BM, BN, DEEP>;
+  constexpr int H = T::H, KP = T::KP, S = T::S, NX = T::NX, STG = T::STG, EX = T::EX, EW = T::EW, D = EX + EW;
   static_assert(EW == 4 || EW == 2, "a wave has 64 columns");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wg = wave >> 2, cw = (wave & 3) % T::CW, rw = (wave & 3) / T::CW, r16 = lane & 15, q4 = lane >> 4;
-  // tile: the ids of one XCD (id mod 8) take a contiguous run of an order that walks 8 tile rows before the next tile column, so the
-  // workgroups of an XCD share their operands' panels in its L2.  Grouped rows: the empty tile rows are the last ones, so the XCDs take pairs of tile
+  // tile: the ids of one XCD (id mod 8) take a contiguous run of an order that walks about 8 tile rows before the next tile column, so the
+  // workgroups of an XCD share their operands' panels in its L2; the tile rows in equal groups (the weights come by once a group: with 8 + 1 tile
+  // rows of 64, 557 rows x 14336, K = 4096 99 us, with 9 77.5).  Grouped rows: the empty tile rows are the last ones, so the XCDs take pairs of tile
   // rows (an expert's, more often than not) in turn, whole, two rows to a column (16 experts of 188 rows, 2048 columns, 40 tile rows with 8 empty
   // ones: in runs two XCDs idle and the others work two rounds, K = 2048 / 1024 77.7 / 45.9 us; so 50.8 / 27.0)
   int mt, nt, group = 0;
@@ -111,7 +102,7 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
   } else {
     const int nwg = (int)gridDim.x, bid = (int)blockIdx.x, q = nwg >> 3, r = nwg & 7, xcd = bid & 7;
     const int lin = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
-    constexpr int GM = 8;
+    const int groups = max((a.MT + 4) >> 3, 1), GM = (a.MT + groups - 1) / groups;
     const int per = GM * a.NT, grp = lin / per, rem = lin - grp * per, first = grp * GM, gsz = min(a.MT - first, GM);
     mt = first + rem % gsz;
     nt = rem / gsz;
@@ -170,19 +161,19 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
   const int c0 = r16 * 128 + (q4 ^ (r16 & 7)) * 16, c1 = c0 ^ 64;
   const unsigned char* const xb = smem + row0 * 128;
   const unsigned char* const wb = smem + T::XB * 2048 + cw * 4 * 2048;
-  s16x8 xa[NX][2], wa[4][2];
-  auto read_x = [&](int o, int h) {
+  s16x8 xa[KP * NX][2], wa[KP * 4][2];
+  auto read_x = [&](int o, int h, int k = 0) {
 #pragma unroll
     for (int i = 0; i < NX; i++) {
-      xa[i][0] = *reinterpret_cast<const s16x8*>(xb + o + c0 + (h * NX + i) * 2048);
-      xa[i][1] = *reinterpret_cast<const s16x8*>(xb + o + c1 + (h * NX + i) * 2048);
+      xa[k * NX + i][0] = *reinterpret_cast<const s16x8*>(xb + o + c0 + (h * NX + i) * 2048);
+      xa[k * NX + i][1] = *reinterpret_cast<const s16x8*>(xb + o + c1 + (h * NX + i) * 2048);
     }
   };
-  auto read_w = [&](int o) {
+  auto read_w = [&](int o, int k = 0) {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-      wa[j][0] = *reinterpret_cast<const s16x8*>(wb + o + c0 + j * 2048);
-      wa[j][1] = *reinterpret_cast<const s16x8*>(wb + o + c1 + j * 2048);
+      wa[k * 4 + j][0] = *reinterpret_cast<const s16x8*>(wb + o + c0 + j * 2048);
+      wa[k * 4 + j][1] = *reinterpret_cast<const s16x8*>(wb + o + c1 + j * 2048);
     }
   };
   f32x4 acc[H * NX][4];
@@ -192,20 +183,24 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
     for (int j = 0; j < 4; j++) acc[i][j] = vra_zero_acc();
   // (a wave's 64 columns, a phase's rows: nothing of them in the matrix, no MFMAs)
   const bool in = n0 + cw * 64 < N && m0 + row0 < a.M, in1 = H == 2 && n0 + cw * 64 < N && m0 + row0 + NX * 16 < a.M;
-  auto compute = [&](auto HH) {
+  auto compute = [&](auto HH, int steps) {  // steps: of the phase's KP those that are within K
     constexpr int h = decltype(HH)::value;
     // the next phase's requests have landed (those of the last S - 2 steps, with two phases of the last step, may be on their way), this phase's reads are done
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(H == 2 ? D : (S - 2) * D) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(H == 2 ? D : (S - 2) * KP * D) : "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     if (h ? in1 : in) {
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int kc = 0; kc < 2; kc++)
+      for (int k = 0; k < KP; k++) {
+        if (k && k >= steps) break;
 #pragma unroll
-        for (int i = 0; i < NX; i++)
+        for (int kc = 0; kc < 2; kc++)
 #pragma unroll
-          for (int j = 0; j < 4; j++) DT::mfma_ready(acc[h * NX + i][j], wa[j][kc], xa[i][kc]);
+          for (int i = 0; i < NX; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) DT::mfma_ready(acc[h * NX + i][j], wa[k * 4 + j][kc], xa[k * NX + i][kc]);
+      }
       __builtin_amdgcn_s_setprio(0);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -228,11 +223,11 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
       __builtin_amdgcn_sched_barrier(0);
       read_x(o, 0);
       stage_x(STG - o, ks + 1, 2, 4);
-      compute(C0{});
+      compute(C0{}, 1);
       read_x(o, 1);
       stage_x(o, ks + 2, 0, 2);
       stage_w(o, ks + 2);
-      compute(C1{});
+      compute(C1{}, 1);
     };
     for (int ks = 0; ks < KT; ks += 2) {
       step(C0{}, ks);
@@ -240,20 +235,23 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
     }
   } else {
 #pragma unroll
-    for (int s = 0; s < S - 1; s++) stage_x(s * STG, s, 0, EX), stage_w(s * STG, s);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * D) : "memory");
+    for (int s = 0; s < (S - 1) * KP; s++) stage_x(s * STG, s, 0, EX), stage_w(s * STG, s);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * KP * D) : "memory");
     __builtin_amdgcn_s_barrier();
     if (wg == 1) __builtin_amdgcn_s_barrier();
-    int o = 0, p = (S - 1) * STG;  // buffers of this step and of the one before it
-    for (int ks = 0; ks < KT; ks++) {
-      read_w(o);
-      read_x(o, 0);
+    int o = 0, p = (S - 1) * KP * STG;  // buffers of this phase and of the one before it
+    for (int ks = 0; ks < KT; ks += KP) {
+#pragma unroll
+      for (int k = 0; k < KP; k++) read_w(o + k * STG, k), read_x(o + k * STG, 0, k);
       __builtin_amdgcn_sched_barrier(0);
-      stage_x(p, ks + S - 1, 0, EX);
-      stage_w(p, ks + S - 1);
-      compute(C0{});
+#pragma unroll
+      for (int k = 0; k < KP; k++) {
+        stage_x(p + k * STG, ks + (S - 1) * KP + k, 0, EX);
+        stage_w(p + k * STG, ks + (S - 1) * KP + k);
+      }
+      compute(C0{}, KT - ks);
       p = o;
-      o = o == (S - 1) * STG ? 0 : o + STG;
+      o = o == (S - 1) * KP * STG ? 0 : o + KP * STG;
     }
   }
   if (wg == 0) __builtin_amdgcn_s_barrier();
@@ -269,13 +267,14 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
 #endif
 }
 
-// Tile for a product of M rows x ncols[0..nseg) columns x `batch`: the least time by this model (us; 198 shapes of 64..8192 rows, 2048..14336 columns,
-// K = 1024..14336, weights from memory: within 4..7 % rms): workgroups run in rounds of `slots`; a launch costs t0, a round `round` (first
-// requests, outputs) and `full` for 64 of K, the last round between `one` (a few workgroups) and `full`.  rows: only tiles of that many (0: any).
+// Tile for a product of M rows x ncols[0..nseg) columns x `batch`: the least time by this model (us; 225 shapes of 33..8192 rows, 2048..14336 columns,
+// K = 1024..14336, weights from memory: within 2..8 % rms, and the tile it picks 0.2 % behind the best on average, 7 % at most): workgroups
+// run in rounds of `slots`; a launch costs t0, a round `round` (first requests, outputs) and `full` for 64 of K, the last round between `one` (a
+// few workgroups) and `full`.  64 x 128 has two forms (gemm_rows_launch).  rows: only tiles of that many (0: any).
 // -> rows / 64 * 16 + columns / 64; *us: the time
 static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch, int K, int rows = 0, double* us = nullptr) {
-  const struct { int bm, bn, slots; double t0, round, one, full; } t[4] = {
-      {256, 256, 256, 3.1, 13.7, 0.80, 1.41}, {128, 256, 256, 1.6, 8.7, 0.54, 0.82}, {128, 128, 256, 1.4, 5.3, 0.33, 0.50}, {64, 128, 512, 2.0, 2.7, 0.28, 0.58}};
+  const struct { int bm, bn, slots; double t0, round, one, full; } t[5] = {{256, 256, 256, 2.0, 14.4, 0.79, 1.39}, {128, 256, 256, 0.7, 9.5, 0.52, 0.78},
+      {128, 128, 256, 1.4, 5.4, 0.35, 0.50}, {64, 128, 512, 2.6, 2.4, 0.27, 0.60}, {64, 128, 256, 3.7, 1.3, 0.28, 0.34}};
   int best = 0;
   double cost = 0.0;
   for (const auto& c : t) {
@@ -283,7 +282,10 @@ static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch,
     long cols = 0;
     for (int s = 0; s < nseg; s++) cols += (ncols[s] + c.bn - 1) / c.bn;
     const long tiles = (M + c.bm - 1) / c.bm * cols * batch, full = tiles / c.slots, rem = tiles % c.slots;
-    const double v = c.t0 + (full + (rem ? 1 : 0)) * c.round + K / 64 * (full * c.full + (rem ? c.one + (c.full - c.one) * rem / c.slots : 0.0));
+    if (c.bm == 64 && (tiles <= 256) != (c.slots == 256)) continue;
+    double last = rem ? c.one + (c.full - c.one) * rem / c.slots : 0.0;
+    if (c.slots == 512 && rem) last = rem <= 256 ? c.one : 0.46 + (c.full - 0.46) * (rem - 256) / 256;  // (the second workgroup of a CU)
+    const double v = c.t0 + (full + (rem ? 1 : 0)) * c.round + K / 64 * (full * c.full + last);
     if (!best || v < cost) best = c.bm / 64 * 16 + c.bn / 64, cost = v;
   }
   if (us) *us = cost;
@@ -291,7 +293,7 @@ static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch,
 }
 static inline bool gemm_rows_has_tile(int tile, int K) { return (tile == 4 * 16 + 4 && K % 128 == 0) || tile == 2 * 16 + 4 || tile == 2 * 16 + 2 || tile == 16 + 2; }
 // fills the tile counts and launches
-template <class DT, int BM, int BN, bool PAIR, class EPI>
+template <class DT, int BM, int BN, bool DEEP, bool PAIR, class EPI>
 static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStream_t st) {
   a.MT = (a.M + BM - 1) / BM;
   a.NT = 0;
@@ -300,18 +302,23 @@ static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStr
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (!((attr_devs >> (dev & 63)) & 1)) {
-    void (*const k)(GemmRowsArgs, EPI) = gemm_rows_kernel<DT, BM, BN, PAIR, EPI>;
+    void (*const k)(GemmRowsArgs, EPI) = gemm_rows_kernel<DT, BM, BN, DEEP, PAIR, EPI>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr_devs |= (uint64_t)1 << (dev & 63);
   }
-  using T = GrTile<BM, BN>;
+  using T = GrTile<BM, BN, DEEP>;
   const int rows = a.tile_group ? (a.MT + 15) / 16 * 16 : a.MT;  // (pairs of tile rows by eight XCDs)
-  gemm_rows_kernel<DT, BM, BN, PAIR, EPI><<<dim3((unsigned)(rows * a.NT), (unsigned)batch), dim3(512), (size_t)T::S * T::STG, st>>>(a, epi);
+  gemm_rows_kernel<DT, BM, BN, DEEP, PAIR, EPI><<<dim3((unsigned)(rows * a.NT), (unsigned)batch), dim3(512), (size_t)T::S * T::KP * T::STG, st>>>(a, epi);
 }
+// 64 x 128: two K steps a phase and twice the LDS where every workgroup has a CU to itself, otherwise two workgroups a CU.  (A phase of one step is two
+// waits for LDS around 8 MFMAs a wave: 64 rows x 4096, K = 14336, 32 workgroups 79.7 us, six buffers 73.2, so 69.6; with the waves in step 94.4.)
 template <class DT, bool PAIR, class EPI>
 static void gemm_rows_launch(const GemmRowsArgs& a, const EPI& epi, int tile, int batch, hipStream_t st) {
-  if (tile == 4 * 16 + 4) gemm_rows_launch_t<DT, 256, 256, PAIR>(a, epi, batch, st);
-  else if (tile == 2 * 16 + 4) gemm_rows_launch_t<DT, 128, 256, PAIR>(a, epi, batch, st);
-  else if (tile == 2 * 16 + 2) gemm_rows_launch_t<DT, 128, 128, PAIR>(a, epi, batch, st);
-  else gemm_rows_launch_t<DT, 64, 128, PAIR>(a, epi, batch, st);
+  if (tile == 4 * 16 + 4) return gemm_rows_launch_t<DT, 256, 256, false, PAIR>(a, epi, batch, st);
+  if (tile == 2 * 16 + 4) return gemm_rows_launch_t<DT, 128, 256, false, PAIR>(a, epi, batch, st);
+  if (tile == 2 * 16 + 2) return gemm_rows_launch_t<DT, 128, 128, false, PAIR>(a, epi, batch, st);
+  long cols = 0;
+  for (int s = 0; s < a.nseg; s++) cols += (a.n[s] + 127) / 128;
+  if ((a.M + 63) / 64 * cols * batch <= 256) gemm_rows_launch_t<DT, 64, 128, true, PAIR>(a, epi, batch, st);
+  else gemm_rows_launch_t<DT, 64, 128, false, PAIR>(a, epi, batch, st);
 }
