@@ -258,7 +258,8 @@ __global__ __launch_bounds__(256) void stk_scale_rows_kernel(const uint16_t* a, 
 }
 
 // ------------------------------------------------------------------------------------------------ GEMM, f32 FMA (any shape)
-// 256 threads: 16 (m) x 16 (n) threads, RM rows x 4 columns each; K in steps of 16 through LDS; k ascending: one fixed order.
+// 256 threads: 16 (m) x 16 (n) threads, RM rows x 4 columns each; K in steps of 16 through LDS; k ascending: one fixed order.  For rows off
+// 16 bytes (f32; bf16 where the matrix form does not take the product).
 template <typename T, int RM>
 __global__ __launch_bounds__(256) void stk_gemm_simple_kernel(StkGemmArgs g) {
   constexpr int TM = 16 * RM;
@@ -323,6 +324,140 @@ __global__ __launch_bounds__(256) void stk_gemm_simple_kernel(StkGemmArgs g) {
       if (g.out_f32) ((float*)g.out)[ob + (int64_t)orow * g.ldo + n] = v;
       else El<T>::st((T*)g.out + ob + (int64_t)orow * g.ldo + n, v);
     }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------ GEMM, f32 MFMA (16-byte rows)
+// A wave is a workgroup and owns MT x NT tiles of 16 x 16 of v_mfma_f32_16x16x4_f32 (weights = A, rows = B: a lane ends with 4 consecutive columns of
+// one row).  That instruction adds its four products one after the other, each fused: the bits of the chain above, k ascending.  Lane (r, q) loads 16
+// bytes of its row a block of 16 k, P blocks ahead, into registers: no LDS, no barrier; lane swaps, which run under the matrix instructions, then put
+// k = 4 s + q where step s reads it.
+// Bound: the loads' addresses (16 rows of 64 bytes each, 64 clocks a load for a CU), about half the matrix units' 157 TFLOP/s; few rows, the chain of
+// a lone wave.  us, the form above -> this, launch included: 2 rows, 2048 x 2048 198 -> 20, K = 8192 805 -> 61, 32000 columns 326 -> 56;
+// 342 rows, 8192 x 2048 479 -> 174; 2048 rows, 1486 -> 915.
+template <int MT, int NT, int P, bool SCALED>
+__global__ __launch_bounds__(64) void stk_gemm_f32_kernel(StkGemmArgs g) {
+  const int lane = threadIdx.x, r16 = lane & 15, q4 = lane >> 4;
+  const int m0 = (int)blockIdx.x * 16 * MT, n0 = (int)blockIdx.y * 16 * NT;
+  int group = 0;
+  if (g.tile_group) {
+    group = g.tile_group[m0 / g.granule];
+    if (group < 0) return;
+  }
+  const float* const A = (const float*)g.a + (int64_t)blockIdx.z * g.a_batch_stride;
+  const float* const Wt = (const float*)g.w + (int64_t)group * g.w_group_stride + (int64_t)blockIdx.z * g.w_batch_stride;
+  const float *xp[MT], *wp[NT];
+  float sc[MT];
+  int orow[MT];  // -1: nothing to store
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    const int row = m0 + i * 16 + r16, idx = row < g.M ? (g.a_row ? g.a_row[row] : row) : -1;
+    xp[i] = A + (int64_t)max(idx, 0) * g.lda + q4 * 4;
+    sc[i] = SCALED && idx >= 0 ? g.a_scale[row] : 1.f;
+    orow[i] = idx < 0 ? -1 : (g.out_row ? g.out_row[row] : row);
+  }
+#pragma unroll
+  for (int j = 0; j < NT; j++) wp[j] = Wt + (int64_t)min(n0 + j * 16 + r16, g.N - 1) * g.K + q4 * 4;
+  f32x4 x[P][MT], w[P][NT];
+  auto fetch = [&](int off, int u) {
+#pragma unroll
+    for (int i = 0; i < MT; i++) x[u][i] = *(const f32x4*)(xp[i] + off * 16);
+#pragma unroll
+    for (int j = 0; j < NT; j++) w[u][j] = *(const f32x4*)(wp[j] + off * 16);
+  };
+  auto turn = [](f32x4& v) {  // value s of lane (r, q): from value q of lane (r, s)
+    float v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3];
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1\n\t"
+                 "v_permlane16_swap_b32 %0, %1\n\tv_permlane16_swap_b32 %2, %3" : "+v"(v0), "+v"(v1), "+v"(v2), "+v"(v3));
+    v = f32x4{v0, v1, v2, v3};
+  };
+  auto turn_x = [&](int u) {
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      if (SCALED) x[u][i] *= sc[i];
+      turn(x[u][i]);
+    }
+  };
+  auto turn_w = [&](int u) {
+#pragma unroll
+    for (int j = 0; j < NT; j++) turn(w[u][j]);
+  };
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; i++)
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int u, int s) {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+        asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(w[u][j][s]), "v"(x[u][i][s]));
+  };
+  const int KF = g.K >> 4;  // whole blocks
+  int left = KF;
+  if (KF >= 2 * P) {
+#pragma unroll
+    for (int u = 0; u < P; u++) fetch(u, u);
+    turn_x(0), turn_w(0);
+    asm volatile("s_nop 1");
+    do {
+#pragma unroll
+      for (int u = 0; u < P; u++) {
+        step(u, 0);
+        turn_x((u + 1) % P);
+        step(u, 1);
+        turn_w((u + 1) % P);
+        step(u, 2);
+        step(u, 3);
+        fetch(P + u, u);
+      }
+#pragma unroll
+      for (int i = 0; i < MT; i++) xp[i] += P * 16;
+#pragma unroll
+      for (int j = 0; j < NT; j++) wp[j] += P * 16;
+      left -= P;
+    } while (left >= 2 * P);
+  } else {
+#pragma unroll
+    for (int u = 0; u < P; u++)
+      if (u < KF) fetch(u, u);
+    if (KF) turn_x(0), turn_w(0);
+  }
+#pragma unroll
+  for (int u = 0; u < 2 * P; u++) {
+    if (u < left) {
+      asm volatile("s_nop 1");
+#pragma unroll
+      for (int s = 0; s < 4; s++) step(u % P, s);
+      if (u < P && u + P < left) fetch(P + u, u);
+      if (u + 1 < left) turn_x((u + 1) % P), turn_w((u + 1) % P);
+    }
+  }
+  if (g.K & 15) {  // (K % 4 == 0: a lane's four values are inside or beyond K together; zeros add nothing)
+    const bool in = KF * 16 + q4 * 4 < g.K;
+#pragma unroll
+    for (int i = 0; i < MT; i++) x[0][i] = in ? *(const f32x4*)(xp[i] + left * 16) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NT; j++) w[0][j] = in ? *(const f32x4*)(wp[j] + left * 16) : f32x4{0.f, 0.f, 0.f, 0.f};
+    turn_x(0), turn_w(0);
+    asm volatile("s_nop 1");
+#pragma unroll
+    for (int s = 0; s < 4; s++) step(0, s);
+  }
+  VRA_MFMA_DRAIN();
+  const int64_t ob = (int64_t)blockIdx.z * g.out_batch_stride;
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    if (orow[i] < 0) continue;
+    float* const o = (float*)g.out + ob + (int64_t)orow[i] * g.ldo;
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int n = n0 + j * 16 + q4 * 4 + e;
+        if (n < g.N) o[n] = plain_value(g, acc[i][j][e] * g.alpha + (g.bias ? g.bias[(int64_t)blockIdx.z * g.bias_batch_stride + n] : 0.f));
+      }
   }
 }
 
@@ -1543,6 +1678,22 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
   }
   VRA_CHECK_ARG(!g.tile, "stack gemm: no such tile for this product");
   VRA_CHECK_ARG(!g.tile_group || g.granule != 128, "stack gemm: granules of 128 rows are for bf16 products on the matrix cores");
+  if (dtype == VRA_F32 && g.K % 4 == 0 && g.lda % 4 == 0 && (uintptr_t)g.a % 16 == 0 && (uintptr_t)g.w % 16 == 0 && g.w_group_stride % 4 == 0 && g.a_batch_stride % 4 == 0 &&
+      g.w_batch_stride % 4 == 0) {
+    // The tile with the least time a block of 16 k: 64 clocks for each load of the waves of a CU, a lone wave's 240, 400 or 700 at the least.  us of
+    // 16 x 16, 32 x 16, 32 x 32 tiles: 64 rows, 2048 x 2048: 21.6, 29.0, 46.0; 128 rows, 3072 x 2048: 50.2, 39.0, 47.9; 342 rows, 8192 x 2048: 313, 264, 175
+    auto waves = [&](int rows, int cols) { return ((int64_t)(g.M + rows - 1) / rows * ((g.N + cols - 1) / cols) * nb + 255) / 256; };
+    const int64_t t11 = std::max<int64_t>(waves(16, 16) * 128, 240), t21 = std::max<int64_t>(waves(32, 16) * 192, 400), t22 = std::max<int64_t>(waves(32, 32) * 256, 700);
+    const bool whole = !g.tile_group || g.granule >= 64;  // (row tiles of 32 lie in one group)
+    auto go = [&](auto scaled) {
+      constexpr bool S = decltype(scaled)::value;
+      if (whole && t22 <= std::min(t11, t21)) stk_gemm_f32_kernel<2, 2, 8, S><<<dim3((g.M + 31) / 32, (g.N + 31) / 32, nb), 64, 0, st>>>(g);
+      else if (whole && t21 < t11) stk_gemm_f32_kernel<2, 1, 8, S><<<dim3((g.M + 31) / 32, (g.N + 15) / 16, nb), 64, 0, st>>>(g);
+      else stk_gemm_f32_kernel<1, 1, 12, S><<<dim3((g.M + 15) / 16, (g.N + 15) / 16, nb), 64, 0, st>>>(g);
+    };
+    launch_checked("stack gemm", [&] { g.a_scale ? go(std::true_type{}) : go(std::false_type{}); });
+    return;
+  }
   if (big) {
     dim3 grid((g.M + 63) / 64, (g.N + 63) / 64, nb);
     if (dtype == VRA_F32) launch_checked("stack gemm", [&] { stk_gemm_simple_kernel<float, 4><<<grid, 256, 0, st>>>(g); });
