@@ -60,10 +60,25 @@ __global__ __launch_bounds__(256) void stk_embed_sinpos_kernel(const uint32_t* i
   }
 }
 
+// a fold over the wave's lanes in wave_sum's order, without LDS: after the exchange at distance 8 the values of 16 lanes repeat every 8, so a rotation by 4
+// is the exchange at distance 4, and so on
+template <class F>
+__device__ __forceinline__ float wave_fold(float v, F f) {
+  auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  v = f(v, vra_dpp_f<0x128>(v));  // row_ror:8, 4, 2, 1
+  v = f(v, vra_dpp_f<0x124>(v));
+  v = f(v, vra_dpp_f<0x122>(v));
+  return f(v, vra_dpp_f<0x121>(v));
+}
+
 // ------------------------------------------------------------------------------------------------ grouped RMS norm (+ router)
 // (ROUTER a template parameter and 8 waves a SIMD: a norm that carries the router's registers, or a router with the 74 it would take, leaves room for 6
 // waves, and 2048 rows are two rounds of workgroups.  2048 rows, us: norm of 2048 7.6 -> 6.8, of 2051 12.4 -> 9.5; with eight router
-// outputs 21.1 -> 19.1, of 1001 17.6 -> 13.3)
+// outputs 21.1 -> 19.1, of 1001 17.6 -> 13.3.  The picks by a wave and not by one thread, five outputs of a wave and not four in a round: 1500 rows of
+// 2048, 16 outputs and a gate 22.0 -> 15.2; 64 outputs, eight picks 76.6 -> 21.7; 160 outputs 163 -> 74)
 template <typename T, bool ROUTER>
 __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
   extern __shared__ float lds[];
@@ -71,7 +86,7 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
   float* rs = lds + a.W;                // [groups] 1 / rms
   float* zs = rs + a.groups;            // [n_router + gate_row]
   const int t = blockIdx.x, W = a.W, gs = W / a.groups;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const float* x = a.x + (size_t)t * W;
   T* h = (T*)a.h + (size_t)t * W;
   auto sums = [&] {
@@ -90,21 +105,50 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
   const float gt = a.gate_in ? a.gate_in[t] : 1.f;
   const bool quads = W % 4 == 0 && gs % 4 == 0 && (((uintptr_t)a.x | (uintptr_t)a.x_out | (uintptr_t)a.o | (uintptr_t)a.p1 | (uintptr_t)a.p2 | (uintptr_t)a.w) % 16) == 0;
   if (quads) {
-    // (four values a load where rows and groups allow it, the weights with them: a row's parts arrive in one round trip instead of W / 256, and the
-    // row stays in registers: 8 rows of 2048: 6.6 us, now 4.0)
+    // (four values a load where rows and groups allow it, two loads of every part of the row ahead of the first sum: its parts arrive in one round trip
+    // instead of one a part, and the row stays in registers: 8 rows of 2048: 6.6 us, now 4.0; 1500 rows of 2048 with two experts' and a shared
+    // expert's parts, with the router 29.4, now 22.5)
     constexpr int R = 2;
     f32x4 keep[R], wt[R];
-    auto load = [&](int c) {
-      f32x4 v = *(const f32x4*)(x + c);
+    auto load = [&](int c0, f32x4 (&v)[R]) {  // (values beyond the row: the last ones again, not kept)
+      f32x4 s[R], s1[R], s2[R], s3[R];
+      int c[R];
+#pragma unroll
+      for (int n = 0; n < R; n++) c[n] = min(c0 + n * 1024, W - 4);
+      auto read = [&](const float* p, f32x4 (&d)[R]) {
+#pragma unroll
+        for (int n = 0; n < R; n++) d[n] = *(const f32x4*)(p + c[n]);
+      };
+      auto add = [&](const f32x4 (&d)[R]) {
+#pragma unroll
+        for (int n = 0; n < R; n++) s[n] += d[n];
+      };
+      read(x, v);
       if (a.o) {
-        f32x4 s = *(const f32x4*)(a.o + (size_t)t * W + c);
-        for (int j = 0; j < a.n1; j++) s += *(const f32x4*)(a.p1 + ((size_t)t * a.n1 + j) * W + c);
-        if (a.p2) s += gt * *(const f32x4*)(a.p2 + (size_t)t * W + c);
-        v += a.mult * s;
-        *(f32x4*)(a.x_out + (size_t)t * W + c) = v;
+        const float* const p1 = a.p1 + (size_t)t * a.n1 * W;
+        read(a.o + (size_t)t * W, s);
+        if (a.n1 > 0) read(p1, s1);
+        if (a.n1 > 1) read(p1 + W, s2);
+        if (a.p2) read(a.p2 + (size_t)t * W, s3);
+        if (a.n1 > 0) add(s1);
+        if (a.n1 > 1) add(s2);
+        for (int j = 2; j < a.n1; j++) {
+          read(p1 + (size_t)j * W, s1);
+          add(s1);
+        }
+        if (a.p2) {
+#pragma unroll
+          for (int n = 0; n < R; n++) s[n] += gt * s3[n];
+        }
+#pragma unroll
+        for (int n = 0; n < R; n++) v[n] += a.mult * s[n];
       }
-      *(f32x4*)(xs + c) = v;
-      return v;
+#pragma unroll
+      for (int n = 0; n < R; n++)
+        if (c0 + n * 1024 < W) {
+          *(f32x4*)(xs + c0 + n * 1024) = v[n];
+          if (a.o) *(f32x4*)(a.x_out + (size_t)t * W + c0 + n * 1024) = v[n];
+        }
     };
     auto put = [&](int c, f32x4 v, f32x4 w) {
       const f32x4 y = v * rs[c / gs] * w;
@@ -112,12 +156,16 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; e++) El<T>::st(h + c + e, y[e]);
     };
+    for (int c = threadIdx.x * 4 + R * 1024; c < W; c += R * 1024) {
+      f32x4 v[R];
+      load(c, v);  // (ahead of what stays in registers)
+    }
+    load(threadIdx.x * 4, keep);
 #pragma unroll
     for (int n = 0; n < R; n++) {
       const int c = threadIdx.x * 4 + n * 1024;
-      if (c < W) wt[n] = *(const f32x4*)(a.w + c), keep[n] = load(c);
+      if (c < W) wt[n] = *(const f32x4*)(a.w + c);
     }
-    for (int c = threadIdx.x * 4 + R * 1024; c < W; c += 1024) load(c);
     sums();
 #pragma unroll
     for (int n = 0; n < R; n++) {
@@ -150,28 +198,32 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
   const int nz = a.n_router + (a.gate_row ? 1 : 0);
   const T* rw = (const T*)a.router_w;
   if (sizeof(T) == 2 && W % 8 == 0 && ((uintptr_t)rw % 16) == 0) {  // 8 weights a load; the lane's partial sums keep one order for a given W
-    for (int e0 = wave; e0 < nz; e0 += 16) {  // four outputs of a wave side by side: their weights are under way together, the row is read once
-      float s[4] = {0.f, 0.f, 0.f, 0.f};
+    constexpr int Q = 5;
+    for (int e0 = wave; e0 < nz; e0 += 4 * Q) {  // up to five outputs of a wave side by side: their weights are under way together, the row is read once
+      float s[Q] = {};
       for (int c = lane * 8; c < W; c += 64 * 8) {
-        u32x4 v[4];
+        u32x4 v[Q];
 #pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = *(const u32x4*)((const uint16_t*)rw + (size_t)min(e0 + q * 4, nz - 1) * W + c);
+        for (int q = 0; q < Q; q++)
+          if (e0 + q * 4 < nz) v[q] = *(const u32x4*)((const uint16_t*)rw + (size_t)(e0 + q * 4) * W + c);
         float f[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) f[i] = xs[c + i];
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+        for (int q = 0; q < Q; q++)
+          if (e0 + q * 4 < nz)
 #pragma unroll
-          for (int i = 0; i < 4; i++) {
-            s[q] = fmaf(f[2 * i], __uint_as_float(v[q][i] << 16), s[q]);
-            s[q] = fmaf(f[2 * i + 1], __uint_as_float(v[q][i] & 0xffff0000u), s[q]);
-          }
+            for (int i = 0; i < 4; i++) {
+              s[q] = fmaf(f[2 * i], __uint_as_float(v[q][i] << 16), s[q]);
+              s[q] = fmaf(f[2 * i + 1], __uint_as_float(v[q][i] & 0xffff0000u), s[q]);
+            }
       }
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        s[q] = wave_sum(s[q]);
-        if (lane == 0 && e0 + q * 4 < nz) zs[e0 + q * 4] = s[q];
-      }
+      for (int q = 0; q < Q; q++)
+        if (e0 + q * 4 < nz) {
+          s[q] = wave_fold(s[q], [](float p, float r) { return p + r; });
+          if (lane == 0) zs[e0 + q * 4] = s[q];
+        }
     }
   } else {
     for (int e = wave; e < nz; e += 4) {
@@ -182,7 +234,37 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
     }
   }
   __syncthreads();
-  // the picks, by one thread from LDS (the row is not needed any more: its place holds the marks)
+  if (a.gate_row && threadIdx.x == 255) a.gate_out[t] = sigmoidf_(zs[a.n_router]);
+  if (wave != 0) return;
+  if (a.n_router <= 4096) {  // the picks, by one wave: the largest of what is left, the first of equal ones; a NaN counts only where it comes first
+    constexpr int NONE = 0x7fffffff;
+    auto least = [&](int v) -> int {
+      if (a.n_router <= 64) return __builtin_ctzll(__ballot(v != NONE));  // (a lane's value is its number)
+      return __float_as_int(wave_fold(__int_as_float(v), [](float p, float r) { return __int_as_float(min(__float_as_int(p), __float_as_int(r))); }));
+    };
+    uint64_t taken = 0;  // bit i: output lane + 64 i
+    for (int j = 0; j < a.top; j++) {
+      int first = NONE, at = NONE;
+      float m = -INFINITY;
+      for (int e = lane, i = 0; e < a.n_router; e += 64, i++) {
+        if (taken >> i & 1) continue;
+        const float z = zs[e];
+        first = min(first, e);
+        if (z > m || (at == NONE && z == m)) m = z, at = e;
+      }
+      int best = least(first);
+      float bz = zs[best];
+      if (!__builtin_isnan(bz)) {
+        bz = wave_fold(m, [](float p, float r) { return fmaxf(p, r); });
+        best = least(m == bz ? at : NONE);
+        bz = zs[best];
+      }
+      if (lane == (best & 63)) taken |= 1ull << (best >> 6);
+      if (lane == 0) a.pair_expert[(size_t)t * a.top + j] = best, a.pair_weight[(size_t)t * a.top + j] = sigmoidf_(bz);
+    }
+    return;
+  }
+  // (more outputs: by one thread from LDS; the row is not needed any more, its place holds the marks)
   if (threadIdx.x == 0) {
     int* taken = (int*)xs;
     const bool marks = a.n_router <= W;  // (more outputs than channels: look the earlier picks up)
@@ -201,7 +283,6 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
       a.pair_expert[(size_t)t * a.top + j] = best;
       a.pair_weight[(size_t)t * a.top + j] = sigmoidf_(bz);
     }
-    if (a.gate_row) a.gate_out[t] = sigmoidf_(zs[a.n_router]);
   }
 }
 
