@@ -268,13 +268,15 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
 }
 
 // Tile for a product of M rows x ncols[0..nseg) columns x `batch`: the least time by this model (us; 225 shapes of 33..8192 rows, 2048..14336 columns,
-// K = 1024..14336, weights from memory: within 2..8 % rms, and the tile it picks 0.2 % behind the best on average, 7 % at most): workgroups
+// K = 1024..14336, weights from memory: within 2..8 % rms, and the tile it picks 0.2 % behind the best on average, 6 % at most): workgroups
 // run in rounds of `slots`; a launch costs t0, a round `round` (first requests, outputs) and `full` for 64 of K, the last round between `one` (a
-// few workgroups) and `full`.  64 x 128 has two forms (gemm_rows_launch).  rows: only tiles of that many (0: any).
+// few workgroups) and `full`.  64 x 128 has two forms (gemm_rows_launch).  192 x 128 is for what is a little more than one round of 128 x 128 and leaves
+// much of one of 128 x 256 idle; us without / with it: 2120 rows x 2048, K = 2048 31.7 / 26.5, K = 5632 67.2 / 56.2; 700 x 8192, K = 2048 35.1 / 30.5;
+// 300 x 14336, K = 4096 51.1 / 44.7; 1280 x 4096, K = 14336 163 / 135.  rows: only tiles of that many (0: any).
 // -> rows / 64 * 16 + columns / 64; *us: the time
 static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch, int K, int rows = 0, double* us = nullptr) {
-  const struct { int bm, bn, slots; double t0, round, one, full; } t[5] = {{256, 256, 256, 2.0, 14.4, 0.79, 1.39}, {128, 256, 256, 0.7, 9.5, 0.52, 0.78},
-      {128, 128, 256, 1.4, 5.4, 0.35, 0.50}, {64, 128, 512, 2.6, 2.4, 0.27, 0.60}, {64, 128, 256, 3.7, 1.3, 0.28, 0.34}};
+  const struct { int bm, bn, slots; double t0, round, one, full; } t[6] = {{256, 256, 256, 2.0, 14.4, 0.79, 1.39}, {128, 256, 256, 0.7, 9.5, 0.52, 0.78},
+      {192, 128, 256, 1.0, 6.5, 0.40, 0.64}, {128, 128, 256, 1.4, 5.4, 0.35, 0.50}, {64, 128, 512, 2.6, 2.4, 0.27, 0.60}, {64, 128, 256, 3.7, 1.3, 0.28, 0.34}};
   int best = 0;
   double cost = 0.0;
   for (const auto& c : t) {
@@ -291,7 +293,7 @@ static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch,
   if (us) *us = cost;
   return best;
 }
-static inline bool gemm_rows_has_tile(int tile, int K) { return (tile == 4 * 16 + 4 && K % 128 == 0) || tile == 2 * 16 + 4 || tile == 2 * 16 + 2 || tile == 16 + 2; }
+static inline bool gemm_rows_has_tile(int tile, int K) { return (tile == 4 * 16 + 4 && K % 128 == 0) || tile == 2 * 16 + 4 || tile == 3 * 16 + 2 || tile == 2 * 16 + 2 || tile == 16 + 2; }
 // fills the tile counts and launches
 template <class DT, int BM, int BN, bool DEEP, bool PAIR, class EPI>
 static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStream_t st) {
@@ -316,6 +318,7 @@ template <class DT, bool PAIR, class EPI>
 static void gemm_rows_launch(const GemmRowsArgs& a, const EPI& epi, int tile, int batch, hipStream_t st) {
   if (tile == 4 * 16 + 4) return gemm_rows_launch_t<DT, 256, 256, false, PAIR>(a, epi, batch, st);
   if (tile == 2 * 16 + 4) return gemm_rows_launch_t<DT, 128, 256, false, PAIR>(a, epi, batch, st);
+  if (tile == 3 * 16 + 2) return gemm_rows_launch_t<DT, 192, 128, false, PAIR>(a, epi, batch, st);
   if (tile == 2 * 16 + 2) return gemm_rows_launch_t<DT, 128, 128, false, PAIR>(a, epi, batch, st);
   long cols = 0;
   for (int s = 0; s < a.nseg; s++) cols += (a.n[s] + 127) / 128;
