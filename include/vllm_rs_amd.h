@@ -159,7 +159,7 @@ void vra_wna16_dequant_frag(const void* qweight_tiled, const void* scales, const
                             int32_t group_size, int32_t is_awq, int32_t scales_layout, int32_t dtype, int32_t vfrag0,
                             int32_t vstride, int64_t stream);
 /* out[m, n] = x[m, k] . wd (+ bias, + residual; roundings as vra_wna16_gemm).  nv = columns of wd; dual != 0: wd interleaves gate and up
- * fragments, out[m, nv/2] = silu(x.Wg) * (x.Wu) (mlp.rs:451-469; no bias).  tile_n: 0 (chosen from the shape), 128 or 256. */
+ * fragments, out[m, nv/2] = silu(x.Wg) * (x.Wu) (mlp.rs:451-469; no bias).  tile_n: 0 (chosen from the shape), 128, 256 or 192 (rows of 256 columns). */
 void vra_dense_frag_gemm(const void* x, const void* wd, const void* bias, const void* residual, void* out, int32_t m, int32_t k,
                          int32_t nv, int32_t dual, int32_t dtype, int32_t tile_n, int64_t stream);
 

@@ -11,7 +11,7 @@
 //
 // Roofline: MFMA (2.5 PFLOP/s dense bf16).  Algorithmic FLOPs 2*M*K*N; bytes K*N*(0.5 + 2 + 2) + M*K*2 + M*N*2.
 //
-// Shape of the GEMM launch (256 x BN output tile, 8 waves = 2 (m) x 4 (n), one workgroup per CU, K-step 64):
+// Shape of the GEMM launch (BM x BN output tile: 256 x 256, 256 x 128 or, three fragments of 16 rows a wave and phase instead of four, 192 x 256; 8 waves = 2 (m) x 4 (n), one workgroup per CU, K-step 64):
 //   * both operands travel global -> LDS by LDS-DMA (`buffer_load_dwordx4 ... lds`: no staging registers, no ds_write pass) as 1 KiB
 //     MFMA FRAGMENTS: a 16-row x 32-k block of x, or 16 columns x 32 k of w.  The dequantised weights are WRITTEN in fragment order
 //     by the dequant pass (one wave load = one contiguous KiB in lane order: the LDS image is lane-linear and `ds_read_b128` at
@@ -42,7 +42,6 @@
 
 #include "wna16.cuh"
 
-#define GX_BM 256
 #define GX_BK 64
 #define GX_THREADS 512
 #define GX_MAX_SEG 3
@@ -78,8 +77,8 @@ struct GemmXArgs {
   uint32_t* err;
 };
 
-static inline size_t gemm_dense_lds_bytes(int bn) {  // the K loop's two buffers, or the epilogue's [256][bn (+ 8)] tile of outputs
-  const size_t loop = (size_t)2 * (32 * 1024 + (size_t)(bn / 16) * 2 * 1024), epi = (size_t)GX_BM * ((size_t)bn * 2 + 16);
+static inline size_t gemm_dense_lds_bytes(int bm, int bn) {  // the K loop's two buffers, or the epilogue's [bm][bn (+ 8)] tile of outputs
+  const size_t loop = (size_t)2 * (bm + bn) / 16 * 2 * 1024, epi = (size_t)bm * ((size_t)bn * 2 + 16);
   return loop > epi ? loop : epi;
 }
 
@@ -130,19 +129,20 @@ __device__ __forceinline__ int gx_slot_xor(int row) {
   return (a >> 1) | (((a ^ (a >> 1)) & 1) << 1);
 }
 
-template <class DT, int BN, bool DUAL>
+template <class DT, int BM, int BN, bool DUAL>
 __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int NF = BN / 16;    // n-frags of the tile
   constexpr int WNF = NF / 4;    // n-frags of a wave (4 | 2)
   constexpr int HNF = WNF / 2;   // ... of one unit
-  constexpr int XB = 32 * 1024;  // bytes of x per buffer: 16 m-frags x 2 k-chunks
+  constexpr int MF = BM / 64;    // m-frags of a wave and phase (4 | 3)
+  constexpr int XB = BM / 16 * 2 * 1024;  // bytes of x per buffer: the m-frags x 2 k-chunks
   constexpr int WB = NF * 2 * 1024;
   constexpr int BUF = XB + WB;
   constexpr int WPU = HNF * 8 / 8;  // LDS-DMA instructions per wave for a unit of w: 4 waves' worth of HNF n-frags x 2 k-chunks over 8 waves
-  constexpr int VMW = 2 * 2 + 2 * (HNF == 2 ? 2 : 1);  // DMA instructions of a K-step (the newest unit of each kind)
+  constexpr int VMW = MF + 2 * (HNF == 2 ? 2 : 1);  // DMA instructions of a wave and K-step (the newest unit of each kind)
   constexpr uint32_t RSRC3 = 0x00020000u;
-  static_assert(BN == 256 || BN == 128, "tile width");
+  static_assert(BM == 256 ? BN == 256 || BN == 128 : BM == 192 && BN == 256, "tile");
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -182,18 +182,20 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
     mt = first + rem % gsz;
     nt = rem / gsz;
   }
-  const int m0 = mt * GX_BM;
+  const int m0 = mt * BM;
 
   // ---- LDS-DMA sources.  x: lane p of a fragment fetch = row p >> 2, chunk slot p & 3 holding chunk (p & 3) ^ gx_slot_xor(row)
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, 0x7FFFFFF0, RSRC3);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.wd), 0, 0x7FFFFFF0, RSRC3);
   const int srow = lane >> 2, schunk = (lane & 3) ^ gx_slot_xor(srow);
-  //   this wave stages m-frag mfs (+4 for U2) of the tile: {0,1,2,3,8,9,10,11}[wave]
-  const int mfs = wave < 4 ? wave : wave + 4;
+  //   256 rows: this wave stages m-frag {0,1,2,3,8,9,10,11}[wave] (+4 for U2), both k-chunks.  192 rows: the six m-frags of a unit are three for each
+  //   wave pair of a group: waves 0-3 stage U0's frags 0-3 whole and half a frag of U2's 4 and 5, waves 4-7 the other way about
+  auto xfrag = [&](int u, int f) { return MF == 4 ? (f < 4 ? f : f + 4) + 4 * u : f / 3 * 6 + f % 3 + 3 * u; };  // frag f of unit u in the tile
+  const bool whole0 = MF == 4 || wave < 4, whole1 = MF == 4 || wave >= 4;  // (a whole frag of U0 / U2)
+  const int xf[2] = {xfrag(0, whole0 ? wave : 4 + ((wave - 4) >> 1)), xfrag(1, MF == 4 ? wave : (whole1 ? wave - 4 : 4 + (wave >> 1)))};
   uint32_t vo_x[2];
 #pragma unroll
-  for (int u = 0; u < 2; u++)
-    vo_x[u] = ((uint32_t)min(m0 + (mfs + 4 * u) * 16 + srow, M - 1) * (uint32_t)a.x_ld + (uint32_t)schunk * 8u) * 2u;
+  for (int u = 0; u < 2; u++) vo_x[u] = ((uint32_t)min(m0 + xf[u] * 16 + srow, M - 1) * (uint32_t)a.x_ld + (uint32_t)schunk * 8u) * 2u;
   const uint32_t vo_w = (uint32_t)lane * 16u;
   //   w units: U3 = the first HNF n-frags of every wave column, U1 = the others.  BN = 256: this wave stages n-frag (wave >> 1) * 4 + (wave & 1)
   //   (+2 for U1), both k-chunks; BN = 128: n-frag (wave >> 1) * 2 (+1), k-chunk wave & 1
@@ -207,10 +209,10 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
   typedef __attribute__((address_space(3))) void* lds_ptr;
   // (no instruction offsets on these loads: with `lds` set the hardware adds inst_offset to the LDS address as well as to the memory address)
   auto stage_x = [&](int buf, int u, int ks) {  // unit U0 (u = 0) / U2 (u = 1) of K-step ks
-    const int kc = min(ks, KS - 1);
-    unsigned char* d = smem + buf * BUF + (mfs + 4 * u) * 2048;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)d, 16, vo_x[u], (uint32_t)kc * 128u, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(d + 1024), 16, vo_x[u], (uint32_t)kc * 128u + 64u, 0, 0);
+    const int kc = min(ks, KS - 1), c0 = (u ? whole1 : whole0) ? 0 : wave & 1;
+    unsigned char* d = smem + buf * BUF + xf[u] * 2048;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(d + c0 * 1024), 16, vo_x[u], (uint32_t)kc * 128u + (uint32_t)c0 * 64u, 0, 0);
+    if (u ? whole1 : whole0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(d + 1024), 16, vo_x[u], (uint32_t)kc * 128u + 64u, 0, 0);
   };
   auto stage_w = [&](int buf, int u, int ks) {  // unit U3 (u = 0) / U1 (u = 1)
     const int kc = min(ks, KS - 1);
@@ -221,14 +223,14 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
   };
 
   // ---- LDS reads: x fragment (m-frag, kc) of this wave's rows, w fragment (n-frag, kc) of its columns
-  const unsigned char* xrd = smem + (wr * 8) * 2048 + (r16 * 4 + (q4 ^ gx_slot_xor(r16))) * 16;
+  const unsigned char* xrd = smem + (wr * 2 * MF) * 2048 + (r16 * 4 + (q4 ^ gx_slot_xor(r16))) * 16;
   const unsigned char* wrd = smem + XB + (wc * WNF) * 2048 + lane * 16;
-  s16x8 xa[4][2], wa[WNF][2];
+  s16x8 xa[MF][2], wa[WNF][2];
   auto read_x = [&](int buf, int mh) {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < MF; i++)
 #pragma unroll
-      for (int kc = 0; kc < 2; kc++) xa[i][kc] = *reinterpret_cast<const s16x8*>(xrd + buf * BUF + ((mh * 4 + i) * 2 + kc) * 1024);
+      for (int kc = 0; kc < 2; kc++) xa[i][kc] = *reinterpret_cast<const s16x8*>(xrd + buf * BUF + ((mh * MF + i) * 2 + kc) * 1024);
   };
   auto read_w = [&](int buf) {
 #pragma unroll
@@ -237,26 +239,25 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
       for (int kc = 0; kc < 2; kc++) wa[j][kc] = *reinterpret_cast<const s16x8*>(wrd + buf * BUF + (j * 2 + kc) * 1024);
   };
 
-  f32x4 acc[8][WNF];
+  f32x4 acc[2 * MF][WNF];
 #pragma unroll
-  for (int i = 0; i < 8; i++)
+  for (int i = 0; i < 2 * MF; i++)
 #pragma unroll
     for (int j = 0; j < WNF; j++) acc[i][j] = vra_zero_acc();
   // waits for the phase's own LDS reads and the next phase's units, then the matrix work between two barriers.  A = weights (16 columns x
   // 32 k), B = x (16 rows x 32 k): D[column][row]
   auto compute = [&](auto MH) {
     constexpr int mh = decltype(MH)::value;
-    if constexpr (VMW == 8) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(VMW) : "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int kc = 0; kc < 2; kc++)
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < MF; i++)
 #pragma unroll
-        for (int j = 0; j < WNF; j++) DT::mfma_ready(acc[mh * 4 + i][j], wa[j][kc], xa[i][kc]);
+        for (int j = 0; j < WNF; j++) DT::mfma_ready(acc[mh * MF + i][j], wa[j][kc], xa[i][kc]);
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
@@ -274,8 +275,7 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
   stage_x(1, 0, ks0 + 1);
   stage_w(1, 0, ks0 + 1);
   stage_w(1, 1, ks0 + 1);
-  if constexpr (VMW == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-  else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(VMW) : "memory");
   __builtin_amdgcn_s_barrier();
   if (wr == 1) __builtin_amdgcn_s_barrier();  // the second wave group runs one barrier behind the first
 
@@ -302,16 +302,16 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
 
   // ---- split-K: the slices of a tile meet through memory (gemm_q4_big.cuh): write-through 16-byte stores, one flag line per slice,
   // the last slice ("owner") polls, adds the slabs to its own partial in slice order and resets the flags
-  if (SK > 1) {
+  if (MF == 4 && SK > 1) {
     const int tile = xtile, ntiles = xtiles;
     const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(a.slabs, 0, 0x7FFFFFF0, RSRC3);
     auto slab_off = [&](int z, int i, int j) {  // bytes: [slice][tile][m-frag][n-frag][thread] x 16 B
-      return (uint32_t)((((z * ntiles + tile) * 8 + i) * WNF + j) * GX_THREADS + tid) * 16u;
+      return (uint32_t)((((z * ntiles + tile) * 2 * MF + i) * WNF + j) * GX_THREADS + tid) * 16u;
     };
     uint32_t* fl = a.counters + (size_t)tile * SK * 16;
     if (zi != SK - 1) {
 #pragma unroll
-      for (int i = 0; i < 8; i++)
+      for (int i = 0; i < 2 * MF; i++)
 #pragma unroll
         for (int j = 0; j < WNF; j++) {
           const u32x4 v = {__float_as_uint(acc[i][j][0]), __float_as_uint(acc[i][j][1]), __float_as_uint(acc[i][j][2]), __float_as_uint(acc[i][j][3])};
@@ -336,7 +336,7 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
     __syncthreads();
     for (int z = 0; z < SK - 1; z++) {  // fixed order; one m-frag row of accumulators per round trip
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
+      for (int i = 0; i < 2 * MF; i++) {
         u32x4 pz[WNF];
 #pragma unroll
         for (int j = 0; j < WNF; j++) pz[j] = __builtin_amdgcn_raw_buffer_load_b128(srs, slab_off(z, i, j), 0, 16);
@@ -374,9 +374,9 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
         bs[0] = DT::to_f32((uint16_t)(bw[0] & 0xffffu)), bs[1] = DT::to_f32((uint16_t)(bw[0] >> 16));
         bs[2] = DT::to_f32((uint16_t)(bw[1] & 0xffffu)), bs[3] = DT::to_f32((uint16_t)(bw[1] >> 16));
       }
-      unsigned char* const lp = smem + (size_t)(wr * 128 + r16) * ROWB + (wc * (NOUT * 16) + jo * 16 + q4 * 4) * 2;
+      unsigned char* const lp = smem + (size_t)(wr * (BM / 2) + r16) * ROWB + (wc * (NOUT * 16) + jo * 16 + q4 * 4) * 2;
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
+      for (int i = 0; i < 2 * MF; i++) {
         float v[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -406,7 +406,7 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
   const int out_ld = c2 ? a.seg[2].out_ld : (c1 ? a.seg[1].out_ld : a.seg[0].out_ld);
   const int n = ocol - (c2 ? a.seg[2].vcol_start : (c1 ? a.seg[1].vcol_start : a.seg[0].vcol_start)) / (DUAL ? 2 : 1);
 #pragma unroll 4
-  for (int p = 0; p < GX_BM / RPP; p++) {
+  for (int p = 0; p < BM / RPP; p++) {
     const int row = p * RPP + crow, m = m0 + row;
     if (m >= M) break;
     u32x4 o = *reinterpret_cast<const u32x4*>(smem + (size_t)row * ROWB + cch * 16);

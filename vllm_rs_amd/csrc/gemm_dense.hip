@@ -14,17 +14,17 @@ static int gx_cur_dev() {
   return dev & 63;
 }
 
-template <class DT, int BN, bool DUAL>
+template <class DT, int BM, int BN, bool DUAL>
 static void launch_gemm_dense_t(const GemmXArgs& a, hipStream_t st) {
-  const size_t lds = gemm_dense_lds_bytes(BN);
+  const size_t lds = gemm_dense_lds_bytes(BM, BN);
   static uint64_t attr_devs = 0;  // per device: function attributes belong to the device current at the call
   if (!((attr_devs >> gx_cur_dev()) & 1)) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dense_kernel<DT, BN, DUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dense_kernel<DT, BM, BN, DUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr_devs |= (uint64_t)1 << gx_cur_dev();
   }
   const int tiles = a.MT * a.NT;
   const unsigned grid = a.tail_sk > 1 ? (unsigned)(a.tail_first + (tiles - a.tail_first) * a.tail_sk) : (unsigned)(tiles * (a.splitk > 1 ? a.splitk : 1));
-  gemm_dense_kernel<DT, BN, DUAL><<<dim3(grid), GX_THREADS, lds, st>>>(a);
+  gemm_dense_kernel<DT, BM, BN, DUAL><<<dim3(grid), GX_THREADS, lds, st>>>(a);
 }
 
 static int gx_num_cus() {
@@ -34,12 +34,12 @@ static int gx_num_cus() {
   return n[dev];
 }
 
-// tile width (256 | 128) and split-K factor (<< 16) for an M x nv x K problem
+// tile (256 rows x 256 | 128 columns, 192: that many rows x 256 columns) and split-K factor (<< 16) for an M x nv x K problem
 int vra_gemm_dense_tile(int M, int nv, int K) {
   static const char* env = getenv("VRA_GX_BN");  // tuning aid: width | splitk << 16
   if (env && ((atoi(env) & 0xffff) == 128 || (atoi(env) & 0xffff) == 256)) return atoi(env);
   const int cus = gx_num_cus();
-  const long mt = (M + GX_BM - 1) / GX_BM;
+  const long mt = (M + 255) / 256;
   const long t256 = mt * ((nv + 255) / 256), t128 = mt * ((nv + 127) / 128);
   // time ~ rounds of `cus` workgroups x tile work.  Measured (tools/gemm_dense_microbench.py --tile): a 128-wide tile does half the work
   // at ~0.8 of the wide tile's rate (o_proj, 4096 rows: 256 wide tiles 107 us, 512 narrow ones 135), and a last round that fills
@@ -78,12 +78,21 @@ int vra_gemm_dense_tile(int M, int nv, int K) {
       }
     }
   }
+  // 192 rows x 256 columns, K whole (the bits of the unsplit tiles above), where that is the least of: rounds x a round's time (256 x 256: 1, 192 x 256:
+  // 0.78, 256 x 128: 0.6), the last of them between 0.7 and 1 of it.  us, the choice so far / this tile: 2185 rows, K = 3584 x 4608 72 / 63, x 37888 520 /
+  // 480; 1500 rows x 6144, K = 4096 83 / 70; 2800 rows x 4096, K = 14336 278 / 233; on 38 of 117 unsplit shapes of 700..8192 rows, 12 % faster on
+  // average there, never slower
+  if (best < 1 << 16) {
+    auto time = [&](long t, double round) { return round * ((double)(t / cus) + (t % cus ? 0.7 + 0.3 * (double)(t % cus) / cus : 0.0)); };
+    const long t192 = (M + 191) / 192 * (long)((nv + 255) / 256);
+    if (time(t192, 0.78) < 0.97 * (best == 256 ? time(t256, 1.0) : time(t128, 0.6))) best = 192;
+  }
   return best;
 }
 
 void vra_launch_gemm_dense(GemmXArgs a, bool dual, int dtype, int bn_sk, int64_t stream) {
-  const int bn = bn_sk & 0xffff, sk = ((bn_sk >> 16) & 0xff) > 1 ? ((bn_sk >> 16) & 0xff) : 1, tsk = (bn_sk >> 24) > 1 ? (bn_sk >> 24) : 1;
-  a.MT = (a.M + GX_BM - 1) / GX_BM;
+  const int bm = (bn_sk & 0xffff) == 192 ? 192 : 256, bn = bm == 192 ? 256 : bn_sk & 0xffff, sk = ((bn_sk >> 16) & 0xff) > 1 ? ((bn_sk >> 16) & 0xff) : 1, tsk = (bn_sk >> 24) > 1 ? (bn_sk >> 24) : 1;
+  a.MT = (a.M + bm - 1) / bm;
   a.NT = (a.NV + bn - 1) / bn;
   a.splitk = sk;
   a.tail_sk = 0, a.tail_first = 0;
@@ -92,7 +101,7 @@ void vra_launch_gemm_dense(GemmXArgs a, bool dual, int dtype, int bn_sk, int64_t
     a.tail_first = tiles / cus * cus;
     a.tail_sk = tsk;
     a.splitk = 1;
-    if (bn != 256 || a.tail_first <= 0 || a.tail_first >= tiles || (a.tail_first & 7) || ((tiles - a.tail_first) * tsk) % 8 || (a.K / 64) % (2 * tsk)) {
+    if (bm != 256 || bn != 256 || a.tail_first <= 0 || a.tail_first >= tiles || (a.tail_first & 7) || ((tiles - a.tail_first) * tsk) % 8 || (a.K / 64) % (2 * tsk)) {
       vra_set_error("gemm_dense: tail split does not fit the shape (tiles=%d, slices=%d)", tiles, tsk);
       return;
     }
@@ -101,24 +110,27 @@ void vra_launch_gemm_dense(GemmXArgs a, bool dual, int dtype, int bn_sk, int64_t
     a.slabs = vra_scratch_slabs();
     a.counters = vra_scratch_counters();
     a.err = vra_scratch_error_word();
-    if (!a.slabs || !a.counters || bn != 256 || (a.K / 64) % (2 * std::max(sk, tsk))) {
+    if (!a.slabs || !a.counters || bm != 256 || bn != 256 || (a.K / 64) % (2 * std::max(sk, tsk))) {
       vra_set_error("gemm_dense: split-K scratch unavailable or K not divisible (K=%d, slices=%d)", a.K, sk);
       return;
     }
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool bf = dtype == VRA_BF16;
-#define VRA_GX(BNV, DU)                                   \
-  do {                                                    \
-    if (bf) launch_gemm_dense_t<BF16, BNV, DU>(a, st);    \
-    else launch_gemm_dense_t<F16, BNV, DU>(a, st);        \
+#define VRA_GX(BMV, BNV, DU)                                   \
+  do {                                                         \
+    if (bf) launch_gemm_dense_t<BF16, BMV, BNV, DU>(a, st);    \
+    else launch_gemm_dense_t<F16, BMV, BNV, DU>(a, st);        \
   } while (0)
-  if (bn == 256) {
-    if (dual) VRA_GX(256, true);
-    else VRA_GX(256, false);
+  if (bm == 192) {
+    if (dual) VRA_GX(192, 256, true);
+    else VRA_GX(192, 256, false);
+  } else if (bn == 256) {
+    if (dual) VRA_GX(256, 256, true);
+    else VRA_GX(256, 256, false);
   } else {
-    if (dual) VRA_GX(128, true);
-    else VRA_GX(128, false);
+    if (dual) VRA_GX(256, 128, true);
+    else VRA_GX(256, 128, false);
   }
 #undef VRA_GX
 }
@@ -220,7 +232,7 @@ extern "C" void vra_dense_frag_gemm(const void* x, const void* wd, const void* b
   VRA_CHECK_ARG(m >= 1 && k % 128 == 0 && nv % 16 == 0 && (!dual || nv % 32 == 0), "dense_frag_gemm: bad shape M=%d K=%d NV=%d", m, k, nv);
   VRA_CHECK_ARG(dtype == VRA_BF16 || dtype == VRA_F16, "dense_frag_gemm: dtype must be bf16/f16");
   VRA_CHECK_ARG(!(dual && bias), "dense_frag_gemm: the gate/up form takes no bias");
-  VRA_CHECK_ARG(tile_n == 0 || (tile_n & 0xffff) == 128 || (tile_n & 0xffff) == 256, "dense_frag_gemm: tile_n must be 0 (auto), 128 or 256 (| split-K slices << 16 | tail slices << 24)");
+  VRA_CHECK_ARG(tile_n == 0 || tile_n == 192 || (tile_n & 0xffff) == 128 || (tile_n & 0xffff) == 256, "dense_frag_gemm: tile_n must be 0 (auto), 192 (rows x 256), 128 or 256 (| split-K slices << 16 | tail slices << 24)");
   if (tile_n >> 16 > 1) vra_scratch_init();
   GemmXArgs a{};
   a.x = x, a.x_ld = k, a.wd = wd, a.residual = residual;

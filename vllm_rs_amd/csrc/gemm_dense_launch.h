@@ -1,7 +1,7 @@
 // gemm_dense_launch.h — launchers of kernel X (gemm_dense.cuh) shared between the C entry points and the native runtime.
 #pragma once
 #include "gemm_dense.cuh"
-// tile width (256 | 128) | split-K slices << 16 for an M x nv (virtual columns) x K problem
+// tile (256 | 128 columns of 256 rows, 192: rows of 256 columns) | split-K slices << 16 for an M x nv (virtual columns) x K problem
 int vra_gemm_dense_tile(int M, int nv, int K);
 // fills MT / NT / the split-K exchange; bn_sk from vra_gemm_dense_tile
 void vra_launch_gemm_dense(GemmXArgs a, bool dual, int dtype, int bn_sk, int64_t stream);
