@@ -289,7 +289,7 @@ void vra_swap_blocks(const void* src, void* dst, const int64_t* h_pairs, int32_t
  * (llama.rs:317-319): values are rounded to `dtype` first, then widened. */
 void vra_dense_gemm(const void* x, const void* w, const void* bias, void* out, int32_t m, int32_t k,
                     int32_t n, int32_t dtype, int32_t out_dtype, int64_t stream);
-/* the same product of 33 rows up on a named tile of the row-major prompt GEMM (rows / 64 * 16 + columns / 64: 0x12, 0x22, 0x32, 0x24 or, K % 128 == 0, 0x44): `nseg` (1..3) tensors of
+/* the same product of 33 rows up on a named tile of the row-major prompt GEMM (rows / 64 * 16 + columns / 64: 0x12, 0x22, 0x32, 0x24 or, K % 128 == 0, 0x34, 0x44): `nseg` (1..3) tensors of
  * n[s] columns side by side, each with its own bias (or null) and output [m, n[s]], or (pair, nseg 2) silu(x . w[0]) * (x . w[1]) into
  * out[0].  The tile changes no bit of the result. */
 void vra_dense_gemm_tile(int32_t tile, const void* x, const void* const* w, const void* const* bias, const int32_t* n, int32_t nseg,
@@ -658,7 +658,7 @@ void vra_stack_op_group_norm(const float* x, const float* w, void* h, int32_t T,
 void vra_stack_op_gemm(const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32,
                        int32_t M, int32_t N, int32_t K, float alpha, const int32_t* tile_group, int32_t granule, const int32_t* a_row,
                        const float* a_scale, const int32_t* out_row, int32_t epi, float limit, int32_t dtype, int64_t stream);
-/* the bf16 product of more than 32 rows on a named tile (0x12, 0x22, 0x24 or, no row groups, 0x32 or, K % 128 == 0, 0x44: rows / 64 * 16 + columns / 64), granules of a tile's rows */
+/* the bf16 product of more than 32 rows on a named tile (0x12, 0x22, 0x24 or, no row groups, 0x32 or, K % 128 == 0, 0x34, 0x44: rows / 64 * 16 + columns / 64), granules of a tile's rows */
 void vra_stack_op_gemm_tile(int32_t tile, const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32,
                             int32_t M, int32_t N, int32_t K, const int32_t* tile_group, const int32_t* a_row, int32_t a_rows,
                             const int32_t* out_row, int32_t epi, float limit, int64_t stream);

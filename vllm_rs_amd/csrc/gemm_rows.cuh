@@ -6,7 +6,7 @@
 // a line that another CU has asked for costs as long).  A 128 x 128 tile needs 32 KiB per 512 clocks of MFMAs, 256 x 256 64 KiB per 2048.
 //
 // Two groups of four waves (a wave of each on every SIMD) run one barrier apart: while one group's MFMAs run, the other reads its operands of the
-// next phase from LDS and requests tiles.  A phase is a K step of 64 — with 256 rows two of them a step, the upper and the lower 64 rows of every wave —
+// next phase from LDS and requests tiles.  A phase is a K step of 64 — with 256 x 256 and 192 x 256 outputs two of them a step, the upper and the lower rows of every wave —
 //   { LDS reads | requests | vmcnt: the next phase's tiles have landed, lgkmcnt: this phase's reads are done | barrier | MFMAs | barrier }
 // and requests go to the buffer that the phase before read: both groups' reads ended ahead of a barrier that the requesting wave has passed.
 // Fragments come from LDS only, so the MFMAs need no wait states between them (10 % of a group's phase).  Against one group in step with itself
@@ -34,7 +34,7 @@ struct GemmRowsArgs {
   int nseg = 1;
   int M = 0, K = 0;  // K % 64 == 0
   int MT = 0, NT = 0;  // tiles along m, and along n over all segments
-  // grouped rows (not on 256-row tiles): tile row t (BM rows) multiplies with w[0] + tile_group[t] * w_group_stride (elements); -1: an empty tile row
+  // grouped rows (on tiles of 64 and 128 rows): tile row t (BM rows) multiplies with w[0] + tile_group[t] * w_group_stride (elements); -1: an empty tile row
   const int* tile_group = nullptr;
   int64_t w_group_stride = 0;
   int64_t x_batch_stride = 0, w_batch_stride = 0;  // elements between the operands of two products of a batch (grid y)
@@ -65,9 +65,9 @@ __device__ __forceinline__ void gr_gather_columns(u32x2 (&v)[2]) {
 // waves of a tile: two groups of four (rows 0 .. BM/2 - 1 and the others), CW of them side by side with 64 columns each
 template <int BM, int BN, bool DEEP>
 struct GrTile {
-  static constexpr int H = BM == 256 ? 2 : 1;                           // phases of a K step (the upper, the lower rows of a wave)
+  static constexpr int H = BM * BN > 128 * 256 ? 2 : 1;                 // phases of a K step (the upper, the lower rows of a wave)
   static constexpr int KP = DEEP ? 2 : 1;                                     // K steps of a phase
-  static constexpr int S = BM == 256 ? 2 : (BM == 128 && BN == 128 ? 4 : 3);  // LDS buffers (of a phase's K steps)
+  static constexpr int S = H == 2 ? 2 : (BM == 128 && BN == 128 ? 4 : 3);  // LDS buffers (of a phase's K steps)
   static constexpr int CW = BN / 64, RW = 4 / CW;
   static constexpr int NX = BM / 32 / RW / H;  // 16-row blocks of a wave in a phase
   static constexpr int XB = BM / 16, WB = BN / 16, STG = (XB + WB) * 2048;
@@ -125,8 +125,14 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
   const __amdgpu_buffer_rsrc_t rhi = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(whi), 0, 0x7FFFFFF0, 0x00020000u);
   // DMA sources: lane p fetches row p >> 3 of an instruction's eight, the chunk that slot p & 7 holds
   const int sr = lane >> 3, sc = (lane & 7) ^ sr;
-  auto xrow8 = [&](int e) {  // instruction e of this wave: eight rows from this one on (two phases: e = 0, 1 upper rows, 2, 3 lower rows)
-    return H == 2 ? (wave < 4 ? wave : wave + 4) * 16 + (e >> 1) * 64 + (e & 1) * 8 : (wave * EX + e) * 8;
+  // instruction e of this wave: eight rows from this one on.  Two phases, of 256 rows: e = 0, 1 upper, 2, 3 lower rows of a group; of 192 rows, a group's
+  // upper and lower 48: waves 0-3 two of the upper rows' instructions and one of the lower ones', waves 4-7 the other way about
+  auto upper = [&](int e) { return EX == 4 ? e < 2 : e == 0 || (e == 1 && wave < 4); };
+  auto xrow8 = [&](int e) {
+    if (H == 1) return (wave * EX + e) * 8;
+    if (EX == 4) return (wave < 4 ? wave : wave + 4) * 16 + (e >> 1) * 64 + (e & 1) * 8;
+    const int i = wave < 4 ? (upper(e) ? wave * 2 + e : 8 + wave) : (upper(e) ? 4 + wave : (wave - 4) * 2 + e - 1);  // of the twelve of its half
+    return i / 6 * 96 + i % 6 * 8 + (upper(e) ? 0 : 48);
   };
   uint32_t vx[EX], vw[EW];
 #pragma unroll
@@ -147,6 +153,11 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
     const uint32_t so = (uint32_t)min(ks, KT - 1) * 128u;
 #pragma unroll
     for (int e = e0; e < e1; e++) __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(smem + o + xrow8(e) * 128), 16, vx[e], so, 0, 0);
+  };
+  auto stage_half = [&](int o, int ks, bool up) {  // the upper or the lower rows
+#pragma unroll
+    for (int e = 0; e < EX; e++)
+      if (upper(e) == up) stage_x(o, ks, e, e + 1);
   };
   auto stage_w = [&](int o, int ks) {
     const uint32_t so = (uint32_t)min(ks, KT - 1) * 128u;
@@ -209,10 +220,10 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
   using C0 = std::integral_constant<int, 0>;
   using C1 = std::integral_constant<int, 1>;
   if constexpr (H == 2) {
-    stage_x(0, 0, 0, 2);
+    stage_half(0, 0, true);
     stage_w(0, 0);
-    stage_x(0, 0, 2, 4);
-    stage_x(STG, 1, 0, 2);
+    stage_half(0, 0, false);
+    stage_half(STG, 1, true);
     stage_w(STG, 1);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(D) : "memory");
     __builtin_amdgcn_s_barrier();
@@ -222,10 +233,10 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
       read_w(o);
       __builtin_amdgcn_sched_barrier(0);
       read_x(o, 0);
-      stage_x(STG - o, ks + 1, 2, 4);
+      stage_half(STG - o, ks + 1, false);
       compute(C0{}, 1);
       read_x(o, 1);
-      stage_x(o, ks + 2, 0, 2);
+      stage_half(o, ks + 2, true);
       stage_w(o, ks + 2);
       compute(C1{}, 1);
     };
@@ -272,15 +283,16 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
 // run in rounds of `slots`; a launch costs t0, a round `round` (first requests, outputs) and `full` for 64 of K, the last round between `one` (a
 // few workgroups) and `full`.  64 x 128 has two forms (gemm_rows_launch).  192 x 128 is for what is a little more than one round of 128 x 128 and leaves
 // much of one of 128 x 256 idle; us without / with it: 2120 rows x 2048, K = 2048 31.7 / 26.5, K = 5632 67.2 / 56.2; 700 x 8192, K = 2048 35.1 / 30.5;
-// 300 x 14336, K = 4096 51.1 / 44.7; 1280 x 4096, K = 14336 163 / 135.  rows: only tiles of that many (0: any).
+// 300 x 14336, K = 4096 51.1 / 44.7; 1280 x 4096, K = 14336 163 / 135.  192 x 256 does the same between 128 x 256 and 256 x 256: 1500 x 8192, K = 2048
+// 57.2 / 48.8; 2120 x 4096, K = 4096 86.1 / 71.6; 2560 x 4096, K = 14336 272 / 235.  rows: only tiles of that many (0: any).
 // -> rows / 64 * 16 + columns / 64; *us: the time
 static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch, int K, int rows = 0, double* us = nullptr) {
-  const struct { int bm, bn, slots; double t0, round, one, full; } t[6] = {{256, 256, 256, 2.0, 14.4, 0.79, 1.39}, {128, 256, 256, 0.7, 9.5, 0.52, 0.78},
+  const struct { int bm, bn, slots; double t0, round, one, full; } t[7] = {{256, 256, 256, 2.0, 14.4, 0.79, 1.39}, {192, 256, 256, 1.0, 10.0, 0.56, 1.10}, {128, 256, 256, 0.7, 9.5, 0.52, 0.78},
       {192, 128, 256, 1.0, 6.5, 0.40, 0.64}, {128, 128, 256, 1.4, 5.4, 0.35, 0.50}, {64, 128, 512, 2.6, 2.4, 0.27, 0.60}, {64, 128, 256, 3.7, 1.3, 0.28, 0.34}};
   int best = 0;
   double cost = 0.0;
   for (const auto& c : t) {
-    if ((rows && c.bm != rows) || (c.bm == 256 && K % 128)) continue;
+    if ((rows && c.bm != rows) || (c.bm * c.bn > 128 * 256 && K % 128)) continue;
     long cols = 0;
     for (int s = 0; s < nseg; s++) cols += (ncols[s] + c.bn - 1) / c.bn;
     const long tiles = (M + c.bm - 1) / c.bm * cols * batch, full = tiles / c.slots, rem = tiles % c.slots;
@@ -293,7 +305,7 @@ static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch,
   if (us) *us = cost;
   return best;
 }
-static inline bool gemm_rows_has_tile(int tile, int K) { return (tile == 4 * 16 + 4 && K % 128 == 0) || tile == 2 * 16 + 4 || tile == 3 * 16 + 2 || tile == 2 * 16 + 2 || tile == 16 + 2; }
+static inline bool gemm_rows_has_tile(int tile, int K) { return ((tile == 4 * 16 + 4 || tile == 3 * 16 + 4) && K % 128 == 0) || tile == 2 * 16 + 4 || tile == 3 * 16 + 2 || tile == 2 * 16 + 2 || tile == 16 + 2; }
 // fills the tile counts and launches
 template <class DT, int BM, int BN, bool DEEP, bool PAIR, class EPI>
 static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStream_t st) {
@@ -317,6 +329,7 @@ static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStr
 template <class DT, bool PAIR, class EPI>
 static void gemm_rows_launch(const GemmRowsArgs& a, const EPI& epi, int tile, int batch, hipStream_t st) {
   if (tile == 4 * 16 + 4) return gemm_rows_launch_t<DT, 256, 256, false, PAIR>(a, epi, batch, st);
+  if (tile == 3 * 16 + 4) return gemm_rows_launch_t<DT, 192, 256, false, PAIR>(a, epi, batch, st);
   if (tile == 2 * 16 + 4) return gemm_rows_launch_t<DT, 128, 256, false, PAIR>(a, epi, batch, st);
   if (tile == 3 * 16 + 2) return gemm_rows_launch_t<DT, 192, 128, false, PAIR>(a, epi, batch, st);
   if (tile == 2 * 16 + 2) return gemm_rows_launch_t<DT, 128, 128, false, PAIR>(a, epi, batch, st);
