@@ -115,6 +115,32 @@ def test_dense_frag_gemm_tail_split(slices):
     assert ops.lib().vra_take_device_error() == 0
 
 
+# tile rows that end in a short group of eight (11, 17) and whole ones (16); four and two slices
+@pytest.mark.parametrize("M,NV,slices", [(2811, 6144, 4), (4300, 4096, 4), (4096, 6144, 2)])
+def test_tail_split_takes_the_last_tiles_of_the_order_of_eights(M, NV, slices):
+    """which outputs sum K in slices is part of the result: the tiles beyond the last whole round of the order that walks eight tile rows, then the
+    next column; every other output has the bits of the unsplit launch"""
+    K, MT, NT = 512, (M + 255) // 256, NV // 256
+    order = []
+    for first in range(0, MT, 8):
+        order += [(m, n) for n in range(NT) for m in range(first, min(first + 8, MT))]
+    r = rng(M + NV)
+    x, wd = ops.dev(rand_dt(r, (M, K), F16)), ops.dev(rand_dt(r, (NV, K), F16, 0.05))
+
+    def run(tile):
+        out = ops.DevBuf(M * NV * 2).fill_bytes(0xEE)
+        ops.lib().vra_dense_frag_gemm(x.ptr, wd.ptr, None, None, out.ptr, M, K, NV, 0, F16, tile, 0)
+        msg = ops.lib().vra_last_error().decode()
+        if "tail split does not fit" in msg:  # (a part with another CU count)
+            ops.lib().vra_clear_error()
+            pytest.skip(msg)
+        ops.check_error()
+        return out.numpy(np.uint16, (M, NV))
+    differ = run(256 | slices << 24) != run(256)
+    got = [differ[m * 256:m * 256 + 256, n * 256:n * 256 + 256].any() for m, n in order]
+    assert got == [i >= 256 for i in range(MT * NT)]
+
+
 @pytest.mark.parametrize("tile", [128, 256])
 @pytest.mark.parametrize("awq", [False, True])
 def test_dense_frag_gemm_gate_up(awq, tile):

@@ -32,8 +32,8 @@
 //     unit has a K-step to land, with two buffers.  After issuing a phase's units a wave waits `vmcnt` down to the newest K-step's
 //     worth of them; what leaves the count is read in the NEXT phase (one barrier later: LDS-DMA data is ordered for a reader only by the
 //     issuing wave's count plus a barrier the reader has passed).  vmcnt never reaches 0 inside the loop;
-//   * workgroup ids are remapped so that the workgroups of one XCD (ids = xcd mod 8) work on neighbouring tiles: 8 m-tiles x 4
-//     n-tiles in flight per XCD share their x and w panels in that XCD's L2;
+//   * workgroup ids are remapped so that the workgroups of one XCD (ids = xcd mod 8) work on neighbouring tiles: about 8 m-tiles
+//     x 4 n-tiles in flight per XCD share their x and w panels in that XCD's L2;
 //   * DUAL (gate/up): the dequant pass interleaves the two tensors fragment by fragment (g0 u0 g1 u1 ...), a wave then holds gate
 //     and up of the same output columns and the epilogue is silu(gate) * up (mlp.rs:451-469); q/k/v: one launch over the
 //     concatenated columns, segments in the epilogue.
@@ -152,7 +152,9 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
   const int KS = K >> 6;  // K-steps (even: K % 128 == 0)
   int SK = a.splitk > 1 ? a.splitk : 1;  // (wave-uniform; per workgroup with a tail split)
 
-  // ---- tile of this workgroup: ids of one XCD (id mod 8) take a contiguous run of the grouped tile order (8 m-tiles per super-row)
+  // ---- tile of this workgroup: ids of one XCD (id mod 8) take a contiguous run of the grouped tile order: the tile rows in equal groups of about eight
+  // (the weights come by once a group).  With a tail split in eights: which tiles are the last ones, and so which outputs sum K in slices, is part of
+  // the result
   int mt, nt, zi, xtile, xtiles;  // xtile of xtiles: the tile's index among the tiles that exchange partial sums
   {
     const int nwg = (int)gridDim.x, bid = (int)blockIdx.x;
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
       zi = lin_sk - lin * SK;
       xtile = lin, xtiles = a.MT * a.NT;
     }
-    const int groups = max((a.MT + 4) >> 3, 1), GM = (a.MT + groups - 1) / groups;  // (equal groups: the weights come by once a group)
+    const int groups = max((a.MT + 4) >> 3, 1), GM = a.tail_sk > 1 ? 8 : (a.MT + groups - 1) / groups;
     const int per = GM * a.NT;
     const int grp = lin / per, rem = lin - grp * per;
     const int first = grp * GM, gsz = min(a.MT - first, GM);
