@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Static check of the gfx950 MFMA register hazards described in vllm_rs_amd/csrc/common.cuh.
 
-For every v_mfma in the given .s files:
+For every v_mfma in the given .s files, along every path of the control flow (an instruction, a branch or a barrier counts as one wait state):
   (1) its destination must not overlap SrcA or SrcB;
   (2) within the next 12 wait states nothing but an MFMA accumulating into the SAME destination may
       read or write the destination registers (the inline-asm form is invisible to hipcc's hazard
@@ -10,10 +10,10 @@ For every v_mfma in the given .s files:
       inline-asm forms carry an `s_nop 1`; DT::mfma_ready does not and is for operands that come from LDS).
 Exit status 1 if any violation is found (the Makefile fails the build).
 
-Also a performance lint (round 4): (3) no kernel may fetch KERNEL ARGUMENTS with vector loads.  A struct field selected under a
+Also a performance lint: (3) no kernel may fetch KERNEL ARGUMENTS with vector loads.  A struct field selected under a
 per-lane index (`a.seg[i].out` with i varying across lanes) makes hipcc select the field's ADDRESS inside the kernel-argument block
 (s[0:1]) and read it with global_load — followed by `s_waitcnt vmcnt(0)`, which also waits for every weight tile in flight: a full HBM
-round trip per occurrence (DESIGN.md §3.1b).  Wave-uniform indices (readfirstlane) give scalar selects and s_loads.
+round trip per occurrence.  Wave-uniform indices (readfirstlane) give scalar selects and s_loads.
 """
 import re
 import sys
@@ -33,80 +33,112 @@ def regset(text):
 
 
 def instrs(path):
-    """yield (function, [instruction lines]) with comments/labels/directives stripped"""
-    cur, body = None, []
+    """yield (function, [instruction lines], {label: index of the instruction behind it}) with comments and directives stripped"""
+    cur, body, labels = None, [], {}
     for line in open(path, errors="ignore"):
         m = re.match(r"^(_Z\w+):", line)
         if m:
             if cur and body:
-                yield cur, body
-            cur, body = m.group(1), []
+                yield cur, body, labels
+            cur, body, labels = m.group(1), [], {}
             continue
         if cur is None:
             continue
+        if line.startswith(".Lfunc_end"):
+            if body:
+                yield cur, body, labels
+            cur, body, labels = None, [], {}
+            continue
         t = line.split(";")[0].strip()
-        if not t or t.startswith(".") or t.endswith(":"):
+        if t.endswith(":"):
+            labels[t[:-1]] = len(body)
+            continue
+        if not t or t.startswith("."):
             continue
         body.append(t)
-        if t.startswith("s_endpgm"):
-            yield cur, body
-            cur, body = None, []
     if cur and body:
-        yield cur, body
+        yield cur, body, labels
+
+
+def flow(body, labels):
+    """successors and predecessors of every instruction"""
+    succ, pred = [[] for _ in body], [[] for _ in body]
+    for i, t in enumerate(body):
+        to = []
+        if t.startswith(("s_cbranch", "s_branch")):
+            to.append(labels.get(t.split()[-1]))
+        if not t.startswith(("s_branch", "s_endpgm", "s_setpc")):
+            to.append(i + 1)
+        for j in to:
+            if j is not None and j < len(body):
+                succ[i].append(j)
+                pred[j].append(i)
+    return succ, pred
+
+
+MFMA = re.compile(r"v_mfma_\w+\s+(\S+),\s*(\S+),\s*(\S+),\s*(\S+)")
+
+
+def states(t):
+    m = re.match(r"s_nop\s+(\d+)", t)
+    return int(m.group(1)) + 1 if m else 1
+
+
+def walk(start, edges, limit, see, body):
+    """calls see(instruction, wait states since the MFMA) along all paths from `start` until `limit` states have passed or it returns a true value;
+    an instruction is looked at again only when it is reached with fewer states"""
+    least, todo = {}, [(j, 0) for j in edges[start]]
+    while todo:
+        i, waited = todo.pop()
+        if waited >= limit or least.get(i, limit) <= waited:
+            continue
+        least[i] = waited
+        if see(body[i], waited):
+            continue
+        todo += [(j, waited + states(body[i])) for j in edges[i]]
 
 
 def check(path):
     total = bad = 0
-    for fn, body in instrs(path):
-        for i, t in enumerate(body):
-            m = re.match(r"v_mfma_\w+\s+(\S+),\s*(\S+),\s*(\S+),\s*(\S+)", t)
-            if not m:
-                continue
+    for fn, body, labels in instrs(path):
+        found = []
+        mfmas = [(i, m) for i, m in ((i, MFMA.match(t)) for i, t in enumerate(body)) if m]
+        if not mfmas:
+            continue
+        succ, pred = flow(body, labels)
+        for i, m in mfmas:
             total += 1
-            d, a, b, c = [x.strip(",") for x in m.groups()]
-            D, A, B = regset(d), regset(a), regset(b)
+            t = body[i]
+            D, A, B, C = (regset(x) for x in m.groups())
             if D & A or D & B:
-                bad += 1
-                print(f"[overlap] {fn}: {t}", file=sys.stderr)
+                found.append(f"[overlap] {fn}: {t}")
                 continue
-            back, ops = 0, A | B | regset(c)
-            for u in reversed(body[max(0, i - 3):i]):
-                mn = re.match(r"s_nop\s+(\d+)", u)
-                if back >= 2 or u.startswith(("s_cbranch", "s_branch", "s_barrier")):
-                    break
-                if u.startswith("v_") and not u.startswith(("v_mfma", "v_cmp", "v_readfirstlane", "v_readlane")):
+            ops = A | B | C
+
+            def written(u, back):
+                if u.startswith("v_") and not u.startswith(("v_mfma", "v_cmp", "v_readfirstlane", "v_readlane", "v_nop")):
                     dst = [regset(x) for x in u.split(None, 1)[1].split(",")[:2 if "swap" in u else 1]]
                     if set().union(*dst) & ops:
-                        bad += 1
-                        print(f"[operand written {back} states ahead] {fn}: {u}  ->  {t}", file=sys.stderr)
-                        break
-                back += int(mn.group(1)) + 1 if mn else 1
-            waited = 0
-            for u in body[i + 1:]:
-                if waited >= WAIT:
-                    break
-                mm = re.match(r"v_mfma_\w+\s+(\S+),\s*(\S+),\s*(\S+),\s*(\S+)", u)
+                        found.append(f"[operand written {back} states ahead] {fn}: {u}  ->  {t}")
+                        return True
+
+            def used(u, waited):
+                mm = MFMA.match(u)
                 if mm:
-                    d2, a2, b2, c2 = [x.strip(",") for x in mm.groups()]
-                    if regset(d2) == D and regset(c2) == D and not (regset(a2) & D) and not (regset(b2) & D):
-                        break  # accumulate chain: the next MFMA takes over the tracking
-                    if (regset(d2) | regset(a2) | regset(b2) | regset(c2)) & D:
-                        bad += 1
-                        print(f"[early use by another mfma after {waited} states] {fn}: {t}  ->  {u}", file=sys.stderr)
-                        break
-                    waited += 1
-                    continue
-                mn = re.match(r"s_nop\s+(\d+)", u)
-                if mn:
-                    waited += int(mn.group(1)) + 1
-                    continue
-                if u.startswith(("s_cbranch", "s_branch", "s_endpgm", "s_setpc")):
-                    break  # control flow: the linear scan ends here (regions are written branch free)
-                if regset(u) & D:
-                    bad += 1
-                    print(f"[early use after {waited} states] {fn}: {t}  ->  {u}", file=sys.stderr)
-                    break
-                waited += 1
+                    d2, a2, b2, c2 = (regset(x) for x in mm.groups())
+                    if d2 == D and c2 == D and not (a2 & D) and not (b2 & D):
+                        return True  # accumulate chain: the next MFMA takes over the tracking
+                    if (d2 | a2 | b2 | c2) & D:
+                        found.append(f"[early use by another mfma after {waited} states] {fn}: {t}  ->  {u}")
+                        return True
+                elif regset(u) & D:
+                    found.append(f"[early use after {waited} states] {fn}: {t}  ->  {u}")
+                    return True
+            walk(i, pred, 2, written, body)
+            walk(i, succ, WAIT, used, body)
+        bad += len(found)
+        for f in found:
+            print(f, file=sys.stderr)
     return total, bad
 
 
@@ -122,7 +154,7 @@ SDST = re.compile(r"^s_\w+\s+(s\[(\d+):(\d+)\]|s(\d+))(?=[,\s]|$)")
 def check_kernarg_vector_loads(path):
     """s[0:1] holds the kernel-argument pointer from entry until something else is written to it"""
     bad = 0
-    for fn, body in instrs(path):
+    for fn, body, _ in instrs(path):
         n = 0
         for t in body:
             if KERNARG_VEC.search(t):

@@ -40,11 +40,13 @@ static inline hipStream_t as_stream(int64_t s) { return reinterpret_cast<hipStre
 //      may copy the accumulator one wait state later, reading it half written.
 // The builtin cannot be told to keep D off A/B (the allocator does it even in straight-line code), so the
 // instruction is issued through inline asm with the accumulator TIED ("+v": D = C, never A or B), every
-// MFMA region is kept branch free (no accumulator copies at control-flow merges), every chain starts from
-// vra_zero_acc(), VRA_MFMA_DRAIN() (12 wait states + scheduling barrier) stands between the last MFMA of
-// a chain and the first non-MFMA use of its accumulator, `s_nop 1` in front of each MFMA covers VALU-written
-// operands — and `make` runs tools/check_mfma_overlap.py over the generated ISA: the build FAILS if any
-// v_mfma has D overlapping A/B or if anything but an accumulating MFMA touches D within 12 wait states.
+// chain starts from vra_zero_acc() or mfma0 / mfma_from, and VRA_MFMA_DRAIN() (12 wait states + scheduling barrier) stands
+// between the last MFMA of a chain and the first non-MFMA use of its accumulator.  Branches around MFMAs are
+// wave-uniform and leave the accumulators where they are (no copies where control flow joins).  `s_nop 1` in front of an
+// MFMA covers VALU-written operands; mfma_ready has none and is for operands that come from LDS.
+// `make` runs tools/check_mfma_overlap.py over the generated ISA, along every path of the control flow: the build FAILS
+// if any v_mfma has D overlapping A/B, if anything but an accumulating MFMA touches D within 12 wait states, or if
+// a vector instruction writes an operand within the two ahead of it.
 #define VRA_MFMA_DRAIN()                \
   do {                                  \
     asm volatile("s_nop 7\n\ts_nop 4"); \
