@@ -203,3 +203,27 @@ def test_marlin_ffi_long_prefill(dense_from):
     ref = orc.wna16_gemm(x, q["idx"], None, q["scales"], gs, BF16, marlin_rounded=True)
     assert_close_dt(out.numpy(np.uint16, (M, N)), ref, BF16, name="marlin ffi, long prefill", abs_floor=2e-3)
     assert not ws.numpy(np.uint32, (N,)).any()
+
+
+# x of 120 MiB up and K from 12288 on: four phases a K-step on 256 x 256 tiles
+@pytest.mark.parametrize("form,NV", [("plain", 528), ("bias residual", 80), ("gate up", 544), ("split", 272)])
+def test_large_x_has_the_bits_of_small_ones(form, NV):
+    """rows of a large product, the first and the last of it, equal the same rows alone, which run in two phases"""
+    M, K, part = 5401, 12544, 300
+    r = rng(NV)
+    dual, both = form == "gate up", form == "bias residual"
+    n = NV // 2 if dual else NV
+    x = np.resize(rand_dt(r, (911, K), F16), (M, K))
+    wd, xd = ops.dev(rand_dt(r, (NV, K), F16, 0.02)), ops.dev(x)
+    bias, res = (ops.dev(rand_dt(r, (n,), F16)), rand_dt(r, (M, n), F16)) if both else (None, None)
+
+    def run(row, rows):
+        out, d_res = ops.DevBuf(rows * n * 2).fill_bytes(0xEE), ops.dev(res[row:row + rows]) if both else None
+        ops.lib().vra_dense_frag_gemm(xd.ptr + row * K * 2, wd.ptr, bias.ptr if both else None, d_res.ptr if both else None, out.ptr, rows, K, NV, int(dual), F16,
+                                      256 | (2 << 16 if form == "split" else 0), 0)
+        ops.check_error()
+        return out.numpy(np.uint16, (rows, n))
+    whole = run(0, M)
+    assert np.array_equal(whole[:part], run(0, part)) and np.array_equal(whole[-part:], run(M - part, part)) and whole.any(axis=1).all()
+    ops.lib().vra_device_sync()
+    assert ops.lib().vra_take_device_error() == 0

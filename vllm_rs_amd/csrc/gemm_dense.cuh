@@ -23,8 +23,8 @@
 //     4 m-frags x BN/64 n-frags x 2 k-halves = 32 MFMAs at BN = 256), each  { LDS reads of the phase's operands | staging units of LDS-DMA
 //     issued | counted vmcnt, lgkmcnt(0) | barrier | MFMAs | barrier }.  The two wave groups (m halves; one wave of each per
 //     SIMD) run ONE barrier apart, so one group's MFMAs cover the other's LDS reads and DMA issue.  The operands come from LDS only: no wait
-//     states between the MFMAs (with them a group's 16 take 296 clocks instead of 256).  Against phases of 16 MFMAs, 8192 x 8192 x 8192:
-//     769 -> 750 us, 2048 clocks of MFMAs in 2240; what is left is the clock, 1.3..1.5 GHz at this power;
+//     states between the MFMAs (with them a group's 16 take 296 clocks instead of 256).  2048 clocks of MFMAs in 2240; what is left is the
+//     clock, 1.3..1.5 GHz at this power;
 //   * two 64 KiB LDS buffers (even / odd K-step), recycled per STAGING UNIT (16 KiB at BN = 256): U0 = the first 64 rows of both
 //     groups' x, U2 = the other 64, U3 = the first half of every wave's columns, U1 = the other half.  Phase 0 reads U0, U3 and U1
 //     (the columns' fragments stay in registers for phase 1), phase 1 reads U2.  A unit is re-staged one phase after its last read (both wave
@@ -32,6 +32,10 @@
 //     unit has a K-step to land, with two buffers.  After issuing a phase's units a wave waits `vmcnt` down to the newest K-step's
 //     worth of them; what leaves the count is read in the NEXT phase (one barrier later: LDS-DMA data is ordered for a reader only by the
 //     issuing wave's count plus a barrier the reader has passed).  vmcnt never reaches 0 inside the loop;
+//   * FOUR phases (a quadrant each, upper rows x U3, upper x U1, lower x U1, lower x U3: 16 MFMAs) where x is large and K long: six of a K-step's eight requests in
+//     one phase come back later once the operands lie in memory and not in the last-level cache.  One unit is staged a phase, two or three
+//     phases after its last read (so lgkmcnt(0) can stand behind the barrier): phase 0 stages U1(t+1), phase 1 U2(t+1), phase 2 U0(t+2), phase 3
+//     U3(t+2); the wait is down to the four newest units, the unit that leaves the count was issued four phases earlier;
 //   * workgroup ids are remapped so that the workgroups of one XCD (ids = xcd mod 8) work on neighbouring tiles: about 8 m-tiles
 //     x 4 n-tiles in flight per XCD share their x and w panels in that XCD's L2;
 //   * DUAL (gate/up): the dequant pass interleaves the two tensors fragment by fragment (g0 u0 g1 u1 ...), a wave then holds gate
@@ -129,19 +133,19 @@ __device__ __forceinline__ int gx_slot_xor(int row) {
   return (a >> 1) | (((a ^ (a >> 1)) & 1) << 1);
 }
 
-template <class DT, int BM, int BN, bool DUAL>
+template <class DT, int BM, int BN, bool DUAL, int PH>  // PH: phases of a K-step
 __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int NF = BN / 16;    // n-frags of the tile
   constexpr int WNF = NF / 4;    // n-frags of a wave (4 | 2)
   constexpr int HNF = WNF / 2;   // ... of one unit
-  constexpr int MF = BM / 64;    // m-frags of a wave and phase (4 | 3)
+  constexpr int MF = BM / 64;    // m-frags of one unit and wave (4 | 3)
   constexpr int XB = BM / 16 * 2 * 1024;  // bytes of x per buffer: the m-frags x 2 k-chunks
   constexpr int WB = NF * 2 * 1024;
   constexpr int BUF = XB + WB;
-  constexpr int WPU = HNF * 8 / 8;  // LDS-DMA instructions per wave for a unit of w: 4 waves' worth of HNF n-frags x 2 k-chunks over 8 waves
   constexpr int VMW = MF + 2 * (HNF == 2 ? 2 : 1);  // DMA instructions of a wave and K-step (the newest unit of each kind)
   constexpr uint32_t RSRC3 = 0x00020000u;
+  static_assert(PH == 2 || PH == 4, "phases");
   static_assert(BM == 256 ? BN == 256 || BN == 128 : BM == 192 && BN == 256, "tile");
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -234,9 +238,9 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
 #pragma unroll
       for (int kc = 0; kc < 2; kc++) xa[i][kc] = *reinterpret_cast<const s16x8*>(xrd + buf * BUF + ((mh * MF + i) * 2 + kc) * 1024);
   };
-  auto read_w = [&](int buf) {
+  auto read_w = [&](int buf, int j0, int j1) {
 #pragma unroll
-    for (int j = 0; j < WNF; j++)
+    for (int j = j0; j < j1; j++)
 #pragma unroll
       for (int kc = 0; kc < 2; kc++) wa[j][kc] = *reinterpret_cast<const s16x8*>(wrd + buf * BUF + (j * 2 + kc) * 1024);
   };
@@ -246,12 +250,13 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
   for (int i = 0; i < 2 * MF; i++)
 #pragma unroll
     for (int j = 0; j < WNF; j++) acc[i][j] = vra_zero_acc();
-  // waits for the phase's own LDS reads and the next phase's units, then the matrix work between two barriers.  A = weights (16 columns x
-  // 32 k), B = x (16 rows x 32 k): D[column][row]
-  auto compute = [&](auto MH) {
-    constexpr int mh = decltype(MH)::value;
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(VMW) : "memory");
+  // waits for the phase's own LDS reads and the next phase's units, then the matrix work of rows mh x n-frags j0..j1 - 1 between two barriers.
+  // A = weights (16 columns x 32 k), B = x (16 rows x 32 k): D[column][row]
+  auto compute = [&](int mh, int j0, int j1) {
+    if constexpr (PH == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(VMW) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(VMW) : "memory");
     __builtin_amdgcn_s_barrier();
+    if constexpr (PH == 4) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -259,7 +264,7 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
 #pragma unroll
       for (int i = 0; i < MF; i++)
 #pragma unroll
-        for (int j = 0; j < WNF; j++) DT::mfma_ready(acc[mh * MF + i][j], wa[j][kc], xa[i][kc]);
+        for (int j = j0; j < j1; j++) DT::mfma_ready(acc[mh * MF + i][j], wa[j][kc], xa[i][kc]);
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
@@ -269,30 +274,46 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
 
   // this workgroup's K-steps (an even count: launcher) — all of them, or slice zi of SK
   const int ks0 = KS / SK * zi, ks1 = ks0 + KS / SK;
-  // ---- prologue: the first K-step entirely, U0 / U3 / U1 of the second (the order the counted waits assume: oldest first)
+  // ---- prologue: the first K-step entirely, U0 / U3 (two phases: and U1) of the second (the order the counted waits assume: oldest first)
   stage_x(0, 0, ks0);
   stage_w(0, 0, ks0);
   stage_w(0, 1, ks0);
   stage_x(0, 1, ks0);
   stage_x(1, 0, ks0 + 1);
   stage_w(1, 0, ks0 + 1);
-  stage_w(1, 1, ks0 + 1);
+  if constexpr (PH == 2) stage_w(1, 1, ks0 + 1);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(VMW) : "memory");
   __builtin_amdgcn_s_barrier();
   if (wr == 1) __builtin_amdgcn_s_barrier();  // the second wave group runs one barrier behind the first
 
   auto kstep = [&](auto BUFC, int ks) {
     constexpr int b = decltype(BUFC)::value;
-    read_w(b);
-    __builtin_amdgcn_sched_barrier(0);
-    read_x(b, 0);
-    stage_x(b ^ 1, 1, ks + 1);
-    compute(C0{});
-    read_x(b, 1);
-    stage_x(b, 0, ks + 2);
-    stage_w(b, 0, ks + 2);
-    stage_w(b, 1, ks + 2);
-    compute(C1{});
+    if constexpr (PH == 2) {
+      read_w(b, 0, WNF);
+      __builtin_amdgcn_sched_barrier(0);
+      read_x(b, 0);
+      stage_x(b ^ 1, 1, ks + 1);
+      compute(0, 0, WNF);
+      read_x(b, 1);
+      stage_x(b, 0, ks + 2);
+      stage_w(b, 0, ks + 2);
+      stage_w(b, 1, ks + 2);
+      compute(1, 0, WNF);
+    } else {
+      read_w(b, 0, HNF);
+      __builtin_amdgcn_sched_barrier(0);
+      read_x(b, 0);
+      stage_w(b ^ 1, 1, ks + 1);
+      compute(0, 0, HNF);
+      read_w(b, HNF, WNF);
+      stage_x(b ^ 1, 1, ks + 1);
+      compute(0, HNF, WNF);
+      read_x(b, 1);
+      stage_x(b, 0, ks + 2);
+      compute(1, HNF, WNF);
+      stage_w(b, 0, ks + 2);
+      compute(1, 0, HNF);
+    }
   };
   for (int ks = ks0; ks < ks1; ks += 2) {
     kstep(C0{}, ks);

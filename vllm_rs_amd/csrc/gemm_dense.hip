@@ -14,17 +14,17 @@ static int gx_cur_dev() {
   return dev & 63;
 }
 
-template <class DT, int BM, int BN, bool DUAL>
+template <class DT, int BM, int BN, bool DUAL, int PH>
 static void launch_gemm_dense_t(const GemmXArgs& a, hipStream_t st) {
   const size_t lds = gemm_dense_lds_bytes(BM, BN);
   static uint64_t attr_devs = 0;  // per device: function attributes belong to the device current at the call
   if (!((attr_devs >> gx_cur_dev()) & 1)) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dense_kernel<DT, BM, BN, DUAL>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dense_kernel<DT, BM, BN, DUAL, PH>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr_devs |= (uint64_t)1 << gx_cur_dev();
   }
   const int tiles = a.MT * a.NT;
   const unsigned grid = a.tail_sk > 1 ? (unsigned)(a.tail_first + (tiles - a.tail_first) * a.tail_sk) : (unsigned)(tiles * (a.splitk > 1 ? a.splitk : 1));
-  gemm_dense_kernel<DT, BM, BN, DUAL><<<dim3(grid), GX_THREADS, lds, st>>>(a);
+  gemm_dense_kernel<DT, BM, BN, DUAL, PH><<<dim3(grid), GX_THREADS, lds, st>>>(a);
 }
 
 static int gx_num_cus() {
@@ -36,8 +36,8 @@ static int gx_num_cus() {
 
 // tile (256 rows x 256 | 128 columns, 192: that many rows x 256 columns) and split-K factor (<< 16) for an M x nv x K problem
 int vra_gemm_dense_tile(int M, int nv, int K) {
-  static const char* env = getenv("VRA_GX_BN");  // tuning aid: width | splitk << 16
-  if (env && ((atoi(env) & 0xffff) == 128 || (atoi(env) & 0xffff) == 256)) return atoi(env);
+  static const char* env = getenv("VRA_GX_BN");  // tuning aid: width (or 192: rows of 256 columns) | splitk << 16
+  if (env && ((atoi(env) & 0xffff) == 128 || (atoi(env) & 0xffff) == 256 || atoi(env) == 192)) return atoi(env);
   const int cus = gx_num_cus();
   const long mt = (M + 255) / 256;
   const long t256 = mt * ((nv + 255) / 256), t128 = mt * ((nv + 127) / 128);
@@ -117,20 +117,27 @@ void vra_launch_gemm_dense(GemmXArgs a, bool dual, int dtype, int bn_sk, int64_t
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool bf = dtype == VRA_BF16;
-#define VRA_GX(BMV, BNV, DU)                                   \
-  do {                                                         \
-    if (bf) launch_gemm_dense_t<BF16, BMV, BNV, DU>(a, st);    \
-    else launch_gemm_dense_t<F16, BMV, BNV, DU>(a, st);        \
+  // 256 x 256, x of 120 MiB up and K from 12288 on: four phases a K-step instead of two (the bits are the same).  us, two / four: 8192 rows x 3584, K = 14336
+  // 650 / 616; 5200 x 8192, K = 14336 974 / 934; 8192 x 4096, K = 14336 683 / 660, in a model's step 679 / 637; 4700 x 3584, K = 28672 797 / 750; below the line two are
+  // faster: 4096 x 4096, K = 14336 310 / 319; 8192 x 4096, K = 11008 489 / 498; 8192 x 8192 x 8192 751 / 762 (profiles/kernel_x_phases.txt)
+  const bool quarters = a.K >= 12288 && (int64_t)a.M * a.K * 2 >= ((int64_t)120 << 20);
+#define VRA_GX(BMV, BNV, DU, PH)                                \
+  do {                                                          \
+    if (bf) launch_gemm_dense_t<BF16, BMV, BNV, DU, PH>(a, st); \
+    else launch_gemm_dense_t<F16, BMV, BNV, DU, PH>(a, st);     \
   } while (0)
   if (bm == 192) {
-    if (dual) VRA_GX(192, 256, true);
-    else VRA_GX(192, 256, false);
+    if (dual) VRA_GX(192, 256, true, 2);
+    else VRA_GX(192, 256, false, 2);
+  } else if (bn == 256 && quarters) {
+    if (dual) VRA_GX(256, 256, true, 4);
+    else VRA_GX(256, 256, false, 4);
   } else if (bn == 256) {
-    if (dual) VRA_GX(256, 256, true);
-    else VRA_GX(256, 256, false);
+    if (dual) VRA_GX(256, 256, true, 2);
+    else VRA_GX(256, 256, false, 2);
   } else {
-    if (dual) VRA_GX(256, 128, true);
-    else VRA_GX(256, 128, false);
+    if (dual) VRA_GX(256, 128, true, 2);
+    else VRA_GX(256, 128, false, 2);
   }
 #undef VRA_GX
 }
