@@ -295,6 +295,8 @@ void vra_dense_gemm(const void* x, const void* w, const void* bias, void* out, i
 void vra_dense_gemm_tile(int32_t tile, const void* x, const void* const* w, const void* const* bias, const int32_t* n, int32_t nseg,
                          int32_t pair, const void* residual, void* const* out, int32_t out_f32, int32_t m, int32_t k, int32_t dtype,
                          int64_t stream);
+/* the tile that the row-major prompt GEMM takes for m rows x nseg tensors of n[s] columns (0: no such product) */
+int32_t vra_dense_gemm_tile_choice(int32_t m, const int32_t* n, int32_t nseg, int32_t k);
 /* logits.argmax(-1) (logits_processor.rs:67-70): first maximal index per row. */
 void vra_argmax_f32(const float* logits, uint32_t* out, int32_t rows, int32_t cols, int64_t stream);
 /* lm_head + greedy sampling as one launch (llama.rs:311-320 followed by logits_processor.rs:67-70): f32 logits as

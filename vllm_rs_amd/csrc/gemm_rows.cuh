@@ -278,17 +278,19 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
 #endif
 }
 
-// Tile for a product of M rows x ncols[0..nseg) columns x `batch`: the least time by this model (us; 225 shapes of 33..8192 rows, 2048..14336 columns,
-// K = 1024..14336, weights from memory: within 2..8 % rms, and the tile it picks 0.2 % behind the best on average, 6 % at most): workgroups
-// run in rounds of `slots`; a launch costs t0, a round `round` (first requests, outputs) and `full` for 64 of K, the last round between `one` (a
-// few workgroups) and `full`.  64 x 128 has two forms (gemm_rows_launch).  192 x 128 is for what is a little more than one round of 128 x 128 and leaves
-// much of one of 128 x 256 idle; us without / with it: 2120 rows x 2048, K = 2048 31.7 / 26.5, K = 5632 67.2 / 56.2; 700 x 8192, K = 2048 35.1 / 30.5;
-// 300 x 14336, K = 4096 51.1 / 44.7; 1280 x 4096, K = 14336 163 / 135.  192 x 256 does the same between 128 x 256 and 256 x 256: 1500 x 8192, K = 2048
-// 57.2 / 48.8; 2120 x 4096, K = 4096 86.1 / 71.6; 2560 x 4096, K = 14336 272 / 235.  rows: only tiles of that many (0: any).
-// -> rows / 64 * 16 + columns / 64; *us: the time
+// Tile for a product of M rows x ncols[0..nseg) columns x `batch`: the least time by this model (us; 3079 shapes of 33..6000 rows, 1024..28672 columns,
+// K = 512..18944, weights from memory: within 6..12 % rms, and the tile it picks 0.05 % behind the best on average, 7 % at most; every third of the
+// shapes in profiles/gemm_rows_tile_times.txt): workgroups run in rounds of `slots`; a launch costs t0, a round `round` (first requests, outputs) and `full` for
+// 64 of K, the last round between `one` (a few workgroups; `half`: every CU with one of its two) and `full`.  64 x 128 has two forms (gemm_rows_launch).
+// With weights from the last-level cache 64 x 128 on two workgroups a CU is as fast as 128 x 128; from memory it is not: 192 rows x 14336, K = 4096 57 / 40 us, 700 x
+// 4096, K = 2048 27 / 20.  192 x 128 is for what is a little more than one round of 128 x 128 and leaves much of one of 128 x 256 idle; us without / with it: 2120
+// rows x 2048, K = 2048 31.7 / 26.5, K = 5632 67.2 / 56.2; 700 x 8192, K = 2048 35.1 / 30.5; 1280 x 4096, K = 14336 163 / 135.  192 x 256 does the same between
+// 128 x 256 and 256 x 256: 1500 x 8192, K = 2048 57.2 / 48.8; 2120 x 4096, K = 4096 86.1 / 71.6; 2560 x 4096, K = 14336 272 / 235.
+// rows: only tiles of that many (0: any).  -> rows / 64 * 16 + columns / 64; *us: the time
 static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch, int K, int rows = 0, double* us = nullptr) {
-  const struct { int bm, bn, slots; double t0, round, one, full; } t[7] = {{256, 256, 256, 2.0, 14.4, 0.79, 1.39}, {192, 256, 256, 1.0, 10.0, 0.56, 1.10}, {128, 256, 256, 0.7, 9.5, 0.52, 0.78},
-      {192, 128, 256, 1.0, 6.5, 0.40, 0.64}, {128, 128, 256, 1.4, 5.4, 0.35, 0.50}, {64, 128, 512, 2.6, 2.4, 0.27, 0.60}, {64, 128, 256, 3.7, 1.3, 0.28, 0.34}};
+  const struct { int bm, bn, slots; double t0, round, one, half, full; } t[7] = {{256, 256, 256, 1.3, 9.2, 0.91, 0, 1.30}, {192, 256, 256, 1.0, 8.1, 0.72, 0, 1.00},
+      {128, 256, 256, 0.5, 5.4, 0.70, 0, 0.81}, {192, 128, 256, 0.5, 5.0, 0.55, 0, 0.64}, {128, 128, 256, 1.3, 3.5, 0.41, 0, 0.51},
+      {64, 128, 512, 3.2, 1.7, 0.34, 0.58, 0.66}, {64, 128, 256, 3.6, 0.0, 0.36, 0, 0.40}};
   int best = 0;
   double cost = 0.0;
   for (const auto& c : t) {
@@ -298,7 +300,7 @@ static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch,
     const long tiles = (M + c.bm - 1) / c.bm * cols * batch, full = tiles / c.slots, rem = tiles % c.slots;
     if (c.bm == 64 && (tiles <= 256) != (c.slots == 256)) continue;
     double last = rem ? c.one + (c.full - c.one) * rem / c.slots : 0.0;
-    if (c.slots == 512 && rem) last = rem <= 256 ? c.one : 0.46 + (c.full - 0.46) * (rem - 256) / 256;  // (the second workgroup of a CU)
+    if (c.slots == 512 && rem) last = rem <= 256 ? c.one : c.half + (c.full - c.half) * (rem - 256) / 256;  // (the second workgroup of a CU)
     const double v = c.t0 + (full + (rem ? 1 : 0)) * c.round + K / 64 * (full * c.full + last);
     if (!best || v < cost) best = c.bm / 64 * 16 + c.bn / 64, cost = v;
   }

@@ -136,3 +136,7 @@ extern "C" void vra_dense_gemm_tile(int32_t tile, const void* x, const void* con
   VRA_CHECK_ARG(vra_gemm_rows_takes(r), "dense gemm tile: a shape or an alignment that these tiles do not take");
   vra_launch_gemm_rows(r, dtype, stream);
 }
+
+extern "C" int32_t vra_dense_gemm_tile_choice(int32_t m, const int32_t* n, int32_t nseg, int32_t k) {
+  return m > 0 && n && nseg >= 1 && nseg <= GR_MAX_SEG && k > 0 ? gemm_rows_tile(m, n, nseg, 1, k) : 0;
+}

@@ -25,8 +25,8 @@ struct GemmRowsCall {
   int tile = 0;  // rows / 64 * 16 + columns / 64 instead of gemm_rows_tile's choice
 };
 // whether the product can run here and is expected to be faster than on kernel B (and behind it the element-wise launches the fused form
-// saves).  Measured, bf16, cold weights, us (here / kernel B): 64 rows, 2048 x 5632: 50 / 22; 128 rows, 5632 x 2048: 24 / 34; 256 rows, 4096 x 4096:
-// 40 / 39; 400 rows, 14336 x 4096: 80 / 234; 2120 rows, 2048 x 5632: 95 / 219
+// saves).  Measured, bf16, weights from memory, us (here / kernel B): 64 rows x 8192, K = 11008 89 / 66; 128 x 4096, K = 5632 41 / 38; 192 x 2048, K = 2048 17 / 20;
+// 192 x 4096, K = 14336 98 / 112; 256 x 2048, K = 8192 52 / 42; 384 x 2048, K = 8192 51 / 64; beyond, the fused forms win: 2120 x 5632, K = 2048 95 / 219
 bool vra_gemm_rows_fits(const GemmRowsCall& c);
 bool vra_gemm_rows_takes(const GemmRowsCall& c);  // whether it can
 void vra_launch_gemm_rows(const GemmRowsCall& c, int dtype, int64_t stream);
