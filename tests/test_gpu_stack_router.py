@@ -20,9 +20,9 @@ def picks(z, top):
     return out
 
 
-# one output, up to and beyond one and two a lane, the largest that lanes keep marks for and one more (picked by one thread)
+# one output, rounds of one to five outputs a wave, up to and beyond one and two a lane, the largest that lanes keep marks for and one more (picked by one thread)
 @pytest.mark.parametrize("dt", [BF16, F32])
-@pytest.mark.parametrize("E,top", [(1, 1), (17, 3), (64, 64), (65, 6), (160, 8), (4096, 4), (4097, 4)])
+@pytest.mark.parametrize("E,top", [(1, 1), (6, 2), (11, 2), (17, 3), (64, 64), (65, 6), (160, 8), (4096, 4), (4097, 4)])
 @pytest.mark.parametrize("gate", [0, 1])
 def test_picks(gate, E, top, dt):
     r = rng(E + gate)

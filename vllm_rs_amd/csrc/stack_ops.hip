@@ -78,8 +78,10 @@ __device__ __forceinline__ float wave_fold(float v, F f) {
 // (ROUTER a template parameter and 8 waves a SIMD: a norm that carries the router's registers, or a router with the 74 it would take, leaves room for 6
 // waves, and 2048 rows are two rounds of workgroups.  2048 rows, us: norm of 2048 7.6 -> 6.8, of 2051 12.4 -> 9.5; with eight router
 // outputs 21.1 -> 19.1, of 1001 17.6 -> 13.3.  The picks by a wave and not by one thread, five outputs of a wave and not four in a round: 1500 rows of
-// 2048, 16 outputs and a gate 22.0 -> 15.2; 64 outputs, eight picks 76.6 -> 21.7; 160 outputs 163 -> 74)
-template <typename T, bool ROUTER>
+// 2048, 16 outputs and a gate 22.0 -> 15.2; 64 outputs, eight picks 76.6 -> 21.7; 160 outputs 163 -> 74.  A wave's outputs of a round
+// counted ahead of the loop over the row, not tested in it: 8 rows of 12288, eight outputs 20.2 -> 15.6.  PARTS a template parameter too, and a row without
+// parts asked for ahead of its weights: 1500 rows of 2048 5.64 -> 5.33, the other way about 5.43)
+template <typename T, bool ROUTER, bool PARTS>
 __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
   extern __shared__ float lds[];
   float* xs = lds;                      // [W] the row, then the normalised row
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
     }
     __syncthreads();
   };
-  const float gt = a.gate_in ? a.gate_in[t] : 1.f;
+  const float gt = PARTS && a.gate_in ? a.gate_in[t] : 1.f;
   const bool quads = W % 4 == 0 && gs % 4 == 0 && (((uintptr_t)a.x | (uintptr_t)a.x_out | (uintptr_t)a.o | (uintptr_t)a.p1 | (uintptr_t)a.p2 | (uintptr_t)a.w) % 16) == 0;
   if (quads) {
     // (four values a load where rows and groups allow it, two loads of every part of the row ahead of the first sum: its parts arrive in one round trip
@@ -124,31 +126,26 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
         for (int n = 0; n < R; n++) s[n] += d[n];
       };
       read(x, v);
-      if (a.o) {
-        const float* const p1 = a.p1 + (size_t)t * a.n1 * W;
-        read(a.o + (size_t)t * W, s);
-        if (a.n1 > 0) read(p1, s1);
-        if (a.n1 > 1) read(p1 + W, s2);
-        if (a.p2) read(a.p2 + (size_t)t * W, s3);
-        if (a.n1 > 0) add(s1);
-        if (a.n1 > 1) add(s2);
-        for (int j = 2; j < a.n1; j++) {
-          read(p1 + (size_t)j * W, s1);
-          add(s1);
-        }
-        if (a.p2) {
+      const float* const p1 = a.p1 + (size_t)t * a.n1 * W;
+      read(a.o + (size_t)t * W, s);
+      if (a.n1 > 0) read(p1, s1);
+      if (a.n1 > 1) read(p1 + W, s2);
+      if (a.p2) read(a.p2 + (size_t)t * W, s3);
+      if (a.n1 > 0) add(s1);
+      if (a.n1 > 1) add(s2);
+      for (int j = 2; j < a.n1; j++) {
+        read(p1 + (size_t)j * W, s1);
+        add(s1);
+      }
+      if (a.p2) {
 #pragma unroll
-          for (int n = 0; n < R; n++) s[n] += gt * s3[n];
-        }
-#pragma unroll
-        for (int n = 0; n < R; n++) v[n] += a.mult * s[n];
+        for (int n = 0; n < R; n++) s[n] += gt * s3[n];
       }
 #pragma unroll
+      for (int n = 0; n < R; n++) v[n] += a.mult * s[n];
+#pragma unroll
       for (int n = 0; n < R; n++)
-        if (c0 + n * 1024 < W) {
-          *(f32x4*)(xs + c0 + n * 1024) = v[n];
-          if (a.o) *(f32x4*)(a.x_out + (size_t)t * W + c0 + n * 1024) = v[n];
-        }
+        if (c0 + n * 1024 < W) *(f32x4*)(xs + c0 + n * 1024) = *(f32x4*)(a.x_out + (size_t)t * W + c0 + n * 1024) = v[n];
     };
     auto put = [&](int c, f32x4 v, f32x4 w) {
       const f32x4 y = v * rs[c / gs] * w;
@@ -156,15 +153,29 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
 #pragma unroll
       for (int e = 0; e < 4; e++) El<T>::st(h + c + e, y[e]);
     };
-    for (int c = threadIdx.x * 4 + R * 1024; c < W; c += R * 1024) {
-      f32x4 v[R];
-      load(c, v);  // (ahead of what stays in registers)
-    }
-    load(threadIdx.x * 4, keep);
+    if constexpr (PARTS) {
+      for (int c = threadIdx.x * 4 + R * 1024; c < W; c += R * 1024) {
+        f32x4 v[R];
+        load(c, v);  // (ahead of what stays in registers)
+      }
+      load(threadIdx.x * 4, keep);
 #pragma unroll
-    for (int n = 0; n < R; n++) {
-      const int c = threadIdx.x * 4 + n * 1024;
-      if (c < W) wt[n] = *(const f32x4*)(a.w + c);
+      for (int n = 0; n < R; n++) {
+        const int c = threadIdx.x * 4 + n * 1024;
+        if (c < W) wt[n] = *(const f32x4*)(a.w + c);
+      }
+    } else {  // (the row alone: its weights with it)
+#pragma unroll
+      for (int n = 0; n < R; n++) {
+        const int c = threadIdx.x * 4 + n * 1024;
+        if (c < W) keep[n] = *(const f32x4*)(x + c), wt[n] = *(const f32x4*)(a.w + c);
+      }
+#pragma unroll
+      for (int n = 0; n < R; n++) {
+        const int c = threadIdx.x * 4 + n * 1024;
+        if (c < W) *(f32x4*)(xs + c) = keep[n];
+      }
+      for (int c = threadIdx.x * 4 + R * 1024; c < W; c += 1024) *(f32x4*)(xs + c) = *(const f32x4*)(x + c);
     }
     sums();
 #pragma unroll
@@ -174,7 +185,7 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
     }
     for (int c = threadIdx.x * 4 + R * 1024; c < W; c += 1024) put(c, *(const f32x4*)(xs + c), *(const f32x4*)(a.w + c));
   } else {
-    if (a.o) {
+    if constexpr (PARTS) {
       for (int c = threadIdx.x; c < W; c += 256) {
         float s = a.o[(size_t)t * W + c];
         for (int j = 0; j < a.n1; j++) s += a.p1[((size_t)t * a.n1 + j) * W + c];
@@ -198,32 +209,38 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
   const int nz = a.n_router + (a.gate_row ? 1 : 0);
   const T* rw = (const T*)a.router_w;
   if (sizeof(T) == 2 && W % 8 == 0 && ((uintptr_t)rw % 16) == 0) {  // 8 weights a load; the lane's partial sums keep one order for a given W
-    constexpr int Q = 5;
-    for (int e0 = wave; e0 < nz; e0 += 4 * Q) {  // up to five outputs of a wave side by side: their weights are under way together, the row is read once
+    auto dots = [&](auto N, int e0) {  // N outputs of a wave side by side: their weights are under way together, the row is read once
+      constexpr int Q = decltype(N)::value;
       float s[Q] = {};
       for (int c = lane * 8; c < W; c += 64 * 8) {
         u32x4 v[Q];
 #pragma unroll
-        for (int q = 0; q < Q; q++)
-          if (e0 + q * 4 < nz) v[q] = *(const u32x4*)((const uint16_t*)rw + (size_t)(e0 + q * 4) * W + c);
+        for (int q = 0; q < Q; q++) v[q] = *(const u32x4*)((const uint16_t*)rw + (size_t)(e0 + q * 4) * W + c);
         float f[8];
 #pragma unroll
         for (int i = 0; i < 8; i++) f[i] = xs[c + i];
 #pragma unroll
         for (int q = 0; q < Q; q++)
-          if (e0 + q * 4 < nz)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-              s[q] = fmaf(f[2 * i], __uint_as_float(v[q][i] << 16), s[q]);
-              s[q] = fmaf(f[2 * i + 1], __uint_as_float(v[q][i] & 0xffff0000u), s[q]);
-            }
+          for (int i = 0; i < 4; i++) {
+            s[q] = fmaf(f[2 * i], __uint_as_float(v[q][i] << 16), s[q]);
+            s[q] = fmaf(f[2 * i + 1], __uint_as_float(v[q][i] & 0xffff0000u), s[q]);
+          }
       }
 #pragma unroll
-      for (int q = 0; q < Q; q++)
-        if (e0 + q * 4 < nz) {
-          s[q] = wave_fold(s[q], [](float p, float r) { return p + r; });
-          if (lane == 0) zs[e0 + q * 4] = s[q];
-        }
+      for (int q = 0; q < Q; q++) {
+        s[q] = wave_fold(s[q], [](float p, float r) { return p + r; });
+        if (lane == 0) zs[e0 + q * 4] = s[q];
+      }
+    };
+    for (int e0 = wave; e0 < nz; e0 += 20) {
+      switch (min((nz - e0 + 3) / 4, 5)) {
+        case 1: dots(std::integral_constant<int, 1>{}, e0); break;
+        case 2: dots(std::integral_constant<int, 2>{}, e0); break;
+        case 3: dots(std::integral_constant<int, 3>{}, e0); break;
+        case 4: dots(std::integral_constant<int, 4>{}, e0); break;
+        default: dots(std::integral_constant<int, 5>{}, e0);
+      }
     }
   } else {
     for (int e = wave; e < nz; e += 4) {
@@ -1803,8 +1820,13 @@ void vra_stack_group_norm(const StkNormArgs& a, int dtype, int64_t stream) {
   const size_t lds = ((size_t)a.W + a.groups + a.n_router + 2) * sizeof(float);
   VRA_CHECK_ARG(lds <= 64 * 1024, "stack norm: row does not fit LDS");
   launch_checked("stack norm", [&] {
-    if (dtype == VRA_F32) a.router_w ? stk_group_norm_kernel<float, true><<<a.T, 256, lds, as_stream(stream)>>>(a) : stk_group_norm_kernel<float, false><<<a.T, 256, lds, as_stream(stream)>>>(a);
-    else a.router_w ? stk_group_norm_kernel<uint16_t, true><<<a.T, 256, lds, as_stream(stream)>>>(a) : stk_group_norm_kernel<uint16_t, false><<<a.T, 256, lds, as_stream(stream)>>>(a);
+    auto go = [&](auto router, auto parts) {
+      constexpr bool RT = decltype(router)::value, PA = decltype(parts)::value;
+      if (dtype == VRA_F32) stk_group_norm_kernel<float, RT, PA><<<a.T, 256, lds, as_stream(stream)>>>(a);
+      else stk_group_norm_kernel<uint16_t, RT, PA><<<a.T, 256, lds, as_stream(stream)>>>(a);
+    };
+    if (a.router_w) a.o ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+    else a.o ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
   });
 }
 
