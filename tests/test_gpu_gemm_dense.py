@@ -205,7 +205,7 @@ def test_marlin_ffi_long_prefill(dense_from):
     assert not ws.numpy(np.uint32, (N,)).any()
 
 
-# x of 120 MiB up and K from 12288 on: four phases a K-step on 256 x 256 tiles
+# x of 120 MiB up and K from 12288 on, or 192 MiB of weights: four phases a K-step on 256 x 256 tiles
 @pytest.mark.parametrize("form,NV", [("plain", 528), ("bias residual", 80), ("gate up", 544), ("split", 272)])
 def test_large_x_has_the_bits_of_small_ones(form, NV):
     """rows of a large product, the first and the last of it, equal the same rows alone, which run in two phases"""

@@ -32,7 +32,7 @@
 //     unit has a K-step to land, with two buffers.  After issuing a phase's units a wave waits `vmcnt` down to the newest K-step's
 //     worth of them; what leaves the count is read in the NEXT phase (one barrier later: LDS-DMA data is ordered for a reader only by the
 //     issuing wave's count plus a barrier the reader has passed).  vmcnt never reaches 0 inside the loop;
-//   * FOUR phases (a quadrant each, upper rows x U3, upper x U1, lower x U1, lower x U3: 16 MFMAs) where x is large and K long: six of a K-step's eight requests in
+//   * FOUR phases (a quadrant each, upper rows x U3, upper x U1, lower x U1, lower x U3: 16 MFMAs) where the weights, or x and K, are large: six of a K-step's eight requests in
 //     one phase come back later once the operands lie in memory and not in the last-level cache.  One unit is staged a phase, two or three
 //     phases after its last read (so lgkmcnt(0) can stand behind the barrier): phase 0 stages U1(t+1), phase 1 U2(t+1), phase 2 U0(t+2), phase 3
 //     U3(t+2); the wait is down to the four newest units, the unit that leaves the count was issued four phases earlier;

@@ -117,10 +117,12 @@ void vra_launch_gemm_dense(GemmXArgs a, bool dual, int dtype, int bn_sk, int64_t
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool bf = dtype == VRA_BF16;
-  // 256 x 256, x of 120 MiB up and K from 12288 on: four phases a K-step instead of two (the bits are the same).  us, two / four: 8192 rows x 3584, K = 14336
-  // 650 / 616; 5200 x 8192, K = 14336 974 / 934; 8192 x 4096, K = 14336 683 / 660, in a model's step 679 / 637; 4700 x 3584, K = 28672 797 / 750; below the line two are
-  // faster: 4096 x 4096, K = 14336 310 / 319; 8192 x 4096, K = 11008 489 / 498; 8192 x 8192 x 8192 751 / 762 (profiles/kernel_x_phases.txt)
-  const bool quarters = a.K >= 12288 && (int64_t)a.M * a.K * 2 >= ((int64_t)120 << 20);
+  // 256 x 256: four phases a K-step instead of two (the bits are the same) where much of what a K-step asks for comes from memory (profiles/kernel_x_phases.txt).
+  // 192 MiB of weights up, which the pass ahead of the product has just written; us of both, two / four: 768 rows, gate/up of 4096 x 14336 231 / 214; 1024 x 8192,
+  // K = 28672 467 / 446; 2048 x 6144, K = 16384 392 / 348; 1280 x 24576, K = 12288 708 / 672; 4096 rows, gate/up of 4096 x 14336 757 / 756.
+  // x of 120 MiB up and K from 12288 on: 8192 rows x 3584, K = 14336 650 / 616; 8192 x 4096, K = 14336 683 / 660, in a model's step 679 / 637.  Below both lines
+  // two are faster: 1280 x 4096, K = 14336 158 / 162; 1536 x 3584, K = 18944 200 / 206; 8192 x 8192 x 8192 751 / 762
+  const bool quarters = (int64_t)a.NV * a.K * 2 >= ((int64_t)192 << 20) || (a.K >= 12288 && (int64_t)a.M * a.K * 2 >= ((int64_t)120 << 20));
 #define VRA_GX(BMV, BNV, DU, PH)                                \
   do {                                                          \
     if (bf) launch_gemm_dense_t<BF16, BMV, BNV, DU, PH>(a, st); \
