@@ -162,6 +162,10 @@ void vra_wna16_dequant_frag(const void* qweight_tiled, const void* scales, const
  * fragments, out[m, nv/2] = silu(x.Wg) * (x.Wu) (mlp.rs:451-469; no bias).  tile_n: 0 (chosen from the shape), 128, 256 or 192 (rows of 256 columns). */
 void vra_dense_frag_gemm(const void* x, const void* wd, const void* bias, const void* residual, void* out, int32_t m, int32_t k,
                          int32_t nv, int32_t dual, int32_t dtype, int32_t tile_n, int64_t stream);
+/* the same product of nseg (1..3) tensors of n[s] columns side by side, each with its own bias (or null) and output [m, n[s]]; every segment begins at a
+ * multiple of 64 columns */
+void vra_dense_frag_gemm_segments(const void* x, const void* wd, const void* const* bias, const int32_t* n, int32_t nseg, void* const* out, int32_t m,
+                                  int32_t k, int32_t dtype, int32_t tile_n, int64_t stream);
 
 /* candle_nn::RmsNorm::forward as used by NormX (src/models/layers/others.rs:11-29):
  * out[t,:] = x[t,:] * rsqrt(mean(x²)+eps) * w, f32 math, one rounding. */

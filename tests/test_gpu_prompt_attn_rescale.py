@@ -54,3 +54,33 @@ def test_rows_whose_maxima_move(profile, prefix, D, dt):
         v = vf[:, h * Hkv // Hq]
         ref, mag = p @ v / p.sum(1, keepdims=True), p @ np.abs(v) / p.sum(1, keepdims=True)
         assert (np.abs(got[:, h] - ref) <= 1.05 * unit * mag + 1e-6).all(), (h, float((np.abs(got[:, h] - ref) / (unit * mag)).max()))
+
+
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("ctxs,prefix", [([1, 33], 0), ([330, 97], 70), ([700], 0)])
+def test_block_sizes_and_the_fp8_cache(ctxs, prefix, D, dt):
+    """where a key or value lies changes no bit, nor does a cache of 8 bits whose numbers hold the values exactly"""
+    r = rng(D + sum(ctxs) + dt)
+    Hq, Hkv = 8, 2
+    lq = [c - min(prefix, c - 1) for c in ctxs]
+    k, v = (orc.to_dt((r.integers(-7, 8, (sum(ctxs), Hkv, D)) / 4.0).astype(np.float32), dt) for _ in range(2))  # (three bits behind the point)
+    q = orc.to_dt(r.standard_normal((sum(lq), Hq, D)).astype(np.float32), dt)
+    outs = []
+    for BS in (64, 32, 128):
+        for fp8 in (False, True):
+            need = [-(-c // BS) for c in ctxs]
+            perm = r.permutation(sum(need) + 2).astype(np.uint32)
+            bt = np.zeros((len(ctxs), max(need)), np.uint32)
+            for b, n in enumerate(need):
+                bt[b, :n] = perm[sum(need[:b]):sum(need[:b + 1])]
+            slots = np.concatenate([bt[b, np.arange(c) // BS].astype(np.int64) * BS + np.arange(c) % BS for b, c in enumerate(ctxs)])
+            bytes_ = (sum(need) + 2) * BS * Hkv * D * (1 if fp8 else 2)
+            kc, vc = (ops.DevBuf(bytes_).fill_bytes(0x7F if fp8 else 0xFF) for _ in range(2))  # (NaN)
+            pa = ops.PagedAttention(Hq, D, D ** -0.5, Hkv, BS, dt, fp8_kvcache=fp8)
+            pa.reshape_and_cache(ops.dev(k), ops.dev(v), kc, vc, ops.dev(slots), len(slots))
+            out = pa.forward_prefill(ops.dev(q), sum(lq), max(lq), ops.dev(np.concatenate([[0], np.cumsum(lq)]).astype(np.uint32)), len(ctxs), k_cache=kc, v_cache=vc,
+                                     block_tables=ops.dev(bt), context_lens=ops.dev(np.array(ctxs, np.uint32)), max_blocks=max(need))
+            outs.append(out.numpy(np.uint16, (sum(lq), Hq, D)))
+    assert np.isfinite(orc.from_dt(outs[0], dt)).all() and outs[0].any()
+    assert all(np.array_equal(o, outs[0]) for o in outs[1:])

@@ -252,3 +252,22 @@ extern "C" void vra_dense_frag_gemm(const void* x, const void* wd, const void* b
   a.M = m, a.NV = nv, a.K = k;
   vra_launch_gemm_dense(a, dual != 0, dtype, tile_n ? tile_n : vra_gemm_dense_tile(m, nv, k), stream);
 }
+extern "C" void vra_dense_frag_gemm_segments(const void* x, const void* wd, const void* const* bias, const int32_t* n, int32_t nseg, void* const* out, int32_t m,
+                                             int32_t k, int32_t dtype, int32_t tile_n, int64_t stream) {
+  VRA_CHECK_ARG(x && wd && bias && n && out && nseg >= 1 && nseg <= GX_MAX_SEG, "dense_frag_gemm_segments: null pointer or bad count");
+  VRA_CHECK_ARG(m >= 1 && k > 0 && k % 128 == 0, "dense_frag_gemm_segments: bad shape M=%d K=%d", m, k);
+  VRA_CHECK_ARG(dtype == VRA_BF16 || dtype == VRA_F16, "dense_frag_gemm_segments: dtype must be bf16/f16");
+  VRA_CHECK_ARG(tile_n == 0 || tile_n == 192 || (tile_n & 0xffff) == 128 || (tile_n & 0xffff) == 256, "dense_frag_gemm_segments: no such tile");
+  GemmXArgs a{};
+  int c0 = 0;
+  for (int s = 0; s < nseg; s++) {
+    VRA_CHECK_ARG(out[s] && n[s] > 0 && n[s] % 16 == 0 && c0 % 64 == 0, "dense_frag_gemm_segments: a segment begins at a multiple of 64 columns and has a multiple of 16");
+    a.seg[s] = GemmXSeg{out[s], bias[s], n[s], c0};
+    c0 += n[s];
+  }
+  if (tile_n >> 16 > 1) vra_scratch_init();
+  a.x = x, a.x_ld = k, a.wd = wd;
+  a.nseg = nseg;
+  a.M = m, a.NV = c0, a.K = k;
+  vra_launch_gemm_dense(a, false, dtype, tile_n ? tile_n : vra_gemm_dense_tile(m, c0, k), stream);
+}
