@@ -1,6 +1,6 @@
 // gemm_dense.cuh — "kernel X": the prefill GEMM on DEQUANTISED 16-bit weights, plus the pass that makes them.
 //
-// Why (round 6): kernel D (gemm_q4_big.cuh) converts int4 -> bf16 inside every 64-row workgroup and pays the exact per-group scale
+// Why: kernel D (gemm_q4_big.cuh) converts int4 -> bf16 inside every 64-row workgroup and pays the exact per-group scale
 // fix-up per accumulator: 3 VALU instructions per MFMA where one is free — 0.30-0.32 of the MFMA peak, and the same skeleton with
 // the conversion removed runs 1.08 PFLOP/s (profiles/r06_kernel_d_probes.txt).  A prompt of M rows repeats that conversion M/64
 // times per weight.  From ~700 rows on it is cheaper to dequantise a GEMM's weights ONCE into a scratch tensor (a streaming pass:
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(GX_THREADS, 2) void gemm_dense_kernel(const GemmXAr
     }
   }
 
-  // ---- epilogue, through LDS (round 6): a lane holds 4 columns x 1 row of each accumulator tile — stored from there, every store
+  // ---- epilogue, through LDS: a lane holds 4 columns x 1 row of each accumulator tile — stored from there, every store
   // instruction touches 16 rows in 32-byte pieces (and the residual is read the same way): a residual cost 13-20 us per tile round
   // that way (tools/gemm_dense_overhead.py: 2 K-steps 22.6 -> 35.8 us; now 21.4 -> 26.8; K = 4096 with residual 132-138 -> 121-126 us).  The rounded outputs (bias / SiLU*mul applied) go to LDS as a [256 rows][columns] tile
   // instead (row stride + 16 bytes: the 64 lanes of a ds_write_b64 cover all banks), and the workgroup stores WHOLE ROWS, 16 bytes per lane,

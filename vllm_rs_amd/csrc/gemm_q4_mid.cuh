@@ -11,7 +11,8 @@
 // conversions of a tile's later fragments lie between the MFMAs of its earlier ones.  Codes, scales and row sums are fetched by the first half
 // alone: it asks for them a phase earlier and so two and a half phases ahead.
 // us a launch with its row sums, both halves in step / so: gate/up of 4096 x 14336, 64 rows 37.6 / 34.6, 150 rows 57.7 / 54.8, 320 rows 104 / 97; down
-// of 18944 x 3584, 150 rows 46.7 / 43.7, 700 rows 218 / 186; AWQ 62.3 / 61.5, 113 / 112, 49.3 / 47.9, 237 / 219 (no shape more than 1.5 % slower).
+// of 18944 x 3584, 150 rows 46.7 / 43.7, 700 rows 218 / 186; AWQ 62.3 / 61.5, 113 / 112, 49.3 / 47.9, 237 / 219.  Where a
+// workgroup has few k-tiles the shift by a barrier shows: 300 rows, 2048 columns, K = 5632 AWQ 29.3 / 30.1, 192 x 4608, K = 3584 20.8 / 21.6; all else within 2 %.
 // Against kernel D or W: gate/up of 4096 x 14336 behind its norm, 150 rows 91 / 53; AWQ, 3584 x 18944, 320 rows 190 / 147.
 //
 // The zero points come off per k-tile, acc += s (acc_g - (C + z) Sx): acc never holds more than the result's own size.  (Taken off once behind the
@@ -74,8 +75,9 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_q4_mid_kernel(const GemmDArgs
   const int SK = a.splitk > 1 ? a.splitk : 1, zi = (int)blockIdx.z;
   const int kt0 = (int)((long)KT * zi / SK), kt1 = (int)((long)KT * (zi + 1) / SK);
 
-  // ---- DMA sources.  A wave fetches MB KiB of x (4 rows each), the codes of its block wm (the other wave of the column pair the other's),
-  // its own copy of its two blocks' scales (lanes 0..15) and zero points (lanes 16..19; the rest fetch the same again), and 4 MB row sums
+  // ---- DMA sources.  Every wave fetches MB KiB of x (4 rows each).  The first row half's waves (wm = 0) alone also fetch, for their pair of columns, the
+  // codes of both blocks, one copy of the blocks' scales (lanes 0..15) and zero points (lanes 16..19; the rest fetch the same again) and 8 MB row
+  // sums: MB + 4 requests a k-tile (PER) against MB
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, 0x7FFFFFF0, RSRC3);
   const __amdgpu_buffer_rsrc_t rw0 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(wt[0]), 0, 0x7FFFFFF0, RSRC3);
   const __amdgpu_buffer_rsrc_t rw1 = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(wt[1]), 0, 0x7FFFFFF0, RSRC3);
