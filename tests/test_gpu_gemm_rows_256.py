@@ -83,10 +83,10 @@ def test_wide_tile_of_a_layer_stack(M, N, K, scatter):
 
 
 @pytest.mark.parametrize("tile", [0x12, 0x22, 0x24])
-@pytest.mark.parametrize("rows128", [1, 17, 33])
-@pytest.mark.parametrize("N", [40, 300])
+@pytest.mark.parametrize("rows128", [1, 3, 17, 33])
+@pytest.mark.parametrize("N", [40, 300, 640, 1160])
 def test_grouped_rows_reach_every_tile(N, rows128, tile):
-    """tile rows around whole rounds of pairs by eight XCDs, empty ones at the end and between, one and several tile columns; every product of a row is
+    """tile rows around whole rounds of pairs by eight XCDs, empty ones at the end and between, tile columns in one part and in several, the last one short; every product of a row is
     a sum of 64 bf16 products in f32: 2e-6 of the result's norm (a chain of 64 roundings), rows of empty tiles are left alone"""
     L = _lib.load()
     r = rng(N + rows128 + tile)

@@ -19,6 +19,7 @@
 // LDS: blocks of 16 rows x 64 k (2 KiB): row r of a block at r * 128 bytes, its 16-byte chunk c in slot c ^ (r & 7), which spreads a fragment
 // read's lanes over all banks; a request (LDS-DMA) fetches 8 rows x 128 bytes, whole lines.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "common.cuh"
@@ -34,6 +35,7 @@ struct GemmRowsArgs {
   int nseg = 1;
   int M = 0, K = 0;  // K % 64 == 0
   int MT = 0, NT = 0;  // tiles along m, and along n over all segments
+  int chunk = 0;  // grouped rows: tile columns of a unit (gemm_rows_launch_t)
   // grouped rows (on tiles of 64 and 128 rows): tile row t (BM rows) multiplies with w[0] + tile_group[t] * w_group_stride (elements); -1: an empty tile row
   const int* tile_group = nullptr;
   int64_t w_group_stride = 0;
@@ -89,13 +91,15 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
   const int wg = wave >> 2, cw = (wave & 3) % T::CW, rw = (wave & 3) / T::CW, r16 = lane & 15, q4 = lane >> 4;
   // tile: the ids of one XCD (id mod 8) take a contiguous run of an order that walks about 8 tile rows before the next tile column, so the
   // workgroups of an XCD share their operands' panels in its L2; the tile rows in equal groups (the weights come by once a group: with 8 + 1 tile
-  // rows of 64, 557 rows x 14336, K = 4096 99 us, with 9 77.5).  Grouped rows: the empty tile rows are the last ones, so the XCDs take pairs of tile
-  // rows (an expert's, more often than not) in turn, whole, two rows to a column (16 experts of 188 rows, 2048 columns, 40 tile rows with 8 empty
+  // rows of 64, 557 rows x 14336, K = 4096 99 us, with 9 77.5).  Grouped rows: the empty tile rows are the last ones, so the XCDs take units of two tile
+  // rows (an expert's, more often than not) in turn, two rows to a column (16 experts of 188 rows, 2048 columns, 40 tile rows with 8 empty
   // ones: in runs two XCDs idle and the others work two rounds, K = 2048 / 1024 77.7 / 45.9 us; so 50.8 / 27.0)
   int mt, nt, group = 0;
   if (H == 1 && a.tile_group) {
-    const int xcd = (int)blockIdx.x & 7, i = (int)blockIdx.x >> 3, pair = xcd + 8 * (i / (2 * a.NT)), rem = i % (2 * a.NT);
-    mt = pair * 2 + (rem & 1), nt = rem >> 1;
+    const int size = 2 * a.chunk, i = (int)blockIdx.x >> 3, unit = ((int)blockIdx.x & 7) + 8 * (i / size), rem = i % size;
+    const int per = (a.NT + a.chunk - 1) / a.chunk;  // units of a pair of tile rows
+    mt = unit / per * 2 + (rem & 1), nt = unit % per * a.chunk + (rem >> 1);
+    if (nt >= a.NT) return;
     if (mt >= a.MT) return;
     group = __builtin_amdgcn_readfirstlane(a.tile_group[mt]);
     if (group < 0) return;
@@ -323,8 +327,19 @@ static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStr
     attr_devs |= (uint64_t)1 << (dev & 63);
   }
   using T = GrTile<BM, BN, DEEP>;
-  const int rows = a.tile_group ? (a.MT + 15) / 16 * 16 : a.MT;  // (pairs of tile rows by eight XCDs)
-  gemm_rows_kernel<DT, BM, BN, DEEP, PAIR, EPI><<<dim3((unsigned)(rows * a.NT), (unsigned)batch), dim3(512), (size_t)T::S * T::KP * T::STG, st>>>(a, epi);
+  unsigned grid = (unsigned)(a.MT * a.NT);
+  if (a.tile_group) {
+    // Units of two tile rows x `chunk` columns, dealt to the eight XCDs in turn: all columns where there are pairs enough for four an XCD, otherwise as many
+    // parts of equal size as make up for it, or an odd number of them, which go round the XCDs.  4 experts x 20 rows, 4096 columns, K = 4096, two tile rows
+    // a unit with all columns / so 59.8 / 26.5 us (in runs 30.2); 8 x 260, 768 columns, K = 2048 27.5 / 17.9 (18.4); with 64 units instead of 32 19.0
+    const int pairs = (a.MT + 1) / 2;
+    int parts = std::min((32 + pairs - 1) / pairs, a.NT);
+    do a.chunk = (a.NT + parts - 1) / parts;
+    while (a.NT % a.chunk && (a.NT + a.chunk - 1) / a.chunk % 2 == 0 && ++parts);
+    const int units = pairs * ((a.NT + a.chunk - 1) / a.chunk);
+    grid = (unsigned)((units + 7) / 8 * 8 * 2 * a.chunk);
+  }
+  gemm_rows_kernel<DT, BM, BN, DEEP, PAIR, EPI><<<dim3(grid, (unsigned)batch), dim3(512), (size_t)T::S * T::KP * T::STG, st>>>(a, epi);
 }
 // 64 x 128: two K steps a phase and twice the LDS where every workgroup has a CU to itself, otherwise two workgroups a CU.  (A phase of one step is two
 // waits for LDS around 8 MFMAs a wave: 64 rows x 4096, K = 14336, 32 workgroups 79.7 us, six buffers 73.2, so 69.6; with the waves in step 94.4.)
