@@ -682,6 +682,9 @@ void vra_stack_op_residual_combine(float* x, const float* o, const float* p1, in
                                    float mult, int32_t T, int32_t W, int64_t stream);
 void vra_stack_op_kv_store(const void* k, const void* v, int32_t ld, void* kc, void* vc, const int64_t* slots, int32_t T,
                            int32_t kdim, int32_t vdim, int32_t dtype, int64_t stream);
+/* out[:, :kv_from] = a w^T's first columns; the kv_k columns behind them are row slots[m] of kc [*, kv_k], the others row slots[m] of vc (below 0: nowhere) */
+void vra_stack_op_gemm_kv(const void* a, int32_t lda, const void* w, void* out, int32_t ldo, void* kc, void* vc, const int64_t* slots, int32_t M,
+                          int32_t N, int32_t K, int32_t kv_from, int32_t kv_k, int32_t dtype, int64_t stream);
 void vra_stack_op_attention(const void* q, int32_t ldq, void* out, const void* kc, const void* vc, const int64_t* positions,
                             const uint32_t* block_tables, const uint32_t* context_lens, const uint32_t* cu_q, int32_t B, int32_t T,
                             int32_t max_q, int32_t H, int32_t G, int32_t dim, int32_t vdim, int32_t BS, int32_t max_blocks,

@@ -210,6 +210,7 @@ def load():
     _sig(lib, "vra_stack_op_gated_act", None, P, P, c_i32, c_i32, c_f32, c_f32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_polynorm", None, P, P, P, c_i32, c_i32, c_f32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_residual_combine", None, P, P, P, c_i32, P, P, c_f32, c_i32, c_i32, c_i64)
+    _sig(lib, "vra_stack_op_gemm_kv", None, P, c_i32, P, P, c_i32, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_kv_store", None, P, P, c_i32, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_attention", None, P, c_i32, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
          c_f32, c_f32, c_f32, c_i32, c_i32, c_i64)

@@ -76,8 +76,9 @@ struct GrTile {
   static constexpr int EX = BM / 64, EW = BN / 64;  // a wave's DMA instructions (8 rows of 128 bytes) a K step
 };
 
-// EPI::store(m, seg, n0, N, q4, acc): the wave's 64 columns n0 .. n0 + 63 (of segment seg) of output row m; the lane holds columns n0 + 16 j + 4 q4 ..
+// EPI::store(m, row, seg, n0, N, q4, acc): the wave's 64 columns n0 .. n0 + 63 (of segment seg) of output row m; the lane holds columns n0 + 16 j + 4 q4 ..
 // + 3 in acc[j].  Called by all lanes (lanes beyond the matrix with m = -1), so that a lane may trade columns with its row's other three.
+// row: EPI::row(m), taken ahead of the loop (rows beyond the matrix: of its last).
 // PAIR: w[0] and w[1] (gate, up; neither grouped nor batched) interleaved in blocks of 16 virtual columns, n[0] = virtual columns.
 template <class DT, int BM, int BN, bool DEEP, bool PAIR, class EPI>
 __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a, const EPI epi) {
@@ -192,10 +193,13 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
     }
   };
   f32x4 acc[H * NX][4];
+  typename EPI::Row erow[H * NX];  // what the epilogue reads of its rows: asked for ahead of the loop, whose first requests come behind it
 #pragma unroll
-  for (int i = 0; i < H * NX; i++)
+  for (int i = 0; i < H * NX; i++) {
+    erow[i] = epi.row(min(m0 + row0 + i * 16 + r16, a.M - 1));
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[i][j] = vra_zero_acc();
+  }
   // (a wave's 64 columns, a phase's rows: nothing of them in the matrix, no MFMAs)
   const bool in = n0 + cw * 64 < N && m0 + row0 < a.M, in1 = H == 2 && n0 + cw * 64 < N && m0 + row0 + NX * 16 < a.M;
   auto compute = [&](auto HH, int steps) {  // steps: of the phase's KP those that are within K
@@ -277,7 +281,7 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
   for (int i = 0; i < H * NX; i++) {
     int m = m0 + row0 + i * 16 + r16;
     if (m >= a.M || (a.x_row && a.x_row[m] < 0)) m = -1;
-    epi.store(m, seg, n0 + cw * 64, N, q4, acc[i]);
+    epi.store(m, erow[i], seg, n0 + cw * 64, N, q4, acc[i]);
   }
 #endif
 }

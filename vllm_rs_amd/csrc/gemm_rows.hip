@@ -13,7 +13,9 @@ struct DenseRowsEpi {
   const uint16_t* bias_up;
   const uint16_t* residual;
   int res_ld, out_f32;
-  __device__ __forceinline__ void store(int m, int seg, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
+  struct Row {};
+  __device__ __forceinline__ Row row(int) const { return {}; }
+  __device__ __forceinline__ void store(int m, const Row&, int seg, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
     constexpr int NJ = DUAL ? 2 : 4;
     const GemmRowsOut* const s = seg == 0 ? &o[0] : (seg == 1 ? &o[1] : &o[2]);
     const int no = DUAL ? n0 / 2 : n0, lim = DUAL ? N / 2 : N;

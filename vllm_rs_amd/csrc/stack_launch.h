@@ -43,6 +43,11 @@ struct StkGemmArgs {
   int batch = 1;
   int64_t a_batch_stride = 0, w_batch_stride = 0, out_batch_stride = 0;
   int64_t bias_batch_stride = 0;  // elements between the bias rows of two products of a batch
+  // columns kv_from .. kv_from + kv_k - 1 of a plain product are the key, the others behind them the value row of cache slot kv_slot[m] (below 0: none):
+  // K [slots, kv_k], V [slots, N - kv_from - kv_k], in the product's type; they do not go to `out`
+  const int64_t* kv_slot = nullptr;
+  void *kv_kc = nullptr, *kv_vc = nullptr;
+  int kv_from = 0, kv_k = 0;
   int tile = 0;  // the tile of gemm_rows_kernel (rows / 64 * 16 + columns / 64) instead of the one of gemm_rows_tile; refused where that kernel does not take the product
 };
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream);

@@ -671,6 +671,13 @@ __global__ __launch_bounds__(64 * WM * WN) void stk_gemm_mfma_kernel(StkGemmArgs
   }
 }
 
+// where a bf16 product with cache columns (StkGemmArgs::kv_slot) stores column n of its row (null: nowhere)
+__device__ __forceinline__ uint16_t* kv_place(uint16_t* row, int64_t slot, void* kc, void* vc, int from, int k, int N, int n) {
+  if (n < from) return row + n;
+  if (slot < 0) return nullptr;
+  return n < from + k ? (uint16_t*)kc + slot * k + (n - from) : (uint16_t*)vc + slot * (N - from - k) + (n - from - k);
+}
+
 // Steps of up to 32 rows (decoding): the weights are the whole traffic, and what bounds it is the CUs that pull at them.  A
 // workgroup takes 16 * NT output columns and its 8 waves take an eighth of K each (whole K-steps of 32, ascending inside a wave); the partial
 // tiles meet in LDS and are summed in wave order.  One fixed order for a given K — another one than the large-M kernel's single chain, so the
@@ -765,7 +772,9 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g)
     if (n >= g.N) return;
     float v = total(c) * g.alpha + (g.bias ? g.bias[(int64_t)blockIdx.z * g.bias_batch_stride + n] : 0.f);
     if (POST) v = plain_value(g, v);
-    if (g.out_f32) ((float*)g.out)[ob + (int64_t)orow * g.ldo + n] = v;
+    if (!POST && !SCALED && g.kv_slot) {
+      if (uint16_t* const p = kv_place((uint16_t*)g.out + (int64_t)row * g.ldo, n < g.kv_from ? 0 : g.kv_slot[row], g.kv_kc, g.kv_vc, g.kv_from, g.kv_k, g.N, n)) *p = BF16::from_f32(v);
+    } else if (g.out_f32) ((float*)g.out)[ob + (int64_t)orow * g.ldo + n] = v;
     else ((uint16_t*)g.out)[ob + (int64_t)orow * g.ldo + n] = BF16::from_f32(v);
   }
 }
@@ -840,7 +849,9 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_eight_kernel(StkGemmArgs g)
   v = v * g.alpha + (g.bias ? g.bias[(int64_t)blockIdx.z * g.bias_batch_stride + n] : 0.f);
   if (POST) v = plain_value(g, v);
   const int64_t at = (int64_t)blockIdx.z * g.out_batch_stride + (int64_t)orow * g.ldo + n;
-  if (g.out_f32) ((float*)g.out)[at] = v;
+  if (!POST && g.kv_slot) {
+    if (uint16_t* const p = kv_place((uint16_t*)g.out + (int64_t)row * g.ldo, n < g.kv_from ? 0 : g.kv_slot[row], g.kv_kc, g.kv_vc, g.kv_from, g.kv_k, g.N, n)) *p = BF16::from_f32(v);
+  } else if (g.out_f32) ((float*)g.out)[at] = v;
   else ((uint16_t*)g.out)[at] = BF16::from_f32(v);
 }
 
@@ -848,7 +859,7 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_eight_kernel(StkGemmArgs g)
 // the kernel is 28 000 instructions long and a launch pays ~12 us for fetching what it jumps over (2048 x 2048 x 2048: 37 us, 24 so).
 // vec: rows of the output start on 16 bytes, a lane stores whole 16-byte pieces (bf16: after trading columns with its row's other
 // three lanes).
-enum StkFn { FN_NONE, FN_PAIR_CLAMPED, FN_PAIR_GELU, FN_PAIR_SILU, FN_GELU, FN_RELU2, FN_TANH, FN_EXPEXP, FN_SOFTCAP };
+enum StkFn { FN_NONE, FN_KV, FN_PAIR_CLAMPED, FN_PAIR_GELU, FN_PAIR_SILU, FN_GELU, FN_RELU2, FN_TANH, FN_EXPEXP, FN_SOFTCAP };
 template <int FN>
 struct StkRowsEpi {
   void* out;
@@ -857,6 +868,9 @@ struct StkRowsEpi {
   int64_t out_batch_stride, bias_batch_stride;
   float alpha, limit, act_alpha, softcap;
   int ldo, out_f32, vec;
+  const int64_t* kv_slot;  // FN_KV
+  void *kc, *vc;
+  int kv_from, kv_k;
   static constexpr bool pair = FN == FN_PAIR_CLAMPED || FN == FN_PAIR_GELU || FN == FN_PAIR_SILU;
   __device__ __forceinline__ float fn(float v) const {
     if (FN == FN_GELU) return gelu_erf_(v);
@@ -866,7 +880,13 @@ struct StkRowsEpi {
     if (FN == FN_SOFTCAP) return softcap * tanhf(v / softcap);
     return v;
   }
-  __device__ __forceinline__ void store(int m, int, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
+  struct None {};
+  typedef std::conditional_t<FN == FN_KV, int64_t, None> Row;
+  __device__ __forceinline__ Row row(int m) const {
+    if constexpr (FN == FN_KV) return kv_slot[m];
+    else return {};
+  }
+  __device__ __forceinline__ void store(int m, const Row& slot, int, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
     constexpr int NJ = pair ? 2 : 4;  // blocks of 16 output columns
     const int orow = m < 0 ? -1 : (out_row ? out_row[m] : m);
     const int64_t ob = (int64_t)blockIdx.y * out_batch_stride + (int64_t)max(orow, 0) * ldo;
@@ -904,7 +924,10 @@ struct StkRowsEpi {
 #pragma unroll
       for (int h = 0; h < NJ / 2; h++) {
         const int n = no + q4 * (NJ * 4) + h * 8;
-        if (orow >= 0 && n < lim) *(u32x4*)(oh + n) = u32x4{v[2 * h][0], v[2 * h][1], v[2 * h + 1][0], v[2 * h + 1][1]};
+        uint16_t* p = orow >= 0 && n < lim ? oh + n : nullptr;
+        if constexpr (FN == FN_KV)
+          if (p) p = kv_place(oh, slot, kc, vc, kv_from, kv_k, N, n);  // (whole pieces: the launcher's condition)
+        if (p) *(u32x4*)p = u32x4{v[2 * h][0], v[2 * h][1], v[2 * h + 1][0], v[2 * h + 1][1]};
       }
       return;
     }
@@ -1691,7 +1714,7 @@ void vra_stack_scale_rows(const void* a, int W, const int* row_token, const floa
 static int rows_fn(const StkGemmArgs& g) {
   if (g.epi == 1) return g.act == 1 ? FN_PAIR_GELU : (g.act == 2 ? FN_PAIR_SILU : FN_PAIR_CLAMPED);
   if (g.epi == 2) return g.act == 3 ? FN_GELU : (g.act == 4 ? FN_RELU2 : (g.act == 5 ? FN_TANH : FN_EXPEXP));
-  return g.softcap > 0.f ? FN_SOFTCAP : FN_NONE;
+  return g.softcap > 0.f ? FN_SOFTCAP : (g.kv_slot ? FN_KV : FN_NONE);
 }
 static bool rows_kernel_takes(const StkGemmArgs& g) {
   if (g.epi == 2 && g.softcap > 0.f) return false;  // (both at once: nobody asks for it)
@@ -1708,7 +1731,28 @@ int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t batch, int32
   return pair || wide > 128 ? 32 : 16;
 }
 
+// Cache columns of a product: in its epilogue where a kernel that has one takes it (in 16-byte pieces: no piece crosses from q to k or k to v), otherwise a copy
+// behind it.  The copy moves little (2048 rows: 8 MB) but is a launch: 5.1 us a layer of a 2048-token prompt, 3.0 and the gap before it of a decode step.
+// Whole steps, 16 + 4 + 4 heads of 128, width 2048, with the copy / so: 4 layers, 2048 tokens 1196 / 1184 us, eight decoded tokens 320 / 306.  A row's slot is
+// read ahead of the product's loop: behind it, where every row waits for its own, the prompt's gain was lost.
+static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream);
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
+  if (!g.kv_slot) return gemm_any(g, dtype, stream);
+  const int kd = g.kv_k, vd = g.N - g.kv_from - g.kv_k;
+  VRA_CHECK_ARG(g.kv_kc && g.kv_vc && g.kv_from > 0 && kd > 0 && vd > 0, "stack gemm: cache columns without a cache, or beyond the product's");
+  VRA_CHECK_ARG(g.batch == 1 && g.epi == 0 && g.softcap <= 0.f && !g.tile_group && !g.a_row && !g.out_row && !g.a_scale && (!g.out_f32 || dtype == VRA_F32),
+                "stack gemm: cache columns come with a plain product in the cache's type");
+  auto al16 = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+  const bool fused = dtype == VRA_BF16 && g.K % 64 == 0 && g.lda % 8 == 0 && al16(g.a) && al16(g.w) && al16(g.out) && g.ldo % 8 == 0 && al16(g.kv_kc) && al16(g.kv_vc) &&
+                     g.kv_from % 8 == 0 && kd % 8 == 0 && vd % 8 == 0 && (g.M <= 32 || (g.N > 128 && rows_kernel_takes(g)));
+  if (fused) return gemm_any(g, dtype, stream);
+  StkGemmArgs p = g;
+  p.kv_slot = nullptr;
+  gemm_any(p, dtype, stream);
+  const int es = dtype == VRA_F32 ? 4 : 2;
+  vra_stack_kv_store((const char*)g.out + (size_t)g.kv_from * es, (const char*)g.out + (size_t)(g.kv_from + kd) * es, g.ldo, g.kv_kc, g.kv_vc, g.kv_slot, g.M, kd, vd, dtype, stream);
+}
+static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream) {
   VRA_CHECK_ARG(g.a && g.w && g.out && g.M > 0 && g.N > 0 && g.K > 0, "stack gemm: null pointer or empty shape");
   VRA_CHECK_ARG(dtype == VRA_BF16 || dtype == VRA_F32, "stack gemm: dtype must be bf16 or f32");
   VRA_CHECK_ARG(!g.tile_group || g.granule == 16 || g.granule == 64 || g.granule == 128, "stack gemm: granule must be 16, 64 or 128");
@@ -1735,7 +1779,8 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
       auto go = [&](auto fn) {
         const int per = g.out_f32 ? 4 : 8;  // elements of 16 bytes
         const bool vec = (uintptr_t)g.out % 16 == 0 && g.ldo % per == 0 && g.out_batch_stride % per == 0 && (g.out_f32 || (g.epi == 1 ? g.N % 32 : g.N % 8) == 0);
-        StkRowsEpi<decltype(fn)::value> e{g.out, g.out_row, g.bias, g.out_batch_stride, g.bias_batch_stride, g.alpha, g.limit, g.act_alpha, g.softcap, g.ldo, g.out_f32, vec ? 1 : 0};
+        StkRowsEpi<decltype(fn)::value> e{g.out, g.out_row, g.bias, g.out_batch_stride, g.bias_batch_stride, g.alpha, g.limit, g.act_alpha, g.softcap, g.ldo, g.out_f32, vec ? 1 : 0,
+                                             g.kv_slot, g.kv_kc, g.kv_vc, g.kv_from, g.kv_k};
         launch_checked("stack gemm", [&] { gemm_rows_launch<BF16, false>(r, e, tile, nb, st); });
       };
       switch (rows_fn(g)) {
@@ -1747,6 +1792,7 @@ void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
         case FN_TANH: go(std::integral_constant<int, FN_TANH>{}); break;
         case FN_EXPEXP: go(std::integral_constant<int, FN_EXPEXP>{}); break;
         case FN_SOFTCAP: go(std::integral_constant<int, FN_SOFTCAP>{}); break;
+        case FN_KV: go(std::integral_constant<int, FN_KV>{}); break;
         default: go(std::integral_constant<int, FN_NONE>{}); break;
       }
     } else if (big) {
@@ -1998,6 +2044,14 @@ extern "C" void vra_stack_op_gemm(const void* a, int32_t lda, const void* w, int
   StkGemmArgs g;
   g.a = a, g.lda = lda, g.w = w, g.w_group_stride = w_group_stride, g.out = out, g.ldo = ldo, g.out_f32 = out_f32, g.M = M, g.N = N, g.K = K;
   g.alpha = alpha, g.tile_group = tile_group, g.granule = granule, g.a_row = a_row, g.a_scale = a_scale, g.out_row = out_row, g.epi = epi, g.limit = limit;
+  vra_stack_gemm(g, dtype, stream);
+}
+extern "C" void vra_stack_op_gemm_kv(const void* a, int32_t lda, const void* w, void* out, int32_t ldo, void* kc, void* vc, const int64_t* slots, int32_t M, int32_t N, int32_t K,
+                                     int32_t kv_from, int32_t kv_k, int32_t dtype, int64_t stream) {
+  VRA_CHECK_ARG(slots, "stack gemm: cache columns without slots");
+  StkGemmArgs g;
+  g.a = a, g.lda = lda, g.w = w, g.out = out, g.ldo = ldo, g.M = M, g.N = N, g.K = K;
+  g.kv_slot = slots, g.kv_kc = kc, g.kv_vc = vc, g.kv_from = kv_from, g.kv_k = kv_k;
   vra_stack_gemm(g, dtype, stream);
 }
 extern "C" void vra_stack_op_gemm_tile(int32_t tile, const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32,

@@ -1179,10 +1179,8 @@ bool StackModel::mixer_softmax(const StackLayer& L, const InputMetadata& md, int
   const int nqkv = L.nqkv();
   StkGemmArgs p;
   p.a = h_, p.lda = W, p.w = L.qkv, p.M = T, p.N = nqkv, p.K = W, p.out = qkv_, p.ldo = nqkv;
+  if (L.owns_cache) p.kv_slot = md.slot_mapping, p.kv_kc = kc_[L.cache], p.kv_vc = vc_[L.cache], p.kv_from = L.nq(), p.kv_k = L.nk();
   vra_stack_gemm(p, dt_, stream);
-  if (L.owns_cache)
-    vra_stack_kv_store((const char*)qkv_ + (size_t)L.nq() * es_, (const char*)qkv_ + (size_t)(L.nq() + L.nk()) * es_, nqkv, kc_[L.cache], vc_[L.cache],
-                       md.slot_mapping, T, L.nk(), L.nv(), dt_, stream);
   StkAttnArgs a;
   a.q = qkv_, a.ldq = nqkv, a.out = attn_, a.kc = kc_[L.cache], a.vc = vc_[L.cache];
   a.positions = md.positions, a.block_tables = md.block_tables, a.context_lens = md.context_lens;
