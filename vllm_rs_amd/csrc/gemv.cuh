@@ -65,6 +65,7 @@ struct GemvArgs {
   int is_awq, scales_layout;
   int silu_dual;  // 1: seg0 = gate, seg1 = up, out = silu(gate)*up into seg0.out
   int out_f32;    // 1: store (float)round_dt(v)
+  float* mirror;  // dense launches with f32 output: the same values at the same places there, too (pinned host memory)
   int n_items;    // work items (n-blocks, or gate/up pairs)
   int m_groups;   // int4 kernel: row-group families (1: all M rows in every workgroup)
   int rows_per_group;
@@ -396,6 +397,7 @@ __global__ __launch_bounds__(GEMV_THREADS, 4) void gemv_kernel(const GemvArgs a)
         }
         if (a.residual) v = rnd_dt<DT>(v) + DT::to_f32(static_cast<const uint16_t*>(a.residual)[(size_t)m * a.res_ld + n]);
         if (!INT4 && NBW == 1 && a.am_out) am_best = gemv_am_max(am_best, gemv_am_key(rnd_dt<DT>(v), (uint32_t)n));
+        if (!INT4 && a.mirror) a.mirror[(size_t)m * sg.out_ld + n] = rnd_dt<DT>(v);
         if (a.out_f32) static_cast<float*>(sg.out)[(size_t)m * sg.out_ld + n] = rnd_dt<DT>(v);
         else static_cast<uint16_t*>(sg.out)[(size_t)m * sg.out_ld + n] = DT::from_f32(v);
       }

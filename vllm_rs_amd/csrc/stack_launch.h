@@ -43,6 +43,7 @@ struct StkGemmArgs {
   int batch = 1;
   int64_t a_batch_stride = 0, w_batch_stride = 0, out_batch_stride = 0;
   int64_t bias_batch_stride = 0;  // elements between the bias rows of two products of a batch
+  float* mirror = nullptr;  // f32 output of up to 32 rows: the same values at the same places there, too (pinned host memory); no groups, no batch
   // columns kv_from .. kv_from + kv_k - 1 of a plain product are the key, the others behind them the value row of cache slot kv_slot[m] (below 0: none):
   // K [slots, kv_k], V [slots, N - kv_from - kv_k], in the product's type; they do not go to `out`
   const int64_t* kv_slot = nullptr;
@@ -51,6 +52,7 @@ struct StkGemmArgs {
   int tile = 0;  // the tile of gemm_rows_kernel (rows / 64 * 16 + columns / 64) instead of the one of gemm_rows_tile; refused where that kernel does not take the product
 };
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream);
+bool vra_stack_gemm_mirrors(const StkGemmArgs& g, int dtype);  // whether it takes StkGemmArgs::mirror
 // columns a workgroup takes of a bf16 product of up to 32 rows (pair: with the gated epilogue): 16 or 32, the sums are the same
 extern "C" int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t batch, int32_t pair);
 // rows per granule the grouped launches of an M-row problem over `groups` groups want (16, 64, or 128 where `tiles128`: both products of the

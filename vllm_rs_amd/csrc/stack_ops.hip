@@ -774,8 +774,10 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g)
     if (POST) v = plain_value(g, v);
     if (!POST && !SCALED && g.kv_slot) {
       if (uint16_t* const p = kv_place((uint16_t*)g.out + (int64_t)row * g.ldo, n < g.kv_from ? 0 : g.kv_slot[row], g.kv_kc, g.kv_vc, g.kv_from, g.kv_k, g.N, n)) *p = BF16::from_f32(v);
-    } else if (g.out_f32) ((float*)g.out)[ob + (int64_t)orow * g.ldo + n] = v;
-    else ((uint16_t*)g.out)[ob + (int64_t)orow * g.ldo + n] = BF16::from_f32(v);
+    } else if (g.out_f32) {
+      if (g.mirror) g.mirror[(int64_t)orow * g.ldo + n] = v;
+      ((float*)g.out)[ob + (int64_t)orow * g.ldo + n] = v;
+    } else ((uint16_t*)g.out)[ob + (int64_t)orow * g.ldo + n] = BF16::from_f32(v);
   }
 }
 
@@ -851,8 +853,10 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_eight_kernel(StkGemmArgs g)
   const int64_t at = (int64_t)blockIdx.z * g.out_batch_stride + (int64_t)orow * g.ldo + n;
   if (!POST && g.kv_slot) {
     if (uint16_t* const p = kv_place((uint16_t*)g.out + (int64_t)row * g.ldo, n < g.kv_from ? 0 : g.kv_slot[row], g.kv_kc, g.kv_vc, g.kv_from, g.kv_k, g.N, n)) *p = BF16::from_f32(v);
-  } else if (g.out_f32) ((float*)g.out)[at] = v;
-  else ((uint16_t*)g.out)[at] = BF16::from_f32(v);
+  } else if (g.out_f32) {
+    if (g.mirror) g.mirror[(int64_t)orow * g.ldo + n] = v;
+    ((float*)g.out)[at] = v;
+  } else ((uint16_t*)g.out)[at] = BF16::from_f32(v);
 }
 
 // Epilogue of gemm_rows_kernel for these products: alpha, bias, FN, row scatter.  FN as a template parameter: with all functions in one epilogue
@@ -1736,6 +1740,10 @@ int32_t vra_stack_op_gemm_few_columns(int32_t M, int32_t N, int32_t batch, int32
 // Whole steps, 16 + 4 + 4 heads of 128, width 2048, with the copy / so: 4 layers, 2048 tokens 1196 / 1184 us, eight decoded tokens 320 / 306.  A row's slot is
 // read ahead of the product's loop: behind it, where every row waits for its own, the prompt's gain was lost.
 static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream);
+bool vra_stack_gemm_mirrors(const StkGemmArgs& g, int dtype) {
+  return dtype == VRA_BF16 && g.M <= 32 && g.out_f32 && g.batch == 1 && g.epi != 1 && !g.tile_group && g.K % 8 == 0 && g.lda % 8 == 0 && (uintptr_t)g.a % 16 == 0 &&
+         (uintptr_t)g.w % 16 == 0;
+}
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream) {
   if (!g.kv_slot) return gemm_any(g, dtype, stream);
   const int kd = g.kv_k, vd = g.N - g.kv_from - g.kv_k;
@@ -1756,6 +1764,7 @@ static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream) {
   VRA_CHECK_ARG(g.a && g.w && g.out && g.M > 0 && g.N > 0 && g.K > 0, "stack gemm: null pointer or empty shape");
   VRA_CHECK_ARG(dtype == VRA_BF16 || dtype == VRA_F32, "stack gemm: dtype must be bf16 or f32");
   VRA_CHECK_ARG(!g.tile_group || g.granule == 16 || g.granule == 64 || g.granule == 128, "stack gemm: granule must be 16, 64 or 128");
+  VRA_CHECK_ARG(!g.mirror || vra_stack_gemm_mirrors(g, dtype), "stack gemm: a second output goes with plain f32 products of up to 32 rows");
   VRA_CHECK_ARG(g.batch >= 1 && (g.batch == 1 || !g.tile_group), "stack gemm: a batched product has no row groups");
   hipStream_t st = as_stream(stream);
   const int nb = g.batch;

@@ -1319,6 +1319,10 @@ static void launch_gemv_dw_n(GemvDWArgs a, hipStream_t st) {
   kern<<<grid, GW_THREADS, lds, st>>>(a);
 }
 void vra_launch_gemv_dw(GemvDWArgs a, int dtype, int64_t stream) {
+  if (a.mirror && (!a.out_f32 || a.out_ld % 4 || (uintptr_t)a.mirror % 16)) {
+    vra_set_error("gemv_dw: a second output goes with f32 results and rows on 16 bytes");
+    return;
+  }
   hipStream_t st = as_stream(stream);
   const bool two = a.M > 16, norm = a.norm_w != nullptr;
   if (dtype == VRA_BF16) {

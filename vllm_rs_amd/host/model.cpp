@@ -1200,6 +1200,7 @@ bool Model::lm_head(const void* xin, int rows, uint32_t* tokens, int64_t stream)
     a.K = H;
     a.group_size = -1;
     a.out_f32 = 1;
+    a.mirror = logits_mirror, logits_mirrored = logits_mirror != nullptr;
     if (tokens && rows <= 8) {  // the greedy tokens out of the same launch (the last workgroup to arrive reduces the candidates)
       a.am_out = tokens, a.am_ws = argmax_ws_;
       tokens = nullptr;
@@ -1215,6 +1216,7 @@ bool Model::lm_head(const void* xin, int rows, uint32_t* tokens, int64_t stream)
       a.am_out = tokens, a.am_ws = argmax_ws_;
       tokens = nullptr;
     }
+    a.mirror = logits_mirror, logits_mirrored = logits_mirror != nullptr;
     vra_launch_gemv_dw(a, dt_, stream);
   } else {
     vra_rms_norm(xin, final_norm_, xn_, rows, H, mc_.rms_norm_eps, dt_, stream);

@@ -68,6 +68,10 @@ class ModelBase {
   // forward -> f32 logits [rows, vocab] on the device; tokens != null: the greedy token of every logits row as well
   virtual bool forward(const InputMetadata& md, int64_t stream, uint32_t* tokens = nullptr) = 0;
   virtual float* logits() const = 0;
+  // pinned host memory (as the device sees it) that takes the next forward's logits, too, rows of vocab floats; the forward says whether its head's launch
+  // wrote them there
+  float* logits_mirror = nullptr;
+  bool logits_mirrored = false;
   virtual size_t weight_bytes() const = 0;
   // decode steps may be captured into hipGraphs at init
   virtual bool graph_capturable() const { return true; }

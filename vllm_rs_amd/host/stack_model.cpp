@@ -1354,6 +1354,7 @@ bool StackModel::forward(const InputMetadata& md, int64_t stream, uint32_t* toke
   }
   StkGemmArgs hd;
   hd.a = hl_, hd.lda = W, hd.w = head_, hd.M = rows, hd.N = vocab_, hd.K = W, hd.out = logits_, hd.ldo = vocab_, hd.out_f32 = 1, hd.alpha = logit_scale_, hd.softcap = logit_softcap_;
+  if (logits_mirror && vra_stack_gemm_mirrors(hd, dt_)) hd.mirror = logits_mirror, logits_mirrored = true;
   vra_stack_gemm(hd, dt_, stream);
   if (tokens) vra_argmax_f32(logits_, tokens, rows, vocab_, stream);
   return !take_stack_err(error, "head");
