@@ -76,7 +76,8 @@ void vra_stack_embed_sinpos(const uint32_t* ids, const int64_t* positions, const
 // of the layer before, in the launch that reads its result).
 struct StkNormArgs {
   const float* x = nullptr;
-  float* x_out = nullptr;  // (with `o`: x itself)
+  float* x_out = nullptr;  // (with `o`: x itself, or null where nobody reads the sum)
+  const uint32_t* rows = nullptr;  // row t of h is row rows[t] of x and its parts (null: row t)
   const float* o = nullptr;
   const float* p1 = nullptr;
   int n1 = 0;

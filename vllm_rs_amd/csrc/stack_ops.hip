@@ -51,8 +51,10 @@ __global__ __launch_bounds__(256) void stk_embed_sinpos_kernel(const uint32_t* i
   uint32_t id = ids[t];
   if (id >= (uint32_t)V) id = 0;
   const float p = (float)pos[t];
+  // (few rows: a row's angles over the grid's second dimension, as a thread's sines and cosines one after the other are most of the launch.  8 rows of 2048: 3.4 us, one
+  // workgroup a row 6.5)
   // (a thread takes both entries of an angle: lanes that alternate between sine and cosine would each wait for the other's)
-  for (int i = threadIdx.x; i < (W + 1) / 2; i += 256) {
+  for (int i = blockIdx.y * 256 + threadIdx.x; i < (W + 1) / 2; i += 256 * gridDim.y) {
     float sn = 0.f, cs = 0.f;
     if (inv_freq) sincosf(p * inv_freq[i], &sn, &cs);
     x[(size_t)t * W + 2 * i] = El<T>::ld(embed + (size_t)id * W + 2 * i) + sn;
@@ -81,15 +83,17 @@ __device__ __forceinline__ float wave_fold(float v, F f) {
 // 2048, 16 outputs and a gate 22.0 -> 15.2; 64 outputs, eight picks 76.6 -> 21.7; 160 outputs 163 -> 74.  A wave's outputs of a round
 // counted ahead of the loop over the row, not tested in it: 8 rows of 12288, eight outputs 20.2 -> 15.6.  PARTS a template parameter too, and a row without
 // parts asked for ahead of its weights: 1500 rows of 2048 5.64 -> 5.33, the other way about 5.43)
+// The final norm takes the last layer's parts and the chosen rows in the same launch (x_out null, rows): behind a sum over all rows and a gather, two launches, 2048 rows of
+// 2048, one wanted 20.7 us, so 4.9; a decode step of 8 rows 6.5, 3.9.
 template <typename T, bool ROUTER, bool PARTS>
 __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
   extern __shared__ float lds[];
   float* xs = lds;                      // [W] the row, then the normalised row
   float* rs = lds + a.W;                // [groups] 1 / rms
   float* zs = rs + a.groups;            // [n_router + gate_row]
-  const int t = blockIdx.x, W = a.W, gs = W / a.groups;
+  const int t = blockIdx.x, W = a.W, gs = W / a.groups, ts = a.rows ? (int)a.rows[t] : t;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const float* x = a.x + (size_t)t * W;
+  const float* x = a.x + (size_t)ts * W;
   T* h = (T*)a.h + (size_t)t * W;
   auto sums = [&] {
     __syncthreads();
@@ -104,7 +108,7 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
     }
     __syncthreads();
   };
-  const float gt = PARTS && a.gate_in ? a.gate_in[t] : 1.f;
+  const float gt = PARTS && a.gate_in ? a.gate_in[ts] : 1.f;
   const bool quads = W % 4 == 0 && gs % 4 == 0 && (((uintptr_t)a.x | (uintptr_t)a.x_out | (uintptr_t)a.o | (uintptr_t)a.p1 | (uintptr_t)a.p2 | (uintptr_t)a.w) % 16) == 0;
   if (quads) {
     // (four values a load where rows and groups allow it, two loads of every part of the row ahead of the first sum: its parts arrive in one round trip
@@ -126,11 +130,11 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
         for (int n = 0; n < R; n++) s[n] += d[n];
       };
       read(x, v);
-      const float* const p1 = a.p1 + (size_t)t * a.n1 * W;
-      read(a.o + (size_t)t * W, s);
+      const float* const p1 = a.p1 + (size_t)ts * a.n1 * W;
+      read(a.o + (size_t)ts * W, s);
       if (a.n1 > 0) read(p1, s1);
       if (a.n1 > 1) read(p1 + W, s2);
-      if (a.p2) read(a.p2 + (size_t)t * W, s3);
+      if (a.p2) read(a.p2 + (size_t)ts * W, s3);
       if (a.n1 > 0) add(s1);
       if (a.n1 > 1) add(s2);
       for (int j = 2; j < a.n1; j++) {
@@ -145,7 +149,10 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
       for (int n = 0; n < R; n++) v[n] += a.mult * s[n];
 #pragma unroll
       for (int n = 0; n < R; n++)
-        if (c0 + n * 1024 < W) *(f32x4*)(xs + c0 + n * 1024) = *(f32x4*)(a.x_out + (size_t)t * W + c0 + n * 1024) = v[n];
+        if (c0 + n * 1024 < W) {
+          *(f32x4*)(xs + c0 + n * 1024) = v[n];
+          if (a.x_out) *(f32x4*)(a.x_out + (size_t)ts * W + c0 + n * 1024) = v[n];
+        }
     };
     auto put = [&](int c, f32x4 v, f32x4 w) {
       const f32x4 y = v * rs[c / gs] * w;
@@ -187,11 +194,11 @@ __global__ __launch_bounds__(256, 8) void stk_group_norm_kernel(StkNormArgs a) {
   } else {
     if constexpr (PARTS) {
       for (int c = threadIdx.x; c < W; c += 256) {
-        float s = a.o[(size_t)t * W + c];
-        for (int j = 0; j < a.n1; j++) s += a.p1[((size_t)t * a.n1 + j) * W + c];
-        if (a.p2) s += gt * a.p2[(size_t)t * W + c];
+        float s = a.o[(size_t)ts * W + c];
+        for (int j = 0; j < a.n1; j++) s += a.p1[((size_t)ts * a.n1 + j) * W + c];
+        if (a.p2) s += gt * a.p2[(size_t)ts * W + c];
         const float v = x[c] + a.mult * s;
-        a.x_out[(size_t)t * W + c] = v;
+        if (a.x_out) a.x_out[(size_t)ts * W + c] = v;
         xs[c] = v;
       }
     } else {
@@ -1861,16 +1868,18 @@ static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream) {
 void vra_stack_embed_sinpos(const uint32_t* ids, const int64_t* positions, const void* embed, const float* inv_freq, float* x, int T, int W, int V,
                             int dtype, int64_t stream) {
   VRA_CHECK_ARG(ids && positions && embed && x && T > 0 && W > 0, "stack embed: null pointer or empty shape");
+  const dim3 grid(T, std::max(1, std::min((W / 2 + 255) / 256, 256 / T)));
   if (dtype == VRA_F32)
-    launch_checked("stack embed", [&] { stk_embed_sinpos_kernel<float><<<T, 256, 0, as_stream(stream)>>>(ids, positions, (const float*)embed, inv_freq, x, W, V); });
+    launch_checked("stack embed", [&] { stk_embed_sinpos_kernel<float><<<grid, 256, 0, as_stream(stream)>>>(ids, positions, (const float*)embed, inv_freq, x, W, V); });
   else
-    launch_checked("stack embed", [&] { stk_embed_sinpos_kernel<uint16_t><<<T, 256, 0, as_stream(stream)>>>(ids, positions, (const uint16_t*)embed, inv_freq, x, W, V); });
+    launch_checked("stack embed", [&] { stk_embed_sinpos_kernel<uint16_t><<<grid, 256, 0, as_stream(stream)>>>(ids, positions, (const uint16_t*)embed, inv_freq, x, W, V); });
 }
 
 void vra_stack_group_norm(const StkNormArgs& a, int dtype, int64_t stream) {
   VRA_CHECK_ARG(a.x && a.w && a.h && a.T > 0 && a.W > 0, "stack norm: null pointer or empty shape");
   VRA_CHECK_ARG(a.groups >= 1 && a.W % a.groups == 0, "stack norm: the width must split into equal groups");
-  VRA_CHECK_ARG(!a.o || (a.x_out == a.x && (a.n1 == 0 || a.p1)), "stack norm: parts of the row without a place for the sum");
+  VRA_CHECK_ARG(!a.o || ((a.x_out == a.x || !a.x_out) && (a.n1 == 0 || a.p1)), "stack norm: parts of the row without a place for the sum");
+  VRA_CHECK_ARG(!a.rows || !a.x_out, "stack norm: chosen rows keep no sum");
   VRA_CHECK_ARG(!a.router_w || (a.pair_expert && a.pair_weight && a.top >= 1 && a.top <= a.n_router && (!a.gate_row || a.gate_out)), "stack norm: router outputs");
   const size_t lds = ((size_t)a.W + a.groups + a.n_router + 2) * sizeof(float);
   VRA_CHECK_ARG(lds <= 64 * 1024, "stack norm: row does not fit LDS");

@@ -1305,7 +1305,8 @@ bool StackModel::forward(const InputMetadata& md, int64_t stream, uint32_t* toke
       vra_stack_group_norm(n, dt_, stream);
       if (!mixer_softmax(L, md, stream)) return false;
       if (!feed_forward(L, T, stream)) return false;
-      if (trace_on_ || li + 1 == layers_.size()) {
+      // (behind the last layer the final norm's launch adds the parts, to the rows whose logits are wanted)
+      if (trace_on_ || (li + 1 == layers_.size() && norm_kind_ != 0)) {
         vra_stack_residual_combine(x_, due_.o, due_.p1, due_.n1, due_.p2, due_.gate, residual_mult_, T, W, stream);
         due_ = {};
         if (take_stack_err(error, "residual")) return false;
@@ -1319,7 +1320,7 @@ bool StackModel::forward(const InputMetadata& md, int64_t stream, uint32_t* toke
         if (!expert_pair(h_, W, L.s_gu, 0, L.s_down, 0, T, L.sffp, L.ff, 0.f, nullptr, 0, nullptr, nullptr, nullptr, pair_out_, stream, 1)) return false;
         pending = pair_out_;
       }
-      if (trace_on_ || li + 1 == layers_.size()) {
+      if (trace_on_ || (li + 1 == layers_.size() && norm_kind_ != 0)) {
         vra_stack_residual_combine(x_, pending, nullptr, 0, nullptr, nullptr, 1.f, T, W, stream);
         pending = nullptr;
         if (take_stack_err(error, "residual")) return false;
@@ -1335,8 +1336,10 @@ bool StackModel::forward(const InputMetadata& md, int64_t stream, uint32_t* toke
   if (sel) {
     rows = md.n_logit_rows > 0 ? md.n_logit_rows : B;
     if (rows > logit_rows_cap_) return error = "forward: more logit rows than the logits buffer holds", false;
-    vra_stack_gather_rows_f32(x_, sel, xl_, rows, W, stream);
-    xin = xl_;
+    if (norm_kind_ != 0) {  // (that norm's launch takes the rows itself)
+      vra_stack_gather_rows_f32(x_, sel, xl_, rows, W, stream);
+      xin = xl_;
+    }
   } else if (rows > logit_rows_cap_) {
     return error = "forward: more logit rows than the logits buffer holds", false;
   }
@@ -1349,8 +1352,11 @@ bool StackModel::forward(const InputMetadata& md, int64_t stream, uint32_t* toke
     vra_stack_dyt(const_cast<float*>(xin), nullptr, final_norm_, final_b_, final_alpha_, hl_, rows, W, dt_, stream);
   } else {
     StkNormArgs fn;
-    fn.x = xin, fn.w = final_norm_, fn.h = hl_, fn.T = rows, fn.W = W, fn.groups = groups_, fn.eps = eps_;
+    fn.x = xin, fn.w = final_norm_, fn.h = hl_, fn.T = rows, fn.W = W, fn.groups = groups_, fn.eps = eps_, fn.rows = sel;
+    if (due_.o) fn.o = due_.o, fn.p1 = due_.p1, fn.n1 = due_.n1, fn.p2 = due_.p2, fn.gate_in = due_.gate, fn.mult = residual_mult_;
+    else if (pending) fn.o = pending;
     vra_stack_group_norm(fn, dt_, stream);
+    due_ = {};
   }
   StkGemmArgs hd;
   hd.a = hl_, hd.lda = W, hd.w = head_, hd.M = rows, hd.N = vocab_, hd.K = W, hd.out = logits_, hd.ldo = vocab_, hd.out_f32 = 1, hd.alpha = logit_scale_, hd.softcap = logit_softcap_;
