@@ -266,6 +266,13 @@ void vra_paged_attention_prefill_sw(void* out, const void* q, const void* k, con
                                     int32_t q_heads, int32_t kv_heads, int32_t head_dim,
                                     int32_t block_size, int32_t max_blocks_per_seq, float scale,
                                     float softcap, int32_t sliding_window, int32_t dtype, int32_t kv_dtype, int64_t stream);
+/* vra_rope_cache_prefill + vra_paged_attention_prefill_sw over the cache (no softcap) with the same bits; where the attention kernel rotates the queries as it reads
+ * them (no window, heads of 64 or 128, blocks of a power of two) q is not written, otherwise rotated in place. */
+void vra_rope_cache_attention_prefill(void* out, void* q, const void* k, const void* v, void* k_cache, void* v_cache, const void* cos, const void* sin,
+                                      const int64_t* positions, const int64_t* slot_mapping, const uint32_t* block_tables,
+                                      const uint32_t* context_lens, const uint32_t* cu_seqlens_q, int32_t batch, int32_t total_q,
+                                      int32_t max_seqlen_q, int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t block_size,
+                                      int32_t max_blocks_per_seq, float scale, int32_t sliding_window, int32_t dtype, int32_t kv_dtype, int64_t stream);
 /* Fused decode step of one layer's attention front half, ONE launch for what the reference issues as
  * FusedRope::apply_inplace + reshape_and_cache + PagedAttention::forward (attention.rs:745-820): rotary on q
  * and k (NeoX pairing, tables [n_pos, head_dim/2] in the model dtype), scatter of the rotated k and of v

@@ -122,6 +122,8 @@ def load():
          c_f32, c_f32, c_i32, P, c_i32, c_i32, c_i64)
     _sig(lib, "vra_paged_attention_prefill_sw", None, P, P, P, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32,
          c_i32, c_i32, c_i32, c_f32, c_f32, c_i32, c_i32, c_i32, c_i64)
+    _sig(lib, "vra_rope_cache_attention_prefill", None, P, P, P, P, P, P, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
+         c_f32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_rope_cache_prefill_slices", c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, P)
     _sig(lib, "vra_rope_cache_attention_decode", None, P, P, P, P, P, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32,
          c_i32, c_i32, c_i32, c_f32, P, c_i32, c_i32, c_i64)

@@ -971,13 +971,15 @@ extern "C" void vra_paged_attention_prefill(void* out, const void* q, const void
                                  max_seqlen_q, q_heads, kv_heads, head_dim, block_size, max_blocks_per_seq, scale, softcap, 0, dtype, kv_dtype,
                                  stream);
 }
-extern "C" void vra_paged_attention_prefill_sw(void* out, const void* q, const void* k, const void* v, const void* k_cache,
-                                               const void* v_cache, const uint32_t* block_tables, const uint32_t* context_lens,
-                                               const uint32_t* cu_seqlens_q, const uint32_t* cu_seqlens_k, int32_t batch,
-                                               int32_t total_q, int32_t max_seqlen_q, int32_t q_heads, int32_t kv_heads,
-                                               int32_t head_dim, int32_t block_size, int32_t max_blocks_per_seq, float scale,
-                                               float softcap, int32_t sliding_window, int32_t dtype, int32_t kv_dtype, int64_t stream) {
-  (void)total_q;
+static bool prefill_tiled(int head_dim, int block_size, int sliding_window) {
+  return sliding_window == 0 && (head_dim == 128 || head_dim == 64) && block_size > 0 && (block_size & (block_size - 1)) == 0 && !getenv("VRA_NO_PREFILL_TILED");
+}
+// cos, sin, positions: of q as the projection left it (tiled kernel only), or null
+static void paged_attention_prefill(void* out, const void* q, const void* k, const void* v, const void* k_cache, const void* v_cache, const uint32_t* block_tables,
+                                    const uint32_t* context_lens, const uint32_t* cu_seqlens_q, const uint32_t* cu_seqlens_k, int32_t batch,
+                                    int32_t max_seqlen_q, int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t block_size,
+                                    int32_t max_blocks_per_seq, float scale, float softcap, int32_t sliding_window, const void* cos, const void* sin,
+                                    const int64_t* positions, int32_t dtype, int32_t kv_dtype, int64_t stream) {
   VRA_CHECK_ARG(sliding_window >= 0, "vra_paged_attention_prefill: sliding_window must be >= 0 (0 = off)");
   VRA_CHECK_ARG(dtype == VRA_BF16 || dtype == VRA_F16, "vra_paged_attention_prefill: dtype must be bf16/f16");
   if (!kv_dtype_ok("vra_paged_attention_prefill", dtype, kv_dtype)) return;
@@ -1014,11 +1016,14 @@ extern "C" void vra_paged_attention_prefill_sw(void* out, const void* q, const v
   a.nsplit = 1;
   a.sliding_window = sliding_window;
   // (a sliding window runs on the generic kernel below — mask + skipped tiles; the LDS-tiled kernel is the full-causal fast path)
-  if (sliding_window == 0 && block_tables && (head_dim == 128 || head_dim == 64) && (block_size & (block_size - 1)) == 0 && !getenv("VRA_NO_PREFILL_TILED")) {
+  const bool tiled = block_tables && prefill_tiled(head_dim, block_size, sliding_window);
+  VRA_CHECK_ARG(tiled || !cos, "vra_paged_attention_prefill: this form takes rotated queries");
+  if (tiled) {
     // the LDS-tiled prefill kernel (attn_prefill.cuh); 2 row tiles per wave once that still leaves >= 2 workgroups per CU
     PrefillAttnArgs p = {};
     p.out = out, p.q = q, p.kc = k_cache, p.vc = v_cache;
     p.block_tables = block_tables, p.context_lens = context_lens, p.cu_q = cu_seqlens_q;
+    p.cosv = cos, p.sinv = sin, p.positions = positions;
     p.Hq = q_heads, p.Hkv = kv_heads, p.BS = block_size, p.max_blocks = max_blocks_per_seq;
     p.bs_shift = __builtin_ctz((unsigned)block_size);
     p.scale = scale, p.scale_log2e = a.scale_log2e, p.softcap = softcap;
@@ -1057,6 +1062,33 @@ extern "C" void vra_paged_attention_prefill_sw(void* out, const void* q, const v
   dim3 grid((max_seqlen_q + 63) / 64, q_heads, batch);
   if (dtype == VRA_BF16) launch_attn<BF16>(a, head_dim, kv_dtype == VRA_FP8_E4M3, grid, as_stream(stream));
   else launch_attn<F16>(a, head_dim, kv_dtype == VRA_FP8_E4M3, grid, as_stream(stream));
+}
+extern "C" void vra_paged_attention_prefill_sw(void* out, const void* q, const void* k, const void* v, const void* k_cache,
+                                               const void* v_cache, const uint32_t* block_tables, const uint32_t* context_lens,
+                                               const uint32_t* cu_seqlens_q, const uint32_t* cu_seqlens_k, int32_t batch,
+                                               int32_t total_q, int32_t max_seqlen_q, int32_t q_heads, int32_t kv_heads,
+                                               int32_t head_dim, int32_t block_size, int32_t max_blocks_per_seq, float scale,
+                                               float softcap, int32_t sliding_window, int32_t dtype, int32_t kv_dtype, int64_t stream) {
+  (void)total_q;
+  paged_attention_prefill(out, q, k, v, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, cu_seqlens_k, batch, max_seqlen_q, q_heads, kv_heads, head_dim,
+                          block_size, max_blocks_per_seq, scale, softcap, sliding_window, nullptr, nullptr, nullptr, dtype, kv_dtype, stream);
+}
+extern "C" void vra_rope_cache_attention_prefill(void* out, void* q, const void* k, const void* v, void* k_cache, void* v_cache, const void* cos, const void* sin,
+                                                 const int64_t* positions, const int64_t* slot_mapping, const uint32_t* block_tables,
+                                                 const uint32_t* context_lens, const uint32_t* cu_seqlens_q, int32_t batch, int32_t total_q,
+                                                 int32_t max_seqlen_q, int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t block_size,
+                                                 int32_t max_blocks_per_seq, float scale, int32_t sliding_window, int32_t dtype, int32_t kv_dtype,
+                                                 int64_t stream) {
+  VRA_CHECK_ARG(out && q && k && v && k_cache && v_cache && cos && sin && positions && slot_mapping && block_tables && context_lens && cu_seqlens_q,
+                "vra_rope_cache_attention_prefill: null pointer");
+  // (the tiled kernel rotates the queries as it reads them; the general one takes them rotated)
+  const bool rotates = prefill_tiled(head_dim, block_size, sliding_window);
+  if (rotates) vra_rope_cache_prefill_kv(k, v, k_cache, v_cache, cos, sin, positions, slot_mapping, total_q, kv_heads, head_dim, block_size, dtype, kv_dtype, stream);
+  else
+    vra_rope_cache_prefill(q, k, v, k_cache, v_cache, cos, sin, positions, slot_mapping, total_q, q_heads, kv_heads, head_dim, block_size, dtype, kv_dtype, stream);
+  paged_attention_prefill(out, q, nullptr, nullptr, k_cache, v_cache, block_tables, context_lens, cu_seqlens_q, nullptr, batch, max_seqlen_q, q_heads, kv_heads,
+                          head_dim, block_size, max_blocks_per_seq, scale, 0.f, sliding_window, rotates ? cos : nullptr, rotates ? sin : nullptr, positions, dtype,
+                          kv_dtype, stream);
 }
 
 extern "C" void vra_rope_cache_attention_decode(void* out, const void* q, const void* k, const void* v, void* k_cache, void* v_cache,

@@ -44,6 +44,10 @@ struct PrefillAttnArgs {
   const uint32_t* block_tables;  // [B, max_blocks]
   const uint32_t* context_lens;  // [B]
   const uint32_t* cu_q;          // [B+1]
+  // q is as the projection left it: rotated here by these tables (model dtype, [positions, D/2]) at positions[token]; null: q is rotated
+  const void* cosv;
+  const void* sinv;
+  const int64_t* positions;
   int Hq, Hkv, BS, max_blocks;
   int bs_shift;  // log2(BS): this kernel takes power-of-two block sizes (others run paged_attn_kernel)
   float scale_log2e, softcap, scale;
@@ -144,6 +148,29 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
       u32x4 v = *reinterpret_cast<const u32x4*>(qp + j * 32 + oct * 8);
       if (!valid) v = u32x4{0u, 0u, 0u, 0u};
       qf[mt][j] = __builtin_bit_cast(s16x8, v);
+    }
+    // (a head's pairs D/2 apart lie in one lane, j and j + DJ/2: the arithmetic and the roundings of rope_cache_kernel, which would read and write all of q
+    // once more.  Its launch and this one, us, q rotated there / here: 32 + 8 heads of 128, 150 tokens 11.8 / 11.5, 600 24.4 / 22.7, 4000 191 / 186; 28 + 4, 1300 43.5 /
+    // 40.1; 32 + 4 of 64, 2048 53.5 / 51.0; 8192 tokens of 32 + 8: that launch 45 / 26, this one no longer)
+    if (a.cosv) {
+      const int64_t pos = a.positions[q0 + (valid ? qtok : 0)];
+      const uint16_t* const cp = static_cast<const uint16_t*>(a.cosv) + pos * (D / 2) + oct * 8;
+      const uint16_t* const sp = static_cast<const uint16_t*>(a.sinv) + pos * (D / 2) + oct * 8;
+#pragma unroll
+      for (int j = 0; j < DJ / 2; j++) {
+        float x1[8], x2[8], cs[8], sn[8], y1[8], y2[8];
+        unpack8<DT>(__builtin_bit_cast(u32x4, qf[mt][j]), x1);
+        unpack8<DT>(__builtin_bit_cast(u32x4, qf[mt][j + DJ / 2]), x2);
+        unpack8<DT>(*reinterpret_cast<const u32x4*>(cp + j * 32), cs);
+        unpack8<DT>(*reinterpret_cast<const u32x4*>(sp + j * 32), sn);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          y1[e] = x1[e] * cs[e] - x2[e] * sn[e];
+          y2[e] = x2[e] * cs[e] + x1[e] * sn[e];
+        }
+        qf[mt][j] = __builtin_bit_cast(s16x8, pack8<DT>(y1));
+        qf[mt][j + DJ / 2] = __builtin_bit_cast(s16x8, pack8<DT>(y2));
+      }
     }
   }
   f32x4 o[MT][DT16];

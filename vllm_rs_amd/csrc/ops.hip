@@ -2,6 +2,7 @@
 // casts, block swap and the synthetic fills.  All HBM-bound streaming kernels: 16 B per lane,
 // f32 math, one rounding per reference op (include/vllm_rs_amd.h §B).
 #include "common.cuh"
+#include "attn_launch.h"
 #include "kvcache.cuh"
 
 // ---------------------------------------------------------------- RMSNorm (+ residual add)
@@ -588,12 +589,12 @@ extern "C" int32_t vra_rope_cache_prefill_slices(int32_t tokens, int32_t kv_head
   if (lds_bytes) *lds_bytes = (int32_t)(g.staged + (g.slices ? kRopeSlotBytes : 0));
   return g.slices;
 }
-extern "C" void vra_rope_cache_prefill(void* q, const void* k, const void* v, void* k_cache, void* v_cache, const void* cos, const void* sin,
-                                       const int64_t* positions, const int64_t* slot_mapping, int32_t tokens, int32_t q_heads, int32_t kv_heads,
-                                       int32_t head_dim, int32_t block_size, int32_t dtype, int32_t kv_dtype, int64_t stream) {
+static void rope_cache_prefill(void* q, const void* k, const void* v, void* k_cache, void* v_cache, const void* cos, const void* sin, const int64_t* positions,
+                               const int64_t* slot_mapping, int32_t tokens, int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t block_size,
+                               int32_t dtype, int32_t kv_dtype, int64_t stream) {
   VRA_CHECK_ARG(dtype == VRA_BF16 || dtype == VRA_F16, "vra_rope_cache_prefill: dtype must be bf16/f16");
   VRA_CHECK_ARG(kv_dtype == dtype || kv_dtype == VRA_FP8_E4M3, "vra_rope_cache_prefill: kv_dtype must be the activation dtype or VRA_FP8_E4M3");
-  VRA_CHECK_ARG(q && k && v && k_cache && v_cache && cos && sin && positions && slot_mapping, "vra_rope_cache_prefill: null pointer");
+  VRA_CHECK_ARG((q || !q_heads) && k && v && k_cache && v_cache && cos && sin && positions && slot_mapping, "vra_rope_cache_prefill: null pointer");
   VRA_CHECK_ARG(head_dim % 16 == 0 && head_dim <= 256, "vra_rope_cache_prefill: head_dim must be a multiple of 16 (<= 256)");
   if (tokens <= 0) return;
   hipStream_t st = as_stream(stream);
@@ -619,6 +620,17 @@ extern "C" void vra_rope_cache_prefill(void* q, const void* k, const void* v, vo
     else VRA_RC(F16, false);
   }
 #undef VRA_RC
+}
+extern "C" void vra_rope_cache_prefill(void* q, const void* k, const void* v, void* k_cache, void* v_cache, const void* cos, const void* sin,
+                                       const int64_t* positions, const int64_t* slot_mapping, int32_t tokens, int32_t q_heads, int32_t kv_heads,
+                                       int32_t head_dim, int32_t block_size, int32_t dtype, int32_t kv_dtype, int64_t stream) {
+  VRA_CHECK_ARG(q, "vra_rope_cache_prefill: null pointer");
+  rope_cache_prefill(q, k, v, k_cache, v_cache, cos, sin, positions, slot_mapping, tokens, q_heads, kv_heads, head_dim, block_size, dtype, kv_dtype, stream);
+}
+void vra_rope_cache_prefill_kv(const void* k, const void* v, void* k_cache, void* v_cache, const void* cos, const void* sin, const int64_t* positions,
+                               const int64_t* slot_mapping, int32_t tokens, int32_t kv_heads, int32_t head_dim, int32_t block_size, int32_t dtype,
+                               int32_t kv_dtype, int64_t stream) {
+  rope_cache_prefill(nullptr, k, v, k_cache, v_cache, cos, sin, positions, slot_mapping, tokens, 0, kv_heads, head_dim, block_size, dtype, kv_dtype, stream);
 }
 
 // ---------------------------------------------------------------- causal mask

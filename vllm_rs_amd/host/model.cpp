@@ -1095,11 +1095,9 @@ bool Model::forward(const InputMetadata& md, int64_t stream, uint32_t* tokens) {
       return false;
     const int sw = mc_.sliding_window > 0 ? mc_.sliding_window : 0;  // llama.rs:46,284 (Mistral-type checkpoints)
     if (md.is_prefill) {
-      // RoPE + KV write in one launch (two in the reference: rotary_emb.rs:88-103, attention.rs:808-820)
-      vra_rope_cache_prefill(q_, k_, v_, kc_[l], vc_[l], cos_, sin_, md.positions, md.slot_mapping, T, hq_, hkv_, D, ec_.block_size, dt_,
-                             kv_dt, stream);
-      vra_paged_attention_prefill_sw(attn_, q_, nullptr, nullptr, kc_[l], vc_[l], md.block_tables, md.context_lens, md.cu_seqlens_q,
-                                     nullptr, B, T, md.max_seqlen_q, hq_, hkv_, D, ec_.block_size, md.max_blocks, scale, 0.f, sw, dt_, kv_dt, stream);
+      // RoPE of k + KV write in one launch, RoPE of q in the attention's (three in the reference: rotary_emb.rs:88-103, attention.rs:808-820)
+      vra_rope_cache_attention_prefill(attn_, q_, k_, v_, kc_[l], vc_[l], cos_, sin_, md.positions, md.slot_mapping, md.block_tables, md.context_lens,
+                                       md.cu_seqlens_q, B, T, md.max_seqlen_q, hq_, hkv_, D, ec_.block_size, md.max_blocks, scale, sw, dt_, kv_dt, stream);
     } else if (sw > 0) {
       // sliding window: the three calls of the reference (rotary embedding, reshape_and_cache, paged attention with the window;
       // attention.rs:745-820) — the fused decode launch is the full-causal fast path
