@@ -117,6 +117,8 @@ void vra_wna16_gate_up_silu(const void* in, const void* qw_gate, const void* sc_
  * 'M').  0: a shape they refuse. */
 int32_t vra_wna16_kernel(int32_t pair, int32_t m, int32_t k, int32_t n, int32_t group_size, int32_t is_awq, int32_t has_norm,
                          int32_t has_bias, int32_t has_residual);
+/* ... that a model's step runs for its down projection: 'M' at some of the shapes of 64..160 rows where vra_wna16_gemm keeps 'W' */
+int32_t vra_wna16_down_kernel(int32_t m, int32_t k, int32_t n, int32_t group_size, int32_t is_awq, int32_t has_bias, int32_t has_residual);
 /* the same products (qw_up null: a single one) on a named kernel, 64 rows up and row-major scales: 'D' (64-row tiles), 'd' (32-row tiles) or 'M' */
 void vra_wna16_gemm_on(int32_t kernel, const void* in, const void* qweight_tiled, const void* scales, const void* qzeros, const void* qw_up,
                        const void* sc_up, const void* qz_up, const void* bias, const void* residual, void* out, int32_t m, int32_t k,

@@ -21,6 +21,8 @@ void vra_launch_gemm_q4_big(const GemmDArgs& a, bool dual, bool awq, int mb, int
 // kernel M (gemm_q4_mid.cuh): int4, 64 rows up, scale groups >= 128: the launch's plan (m-tiles a wave | K slices << 8) and its estimated time,
 // or 0 where the shape is not its own.  GemmDArgs::xsum has to be set.
 int vra_gemm_q4_mid_plan(bool dual, int M, int cols, int K, int group_size, const GemmDArgs* segs, bool awq, bool summed, double* us);
+// kernel M's plan (for vra_launch_gemm_q4_big) for a down projection that vra_wna16_gemm leaves to kernel W's row blocks, or 0 where those are quicker
+int vra_down_mid_plan(int M, int K, int N, int group_size, bool awq, bool has_res, bool has_bias);
 void vra_launch_gemm_q4_mid(GemmDArgs a, bool dual, bool awq, int plan, int dtype, int64_t stream);
 // kernel E (gemv_q4s.cuh): int4, 1..4 rows, scale groups >= 128 (or channel-wise), n_units = 16-column blocks (pairs count once).
 // ns = 1 | 2 (gate/up pair with SiLU*mul).  The launcher fills KT / TPW / the unit distribution / gsh.

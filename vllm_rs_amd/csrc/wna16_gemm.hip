@@ -1065,6 +1065,26 @@ extern "C" int32_t vra_wna16_kernel(int32_t pair, int32_t m, int32_t k, int32_t 
   return general_kernel(ns, m, k, n, group_size, is_awq != 0, &plan);
 }
 
+// The model's down_proj of 64..96 and 129..160 rows: kernel M instead of kernel W's row blocks (which vra_wna16_gemm keeps: a row there has the bits of a 32-row
+// launch, in a model's step the products ahead of it do not).  W converts every code once per 32 rows and takes 11 us and 1.85 (AWQ 1.92) for each 16 columns of a
+// workgroup; M converts it twice in all and takes 0.92 (0.96) of its plan's estimate.  us, W / M, over K = 4608..28672 x 1024..8192: 14336 x 4096, 64 rows 24.9 / 22.6,
+// 96 rows 34.4 / 28.3, 145 rows 49.4 / 38.6; AWQ 18944 x 3584, 145 rows 57.1 / 48.4; few columns stay: 14336 x 1024, 145 rows 22 / 36, 8192 x 3584 28 / 32.
+int vra_down_mid_plan(int M, int K, int N, int group_size, bool awq, bool has_res, bool has_bias) {
+  if (M < 64 || K <= 4096 || N % 16 || !vra_gemv_w_fits(1, M, K, group_size, N / 16, has_res, has_bias)) return 0;
+  static const char* mid_env = getenv("VRA_NO_KERNEL_M");  // tuning aid
+  if (mid_env && mid_env[0] == '1') return 0;
+  int kz, ktz, groups;
+  if (!gemv_w_kz_plan(K, N / 16, (M + 31) / 32, &kz, &ktz, &groups)) return 0;
+  double mid_us = 0.0;
+  const int plan = vra_gemm_q4_mid_plan(false, M, N, K, group_size, nullptr, awq, false, &mid_us);
+  const double w_us = 11.0 + (awq ? 1.92 : 1.85) * ((N / 16 + groups - 1) / groups);
+  return plan && mid_us * (awq ? 0.96 : 0.92) < w_us ? plan | kMidPlan : 0;
+}
+extern "C" int32_t vra_wna16_down_kernel(int32_t m, int32_t k, int32_t n, int32_t group_size, int32_t is_awq, int32_t has_bias, int32_t has_residual) {
+  if (!check_gemm_shape("vra_wna16_down_kernel", m, k, n, group_size)) return 0;
+  return vra_down_mid_plan(m, k, n, group_size, is_awq != 0, has_residual != 0, has_bias != 0) ? 'M' : vra_wna16_kernel(0, m, k, n, group_size, is_awq, 0, has_bias, has_residual);
+}
+
 extern "C" void vra_wna16_gemm_on(int32_t kernel, const void* in, const void* w0, const void* sc0, const void* qz0, const void* w1, const void* sc1,
                                   const void* qz1, const void* bias, const void* residual, void* out, int32_t m, int32_t k, int32_t n, int32_t group_size,
                                   int32_t is_awq, int32_t dtype, int64_t stream) {

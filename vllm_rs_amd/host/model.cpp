@@ -616,6 +616,14 @@ bool Model::linear(const QLinear& l0, const void* x, void* out, int M, const voi
       vra_launch_gemm_dense(a, false, dt_, vra_gemm_dense_tile(M, l.N, l.K), stream);
       return !take_err(error, "linear (gemm_dense, resident weights)");
     }
+    const bool zeros = l.awq && l.qzeros != nullptr;
+    if (const int plan = vra_down_mid_plan(M, l.K, l.N, mc_.group_size, zeros, residual != nullptr, l.bias != nullptr)) {
+      GemmDArgs d = {};
+      d.w0 = l.w, d.sc0 = l.scales, d.qz0 = (const uint32_t*)l.qzeros, d.bias0 = l.bias, d.residual = residual, d.res_ld = l.N;
+      d.x = x, d.x_ld = l.K, d.out = out, d.out_ld = l.N, d.M = M, d.N = l.N, d.K = l.K, d.group_size = mc_.group_size;
+      vra_launch_gemm_q4_big(d, false, zeros, plan, dt_, stream);
+      return !take_err(error, "linear (kernel M)");
+    }
     vra_wna16_gemm(x, l.w, l.scales, l.qzeros, l.bias, residual, out, M, l.K, l.N, mc_.group_size, l.awq ? 1 : 0,
                    VRA_SCALES_ROWMAJOR, dt_, stream);
   } else if (!residual) {
@@ -935,6 +943,7 @@ bool Model::gemv_s_ok(int which, int M) const {
   const LayerWeights& L = layers_[0];
   if (!L.q.quant || !L.qkv_s_um || !L.o.s_um || !L.gate.s_um || !L.up.s_um || !L.down.s_um) return false;
   const bool bias = which == 0 ? (L.q.bias || L.k.bias || L.v.bias) : (which == 2 ? (L.gate.bias || L.up.bias) : (which == 1 ? L.o.bias != nullptr : L.down.bias != nullptr));
+  if (which == 3 && vra_down_mid_plan(M, inter_, mc_.hidden_size, mc_.group_size, L.down.awq && L.down.qzeros != nullptr, world_ == 1, bias)) return false;
   return family_takes(which, M, mc_.hidden_size, inter_, hq_, hkv_, mc_.head_dim, mc_.group_size, bias);
 }
 // which fused-norm launches of an M-row step of layer `layer` apply the RMSNorm factor in their epilogue (model.h); takes(which) =
