@@ -65,6 +65,8 @@ struct GemvArgs {
   int is_awq, scales_layout;
   int silu_dual;  // 1: seg0 = gate, seg1 = up, out = silu(gate)*up into seg0.out
   int out_f32;    // 1: store (float)round_dt(v)
+  // row m of x is its row x_rows[m] (null: m): the rows whose logits are wanted, which a launch of its own gathered ahead of the head's for 4.7 us
+  const uint32_t* x_rows;
   float* mirror;  // dense launches with f32 output: the same values at the same places there, too (pinned host memory)
   int n_items;    // work items (n-blocks, or gate/up pairs)
   int m_groups;   // int4 kernel: row-group families (1: all M rows in every workgroup)
@@ -124,7 +126,9 @@ __device__ __forceinline__ void gemv_stage_x(const GemvArgs& a, uint32_t* xs, fl
   const int octs = a.K >> 3;
   const int nf = octs / opg;
   for (int m = 0; m < a.M; m++) {
-    const u32x4* xr = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.x) + (size_t)m * a.x_ld);
+    // (a scalar load: a vector load would wait behind the weights in flight)
+    const uint32_t row = a.x_rows ? reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(reinterpret_cast<uintptr_t>(a.x_rows))[m] : (uint32_t)m;
+    const u32x4* xr = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.x) + (size_t)row * a.x_ld);
     float rstd = 1.0f;
     if (a.norm_w) {
       float ss = 0.f;

@@ -28,6 +28,7 @@
 
 struct GemvDWArgs {
   const void* x;       // [M, x_ld]
+  const uint32_t* x_rows;  // row m of x is its row x_rows[m] (null: m)
   int x_ld;
   const void* norm_w;  // fused RMSNorm weights [K] (NORM variants), else null
   float eps;
@@ -89,6 +90,13 @@ __global__ __launch_bounds__(GW_THREADS) void gemv_dw_kernel(const GemvDWArgs a)
 #pragma unroll
     for (int j = 0; j < 4; j++) w[j] = __builtin_nontemporal_load(p + j * jstep);
   };
+  uint32_t xrow[MT];  // (asked for ahead of the weights)
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) {
+    xrow[mt] = min(mt * 16 + (lane & 15), M - 1);
+    if (a.x_rows) xrow[mt] = a.x_rows[xrow[mt]];
+  }
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int sl = 0; sl < GDW_RING; sl++) issue(sl, wb[sl]);
   __builtin_amdgcn_sched_barrier(0);
@@ -100,7 +108,7 @@ __global__ __launch_bounds__(GW_THREADS) void gemv_dw_kernel(const GemvDWArgs a)
     const int kt = min(wave + GW_WAVES * ti, KT - 1);
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-      const uint16_t* xr = static_cast<const uint16_t*>(a.x) + (size_t)min(mt * 16 + nn, M - 1) * a.x_ld + kt * 128 + oct * 8;
+      const uint16_t* xr = static_cast<const uint16_t*>(a.x) + (size_t)xrow[mt] * a.x_ld + kt * 128 + oct * 8;
 #pragma unroll
       for (int j = 0; j < 4; j++) xf[ti][j][mt] = *reinterpret_cast<const u32x4*>(xr + (j ^ (nn & 1)) * 32);
     }

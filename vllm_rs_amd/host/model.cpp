@@ -1171,26 +1171,24 @@ bool Model::forward(const InputMetadata& md, int64_t stream, uint32_t* tokens) {
     }
   }
   // last token of every sequence (llama.rs:306-310), final norm, lm_head -> f32 (llama.rs:311-320)
-  const void* xin = h_;
+  const uint32_t* sel = nullptr;
   int rows = T;
   if (md.n_logit_rows > 0) {  // explicit rows (replayed traces): any rows of the step, as many as the logits buffer holds
     if (md.n_logit_rows > max_seqs_) {
       error = "forward: more logit rows than max_num_seqs";
       return false;
     }
-    vra_index_select_rows(h_, md.logit_rows, last_, md.n_logit_rows, H, dt_, stream);
-    xin = last_;
+    sel = md.logit_rows;
     rows = md.n_logit_rows;
   } else if (md.is_prefill) {
-    vra_index_select_rows(h_, md.last_token_rows, last_, B, H, dt_, stream);
-    xin = last_;
+    sel = md.last_token_rows;
     rows = B;
   }
-  return lm_head(xin, rows, tokens, stream);
+  return lm_head(h_, rows, tokens, stream, sel);
 }
 
-// final norm + lm_head -> f32 logits (llama.rs:311-320) and, when `tokens` is given, the greedy tokens (logits_processor.rs:67-70)
-bool Model::lm_head(const void* xin, int rows, uint32_t* tokens, int64_t stream) {
+// final norm + lm_head of xin's rows sel[0 .. rows) (null: of its first) -> f32 logits (llama.rs:311-320) and, when `tokens` is given, the greedy tokens (logits_processor.rs:67-70)
+bool Model::lm_head(const void* xin, int rows, uint32_t* tokens, int64_t stream, const uint32_t* sel) {
   const int H = mc_.hidden_size;
   // 1..3 rows: kernel A (x in LDS); 4..32 rows: the dense W kernel where it fits (measured 0.6 % of the step faster than kernel A at 4..7
   // rows, equal at 1..2), else kernel A / kernel B behind a norm launch
@@ -1199,7 +1197,7 @@ bool Model::lm_head(const void* xin, int rows, uint32_t* tokens, int64_t stream)
     a.nseg = 1;
     a.seg[0] = GemvSeg{lm_head_tiled_ ? lm_head_tiled_ : lm_head_.w, nullptr, nullptr, nullptr, logits_, lm_head_.N, lm_head_.N, 0};
     a.dense_tiled = lm_head_tiled_ ? 1 : 0;
-    a.x = xin;
+    a.x = xin, a.x_rows = sel;
     a.x_ld = H;
     a.norm_w = final_norm_;
     a.eps = mc_.rms_norm_eps;
@@ -1215,7 +1213,7 @@ bool Model::lm_head(const void* xin, int rows, uint32_t* tokens, int64_t stream)
     vra_launch_gemv(a, false, dt_, stream);
   } else if (vra_gemv_dw_fits(rows, H, lm_head_.N)) {  // 9..32 rows: final norm + lm_head in one launch (gemv_dw.cuh)
     GemvDWArgs a = {};
-    a.x = xin, a.x_ld = H, a.norm_w = final_norm_, a.eps = mc_.rms_norm_eps;
+    a.x = xin, a.x_rows = sel, a.x_ld = H, a.norm_w = final_norm_, a.eps = mc_.rms_norm_eps;
     a.w = lm_head_tiled_ ? lm_head_tiled_ : lm_head_.w, a.dense_tiled = lm_head_tiled_ ? 1 : 0, a.out = logits_, a.out_ld = lm_head_.N, a.out_f32 = 1;
     a.M = rows, a.K = H, a.n_units = lm_head_.N / 16;
     static const char* dwam_env = getenv("VRA_DW_ARGMAX");  // tuning aid: 0 = separate argmax launch behind the dense W kernel
@@ -1226,6 +1224,10 @@ bool Model::lm_head(const void* xin, int rows, uint32_t* tokens, int64_t stream)
     a.mirror = logits_mirror, logits_mirrored = logits_mirror != nullptr;
     vra_launch_gemv_dw(a, dt_, stream);
   } else {
+    if (sel) {
+      vra_index_select_rows(xin, sel, last_, rows, H, dt_, stream);
+      xin = last_;
+    }
     vra_rms_norm(xin, final_norm_, xn_, rows, H, mc_.rms_norm_eps, dt_, stream);
     vra_dense_gemm(xn_, lm_head_.w, nullptr, logits_, rows, H, lm_head_.N, dt_, VRA_F32, stream);
   }

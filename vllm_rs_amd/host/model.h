@@ -86,7 +86,7 @@ class Model : public ModelBase {
   // microbenchmark hooks (bench.py roofline leg): launch one decode-shaped GEMM of layer `layer`
   // which: 0 qkv(fused norm) 1 o_proj 2 gate_up 3 down 4 lm_head ; M rows
   bool launch_gemm(int which, int layer, int M, int64_t stream) override;
-  bool lm_head(const void* xin, int rows, uint32_t* tokens, int64_t stream);
+  bool lm_head(const void* xin, int rows, uint32_t* tokens, int64_t stream, const uint32_t* sel = nullptr);
   int64_t gemm_algorithmic_bytes(int which, int M) const override;
   // which fused-norm launches of a step of M rows apply the RMSNorm factor in their EPILOGUE (kernel E at 1..4 rows, gemv_q4s.cuh;
   // the oracle restates that order): bit 0 = norm + q/k/v, bit 1 = norm + gate/up.  0 for every other step.
