@@ -44,21 +44,53 @@ __device__ __forceinline__ float gated_pair(float g, float u, float limit, float
 }
 
 // ------------------------------------------------------------------------------------------------ embedding + positions
-template <typename T>
+// A thread takes both entries of an angle: lanes that alternate between sine and cosine would each wait for the other's.
+// N angles at a time: one load and one store for all of them where rows start on 16 bytes (N = 2), and the rows of a long prompt (DEPTH) asked for ahead of
+// the first sine.  2048 rows of 2048: 16.0 us one angle after the other, now 12.6; 1500 rows 13.5, 8.9.
+template <typename T, int N, int DEPTH>
 __global__ __launch_bounds__(256) void stk_embed_sinpos_kernel(const uint32_t* ids, const int64_t* pos, const T* embed, const float* inv_freq, float* x,
                                                                int W, int V) {
+  typedef T tvec __attribute__((ext_vector_type(2 * N)));
+  typedef float fvec __attribute__((ext_vector_type(N)));
+  typedef float ovec __attribute__((ext_vector_type(2 * N)));
   const int t = blockIdx.x;
   uint32_t id = ids[t];
   if (id >= (uint32_t)V) id = 0;
   const float p = (float)pos[t];
+  const T* const er = embed + (size_t)id * W;
+  float* const xr = x + (size_t)t * W;
   // (few rows: a row's angles over the grid's second dimension, as a thread's sines and cosines one after the other are most of the launch.  8 rows of 2048: 3.4 us, one
   // workgroup a row 6.5)
-  // (a thread takes both entries of an angle: lanes that alternate between sine and cosine would each wait for the other's)
-  for (int i = blockIdx.y * 256 + threadIdx.x; i < (W + 1) / 2; i += 256 * gridDim.y) {
-    float sn = 0.f, cs = 0.f;
-    if (inv_freq) sincosf(p * inv_freq[i], &sn, &cs);
-    x[(size_t)t * W + 2 * i] = El<T>::ld(embed + (size_t)id * W + 2 * i) + sn;
-    if (2 * i + 1 < W) x[(size_t)t * W + 2 * i + 1] = El<T>::ld(embed + (size_t)id * W + 2 * i + 1) + cs;
+  const int first = (blockIdx.y * 256 + threadIdx.x) * N, step = 256 * gridDim.y * N, angles = (W + 1) / 2;
+  for (int i0 = first; i0 < angles; i0 += step * DEPTH) {
+    if constexpr (N == 1) {
+      float sn = 0.f, cs = 0.f;
+      if (inv_freq) sincosf(p * inv_freq[i0], &sn, &cs);
+      xr[2 * i0] = El<T>::ld(er + 2 * i0) + sn;
+      if (2 * i0 + 1 < W) xr[2 * i0 + 1] = El<T>::ld(er + 2 * i0 + 1) + cs;
+    } else {
+      tvec e[DEPTH];
+      fvec f[DEPTH];
+#pragma unroll
+      for (int d = 0; d < DEPTH; d++) {
+        const int i = min(i0 + d * step, angles - N);
+        e[d] = *(const tvec*)(er + 2 * i);
+        f[d] = inv_freq ? *(const fvec*)(inv_freq + i) : (fvec)(0.f);
+      }
+#pragma unroll
+      for (int d = 0; d < DEPTH; d++) {
+        const int i = i0 + d * step;
+        ovec o;
+#pragma unroll
+        for (int n = 0; n < N; n++) {
+          float sn = 0.f, cs = 0.f;
+          if (inv_freq) sincosf(p * f[d][n], &sn, &cs);
+          const T pair[2] = {e[d][2 * n], e[d][2 * n + 1]};
+          o[2 * n] = El<T>::ld(pair) + sn, o[2 * n + 1] = El<T>::ld(pair + 1) + cs;
+        }
+        if (i < angles) *(ovec*)(xr + 2 * i) = o;
+      }
+    }
   }
 }
 
@@ -1869,10 +1901,17 @@ void vra_stack_embed_sinpos(const uint32_t* ids, const int64_t* positions, const
                             int dtype, int64_t stream) {
   VRA_CHECK_ARG(ids && positions && embed && x && T > 0 && W > 0, "stack embed: null pointer or empty shape");
   const dim3 grid(T, std::max(1, std::min((W / 2 + 255) / 256, 256 / T)));
-  if (dtype == VRA_F32)
-    launch_checked("stack embed", [&] { stk_embed_sinpos_kernel<float><<<grid, 256, 0, as_stream(stream)>>>(ids, positions, (const float*)embed, inv_freq, x, W, V); });
-  else
-    launch_checked("stack embed", [&] { stk_embed_sinpos_kernel<uint16_t><<<grid, 256, 0, as_stream(stream)>>>(ids, positions, (const uint16_t*)embed, inv_freq, x, W, V); });
+  const bool quads = W % 4 == 0 && (((uintptr_t)embed | (uintptr_t)inv_freq | (uintptr_t)x) % 16) == 0;
+  auto go = [&](auto one) {
+    typedef decltype(one) E;
+    hipStream_t st = as_stream(stream);
+    launch_checked("stack embed", [&] {
+      if (!quads || T < 256) stk_embed_sinpos_kernel<E, 1, 1><<<grid, 256, 0, st>>>(ids, positions, (const E*)embed, inv_freq, x, W, V);
+      else stk_embed_sinpos_kernel<E, 2, 2><<<grid, 256, 0, st>>>(ids, positions, (const E*)embed, inv_freq, x, W, V);
+    });
+  };
+  if (dtype == VRA_F32) go(float{});
+  else go(uint16_t{});
 }
 
 void vra_stack_group_norm(const StkNormArgs& a, int dtype, int64_t stream) {
