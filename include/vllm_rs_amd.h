@@ -310,6 +310,9 @@ void vra_dense_gemm_tile(int32_t tile, const void* x, const void* const* w, cons
                          int64_t stream);
 /* the tile that the row-major prompt GEMM takes for m rows x nseg tensors of n[s] columns (0: no such product) */
 int32_t vra_dense_gemm_tile_choice(int32_t m, const int32_t* n, int32_t nseg, int32_t k);
+/* ... for one tensor (or a pair's 2 n columns), which may be on two tiles: 0x44 with the number of 256-column strips on 256 x 256 in the bits from 8 on, the rest on 128 x 256;
+ * vra_dense_gemm_tile takes that, too */
+int32_t vra_dense_gemm_tiles_choice(int32_t m, int32_t n, int32_t k);
 /* logits.argmax(-1) (logits_processor.rs:67-70): first maximal index per row. */
 void vra_argmax_f32(const float* logits, uint32_t* out, int32_t rows, int32_t cols, int64_t stream);
 /* lm_head + greedy sampling as one launch (llama.rs:311-320 followed by logits_processor.rs:67-70): f32 logits as

@@ -132,6 +132,7 @@ def load():
     _sig(lib, "vra_swap_blocks", None, P, P, P, c_i32, c_i64, c_i32, c_i64)
     _sig(lib, "vra_dense_gemm_tile", None, c_i32, P, P, P, P, c_i32, c_i32, P, P, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_dense_gemm_tile_choice", c_i32, c_i32, P, c_i32, c_i32)
+    _sig(lib, "vra_dense_gemm_tiles_choice", c_i32, c_i32, c_i32, c_i32)
     _sig(lib, "vra_dense_gemm", None, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_argmax_f32", None, P, P, c_i32, c_i32, c_i64)
     _sig(lib, "vra_dense_gemm_argmax_workspace_bytes", c_i64)

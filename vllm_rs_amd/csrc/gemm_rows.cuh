@@ -36,6 +36,7 @@ struct GemmRowsArgs {
   int M = 0, K = 0;  // K % 64 == 0
   int MT = 0, NT = 0;  // tiles along m, and along n over all segments
   int chunk = 0;  // grouped rows: tile columns of a unit (gemm_rows_launch_t)
+  int mixed = 0;  // gemm_rows_mixed_kernel: tile columns of 256 x 256
   // grouped rows (on tiles of 64 and 128 rows): tile row t (BM rows) multiplies with w[0] + tile_group[t] * w_group_stride (elements); -1: an empty tile row
   const int* tile_group = nullptr;
   int64_t w_group_stride = 0;
@@ -76,13 +77,26 @@ struct GrTile {
   static constexpr int EX = BM / 64, EW = BN / 64;  // a wave's DMA instructions (8 rows of 128 bytes) a K step
 };
 
+// place of workgroup bid of nwg in an order whose contiguous runs go to one XCD (ids mod 8) each, and a place's tile of MT x NT: about 8 tile rows, in equal
+// groups, before the next tile column
+__device__ __forceinline__ int gr_xcd_run(int bid, int nwg) {
+  const int q = nwg >> 3, r = nwg & 7, xcd = bid & 7;
+  return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
+}
+__device__ __forceinline__ void gr_tile_of(int lin, int MT, int NT, int& mt, int& nt) {
+  const int groups = max((MT + 4) >> 3, 1), GM = (MT + groups - 1) / groups;
+  const int per = GM * NT, grp = lin / per, rem = lin - grp * per, first = grp * GM, gsz = min(MT - first, GM);
+  mt = first + rem % gsz;
+  nt = rem / gsz;
+}
+
 // EPI::store(m, row, seg, n0, N, q4, acc): the wave's 64 columns n0 .. n0 + 63 (of segment seg) of output row m; the lane holds columns n0 + 16 j + 4 q4 ..
 // + 3 in acc[j].  Called by all lanes (lanes beyond the matrix with m = -1), so that a lane may trade columns with its row's other three.
 // row: EPI::row(m), taken ahead of the loop (rows beyond the matrix: of its last).
 // PAIR: w[0] and w[1] (gate, up; neither grouped nor batched) interleaved in blocks of 16 virtual columns, n[0] = virtual columns.
+// tile (mt, nt) of segment seg (w, N columns)
 template <class DT, int BM, int BN, bool DEEP, bool PAIR, class EPI>
-__global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a, const EPI epi) {
-#ifdef __HIP_DEVICE_COMPILE__
+__device__ __forceinline__ void gemm_rows_tile_product(const GemmRowsArgs& a, const EPI& epi, int mt, int nt, int seg, int N, const uint16_t* w, int group) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   using T = GrTile<BM, BN, DEEP>;
   constexpr int H = T::H, KP = T::KP, S = T::S, NX = T::NX, STG = T::STG, EX = T::EX, EW = T::EW, D = EX + EW;
@@ -90,35 +104,6 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wg = wave >> 2, cw = (wave & 3) % T::CW, rw = (wave & 3) / T::CW, r16 = lane & 15, q4 = lane >> 4;
-  // tile: the ids of one XCD (id mod 8) take a contiguous run of an order that walks about 8 tile rows before the next tile column, so the
-  // workgroups of an XCD share their operands' panels in its L2; the tile rows in equal groups (the weights come by once a group: with 8 + 1 tile
-  // rows of 64, 557 rows x 14336, K = 4096 99 us, with 9 77.5).  Grouped rows: the empty tile rows are the last ones, so the XCDs take units of two tile
-  // rows (an expert's, more often than not) in turn, two rows to a column (16 experts of 188 rows, 2048 columns, 40 tile rows with 8 empty
-  // ones: in runs two XCDs idle and the others work two rounds, K = 2048 / 1024 77.7 / 45.9 us; so 50.8 / 27.0)
-  int mt, nt, group = 0;
-  if (H == 1 && a.tile_group) {
-    const int size = 2 * a.chunk, i = (int)blockIdx.x >> 3, unit = ((int)blockIdx.x & 7) + 8 * (i / size), rem = i % size;
-    const int per = (a.NT + a.chunk - 1) / a.chunk;  // units of a pair of tile rows
-    mt = unit / per * 2 + (rem & 1), nt = unit % per * a.chunk + (rem >> 1);
-    if (nt >= a.NT) return;
-    if (mt >= a.MT) return;
-    group = __builtin_amdgcn_readfirstlane(a.tile_group[mt]);
-    if (group < 0) return;
-  } else {
-    const int nwg = (int)gridDim.x, bid = (int)blockIdx.x, q = nwg >> 3, r = nwg & 7, xcd = bid & 7;
-    const int lin = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (bid >> 3);
-    const int groups = max((a.MT + 4) >> 3, 1), GM = (a.MT + groups - 1) / groups;
-    const int per = GM * a.NT, grp = lin / per, rem = lin - grp * per, first = grp * GM, gsz = min(a.MT - first, GM);
-    mt = first + rem % gsz;
-    nt = rem / gsz;
-  }
-  // segment of the tile column (whole tiles per segment)
-  int seg = 0, N = a.n[0];
-  const uint16_t* w = static_cast<const uint16_t*>(a.w[0]);
-  if (!PAIR) {
-    if (a.nseg > 1 && nt >= (N + BN - 1) / BN) nt -= (N + BN - 1) / BN, seg = 1, N = a.n[1], w = static_cast<const uint16_t*>(a.w[1]);
-    if (seg == 1 && a.nseg > 2 && nt >= (N + BN - 1) / BN) nt -= (N + BN - 1) / BN, seg = 2, N = a.n[2], w = static_cast<const uint16_t*>(a.w[2]);
-  }
   const int m0 = mt * BM, n0 = nt * BN, K = a.K, KT = K >> 6;
   const uint16_t* const x = static_cast<const uint16_t*>(a.x) + (int64_t)blockIdx.y * a.x_batch_stride;
   w += (int64_t)group * a.w_group_stride + (int64_t)blockIdx.y * a.w_batch_stride;
@@ -283,6 +268,64 @@ __global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a,
     if (m >= a.M || (a.x_row && a.x_row[m] < 0)) m = -1;
     epi.store(m, erow[i], seg, n0 + cw * 64, N, q4, acc[i]);
   }
+}
+
+template <class DT, int BM, int BN, bool DEEP, bool PAIR, class EPI>
+__global__ __launch_bounds__(512, 2) void gemm_rows_kernel(const GemmRowsArgs a, const EPI epi) {
+#ifdef __HIP_DEVICE_COMPILE__
+  // tile: the ids of one XCD (id mod 8) take a contiguous run of an order that walks about 8 tile rows before the next tile column, so the
+  // workgroups of an XCD share their operands' panels in its L2; the tile rows in equal groups (the weights come by once a group: with 8 + 1 tile
+  // rows of 64, 557 rows x 14336, K = 4096 99 us, with 9 77.5).  Grouped rows: the empty tile rows are the last ones, so the XCDs take units of two tile
+  // rows (an expert's, more often than not) in turn, two rows to a column (16 experts of 188 rows, 2048 columns, 40 tile rows with 8 empty
+  // ones: in runs two XCDs idle and the others work two rounds, K = 2048 / 1024 77.7 / 45.9 us; so 50.8 / 27.0)
+  int mt, nt, group = 0;
+  if (GrTile<BM, BN, DEEP>::H == 1 && a.tile_group) {
+    const int size = 2 * a.chunk, i = (int)blockIdx.x >> 3, unit = ((int)blockIdx.x & 7) + 8 * (i / size), rem = i % size;
+    const int per = (a.NT + a.chunk - 1) / a.chunk;  // units of a pair of tile rows
+    mt = unit / per * 2 + (rem & 1), nt = unit % per * a.chunk + (rem >> 1);
+    if (nt >= a.NT) return;
+    if (mt >= a.MT) return;
+    group = __builtin_amdgcn_readfirstlane(a.tile_group[mt]);
+    if (group < 0) return;
+  } else {
+    gr_tile_of(gr_xcd_run((int)blockIdx.x, (int)gridDim.x), a.MT, a.NT, mt, nt);
+  }
+  // segment of the tile column (whole tiles per segment)
+  int seg = 0, N = a.n[0];
+  const uint16_t* w = static_cast<const uint16_t*>(a.w[0]);
+  if (!PAIR) {
+    if (a.nseg > 1 && nt >= (N + BN - 1) / BN) nt -= (N + BN - 1) / BN, seg = 1, N = a.n[1], w = static_cast<const uint16_t*>(a.w[1]);
+    if (seg == 1 && a.nseg > 2 && nt >= (N + BN - 1) / BN) nt -= (N + BN - 1) / BN, seg = 2, N = a.n[2], w = static_cast<const uint16_t*>(a.w[2]);
+  }
+  gemm_rows_tile_product<DT, BM, BN, DEEP, PAIR>(a, epi, mt, nt, seg, N, w, group);
+#endif
+}
+
+// One segment on two tiles: 256 x 256 for the first `mixed` tile columns of the whole 256-row blocks, 128 x 256 for the columns behind them and the rows
+// below.  256 x 256 is the faster tile for the work it does, but its rounds are long: what is left of the last one idles.  2120 x (5632 gate + 5632 up),
+// K = 2048: 8.3 x 44 of the large tile are 1.5 rounds, 16.6 x 44 of the small one 2.9; 256 of the one and 236 of the other are a round each.
+// us, the best single tile / so (weights from memory): that pair 105 / 97, K = 4096 185 / 167; 3300 x 12288, K = 2048 156 / 143; 8192 x 3072 120 / 93; 6500 x 8192, K = 4096 367 / 342; over the
+// 46 products of 1021..8192 rows, 3072..28672 columns that the rule takes 1.004..1.28 times as fast, 1.06 on average
+template <class DT, bool PAIR, class EPI>
+__global__ __launch_bounds__(512, 2) void gemm_rows_mixed_kernel(const GemmRowsArgs a, const EPI epi) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const int N = a.n[0], fa = a.M >> 8, ca = a.mixed, large = fa * ca;
+  const uint16_t* const w = static_cast<const uint16_t*>(a.w[0]);
+  int bid = (int)blockIdx.x, mt, nt;
+  if (bid < large) {
+    gr_tile_of(gr_xcd_run(bid, large), fa, ca, mt, nt);
+    gemm_rows_tile_product<DT, 256, 256, false, PAIR>(a, epi, mt, nt, 0, N, w, 0);
+    return;
+  }
+  const int MT = (a.M + 127) >> 7, right = MT * (a.NT - ca), lin = gr_xcd_run(bid - large, (int)gridDim.x - large);
+  if (lin < right) {
+    gr_tile_of(lin, MT, a.NT - ca, mt, nt);
+    nt += ca;
+  } else {
+    gr_tile_of(lin - right, MT - 2 * fa, ca, mt, nt);
+    mt += 2 * fa;
+  }
+  gemm_rows_tile_product<DT, 128, 256, false, PAIR>(a, epi, mt, nt, 0, N, w, 0);
 #endif
 }
 
@@ -315,7 +358,27 @@ static inline int gemm_rows_tile(long M, const int* ncols, int nseg, long batch,
   if (us) *us = cost;
   return best;
 }
+// ... for one segment that may be on two tiles (gemm_rows_mixed_kernel): the choice above, or 0x44 with the columns of 256 x 256 in the bits from 8 on.  The CUs
+// that the last round of large tiles leaves free start on small ones; taken where the same model says 4 % or more.
+static inline int gemm_rows_tiles(long M, int N, int K) {
+  double us = 0.0;
+  const int one = gemm_rows_tile(M, &N, 1, 1, K, 0, &us);
+  const long fa = M / 256, MT = (M + 127) / 128, NT = (N + 255) / 256, KT = K / 64;
+  if (K % 128 || fa == 0 || MT * NT <= 256) return one;
+  const double large = 9.2 + KT * 1.30, small = 5.4 + KT * 0.81;
+  int best = one;
+  us *= 0.96;
+  for (long ca = 1; ca <= NT; ca++) {
+    const long rounds = (fa * ca + 255) / 256, early = (rounds * 256 - fa * ca) * (long)(large / small);
+    const long rest = std::max(0L, MT * (NT - ca) + (MT - 2 * fa) * ca - early), full = rest / 256, rem = rest % 256;
+    const double v = 1.3 + rounds * large + full * small + (rem ? 5.4 + KT * (0.70 + 0.11 * rem / 256) : 0.0);
+    if (v < us) best = 0x44 | (int)ca << 8, us = v;
+  }
+  return best;
+}
 static inline bool gemm_rows_has_tile(int tile, int K) { return ((tile == 4 * 16 + 4 || tile == 3 * 16 + 4) && K % 128 == 0) || tile == 2 * 16 + 4 || tile == 3 * 16 + 2 || tile == 2 * 16 + 2 || tile == 16 + 2; }
+// (columns of 256 x 256 in the bits from 8 on, a product of M rows and N columns)
+static inline bool gemm_rows_has_tiles(int tile, int M, int N, int K) { return (tile & 0xff) == 0x44 && tile >> 8 > 0 && K % 128 == 0 && M >= 256 && (tile >> 8) * 256 < N + 256; }
 // fills the tile counts and launches
 template <class DT, int BM, int BN, bool DEEP, bool PAIR, class EPI>
 static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStream_t st) {
@@ -345,10 +408,30 @@ static void gemm_rows_launch_t(GemmRowsArgs a, const EPI& epi, int batch, hipStr
   }
   gemm_rows_kernel<DT, BM, BN, DEEP, PAIR, EPI><<<dim3(grid, (unsigned)batch), dim3(512), (size_t)T::S * T::KP * T::STG, st>>>(a, epi);
 }
+template <class DT, bool PAIR, class EPI>
+static void gemm_rows_launch_mixed(GemmRowsArgs a, const EPI& epi, int columns, hipStream_t st) {
+  a.mixed = columns;
+  a.NT = (a.n[0] + 255) / 256;
+  void (*const k)(GemmRowsArgs, EPI) = gemm_rows_mixed_kernel<DT, PAIR, EPI>;
+  static uint64_t attr_devs = 0;  // (as above)
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  if (!((__atomic_load_n(&attr_devs, __ATOMIC_RELAXED) >> (dev & 63)) & 1)) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    __atomic_fetch_or(&attr_devs, (uint64_t)1 << (dev & 63), __ATOMIC_RELAXED);
+  }
+  using A = GrTile<256, 256, false>;
+  using B = GrTile<128, 256, false>;
+  const int fa = a.M / 256, MT = (a.M + 127) / 128;
+  const unsigned grid = (unsigned)(fa * columns + MT * (a.NT - columns) + (MT - 2 * fa) * columns);
+  k<<<grid, 512, (size_t)std::max(A::S * A::STG, B::S * B::STG), st>>>(a, epi);
+}
 // 64 x 128: two K steps a phase and twice the LDS where every workgroup has a CU to itself, otherwise two workgroups a CU.  (A phase of one step is two
 // waits for LDS around 8 MFMAs a wave: 64 rows x 4096, K = 14336, 32 workgroups 79.7 us, six buffers 73.2, so 69.6; with the waves in step 94.4.)
 template <class DT, bool PAIR, class EPI>
 static void gemm_rows_launch(const GemmRowsArgs& a, const EPI& epi, int tile, int batch, hipStream_t st) {
+  if constexpr (EPI::mixes)
+    if (tile >> 8) return gemm_rows_launch_mixed<DT, PAIR>(a, epi, tile >> 8, st);
   if (tile == 4 * 16 + 4) return gemm_rows_launch_t<DT, 256, 256, false, PAIR>(a, epi, batch, st);
   if (tile == 3 * 16 + 4) return gemm_rows_launch_t<DT, 192, 256, false, PAIR>(a, epi, batch, st);
   if (tile == 2 * 16 + 4) return gemm_rows_launch_t<DT, 128, 256, false, PAIR>(a, epi, batch, st);

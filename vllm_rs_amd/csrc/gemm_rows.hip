@@ -13,6 +13,7 @@ struct DenseRowsEpi {
   const uint16_t* bias_up;
   const uint16_t* residual;
   int res_ld, out_f32;
+  static constexpr bool mixes = true;  // (with gemm_rows_mixed_kernel)
   struct Row {};
   __device__ __forceinline__ Row row(int) const { return {}; }
   __device__ __forceinline__ void store(int m, const Row&, int seg, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
@@ -112,7 +113,7 @@ void vra_launch_gemm_rows(const GemmRowsCall& c, int dtype, int64_t stream) {
   a.nseg = c.dual ? 1 : c.nseg;
   for (int s = 0; s < c.nseg; s++) a.w[s] = c.w[s], a.n[s] = c.n[s];
   if (c.dual) a.n[0] = 2 * c.n[0];
-  const int tile = c.tile ? c.tile : gemm_rows_tile(c.M, a.n, a.nseg, 1, c.K);
+  const int tile = c.tile ? c.tile : (a.nseg == 1 ? gemm_rows_tiles(c.M, a.n[0], c.K) : gemm_rows_tile(c.M, a.n, a.nseg, 1, c.K));
   auto go = [&](auto dt, auto dual) {
     DenseRowsEpi<decltype(dt), decltype(dual)::value> e = {};
     for (int s = 0; s < a.nseg; s++) e.o[s] = GemmRowsOut{c.out[s], c.bias[s], c.out_ld[s]};
@@ -128,7 +129,7 @@ extern "C" void vra_dense_gemm_tile(int32_t tile, const void* x, const void* con
                                     int32_t pair, const void* residual, void* const* out, int32_t out_f32, int32_t m, int32_t k, int32_t dtype,
                                     int64_t stream) {
   VRA_CHECK_ARG(x && w && bias && n && out && m > 0 && k > 0 && (pair ? nseg == 2 && n[0] == n[1] : nseg >= 1 && nseg <= GR_MAX_SEG), "dense gemm tile: null pointer or bad segments");
-  VRA_CHECK_ARG((dtype == VRA_BF16 || dtype == VRA_F16) && gemm_rows_has_tile(tile, k) && !(pair && residual), "dense gemm tile: no such form");
+  VRA_CHECK_ARG((dtype == VRA_BF16 || dtype == VRA_F16) && (gemm_rows_has_tile(tile, k) || gemm_rows_has_tiles(tile, m, pair ? 2 * n[0] : (nseg == 1 ? n[0] : 0), k)) && !(pair && residual), "dense gemm tile: no such form");
   GemmRowsCall r;
   r.x = x, r.x_ld = k, r.M = m, r.K = k, r.nseg = nseg, r.dual = pair != 0, r.tile = tile, r.out_f32 = out_f32, r.residual = residual, r.res_ld = n[0];
   for (int s = 0; s < nseg; s++) {
@@ -139,6 +140,7 @@ extern "C" void vra_dense_gemm_tile(int32_t tile, const void* x, const void* con
   vra_launch_gemm_rows(r, dtype, stream);
 }
 
+extern "C" int32_t vra_dense_gemm_tiles_choice(int32_t m, int32_t n, int32_t k) { return m > 0 && n > 0 && k > 0 ? gemm_rows_tiles(m, n, k) : 0; }
 extern "C" int32_t vra_dense_gemm_tile_choice(int32_t m, const int32_t* n, int32_t nseg, int32_t k) {
   return m > 0 && n && nseg >= 1 && nseg <= GR_MAX_SEG && k > 0 ? gemm_rows_tile(m, n, nseg, 1, k) : 0;
 }

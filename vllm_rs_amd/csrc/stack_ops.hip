@@ -923,6 +923,7 @@ struct StkRowsEpi {
     if (FN == FN_SOFTCAP) return softcap * tanhf(v / softcap);
     return v;
   }
+  static constexpr bool mixes = FN == FN_NONE || FN == FN_KV || FN == FN_PAIR_CLAMPED;  // (with gemm_rows_mixed_kernel)
   struct None {};
   typedef std::conditional_t<FN == FN_KV, int64_t, None> Row;
   __device__ __forceinline__ Row row(int m) const {
@@ -1823,7 +1824,9 @@ static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream) {
       GemmRowsArgs r;
       r.x = g.a, r.x_ld = g.lda, r.x_row = g.a_row, r.w[0] = g.w, r.n[0] = g.N, r.M = g.M, r.K = g.K;
       r.tile_group = g.tile_group, r.w_group_stride = g.w_group_stride, r.x_batch_stride = g.a_batch_stride, r.w_batch_stride = g.w_batch_stride;
-      const int tile = g.tile ? g.tile : gemm_rows_tile(g.tile_group && g.likely_rows > 0 ? g.likely_rows : g.M, r.n, 1, nb, g.K, g.tile_group ? g.granule : 0);  // (a tile row is one granule)
+      const int fn = rows_fn(g);
+      const bool mixes = nb == 1 && !g.tile_group && (fn == FN_NONE || fn == FN_KV || fn == FN_PAIR_CLAMPED);
+      const int tile = g.tile ? g.tile : mixes ? gemm_rows_tiles(g.M, r.n[0], g.K) : gemm_rows_tile(g.tile_group && g.likely_rows > 0 ? g.likely_rows : g.M, r.n, 1, nb, g.K, g.tile_group ? g.granule : 0);  // (a tile row is one granule)
       auto go = [&](auto fn) {
         const int per = g.out_f32 ? 4 : 8;  // elements of 16 bytes
         const bool vec = (uintptr_t)g.out % 16 == 0 && g.ldo % per == 0 && g.out_batch_stride % per == 0 && (g.out_f32 || (g.epi == 1 ? g.N % 32 : g.N % 8) == 0);
