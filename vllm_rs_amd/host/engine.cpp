@@ -1217,7 +1217,7 @@ static int32_t forward_raw_impl(Engine* en, const uint32_t* h_ids, const int64_t
   en->model_->logits_mirror = h_logits_out && !launched ? pinned_device_view(h_logits_out, logit_bytes) : nullptr;
   en->model_->logits_mirrored = false;
   struct NoMirror {  // (the caller's array is this call's, however it ends)
-    ModelBase* m;
+    vra::ModelBase* m;
     ~NoMirror() { m->logits_mirror = nullptr; }
   } const no_mirror{en->model_.get()};
   const bool ran = launched || en->model_->forward(md, (int64_t)en->stream_, h_tokens_out ? en->d_tokens_ : nullptr);
