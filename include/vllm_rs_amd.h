@@ -640,6 +640,9 @@ int32_t vra_engine_forward_raw(void* eng, const uint32_t* h_ids, const int64_t* 
                                const uint32_t* h_block_tables, int32_t max_blocks,
                                const uint32_t* h_context_lens, const uint32_t* h_cu_seqlens_q,
                                int32_t n_seqs, float* h_logits_out);
+/* the rows of logits_out that the head's launch may store there itself where that memory is pinned (0: a copy behind it): n_rows wanted ones (0: one a sequence)
+ * of a step of step_seqs sequences, padding included, n_seqs of them the caller's */
+int32_t vra_logit_rows_in_place(int32_t n_rows, int32_t n_seqs, int32_t step_seqs);
 /* The same forward, answered with the SAMPLED TOKEN IDS instead of the logits — what the reference's runner process sends back
  * (RunResponse, runner.rs:246-292).  Decode steps replay the hipGraph of their batch / context bucket when the engine was built with
  * use_graph (the reference replays its captured decode graphs the same way, graph.rs:370-377); greedy tokens are the first maximal

@@ -46,6 +46,15 @@ def test_rotary_and_cache_store_stay_within_the_default_lds():
     assert [plan(n, 8, 128, 64, 0, None) for n in (1200, 1500, 3000, 8192)] == [7, 6, 3, 1]
 
 
+def test_no_more_logit_rows_in_place_than_the_callers_array_holds():
+    """a step padded to its bucket computes more rows than the caller asked for: those go to the device's rows only"""
+    rows = _lib.load().vra_logit_rows_in_place
+    for seqs in range(1, 41):
+        for step in range(seqs, 65):
+            assert rows(0, seqs, step) == (seqs if step == seqs else 0)
+            assert rows(7, seqs, step) == 7  # (wanted rows: as many as the step's head computes)
+
+
 @pytest.mark.parametrize("dim", [4, 32, 64, 128, 256])
 def test_linear_recurrence_stages_one_token_for_one(dim):
     """a decode step's workgroups stage one token: q, k, decays, value and output of it and three numbers"""

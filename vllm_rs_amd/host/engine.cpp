@@ -1099,6 +1099,9 @@ static float* pinned_device_view(float* host, size_t bytes) {
   if (!ok) (void)hipGetLastError();  // (an address that the runtime does not know is no error of this call)
   return ok ? (float*)a.devicePointer : nullptr;
 }
+// Rows that a step's head may store in the caller's array itself: all that the array holds (the wanted ones, or one a sequence), or none where the step runs
+// with more sequences than the caller's (a decode step that is padded to its bucket): the copy takes the first of them.
+extern "C" int32_t vra_logit_rows_in_place(int32_t n_rows, int32_t n_seqs, int32_t step_seqs) { return n_rows > 0 ? n_rows : (step_seqs == n_seqs ? n_seqs : 0); }
 static int32_t forward_raw_impl(Engine* en, const uint32_t* h_ids, const int64_t* h_positions, const int64_t* h_slot_mapping,
                                 int32_t n_tokens, int32_t is_prefill, const uint32_t* h_block_tables, int32_t max_blocks,
                                 const uint32_t* h_context_lens, const uint32_t* h_cu_seqlens_q, int32_t n_seqs,
@@ -1214,15 +1217,19 @@ static int32_t forward_raw_impl(Engine* en, const uint32_t* h_ids, const int64_t
     }
   }
   const size_t logit_bytes = (size_t)(n_rows > 0 ? n_rows : n_seqs) * en->mc_.vocab_size * 4;
-  en->model_->logits_mirror = h_logits_out && !launched ? pinned_device_view(h_logits_out, logit_bytes) : nullptr;
+  const bool in_place = h_logits_out && !launched && vra_logit_rows_in_place(n_rows, n_seqs, md.n_seqs) > 0;
+  en->model_->logits_mirror = in_place ? pinned_device_view(h_logits_out, logit_bytes) : nullptr;
   en->model_->logits_mirrored = false;
-  struct NoMirror {  // (the caller's array is this call's, however it ends)
-    vra::ModelBase* m;
-    ~NoMirror() { m->logits_mirror = nullptr; }
-  } const no_mirror{en->model_.get()};
+  struct Mirror {  // (the caller's array is this call's: however it ends, no launch is left that may still write there)
+    Engine* en;
+    bool waited = false;
+    ~Mirror() {
+      en->model_->logits_mirror = nullptr;
+      if (en->model_->logits_mirrored && !waited) (void)hipStreamSynchronize(en->stream_);
+    }
+  } mirror{en};
   const bool ran = launched || en->model_->forward(md, (int64_t)en->stream_, h_tokens_out ? en->d_tokens_ : nullptr);
   if (!ran) {
-    if (en->model_->logits_mirrored) (void)hipStreamSynchronize(en->stream_);  // (the head's launch may still be writing there)
     en->error = en->model_->error;
     return -1;
   }
@@ -1242,6 +1249,7 @@ static int32_t forward_raw_impl(Engine* en, const uint32_t* h_ids, const int64_t
   // the error words (a split-K slice or a tensor-parallel peer that never arrived) are checked as in step()
   uint32_t* comm_err = en->comm_ ? vra_comm_error_word(en->comm_) : nullptr;
   if (comm_err) (void)hipMemcpyAsync(en->h_err_ + 1, comm_err, 4, hipMemcpyDeviceToHost, en->stream_);
+  mirror.waited = true;
   if (hipStreamSynchronize(en->stream_) != hipSuccess) {
     en->error = "stream error in forward_raw";
     return -1;
