@@ -679,7 +679,8 @@ void vra_stack_op_group_norm(const float* x, const float* w, void* h, int32_t T,
 void vra_stack_op_gemm(const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32,
                        int32_t M, int32_t N, int32_t K, float alpha, const int32_t* tile_group, int32_t granule, const int32_t* a_row,
                        const float* a_scale, const int32_t* out_row, int32_t epi, float limit, int32_t dtype, int64_t stream);
-/* the bf16 product of more than 32 rows on a named tile (0x12, 0x22, 0x24 or, no row groups, 0x32 or, K % 128 == 0, 0x34, 0x44: rows / 64 * 16 + columns / 64), granules of a tile's rows */
+/* the bf16 product of more than 32 rows on a named tile (0x12, 0x22, 0x24 or, no row groups, 0x32 or, K % 128 == 0, 0x34, 0x44: rows / 64 * 16 + columns / 64), granules of a tile's
+ * rows; no row groups: also the two tiles of vra_dense_gemm_tiles_choice, for a plain or a clamped gated product */
 void vra_stack_op_gemm_tile(int32_t tile, const void* a, int32_t lda, const void* w, int64_t w_group_stride, void* out, int32_t ldo, int32_t out_f32,
                             int32_t M, int32_t N, int32_t K, const int32_t* tile_group, const int32_t* a_row, int32_t a_rows,
                             const int32_t* out_row, int32_t epi, float limit, int64_t stream);
@@ -700,6 +701,9 @@ void vra_stack_op_kv_store(const void* k, const void* v, int32_t ld, void* kc, v
 /* out[:, :kv_from] = a w^T's first columns; the kv_k columns behind them are row slots[m] of kc [*, kv_k], the others row slots[m] of vc (below 0: nowhere) */
 void vra_stack_op_gemm_kv(const void* a, int32_t lda, const void* w, void* out, int32_t ldo, void* kc, void* vc, const int64_t* slots, int32_t M,
                           int32_t N, int32_t K, int32_t kv_from, int32_t kv_k, int32_t dtype, int64_t stream);
+/* ... on a named tile (as vra_stack_op_gemm_tile's; 0: by size) */
+void vra_stack_op_gemm_kv_tile(int32_t tile, const void* a, int32_t lda, const void* w, void* out, int32_t ldo, void* kc, void* vc, const int64_t* slots,
+                               int32_t M, int32_t N, int32_t K, int32_t kv_from, int32_t kv_k, int32_t dtype, int64_t stream);
 void vra_stack_op_attention(const void* q, int32_t ldq, void* out, const void* kc, const void* vc, const int64_t* positions,
                             const uint32_t* block_tables, const uint32_t* context_lens, const uint32_t* cu_q, int32_t B, int32_t T,
                             int32_t max_q, int32_t H, int32_t G, int32_t dim, int32_t vdim, int32_t BS, int32_t max_blocks,

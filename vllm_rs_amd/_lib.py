@@ -215,6 +215,7 @@ def load():
     _sig(lib, "vra_stack_op_polynorm", None, P, P, P, c_i32, c_i32, c_f32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_residual_combine", None, P, P, P, c_i32, P, P, c_f32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_gemm_kv", None, P, c_i32, P, P, c_i32, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
+    _sig(lib, "vra_stack_op_gemm_kv_tile", None, c_i32, P, c_i32, P, P, c_i32, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_kv_store", None, P, P, c_i32, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i64)
     _sig(lib, "vra_stack_op_attention", None, P, c_i32, P, P, P, P, P, P, P, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32, c_i32,
          c_f32, c_f32, c_f32, c_i32, c_i32, c_i64)

@@ -49,7 +49,7 @@ struct StkGemmArgs {
   const int64_t* kv_slot = nullptr;
   void *kv_kc = nullptr, *kv_vc = nullptr;
   int kv_from = 0, kv_k = 0;
-  int tile = 0;  // the tile of gemm_rows_kernel (rows / 64 * 16 + columns / 64) instead of the one of gemm_rows_tile; refused where that kernel does not take the product
+  int tile = 0;  // the tile of gemm_rows_kernel (rows / 64 * 16 + columns / 64), or the two of gemm_rows_tiles, instead of the choice by size; refused where that kernel does not take the product
 };
 void vra_stack_gemm(const StkGemmArgs& g, int dtype, int64_t stream);
 bool vra_stack_gemm_mirrors(const StkGemmArgs& g, int dtype);  // whether it takes StkGemmArgs::mirror

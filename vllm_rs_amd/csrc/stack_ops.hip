@@ -903,6 +903,9 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_eight_kernel(StkGemmArgs g)
 // vec: rows of the output start on 16 bytes, a lane stores whole 16-byte pieces (bf16: after trading columns with its row's other
 // three lanes).
 enum StkFn { FN_NONE, FN_KV, FN_PAIR_CLAMPED, FN_PAIR_GELU, FN_PAIR_SILU, FN_GELU, FN_RELU2, FN_TANH, FN_EXPEXP, FN_SOFTCAP };
+// the epilogues that gemm_rows_mixed_kernel is built with: q | k | v, o, up, down and the clamped pairs, whose prompts were measured on it.  The others were not measured
+// there; they have the single tiles
+static constexpr bool stk_mixes(int fn) { return fn == FN_NONE || fn == FN_KV || fn == FN_PAIR_CLAMPED; }
 template <int FN>
 struct StkRowsEpi {
   void* out;
@@ -923,7 +926,7 @@ struct StkRowsEpi {
     if (FN == FN_SOFTCAP) return softcap * tanhf(v / softcap);
     return v;
   }
-  static constexpr bool mixes = FN == FN_NONE || FN == FN_KV || FN == FN_PAIR_CLAMPED;  // (with gemm_rows_mixed_kernel)
+  static constexpr bool mixes = stk_mixes(FN);  // (with gemm_rows_mixed_kernel)
   struct None {};
   typedef std::conditional_t<FN == FN_KV, int64_t, None> Row;
   __device__ __forceinline__ Row row(int m) const {
@@ -1819,13 +1822,14 @@ static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream) {
   VRA_CHECK_ARG(g.epi != 1 || (mfma && g.N % 32 == 0), "stack gemm: the gated epilogue needs the bf16 MFMA path and whole gate / up blocks");
   if (mfma) {
     const bool rows = big && !g.a_scale && rows_kernel_takes(g);
-    VRA_CHECK_ARG(!g.tile || (rows && gemm_rows_has_tile(g.tile, g.K) && (!g.tile_group || g.granule == (g.tile >> 4) * 64)), "stack gemm: no such tile for this product");
+    const int fn = rows_fn(g);
+    const bool mixes = nb == 1 && !g.tile_group && stk_mixes(fn);
+    VRA_CHECK_ARG(!g.tile || (rows && ((gemm_rows_has_tile(g.tile, g.K) && (!g.tile_group || g.granule == (g.tile >> 4) * 64)) || (mixes && gemm_rows_has_tiles(g.tile, g.M, g.N, g.K)))),
+                  "stack gemm: no such tile for this product");
     if (rows) {
       GemmRowsArgs r;
       r.x = g.a, r.x_ld = g.lda, r.x_row = g.a_row, r.w[0] = g.w, r.n[0] = g.N, r.M = g.M, r.K = g.K;
       r.tile_group = g.tile_group, r.w_group_stride = g.w_group_stride, r.x_batch_stride = g.a_batch_stride, r.w_batch_stride = g.w_batch_stride;
-      const int fn = rows_fn(g);
-      const bool mixes = nb == 1 && !g.tile_group && (fn == FN_NONE || fn == FN_KV || fn == FN_PAIR_CLAMPED);
       const int tile = g.tile ? g.tile : mixes ? gemm_rows_tiles(g.M, r.n[0], g.K) : gemm_rows_tile(g.tile_group && g.likely_rows > 0 ? g.likely_rows : g.M, r.n, 1, nb, g.K, g.tile_group ? g.granule : 0);  // (a tile row is one granule)
       auto go = [&](auto fn) {
         const int per = g.out_f32 ? 4 : 8;  // elements of 16 bytes
@@ -1834,7 +1838,7 @@ static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream) {
                                              g.kv_slot, g.kv_kc, g.kv_vc, g.kv_from, g.kv_k};
         launch_checked("stack gemm", [&] { gemm_rows_launch<BF16, false>(r, e, tile, nb, st); });
       };
-      switch (rows_fn(g)) {
+      switch (fn) {
         case FN_PAIR_CLAMPED: go(std::integral_constant<int, FN_PAIR_CLAMPED>{}); break;
         case FN_PAIR_GELU: go(std::integral_constant<int, FN_PAIR_GELU>{}); break;
         case FN_PAIR_SILU: go(std::integral_constant<int, FN_PAIR_SILU>{}); break;
@@ -2108,9 +2112,13 @@ extern "C" void vra_stack_op_gemm(const void* a, int32_t lda, const void* w, int
 }
 extern "C" void vra_stack_op_gemm_kv(const void* a, int32_t lda, const void* w, void* out, int32_t ldo, void* kc, void* vc, const int64_t* slots, int32_t M, int32_t N, int32_t K,
                                      int32_t kv_from, int32_t kv_k, int32_t dtype, int64_t stream) {
+  vra_stack_op_gemm_kv_tile(0, a, lda, w, out, ldo, kc, vc, slots, M, N, K, kv_from, kv_k, dtype, stream);
+}
+extern "C" void vra_stack_op_gemm_kv_tile(int32_t tile, const void* a, int32_t lda, const void* w, void* out, int32_t ldo, void* kc, void* vc, const int64_t* slots, int32_t M,
+                                          int32_t N, int32_t K, int32_t kv_from, int32_t kv_k, int32_t dtype, int64_t stream) {
   VRA_CHECK_ARG(slots, "stack gemm: cache columns without slots");
   StkGemmArgs g;
-  g.a = a, g.lda = lda, g.w = w, g.out = out, g.ldo = ldo, g.M = M, g.N = N, g.K = K;
+  g.a = a, g.lda = lda, g.w = w, g.out = out, g.ldo = ldo, g.M = M, g.N = N, g.K = K, g.tile = tile;
   g.kv_slot = slots, g.kv_kc = kc, g.kv_vc = vc, g.kv_from = kv_from, g.kv_k = kv_k;
   vra_stack_gemm(g, dtype, stream);
 }
