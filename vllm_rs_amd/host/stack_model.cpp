@@ -1358,6 +1358,7 @@ bool StackModel::forward(const InputMetadata& md, int64_t stream, uint32_t* toke
     vra_stack_group_norm(fn, dt_, stream);
     due_ = {};
   }
+  if (take_stack_err(error, "final norm")) return false;  // (ahead of the head, whose launch may store in the caller's array)
   StkGemmArgs hd;
   hd.a = hl_, hd.lda = W, hd.w = head_, hd.M = rows, hd.N = vocab_, hd.K = W, hd.out = logits_, hd.ldo = vocab_, hd.out_f32 = 1, hd.alpha = logit_scale_, hd.softcap = logit_softcap_;
   if (logits_mirror && vra_stack_gemm_mirrors(hd, dt_)) hd.mirror = logits_mirror, logits_mirrored = true;
