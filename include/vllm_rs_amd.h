@@ -634,12 +634,16 @@ int32_t vra_engine_request_times(const void* eng, int64_t req, double h_times[3]
 void vra_engine_release_request(void* eng, int64_t req);
 /* low-level: one model forward with caller-built metadata, for parity tests of a1/a14.
  * Mirrors `forward(input_ids, positions, kv_caches, input_metadata)` (llama.rs:323-339): all
- * arrays are HOST arrays; logits_out is a HOST [n_seqs, vocab] f32 buffer. */
+ * arrays are HOST arrays; logits_out is a HOST [n_seqs, vocab] f32 buffer.  Where it lies on 16 bytes in memory that the runtime pinned, the head's launch
+ * stores the rows there itself (up to 32; not of f32 models).  A step that fails ahead of its head leaves the buffer as it was, one that is reported invalid
+ * behind it (an exchange that timed out) does not. */
 int32_t vra_engine_forward_raw(void* eng, const uint32_t* h_ids, const int64_t* h_positions,
                                const int64_t* h_slot_mapping, int32_t n_tokens, int32_t is_prefill,
                                const uint32_t* h_block_tables, int32_t max_blocks,
                                const uint32_t* h_context_lens, const uint32_t* h_cu_seqlens_q,
                                int32_t n_seqs, float* h_logits_out);
+/* whether the head's launch stored the rows of the vra_engine_forward_raw just before (otherwise a copy did) */
+int32_t vra_engine_logits_in_place(void* eng);
 /* the rows of logits_out that the head's launch may store there itself where that memory is pinned (0: a copy behind it): n_rows wanted ones (0: one a sequence)
  * of a step of step_seqs sequences, padding included, n_seqs of them the caller's */
 int32_t vra_logit_rows_in_place(int32_t n_rows, int32_t n_seqs, int32_t step_seqs);

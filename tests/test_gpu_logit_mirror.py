@@ -1,6 +1,7 @@
 """Logits that the head's launch stores in pinned host memory itself (host/engine.cpp pinned_device_view; csrc/gemv.cuh, gemv_dw.cuh, stack_ops.hip `mirror`)
 against the copy that an ordinary or an unaligned buffer takes, and the model's own device rows: bit for bit, nothing before or behind them, at the edges of the
-heads' forms (1..3 rows, one and two tiles of rows, more rows than they take; 8, 16 and 32 rows of a layer stack, float32)."""
+heads' forms (1..3 rows, one and two tiles of rows, more rows than they take; 8, 16 and 32 rows of a layer stack, float32).  Which of the two ways a step took is
+asked of the engine."""
 import ctypes as C
 
 import numpy as np
@@ -48,11 +49,13 @@ def test_pinned_rows_are_those_of_the_copy(form):
                 plain = np.full(n + 2, 0xABABABAB, np.uint32)
                 r2 = np.random.default_rng(seed)
                 step(B, plain.ctypes.data + 4, prompt)
+                assert not L.vra_engine_logits_in_place(eng.h)
                 assert plain[0] == plain[-1] == 0xABABABAB and np.isfinite(plain[1:-1].view(np.float32)).all() and plain[1:-1].any()
                 for start in (room // 4 - n, 16, 15):  # to the last byte, in the middle, off 16 bytes
                     pinned[:] = 0xCDCDCDCD
                     r2 = np.random.default_rng(seed)
                     step(B, ptr + start * 4, prompt)
+                    assert L.vra_engine_logits_in_place(eng.h) == (start % 4 == 0 and B <= 32 and form != "stack f32"), (B, prompt, start)
                     assert np.array_equal(pinned[start:start + n], plain[1:-1]), (B, prompt, start)
                     assert (pinned[:start] == 0xCDCDCDCD).all() and (pinned[start + n:] == 0xCDCDCDCD).all()
                     kept = np.empty(n, np.uint32)  # (the device's rows are there as before)

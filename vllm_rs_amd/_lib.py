@@ -265,6 +265,7 @@ def load():
     _sig(lib, "vra_engine_load_tensor", c_i32, P, C.c_char_p, P, P, c_i32, c_i32)
     _sig(lib, "vra_engine_finalize_weights", c_i32, P)
     _sig(lib, "vra_engine_copy_logits", c_i32, P, P, c_i32)
+    _sig(lib, "vra_engine_logits_in_place", c_i32, P)
     _sig(lib, "vra_logit_rows_in_place", c_i32, c_i32, c_i32, c_i32)
     _sig(lib, "vra_engine_debug_tp_snapshots", None, P, c_i32)
     _sig(lib, "vra_engine_norm_deferred", c_i32, P, c_i32, c_i32)

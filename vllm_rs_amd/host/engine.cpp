@@ -1268,6 +1268,10 @@ static int32_t forward_raw_impl(Engine* en, const uint32_t* h_ids, const int64_t
   if (h_tokens_out) memcpy(h_tokens_out, en->h_tokens_, (size_t)n_seqs * 4);
   return 0;
 }
+extern "C" int32_t vra_engine_logits_in_place(void* e) {
+  auto* en = static_cast<Engine*>(e);
+  return !en->dry() && en->model_->logits_mirrored;
+}
 extern "C" int32_t vra_engine_forward_raw(void* e, const uint32_t* h_ids, const int64_t* h_positions, const int64_t* h_slot_mapping,
                                           int32_t n_tokens, int32_t is_prefill, const uint32_t* h_block_tables, int32_t max_blocks,
                                           const uint32_t* h_context_lens, const uint32_t* h_cu_seqlens_q, int32_t n_seqs,
