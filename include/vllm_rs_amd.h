@@ -308,9 +308,10 @@ void vra_dense_gemm(const void* x, const void* w, const void* bias, void* out, i
 void vra_dense_gemm_tile(int32_t tile, const void* x, const void* const* w, const void* const* bias, const int32_t* n, int32_t nseg,
                          int32_t pair, const void* residual, void* const* out, int32_t out_f32, int32_t m, int32_t k, int32_t dtype,
                          int64_t stream);
-/* the tile that the row-major prompt GEMM takes for m rows x nseg tensors of n[s] columns (0: no such product) */
+/* the best single tile of the row-major prompt GEMM for m rows x nseg tensors of n[s] columns (0: no such product): what several tensors run on, and one tensor unless
+ * vra_dense_gemm_tiles_choice names two */
 int32_t vra_dense_gemm_tile_choice(int32_t m, const int32_t* n, int32_t nseg, int32_t k);
-/* ... for one tensor (or a pair's 2 n columns), which may be on two tiles: 0x44 with the number of 256-column strips on 256 x 256 in the bits from 8 on, the rest on 128 x 256;
+/* what it takes for one tensor (or a pair's 2 n columns): that tile, or two: 0x44 with the number of 256-column strips on 256 x 256 in the bits from 8 on, the rest on 128 x 256;
  * vra_dense_gemm_tile takes that, too */
 int32_t vra_dense_gemm_tiles_choice(int32_t m, int32_t n, int32_t k);
 /* logits.argmax(-1) (logits_processor.rs:67-70): first maximal index per row. */
@@ -635,7 +636,7 @@ void vra_engine_release_request(void* eng, int64_t req);
 /* low-level: one model forward with caller-built metadata, for parity tests of a1/a14.
  * Mirrors `forward(input_ids, positions, kv_caches, input_metadata)` (llama.rs:323-339): all
  * arrays are HOST arrays; logits_out is a HOST [n_seqs, vocab] f32 buffer.  Where it lies on 16 bytes in memory that the runtime pinned, the head's launch
- * stores the rows there itself (up to 32; not of f32 models).  A step that fails ahead of its head leaves the buffer as it was, one that is reported invalid
+ * stores the rows there itself (up to 32, where its kernel takes them; not of f32 models).  A step that fails ahead of its head leaves the buffer as it was, one that is reported invalid
  * behind it (an exchange that timed out) does not. */
 int32_t vra_engine_forward_raw(void* eng, const uint32_t* h_ids, const int64_t* h_positions,
                                const int64_t* h_slot_mapping, int32_t n_tokens, int32_t is_prefill,

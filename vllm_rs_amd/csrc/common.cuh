@@ -95,8 +95,8 @@ struct BF16 {
   static constexpr int id = VRA_BF16;
   typedef bf16x8_t vec8;
   static __device__ __forceinline__ float to_f32(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-  // RNE, NaN quieted (== oracle f32_to_bf16 for each of the 2^32 floats), in gfx950's one instruction: the integer form takes ten and a branch for NaN,
-  // 1.3 us for 16 rows x 64 columns a wave in a GEMM epilogue (2048 x 3072, K = 2048: 33.6 us / 30.4; SiLU pairs 2120 x 11264, K = 2048: 112 / 100)
+  // RNE, NaN quieted, in gfx950's one instruction (compared on the card with the integer form, which is the oracle's f32_to_bf16, over all 2^32 floats: no
+  // difference; the test keeps six lower halves of every upper one): the integer form takes ten and a branch for NaN, 1.3 us for 16 rows x 64 columns a wave in a GEMM epilogue (2048 x 3072, K = 2048: 33.6 us / 30.4; SiLU pairs 2120 x 11264, K = 2048: 112 / 100)
   static __device__ __forceinline__ uint16_t from_f32(float f) {
     return __builtin_bit_cast(uint16_t, (__bf16)f);
   }

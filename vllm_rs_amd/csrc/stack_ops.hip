@@ -45,8 +45,8 @@ __device__ __forceinline__ float gated_pair(float g, float u, float limit, float
 
 // ------------------------------------------------------------------------------------------------ embedding + positions
 // A thread takes both entries of an angle: lanes that alternate between sine and cosine would each wait for the other's.
-// N angles at a time: one load and one store for all of them where rows start on 16 bytes (N = 2), and the rows of a long prompt (DEPTH) asked for ahead of
-// the first sine.  2048 rows of 2048: 16.0 us one angle after the other, now 12.6; 1500 rows 13.5, 8.9.
+// N angles at a time: one load and one store for all of them where rows are whole fours of columns (N = 2: 8 bytes of bf16, 16 of f32), and the rows of a long prompt
+// (DEPTH) asked for ahead of the first sine.  2048 rows of 2048: 16.0 us one angle after the other, now 12.6; 1500 rows 13.5, 8.9.
 template <typename T, int N, int DEPTH>
 __global__ __launch_bounds__(256) void stk_embed_sinpos_kernel(const uint32_t* ids, const int64_t* pos, const T* embed, const float* inv_freq, float* x,
                                                                int W, int V) {
@@ -1908,6 +1908,9 @@ void vra_stack_embed_sinpos(const uint32_t* ids, const int64_t* positions, const
                             int dtype, int64_t stream) {
   VRA_CHECK_ARG(ids && positions && embed && x && T > 0 && W > 0, "stack embed: null pointer or empty shape");
   const dim3 grid(T, std::max(1, std::min((W / 2 + 255) / 256, 256 / T)));
+  // Two by two from 256 rows on.  us a launch, one angle / two by two (bf16): 2048 columns, 16 rows 1.98 / 2.05, 64 2.09 / 2.12, 128 2.62 / 2.22, 160 3.54 / 2.34, 255
+  // 3.67 / 2.47, 512 4.08 / 2.81; 4096 columns, 32 rows 2.07 / 2.12, 64 2.66 / 2.22, 160 5.68 / 3.17.  What decides is whether a thread would take a second angle
+  // (256 * grid.y < W / 2): the line could lie lower, at 65 rows of 2048
   const bool quads = W % 4 == 0 && (((uintptr_t)embed | (uintptr_t)inv_freq | (uintptr_t)x) % 16) == 0;
   auto go = [&](auto one) {
     typedef decltype(one) E;

@@ -494,9 +494,9 @@ bool vra_gemv_w_fits(int ns, int M, int K, int group_size, int n_units, bool has
     if (g < K && (g < 128 || (g & (g - 1)))) return false;
     int kz, ktz, groups;
     const int rb = (M + 31) / 32;
-    // which row counts: up to 63 rows no other kernel but B takes the launch; 64..96 and 129..160 rows stayed here when kernel M came, with the bits of a
-    // 32-row launch, though kernel M is quicker at most of them (down of Llama-3-8B with its residual, us, here / kernel M: 64 rows 27.9 /
-    // 25.6, 96 rows 38.4 / 32.0, 150 rows 55.0 / 45.1); at 97..128 rows and beyond 160 this form was the slower one before, too
+    // which row counts: up to 63 rows no other kernel but B takes the launch; 64..96 and 129..160 rows stay here, with the bits of a 32-row launch, though
+    // kernel M is quicker at most of them: a model's step goes there for its down projection (vra_down_mid_plan, which has both sides' times); at
+    // 97..128 rows and beyond 160 this form was the slower one when it was chosen
     static const char* any_rb = getenv("VRA_GEMV_W_KZ_ANY_RB");  // tuning aid: 1 = every row-block count up to the row limit
     if (rb > 3 && rb != 5 && !(any_rb && any_rb[0] == '1')) return false;
     if (!gemv_w_kz_plan(K, n_units, rb, &kz, &ktz, &groups)) return false;
@@ -1067,8 +1067,10 @@ extern "C" int32_t vra_wna16_kernel(int32_t pair, int32_t m, int32_t k, int32_t 
 
 // The model's down_proj of 64..96 and 129..160 rows: kernel M instead of kernel W's row blocks (which vra_wna16_gemm keeps: a row there has the bits of a 32-row
 // launch, in a model's step the products ahead of it do not).  W converts every code once per 32 rows and takes 11 us and 1.85 (AWQ 1.92) for each 16 columns of a
-// workgroup; M converts it twice in all and takes 0.92 (0.96) of its plan's estimate.  us, W / M, over K = 4608..28672 x 1024..8192: 14336 x 4096, 64 rows 24.9 / 22.6,
-// 96 rows 34.4 / 28.3, 145 rows 49.4 / 38.6; AWQ 18944 x 3584, 145 rows 57.1 / 48.4; few columns stay: 14336 x 1024, 145 rows 22 / 36, 8192 x 3584 28 / 32.
+// workgroup; M converts it twice in all and takes 0.92 (0.96) of its plan's estimate.  us, W / M, with the residual: 14336 x 4096, 64 rows 25.1 / 22.7,
+// 96 rows 34.6 / 28.2, 145 rows 49.7 / 38.5; AWQ 18944 x 3584, 145 rows 58.0 / 48.5; few columns stay: 14336 x 1024, 145 rows 22 / 36, 8192 x 3584 28 / 32.  Over K = 4608..28672 x
+// 1024..8192 the rule takes M at 183 of the shapes, 1.23 times as fast on average (two of them 1 % slower); it leaves 18 that M would do 5..12 % faster (28672 x 2048,
+// 145 rows 50.8 / 45.7).  Errors against 64 bits: alike to six digits.
 int vra_down_mid_plan(int M, int K, int N, int group_size, bool awq, bool has_res, bool has_bias) {
   if (M < 64 || K <= 4096 || N % 16 || !vra_gemv_w_fits(1, M, K, group_size, N / 16, has_res, has_bias)) return 0;
   static const char* mid_env = getenv("VRA_NO_KERNEL_M");  // tuning aid

@@ -1087,7 +1087,11 @@ struct RawSampling {
   uint64_t seed = 0;
 };
 // The device's address of host memory that the runtime pinned, if all `bytes` lie in one such allocation of the current device (otherwise null: a copy).
-// The head's launch then stores the logits there itself: a copy behind it waits for the last of them and takes 45 us for 16 rows of 32 000 (0.1 us for this).
+// The head's launch then stores the logits there itself, where its kernel can (kernel A, the dense kernel W, a layer stack's few-row kernels: up to 32 rows): a copy behind it
+// waits for the last of them.  Asking for the address takes 0.1 us.  us of a step of one layer, hidden 4096, with the copy / so: 32 000 columns, 1 row 114 / 97, 4 rows
+// 114 / 98, 16 rows 162 / 146, 32 rows 208 / 194; 128 256 columns 232 / 209, 259 / 237, 402 / 375, 547 / 528; 152 064 columns, 1 row 263 / 239, 4 rows 294 / 246 (8..32
+// rows of so many do not fit the dense kernel W: a copy); a layer stack, hidden 2048, 32 000 columns, 1, 8, 32 rows 90 / 74, 112 / 86, 199 / 152; 152 064 columns
+// 181 / 162, 280 / 191, 672 / 451.  Below 64 KB of logits the two are equal (512 columns, 1..16 rows within 1 us).
 static float* pinned_device_view(float* host, size_t bytes) {
   hipPointerAttribute_t a = {};
   hipDeviceptr_t base = nullptr;
