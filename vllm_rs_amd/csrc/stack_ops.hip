@@ -721,7 +721,8 @@ __device__ __forceinline__ uint16_t* kv_place(uint16_t* row, int64_t slot, void*
 // workgroup takes 16 * NT output columns and its 8 waves take an eighth of K each (whole K-steps of 32, ascending inside a wave); the partial
 // tiles meet in LDS and are summed in wave order.  One fixed order for a given K — another one than the large-M kernel's single chain, so the
 // two agree to rounding, not to the bit.
-template <bool SCALED, bool POST, int NT>
+// MORE: cache columns or a second output, whose places the plain form does not ask for (with both in one kernel its loop had fewer loads in flight: see STK_SMALL).
+template <bool SCALED, bool POST, int NT, bool MORE = false>
 __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g) {
   constexpr int BN = 16 * NT, NW = 8;
   __shared__ float part[NW][16 * BN];
@@ -811,10 +812,10 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g)
     if (n >= g.N) return;
     float v = total(c) * g.alpha + (g.bias ? g.bias[(int64_t)blockIdx.z * g.bias_batch_stride + n] : 0.f);
     if (POST) v = plain_value(g, v);
-    if (!POST && !SCALED && g.kv_slot) {
+    if (MORE && !POST && g.kv_slot) {
       if (uint16_t* const p = kv_place((uint16_t*)g.out + (int64_t)row * g.ldo, n < g.kv_from ? 0 : g.kv_slot[row], g.kv_kc, g.kv_vc, g.kv_from, g.kv_k, g.N, n)) *p = BF16::from_f32(v);
     } else if (g.out_f32) {
-      if (g.mirror) g.mirror[(int64_t)orow * g.ldo + n] = v;
+      if (MORE && g.mirror) g.mirror[(int64_t)orow * g.ldo + n] = v;
       ((float*)g.out)[ob + (int64_t)orow * g.ldo + n] = v;
     } else ((uint16_t*)g.out)[ob + (int64_t)orow * g.ldo + n] = BF16::from_f32(v);
   }
@@ -826,7 +827,7 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_small_kernel(StkGemmArgs g)
 // count: the even step as loaded, the odd one with the halves of the lanes' rows of sixteen traded.  What bounds it is what a CU pulls past L2 and the latency
 // of its rounds.  8 rows, us, sixteen columns / eight: 2048 columns, K = 2048 6.7 / 5.6, 5632 11.8 / 8.6, 8192 14.8 / 10.4 (one row 11.8 / 8.4); 1024
 // columns, K = 8192 14.4 / 9.9.  Beyond one workgroup a CU it gives nothing: 3072 columns, K = 2048 6.9 / 6.9; 4096, K = 4096 9.5 / 10.0, 14336 25.4 / 29.4.
-template <bool POST>
+template <bool POST, bool MORE = false>
 __global__ __launch_bounds__(512) void stk_gemm_mfma_eight_kernel(StkGemmArgs g) {
   constexpr int NW = 8, U = 2;  // steps of 64 a round, the next round's loads ahead of this one's MFMAs (without: 12.8 us at 2048 x 8192)
   __shared__ float part[NW][64];
@@ -890,10 +891,10 @@ __global__ __launch_bounds__(512) void stk_gemm_mfma_eight_kernel(StkGemmArgs g)
   v = v * g.alpha + (g.bias ? g.bias[(int64_t)blockIdx.z * g.bias_batch_stride + n] : 0.f);
   if (POST) v = plain_value(g, v);
   const int64_t at = (int64_t)blockIdx.z * g.out_batch_stride + (int64_t)orow * g.ldo + n;
-  if (!POST && g.kv_slot) {
+  if (MORE && !POST && g.kv_slot) {
     if (uint16_t* const p = kv_place((uint16_t*)g.out + (int64_t)row * g.ldo, n < g.kv_from ? 0 : g.kv_slot[row], g.kv_kc, g.kv_vc, g.kv_from, g.kv_k, g.N, n)) *p = BF16::from_f32(v);
   } else if (g.out_f32) {
-    if (g.mirror) g.mirror[(int64_t)orow * g.ldo + n] = v;
+    if (MORE && g.mirror) g.mirror[(int64_t)orow * g.ldo + n] = v;
     ((float*)g.out)[at] = v;
   } else ((uint16_t*)g.out)[at] = BF16::from_f32(v);
 }
@@ -1857,17 +1858,21 @@ static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream) {
       else if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<2, 4, 2, 2, false, true><<<grid, 256, 0, st>>>(g); });
       else launch_checked("stack gemm", [&] { stk_gemm_mfma_kernel<2, 4, 2, 2, false><<<grid, 256, 0, st>>>(g); });
     } else {
-      const bool wide = vra_stack_op_gemm_few_columns(g.M, g.N, nb, g.epi == 1) == 32;
+      const bool wide = vra_stack_op_gemm_few_columns(g.M, g.N, nb, g.epi == 1) == 32, more = g.kv_slot || g.mirror;
 #define STK_SMALL(NTV)                                                                                                                 \
   do {                                                                                                                               \
     dim3 grid((g.M + 15) / 16, (g.N + 16 * NTV - 1) / (16 * NTV), nb);                                                               \
     if (g.a_scale) launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<true, false, NTV><<<grid, 512, 0, st>>>(g); });     \
+    else if (post && more) launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false, true, NTV, true><<<grid, 512, 0, st>>>(g); }); \
     else if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false, true, NTV><<<grid, 512, 0, st>>>(g); });     \
+    else if (more) launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false, false, NTV, true><<<grid, 512, 0, st>>>(g); }); \
     else launch_checked("stack gemm", [&] { stk_gemm_mfma_small_kernel<false, false, NTV><<<grid, 512, 0, st>>>(g); });              \
   } while (0)
       if (!wide && g.M <= 8 && (int64_t)((g.N + 7) / 8) * nb <= 256 && !g.a_scale && !g.tile_group) {
         dim3 grid(1, (g.N + 7) / 8, nb);
-        if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_eight_kernel<true><<<grid, 512, 0, st>>>(g); });
+        if (post && more) launch_checked("stack gemm", [&] { stk_gemm_mfma_eight_kernel<true, true><<<grid, 512, 0, st>>>(g); });
+        else if (post) launch_checked("stack gemm", [&] { stk_gemm_mfma_eight_kernel<true><<<grid, 512, 0, st>>>(g); });
+        else if (more) launch_checked("stack gemm", [&] { stk_gemm_mfma_eight_kernel<false, true><<<grid, 512, 0, st>>>(g); });
         else launch_checked("stack gemm", [&] { stk_gemm_mfma_eight_kernel<false><<<grid, 512, 0, st>>>(g); });
       } else if (wide) STK_SMALL(2);
       else STK_SMALL(1);
