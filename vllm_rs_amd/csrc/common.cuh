@@ -100,6 +100,13 @@ struct BF16 {
   static __device__ __forceinline__ uint16_t from_f32(float f) {
     return __builtin_bit_cast(uint16_t, (__bf16)f);
   }
+  // the same in integer steps (where the instruction's form costs the loop ahead of it more)
+  static __device__ __forceinline__ uint16_t from_f32_steps(float f) {
+    uint32_t u = __float_as_uint(f);
+    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return (uint16_t)(u >> 16);
+  }
   // two floats -> packed pair (lo = a)
   static __device__ __forceinline__ uint32_t pack2(float a, float b) {
     typedef float f2 __attribute__((ext_vector_type(2)));

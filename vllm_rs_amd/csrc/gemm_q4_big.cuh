@@ -450,6 +450,13 @@ __global__ __launch_bounds__(GD_THREADS, 2) void gemm_q4_big_kernel(const GemmDA
   }
 
   // ---- epilogue: D[column (lane>>4)*4 + r][row lane&15] of tile (b, mt)
+  // (AWQ on four m-tiles: the loop holds all registers and reloads some; with the conversion instruction here it is laid out differently and every launch slower.  bf16, us,
+  // integer steps / instruction: 767 rows x 14336, K = 4096 159 / 192, 256 x 4096, K = 14336 217 / 244, pairs of 300 x 18944, K = 3584 186 / 198.  Without zero points
+  // or on two m-tiles the instruction is the faster one: 704 x 14336, K = 4096 137.7 / 132.2)
+  auto rnd = [](float v) {
+    if constexpr (AWQ && MB == 4 && DT::id == VRA_BF16) return DT::to_f32(BF16::from_f32_steps(v));
+    else return rnd_dt<DT>(v);
+  };
   constexpr int NBO = DUAL ? 2 : NB;  // output n-blocks of the wave
 #pragma unroll
   for (int b = 0; b < NBO; b++) {
@@ -473,25 +480,25 @@ __global__ __launch_bounds__(GD_THREADS, 2) void gemm_q4_big_kernel(const GemmDA
       float v[4];
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        float t = rnd_dt<DT>(acc[b][mt][r >> 1][r & 1]);
-        if (biast[0]) t = rnd_dt<DT>(t + bs[r]);
+        float t = rnd(acc[b][mt][r >> 1][r & 1]);
+        if (biast[0]) t = rnd(t + bs[r]);
         if (DUAL) {
-          float u = rnd_dt<DT>(acc[b + 2][mt][r >> 1][r & 1]);
-          if (biast[1]) u = rnd_dt<DT>(u + bs2[r]);
-          const float sl = rnd_dt<DT>(t / (1.0f + expf(-t)));
+          float u = rnd(acc[b + 2][mt][r >> 1][r & 1]);
+          if (biast[1]) u = rnd(u + bs2[r]);
+          const float sl = rnd(t / (1.0f + expf(-t)));
           t = sl * u;
         }
         v[r] = t;
       }
       if (a.residual) {
         const u32x2 rw2 = *reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(a.residual) + (size_t)m * a.res_ld + n);
-        v[0] = rnd_dt<DT>(v[0]) + DT::to_f32((uint16_t)(rw2[0] & 0xffffu));
-        v[1] = rnd_dt<DT>(v[1]) + DT::to_f32((uint16_t)(rw2[0] >> 16));
-        v[2] = rnd_dt<DT>(v[2]) + DT::to_f32((uint16_t)(rw2[1] & 0xffffu));
-        v[3] = rnd_dt<DT>(v[3]) + DT::to_f32((uint16_t)(rw2[1] >> 16));
+        v[0] = rnd(v[0]) + DT::to_f32((uint16_t)(rw2[0] & 0xffffu));
+        v[1] = rnd(v[1]) + DT::to_f32((uint16_t)(rw2[0] >> 16));
+        v[2] = rnd(v[2]) + DT::to_f32((uint16_t)(rw2[1] & 0xffffu));
+        v[3] = rnd(v[3]) + DT::to_f32((uint16_t)(rw2[1] >> 16));
       }
       if (a.out_f32) {
-        const f32x4 o = {rnd_dt<DT>(v[0]), rnd_dt<DT>(v[1]), rnd_dt<DT>(v[2]), rnd_dt<DT>(v[3])};
+        const f32x4 o = {rnd(v[0]), rnd(v[1]), rnd(v[2]), rnd(v[3])};
         *reinterpret_cast<f32x4*>(static_cast<float*>(outp) + (size_t)m * out_ld + n) = o;
       } else {
         const u32x2 o = {DT::pack2(v[0], v[1]), DT::pack2(v[2], v[3])};
