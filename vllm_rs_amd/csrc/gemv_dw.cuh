@@ -54,7 +54,8 @@ static inline size_t gemv_dw_lds_bytes(int mt, int max_units) {
   return (size_t)2 * GW_WAVES * mt * 1024 + (size_t)GW_WAVES * 32 * 4 + (size_t)max_units * mt * 256 * 4 + 64;
 }
 
-template <class DT, int MT, bool NORM>
+// HEAD: chosen rows of x and the second output, as in gemv_kernel
+template <class DT, int MT, bool NORM, bool HEAD>
 __global__ __launch_bounds__(GW_THREADS) void gemv_dw_kernel(const GemvDWArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(GW_THREADS) void gemv_dw_kernel(const GemvDWArgs a)
 #pragma unroll
   for (int mt = 0; mt < MT; mt++) {
     xrow[mt] = min(mt * 16 + (lane & 15), M - 1);
-    if (a.x_rows) xrow[mt] = a.x_rows[xrow[mt]];
+    if (HEAD && a.x_rows) xrow[mt] = a.x_rows[xrow[mt]];
   }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -221,7 +222,7 @@ __global__ __launch_bounds__(GW_THREADS) void gemv_dw_kernel(const GemvDWArgs a)
   // to the model dtype, the bias added, rounded again; an f32 output carries the same value widened)
   // (OPU divides GW_THREADS: a thread holds the same row / column of every unit it stores — its argmax candidate is a register)
   unsigned long long am_best = 0ull;
-  if (a.mirror)
+  if (HEAD && a.mirror)
     for (int i = tid; i < M * nu * 4; i += GW_THREADS) {
       const int row = i / (nu * 4), c = (i - row * nu * 4) * 4, n = u0 * 16 + c;
       f32x4 v = *reinterpret_cast<const f32x4*>(outs + (c >> 4) * OPU + row * 16 + (c & 15));

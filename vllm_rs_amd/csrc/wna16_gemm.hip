@@ -155,13 +155,13 @@ extern "C" void vra_debug_ts(unsigned long long* host, int n) { (void)hipMemcpy(
 #endif
 struct GemvArgs;
 static void gemv_debug_args(GemvArgs& a);
-template <class DT, bool INT4, int NBW, int SPT, bool AWQ>
+template <class DT, bool INT4, int NBW, int SPT, bool AWQ, bool HEAD = false>
 static void launch_gemv_v(GemvArgs a, int nblocks, size_t lds, hipStream_t st) {
   static uint64_t attr_devs = 0;  // per device: function attributes belong to the device current at the call
   const bool attr_set = dev_seen(attr_devs);
   static size_t occ_lds = ~(size_t)0;
   static int occ_val = 1;
-  auto kern = gemv_kernel<DT, INT4, NBW, SPT, AWQ>;
+  auto kern = gemv_kernel<DT, INT4, NBW, SPT, AWQ, HEAD>;
   if (!attr_set) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kMaxDynLds);
     dev_mark(attr_devs);
@@ -316,7 +316,8 @@ void vra_launch_gemv(const GemvArgs& a, bool int4, int dtype, int64_t stream) {
     else launch_gemv_q4_t<F16, 1>(a, nblocks, st);
   } else {
     const size_t lds = gemv_lds_bytes(false, 1, a.M, a.K, a.group_size);
-    if (bf) launch_gemv_v<BF16, false, 1, 1, false>(a, nblocks, lds, st);
+    if (a.x_rows || a.mirror) bf ? launch_gemv_v<BF16, false, 1, 1, false, true>(a, nblocks, lds, st) : launch_gemv_v<F16, false, 1, 1, false, true>(a, nblocks, lds, st);
+    else if (bf) launch_gemv_v<BF16, false, 1, 1, false>(a, nblocks, lds, st);
     else launch_gemv_v<F16, false, 1, 1, false>(a, nblocks, lds, st);
   }
 }
@@ -1321,10 +1322,10 @@ bool vra_gemv_dw_fits(int M, int K, int N) {
   const int mu = q + (r ? 1 : 0);
   return mu <= GDW_MAX_UNITS && gemv_dw_lds_bytes(M > 16 ? 2 : 1, mu) <= (size_t)kMaxDynLds;
 }
-template <class DT, int MT, bool NORM>
+template <class DT, int MT, bool NORM, bool HEAD>
 static void launch_gemv_dw_n(GemvDWArgs a, hipStream_t st) {
   static uint64_t attr_devs = 0;
-  auto kern = gemv_dw_kernel<DT, MT, NORM>;
+  auto kern = gemv_dw_kernel<DT, MT, NORM, HEAD>;
   if (!dev_seen(attr_devs)) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kMaxDynLds);
     dev_mark(attr_devs);
@@ -1347,13 +1348,14 @@ void vra_launch_gemv_dw(GemvDWArgs a, int dtype, int64_t stream) {
   }
   hipStream_t st = as_stream(stream);
   const bool two = a.M > 16, norm = a.norm_w != nullptr;
-  if (dtype == VRA_BF16) {
-    if (two) norm ? launch_gemv_dw_n<BF16, 2, true>(a, st) : launch_gemv_dw_n<BF16, 2, false>(a, st);
-    else norm ? launch_gemv_dw_n<BF16, 1, true>(a, st) : launch_gemv_dw_n<BF16, 1, false>(a, st);
-  } else {
-    if (two) norm ? launch_gemv_dw_n<F16, 2, true>(a, st) : launch_gemv_dw_n<F16, 2, false>(a, st);
-    else norm ? launch_gemv_dw_n<F16, 1, true>(a, st) : launch_gemv_dw_n<F16, 1, false>(a, st);
-  }
+  auto go = [&](auto dt, auto head) {
+    typedef decltype(dt) DT;
+    constexpr bool H = decltype(head)::value;
+    if (two) norm ? launch_gemv_dw_n<DT, 2, true, H>(a, st) : launch_gemv_dw_n<DT, 2, false, H>(a, st);
+    else norm ? launch_gemv_dw_n<DT, 1, true, H>(a, st) : launch_gemv_dw_n<DT, 1, false, H>(a, st);
+  };
+  if (a.x_rows || a.mirror) dtype == VRA_BF16 ? go(BF16{}, std::true_type{}) : go(F16{}, std::true_type{});
+  else dtype == VRA_BF16 ? go(BF16{}, std::false_type{}) : go(F16{}, std::false_type{});
 }
 extern "C" void vra_dense_gemm(const void* x, const void* w, const void* bias, void* out, int32_t m, int32_t k, int32_t n,
                                int32_t dtype, int32_t out_dtype, int64_t stream) {
