@@ -1036,7 +1036,11 @@ static void paged_attention_prefill(void* out, const void* q, const void* k, con
     const int mt = wgs2 >= (mt_env ? atol(mt_env) : 512) ? 2 : 1;
     dim3 pg(q_heads, (max_seqlen_q + 64 * mt - 1) / (64 * mt), batch);  // x: heads (fastest), y: row blocks, heaviest first
     hipStream_t st = as_stream(stream);
-#define VRA_PF(DT, DD, K8, MM) prefill_attn_kernel<DT, DD, K8, MM><<<pg, PF_THREADS, 0, st>>>(p)
+#define VRA_PF(DT, DD, K8, MM)                                                               \
+  do {                                                                                       \
+    if (cos) prefill_attn_kernel<DT, DD, K8, MM, true><<<pg, PF_THREADS, 0, st>>>(p);        \
+    else prefill_attn_kernel<DT, DD, K8, MM, false><<<pg, PF_THREADS, 0, st>>>(p);           \
+  } while (0)
 #define VRA_PF_MT(DT, DD, K8) \
   do {                        \
     if (mt == 2) VRA_PF(DT, DD, K8, 2); \

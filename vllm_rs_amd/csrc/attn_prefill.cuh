@@ -44,7 +44,7 @@ struct PrefillAttnArgs {
   const uint32_t* block_tables;  // [B, max_blocks]
   const uint32_t* context_lens;  // [B]
   const uint32_t* cu_q;          // [B+1]
-  // q is as the projection left it: rotated here by these tables (model dtype, [positions, D/2]) at positions[token]; null: q is rotated
+  // ROT: q is as the projection left it, rotated here by these tables (model dtype, [positions, D/2]) at positions[token]
   const void* cosv;
   const void* sinv;
   const int64_t* positions;
@@ -97,7 +97,8 @@ __device__ __forceinline__ float pf_xor32_max(float x) {
   return vra_max(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-template <class DT, int D, bool KV8, int MT>
+// ROT: q is rotated here (a form of its own: with the test in the other one, rotated queries took 1..2 % longer at up to 600 tokens, 12.05 -> 12.25 us)
+template <class DT, int D, bool KV8, int MT, bool ROT>
 __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const PrefillAttnArgs a) {
   typedef typename KVT<KV8>::elem kv_t;
   typedef typename std::conditional<KV8, u32x2, u32x4>::type raw_t;  // 8 cache elements as loaded
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(PF_THREADS, 2) void prefill_attn_kernel(const Prefi
     // (a head's pairs D/2 apart lie in one lane, j and j + DJ/2: the arithmetic and the roundings of rope_cache_kernel, which would read and write all of q
     // once more.  Its launch and this one, us, q rotated there / here: 32 + 8 heads of 128, 150 tokens 11.8 / 11.5, 600 24.4 / 22.7, 4000 191 / 186; 28 + 4, 1300 43.5 /
     // 40.1; 32 + 4 of 64, 2048 53.5 / 51.0; 8192 tokens of 32 + 8: that launch 45 / 26, this one no longer)
-    if (a.cosv) {
+    if constexpr (ROT) {
       const int64_t pos = a.positions[q0 + (valid ? qtok : 0)];
       const uint16_t* const cp = static_cast<const uint16_t*>(a.cosv) + pos * (D / 2) + oct * 8;
       const uint16_t* const sp = static_cast<const uint16_t*>(a.sinv) + pos * (D / 2) + oct * 8;
