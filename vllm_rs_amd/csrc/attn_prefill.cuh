@@ -44,14 +44,14 @@ struct PrefillAttnArgs {
   const uint32_t* block_tables;  // [B, max_blocks]
   const uint32_t* context_lens;  // [B]
   const uint32_t* cu_q;          // [B+1]
-  // ROT: q is as the projection left it, rotated here by these tables (model dtype, [positions, D/2]) at positions[token]
-  const void* cosv;
-  const void* sinv;
-  const int64_t* positions;
   int Hq, Hkv, BS, max_blocks;
   int bs_shift;  // log2(BS): this kernel takes power-of-two block sizes (others run paged_attn_kernel)
   float scale_log2e, softcap, scale;
   unsigned long long* ts;  // -DVRA_GEMV_TS builds: per-wave phase cycle sums (tools/attn_prefill_ts.py)
+  // ROT: q is as the projection left it, rotated here by these tables (model dtype, [positions, D/2]) at positions[token]
+  const void* cosv;
+  const void* sinv;
+  const int64_t* positions;
 };
 #ifdef VRA_GEMV_TS
 #define PF_STAMP(v)                               \

@@ -65,9 +65,6 @@ struct GemvArgs {
   int is_awq, scales_layout;
   int silu_dual;  // 1: seg0 = gate, seg1 = up, out = silu(gate)*up into seg0.out
   int out_f32;    // 1: store (float)round_dt(v)
-  // row m of x is its row x_rows[m] (null: m): the rows whose logits are wanted, which a launch of its own gathered ahead of the head's for 4.7 us
-  const uint32_t* x_rows;
-  float* mirror;  // dense launches with f32 output: the same values at the same places there, too (pinned host memory)
   int n_items;    // work items (n-blocks, or gate/up pairs)
   int m_groups;   // int4 kernel: row-group families (1: all M rows in every workgroup)
   int rows_per_group;
@@ -88,6 +85,9 @@ struct GemvArgs {
   // [n, K].  A row-major wave load touches 16 rows x 64 bytes — half a 128-byte line of 16 different lines, the other halves by the
   // next load: the 1 GB lm_head streamed at 5.5 TB/s in that form whatever the ring depth (a plain contiguous read: 6.75)
   int dense_tiled;
+  // row m of x is its row x_rows[m] (null: m): the rows whose logits are wanted, which a launch of its own gathered ahead of the head's for 4.7 us
+  const uint32_t* x_rows;
+  float* mirror;  // dense launches with f32 output: the same values at the same places there, too (pinned host memory)
 };
 #ifdef VRA_GEMV_TS
 // (round 6) stamps are parked in LDS and leave in ONE store per thread at the end of the kernel (GEMV_STAMP_FLUSH).  Rounds 2-5 stored

@@ -28,7 +28,6 @@
 
 struct GemvDWArgs {
   const void* x;       // [M, x_ld]
-  const uint32_t* x_rows;  // row m of x is its row x_rows[m] (null: m)
   int x_ld;
   const void* norm_w;  // fused RMSNorm weights [K] (NORM variants), else null
   float eps;
@@ -48,6 +47,7 @@ struct GemvDWArgs {
   // behind the launch: step of 16 rows x 32 000, K = 3584 (four layers of Qwen2-7B), 411 -> 391 us (in pieces of 64 bytes 397), of 4 rows 291 -> 273.  Behind the stream: a store on its
   // way over the link holds up the waits for a wave's own loads (a unit at a time 398), and a ninth wave for it leaves the others 168 registers of 208 (418)
   float* mirror;
+  const uint32_t* x_rows;  // row m of x is its row x_rows[m] (null: m)
 };
 
 static inline size_t gemv_dw_lds_bytes(int mt, int max_units) {
