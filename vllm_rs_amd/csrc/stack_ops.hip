@@ -1913,15 +1913,18 @@ void vra_stack_embed_sinpos(const uint32_t* ids, const int64_t* positions, const
                             int dtype, int64_t stream) {
   VRA_CHECK_ARG(ids && positions && embed && x && T > 0 && W > 0, "stack embed: null pointer or empty shape");
   const dim3 grid(T, std::max(1, std::min((W / 2 + 255) / 256, 256 / T)));
-  // Two by two from 256 rows on.  us a launch, one angle / two by two (bf16): 2048 columns, 16 rows 1.98 / 2.05, 64 2.09 / 2.12, 128 2.62 / 2.22, 160 3.54 / 2.34, 255
+  // Two by two from 256 rows of more than 512 columns on, and from 1024 rows of 256 or 512: up to 512 columns a thread has one angle at most, and two by two leaves half of the
+  // workgroup idle, which pays only where whole waves are left and the rows are many (512 columns, 300 rows 2.05 / 2.13, 1024 2.64 / 2.39, 8192 8.17 / 7.33; 384 columns, 512 rows
+  // 2.12 / 2.24, 8192 6.99 / 7.09; 64 columns, 8192 rows 3.99 / 4.51).  us a launch, one angle / two by two (bf16): 2048 columns, 16 rows 1.98 / 2.05, 64 2.09 / 2.12, 128 2.62 / 2.22, 160 3.54 / 2.34, 255
   // 3.67 / 2.47, 512 4.08 / 2.81; 4096 columns, 32 rows 2.07 / 2.12, 64 2.66 / 2.22, 160 5.68 / 3.17.  What decides is whether a thread would take a second angle
   // (256 * grid.y < W / 2): the line could lie lower, at 65 rows of 2048
   const bool quads = W % 4 == 0 && (((uintptr_t)embed | (uintptr_t)inv_freq | (uintptr_t)x) % 16) == 0;
+  const bool two = quads && T >= 256 && (W > 512 || (T >= 1024 && W % 256 == 0));
   auto go = [&](auto one) {
     typedef decltype(one) E;
     hipStream_t st = as_stream(stream);
     launch_checked("stack embed", [&] {
-      if (!quads || T < 256) stk_embed_sinpos_kernel<E, 1, 1><<<grid, 256, 0, st>>>(ids, positions, (const E*)embed, inv_freq, x, W, V);
+      if (!two) stk_embed_sinpos_kernel<E, 1, 1><<<grid, 256, 0, st>>>(ids, positions, (const E*)embed, inv_freq, x, W, V);
       else stk_embed_sinpos_kernel<E, 2, 2><<<grid, 256, 0, st>>>(ids, positions, (const E*)embed, inv_freq, x, W, V);
     });
   };
