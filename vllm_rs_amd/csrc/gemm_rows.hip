@@ -16,6 +16,11 @@ struct DenseRowsEpi {
   static constexpr bool mixes = true;  // (with gemm_rows_mixed_kernel)
   struct Row {};
   __device__ __forceinline__ Row row(int) const { return {}; }
+  template <class F>
+  __device__ __forceinline__ void in_form(const F& f) const {
+    f(std::integral_constant<int, 0>{});
+  }
+  template <int>
   __device__ __forceinline__ void store(int m, const Row&, int seg, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
     constexpr int NJ = DUAL ? 2 : 4;
     const GemmRowsOut* const s = seg == 0 ? &o[0] : (seg == 1 ? &o[1] : &o[2]);

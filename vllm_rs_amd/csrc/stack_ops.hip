@@ -914,7 +914,7 @@ struct StkRowsEpi {
   const float* bias;
   int64_t out_batch_stride, bias_batch_stride;
   float alpha, limit, act_alpha, softcap;
-  int ldo, out_f32, vec;
+  int ldo, out_f32, vec, form;
   const int64_t* kv_slot;  // FN_KV
   void *kc, *vc;
   int kv_from, kv_k;
@@ -934,9 +934,18 @@ struct StkRowsEpi {
     if constexpr (FN == FN_KV) return kv_slot[m];
     else return {};
   }
+  // form: rows as they lie, no bias, whole 16-byte pieces, bf16 (1) or f32 (2); everything else (0).  (Clamped pairs of 3300 x 14336, K = 4096, the tests at each of a wave's
+  // blocks of 16 rows / once: 297 / 293 us)
+  template <class F>
+  __device__ __forceinline__ void in_form(const F& f) const {
+    if (form == 2) f(std::integral_constant<int, 2>{});
+    else if (form == 1) f(std::integral_constant<int, 1>{});
+    else f(std::integral_constant<int, 0>{});
+  }
+  template <int FORM>
   __device__ __forceinline__ void store(int m, const Row& slot, int, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
     constexpr int NJ = pair ? 2 : 4;  // blocks of 16 output columns
-    const int orow = m < 0 ? -1 : (out_row ? out_row[m] : m);
+    const int orow = m < 0 ? -1 : (FORM == 0 && out_row ? out_row[m] : m);
     const int64_t ob = (int64_t)blockIdx.y * out_batch_stride + (int64_t)max(orow, 0) * ldo;
     float* const of = (float*)out + ob;
     uint16_t* const oh = (uint16_t*)out + ob;
@@ -952,7 +961,7 @@ struct StkRowsEpi {
       for (int j = 0; j < NJ; j++)
 #pragma unroll
         for (int e = 0; e < 4; e++) y[j][e] = acc[j][e] * alpha + 0.f;  // (the sum of the form with a bias: -0 becomes 0)
-      if (bias) {
+      if (FORM == 0 && bias) {
         const float* const b = bias + (int64_t)blockIdx.y * bias_batch_stride;
 #pragma unroll
         for (int j = 0; j < NJ; j++)
@@ -964,7 +973,7 @@ struct StkRowsEpi {
 #pragma unroll
         for (int e = 0; e < 4; e++) y[j][e] = fn(y[j][e]);
     }
-    if (vec && !out_f32) {
+    if (FORM == 1 || (FORM == 0 && vec && !out_f32)) {
       u32x2 v[NJ];
 #pragma unroll
       for (int j = 0; j < NJ; j++) v[j] = u32x2{BF16::pack2(y[j][0], y[j][1]), BF16::pack2(y[j][2], y[j][3])};
@@ -976,6 +985,18 @@ struct StkRowsEpi {
         if constexpr (FN == FN_KV)
           if (p) p = kv_place(oh, slot, kc, vc, kv_from, kv_k, N, n);  // (whole pieces: the launcher's condition)
         if (p) *(u32x4*)p = u32x4{v[2 * h][0], v[2 * h][1], v[2 * h + 1][0], v[2 * h + 1][1]};
+      }
+      return;
+    }
+    if constexpr (FORM == 2) {
+      // The stores of the sixteen rows before are through ahead of these: waves that run ahead of each other write too many rows at a time (2048 x 8192, K = 512 / 2048
+      // 27.8 / 62.3 us without the wait, 25.2 / 60.2 so)
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < NJ; j++) {
+        if (orow >= 0 && no + j * 16 + q4 * 4 < lim) *(f32x4*)(of + no + j * 16 + q4 * 4) = f32x4{y[j][0], y[j][1], y[j][2], y[j][3]};
+        __builtin_amdgcn_sched_barrier(0);
       }
       return;
     }
@@ -1835,7 +1856,8 @@ static void gemm_any(const StkGemmArgs& g, int dtype, int64_t stream) {
       auto go = [&](auto fn) {
         const int per = g.out_f32 ? 4 : 8;  // elements of 16 bytes
         const bool vec = (uintptr_t)g.out % 16 == 0 && g.ldo % per == 0 && g.out_batch_stride % per == 0 && (g.out_f32 || (g.epi == 1 ? g.N % 32 : g.N % 8) == 0);
-        StkRowsEpi<decltype(fn)::value> e{g.out, g.out_row, g.bias, g.out_batch_stride, g.bias_batch_stride, g.alpha, g.limit, g.act_alpha, g.softcap, g.ldo, g.out_f32, vec ? 1 : 0,
+        const int form = !vec || g.out_row || g.bias ? 0 : (!g.out_f32 ? 1 : ((g.epi == 1 ? g.N / 2 : g.N) % 4 == 0 ? 2 : 0));
+        StkRowsEpi<decltype(fn)::value> e{g.out, g.out_row, g.bias, g.out_batch_stride, g.bias_batch_stride, g.alpha, g.limit, g.act_alpha, g.softcap, g.ldo, g.out_f32, vec ? 1 : 0, form,
                                              g.kv_slot, g.kv_kc, g.kv_vc, g.kv_from, g.kv_k};
         launch_checked("stack gemm", [&] { gemm_rows_launch<BF16, false>(r, e, tile, nb, st); });
       };
