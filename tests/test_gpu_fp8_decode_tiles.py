@@ -37,3 +37,31 @@ def test_tiles_of_a_wave(ctxs, Hq, Hkv, D, dt):
                                max(ctxs), None)
     # (two storage ulps as in the other decode tests: the rotated q and k may each round to the neighbour, an E4M3 step of one key in hundreds)
     assert_close_dt(out.numpy(np.uint16, (B, Hq, D)), ref, dt, max_ulp=2.0, max_mismatch_frac=0.5, name="fp8 decode tiles", abs_floor=8e-3 if dt == BF16 else 1.5e-3)
+
+
+# many sequences: waves that load a tile, then compute it (three tiles on a full chip, heads of 64 beyond three workgroups a CU, heads of 128 in one round of two), against the same
+# sequences by threes, whose waves request a tile ahead: the same bits
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("B,Hq,Hkv,D,ctxs", [(33, 16, 8, 128, [384, 257, 33, 1]), (33, 8, 8, 128, [1024, 641, 96, 130]), (33, 8, 8, 64, [384, 290, 5, 32]),
+                                             (98, 32, 8, 64, [700, 1, 129, 544])])
+def test_many_sequences_have_the_bits_of_few(B, Hq, Hkv, D, ctxs, dt):
+    BS = 64
+    r = rng(B + D + ctxs[0])
+    mb, ctx = (max(ctxs) + BS - 1) // BS, np.array([ctxs[b % len(ctxs)] for b in range(B)], np.uint32)
+    bt = r.permutation(B * mb).reshape(B, mb).astype(np.uint32)
+    kc, vc = (ops.dev(r.integers(0, 0x78, (B * mb, Hkv, BS * D // 4, 4), np.uint8).view(np.uint32)) for _ in range(2))
+    q, k, v = rand_dt(r, (B, Hq, D), dt), rand_dt(r, (B, Hkv, D), dt, 2.0), rand_dt(r, (B, Hkv, D), dt, 2.0)
+    pos = ctx.astype(np.int64) - 1
+    slots = bt[np.arange(B), pos // BS].astype(np.int64) * BS + pos % BS
+    cos, sin = (ops.dev(orc.to_dt(t, dt)) for t in orc.rope_tables(D, 10000.0, 2048))
+    pa = ops.PagedAttention(Hq, D, D ** -0.5, Hkv, BS, dt, fp8_kvcache=True)
+
+    def run(b):
+        out = pa.rope_cache_decode(ops.dev(q[b]), ops.dev(k[b]), ops.dev(v[b]), kc, vc, cos, sin, ops.dev(pos[b]), ops.dev(slots[b]), ops.dev(bt[b]), ops.dev(ctx[b]), len(q[b]), mb,
+                                   int(ctx.max()), None)
+        return out.numpy(np.uint16, (len(q[b]), Hq, D))
+
+    many = run(slice(None))
+    assert np.isfinite(orc.from_dt(many, dt)).all() and many.any()
+    for b in range(0, B, 3):
+        assert np.array_equal(run(slice(b, b + 3)), many[b:b + 3]), b

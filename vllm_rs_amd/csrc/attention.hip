@@ -390,7 +390,8 @@ __device__ __forceinline__ size_t vra_frag_index16(int m, int c) {
 // trace it LOST: 8.69 against 7.47 us per launch (profiles/r06_trace_attention.txt) — with 8..16 workgroups on the chip the K/V tiles
 // arrive at the L1 fill rate of 8..16 CUs, and twice the requests (the clamped second tile of waves that own one included) is twice
 // the time.  Removed.)
-template <class DT, int D, bool KV8>
+// AHEAD: the loop requests a tile ahead (FP8 cache, where decode_tile_ahead says so)
+template <class DT, int D, bool KV8, bool AHEAD>
 __global__ __launch_bounds__(FD_THREADS) void decode_attn_fused_kernel(const FusedDecodeArgs a) {
   typedef typename KVT<KV8>::elem kv_t;
   constexpr int DJ = D / 32, DT16 = D / 16, HALF = D / 2;
@@ -726,10 +727,10 @@ __global__ __launch_bounds__(FD_THREADS) void decode_attn_fused_kernel(const Fus
   };
   if (kv_w0 < kv_w1) compute_tile(kv_w0, ka0, ka1, va, std::true_type{});  // (its loads went out in front of the barrier)
   int tile = kv_w0 + 1;
-  if constexpr (KV8) {
+  if constexpr (AHEAD) {
     // FP8 cache: the tile behind the one that is computed is on its way (beyond the wave's last one the last again, so that the requests are counted), as the
     // conversions to 16 bits take longer than the half as many bytes: 4 sequences of 9000 tokens, 8 kv heads 27.2 / 23.8 us with the merge, 16 of 1900 24.9 / 22.2,
-    // 300 tokens 10.1 / 10.1.  The 16-bit cache streams at 5.1 TB/s either way (4 x 9000: 35.5 / 36.2 us), and two tiles of it leave registers for little else.
+    // 300 tokens 10.1 / 10.1 (where it is the slower loop: decode_tile_ahead).  The 16-bit cache streams at 5.1 TB/s either way (4 x 9000: 35.5 / 36.2 us), and two tiles of it leave registers for little else.
     for (; tile + 1 < kv_w1; tile += 2) {
       load_tile(tile + 1, tile_blk(tile + 1), ka0, ka1, va);
       __builtin_amdgcn_sched_barrier(0);
@@ -866,6 +867,17 @@ static int decode_nsplit(int batch, int kv_heads, int max_context_len) {
   return s;
 }
 
+// FP8 cache: whether the waves request a tile ahead of the one they compute.  us, one after the other / a tile ahead, attention and merge, over 14..32 heads and 1..256 sequences of 40..9000
+// tokens.  It pays where a CU has one workgroup (8 kv heads of 128, 16 x 9000 tokens 71.0 / 54.6) or its rounds of two are not whole (96 x 2000 85.1 / 78.7).  It does not:
+// - heads of 64, beyond three workgroups a CU: the second tile's registers (148 against 124) leave no place for the fourth (8 kv heads, 128 x 600 19.9 / 21.1, 256 x 150 16.7 / 18.2);
+// - waves of three tiles on a full chip, which request one tile too many (64 x 300 15.0 / 15.6);
+// - heads of 128 in one whole round of two workgroups a CU, which hide each other's loads, up to 8 tiles a wave (32 x 1000 21.7 / 22.2; 64 x 2000, 16 tiles, 0.99).
+static bool decode_tile_ahead(int head_dim, int workgroups, int tiles, int nsplit) {
+  const int wave = ((tiles + nsplit - 1) / nsplit + FD_WAVES - 1) / FD_WAVES;  // tiles of a wave
+  if (head_dim == 64 && workgroups > 3 * 256) return false;
+  if (wave == 3 && workgroups >= 256) return false;
+  return !(head_dim == 128 && workgroups > 256 && workgroups <= 512 && wave <= 8);
+}
 extern "C" size_t vra_paged_attention_decode_workspace_bytes(int32_t max_batch, int32_t q_heads, int32_t head_dim,
                                                              int32_t max_context_len) {
   (void)max_context_len;
@@ -1150,11 +1162,12 @@ void vra_rope_cache_attention_decode_frag(void* out, const void* q, const void* 
   a.out_frag = (q_heads * head_dim) % 128 == 0 ? static_cast<uint16_t*>(out_frag) : nullptr;
   dim3 grid(a.nsplit, kv_heads, batch);
   hipStream_t st = as_stream(stream);
-  const bool kv8 = kv_dtype == VRA_FP8_E4M3;
+  const bool kv8 = kv_dtype == VRA_FP8_E4M3, ahead = kv8 && decode_tile_ahead(head_dim, a.nsplit * kv_heads * batch, (max_context_len + 31) / 32, a.nsplit);
 #define VRA_FD(DT, DD)                                                                   \
   do {                                                                                   \
-    if (kv8) decode_attn_fused_kernel<DT, DD, true><<<grid, FD_THREADS, 0, st>>>(a);     \
-    else decode_attn_fused_kernel<DT, DD, false><<<grid, FD_THREADS, 0, st>>>(a);        \
+    if (ahead) decode_attn_fused_kernel<DT, DD, true, true><<<grid, FD_THREADS, 0, st>>>(a);         \
+    else if (kv8) decode_attn_fused_kernel<DT, DD, true, false><<<grid, FD_THREADS, 0, st>>>(a);     \
+    else decode_attn_fused_kernel<DT, DD, false, false><<<grid, FD_THREADS, 0, st>>>(a);             \
   } while (0)
   if (dtype == VRA_BF16) {
     if (head_dim == 128) VRA_FD(BF16, 128);
