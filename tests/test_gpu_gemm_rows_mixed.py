@@ -5,6 +5,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+from oracle import oracle as orc
 from tests.util import BF16, F16, rand_dt, rng
 from vllm_rs_amd import _lib, ops
 
@@ -121,6 +122,25 @@ def test_two_tiles_of_a_layer_stack_by_size(form):
     one, got = (stack_product(t, form, *args, M, N, K, 2048, 512, rows) for t in (0x12, 0))
     assert all(np.array_equal(a, b) for a, b in zip(got, one))
     check_untouched(got, form, M, dst, slots)
+
+
+# a bias, loaded once for all rows of a wave: the sums without it and the bias in f32, bit for bit (columns off 16 bytes; whole pieces on one tile and on two)
+@pytest.mark.parametrize("M,N,K", [(40, 70, 64), (530, 781, 256), (530, 784, 256), (2120, 3076, 1024), (8192, 3072, 128)])
+def test_bias_of_a_layer_stack(M, N, K):
+    r = rng(M + N)
+    a, w, bias = ops.dev(rand_dt(r, (M, K), BF16)), ops.dev(rand_dt(r, (N, K), BF16, 0.05)), r.standard_normal(N).astype(np.float32)
+    bd = ops.dev(bias)
+
+    def run(b, f32):
+        out = ops.DevBuf((M + 1) * N * 4).fill_bytes(NO_SLOT)
+        ops.lib().vra_stack_op_gemm_ex(a.ptr, K, w.ptr, out.ptr, N, f32, M, N, K, 1.0, b, 0, 0, 1, 0, 0, 0, BF16, 0)
+        ops.check_error()
+        got = out.numpy(np.float32 if f32 else np.uint16, (M + 1, N))
+        assert (got[M].view(np.uint8) == NO_SLOT).all()
+        return got[:M]
+
+    want = run(None, 1) + bias
+    assert np.array_equal(run(bd.ptr, 1), want) and np.array_equal(run(bd.ptr, 0), orc.to_dt(want, BF16))
 
 
 def test_two_tiles_of_a_layer_stack_are_refused():

@@ -90,8 +90,9 @@ __device__ __forceinline__ void gr_tile_of(int lin, int MT, int NT, int& mt, int
   nt = rem / gsz;
 }
 
-// EPI::in_form(f): f(form), a constant that store takes as its template argument: what is the same for all rows is decided once.
-// EPI::store(m, row, seg, n0, N, q4, acc): the wave's 64 columns n0 .. n0 + 63 (of segment seg) of output row m; the lane holds columns n0 + 16 j + 4 q4 ..
+// EPI::in_form(n0, N, q4, f): f(form, columns): a constant that store takes as its template argument, and what it reads of the lane's columns: what is the same for
+// all rows is decided and loaded once.
+// EPI::store(m, row, columns, seg, n0, N, q4, acc): the wave's 64 columns n0 .. n0 + 63 (of segment seg) of output row m; the lane holds columns n0 + 16 j + 4 q4 ..
 // + 3 in acc[j].  Called by all lanes (lanes beyond the matrix with m = -1), so that a lane may trade columns with its row's other three.
 // row: EPI::row(m), taken ahead of the loop (rows beyond the matrix: of its last).
 // PAIR: w[0] and w[1] (gate, up; neither grouped nor batched) interleaved in blocks of 16 virtual columns, n[0] = virtual columns.
@@ -272,12 +273,12 @@ __device__ __forceinline__ void gemm_rows_tile_product(const GemmRowsArgs& a, co
   // (the requests beyond K still write LDS: they end before the workgroup does)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   VRA_MFMA_DRAIN();
-  epi.in_form([&](auto F) {
+  epi.in_form(n0 + cw * 64, N, q4, [&](auto F, const auto& columns) {
 #pragma unroll
     for (int i = 0; i < H * NX; i++) {
       int m = m0 + row0 + i * 16 + r16;
       if (m >= a.M || (a.x_row && a.x_row[m] < 0)) m = -1;
-      epi.template store<decltype(F)::value>(m, erow[i], seg, n0 + cw * 64, N, q4, acc[i]);
+      epi.template store<decltype(F)::value>(m, erow[i], columns, seg, n0 + cw * 64, N, q4, acc[i]);
     }
   });
 }

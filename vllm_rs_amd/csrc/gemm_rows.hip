@@ -17,11 +17,11 @@ struct DenseRowsEpi {
   struct Row {};
   __device__ __forceinline__ Row row(int) const { return {}; }
   template <class F>
-  __device__ __forceinline__ void in_form(const F& f) const {
-    f(std::integral_constant<int, 0>{});
+  __device__ __forceinline__ void in_form(int, int, int, const F& f) const {
+    f(std::integral_constant<int, 0>{}, Row{});
   }
   template <int>
-  __device__ __forceinline__ void store(int m, const Row&, int seg, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
+  __device__ __forceinline__ void store(int m, const Row&, const Row&, int seg, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
     constexpr int NJ = DUAL ? 2 : 4;
     const GemmRowsOut* const s = seg == 0 ? &o[0] : (seg == 1 ? &o[1] : &o[2]);
     const int no = DUAL ? n0 / 2 : n0, lim = DUAL ? N / 2 : N;

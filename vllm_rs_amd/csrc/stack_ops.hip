@@ -935,15 +935,30 @@ struct StkRowsEpi {
     else return {};
   }
   // form: rows as they lie, no bias, whole 16-byte pieces, bf16 (1) or f32 (2); everything else (0).  (Clamped pairs of 3300 x 14336, K = 4096, the tests at each of a wave's
-  // blocks of 16 rows / once: 297 / 293 us)
+  // blocks of 16 rows / once: 297 / 293 us.)  The lane's 16 bias values are loaded once for all its rows (2048 x 8192, K = 2048, us, at each block / once: f32 60.9 / 59.9, bf16 57.7 /
+  // 55.5; 4096 x 3072, K = 1024, exp(-exp) 41.5 / 39.1)
+  struct Bias {
+    float b[4][4];
+  };
   template <class F>
-  __device__ __forceinline__ void in_form(const F& f) const {
-    if (form == 2) f(std::integral_constant<int, 2>{});
-    else if (form == 1) f(std::integral_constant<int, 1>{});
-    else f(std::integral_constant<int, 0>{});
+  __device__ __forceinline__ void in_form(int n0, int N, int q4, const F& f) const {
+    if (form == 2) f(std::integral_constant<int, 2>{}, None{});
+    else if (form == 1) f(std::integral_constant<int, 1>{}, None{});
+    else if constexpr (pair) f(std::integral_constant<int, 0>{}, None{});
+    else {
+      Bias c = {};
+      if (bias) {
+        const float* const b = bias + (int64_t)blockIdx.y * bias_batch_stride;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) c.b[j][e] = b[min(n0 + j * 16 + q4 * 4 + e, N - 1)];
+      }
+      f(std::integral_constant<int, 0>{}, c);
+    }
   }
-  template <int FORM>
-  __device__ __forceinline__ void store(int m, const Row& slot, int, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
+  template <int FORM, class COLUMNS>
+  __device__ __forceinline__ void store(int m, const Row& slot, const COLUMNS& columns, int, int n0, int N, int q4, const f32x4 (&acc)[4]) const {
     constexpr int NJ = pair ? 2 : 4;  // blocks of 16 output columns
     const int orow = m < 0 ? -1 : (FORM == 0 && out_row ? out_row[m] : m);
     const int64_t ob = (int64_t)blockIdx.y * out_batch_stride + (int64_t)max(orow, 0) * ldo;
@@ -960,14 +975,11 @@ struct StkRowsEpi {
 #pragma unroll
       for (int j = 0; j < NJ; j++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) y[j][e] = acc[j][e] * alpha + 0.f;  // (the sum of the form with a bias: -0 becomes 0)
-      if (FORM == 0 && bias) {
-        const float* const b = bias + (int64_t)blockIdx.y * bias_batch_stride;
-#pragma unroll
-        for (int j = 0; j < NJ; j++)
-#pragma unroll
-          for (int e = 0; e < 4; e++) y[j][e] = acc[j][e] * alpha + b[min(no + j * 16 + q4 * 4 + e, lim - 1)];
-      }
+        for (int e = 0; e < 4; e++) {
+          float b = 0.f;  // (added without a bias, too: -0 becomes 0)
+          if constexpr (FORM == 0) b = columns.b[j][e];
+          y[j][e] = acc[j][e] * alpha + b;
+        }
 #pragma unroll
       for (int j = 0; j < NJ; j++)
 #pragma unroll
@@ -988,9 +1000,9 @@ struct StkRowsEpi {
       }
       return;
     }
-    if constexpr (FORM == 2) {
+    if (FORM == 2 || (FORM == 0 && vec && out_f32 && lim % 4 == 0)) {
       // The stores of the sixteen rows before are through ahead of these: waves that run ahead of each other write too many rows at a time (2048 x 8192, K = 512 / 2048
-      // 27.8 / 62.3 us without the wait, 25.2 / 60.2 so)
+      // 27.8 / 62.3 us without the wait, 25.2 / 60.2 so; with a bias 4096 x 8192, K = 2048 117.4 / 114.9)
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
